@@ -265,7 +265,7 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias,
  * launch plus a small fixed-order reduction.  A.B is rounded to the storage type before the
  * multiplication, as when the product is stored and re-read.  Operands as for ptj_gemm; `mul`
  * and C are row-major with row strides mul_rs / c_rs.  `workspace` must hold
- * ptj_gemm_mul_colsum_workspace_bytes(n, m) bytes (one fp32 row of sums per 64 rows of C). */
+ * ptj_gemm_mul_colsum_workspace_bytes(n, m) bytes (one fp32 row of sums per 32 rows of C). */
 size_t ptj_gemm_mul_colsum_workspace_bytes(int64_t n, int64_t m);
 int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul, void* c, void* colsum,
                         int64_t n, int64_t m, int64_t k,

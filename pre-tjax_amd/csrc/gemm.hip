@@ -1,16 +1,21 @@
 // ptj_gemm: C = A.B (+bias) (gelu) for every operand layout; kernels and launch logic in gemm_core.h.  The bf16
 // kernels are instantiated here, the fp32 ones in gemm_f32.hip (the two compile side by side).
 #include "gemm_core.h"
+#include "gemm_plan.h"
 
 extern "C" {
 
 size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
     if (n <= 0 || m <= 0 || k <= 0) return 0;
+    // which of the two kernel families runs depends on the operands' strides as well: enough for either
     const int elt = dtype == PTJ_BF16 ? 2 : 4;
     const int s = choose_splits(n, m, k, elt, (size_t)-1);
-    if (s > 1) return (size_t)s * n * m * sizeof(float);
     int first, ts, tkps;
-    return choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
+    size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
+    const GemmPlan plan = gemm_plan(n, m, k, elt, (size_t)-1, s, num_cus());
+    if (plan.cfg >= 0 && plan.splits > 1 && (size_t)plan.splits * n * m * sizeof(float) > need)
+        need = (size_t)plan.splits * n * m * sizeof(float);
+    return need;
 }
 
 int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n, int64_t m, int64_t k, int64_t a_rs,
@@ -43,8 +48,16 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n,
     g.mul = nullptr; g.mul_rs = 0; g.colpart = nullptr;
     if (epilogue == PTJ_EPI_ACCUMULATE) workspace = nullptr;   // no K split: the partial sums would not see the stored C
     int splits = workspace ? choose_splits(n, m, k, elt, workspace_bytes) : 1;
+    const int am = elt == 2 ? pick_mode<bf16>(a, a_rs, a_cs) : pick_mode<float>(a, a_rs, a_cs);
+    const int bm = elt == 2 ? pick_mode<bf16>(b, b_cs, b_rs) : pick_mode<float>(b, b_cs, b_rs);
+    GemmPlan plan = {-1, 1, 0};
+    if (epilogue != PTJ_EPI_ACCUMULATE && gt_eligible(g, am, bm))
+        plan = gemm_plan(n, m, k, elt, workspace && ptj_aligned16(workspace) ? workspace_bytes : 0, splits, num_cus());
     int64_t kps = k;
-    if (splits > 1) {
+    if (plan.cfg >= 0) {
+        splits = plan.splits;
+        kps = plan.kps;
+    } else if (splits > 1) {
         kps = ((k + splits - 1) / splits + bk - 1) / bk * bk;
         splits = (int)((k + kps - 1) / kps);
     }
@@ -52,7 +65,7 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n,
     g.k_per_split = (int)kps;
     g.splits = splits;
     g.tail_first = 0; g.tail_splits = 1; g.tail_kps = 0;
-    if (splits == 1 && workspace && ptj_aligned16(workspace))
+    if (plan.cfg < 0 && splits == 1 && workspace && ptj_aligned16(workspace))
         choose_tail_split(n, m, k, elt, workspace_bytes, &g.tail_first, &g.tail_splits, &g.tail_kps);
     {
         const int64_t v = 16 / elt;
@@ -63,9 +76,14 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n,
         g.vec_out = ok ? 1 : 0;
     }
     g.partial = (splits > 1 || g.tail_splits > 1) ? (float*)workspace : nullptr;
+    hipStream_t st = (hipStream_t)stream;
+    if (plan.cfg >= 0) {
+        g.stream = 0;
+        return dtype == PTJ_F32 ? ptj_gemm_detail::gemm_tile_launch_f32(g, plan.cfg, am, bm, st)
+                                : ptj_gemm_detail::gemm_tile_launch_bf16(g, plan.cfg, am, bm, st);
+    }
     // streamed tiles need whole, evenly many K panels (the two-step loop body) and vector-aligned outputs
     g.stream = (splits == 1 && g.vec_out && k >= 2 * bk && k % bk == 0) ? 1 : 0;
-    hipStream_t st = (hipStream_t)stream;
     return dtype == PTJ_F32 ? ptj_gemm_detail::launch_plain_f32(g, splits, st) : gemm_impl<bf16>(g, splits, st);
 }
 

@@ -64,6 +64,13 @@ struct GemmArgs {
     float* colpart;
 };
 int launch_plain_f32(const GemmArgs& g, int splits, hipStream_t st);   // gemm_f32.hip
+// gemm_tile_bf16.hip, gemm_tile_f32.hip: configuration `cfg` of the one-tile-per-workgroup kernels (gemm_plan.h), with
+// the second stage of its K split; am / bm: operand layouts (LoadMode).  The multiplying epilogue leaves one row of
+// column sums per *mul_rows rows of C in g.colpart.
+int gemm_tile_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
+int gemm_tile_launch_f32(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
+int gemm_tile_mul_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipStream_t st);
+int gemm_tile_mul_launch_f32(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipStream_t st);
 }  // namespace ptj_gemm_detail
 
 namespace {
@@ -878,7 +885,26 @@ __global__ __launch_bounds__(256) void gemm_tail_reduce_kernel(const GemmArgs g)
     }
 }
 
+template <typename T>
+int launch_splitk_reduce(const GemmArgs& g, int splits, hipStream_t st) {
+    const int64_t total = (int64_t)g.n * g.m;
+    const bool quad = g.vec_out && g.m % 4 == 0 && ptj_aligned16(g.partial);
+    int64_t blocks = ((quad ? total / 4 : total) + 255) / 256;
+    if (blocks > 256 * 8) blocks = 256 * 8;
+    if (quad)
+        hipLaunchKernelGGL((gemm_splitk_reduce4_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st,
+                           (const float*)g.partial, splits, g.n, g.m, (T*)g.c, g.c_rs, (const T*)g.bias, g.epilogue,
+                           (T*)g.c_aux, g.c_aux_rs);
+    else
+        hipLaunchKernelGGL((gemm_splitk_reduce_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st,
+                           (const float*)g.partial, splits, g.n, g.m, (T*)g.c, g.c_rs, (const T*)g.bias, g.epilogue,
+                           (T*)g.c_aux, g.c_aux_rs);
+    PTJ_CHECK_LAUNCH();
+    return PTJ_OK;
+}
+
 #include "gemm_direct.h"
+#include "gemm_tile.h"
 
 template <typename T>
 int pick_mode(const void* p, int64_t s_row, int64_t s_k) {
@@ -956,19 +982,8 @@ int gemm_impl(GemmArgs g, int splits, hipStream_t st) {
     }
     PTJ_CHECK_LAUNCH();
     if (splits > 1) {
-        const int64_t total = (int64_t)g.n * g.m;
-        const bool quad = g.vec_out && g.m % 4 == 0 && ptj_aligned16(g.partial);
-        int64_t blocks = ((quad ? total / 4 : total) + 255) / 256;
-        if (blocks > 256 * 8) blocks = 256 * 8;
-        if (quad)
-            hipLaunchKernelGGL((gemm_splitk_reduce4_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st,
-                               (const float*)g.partial, splits, g.n, g.m, (T*)g.c, g.c_rs, (const T*)g.bias, g.epilogue,
-                               (T*)g.c_aux, g.c_aux_rs);
-        else
-            hipLaunchKernelGGL((gemm_splitk_reduce_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st,
-                               (const float*)g.partial, splits, g.n, g.m, (T*)g.c, g.c_rs, (const T*)g.bias, g.epilogue,
-                               (T*)g.c_aux, g.c_aux_rs);
-        PTJ_CHECK_LAUNCH();
+        const int rc = launch_splitk_reduce<T>(g, splits, st);
+        if (rc != PTJ_OK) return rc;
     }
     if (g.tail_splits > 1) {
         hipLaunchKernelGGL((gemm_tail_reduce_kernel<T>), dim3((unsigned)(num_m * num_n - g.tail_first), 12), dim3(256), 0,

@@ -2,10 +2,11 @@
 // stores (kernels and launch logic in gemm_core.h), the second stage of those sums, and the two-pass form
 // for operand layouts that the GEMM reads element by element.
 #include "gemm_core.h"
+#include "gemm_plan.h"
 
 namespace {
 
-// Second stage of the MUL epilogue: out[col] = sum over the 64-row blocks of colpart[block][col].  A
+// Second stage of the MUL epilogue: out[col] = sum over the row blocks of colpart[block][col].  A
 // workgroup owns 64 columns; its four wavefronts take the blocks b = w, w + 4, ... (independent,
 // coalesced loads, eight in flight) and their sums are combined in wavefront order: the order of
 // the additions is fixed.
@@ -57,7 +58,7 @@ extern "C" {
 
 size_t ptj_gemm_mul_colsum_workspace_bytes(int64_t n, int64_t m) {
     if (n <= 0 || m <= 0) return 0;
-    return (size_t)((n + 63) / 64) * (size_t)m * sizeof(float);
+    return (size_t)((n + 31) / 32) * (size_t)m * sizeof(float);   // a block of sums has 64 rows, 32 in the smallest tiles
 }
 
 int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul, void* c, void* colsum, int64_t n, int64_t m,
@@ -70,6 +71,7 @@ int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul, void* c, 
     PTJ_CHECK_ARG(colsum, "gemm_mul_colsum: null pointer");
     hipStream_t st = (hipStream_t)stream;
     const size_t need = ptj_gemm_mul_colsum_workspace_bytes(n, m);
+    int mul_rows = 64;   // rows of C per row of partial sums
     if (n > 0) {
         PTJ_CHECK_ARG(c && mul && (k == 0 || (a && b)), "gemm_mul_colsum: null pointer");
         PTJ_CHECK_ARG(c_rs >= m && mul_rs >= m, "gemm_mul_colsum: row stride below m %lld", (long long)m);
@@ -94,10 +96,15 @@ int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul, void* c, 
         g.vec_out = (ptj_aligned16(c) && c_rs % v == 0 && ptj_aligned16(mul) && mul_rs % v == 0 && ptj_aligned16(workspace) &&
                      m % 4 == 0) ? 1 : 0;
         g.stream = (g.vec_out && k >= 2 * bk && k % bk == 0) ? 1 : 0;
-        const bool vector_operands =
-            dtype == PTJ_F32 ? (pick_mode<float>(a, g.a_row, g.a_k) != GENERIC && pick_mode<float>(b, g.b_row, g.b_k) != GENERIC)
-                             : (pick_mode<bf16>(a, g.a_row, g.a_k) != GENERIC && pick_mode<bf16>(b, g.b_row, g.b_k) != GENERIC);
-        if (vector_operands) {
+        const int am = dtype == PTJ_F32 ? pick_mode<float>(a, g.a_row, g.a_k) : pick_mode<bf16>(a, g.a_row, g.a_k);
+        const int bm = dtype == PTJ_F32 ? pick_mode<float>(b, g.b_row, g.b_k) : pick_mode<bf16>(b, g.b_row, g.b_k);
+        GemmPlan plan = {-1, 1, 0};
+        if (gt_eligible(g, am, bm)) plan = gemm_plan(n, m, k, elt, 0, 1, num_cus());
+        if (plan.cfg >= 0) {
+            const int rc = dtype == PTJ_F32 ? ptj_gemm_detail::gemm_tile_mul_launch_f32(g, plan.cfg, am, bm, &mul_rows, st)
+                                            : ptj_gemm_detail::gemm_tile_mul_launch_bf16(g, plan.cfg, am, bm, &mul_rows, st);
+            if (rc != PTJ_OK) return rc;
+        } else if (am != GENERIC && bm != GENERIC) {
             const int rc = dtype == PTJ_F32 ? gemm_impl<float, true>(g, 1, st) : gemm_impl<bf16, true>(g, 1, st);
             if (rc != PTJ_OK) return rc;
         } else {
@@ -115,7 +122,7 @@ int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul, void* c, 
             PTJ_CHECK_LAUNCH();
         }
     }
-    const int blocks = (int)((n + 63) / 64);
+    const int blocks = (int)((n + mul_rows - 1) / mul_rows);
     const dim3 grid((unsigned)((m + 63) / 64));
     if (dtype == PTJ_F32)
         hipLaunchKernelGGL((gemm_colpart_reduce_kernel<float>), grid, dim3(256), 0, st, (const float*)workspace, blocks,

@@ -1,0 +1,106 @@
+// Which GEMM kernel a product takes.  Two families exist: the persistent 256x192 kernels (gemm_core.h,
+// gemm_direct.h), which stream tile after tile through every CU and win when there are several rounds of
+// tiles, and the one-tile-per-workgroup kernels of gemm_tile.h, which win when the 256x192 tiles would
+// leave CUs idle or when a border would take the slow element-wise loader.
+//
+// The choice minimises a time estimate,
+//     start + rounds * (K steps * step + finish)  [+ second stage of a K split],
+// where a round is one workgroup in every slot (256 CUs x workgroups per CU).  start, step and finish
+// (microseconds) are fitted per kernel to timings of 11 products of GPT-2's feature widths at 64 to 8192
+// tokens in all operand layouts (launches replayed from a graph, operands rotating over 200 MB): the
+// estimate is within 10 % of the measurement on average, and the kernel it picks within 1.2 % of the
+// best one.
+#pragma once
+#include "common.h"
+
+namespace {
+
+struct TileCost {
+    int tbm, tbn;        // C tile
+    int bkt;             // contraction elements per K step (panels of 128 bytes x K groups)
+    int per_cu;          // workgroups per CU
+    double start, step, finish;   // us
+    double shared;       // step time with every slot of a CU taken, relative to one workgroup per CU
+};
+
+// bf16 / fp32; the index is the configuration number of gemm_tile_launch
+constexpr int GT_CONFIGS = 7;
+constexpr TileCost GT_COST[2][GT_CONFIGS] = {
+    {{32, 32, 256, 1, 2.03, 0.522, 1.24, 1.0},
+     {64, 64, 128, 1, 2.49, 0.372, 1.81, 1.0},
+     {64, 128, 64, 2, 3.49, 0.299, 1.21, 1.89},
+     {128, 128, 64, 1, 1.84, 0.402, 3.18, 1.0},
+     {128, 128, 64, 2, 2.73, 0.714, 1.88, 1.39},
+     {128, 192, 64, 2, 2.45, 0.922, 5.00, 1.50},
+     {256, 192, 64, 1, 2.00, 1.250, 8.00, 1.0}},
+    {{32, 32, 128, 1, 2.84, 0.684, 1.69, 1.0},
+     {64, 64, 64, 1, 3.05, 1.091, 2.52, 1.0},
+     {64, 64, 64, 2, 2.85, 1.370, 2.15, 1.47},
+     {64, 128, 32, 2, 4.85, 1.047, 1.75, 1.86},
+     {128, 128, 32, 2, 3.06, 2.036, 2.59, 1.83},
+     {128, 96, 64, 1, 4.62, 3.027, 3.34, 1.27},
+     {128, 192, 32, 2, 2.44, 2.985, 6.70, 1.84}},
+};
+
+struct GemmPlan {
+    int cfg;      // configuration of gemm_tile.h, or -1: the persistent kernels with their own K split
+    int splits;   // K splits of cfg >= 0
+    int kps;      // contraction elements per split (a multiple of bkt)
+};
+
+inline int64_t gp_ceil(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Second stage of a K split: its launch, and the partial sums written and read once more.
+inline double gp_reduce_us(int64_t n, int64_t m, int splits) {
+    return splits > 1 ? 2.6 + 0.35e-6 * 4.0 * (double)splits * (double)n * (double)m : 0.0;
+}
+
+inline double gp_tile_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int splits, int cus) {
+    const int64_t work = gp_ceil(n, c.tbm) * gp_ceil(m, c.tbn) * splits;
+    const int64_t steps = gp_ceil(gp_ceil(k, splits), c.bkt);
+    const int64_t slots = (int64_t)cus * c.per_cu, full = work / slots, rem = work % slots;
+    double t = c.start + (double)full * ((double)steps * c.step * c.shared + c.finish);
+    if (rem) t += (double)steps * c.step * (rem > cus ? c.shared : 1.0) + c.finish;
+    // a chip that stays full over several rounds shares the path from L2: measured 10 % at 1.5 rounds, 30 % at many
+    const double rounds = (double)work / (double)slots;
+    if (rounds > 1.0) t *= 1.0 + 0.3 * (1.0 - 1.0 / rounds);
+    return t + gp_reduce_us(n, m, splits);
+}
+
+// The persistent kernels: 20 us (fp32: 135 us) per round of 256x192 tiles at k = 768; a partial panel along K goes
+// through the element-wise loader.
+inline double gp_persistent_us(int64_t n, int64_t m, int64_t k, int elt, int splits, int cus) {
+    const int bk = 128 / elt;
+    const int64_t work = gp_ceil(n, 256) * gp_ceil(m, 192) * splits, steps = gp_ceil(gp_ceil(k, splits), bk);
+    const int64_t full = work / cus, rem = work % cus;
+    const double rounds = (double)full + (rem ? 0.35 + 0.65 * (double)rem / cus : 0.0);
+    double t = elt == 2 ? 7.0 + rounds * (1.2 * (double)steps + 4.3) : 12.0 + rounds * (5.3 * (double)steps + 7.0);
+    if (n % 256 != 0 || m % 192 != 0) t += elt == 2 ? 8.0 : 4.0;
+    if (k % bk != 0) t += elt == 2 ? 20.0 : 30.0;
+    return t + gp_reduce_us(n, m, splits);
+}
+
+// `persistent_splits`: what choose_splits gives the persistent kernels; `ws_bytes`: workspace for fp32 partial sums.
+// Contractions shorter than 1024 are not split, so that a product and the same product with another epilogue
+// add in the same order.
+inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int persistent_splits, int cus) {
+    GemmPlan best = {-1, 1, (int)k};
+    // within 8 % the persistent kernels are kept: in a training step their loads run on from product to product
+    double best_us = 0.92 * gp_persistent_us(n, m, k, elt, persistent_splits, cus);
+    for (int i = 0; i < GT_CONFIGS; ++i) {
+        const TileCost& c = GT_COST[elt == 2 ? 0 : 1][i];
+        for (int s = 1; s <= 16; ++s) {
+            if (s > 1 && (k < 1024 || k / s < 256 || (size_t)s * (size_t)n * (size_t)m * sizeof(float) > ws_bytes)) break;
+            const int64_t kps = gp_ceil(gp_ceil(k, s), c.bkt) * c.bkt;
+            if (s > 1 && gp_ceil(k, kps) != s) continue;
+            const double us = gp_tile_us(c, n, m, k, s, cus);
+            if (us < best_us) {
+                best_us = us;
+                best = {i, s, (int)(s > 1 ? kps : k)};
+            }
+        }
+    }
+    return best;
+}
+
+}  // namespace
