@@ -362,6 +362,36 @@ int ptj_attn_bwd(const void* d_o, const void* q, const void* k, const void* v, c
                  int64_t dv_b_stride, int64_t dv_h_stride, int64_t dv_row_stride,
                  int train, int64_t seed, int dtype, void* stream);
 
+/* ---- the transformer stack ------------------------------------------------ */
+
+/* Embedding, all blocks and the final LayerNorm, forward and backward, as one call each: the launch
+ * sequence of t_gpt2_tlayers_fwd3_t and of t_gpt2_bkwd3_p_t below the LM head
+ * (model_triton.py:2334-2351, :2583-2593), made of the entry points above.  Head dimension 64
+ * (dim = 64 * heads), seq a multiple of 64; every tensor contiguous.
+ *   params  3 + 10 * layers + 2 pointers in the order of the parameter nest
+ *           (model_torch_func.py:36-43): table [vocab, dim], its bias (not read), positions
+ *           [>= seq, dim]; per block ln1 gain and shift, Wqkv, Wo, ln2 gain and shift, W1, b1, W2, b2;
+ *           final gain and shift.  `params`, `seeds` and `grads` are HOST arrays.
+ *   seeds   1 + 3 * layers dropout seeds (train != 0), in the order of p_gen_aux (:2344)
+ *   mask    as for ptj_attn_fwd
+ *   acts    ptj_gpt2_acts_bytes(shape, keep) bytes; keep != 0: everything the backward reads stays
+ *           there, keep == 0: one block's worth, for a forward without a backward
+ *   x_last, h   [batch * seq, dim]: the last block's output and its LayerNorm
+ * ptj_gpt2_bwd takes dh = the gradient of h and writes grads[3 ..] (entries like `params`; the first
+ * three are not touched) and demb [batch * seq, dim] = the gradient of table row + position of every
+ * token.  Each result is bit-equal to the same sequence of single calls. */
+typedef struct ptj_gpt2_shape {
+    int64_t layers, batch, seq, dim, heads, ffn, vocab, dtype, train;
+} ptj_gpt2_shape;
+size_t ptj_gpt2_acts_bytes(const ptj_gpt2_shape* shape, int keep);
+size_t ptj_gpt2_workspace_bytes(const ptj_gpt2_shape* shape, int backward);
+int ptj_gpt2_fwd(const ptj_gpt2_shape* shape, const void* const* params, const int64_t* tokens, const uint32_t* mask,
+                 const int64_t* seeds, void* acts, size_t acts_bytes, int keep, void* x_last, void* h,
+                 void* workspace, size_t workspace_bytes, void* stream);
+int ptj_gpt2_bwd(const ptj_gpt2_shape* shape, const void* const* params, const uint32_t* mask, const int64_t* seeds,
+                 const void* acts, size_t acts_bytes, const void* x_last, const void* dh, void* const* grads, void* demb,
+                 void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

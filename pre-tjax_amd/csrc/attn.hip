@@ -36,6 +36,7 @@
 // delta = rowsum(dO * O) of its queries and stores it), then (dK, dV) over key tiles,
 // which reads delta; both recompute S and dP.
 #include "common.h"
+#include "internal.h"
 #include "mma_tile.h"
 
 namespace {
@@ -254,10 +255,13 @@ __device__ __forceinline__ void store_rows(T* __restrict__ row, const f32x16 (&a
 }
 
 // ---- keep-bit line per batch-head ---------------------------------------------------
-__global__ __launch_bounds__(256) void attn_keepbits_kernel(uint32_t* __restrict__ bits, int bitwords, uint64_t seed) {
+constexpr int KEEP_SEEDS = 64;   // attention calls per launch
+struct KeepSeeds { uint64_t s[KEEP_SEEDS]; };
+__global__ __launch_bounds__(256) void attn_keepbits_kernel(uint32_t* __restrict__ bits, int bitwords, const KeepSeeds seeds) {
     const int bh = blockIdx.y;
+    bits += (int64_t)blockIdx.z * gridDim.y * bitwords;
     const int o = blockIdx.x * 256 + threadIdx.x;
-    const uint64_t s = seed + (uint64_t)bh;
+    const uint64_t s = seeds.s[blockIdx.z] + (uint64_t)bh;
     const bool keep = philox_keep((uint32_t)o, (uint32_t)s, (uint32_t)(s >> 32));
     const uint64_t m = __ballot(keep);
     if ((threadIdx.x & 63) == 0) {
@@ -856,7 +860,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_bwd_
     } while (0)
 
 // ---- host side ----------------------------------------------------------------------------
-inline size_t bits_bytes(int64_t BH, int64_t T) { return (size_t)BH * (2 * T / 32 + 2) * sizeof(uint32_t); }
+inline size_t bits_bytes(int64_t BH, int64_t T) { return (size_t)BH * ptj_attn_bitwords(T) * sizeof(uint32_t); }
 inline size_t delta_bytes(int64_t BH, int64_t T) { return (size_t)BH * T * sizeof(float); }
 
 int check_common(const char* what, int64_t B, int64_t H, int64_t T, int64_t dh, int dtype,
@@ -874,14 +878,95 @@ int check_common(const char* what, int64_t B, int64_t H, int64_t T, int64_t dh, 
     return PTJ_OK;
 }
 
-int launch_keepbits(uint32_t* bits, int64_t BH, int bitwords, int64_t seed, hipStream_t st) {
-    hipLaunchKernelGGL(attn_keepbits_kernel, dim3((bitwords * 32 + 255) / 256, (unsigned)BH), dim3(256), 0, st, bits,
-                       bitwords, (uint64_t)seed);
+int launch_keepbits(uint32_t* bits, int64_t count, const int64_t* seeds, int64_t stride, int64_t BH, int bitwords,
+                    hipStream_t st) {
+    for (int64_t c = 0; c < count; c += KEEP_SEEDS) {
+        const int64_t n = count - c < KEEP_SEEDS ? count - c : KEEP_SEEDS;
+        KeepSeeds ks = {};
+        for (int64_t i = 0; i < n; ++i) ks.s[i] = (uint64_t)seeds[(c + i) * stride];
+        hipLaunchKernelGGL(attn_keepbits_kernel, dim3((bitwords * 32 + 255) / 256, (unsigned)BH, (unsigned)n), dim3(256), 0, st,
+                           bits + c * BH * bitwords, bitwords, ks);
+        PTJ_CHECK_LAUNCH();
+    }
+    return PTJ_OK;
+}
+
+void launch_fwd(const AttnArgs& a, int dtype, hipStream_t st) {
+    const dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.T + 127) / 128));
+    if (dtype == PTJ_F32) ATTN_LAUNCH(attn_fwd_kernel, float, grid, st, a);
+    else ATTN_LAUNCH(attn_fwd_kernel, bf16, grid, st, a);
+}
+
+// The dQ pass also writes delta, which the dK/dV pass reads.
+void launch_bwd(const AttnArgs& dq, const AttnArgs& dkdv, int dtype, hipStream_t st) {
+    const dim3 grid((unsigned)(dq.B * dq.H), (unsigned)((dq.T + 127) / 128));
+    if (dtype == PTJ_F32) {
+        ATTN_LAUNCH(attn_bwd_dq_kernel, float, grid, st, dq);
+        ATTN_LAUNCH(attn_bwd_dkdv_kernel, float, grid, st, dkdv);
+    } else {
+        ATTN_LAUNCH(attn_bwd_dq_kernel, bf16, grid, st, dq);
+        ATTN_LAUNCH(attn_bwd_dkdv_kernel, bf16, grid, st, dkdv);
+    }
+}
+
+// Q, K, V as the column slices of one [B*T, H*3*64] buffer, O as [B*T, H*64].
+AttnArgs packed_args(const void* qkv, const uint32_t* mask, float* ms, float* ls, const uint32_t* bits, int64_t B, int64_t H,
+                     int64_t T, int train, int dtype) {
+    AttnArgs a = {};
+    const int64_t e = dtype == PTJ_BF16 ? 2 : 4, row = H * 3 * DH;
+    a.q = qkv;
+    a.k = (const char*)qkv + DH * e;
+    a.v = (const char*)qkv + 2 * DH * e;
+    a.mask = mask; a.ms = ms; a.ls = ls; a.keepbits = bits;
+    a.B = (int)B; a.H = (int)H; a.T = (int)T; a.bitwords = (int)ptj_attn_bitwords(T);
+    a.q_bs = a.k_bs = a.v_bs = T * row;
+    a.q_hs = a.k_hs = a.v_hs = 3 * DH;
+    a.q_rs = a.k_rs = a.v_rs = row;
+    a.train = train != 0;
+    a.scale = 0.125f;
+    return a;
+}
+
+}  // namespace
+
+int ptj_attn_keepbits_many(uint32_t* bits, int64_t count, const int64_t* seeds, int64_t stride, int64_t BH, int64_t T,
+                           hipStream_t st) {
+    return launch_keepbits(bits, count, seeds, stride, BH, (int)ptj_attn_bitwords(T), st);
+}
+
+int ptj_attn_fwd_packed(const void* qkv, const uint32_t* mask, void* o, float* ms, float* ls, const uint32_t* bits, int64_t B,
+                        int64_t H, int64_t T, int train, int dtype, hipStream_t st) {
+    const int rc = check_common("attn_fwd", B, H, T, DH, dtype, {qkv, o}, {});
+    if (rc) return rc;
+    AttnArgs a = packed_args(qkv, mask, ms, ls, bits, B, H, T, train, dtype);
+    a.out0 = o;
+    a.out0_bs = T * H * DH; a.out0_hs = DH; a.out0_rs = H * DH;
+    launch_fwd(a, dtype, st);
     PTJ_CHECK_LAUNCH();
     return PTJ_OK;
 }
 
-}  // namespace
+int ptj_attn_bwd_packed(const void* d_o, const void* qkv, const void* o, const float* ms, const float* ls,
+                        const uint32_t* mask, void* dqkv, float* delta, const uint32_t* bits, int64_t B, int64_t H, int64_t T,
+                        int train, int dtype, hipStream_t st) {
+    const int rc = check_common("attn_bwd", B, H, T, DH, dtype, {d_o, qkv, o, dqkv}, {});
+    if (rc) return rc;
+    AttnArgs a = packed_args(qkv, mask, const_cast<float*>(ms), const_cast<float*>(ls), bits, B, H, T, train, dtype);
+    a.o = o; a.d_o = d_o; a.delta = delta;
+    a.o_bs = a.do_bs = T * H * DH;
+    a.o_hs = a.do_hs = DH;
+    a.o_rs = a.do_rs = H * DH;
+    const int64_t e = dtype == PTJ_BF16 ? 2 : 4;
+    AttnArgs kv = a, q = a;
+    q.out0 = dqkv;
+    q.out0_bs = a.q_bs; q.out0_hs = a.q_hs; q.out0_rs = a.q_rs;
+    kv.out0 = (char*)dqkv + DH * e;
+    kv.out1 = (char*)dqkv + 2 * DH * e;
+    kv.out0_bs = kv.out1_bs = a.q_bs; kv.out0_hs = kv.out1_hs = a.q_hs; kv.out0_rs = kv.out1_rs = a.q_rs;
+    launch_bwd(q, kv, dtype, st);
+    PTJ_CHECK_LAUNCH();
+    return PTJ_OK;
+}
 
 extern "C" {
 
@@ -927,7 +1012,7 @@ int ptj_attn_fwd(const void* q, const void* k, const void* v, const uint32_t* ma
     hipStream_t st = (hipStream_t)stream;
     AttnArgs a = {};
     a.q = q; a.k = k; a.v = v; a.out0 = o; a.mask = mask; a.ms = ms; a.ls = ls;
-    a.B = (int)B; a.H = (int)H; a.T = (int)T; a.bitwords = (int)(2 * T / 32 + 2);
+    a.B = (int)B; a.H = (int)H; a.T = (int)T; a.bitwords = (int)ptj_attn_bitwords(T);
     a.q_bs = q_bs; a.q_hs = q_hs; a.q_rs = q_rs; a.k_bs = k_bs; a.k_hs = k_hs; a.k_rs = k_rs;
     a.v_bs = v_bs; a.v_hs = v_hs; a.v_rs = v_rs;
     a.out0_bs = o_bs; a.out0_hs = o_hs; a.out0_rs = o_rs;
@@ -936,12 +1021,10 @@ int ptj_attn_fwd(const void* q, const void* k, const void* v, const uint32_t* ma
         if (!workspace || workspace_bytes < bits_bytes(BH, T))
             return ptj_set_error(PTJ_ERR_WORKSPACE, "attn_fwd: workspace %zu < %zu bytes", workspace_bytes, bits_bytes(BH, T));
         a.keepbits = (const uint32_t*)workspace;
-        rc = launch_keepbits((uint32_t*)workspace, BH, a.bitwords, seed, st);
+        rc = launch_keepbits((uint32_t*)workspace, 1, &seed, 1, BH, a.bitwords, st);
         if (rc) return rc;
     }
-    dim3 grid((unsigned)BH, (unsigned)((T + 127) / 128));
-    if (dtype == PTJ_F32) ATTN_LAUNCH(attn_fwd_kernel, float, grid, st, a);
-    else ATTN_LAUNCH(attn_fwd_kernel, bf16, grid, st, a);
+    launch_fwd(a, dtype, st);
     PTJ_CHECK_LAUNCH();
     return PTJ_OK;
 }
@@ -970,28 +1053,21 @@ int ptj_attn_bwd(const void* d_o, const void* q, const void* k, const void* v, c
     AttnArgs a = {};
     a.q = q; a.k = k; a.v = v; a.o = o; a.d_o = d_o; a.mask = mask;
     a.ms = const_cast<float*>(ms); a.ls = const_cast<float*>(ls); a.delta = delta; a.keepbits = bits;
-    a.B = (int)B; a.H = (int)H; a.T = (int)T; a.bitwords = (int)(2 * T / 32 + 2);
+    a.B = (int)B; a.H = (int)H; a.T = (int)T; a.bitwords = (int)ptj_attn_bitwords(T);
     a.q_bs = q_bs; a.q_hs = q_hs; a.q_rs = q_rs; a.k_bs = k_bs; a.k_hs = k_hs; a.k_rs = k_rs;
     a.v_bs = v_bs; a.v_hs = v_hs; a.v_rs = v_rs; a.o_bs = o_bs; a.o_hs = o_hs; a.o_rs = o_rs;
     a.do_bs = do_bs; a.do_hs = do_hs; a.do_rs = do_rs;
     a.train = train != 0; a.scale = 0.125f;
     if (a.train) {
-        rc = launch_keepbits(bits, BH, a.bitwords, seed, st);
+        rc = launch_keepbits(bits, 1, &seed, 1, BH, a.bitwords, st);
         if (rc) return rc;
     }
-    dim3 grid((unsigned)BH, (unsigned)((T + 127) / 128));
     AttnArgs a1 = a;
     a1.out0 = dk; a1.out0_bs = dk_bs; a1.out0_hs = dk_hs; a1.out0_rs = dk_rs;
     a1.out1 = dv; a1.out1_bs = dv_bs; a1.out1_hs = dv_hs; a1.out1_rs = dv_rs;
     AttnArgs a2 = a;
     a2.out0 = dq; a2.out0_bs = dq_bs; a2.out0_hs = dq_hs; a2.out0_rs = dq_rs;
-    if (dtype == PTJ_F32) {
-        ATTN_LAUNCH(attn_bwd_dq_kernel, float, grid, st, a2);      // also writes delta ...
-        ATTN_LAUNCH(attn_bwd_dkdv_kernel, float, grid, st, a1);    // ... which this pass reads
-    } else {
-        ATTN_LAUNCH(attn_bwd_dq_kernel, bf16, grid, st, a2);
-        ATTN_LAUNCH(attn_bwd_dkdv_kernel, bf16, grid, st, a1);
-    }
+    launch_bwd(a2, a1, dtype, st);
     PTJ_CHECK_LAUNCH();
     return PTJ_OK;
 }

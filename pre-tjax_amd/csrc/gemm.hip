@@ -3,6 +3,25 @@
 #include "gemm_core.h"
 #include "gemm_plan.h"
 
+namespace {
+
+// gemm_plan through a small per-thread table: a training loop asks for the same few dozen products again and again,
+// and the estimate over all tile shapes and splits takes a microsecond.
+GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int persistent_splits) {
+    struct Entry { int64_t n, m, k; size_t ws; int elt, splits, cus; GemmPlan plan; };
+    constexpr int ENTRIES = 128;
+    static thread_local Entry table[ENTRIES] = {};
+    const int cus = num_cus();
+    const uint64_t h = ((uint64_t)n * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)m * 0xC2B2AE3D27D4EB4Full) ^
+                       ((uint64_t)k * 0x165667B19E3779F9ull) ^ ((uint64_t)ws_bytes * 0xD6E8FEB86659FD93ull);
+    Entry& e = table[(h >> 40) % ENTRIES];
+    if (e.n != n || e.m != m || e.k != k || e.ws != ws_bytes || e.elt != elt || e.splits != persistent_splits || e.cus != cus)
+        e = {n, m, k, ws_bytes, elt, persistent_splits, cus, gemm_plan(n, m, k, elt, ws_bytes, persistent_splits, cus)};
+    return e.plan;
+}
+
+}  // namespace
+
 extern "C" {
 
 size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
@@ -12,7 +31,7 @@ size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
     const int s = choose_splits(n, m, k, elt, (size_t)-1);
     int first, ts, tkps;
     size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
-    const GemmPlan plan = gemm_plan(n, m, k, elt, (size_t)-1, s, num_cus());
+    const GemmPlan plan = cached_plan(n, m, k, elt, (size_t)-1, s);
     if (plan.cfg >= 0 && plan.splits > 1 && (size_t)plan.splits * n * m * sizeof(float) > need)
         need = (size_t)plan.splits * n * m * sizeof(float);
     return need;
@@ -52,7 +71,7 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n,
     const int bm = elt == 2 ? pick_mode<bf16>(b, b_cs, b_rs) : pick_mode<float>(b, b_cs, b_rs);
     GemmPlan plan = {-1, 1, 0};
     if (epilogue != PTJ_EPI_ACCUMULATE && gt_eligible(g, am, bm))
-        plan = gemm_plan(n, m, k, elt, workspace && ptj_aligned16(workspace) ? workspace_bytes : 0, splits, num_cus());
+        plan = cached_plan(n, m, k, elt, workspace && ptj_aligned16(workspace) ? workspace_bytes : 0, splits);
     int64_t kps = k;
     if (plan.cfg >= 0) {
         splits = plan.splits;

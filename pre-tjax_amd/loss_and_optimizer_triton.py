@@ -215,33 +215,24 @@ def adam_w_in_place(params, grads, lr, betas, epsilon, moments, i, weight_decay=
     low-precision copies) is refreshed from them."""
     master = params
     t = i + 1
-    ps, ms_, vs, gs, ss, ns, wds = [], [], [], [], [], [], []
-    keep = []                                    # contiguous gradient copies must outlive the launch
-    gdt = sdt = None
-    for gi, grp in enumerate(master):
-        for pi, p in enumerate(grp):
-            g = grads[gi][pi]
-            if not g.is_contiguous():
-                g = g.contiguous()
-                keep.append(g)
-            sh = shadow[gi][pi] if shadow is not None else None
-            assert p.dtype == torch.float32 and p.is_contiguous() and g.numel() == p.numel()
-            assert gdt in (None, g.dtype) and (sh is None or sdt in (None, sh.dtype)), "mixed gradient / shadow dtypes"
-            gdt = g.dtype
-            if sh is not None:
-                sdt = sh.dtype
-            ps.append(p.data_ptr())
-            ms_.append(moments[0][gi][pi].data_ptr())
-            vs.append(moments[1][gi][pi].data_ptr())
-            gs.append(g.data_ptr())
-            ss.append(sh.data_ptr() if sh is not None else 0)
-            ns.append(p.numel())
-            wds.append(weight_decay if (weight_decay_mask is None or weight_decay_mask[gi][pi]) else 0.0)
+    ps = [p for grp in master for p in grp]
+    gs = [g if g.is_contiguous() else g.contiguous() for grp in grads for g in grp]   # copies outlive the launch
+    ms = [m for grp in moments[0] for m in grp]
+    vs = [v for grp in moments[1] for v in grp]
+    ss = [x for grp in shadow for x in grp] if shadow is not None else None
     cnt = len(ps)
     if cnt:
-        arr = lambda vals: (ctypes.c_void_p * cnt)(*vals)
+        ns = [p.numel() for p in ps]
+        assert all(p.dtype == torch.float32 and p.is_contiguous() for p in ps) and ns == [g.numel() for g in gs]
+        gdt, sdt = gs[0].dtype, ss[0].dtype if ss is not None else None
+        assert all(g.dtype == gdt for g in gs) and (ss is None or all(x.dtype == sdt for x in ss)), "mixed gradient / shadow dtypes"
+        if weight_decay_mask is None:
+            wds = [weight_decay] * cnt
+        else:
+            wds = [weight_decay if on else 0.0 for grp in weight_decay_mask for on in grp]
+        arr = lambda tensors: (ctypes.c_void_p * cnt)(*[x.data_ptr() for x in tensors])
         code = {torch.float32: 0, torch.bfloat16: 1}
-        check(lib().ptj_adamw_multi(cnt, arr(ps), arr(ms_), arr(vs), arr(gs), arr(ss) if shadow is not None else None,
+        check(lib().ptj_adamw_multi(cnt, arr(ps), arr(ms), arr(vs), arr(gs), arr(ss) if ss is not None else None,
                                     (ctypes.c_int64 * cnt)(*ns), (ctypes.c_float * cnt)(*wds), lr, betas[0], betas[1],
                                     epsilon, t, code[gdt], code[sdt] if sdt is not None else -1, stream()),
               "ptj_adamw_multi")

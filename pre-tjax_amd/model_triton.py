@@ -6,6 +6,7 @@ Each ``*_t`` function allocates its outputs, passes raw pointers / strides to th
 ABI and returns tensors shaped like the reference's.  Launches are asynchronous on
 torch's current stream; nothing here synchronises.  Inputs are never modified.
 """
+import ctypes
 import math
 
 import torch
@@ -719,8 +720,83 @@ def t_gpt2_tlayer_bkwd3_t(dloss_dx, acts, layer_params, y, mask, train=True, p_g
     return dx_in, grads
 
 
+# ---- the whole stack in one native call (csrc/gpt2.hip) -------------------------------------------
+NATIVE_STACK = True    # False: issue the stack one wrapper call at a time (same kernels, same bits)
+
+
+class _StackActs:
+    """What ptj_gpt2_fwd left for ptj_gpt2_bwd: the activation buffer, the shape record, the packed mask and the seeds."""
+    __slots__ = ("buf", "shape", "mask", "seeds")
+
+
+def _native_params(params):
+    """The parameter nest flattened, if the native stack can take it as it is: blocks present, head size 64, one
+    storage type, every tensor contiguous and on the GPU; else None."""
+    if not NATIVE_STACK or len(params) < 4:
+        return None
+    flat = [p for grp in params for p in grp]
+    dt = flat[0].dtype
+    if dt != torch.bfloat16 and dt != torch.float32:
+        return None
+    if params[2][2].shape[2] != ATTN_DH or len(flat) != 5 + 10 * (len(params) - 3):
+        return None
+    for p in flat:
+        if p.dtype != dt or not p.is_contiguous() or not p.is_cuda:
+            return None
+    return flat
+
+
+def _pointers(tensors):
+    return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
+def _native_fwd(params, flat, y, mask, train, p_gen_aux, keep):
+    """-> (h [B,T,D], x_last [B,T,D], _StackActs)."""
+    require_gpu(y)
+    L = len(params) - 3
+    V, D = flat[0].shape
+    H = params[2][2].shape[0]
+    B, T = y.shape
+    assert flat[2].shape[0] >= T and flat[2].shape[1] == D, "sequence longer than the positional table"
+    dt, dev = flat[0].dtype, flat[0].device
+    acts = _StackActs()
+    acts.mask = _mask_arg(mask, B, T)
+    acts.shape = (ctypes.c_int64 * 9)(L, B, T, D, H, params[2][6].shape[0], V, dtype_code(flat[0]), int(bool(train)))
+    acts.seeds = (ctypes.c_int64 * (1 + 3 * L))(*p_gen_aux) if train else None
+    tok = y.reshape(-1).to(torch.int64).contiguous()
+    nbytes = lib().ptj_gpt2_acts_bytes(acts.shape, int(keep))
+    acts.buf = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    ws_bytes = lib().ptj_gpt2_workspace_bytes(acts.shape, 0)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    x_last = torch.empty((B, T, D), dtype=dt, device=dev)
+    h = torch.empty((B, T, D), dtype=dt, device=dev)
+    check(lib().ptj_gpt2_fwd(acts.shape, _pointers(flat), tok.data_ptr(), ptr(acts.mask), acts.seeds, acts.buf.data_ptr(), nbytes,
+                             int(keep), x_last.data_ptr(), h.data_ptr(), ws.data_ptr(), ws_bytes, stream()), "ptj_gpt2_fwd")
+    return h, x_last, acts
+
+
+def _native_bwd(acts, params, x_last, dh):
+    """-> (gradients of the blocks and the final norm as the nest's groups 2.., demb [N,D])."""
+    require_gpu(dh)
+    groups = [[torch.empty_like(p) for p in grp] for grp in params[2:]]
+    flat = [params[0][0], params[0][1], params[1][0]] + [g for grp in groups for g in grp]   # the first three stay untouched
+    dh = dh.contiguous()
+    demb = torch.empty_like(dh)
+    ws_bytes = lib().ptj_gpt2_workspace_bytes(acts.shape, 1)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dh.device)
+    weights = [p.contiguous() for grp in params for p in grp]
+    check(lib().ptj_gpt2_bwd(acts.shape, _pointers(weights), ptr(acts.mask), acts.seeds,
+                             acts.buf.data_ptr(), acts.buf.numel(), x_last.data_ptr(), dh.data_ptr(), _pointers(flat),
+                             demb.data_ptr(), ws.data_ptr(), ws_bytes, stream()), "ptj_gpt2_bwd")
+    return groups, demb
+
+
 def t_gpt2_tlayers_fwd3_t(params, y, mask, indices, train=True, p_gen_aux=None):
     """model_triton.py:2334-2351.  y int [B,T] -> (h [B,T,D], acts)."""
+    flat = _native_params(params)
+    if flat is not None:
+        h, x, layer_acts = _native_fwd(params, flat, y, mask, train, p_gen_aux, True)
+        return h, [layer_acts, x]
     L = len(params) - 3
     if not train:
         p_gen_aux = [0] * (1 + 3 * L)
@@ -745,15 +821,22 @@ def t_gpt2_forward_with_acts_t(params, y, y_mask, y_indices, train, p_gen_aux=No
     """model_triton.py:2535-2539: -> (logits [B,T,V], acts).  The logits are a view of a
     row-padded buffer (unit column stride)."""
     h, acts = t_gpt2_tlayers_fwd3_t(params, y, y_mask, y_indices, train, p_gen_aux)
+    return _lm_head(params, h), [acts, h]
+
+
+def _lm_head(params, h):
     B, T, D = h.shape
     wemb, bemb = params[0]
     V = wemb.shape[0]
     logits = _padded_logits(B * T, V, h.dtype, h.device)
     matmul_t(h.view(B * T, D), wemb.t(), bemb, out=logits)
-    return logits.view(B, T, V), [acts, h]
+    return logits.view(B, T, V)
 
 
 def t_gpt2_forward_t(params, y, y_mask, y_indices, train, p_gen_aux=None):
+    flat = _native_params(params)
+    if flat is not None:      # no backward follows: one block's activations serve all of them
+        return _lm_head(params, _native_fwd(params, flat, y, y_mask, train, p_gen_aux, False)[0])
     return t_gpt2_forward_with_acts_t(params, y, y_mask, y_indices, train, p_gen_aux)[0]
 
 
@@ -779,17 +862,10 @@ def t_gpt2_bkwd3_p_t(dloss_dx, acts, params, y, y_mask, y_indices, train, p_gen_
     return gpt2_bkwd_below_head_t(dh, dwemb, dbemb, acts, params, y, y_mask, train, p_gen_aux)
 
 
-def gpt2_bkwd_below_head_t(dh, dwemb, dbemb, acts, params, y, y_mask, train, p_gen_aux=None):
-    """t_gpt2_bkwd3_p_t from the gradient of the final LayerNorm's output on (model_triton.py:2583-2593
-    after the LM head's own three products): `dh` [N,D] = dlogits @ Wemb, `dwemb` [V,D] = the head's
-    weight gradient (the embedding's is added onto it), `dbemb` [V] its bias gradient."""
+def _bkwd_stack(dh, layer_acts, x_last, params, y_mask, train, p_gen_aux):
+    """The stack's backward one wrapper call at a time: -> (demb [N,D], per-block gradients, final gain and shift)."""
     L = len(params) - 3
-    if not train:
-        p_gen_aux = [0] * (1 + 3 * L)
-    (layer_acts, x_last), _ = acts
-    D = dh.shape[1]
-    B, T = y.shape
-    N = B * T
+    N, D = dh.shape
     # Every dropout backward acts on a gradient that a LayerNorm backward has just produced,
     # so each LayerNorm backward also writes the dropped copy its consumer needs: the final
     # norm for the last block's FFN dropout (seed 3L), block i's first norm for block i-1's
@@ -811,7 +887,25 @@ def gpt2_bkwd_below_head_t(dh, dwemb, dbemb, acts, params, y, y_mask, train, p_g
                                     drop_out_sum=i > 0)
         dx, layer_grads[i], dropped = res[:3]
         dsum = res[3] if i > 0 else None
-    d = dropped                                                         # [N,D] = dropout_bkwd(dx, seed 0)
+    return dropped, layer_grads, dlnfg, dlnfb                           # dropped [N,D] = dropout_bkwd(dx, seed 0)
+
+
+def gpt2_bkwd_below_head_t(dh, dwemb, dbemb, acts, params, y, y_mask, train, p_gen_aux=None):
+    """t_gpt2_bkwd3_p_t from the gradient of the final LayerNorm's output on (model_triton.py:2583-2593
+    after the LM head's own three products): `dh` [N,D] = dlogits @ Wemb, `dwemb` [V,D] = the head's
+    weight gradient (the embedding's is added onto it), `dbemb` [V] its bias gradient."""
+    L = len(params) - 3
+    if not train:
+        p_gen_aux = [0] * (1 + 3 * L)
+    (layer_acts, x_last), _ = acts
+    D = dh.shape[1]
+    B, T = y.shape
+    N = B * T
+    if isinstance(layer_acts, _StackActs):
+        groups, d = _native_bwd(layer_acts, params, x_last, dh)
+        layer_grads, (dlnfg, dlnfb) = groups[:-1], groups[-1]
+    else:
+        d, layer_grads, dlnfg, dlnfb = _bkwd_stack(dh, layer_acts, x_last, params, y_mask, train, p_gen_aux)
     # positional table: sum over the batch (model_triton.py:2518 with indices = arange(T))
     table_rows = params[1][0].shape[0]
     dpos = torch.empty_like(params[1][0])

@@ -1,0 +1,49 @@
+"""The transformer stack issued by one native call per direction against the same launches issued one
+wrapper call at a time: bit-equal losses and gradients, with and without dropout, with and without a
+mask tensor, in both storage types, and the forward that keeps no activations."""
+import pytest
+import torch
+
+from oracle import gpt2 as ogpt2
+from util import DTYPES
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("L,B,T,masked", [(1, 1, 64, True), (3, 2, 192, False)])
+def test_native_stack_is_bit_equal(mt, lo, monkeypatch, dtype, train, L, B, T, masked):
+    V, D, H, F = 203, 128, 2, 256
+    params = [[p.to(DEV).to(dtype) for p in grp] for grp in ogpt2.init_transformer_gpt2(V, D, L, H, F, T + 5, seed=3)]
+    g = torch.Generator().manual_seed(4)
+    y = torch.randint(0, V, (B, T + 1), generator=g).to(DEV)
+    mask = torch.tril(torch.ones(T, T, dtype=torch.bool)).expand(B, T, T).clone()
+    mask[-1, :, T - 9:] = False
+    mask = mask.to(DEV) if masked else None
+    seeds = list(range(100, 101 + 3 * L))
+    runs = []
+    for native in (True, False):
+        monkeypatch.setattr(mt, "NATIVE_STACK", native)
+        grads, (loss, acc, frac) = lo.t_loss_bkwd3_t(params, y, mask, None, train, seeds)
+        logits = mt.t_gpt2_forward_t(params, y[:, :-1], mask, None, train, seeds)
+        runs.append([loss, acc, logits] + [p for grp in grads for p in grp])
+    assert len(runs[0]) == 3 + 5 + 10 * L
+    for a, b in zip(*runs):
+        assert a.shape == b.shape and torch.equal(a, b)
+
+
+def test_native_stack_steps_aside(mt, lo):
+    """A parameter that is not contiguous takes the call-by-call path and gives the same result."""
+    V, D, L, H, F, T, B = 101, 128, 2, 2, 256, 64, 1
+    params = [[p.to(DEV) for p in grp] for grp in ogpt2.init_transformer_gpt2(V, D, L, H, F, T, seed=3)]
+    y = torch.randint(0, V, (B, T + 1), generator=torch.Generator().manual_seed(5)).to(DEV)
+    seeds = list(range(10, 11 + 3 * L))
+    want, _ = lo.t_loss_bkwd3_t(params, y, None, None, True, seeds)
+    odd = [list(grp) for grp in params]
+    odd[2][3] = params[2][3].t().contiguous().t()
+    got, _ = lo.t_loss_bkwd3_t(odd, y, None, None, True, seeds)
+    for wg, gg in zip(want, got):
+        for a, b in zip(wg, gg):
+            assert (a - b).norm() <= 1e-5 * a.norm()
