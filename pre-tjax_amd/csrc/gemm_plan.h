@@ -24,8 +24,8 @@ struct TileCost {
 };
 
 // bf16 / fp32; the index is the configuration number of gemm_tile_launch
-constexpr int GT_CONFIGS = 7;
-constexpr TileCost GT_COST[2][GT_CONFIGS] = {
+constexpr int GT_CONFIGS[2] = {7, 6};
+constexpr TileCost GT_COST[2][7] = {
     {{32, 32, 256, 1, 2.03, 0.522, 1.24, 1.0},
      {64, 64, 128, 1, 2.49, 0.372, 1.81, 1.0},
      {64, 128, 64, 2, 3.49, 0.299, 1.21, 1.89},
@@ -33,13 +33,13 @@ constexpr TileCost GT_COST[2][GT_CONFIGS] = {
      {128, 128, 64, 2, 2.73, 0.714, 1.88, 1.39},
      {128, 192, 64, 2, 2.45, 0.922, 5.00, 1.50},
      {256, 192, 64, 1, 2.00, 1.250, 8.00, 1.0}},
-    {{32, 32, 128, 1, 2.84, 0.684, 1.69, 1.0},
-     {64, 64, 64, 1, 3.05, 1.091, 2.52, 1.0},
-     {64, 64, 64, 2, 2.85, 1.370, 2.15, 1.47},
-     {64, 128, 32, 2, 4.85, 1.047, 1.75, 1.86},
-     {128, 128, 32, 2, 3.06, 2.036, 2.59, 1.83},
-     {128, 96, 64, 1, 4.62, 3.027, 3.34, 1.27},
-     {128, 192, 32, 2, 2.44, 2.985, 6.70, 1.84}},
+    // fp32: the last two multiply on the bf16 pipe (gemm_split.h)
+    {{32, 32, 128, 1, 3.25, 0.663, 1.67, 1.0},
+     {64, 64, 64, 1, 3.56, 1.077, 2.37, 1.0},
+     {64, 64, 64, 2, 4.16, 1.326, 1.45, 1.51},
+     {64, 128, 32, 2, 6.44, 1.035, 0.56, 1.88},
+     {128, 128, 32, 1, 3.10, 1.218, 3.22, 1.0},
+     {64, 64, 32, 2, 5.87, 0.640, 0.00, 1.32}},
 };
 
 struct GemmPlan {
@@ -55,28 +55,29 @@ inline double gp_reduce_us(int64_t n, int64_t m, int splits) {
     return splits > 1 ? 2.6 + 0.35e-6 * 4.0 * (double)splits * (double)n * (double)m : 0.0;
 }
 
-inline double gp_tile_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int splits, int cus) {
+inline double gp_tile_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int elt, int splits, int cus) {
     const int64_t work = gp_ceil(n, c.tbm) * gp_ceil(m, c.tbn) * splits;
     const int64_t steps = gp_ceil(gp_ceil(k, splits), c.bkt);
     const int64_t slots = (int64_t)cus * c.per_cu, full = work / slots, rem = work % slots;
     double t = c.start + (double)full * ((double)steps * c.step * c.shared + c.finish);
     if (rem) t += (double)steps * c.step * (rem > cus ? c.shared : 1.0) + c.finish;
-    // a chip that stays full over several rounds shares the path from L2: measured 10 % at 1.5 rounds, 30 % at many
+    // bf16: a chip that stays full over several rounds shares the path from L2: measured 10 % at 1.5 rounds, 30 % at many
     const double rounds = (double)work / (double)slots;
-    if (rounds > 1.0) t *= 1.0 + 0.3 * (1.0 - 1.0 / rounds);
+    if (elt == 2 && rounds > 1.0) t *= 1.0 + 0.3 * (1.0 - 1.0 / rounds);
     return t + gp_reduce_us(n, m, splits);
 }
 
-// The persistent kernels: 20 us (fp32: 135 us) per round of 256x192 tiles at k = 768; a partial panel along K goes
-// through the element-wise loader.
+// The persistent bf16 kernels: 20 us per round of 256x192 tiles at k = 768; a partial panel along K goes through the
+// element-wise loader.  In fp32 they are never the fastest (158 us against 120 for 4096x3072x768) and serve only operands
+// that the tile kernels do not take.
 inline double gp_persistent_us(int64_t n, int64_t m, int64_t k, int elt, int splits, int cus) {
-    const int bk = 128 / elt;
-    const int64_t work = gp_ceil(n, 256) * gp_ceil(m, 192) * splits, steps = gp_ceil(gp_ceil(k, splits), bk);
+    if (elt != 2) return 1e30;
+    const int64_t work = gp_ceil(n, 256) * gp_ceil(m, 192) * splits, steps = gp_ceil(gp_ceil(k, splits), 64);
     const int64_t full = work / cus, rem = work % cus;
     const double rounds = (double)full + (rem ? 0.35 + 0.65 * (double)rem / cus : 0.0);
-    double t = elt == 2 ? 7.0 + rounds * (1.2 * (double)steps + 4.3) : 12.0 + rounds * (5.3 * (double)steps + 7.0);
-    if (n % 256 != 0 || m % 192 != 0) t += elt == 2 ? 8.0 : 4.0;
-    if (k % bk != 0) t += elt == 2 ? 20.0 : 30.0;
+    double t = 7.0 + rounds * (1.2 * (double)steps + 4.3);
+    if (n % 256 != 0 || m % 192 != 0) t += 8.0;
+    if (k % 64 != 0) t += 20.0;
     return t + gp_reduce_us(n, m, splits);
 }
 
@@ -87,13 +88,14 @@ inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_by
     GemmPlan best = {-1, 1, (int)k};
     // within 8 % the persistent kernels are kept: in a training step their loads run on from product to product
     double best_us = 0.92 * gp_persistent_us(n, m, k, elt, persistent_splits, cus);
-    for (int i = 0; i < GT_CONFIGS; ++i) {
-        const TileCost& c = GT_COST[elt == 2 ? 0 : 1][i];
+    const int type = elt == 2 ? 0 : 1;
+    for (int i = 0; i < GT_CONFIGS[type]; ++i) {
+        const TileCost& c = GT_COST[type][i];
         for (int s = 1; s <= 16; ++s) {
             if (s > 1 && (k < 1024 || k / s < 256 || (size_t)s * (size_t)n * (size_t)m * sizeof(float) > ws_bytes)) break;
             const int64_t kps = gp_ceil(gp_ceil(k, s), c.bkt) * c.bkt;
             if (s > 1 && gp_ceil(k, kps) != s) continue;
-            const double us = gp_tile_us(c, n, m, k, s, cus);
+            const double us = gp_tile_us(c, n, m, k, elt, s, cus);
             if (us < best_us) {
                 best_us = us;
                 best = {i, s, (int)(s > 1 ? kps : k)};

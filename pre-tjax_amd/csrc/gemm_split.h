@@ -1,0 +1,277 @@
+// fp32 GEMM on the bf16 matrix pipe.  Included by gemm_tile_launch.h inside its unnamed namespace.
+//
+// Every fp32 value is the exact sum of three bf16 values h + m + l (each the round-to-nearest of what is left: 8 + 8 + 8
+// significant bits and two signs cover the 24), so a product of two is the sum of nine products of bf16 values, all
+// exact in the fp32 accumulator.  Six of them are formed (hh, hm, mh, hl, lh, mm); the other three together are below
+// 2^-26 |a b|, a quarter of the rounding that the fp32 multiply-add they stand in for makes.  Sixteen products enter the
+// accumulator per rounding instead of two.  Measured against fp64 at k = 768: rms 5.7e-9 of sum |a b| for N(0,1) operands
+// and 7.2e-8 for positive ones, where the fp32 matrix instructions leave 1.4e-8 and 1.0e-7 (tests/test_gpu_gemm_split.py
+// holds the order).  Six v_mfma_f32_32x32x16_bf16 take 192 clocks where eight
+// v_mfma_f32_32x32x2_f32 take 512.  Non-finite inputs: NaN stays NaN, an infinity gives NaN (inf - inf in the split)
+// where the fp32 instruction would give an infinity; parts of values below 2^-110 underflow.
+//
+// 4096x3072x768: 120 us, 155-163 on the fp32 instructions.
+//
+// Panels travel HBM -> registers as fp32, two steps ahead, are split once per workgroup and stored as three bf16 planes
+// (the conversion costs 5.5 vector instructions per element, spread between the MFMAs), 32 contraction elements per
+// step, double-buffered in LDS.  KMAJOR operands: [row][64 bytes], 16-byte chunks XOR-swizzled; MNMAJOR: [k][rows], read
+// through ds_read_b64_tr_b16.  Border handling (buffer descriptors) and write-back are those of gemm_tile.h.
+typedef float gs_f32x2 __attribute__((ext_vector_type(2)));
+typedef short gs_i16x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ uint32_t gs_pk(float a, float b) {
+    const gs_f32x2 f = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+}
+// two values -> their h, m and l parts, packed
+__device__ __forceinline__ void gs_split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = gs_pk(x0, x1);
+    const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
+    m = gs_pk(r0, r1);
+    l = gs_pk(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xffff0000u));
+}
+
+template <int MODE, int ROWS, int NT, int NTHREADS>
+struct GsOperand {
+    static constexpr int BK = 32, VEC = 4;
+    static constexpr int PLANE = ROWS * BK * 2;                 // bytes of one bf16 plane
+    static constexpr int PER = ROWS * BK / VEC / NTHREADS;      // float4 loads per thread and step
+    static constexpr int PITCH = ROWS * 2;                      // MNMAJOR: bytes per k-row of a plane
+    static_assert(PER * NTHREADS * VEC == ROWS * BK, "loads divide evenly among the threads");
+    uint32_t voff[PER];
+    uint32_t loff[PER];                                         // LDS offset inside a plane
+    const char* base;
+    int64_t left, step;
+    gt_u32x4 r[2][PER];                                         // two steps in flight
+
+    __device__ __forceinline__ void init(const void* p, int64_t s_row, int64_t s_k, int row0, int nrows, int kbeg, int k, int tid) {
+        const float* first = (const float*)p + (MODE == KMAJOR ? (int64_t)row0 * s_row + kbeg : (int64_t)kbeg * s_k + row0);
+        base = (const char*)first;
+        left = 4 * (MODE == KMAJOR ? (int64_t)(nrows - 1 - row0) * s_row + ((k - kbeg + 3) / 4) * 4
+                                   : (int64_t)(k - 1 - kbeg) * s_k + ((nrows - row0 + 3) / 4) * 4);
+        step = (MODE == KMAJOR ? (int64_t)1 : s_k) * BK * 4;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int v = i * NTHREADS + tid;
+            if constexpr (MODE == KMAJOR) {
+                const int row = v >> 3, g = v & 7;              // group of four k
+                voff[i] = ((uint32_t)row * (uint32_t)s_row + (uint32_t)g * 4u) * 4u;
+                loff[i] = row * 64 + (((g >> 1) ^ ((row >> 2) & 3)) << 4) + (g & 1) * 8;
+            } else {
+                constexpr int VPR = ROWS / 4;                   // vectors per k-row
+                const int kk = v / VPR, rv = v - kk * VPR;
+                voff[i] = ((uint32_t)kk * (uint32_t)s_k + (uint32_t)rv * 4u) * 4u;
+                loff[i] = kk * PITCH + (((rv >> 1) ^ gt_mn_swz<ROWS>(kk)) << 4) + (rv & 1) * 8;
+            }
+        }
+    }
+
+    // Requests the next step's values into register set SET.  kleft: contraction elements from its first one to the end.
+    template <int SET>
+    __device__ __forceinline__ void load(int kleft, int tid) {
+        const uint32_t records = kleft <= 0 ? 0u : (uint32_t)(left < 0xFFFFFF00ll ? left : 0xFFFFFF00ll);
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, records, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            uint32_t v = voff[i];
+            if constexpr (MODE == KMAJOR) {
+                v = ((i * NTHREADS + tid) & 7) * 4 < kleft ? v : 0xFFFFFFF0u;
+            }
+            r[SET][i] = __builtin_bit_cast(gt_u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, v, 0, 0));
+        }
+        base += step;
+        left -= step;
+    }
+
+    // Splits vector I of register set SET and stores its parts into the planes at `lds`.  CLEAR: the step ends inside a
+    // vector of a KMAJOR row; its elements past kleft (the next row's, or padding) count as zero.
+    template <int SET, int I, bool CLEAR>
+    __device__ __forceinline__ void split_store(char* __restrict__ lds, int kleft, int tid) const {
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = __uint_as_float(r[SET][I][e]);
+        if constexpr (MODE == KMAJOR && CLEAR) {
+            const int k0 = ((I * NTHREADS + tid) & 7) * 4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = k0 + e < kleft ? x[e] : 0.f;
+        }
+        gt_u32x2 h, m, l;
+        uint32_t a, b, c;
+        gs_split2(x[0], x[1], a, b, c);
+        h[0] = a; m[0] = b; l[0] = c;
+        gs_split2(x[2], x[3], a, b, c);
+        h[1] = a; m[1] = b; l[1] = c;
+        *reinterpret_cast<gt_u32x2*>(lds + loff[I]) = h;
+        *reinterpret_cast<gt_u32x2*>(lds + PLANE + loff[I]) = m;
+        *reinterpret_cast<gt_u32x2*>(lds + 2 * PLANE + loff[I]) = l;
+    }
+
+    // Part `plane` of the fragment of MFMA tile t (rows wrow + 32 t ...), contraction chunk c of the step
+    __device__ __forceinline__ static bf16x8 frag(const char* __restrict__ lds, int plane, int wrow, int t, int c, int lane) {
+        if constexpr (MODE == KMAJOR) {
+            const int row = wrow + t * 32 + (lane & 31), ch = c * 2 + (lane >> 5);
+            return *reinterpret_cast<const bf16x8*>(lds + plane * PLANE + row * 64 + ((ch ^ ((row >> 2) & 3)) << 4));
+        } else {
+            const int l16 = lane & 15, mhalf = (lane >> 4) & 1, lg = lane >> 5, kq = l16 >> 2;
+            const int piece = (wrow >> 3) + t * 4 + 2 * mhalf + ((l16 & 3) >> 1);
+            const char* p = lds + plane * PLANE + (16 * c + 8 * lg + kq) * PITCH + ((piece ^ gt_mn_swz<ROWS>(kq)) << 4) + 8 * (l16 & 1);
+            const gs_i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) gs_i16x4*)(p));
+            const gs_i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) gs_i16x4*)(p + 4 * PITCH));
+            return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    }
+};
+
+template <int TBM_, int TBN_, int WM_, int WN_>
+struct GsCfg {
+    static constexpr int TBM = TBM_, TBN = TBN_, WM = WM_, WN = WN_, KG = 1;
+    static constexpr int NW = WM * WN, THREADS = NW * 64;
+    static constexpr int TMW = TBM / WM / 32, TNW = TBN / WN / 32;
+    static_assert(TMW * WM * 32 == TBM && TNW * WN * 32 == TBN, "whole MFMA tiles per wavefront");
+    static constexpr int CW = TNW * 32;
+    static constexpr int STAGE = 3 * (TBM + TBN) * 64;               // planes of one step
+    static constexpr int OUT_PITCH = CW + 4, OUT_WAVE = 32 * OUT_PITCH * 4;
+    static constexpr int SMEM = 2 * STAGE > NW * OUT_WAVE ? 2 * STAGE : NW * OUT_WAVE;
+    static constexpr int BLOCKS = SMEM > 81920 ? 1 : 2;
+    static constexpr int WAVES_EU = (BLOCKS * NW + 3) / 4;
+};
+
+template <int AMODE, int BMODE, typename C, bool MUL>
+__global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(const GemmArgs g) {
+    constexpr int BK = 32, TMW = C::TMW, TNW = C::TNW;
+    __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / C::WN, wn = wave - wm * C::WN;
+    const int num_m = (g.n + C::TBM - 1) / C::TBM, num_n = (g.m + C::TBN - 1) / C::TBN;
+    int tile_m, tile_n, z;
+    gt_item(g, blockIdx.x, num_m, num_n, tile_m, tile_n, z);
+    const int row0 = tile_m * C::TBM, col0 = tile_n * C::TBN;
+    const int kbeg = z * g.k_per_split;
+    const int kend = g.splits > 1 && kbeg + g.k_per_split < g.k ? kbeg + g.k_per_split : g.k;
+    const int klen = kend - kbeg, nk = (klen + BK - 1) / BK;
+
+    typedef GsOperand<AMODE, C::TBM, TMW, C::THREADS> OA;
+    typedef GsOperand<BMODE, C::TBN, TNW, C::THREADS> OB;
+    OA oa;
+    OB ob;
+    oa.init(g.a, g.a_row, g.a_k, row0, g.n, kbeg, g.k, tid);
+    ob.init(g.b, g.b_row, g.b_k, col0, g.m, kbeg, g.k, tid);
+    constexpr int NV = OA::PER + OB::PER;                            // vectors per thread and step
+    char* const sA = smem;
+    char* const sB = smem + 3 * OA::PLANE;                           // behind the A planes of the same stage
+
+    // The matrix pipe rounds its accumulator once per instruction, more coarsely than a vector add: the products of the
+    // leading parts are summed over one step (part) and added to acc by the vector ALU, and the five small terms are
+    // kept out of the sum that is large (low).
+    f32x16 acc[TNW][TMW], part[TNW][TMW], low[TNW][TMW];
+#pragma unroll
+    for (int i = 0; i < TNW; ++i)
+#pragma unroll
+        for (int j = 0; j < TMW; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) { acc[i][j][e] = 0.f; low[i][j][e] = 0.f; }
+
+    const bool ragged = klen % 4 != 0 && (AMODE == KMAJOR || BMODE == KMAJOR);
+    auto split_piece = [&](auto set, auto i, auto clear, int buf, int kleft) {
+        if constexpr (i < OA::PER) oa.template split_store<set, i, clear>(sA + buf * C::STAGE, kleft, tid);
+        else ob.template split_store<set, i - OA::PER, clear>(sB + buf * C::STAGE, kleft, tid);
+    };
+    // One contraction chunk (16 wide) of stage `buf`: six products per MFMA tile; with `split` the vectors [v0, v1) of
+    // register set `set` are converted into the other stage between them.
+    auto chunk = [&](auto c, auto buf, auto set, auto v0, auto v1) {
+        bf16x8 fa[3][TMW], fb[3][TNW];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+#pragma unroll
+            for (int t = 0; t < TMW; ++t) fa[p][t] = OA::frag(sA + buf * C::STAGE, p, wm * TMW * 32, t, c, lane);
+#pragma unroll
+            for (int t = 0; t < TNW; ++t) fb[p][t] = OB::frag(sB + buf * C::STAGE, p, wn * TNW * 32, t, c, lane);
+        }
+        constexpr int PA[6] = {0, 2, 0, 1, 1, 0}, PB[6] = {0, 0, 2, 1, 0, 1};
+        gt_unroll<0, 6>([&](auto term) {
+#pragma unroll
+            for (int tn = 0; tn < TNW; ++tn)
+#pragma unroll
+                for (int tm = 0; tm < TMW; ++tm) {
+                    const bf16x8 b = fb[PB[term]][tn], a = fa[PA[term]][tm];
+                    if constexpr (term == 0) {
+                        f32x16 zero;
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) zero[e] = 0.f;
+                        part[tn][tm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, c == 0 ? zero : part[tn][tm], 0, 0, 0);
+                    } else {
+                        low[tn][tm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, low[tn][tm], 0, 0, 0);
+                    }
+                    if constexpr (c == 1 && term == 4) {
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[tn][tm][e] += part[tn][tm][e];
+                    }
+                }
+            constexpr int nv = v1 - v0;
+            if constexpr (nv > 0)
+                gt_unroll<v0 + term * nv / 6, v0 + (term + 1) * nv / 6>(
+                    [&](auto i) { split_piece(set, i, std::false_type{}, 1 - buf, 0); });
+        });
+    };
+    auto load = [&](auto set, int kleft) {
+        oa.template load<set>(kleft, tid);
+        ob.template load<set>(kleft, tid);
+    };
+    constexpr std::integral_constant<int, 0> I0{};
+    constexpr std::integral_constant<int, 1> I1{};
+    constexpr std::integral_constant<int, (NV + 1) / 2> IH{};
+    constexpr std::integral_constant<int, NV> IN{};
+    // Step kt (stage kt & 1) while the values of step kt + 1 (register set (kt + 1) & 1) are split into the other stage;
+    // the set is then refilled with step kt + 3.
+    auto step = [&](auto par, int kt) {
+        constexpr std::integral_constant<int, 1 - par> NEXT{};
+        const int l1 = klen - (kt + 1) * BK;
+        if (ragged && l1 > 0 && l1 < BK) {
+            chunk(I0, par, NEXT, I0, I0);
+            chunk(I1, par, NEXT, I0, I0);
+            gt_unroll<0, NV>([&](auto i) { split_piece(NEXT, i, std::true_type{}, NEXT, l1); });
+        } else {
+            chunk(I0, par, NEXT, I0, IH);
+            chunk(I1, par, NEXT, IH, IN);
+        }
+        load(NEXT, klen - (kt + 3) * BK);
+        __syncthreads();
+    };
+    if (nk > 0) {
+        load(I0, klen);
+        load(I1, klen - BK);
+        gt_unroll<0, NV>([&](auto i) { split_piece(I0, i, std::true_type{}, 0, klen); });
+        load(I0, klen - 2 * BK);
+        __syncthreads();
+        for (int kt = 0; kt < nk; kt += 2) {
+            step(I0, kt);
+            if (kt + 1 >= nk) break;
+            step(I1, kt + 1);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TNW; ++i)
+#pragma unroll
+        for (int j = 0; j < TMW; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] += low[i][j][e];
+    __syncthreads();
+    gt_write_back<float, C, MUL>(g, acc, smem, row0, col0, z, wave, lane);
+}
+
+template <typename C, bool MUL>
+int gs_launch(const GemmArgs& g, int am, int bm, hipStream_t st) {
+    const int64_t work = (int64_t)((g.n + C::TBM - 1) / C::TBM) * ((g.m + C::TBN - 1) / C::TBN) * g.splits;
+    const dim3 grid((unsigned)work), block(C::THREADS);
+#define GS_LAUNCH(AM, BMD) hipLaunchKernelGGL((gemm_split_kernel<AM, BMD, C, MUL>), grid, block, 0, st, g)
+    switch (am * 3 + bm) {
+        case 0: GS_LAUNCH(KMAJOR, KMAJOR); break;
+        case 1: GS_LAUNCH(KMAJOR, MNMAJOR); break;
+        case 3: GS_LAUNCH(MNMAJOR, KMAJOR); break;
+        default: GS_LAUNCH(MNMAJOR, MNMAJOR); break;
+    }
+#undef GS_LAUNCH
+    PTJ_CHECK_LAUNCH();
+    return PTJ_OK;
+}

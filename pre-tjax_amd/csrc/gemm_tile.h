@@ -223,6 +223,162 @@ __device__ __forceinline__ void gt_item(const GemmArgs& g, int pid, int num_m, i
     tile_n = (idx % width) / gsz;
 }
 
+// Write-back of a finished tile: 32 rows at a time through an fp32 staging area per wavefront (the K groups'
+// accumulators are added in group order on the way), then rows of 16-byte vectors with the epilogue applied.
+// acc[tn][tm][i] of lane (lr, lg) is C[row0 + (wm * TMW + tm) * 32 + lr][col0 + wn * CW + tn * 32 + (i/4)*8 + lg*4 + i%4].
+template <typename T, typename C, bool MUL>
+__device__ __forceinline__ void gt_write_back(const GemmArgs& g, const f32x16 (&acc)[C::TNW][C::TMW], char* __restrict__ smem,
+                                              int row0, int col0, int z, int wave, int lane) {
+    constexpr int VEC = 16 / (int)sizeof(T), TMW = C::TMW, TNW = C::TNW, KG = C::KG;
+    const int kg = wave / (C::WM * C::WN), wpos = wave - kg * (C::WM * C::WN);
+    const int wm = wpos / C::WN, wn = wpos - wm * C::WN;
+    float* const st = (float*)(smem + wave * C::OUT_WAVE);
+    constexpr int GROUP_STEP = C::WM * C::WN * C::OUT_WAVE / 4;      // staging areas of the K groups of one position
+    const float* const st0 = (const float*)(smem + wpos * C::OUT_WAVE);
+    constexpr int LPR = C::CW / VEC;                                 // vectors per row
+    constexpr int ROWS = 32 / KG;                                    // rows of a pass that this wavefront writes
+    const int lr = lane & 31, lg = lane >> 5;
+    const int gc0 = col0 + wn * C::CW;
+    const bool partial = !MUL && g.splits > 1;
+    float* const part = partial ? g.partial + (int64_t)z * g.n * (int64_t)g.m : nullptr;
+    float csum[(C::CW + 63) / 64];
+#pragma unroll
+    for (int i = 0; i < (C::CW + 63) / 64; ++i) csum[i] = 0.f;
+#pragma unroll
+    for (int tm = 0; tm < TMW; ++tm) {
+#pragma unroll
+        for (int tn = 0; tn < TNW; ++tn)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<f32x4*>(st + lr * C::OUT_PITCH + tn * 32 + q * 8 + lg * 4) =
+                    f32x4{acc[tn][tm][q * 4], acc[tn][tm][q * 4 + 1], acc[tn][tm][q * 4 + 2], acc[tn][tm][q * 4 + 3]};
+        if constexpr (KG > 1) __syncthreads();
+        else __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        const int gr0 = row0 + (wm * TMW + tm) * 32;
+        for (int idx = lane; idx < ROWS * LPR; idx += 64) {
+            const int r = kg * ROWS + idx / LPR, c = (idx % LPR) * VEC;
+            float v[VEC];
+#pragma unroll
+            for (int h = 0; h < VEC / 4; ++h) {
+                f32x4 s = *reinterpret_cast<const f32x4*>(st0 + r * C::OUT_PITCH + c + h * 4);
+#pragma unroll
+                for (int k2 = 1; k2 < KG; ++k2)
+                    s += *reinterpret_cast<const f32x4*>(st0 + k2 * GROUP_STEP + r * C::OUT_PITCH + c + h * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[h * 4 + e] = s[e];
+            }
+            const int row = gr0 + r, col = gc0 + c;
+            const bool inside = row < g.n && col < g.m;
+            const bool whole = g.vec_out && col + VEC <= g.m;
+            const int ne = g.m - col < VEC ? g.m - col : VEC;
+            if constexpr (MUL) {
+                const T* mp = (const T*)g.mul + (int64_t)row * g.mul_rs + col;
+                T* p = (T*)g.c + (int64_t)row * g.c_rs + col;
+                float o[VEC];
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) o[e] = 0.f;
+                if (inside && whole) {
+                    const Pack<T, VEC> mv = *reinterpret_cast<const Pack<T, VEC>*>(mp);
+                    Pack<T, VEC> s;
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {
+                        s.v[e] = from_f32<T>(to_f32(from_f32<T>(v[e])) * to_f32(mv.v[e]));
+                        o[e] = to_f32(s.v[e]);
+                    }
+                    *reinterpret_cast<Pack<T, VEC>*>(p) = s;
+                } else if (inside) {
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e)
+                        if (e < ne) {
+                            const T s = from_f32<T>(to_f32(from_f32<T>(v[e])) * to_f32(mp[e]));
+                            p[e] = s;
+                            o[e] = to_f32(s);
+                        }
+                }
+                // the stored values take the place of the first group's, for the column sums
+#pragma unroll
+                for (int h = 0; h < VEC / 4; ++h)
+                    *reinterpret_cast<f32x4*>(const_cast<float*>(st0) + r * C::OUT_PITCH + c + h * 4) =
+                        f32x4{o[h * 4], o[h * 4 + 1], o[h * 4 + 2], o[h * 4 + 3]};
+            } else if (inside) {
+                if (partial) {
+                    float* p = part + (int64_t)row * g.m + col;
+                    if (whole) {
+#pragma unroll
+                        for (int h = 0; h < VEC / 4; ++h)
+                            *reinterpret_cast<f32x4*>(p + h * 4) = f32x4{v[h * 4], v[h * 4 + 1], v[h * 4 + 2], v[h * 4 + 3]};
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < VEC; ++e)
+                            if (e < ne) p[e] = v[e];
+                    }
+                } else {
+                    const bool deriv = g.epilogue == PTJ_EPI_BIAS_GELU_DERIV;
+                    const bool act = deriv || g.epilogue == PTJ_EPI_BIAS_GELU;
+                    T* p = (T*)g.c + (int64_t)row * g.c_rs + col;
+                    T* pa = g.c_aux != nullptr ? (T*)g.c_aux + (int64_t)row * g.c_aux_rs + col : nullptr;
+                    const T* add = g.epilogue == PTJ_EPI_ACCUMULATE ? p : g.epilogue != PTJ_EPI_NONE ? (const T*)g.bias + col : nullptr;
+                    if (whole) {
+                        if (add != nullptr) {
+                            const Pack<T, 4> b0 = *reinterpret_cast<const Pack<T, 4>*>(add);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) v[e] += to_f32(b0.v[e]);
+                            if constexpr (VEC == 8) {
+                                const Pack<T, 4> b1 = *reinterpret_cast<const Pack<T, 4>*>(add + 4);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) v[4 + e] += to_f32(b1.v[e]);
+                            }
+                        }
+                        if (pa != nullptr) {
+                            float o[VEC];
+#pragma unroll
+                            for (int e = 0; e < VEC; ++e) o[e] = deriv ? gelu_grad_f(v[e]) : v[e];
+                            store_vec<T, VEC>(pa, o);
+                        }
+                        if (act) {
+#pragma unroll
+                            for (int e = 0; e < VEC; ++e) v[e] = gelu_f(v[e]);
+                        }
+                        store_vec<T, VEC>(p, v);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < VEC; ++e)
+                            if (e < ne) {
+                                float x = v[e];
+                                if (add != nullptr) x += to_f32(add[e]);
+                                if (pa != nullptr) pa[e] = from_f32<T>(deriv ? gelu_grad_f(x) : x);
+                                p[e] = from_f32<T>(act ? gelu_f(x) : x);
+                            }
+                    }
+                }
+            }
+        }
+        if constexpr (MUL) {
+            if constexpr (KG > 1) __syncthreads();
+            else __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            if (kg == 0) {
+#pragma unroll
+                for (int i = 0; i < (C::CW + 63) / 64; ++i)
+                    if (i * 64 + lane < C::CW)
+                        for (int r = 0; r < 32; ++r) csum[i] += st0[r * C::OUT_PITCH + i * 64 + lane];
+            }
+        }
+        if constexpr (KG > 1) __syncthreads();
+        else __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
+    if constexpr (MUL) {
+        // one row of sums per wavefront's block of rows (TMW * 32 of them)
+        const int gr = row0 + wm * TMW * 32;
+        if (kg == 0 && gr < g.n) {
+#pragma unroll
+            for (int i = 0; i < (C::CW + 63) / 64; ++i) {
+                const int c = i * 64 + lane;
+                if (c < C::CW && gc0 + c < g.m) g.colpart[(int64_t)(gr / (TMW * 32)) * g.m + gc0 + c] = csum[i];
+            }
+        }
+    }
+}
+
 template <typename T, int AMODE, int BMODE, typename C, bool MUL>
 __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_tile_kernel(const GemmArgs g) {
     constexpr int ELT = (int)sizeof(T), VEC = 16 / ELT, BK = BKB / ELT, BKT = BK * C::KG;
@@ -374,152 +530,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_tile_kernel(cons
     // nothing may still be on its way into the ring when the output staging takes its place
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-    // ---- write-back: 32 rows at a time through an fp32 staging area per wavefront, then rows of 16-byte vectors
-    float* const st = (float*)(smem + wave * C::OUT_WAVE);
-    constexpr int GROUP_STEP = C::WM * C::WN * C::OUT_WAVE / 4;      // staging areas of the K groups of one position
-    const float* const st0 = (const float*)(smem + wpos * C::OUT_WAVE);
-    constexpr int LPR = C::CW / VEC;                                 // vectors per row
-    constexpr int ROWS = 32 / KG;                                    // rows of a pass that this wavefront writes
-    const int lr = lane & 31, lg = lane >> 5;
-    const int gc0 = col0 + wn * C::CW;
-    const bool partial = !MUL && g.splits > 1;
-    float* const part = partial ? g.partial + (int64_t)z * g.n * (int64_t)g.m : nullptr;
-    float csum[(C::CW + 63) / 64];
-#pragma unroll
-    for (int i = 0; i < (C::CW + 63) / 64; ++i) csum[i] = 0.f;
-#pragma unroll
-    for (int tm = 0; tm < TMW; ++tm) {
-#pragma unroll
-        for (int tn = 0; tn < TNW; ++tn)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *reinterpret_cast<f32x4*>(st + lr * C::OUT_PITCH + tn * 32 + q * 8 + lg * 4) =
-                    f32x4{acc[tn][tm][q * 4], acc[tn][tm][q * 4 + 1], acc[tn][tm][q * 4 + 2], acc[tn][tm][q * 4 + 3]};
-        if constexpr (KG > 1) __syncthreads();
-        else __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const int gr0 = row0 + (wm * TMW + tm) * 32;
-        for (int idx = lane; idx < ROWS * LPR; idx += 64) {
-            const int r = kg * ROWS + idx / LPR, c = (idx % LPR) * VEC;
-            float v[VEC];
-#pragma unroll
-            for (int h = 0; h < VEC / 4; ++h) {
-                f32x4 s = *reinterpret_cast<const f32x4*>(st0 + r * C::OUT_PITCH + c + h * 4);
-#pragma unroll
-                for (int k2 = 1; k2 < KG; ++k2)
-                    s += *reinterpret_cast<const f32x4*>(st0 + k2 * GROUP_STEP + r * C::OUT_PITCH + c + h * 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[h * 4 + e] = s[e];
-            }
-            const int row = gr0 + r, col = gc0 + c;
-            const bool inside = row < g.n && col < g.m;
-            const bool whole = g.vec_out && col + VEC <= g.m;
-            const int ne = g.m - col < VEC ? g.m - col : VEC;
-            if constexpr (MUL) {
-                const T* mp = (const T*)g.mul + (int64_t)row * g.mul_rs + col;
-                T* p = (T*)g.c + (int64_t)row * g.c_rs + col;
-                float o[VEC];
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) o[e] = 0.f;
-                if (inside && whole) {
-                    const Pack<T, VEC> mv = *reinterpret_cast<const Pack<T, VEC>*>(mp);
-                    Pack<T, VEC> s;
-#pragma unroll
-                    for (int e = 0; e < VEC; ++e) {
-                        s.v[e] = from_f32<T>(to_f32(from_f32<T>(v[e])) * to_f32(mv.v[e]));
-                        o[e] = to_f32(s.v[e]);
-                    }
-                    *reinterpret_cast<Pack<T, VEC>*>(p) = s;
-                } else if (inside) {
-#pragma unroll
-                    for (int e = 0; e < VEC; ++e)
-                        if (e < ne) {
-                            const T s = from_f32<T>(to_f32(from_f32<T>(v[e])) * to_f32(mp[e]));
-                            p[e] = s;
-                            o[e] = to_f32(s);
-                        }
-                }
-                // the stored values take the place of the first group's, for the column sums
-#pragma unroll
-                for (int h = 0; h < VEC / 4; ++h)
-                    *reinterpret_cast<f32x4*>(const_cast<float*>(st0) + r * C::OUT_PITCH + c + h * 4) =
-                        f32x4{o[h * 4], o[h * 4 + 1], o[h * 4 + 2], o[h * 4 + 3]};
-            } else if (inside) {
-                if (partial) {
-                    float* p = part + (int64_t)row * g.m + col;
-                    if (whole) {
-#pragma unroll
-                        for (int h = 0; h < VEC / 4; ++h)
-                            *reinterpret_cast<f32x4*>(p + h * 4) = f32x4{v[h * 4], v[h * 4 + 1], v[h * 4 + 2], v[h * 4 + 3]};
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < VEC; ++e)
-                            if (e < ne) p[e] = v[e];
-                    }
-                } else {
-                    const bool deriv = g.epilogue == PTJ_EPI_BIAS_GELU_DERIV;
-                    const bool act = deriv || g.epilogue == PTJ_EPI_BIAS_GELU;
-                    T* p = (T*)g.c + (int64_t)row * g.c_rs + col;
-                    T* pa = g.c_aux != nullptr ? (T*)g.c_aux + (int64_t)row * g.c_aux_rs + col : nullptr;
-                    const T* add = g.epilogue == PTJ_EPI_ACCUMULATE ? p : g.epilogue != PTJ_EPI_NONE ? (const T*)g.bias + col : nullptr;
-                    if (whole) {
-                        if (add != nullptr) {
-                            const Pack<T, 4> b0 = *reinterpret_cast<const Pack<T, 4>*>(add);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) v[e] += to_f32(b0.v[e]);
-                            if constexpr (VEC == 8) {
-                                const Pack<T, 4> b1 = *reinterpret_cast<const Pack<T, 4>*>(add + 4);
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) v[4 + e] += to_f32(b1.v[e]);
-                            }
-                        }
-                        if (pa != nullptr) {
-                            float o[VEC];
-#pragma unroll
-                            for (int e = 0; e < VEC; ++e) o[e] = deriv ? gelu_grad_f(v[e]) : v[e];
-                            store_vec<T, VEC>(pa, o);
-                        }
-                        if (act) {
-#pragma unroll
-                            for (int e = 0; e < VEC; ++e) v[e] = gelu_f(v[e]);
-                        }
-                        store_vec<T, VEC>(p, v);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < VEC; ++e)
-                            if (e < ne) {
-                                float x = v[e];
-                                if (add != nullptr) x += to_f32(add[e]);
-                                if (pa != nullptr) pa[e] = from_f32<T>(deriv ? gelu_grad_f(x) : x);
-                                p[e] = from_f32<T>(act ? gelu_f(x) : x);
-                            }
-                    }
-                }
-            }
-        }
-        if constexpr (MUL) {
-            if constexpr (KG > 1) __syncthreads();
-            else __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            if (kg == 0) {
-#pragma unroll
-                for (int i = 0; i < (C::CW + 63) / 64; ++i)
-                    if (i * 64 + lane < C::CW)
-                        for (int r = 0; r < 32; ++r) csum[i] += st0[r * C::OUT_PITCH + i * 64 + lane];
-            }
-        }
-        if constexpr (KG > 1) __syncthreads();
-        else __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    }
-    if constexpr (MUL) {
-        // one row of sums per wavefront's block of rows (TMW * 32 of them)
-        const int gr = row0 + wm * TMW * 32;
-        if (kg == 0 && gr < g.n) {
-#pragma unroll
-            for (int i = 0; i < (C::CW + 63) / 64; ++i) {
-                const int c = i * 64 + lane;
-                if (c < C::CW && gc0 + c < g.m) g.colpart[(int64_t)(gr / (TMW * 32)) * g.m + gc0 + c] = csum[i];
-            }
-        }
-    }
+    gt_write_back<T, C, MUL>(g, acc, smem, row0, col0, z, wave, lane);
 }
 
 // Whether a launch can take these kernels: vector-loadable operands with non-overlapping rows, and 32-bit offsets inside a tile.

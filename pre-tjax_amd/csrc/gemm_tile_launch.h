@@ -12,9 +12,13 @@ typedef GtCfg<64, 64, 1, 2, 2, 2, 4> GtSmall2;      // two workgroups per CU
 typedef GtCfg<64, 128, 1, 4, 1, 3, 4> GtWide;
 typedef GtCfg<128, 128, 2, 4, 1, 3, 4> GtSquare;
 typedef GtCfg<128, 128, 2, 4, 1, 2, 2> GtSquare2;   // two workgroups per CU
-typedef GtCfg<128, 96, 2, 1, 2, 2, 2> GtGroups;
 typedef GtCfg<128, 192, 2, 2, 1, 2, 2> GtLarge;     // two workgroups per CU
 typedef GtCfg<256, 192, 4, 2, 1, 2, 2> GtFull;
+
+#include "gemm_split.h"
+
+typedef GsCfg<128, 128, 4, 2> GsSquare;
+typedef GsCfg<64, 64, 2, 2> GsSmall;                // two workgroups per CU
 
 template <typename T, bool MUL, typename C>
 int gt_run(const GemmArgs& g, int am, int bm, int* mul_rows, hipStream_t st) {
@@ -22,6 +26,14 @@ int gt_run(const GemmArgs& g, int am, int bm, int* mul_rows, hipStream_t st) {
     const int rc = gt_launch<T, C, MUL>(g, am, bm, st);
     if (rc != PTJ_OK || g.splits <= 1) return rc;
     return launch_splitk_reduce<T>(g, g.splits, st);
+}
+
+template <bool MUL, typename C>
+int gs_run(const GemmArgs& g, int am, int bm, int* mul_rows, hipStream_t st) {
+    if (mul_rows != nullptr) *mul_rows = C::TMW * 32;
+    const int rc = gs_launch<C, MUL>(g, am, bm, st);
+    if (rc != PTJ_OK || g.splits <= 1) return rc;
+    return launch_splitk_reduce<float>(g, g.splits, st);
 }
 
 template <typename T, bool MUL>
@@ -42,9 +54,8 @@ int gt_dispatch(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipSt
             case 1: return gt_run<T, MUL, GtSmall>(g, am, bm, mul_rows, st);
             case 2: return gt_run<T, MUL, GtSmall2>(g, am, bm, mul_rows, st);
             case 3: return gt_run<T, MUL, GtWide>(g, am, bm, mul_rows, st);
-            case 4: return gt_run<T, MUL, GtSquare2>(g, am, bm, mul_rows, st);
-            case 5: return gt_run<T, MUL, GtGroups>(g, am, bm, mul_rows, st);
-            default: return gt_run<T, MUL, GtLarge>(g, am, bm, mul_rows, st);
+            case 4: return gs_run<MUL, GsSquare>(g, am, bm, mul_rows, st);
+            default: return gs_run<MUL, GsSmall>(g, am, bm, mul_rows, st);
         }
     }
 }
