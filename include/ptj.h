@@ -379,7 +379,8 @@ int ptj_attn_bwd(const void* d_o, const void* q, const void* k, const void* v, c
  *   x_last, h   [batch * seq, dim]: the last block's output and its LayerNorm
  * ptj_gpt2_bwd takes dh = the gradient of h and writes grads[3 ..] (entries like `params`; the first
  * three are not touched) and demb [batch * seq, dim] = the gradient of table row + position of every
- * token.  Each result is bit-equal to the same sequence of single calls. */
+ * token.  The arithmetic is that of the same sequence of single calls; two
+ * products that share a launch may add their contraction in another order. */
 typedef struct ptj_gpt2_shape {
     int64_t layers, batch, seq, dim, heads, ffn, vocab, dtype, train;
 } ptj_gpt2_shape;

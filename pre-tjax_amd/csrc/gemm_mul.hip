@@ -3,35 +3,9 @@
 // for operand layouts that the GEMM reads element by element.
 #include "gemm_core.h"
 #include "gemm_plan.h"
+#include "internal.h"
 
 namespace {
-
-// Second stage of the MUL epilogue: out[col] = sum over the row blocks of colpart[block][col].  A
-// workgroup owns 64 columns; its four wavefronts take the blocks b = w, w + 4, ... (independent,
-// coalesced loads, eight in flight) and their sums are combined in wavefront order: the order of
-// the additions is fixed.
-template <typename T>
-__global__ __launch_bounds__(256) void gemm_colpart_reduce_kernel(const float* __restrict__ colpart, int blocks, int m,
-                                                                   T* __restrict__ out) {
-    __shared__ float part[4][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int col = blockIdx.x * 64 + lane;
-    float s = 0.f;
-    if (col < m) {
-        int b = w;
-        for (; b + 28 < blocks; b += 32) {
-            float v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = colpart[(int64_t)(b + 4 * u) * m + col];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) s += v[u];
-        }
-        for (; b < blocks; b += 4) s += colpart[(int64_t)b * m + col];
-    }
-    part[w][lane] = s;
-    __syncthreads();
-    if (w == 0 && col < m) out[col] = from_f32<T>((part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]));
-}
 
 // The multiplying epilogue as a pass of its own, for operand layouts the GEMM reads element by
 // element: C = round(C * mul) in place and the column sums of the result per block of 64 rows.
@@ -54,22 +28,19 @@ __global__ __launch_bounds__(256) void gemm_mul_colpart_kernel(T* __restrict__ c
 
 }  // namespace
 
-extern "C" {
-
-size_t ptj_gemm_mul_colsum_workspace_bytes(int64_t n, int64_t m) {
+extern "C" size_t ptj_gemm_mul_colsum_workspace_bytes(int64_t n, int64_t m) {
     if (n <= 0 || m <= 0) return 0;
     return (size_t)((n + 31) / 32) * (size_t)m * sizeof(float);   // a block of sums has 64 rows, 32 in the smallest tiles
 }
 
-int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul, void* c, void* colsum, int64_t n, int64_t m,
-                        int64_t k, int64_t a_rs, int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t mul_rs, int64_t c_rs,
-                        void* workspace, size_t workspace_bytes, int dtype, void* stream) {
+int ptj_gemm_mul_colsum_later(const void* a, const void* b, const void* mul, void* c, void* colsum, int64_t n, int64_t m,
+                              int64_t k, int64_t a_rs, int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t mul_rs, int64_t c_rs,
+                              void* workspace, size_t workspace_bytes, int dtype, PtjPartialSums* later, hipStream_t st) {
     PTJ_CHECK_ARG(n >= 0 && m >= 0 && k >= 0, "gemm_mul_colsum: negative dimension");
     PTJ_CHECK_ARG(n < (1ll << 31) && m < (1ll << 31) && k < (1ll << 31), "gemm_mul_colsum: dimension exceeds 31 bits");
     PTJ_CHECK_ARG(dtype == PTJ_F32 || dtype == PTJ_BF16, "gemm_mul_colsum: unknown dtype %d", dtype);
     if (m == 0) return PTJ_OK;
     PTJ_CHECK_ARG(colsum, "gemm_mul_colsum: null pointer");
-    hipStream_t st = (hipStream_t)stream;
     const size_t need = ptj_gemm_mul_colsum_workspace_bytes(n, m);
     int mul_rows = 64;   // rows of C per row of partial sums
     if (n > 0) {
@@ -110,7 +81,7 @@ int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul, void* c, 
         } else {
             // plain product first, then the multiplication and the sums as a pass over C
             const int rc = ptj_gemm(a, b, c, nullptr, n, m, k, a_rs, a_cs, b_rs, b_cs, c_rs, PTJ_EPI_NONE, nullptr, 0, nullptr, 0,
-                                    dtype, stream);
+                                    dtype, (void*)st);
             if (rc != PTJ_OK) return rc;
             const dim3 grid2((unsigned)((m + 255) / 256), (unsigned)((n + 63) / 64));
             if (dtype == PTJ_F32)
@@ -122,16 +93,16 @@ int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul, void* c, 
             PTJ_CHECK_LAUNCH();
         }
     }
-    const int blocks = (int)((n + mul_rows - 1) / mul_rows);
-    const dim3 grid((unsigned)((m + 63) / 64));
-    if (dtype == PTJ_F32)
-        hipLaunchKernelGGL((gemm_colpart_reduce_kernel<float>), grid, dim3(256), 0, st, (const float*)workspace, blocks,
-                           (int)m, (float*)colsum);
-    else
-        hipLaunchKernelGGL((gemm_colpart_reduce_kernel<bf16>), grid, dim3(256), 0, st, (const float*)workspace, blocks,
-                           (int)m, (bf16*)colsum);
-    PTJ_CHECK_LAUNCH();
-    return PTJ_OK;
+    // second stage: the column sums over the row blocks
+    PtjPartialSums now, &sums = later != nullptr ? *later : now;
+    if (!sums.add((const float*)workspace, colsum, (n + mul_rows - 1) / mul_rows, m, m))
+        return ptj_set_error(PTJ_ERR_INVALID, "gemm_mul_colsum: too many pending sums");
+    return later != nullptr ? PTJ_OK : ptj_partial_sums(now, dtype, st);
 }
 
-}  // extern "C"
+extern "C" int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul, void* c, void* colsum, int64_t n, int64_t m,
+                                   int64_t k, int64_t a_rs, int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t mul_rs, int64_t c_rs,
+                                   void* workspace, size_t workspace_bytes, int dtype, void* stream) {
+    return ptj_gemm_mul_colsum_later(a, b, mul, c, colsum, n, m, k, a_rs, a_cs, b_rs, b_cs, mul_rs, c_rs, workspace,
+                                     workspace_bytes, dtype, nullptr, (hipStream_t)stream);
+}

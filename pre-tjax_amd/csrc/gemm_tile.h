@@ -380,17 +380,16 @@ __device__ __forceinline__ void gt_write_back(const GemmArgs& g, const f32x16 (&
 }
 
 template <typename T, int AMODE, int BMODE, typename C, bool MUL>
-__global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_tile_kernel(const GemmArgs g) {
+__device__ __forceinline__ void gt_tile(const GemmArgs& g, int pid, char* __restrict__ smem) {
     constexpr int ELT = (int)sizeof(T), VEC = 16 / ELT, BK = BKB / ELT, BKT = BK * C::KG;
     constexpr int TMW = C::TMW, TNW = C::TNW, S = C::S, KG = C::KG;
-    __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = wave / (C::WM * C::WN), wpos = wave - kg * (C::WM * C::WN);
     const int wm = wpos / C::WN, wn = wpos - wm * C::WN;
     const int num_m = (g.n + C::TBM - 1) / C::TBM, num_n = (g.m + C::TBN - 1) / C::TBN;
     int tile_m, tile_n, z;
-    gt_item(g, blockIdx.x, num_m, num_n, tile_m, tile_n, z);
+    gt_item(g, pid, num_m, num_n, tile_m, tile_n, z);
     const int row0 = tile_m * C::TBM, col0 = tile_n * C::TBN;
     const int kbeg = z * g.k_per_split;
     const int kend = g.splits > 1 && kbeg + g.k_per_split < g.k ? kbeg + g.k_per_split : g.k;
@@ -531,6 +530,12 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_tile_kernel(cons
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
     gt_write_back<T, C, MUL>(g, acc, smem, row0, col0, z, wave, lane);
+}
+
+template <typename T, int AMODE, int BMODE, typename C, bool MUL>
+__global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_tile_kernel(const GemmArgs g) {
+    __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
+    gt_tile<T, AMODE, BMODE, C, MUL>(g, (int)blockIdx.x, smem);
 }
 
 // Whether a launch can take these kernels: vector-loadable operands with non-overlapping rows, and 32-bit offsets inside a tile.

@@ -2,8 +2,9 @@
 // call each: the sequence of launches that model_triton.py strings together per layer (:2214-2223, :2291-2299,
 // :2334-2351, :2583-2593), issued from native code.
 //
-// Nothing here computes: every step is an entry point of the C ABI (attention: on keep bits that one launch
-// makes for all layers).  What this file is for is the host's time.  A step of a 12-layer model is about 300
+// Nothing here computes: every step is an entry point of the C ABI or its twin in internal.h (attention on keep bits that
+// one launch makes for all layers, the two products of a linear layer's backward side by side, the second stages of all
+// column sums in one launch at the end).  What this file is for is the host's time.  A step of a 12-layer model is about 300
 // launches; issued one wrapper call at a time (allocation, pointer and stride queries, argument conversion) they
 // took 14 us each, 1.6 ms for a forward of 64 tokens and 5.1 ms for a training step of 512, several times what
 // the kernels need.  Activations live in one buffer laid out by `Layout`, temporaries in the workspace.
@@ -67,14 +68,15 @@ size_t gemm_scratch(const ptj_gpt2_shape& s, bool backward) {
     want(N, 3 * D, D); want(N, D, D); want(N, F, D); want(N, D, F);
     if (backward) {
         want(D, F, N); want(F, D, N); want(D, D, N); want(3 * D, D, N); want(N, D, 3 * D);
-        w = max2(w, ptj_gemm_mul_colsum_workspace_bytes(N, F));
-        w = max2(w, ptj_layernorm_bwd_workspace_bytes(N, D));
     }
     return w;
 }
 
 // Temporaries of the two directions in front of the scratch area that the single steps share.
-struct Temps { int64_t t1, df1, dqkv, dxm, dm, dx[2], dr[2], delta, scratch; size_t scratch_bytes, total; };
+struct Temps {
+    int64_t t1, df1, dqkv, dxm, dm, dx[2], dr[2], delta, ln_parts, mul_parts, scratch;   // partial rows: one slot per sum
+    size_t ln_slot, mul_slot, scratch_bytes, total;
+};
 Temps make_temps(const ptj_gpt2_shape& s, bool backward) {
     // the split counts behind the scratch size take some twenty estimates: kept for the shape asked for last
     static thread_local ptj_gpt2_shape last[2] = {};
@@ -93,6 +95,10 @@ Temps make_temps(const ptj_gpt2_shape& s, bool backward) {
         t.dm = take(nd);
         for (int i = 0; i < 2; ++i) { t.dx[i] = take(nd); t.dr[i] = take(nd); }
         t.delta = take(up(s.batch * s.heads * s.seq * 4));
+        t.ln_slot = (size_t)up((int64_t)ptj_layernorm_bwd_parts_bytes(N, s.dim));
+        t.mul_slot = (size_t)up((int64_t)ptj_gemm_mul_colsum_workspace_bytes(N, s.ffn));
+        t.ln_parts = take((2 * s.layers + 1) * (int64_t)t.ln_slot);
+        t.mul_parts = take(s.layers * (int64_t)t.mul_slot);
     }
     t.scratch = at;
     t.scratch_bytes = gemm_scratch(s, backward);
@@ -221,10 +227,20 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* sp, const void* const* params, const uint
 
     // Every dropout backward acts on a gradient that a LayerNorm backward has just produced, so each of those also
     // writes the dropped copy its consumer needs, and the column sums that are the bias gradient behind it.
+    // The second stages of all column sums wait in `sums` for one launch at the end (beyond some 80 layers: several).
+    PtjPartialSums sums;
+    auto ln_bwd = [&](int64_t slot, const void* dy, const void* x, const void* const* gb, const void* res, void* dx, void* const* dgb,
+                      void* dropped, void* dropped_sum, int64_t sd, const void* keep) {
+        if (sums.count + 8 > PtjPartialSums::MAX) {
+            STEP(ptj_partial_sums(sums, dt, st));
+            sums.count = 0;
+        }
+        return ptj_layernorm_bwd_later(dy, x, gb[0], res, dx, dgb[0], dgb[1], dropped, dropped_sum, train, sd, keep,
+                                       ws + t.ln_parts + slot * (int64_t)t.ln_slot, t.ln_slot, N, D, dt, &sums, st);
+    };
     int cur = 0;
-    STEP(ptj_layernorm_bwd_dropout(dh, x_last, fin[0], nullptr, ws + t.dx[0], gfin[0], gfin[1], ws + t.dr[0],
-                                   grads[P_FIRST + (L - 1) * P_BLOCK + P_B2], train, seed(3 * L), kb ? block(L - 1) + l.keep2 : nullptr,
-                                   scratch, sb, N, D, D, D, D, dt, stream));
+    STEP(ln_bwd(2 * L, dh, x_last, fin, nullptr, ws + t.dx[0], gfin, ws + t.dr[0], grads[P_FIRST + (L - 1) * P_BLOCK + P_B2],
+                seed(3 * L), kb ? block(L - 1) + l.keep2 : nullptr));
     for (int64_t i = L - 1; i >= 0; --i) {
         const void* const* w = params + P_FIRST + i * P_BLOCK;
         void* const* g = grads + P_FIRST + i * P_BLOCK;
@@ -234,33 +250,27 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* sp, const void* const* params, const uint
         const char* const dx = ws + t.dx[cur];
         const char* const d = ws + t.dr[cur];
         char* const t1 = ws + t.t1;
+        float* const colpart = (float*)(ws + t.mul_parts + i * (int64_t)t.mul_slot);
         // x_out = x_mid + dropout(ffn(ln2(x_mid)))
-        STEP(ptj_gemm(d, a + l.g1, g[P_W2], nullptr, D, F, N, 1, D, F, 1, F, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt, stream));
-        STEP(ptj_gemm_mul_colsum(d, w[P_W2], a + l.f1, ws + t.df1, g[P_B1], N, F, D, D, 1, F, 1, F, F, scratch, sb, dt, stream));
-        STEP(ptj_gemm(ws + t.df1, a + l.h2, g[P_W1], nullptr, F, D, N, 1, F, D, 1, D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt,
-                      stream));
-        STEP(ptj_gemm(ws + t.df1, w[P_W1], t1, nullptr, N, D, F, F, 1, D, 1, D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt, stream));
-        STEP(ptj_layernorm_bwd_dropout(t1, a + l.xmid, w[P_LN2G], dx, ws + t.dxm, g[P_LN2G], g[P_LN2B], ws + t.dm, nullptr, train,
-                                       seed(2 + 3 * i), kb ? a + l.keep1 : nullptr, scratch, sb, N, D, D, D, D, dt, stream));
+        STEP(ptj_linear_bwd({d, w[P_W2], a + l.g1, ws + t.df1, g[P_W2], N, D, F, a + l.f1, colpart, g[P_B1]}, scratch, sb, dt, &sums, st));
+        STEP(ptj_linear_bwd({ws + t.df1, w[P_W1], a + l.h2, t1, g[P_W1], N, F, D, nullptr, nullptr, nullptr}, scratch, sb, dt, &sums,
+                            st));
+        STEP(ln_bwd(2 * i + 1, t1, a + l.xmid, w + P_LN2G, dx, ws + t.dxm, g + P_LN2G, ws + t.dm, nullptr, seed(2 + 3 * i),
+                    kb ? a + l.keep1 : nullptr));
         // x_mid = x_in + dropout(attn(ln1(x_in)))
-        STEP(ptj_gemm(ws + t.dm, a + l.o, g[P_WO], nullptr, D, D, N, 1, D, D, 1, D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt,
-                      stream));
-        STEP(ptj_gemm(ws + t.dm, w[P_WO], t1, nullptr, N, D, D, D, 1, D, 1, D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt, stream));
+        STEP(ptj_linear_bwd({ws + t.dm, w[P_WO], a + l.o, t1, g[P_WO], N, D, D, nullptr, nullptr, nullptr}, scratch, sb, dt, &sums, st));
         STEP(ptj_attn_bwd_packed(t1, a + l.qkv, a + l.o, (const float*)(a + l.ms), (const float*)(a + l.ls), mask, ws + t.dqkv,
                                  (float*)(ws + t.delta), bits ? bits + i * bitlen : nullptr, B, H, T, train, dt, st));
-        STEP(ptj_gemm(ws + t.dqkv, h1, g[P_WQKV], nullptr, 3 * D, D, N, 1, 3 * D, D, 1, D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt,
-                      stream));
-        STEP(ptj_gemm(ws + t.dqkv, w[P_WQKV], t1, nullptr, N, D, 3 * D, 3 * D, 1, D, 1, D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt,
-                      stream));
+        STEP(ptj_linear_bwd({ws + t.dqkv, w[P_WQKV], h1, t1, g[P_WQKV], N, 3 * D, D, nullptr, nullptr, nullptr}, scratch, sb, dt, &sums,
+                            st));
         // the dropped copy feeds block i - 1 (its feed-forward dropout) or the embedding
         const bool first = i == 0;
-        STEP(ptj_layernorm_bwd_dropout(t1, x_in, w[P_LN1G], ws + t.dxm, ws + t.dx[cur ^ 1], g[P_LN1G], g[P_LN1B],
-                                       first ? demb : ws + t.dr[cur ^ 1], first ? nullptr : grads[P_FIRST + (i - 1) * P_BLOCK + P_B2],
-                                       train, seed(3 * i), kb && !first ? block(i - 1) + l.keep2 : nullptr, scratch, sb, N, D, D, D, D,
-                                       dt, stream));
+        STEP(ln_bwd(2 * i, t1, x_in, w + P_LN1G, ws + t.dxm, ws + t.dx[cur ^ 1], g + P_LN1G, first ? demb : ws + t.dr[cur ^ 1],
+                    first ? nullptr : grads[P_FIRST + (i - 1) * P_BLOCK + P_B2], seed(3 * i),
+                    kb && !first ? block(i - 1) + l.keep2 : nullptr));
         cur ^= 1;
     }
-    return PTJ_OK;
+    return ptj_partial_sums(sums, dt, st);
 }
 
 }  // extern "C"

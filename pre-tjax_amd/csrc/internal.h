@@ -16,3 +16,54 @@ int ptj_attn_fwd_packed(const void* qkv, const uint32_t* mask, void* o, float* m
 int ptj_attn_bwd_packed(const void* d_o, const void* qkv, const void* o, const float* ms, const float* ls,
                         const uint32_t* mask, void* dqkv, float* delta, const uint32_t* bits, int64_t B, int64_t H, int64_t T,
                         int train, int dtype, hipStream_t st);
+
+// A column sum over partial rows that is still to be formed: out[c] = sum_p part[p * stride + c], in a fixed order.
+// Producers that take a list append to it instead of launching their second stage, and ptj_partial_sums forms the
+// sums of a whole list in one launch (a launch per bias or norm gradient is 3-5 us of latency for 0.2 us of work).
+struct PtjPartialSum {
+    const float* part;
+    void* out;
+    int64_t nparts, cols, stride;
+};
+struct PtjPartialSums {
+    static constexpr int MAX = 512;
+    PtjPartialSum it[MAX];
+    int count = 0;
+    bool add(const float* part, void* out, int64_t nparts, int64_t cols, int64_t stride) {
+        if (count == MAX) return false;
+        it[count++] = {part, out, nparts, cols, stride};
+        return true;
+    }
+};
+int ptj_partial_sums(const PtjPartialSums& sums, int dtype, hipStream_t st);
+
+// ptj_layernorm_bwd_dropout whose second stage goes to `later` (nullptr: launched at once, as in the C ABI).
+int ptj_layernorm_bwd_later(const void* dy, const void* x, const void* gamma, const void* residual, void* dx, void* dgamma,
+                            void* dbeta, void* dropped, void* dropped_colsum, int drop_train, int64_t drop_seed,
+                            const void* keep_bytes, void* workspace, size_t workspace_bytes, int64_t rows, int64_t cols,
+                            int dtype, PtjPartialSums* later, hipStream_t st);
+
+// Workspace that one such call fills: the partial rows, three sums of them.
+inline size_t ptj_layernorm_bwd_parts_bytes(int64_t rows, int64_t cols) {
+    const int64_t per = cols <= 1024 ? (rows + 7) / 8 : rows;     // rows of up to 1024 columns: eight per workgroup
+    return (size_t)((per < 512 ? per : 512) * 3 * cols) * sizeof(float);
+}
+
+// ptj_gemm_mul_colsum whose second stage goes to `later`.
+int ptj_gemm_mul_colsum_later(const void* a, const void* b, const void* mul, void* c, void* colsum, int64_t n, int64_t m,
+                              int64_t k, int64_t a_rs, int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t mul_rs, int64_t c_rs,
+                              void* workspace, size_t workspace_bytes, int dtype, PtjPartialSums* later, hipStream_t st);
+
+// The two products of a linear layer's backward, which do not depend on each other: dx = d.w and dw = d^T.x with d [n, m],
+// w [m, k], x [n, k] row-major and contiguous.  In one launch where each alone would leave the chip half empty, else one
+// after the other.  With `mul` [n, k]: dx = round(d.w) * mul and its column sums to `colsum` (ptj_gemm_mul_colsum; the
+// partial rows in `colpart`, ptj_gemm_mul_colsum_workspace_bytes(n, k) bytes, the sums appended to `later`).
+struct PtjLinearBwd {
+    const void *d, *w, *x;
+    void *dx, *dw;
+    int64_t n, m, k;
+    const void* mul;
+    float* colpart;
+    void* colsum;
+};
+int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, int dtype, PtjPartialSums* later, hipStream_t st);

@@ -4,6 +4,7 @@
 // single HBM read and the single HBM write; all global accesses are 16-byte vectors
 // when shapes allow (VEC = 16/sizeof(T)), scalar otherwise.
 #include "common.h"
+#include "internal.h"
 
 #include <mutex>
 
@@ -575,17 +576,24 @@ __device__ __forceinline__ float reduce_partials(const float* __restrict__ col_b
     return r;
 }
 
-// Second stage: out[which][c] = sum_p part[p][which][c], fixed order.  grid = (ceil(cols/32), np)
-// with np = 2 (dgamma, dbeta) or 3 (and the column sums of the dropped output).
+// Second stages of column sums, any number per launch: workgroup b belongs to the last sum whose first_block <= b and
+// forms 32 of its columns.
+constexpr int PARTIAL_SUMS_PER_LAUNCH = 64;
+struct PartialSumItem { const float* part; void* out; int64_t stride; int nparts, cols, first_block, pad; };
+struct PartialSumBatch { PartialSumItem it[PARTIAL_SUMS_PER_LAUNCH]; int count; };
 template <typename T>
-__global__ __launch_bounds__(RED_THREADS) void layernorm_bwd_reduce_kernel(const float* __restrict__ part, int nparts,
-                                                                            int cols, T* __restrict__ dgamma,
-                                                                            T* __restrict__ dbeta, T* __restrict__ dsum) {
+__global__ __launch_bounds__(RED_THREADS) void partial_sums_kernel(const PartialSumBatch b) {
     __shared__ float sm[32][33];
-    const int c = blockIdx.x * 32 + (threadIdx.x & 31);
-    const int which = blockIdx.y, np = gridDim.y;
-    const float r = reduce_partials(part + (int64_t)which * cols + c, np * (int64_t)cols, nparts, c < cols, sm);
-    if ((threadIdx.x >> 5) == 0 && c < cols) (which == 0 ? dgamma : which == 1 ? dbeta : dsum)[c] = from_f32<T>(r);
+    int idx = 0, end = b.count;      // bisection: each step is a dependent scalar load from the kernel arguments
+    while (end - idx > 1) {
+        const int mid = (idx + end) >> 1;
+        if ((int)blockIdx.x >= b.it[mid].first_block) idx = mid;
+        else end = mid;
+    }
+    const PartialSumItem& t = b.it[idx];
+    const int c = ((int)blockIdx.x - t.first_block) * 32 + (threadIdx.x & 31);
+    const float r = reduce_partials(t.part + c, t.stride, t.nparts, c < t.cols, sm);
+    if ((threadIdx.x >> 5) == 0 && c < t.cols) ((T*)t.out)[c] = from_f32<T>(r);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1124,7 +1132,8 @@ template <typename T>
 int layernorm_bwd_impl(const void* dy, const void* x, const void* gamma, const void* res, void* dx, void* dgamma,
                        void* dbeta,
                        void* ws, size_t ws_bytes, int64_t rows, int64_t cols, int64_t dys, int64_t xs, int64_t dxs,
-                       void* drop, int drop_train, int64_t drop_seed, const void* keep, void* drop_sum, hipStream_t st) {
+                       void* drop, int drop_train, int64_t drop_seed, const void* keep, void* drop_sum, hipStream_t st,
+                       PtjPartialSums* later = nullptr) {
     RowCfg cfg;
     const bool vok = rows_vec_ok<T>(cols, {dy, x, gamma, dx, res, drop}, {dys, xs, dx ? dxs : 0});
     if (keep != nullptr && !(vok && VecOf<T>::N == 8))
@@ -1185,9 +1194,13 @@ int layernorm_bwd_impl(const void* dy, const void* x, const void* gamma, const v
 #undef LAUNCH_F
     PTJ_CHECK_LAUNCH();
     if (want_dgb) {
-        hipLaunchKernelGGL((layernorm_bwd_reduce_kernel<T>), dim3((unsigned)((cols + 31) / 32), np), dim3(RED_THREADS), 0, st,
-                           (const float*)ws, nparts, (int)cols, (T*)dgamma, (T*)dbeta, (T*)drop_sum);
-        PTJ_CHECK_LAUNCH();
+        const float* part = (const float*)ws;
+        PtjPartialSums now, &sums = later != nullptr ? *later : now;
+        if (sums.count + np > PtjPartialSums::MAX) return ptj_set_error(PTJ_ERR_INVALID, "layernorm_bwd: too many pending sums");
+        sums.add(part, dgamma, nparts, cols, np * cols);
+        sums.add(part + cols, dbeta, nparts, cols, np * cols);
+        if (np == 3) sums.add(part + 2 * cols, drop_sum, nparts, cols, np * cols);
+        if (later == nullptr) return ptj_partial_sums(now, sizeof(T) == 2 ? PTJ_BF16 : PTJ_F32, st);
     }
     return PTJ_OK;
 }
@@ -1313,6 +1326,34 @@ static int colsum_static_scratch(void** out) {
     }
     *out = g_scratch_ptr[dev];
     return PTJ_OK;
+}
+
+int ptj_partial_sums(const PtjPartialSums& sums, int dtype, hipStream_t st) {
+    for (int first = 0; first < sums.count; first += PARTIAL_SUMS_PER_LAUNCH) {
+        PartialSumBatch b;
+        b.count = sums.count - first < PARTIAL_SUMS_PER_LAUNCH ? sums.count - first : PARTIAL_SUMS_PER_LAUNCH;
+        int blocks = 0;
+        for (int i = 0; i < b.count; ++i) {
+            const PtjPartialSum& t = sums.it[first + i];
+            b.it[i] = {t.part, t.out, t.stride, (int)t.nparts, (int)t.cols, blocks, 0};
+            blocks += (int)((t.cols + 31) / 32);
+        }
+        if (dtype == PTJ_F32) hipLaunchKernelGGL((partial_sums_kernel<float>), dim3(blocks), dim3(RED_THREADS), 0, st, b);
+        else hipLaunchKernelGGL((partial_sums_kernel<bf16>), dim3(blocks), dim3(RED_THREADS), 0, st, b);
+        PTJ_CHECK_LAUNCH();
+    }
+    return PTJ_OK;
+}
+
+int ptj_layernorm_bwd_later(const void* dy, const void* x, const void* gamma, const void* residual, void* dx, void* dgamma,
+                            void* dbeta, void* dropped, void* dropped_colsum, int drop_train, int64_t drop_seed,
+                            const void* keep_bytes, void* workspace, size_t workspace_bytes, int64_t rows, int64_t cols,
+                            int dtype, PtjPartialSums* later, hipStream_t st) {
+    DTYPE_SWITCH(dtype,
+                 (layernorm_bwd_impl<float>(dy, x, gamma, residual, dx, dgamma, dbeta, workspace, workspace_bytes, rows, cols, cols,
+                                            cols, cols, dropped, drop_train, drop_seed, keep_bytes, dropped_colsum, st, later)),
+                 (layernorm_bwd_impl<bf16>(dy, x, gamma, residual, dx, dgamma, dbeta, workspace, workspace_bytes, rows, cols, cols,
+                                           cols, cols, dropped, drop_train, drop_seed, keep_bytes, dropped_colsum, st, later)));
 }
 
 extern "C" {
