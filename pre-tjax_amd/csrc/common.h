@@ -49,6 +49,9 @@ template <> struct VecOf<bf16> { static constexpr int N = 8; };
 
 template <typename T, int N> struct alignas(sizeof(T) * N) Pack { T v[N]; };
 
+// The same at any element's address (the hardware takes 16-byte accesses at every alignment).
+template <typename T, int N> struct __attribute__((packed, aligned(sizeof(T)))) LoosePack { T v[N]; };
+
 // Load N elements (N*sizeof(T) bytes, naturally aligned) and widen to float.
 template <typename T, int N>
 __device__ __forceinline__ void load_vec(const T* __restrict__ p, float (&out)[N]) {
@@ -62,6 +65,13 @@ __device__ __forceinline__ void store_vec(T* __restrict__ p, const float (&in)[N
 #pragma unroll
     for (int i = 0; i < N; ++i) t.v[i] = from_f32<T>(in[i]);
     *reinterpret_cast<Pack<T, N>*>(p) = t;
+}
+template <typename T, int N>
+__device__ __forceinline__ void store_loose(T* __restrict__ p, const float* __restrict__ in) {
+    LoosePack<T, N> t;
+#pragma unroll
+    for (int i = 0; i < N; ++i) t.v[i] = from_f32<T>(in[i]);
+    *reinterpret_cast<LoosePack<T, N>*>(p) = t;
 }
 
 // ---- wavefront (64 lanes) reductions --------------------------------------------

@@ -7,16 +7,18 @@ namespace {
 
 // gemm_plan through a small per-thread table: a training loop asks for the same few dozen products again and again,
 // and the estimate over all tile shapes and splits takes a microsecond.
-GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int persistent_splits) {
-    struct Entry { int64_t n, m, k; size_t ws; int elt, splits, cus; GemmPlan plan; };
+GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int persistent_splits, int loose) {
+    struct Entry { int64_t n, m, k; size_t ws; int elt, splits, cus, loose; GemmPlan plan; };
     constexpr int ENTRIES = 128;
     static thread_local Entry table[ENTRIES] = {};
     const int cus = num_cus();
     const uint64_t h = ((uint64_t)n * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)m * 0xC2B2AE3D27D4EB4Full) ^
-                       ((uint64_t)k * 0x165667B19E3779F9ull) ^ ((uint64_t)ws_bytes * 0xD6E8FEB86659FD93ull);
+                       ((uint64_t)k * 0x165667B19E3779F9ull) ^ ((uint64_t)(ws_bytes + loose) * 0xD6E8FEB86659FD93ull);
     Entry& e = table[(h >> 40) % ENTRIES];
-    if (e.n != n || e.m != m || e.k != k || e.ws != ws_bytes || e.elt != elt || e.splits != persistent_splits || e.cus != cus)
-        e = {n, m, k, ws_bytes, elt, persistent_splits, cus, gemm_plan(n, m, k, elt, ws_bytes, persistent_splits, cus)};
+    if (e.n != n || e.m != m || e.k != k || e.ws != ws_bytes || e.elt != elt || e.splits != persistent_splits || e.cus != cus ||
+        e.loose != loose)
+        e = {n, m, k, ws_bytes, elt, persistent_splits, cus, loose,
+             gemm_plan(n, m, k, elt, ws_bytes, persistent_splits, cus, loose)};
     return e.plan;
 }
 
@@ -26,14 +28,16 @@ extern "C" {
 
 size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
     if (n <= 0 || m <= 0 || k <= 0) return 0;
-    // which of the two kernel families runs depends on the operands' strides as well: enough for either
+    // which kernels run depends on the operands' strides and alignment as well: enough for any
     const int elt = dtype == PTJ_BF16 ? 2 : 4;
     const int s = choose_splits(n, m, k, elt, (size_t)-1);
     int first, ts, tkps;
     size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
-    const GemmPlan plan = cached_plan(n, m, k, elt, (size_t)-1, s);
-    if (plan.cfg >= 0 && plan.splits > 1 && (size_t)plan.splits * n * m * sizeof(float) > need)
-        need = (size_t)plan.splits * n * m * sizeof(float);
+    for (const int loose : {ALIGNED, LOOSE_OUTPUT, LOOSE_OPERAND}) {
+        const GemmPlan plan = cached_plan(n, m, k, elt, (size_t)-1, s, loose);
+        if (plan.cfg >= 0 && plan.splits > 1 && (size_t)plan.splits * n * m * sizeof(float) > need)
+            need = (size_t)plan.splits * n * m * sizeof(float);
+    }
     return need;
 }
 
@@ -67,11 +71,21 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n,
     g.mul = nullptr; g.mul_rs = 0; g.colpart = nullptr;
     if (epilogue == PTJ_EPI_ACCUMULATE) workspace = nullptr;   // no K split: the partial sums would not see the stored C
     int splits = workspace ? choose_splits(n, m, k, elt, workspace_bytes) : 1;
-    const int am = elt == 2 ? pick_mode<bf16>(a, a_rs, a_cs) : pick_mode<float>(a, a_rs, a_cs);
-    const int bm = elt == 2 ? pick_mode<bf16>(b, b_cs, b_rs) : pick_mode<float>(b, b_cs, b_rs);
+    int am = elt == 2 ? pick_mode<bf16>(a, a_rs, a_cs) : pick_mode<float>(a, a_rs, a_cs);
+    int bm = elt == 2 ? pick_mode<bf16>(b, b_cs, b_rs) : pick_mode<float>(b, b_cs, b_rs);
+    const bool ragged = am == GENERIC || bm == GENERIC;
+    if (ragged) {
+        am = stride_mode(a_rs, a_cs);
+        bm = stride_mode(b_cs, b_rs);
+    }
+    const int64_t v = 16 / elt;
+    bool outputs_aligned = ptj_aligned16(c) && c_rs % v == 0;
+    if (c_pre) outputs_aligned = outputs_aligned && ptj_aligned16(c_pre) && c_pre_rs % v == 0;
+    if (bias) outputs_aligned = outputs_aligned && (reinterpret_cast<uintptr_t>(bias) % (4 * (size_t)elt)) == 0;
     GemmPlan plan = {-1, 1, 0};
-    if (epilogue != PTJ_EPI_ACCUMULATE && gt_eligible(g, am, bm))
-        plan = cached_plan(n, m, k, elt, workspace && ptj_aligned16(workspace) ? workspace_bytes : 0, splits);
+    if (epilogue != PTJ_EPI_ACCUMULATE && gt_eligible(g, am, bm, ragged ? 8 : 1))
+        plan = cached_plan(n, m, k, elt, workspace && ptj_aligned16(workspace) ? workspace_bytes : 0, splits,
+                           ragged ? LOOSE_OPERAND : outputs_aligned ? ALIGNED : LOOSE_OUTPUT);
     int64_t kps = k;
     if (plan.cfg >= 0) {
         splits = plan.splits;
@@ -86,18 +100,13 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n,
     g.tail_first = 0; g.tail_splits = 1; g.tail_kps = 0;
     if (plan.cfg < 0 && splits == 1 && workspace && ptj_aligned16(workspace))
         choose_tail_split(n, m, k, elt, workspace_bytes, &g.tail_first, &g.tail_splits, &g.tail_kps);
-    {
-        const int64_t v = 16 / elt;
-        bool ok = ptj_aligned16(c) && c_rs % v == 0;
-        if (c_pre) ok = ok && ptj_aligned16(c_pre) && c_pre_rs % v == 0;
-        if (bias) ok = ok && (reinterpret_cast<uintptr_t>(bias) % (4 * (size_t)elt)) == 0;
-        if (splits > 1) ok = ok && ptj_aligned16(workspace) && m % 4 == 0;
-        g.vec_out = ok ? 1 : 0;
-    }
+    g.vec_out = outputs_aligned && (splits <= 1 || (ptj_aligned16(workspace) && m % 4 == 0)) ? 1 : 0;
     g.partial = (splits > 1 || g.tail_splits > 1) ? (float*)workspace : nullptr;
     hipStream_t st = (hipStream_t)stream;
     if (plan.cfg >= 0) {
         g.stream = 0;
+        if (ragged && dtype == PTJ_BF16)
+            return ptj_gemm_detail::gemm_ragged_launch_bf16(g, plan.cfg - RAGGED_FIRST[0], am, bm, st);
         return dtype == PTJ_F32 ? ptj_gemm_detail::gemm_tile_launch_f32(g, plan.cfg, am, bm, st)
                                 : ptj_gemm_detail::gemm_tile_launch_bf16(g, plan.cfg, am, bm, st);
     }

@@ -69,6 +69,8 @@ int launch_plain_f32(const GemmArgs& g, int splits, hipStream_t st);   // gemm_f
 // column sums per *mul_rows rows of C in g.colpart.
 int gemm_tile_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
 int gemm_tile_launch_f32(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
+// gemm_ragged.hip: bf16 operands without 16-byte alignment, configuration RAGGED_BF16 + cfg of gemm_plan.h
+int gemm_ragged_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
 int gemm_tile_mul_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipStream_t st);
 int gemm_tile_mul_launch_f32(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipStream_t st);
 }  // namespace ptj_gemm_detail
@@ -914,6 +916,9 @@ int pick_mode(const void* p, int64_t s_row, int64_t s_k) {
     if (s_row == 1 && s_k % VEC == 0) return MNMAJOR;
     return GENERIC;
 }
+
+// The layout by strides alone, whatever the alignment.
+inline int stride_mode(int64_t s_row, int64_t s_k) { return s_k == 1 ? KMAJOR : s_row == 1 ? MNMAJOR : GENERIC; }
 
 template <typename T, bool MUL = false>
 int gemm_impl(GemmArgs g, int splits, hipStream_t st) {

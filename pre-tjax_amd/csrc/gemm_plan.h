@@ -9,7 +9,7 @@
 // (microseconds) are fitted per kernel to timings of 11 products of GPT-2's feature widths at 64 to 8192
 // tokens in all operand layouts (launches replayed from a graph, operands rotating over 200 MB): the
 // estimate is within 10 % of the measurement on average, and the kernel it picks within 1.2 % of the
-// best one.
+// best one.  The kernels for unaligned bf16 operands: 30 products with odd sizes up to 4001, and the LM head's.
 #pragma once
 #include "common.h"
 
@@ -25,14 +25,18 @@ struct TileCost {
 
 // bf16 / fp32; the index is the configuration number of gemm_tile_launch
 constexpr int GT_CONFIGS[2] = {7, 6};
-constexpr TileCost GT_COST[2][7] = {
+// operands without 16-byte alignment: the configurations from here on (bf16: gemm_ragged.h; fp32: gemm_split.h)
+constexpr int RAGGED_FIRST[2] = {7, 4}, RAGGED_END[2] = {9, 6};
+constexpr TileCost GT_COST[2][9] = {
     {{32, 32, 256, 1, 2.03, 0.522, 1.24, 1.0},
      {64, 64, 128, 1, 2.49, 0.372, 1.81, 1.0},
      {64, 128, 64, 2, 3.49, 0.299, 1.21, 1.89},
      {128, 128, 64, 1, 1.84, 0.402, 3.18, 1.0},
      {128, 128, 64, 2, 2.73, 0.714, 1.88, 1.39},
      {128, 192, 64, 2, 2.45, 0.922, 5.00, 1.50},
-     {256, 192, 64, 1, 2.00, 1.250, 8.00, 1.0}},
+     {256, 192, 64, 1, 2.00, 1.250, 8.00, 1.0},
+     {128, 128, 64, 2, 4.32, 0.765, 5.66, 1.57},
+     {64, 64, 64, 2, 4.51, 0.471, 1.01, 1.08}},
     // fp32: the last two multiply on the bf16 pipe (gemm_split.h)
     {{32, 32, 128, 1, 3.25, 0.663, 1.67, 1.0},
      {64, 64, 64, 1, 3.56, 1.077, 2.37, 1.0},
@@ -41,6 +45,8 @@ constexpr TileCost GT_COST[2][7] = {
      {128, 128, 32, 1, 3.10, 1.218, 3.22, 1.0},
      {64, 64, 32, 2, 5.87, 0.640, 0.00, 1.32}},
 };
+
+enum { ALIGNED = 0, LOOSE_OUTPUT = 1, LOOSE_OPERAND = 2 };   // what of a product does not come in aligned 16-byte vectors
 
 struct GemmPlan {
     int cfg;      // configuration of gemm_tile.h, or -1: the persistent kernels with their own K split
@@ -83,13 +89,16 @@ inline double gp_persistent_us(int64_t n, int64_t m, int64_t k, int elt, int spl
 
 // `persistent_splits`: what choose_splits gives the persistent kernels; `ws_bytes`: workspace for fp32 partial sums.
 // Contractions shorter than 1024 are not split, so that a product and the same product with another epilogue
-// add in the same order.
-inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int persistent_splits, int cus) {
+// add in the same order.  `loose`: the persistent kernels read operands without 16-byte alignment element by element (an
+// order of magnitude slower) and write such outputs so (twice the time at k = 768); the tile kernels write any.
+inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int persistent_splits, int cus,
+                          int loose = ALIGNED) {
+    const bool ragged = loose == LOOSE_OPERAND;
     GemmPlan best = {-1, 1, (int)k};
     // within 8 % the persistent kernels are kept: in a training step their loads run on from product to product
-    double best_us = 0.92 * gp_persistent_us(n, m, k, elt, persistent_splits, cus);
+    double best_us = ragged ? 1e30 : (loose ? 2.0 : 0.92) * gp_persistent_us(n, m, k, elt, persistent_splits, cus);
     const int type = elt == 2 ? 0 : 1;
-    for (int i = 0; i < GT_CONFIGS[type]; ++i) {
+    for (int i = ragged ? RAGGED_FIRST[type] : 0; i < (ragged ? RAGGED_END[type] : GT_CONFIGS[type]); ++i) {
         const TileCost& c = GT_COST[type][i];
         for (int s = 1; s <= 16; ++s) {
             if (s > 1 && (k < 1024 || k / s < 256 || (size_t)s * (size_t)n * (size_t)m * sizeof(float) > ws_bytes)) break;

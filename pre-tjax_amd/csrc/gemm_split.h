@@ -15,7 +15,9 @@
 // Panels travel HBM -> registers as fp32, two steps ahead, are split once per workgroup and stored as three bf16 planes
 // (the conversion costs 5.5 vector instructions per element, spread between the MFMAs), 32 contraction elements per
 // step, double-buffered in LDS.  KMAJOR operands: [row][64 bytes], 16-byte chunks XOR-swizzled; MNMAJOR: [k][rows], read
-// through ds_read_b64_tr_b16.  Border handling (buffer descriptors) and write-back are those of gemm_tile.h.
+// through ds_read_b64_tr_b16.  Rows may start at any element: a buffer load needs 4-byte alignment.  What
+// lies past the operand's end reads as zero (buffer descriptors), and the last step, whose vectors may hold elements of
+// the next row or cross that end, is fetched element by element.  Write-back is that of gemm_tile.h.
 typedef float gs_f32x2 __attribute__((ext_vector_type(2)));
 typedef short gs_i16x4 __attribute__((ext_vector_type(4)));
 
@@ -42,13 +44,15 @@ struct GsOperand {
     uint32_t loff[PER];                                         // LDS offset inside a plane
     const char* base;
     int64_t left, step;
+    bool cut;                                                   // MNMAJOR: the tile ends inside a vector
     gt_u32x4 r[2][PER];                                         // two steps in flight
 
     __device__ __forceinline__ void init(const void* p, int64_t s_row, int64_t s_k, int row0, int nrows, int kbeg, int k, int tid) {
         const float* first = (const float*)p + (MODE == KMAJOR ? (int64_t)row0 * s_row + kbeg : (int64_t)kbeg * s_k + row0);
         base = (const char*)first;
-        left = 4 * (MODE == KMAJOR ? (int64_t)(nrows - 1 - row0) * s_row + ((k - kbeg + 3) / 4) * 4
-                                   : (int64_t)(k - 1 - kbeg) * s_k + ((nrows - row0 + 3) / 4) * 4);
+        left = 4 * (MODE == KMAJOR ? (int64_t)(nrows - 1 - row0) * s_row + (k - kbeg)
+                                   : (int64_t)(k - 1 - kbeg) * s_k + (nrows - row0));
+        cut = nrows - row0 < ROWS && (nrows - row0) % 4 != 0;
         step = (MODE == KMAJOR ? (int64_t)1 : s_k) * BK * 4;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
@@ -71,30 +75,30 @@ struct GsOperand {
     __device__ __forceinline__ void load(int kleft, int tid) {
         const uint32_t records = kleft <= 0 ? 0u : (uint32_t)(left < 0xFFFFFF00ll ? left : 0xFFFFFF00ll);
         const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, records, 0x00020000);
+        if (MODE == KMAJOR ? kleft > 0 && kleft < BK : cut && kleft > 0 && kleft <= BK) {
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            uint32_t v = voff[i];
-            if constexpr (MODE == KMAJOR) {
-                v = ((i * NTHREADS + tid) & 7) * 4 < kleft ? v : 0xFFFFFFF0u;
-            }
-            r[SET][i] = __builtin_bit_cast(gt_u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, v, 0, 0));
+            for (int i = 0; i < PER; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    uint32_t v = voff[i] + 4 * e;
+                    if constexpr (MODE == KMAJOR) v = ((i * NTHREADS + tid) & 7) * 4 + e < kleft ? v : 0xFFFFFFF0u;
+                    r[SET][i][e] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, v, 0, 0);
+                }
+        } else {
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                r[SET][i] = __builtin_bit_cast(gt_u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff[i], 0, 0));
         }
         base += step;
         left -= step;
     }
 
-    // Splits vector I of register set SET and stores its parts into the planes at `lds`.  CLEAR: the step ends inside a
-    // vector of a KMAJOR row; its elements past kleft (the next row's, or padding) count as zero.
-    template <int SET, int I, bool CLEAR>
-    __device__ __forceinline__ void split_store(char* __restrict__ lds, int kleft, int tid) const {
+    // Splits vector I of register set SET and stores its parts into the planes at `lds`.
+    template <int SET, int I>
+    __device__ __forceinline__ void split_store(char* __restrict__ lds) const {
         float x[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[e] = __uint_as_float(r[SET][I][e]);
-        if constexpr (MODE == KMAJOR && CLEAR) {
-            const int k0 = ((I * NTHREADS + tid) & 7) * 4;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] = k0 + e < kleft ? x[e] : 0.f;
-        }
         gt_u32x2 h, m, l;
         uint32_t a, b, c;
         gs_split2(x[0], x[1], a, b, c);
@@ -172,10 +176,9 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
 #pragma unroll
             for (int e = 0; e < 16; ++e) { acc[i][j][e] = 0.f; low[i][j][e] = 0.f; }
 
-    const bool ragged = klen % 4 != 0 && (AMODE == KMAJOR || BMODE == KMAJOR);
-    auto split_piece = [&](auto set, auto i, auto clear, int buf, int kleft) {
-        if constexpr (i < OA::PER) oa.template split_store<set, i, clear>(sA + buf * C::STAGE, kleft, tid);
-        else ob.template split_store<set, i - OA::PER, clear>(sB + buf * C::STAGE, kleft, tid);
+    auto split_piece = [&](auto set, auto i, int buf) {
+        if constexpr (i < OA::PER) oa.template split_store<set, i>(sA + buf * C::STAGE);
+        else ob.template split_store<set, i - OA::PER>(sB + buf * C::STAGE);
     };
     // One contraction chunk (16 wide) of stage `buf`: six products per MFMA tile; with `split` the vectors [v0, v1) of
     // register set `set` are converted into the other stage between them.
@@ -211,7 +214,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
             constexpr int nv = v1 - v0;
             if constexpr (nv > 0)
                 gt_unroll<v0 + term * nv / 6, v0 + (term + 1) * nv / 6>(
-                    [&](auto i) { split_piece(set, i, std::false_type{}, 1 - buf, 0); });
+                    [&](auto i) { split_piece(set, i, 1 - buf); });
         });
     };
     auto load = [&](auto set, int kleft) {
@@ -226,22 +229,15 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
     // the set is then refilled with step kt + 3.
     auto step = [&](auto par, int kt) {
         constexpr std::integral_constant<int, 1 - par> NEXT{};
-        const int l1 = klen - (kt + 1) * BK;
-        if (ragged && l1 > 0 && l1 < BK) {
-            chunk(I0, par, NEXT, I0, I0);
-            chunk(I1, par, NEXT, I0, I0);
-            gt_unroll<0, NV>([&](auto i) { split_piece(NEXT, i, std::true_type{}, NEXT, l1); });
-        } else {
-            chunk(I0, par, NEXT, I0, IH);
-            chunk(I1, par, NEXT, IH, IN);
-        }
+        chunk(I0, par, NEXT, I0, IH);
+        chunk(I1, par, NEXT, IH, IN);
         load(NEXT, klen - (kt + 3) * BK);
         __syncthreads();
     };
     if (nk > 0) {
         load(I0, klen);
         load(I1, klen - BK);
-        gt_unroll<0, NV>([&](auto i) { split_piece(I0, i, std::true_type{}, 0, klen); });
+        gt_unroll<0, NV>([&](auto i) { split_piece(I0, i, 0); });
         load(I0, klen - 2 * BK);
         __syncthreads();
         for (int kt = 0; kt < nk; kt += 2) {

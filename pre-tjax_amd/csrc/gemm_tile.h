@@ -269,7 +269,7 @@ __device__ __forceinline__ void gt_write_back(const GemmArgs& g, const f32x16 (&
             }
             const int row = gr0 + r, col = gc0 + c;
             const bool inside = row < g.n && col < g.m;
-            const bool whole = g.vec_out && col + VEC <= g.m;
+            const bool whole = col + VEC <= g.m;       // rows may start at any element
             const int ne = g.m - col < VEC ? g.m - col : VEC;
             if constexpr (MUL) {
                 const T* mp = (const T*)g.mul + (int64_t)row * g.mul_rs + col;
@@ -278,14 +278,14 @@ __device__ __forceinline__ void gt_write_back(const GemmArgs& g, const f32x16 (&
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) o[e] = 0.f;
                 if (inside && whole) {
-                    const Pack<T, VEC> mv = *reinterpret_cast<const Pack<T, VEC>*>(mp);
-                    Pack<T, VEC> s;
+                    const LoosePack<T, VEC> mv = *reinterpret_cast<const LoosePack<T, VEC>*>(mp);
+                    LoosePack<T, VEC> s;
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) {
                         s.v[e] = from_f32<T>(to_f32(from_f32<T>(v[e])) * to_f32(mv.v[e]));
                         o[e] = to_f32(s.v[e]);
                     }
-                    *reinterpret_cast<Pack<T, VEC>*>(p) = s;
+                    *reinterpret_cast<LoosePack<T, VEC>*>(p) = s;
                 } else if (inside) {
 #pragma unroll
                     for (int e = 0; e < VEC; ++e)
@@ -306,7 +306,7 @@ __device__ __forceinline__ void gt_write_back(const GemmArgs& g, const f32x16 (&
                     if (whole) {
 #pragma unroll
                         for (int h = 0; h < VEC / 4; ++h)
-                            *reinterpret_cast<f32x4*>(p + h * 4) = f32x4{v[h * 4], v[h * 4 + 1], v[h * 4 + 2], v[h * 4 + 3]};
+                            store_loose<float, 4>(p + h * 4, v + h * 4);
                     } else {
 #pragma unroll
                         for (int e = 0; e < VEC; ++e)
@@ -320,26 +320,21 @@ __device__ __forceinline__ void gt_write_back(const GemmArgs& g, const f32x16 (&
                     const T* add = g.epilogue == PTJ_EPI_ACCUMULATE ? p : g.epilogue != PTJ_EPI_NONE ? (const T*)g.bias + col : nullptr;
                     if (whole) {
                         if (add != nullptr) {
-                            const Pack<T, 4> b0 = *reinterpret_cast<const Pack<T, 4>*>(add);
+                            const LoosePack<T, VEC> b = *reinterpret_cast<const LoosePack<T, VEC>*>(add);
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) v[e] += to_f32(b0.v[e]);
-                            if constexpr (VEC == 8) {
-                                const Pack<T, 4> b1 = *reinterpret_cast<const Pack<T, 4>*>(add + 4);
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) v[4 + e] += to_f32(b1.v[e]);
-                            }
+                            for (int e = 0; e < VEC; ++e) v[e] += to_f32(b.v[e]);
                         }
                         if (pa != nullptr) {
                             float o[VEC];
 #pragma unroll
                             for (int e = 0; e < VEC; ++e) o[e] = deriv ? gelu_grad_f(v[e]) : v[e];
-                            store_vec<T, VEC>(pa, o);
+                            store_loose<T, VEC>(pa, o);
                         }
                         if (act) {
 #pragma unroll
                             for (int e = 0; e < VEC; ++e) v[e] = gelu_f(v[e]);
                         }
-                        store_vec<T, VEC>(p, v);
+                        store_loose<T, VEC>(p, v);
                     } else {
 #pragma unroll
                         for (int e = 0; e < VEC; ++e)
@@ -538,13 +533,14 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_tile_kernel(cons
     gt_tile<T, AMODE, BMODE, C, MUL>(g, (int)blockIdx.x, smem);
 }
 
-// Whether a launch can take these kernels: vector-loadable operands with non-overlapping rows, and 32-bit offsets inside a tile.
-inline bool gt_eligible(const GemmArgs& g, int am, int bm) {
+// Whether a launch can take these kernels: operands with one unit stride (with the alignment of pick_mode, or for the
+// kernels that take any: rows of at least one vector), non-overlapping rows, and 32-bit offsets inside a tile.
+inline bool gt_eligible(const GemmArgs& g, int am, int bm, int64_t least_pitch = 1) {
     if (am == GENERIC || bm == GENERIC || g.k < 1) return false;
     const int64_t lim = 1 << 21;
-    const bool a_ok = am == KMAJOR ? g.a_row >= g.k && g.a_row < lim : g.a_k >= g.n && g.a_k < lim;
-    const bool b_ok = bm == KMAJOR ? g.b_row >= g.k && g.b_row < lim : g.b_k >= g.m && g.b_k < lim;
-    return a_ok && b_ok;
+    const int64_t a_pitch = am == KMAJOR ? g.a_row : g.a_k, b_pitch = bm == KMAJOR ? g.b_row : g.b_k;
+    return a_pitch >= (am == KMAJOR ? g.k : g.n) && a_pitch >= least_pitch && a_pitch < lim &&
+           b_pitch >= (bm == KMAJOR ? g.k : g.m) && b_pitch >= least_pitch && b_pitch < lim;
 }
 
 template <typename T, typename C, bool MUL>
