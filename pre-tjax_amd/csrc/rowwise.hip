@@ -576,22 +576,25 @@ __device__ __forceinline__ float reduce_partials(const float* __restrict__ col_b
     return r;
 }
 
-// Second stages of column sums, any number per launch: workgroup b belongs to the last sum whose first_block <= b and
-// forms 32 of its columns.
-constexpr int PARTIAL_SUMS_PER_LAUNCH = 64;
-struct PartialSumItem { const float* part; void* out; int64_t stride; int nparts, cols, first_block, pad; };
-struct PartialSumBatch { PartialSumItem it[PARTIAL_SUMS_PER_LAUNCH]; int count; };
-template <typename T>
-__global__ __launch_bounds__(RED_THREADS) void partial_sums_kernel(const PartialSumBatch b) {
+// Second stages of column sums, up to N per launch: workgroup b belongs to the last sum whose first_block <= b and forms 32
+// of its columns.  Kernel arguments are read from host memory, two round trips here: all of first_block at once, then the
+// sum's own entry (a search that read entry after entry made one LayerNorm's second stage 1.6 us slower than a kernel of
+// its own).  The entries behind `count` repeat the grid's size in first_block, so none of them is chosen.
+constexpr int PARTIAL_SUMS_FEW = 4, PARTIAL_SUMS_MANY = 64;
+struct PartialSumItem { const float* part; void* out; int64_t stride; int nparts, cols; };
+template <int N> struct PartialSumBatch { int first_block[N]; PartialSumItem it[N]; };
+template <typename T, int N>
+__global__ __launch_bounds__(RED_THREADS) void partial_sums_kernel(const PartialSumBatch<N> b) {
     __shared__ float sm[32][33];
-    int idx = 0, end = b.count;      // bisection: each step is a dependent scalar load from the kernel arguments
-    while (end - idx > 1) {
-        const int mid = (idx + end) >> 1;
-        if ((int)blockIdx.x >= b.it[mid].first_block) idx = mid;
-        else end = mid;
+    int idx = 0, first = 0;
+#pragma unroll
+    for (int k = 1; k < N; ++k) {
+        const bool mine = (int)blockIdx.x >= b.first_block[k];
+        idx = mine ? k : idx;
+        first = mine ? b.first_block[k] : first;
     }
     const PartialSumItem& t = b.it[idx];
-    const int c = ((int)blockIdx.x - t.first_block) * 32 + (threadIdx.x & 31);
+    const int c = ((int)blockIdx.x - first) * 32 + (threadIdx.x & 31);
     const float r = reduce_partials(t.part + c, t.stride, t.nparts, c < t.cols, sm);
     if ((threadIdx.x >> 5) == 0 && c < t.cols) ((T*)t.out)[c] = from_f32<T>(r);
 }
@@ -1328,21 +1331,29 @@ static int colsum_static_scratch(void** out) {
     return PTJ_OK;
 }
 
-int ptj_partial_sums(const PtjPartialSums& sums, int dtype, hipStream_t st) {
-    for (int first = 0; first < sums.count; first += PARTIAL_SUMS_PER_LAUNCH) {
-        PartialSumBatch b;
-        b.count = sums.count - first < PARTIAL_SUMS_PER_LAUNCH ? sums.count - first : PARTIAL_SUMS_PER_LAUNCH;
+template <typename T, int N>
+static int partial_sums_launch(const PtjPartialSums& sums, hipStream_t st) {
+    for (int first = 0; first < sums.count; first += N) {
+        PartialSumBatch<N> b;
         int blocks = 0;
-        for (int i = 0; i < b.count; ++i) {
+        for (int i = 0; i < N && first + i < sums.count; ++i) {
             const PtjPartialSum& t = sums.it[first + i];
-            b.it[i] = {t.part, t.out, t.stride, (int)t.nparts, (int)t.cols, blocks, 0};
+            b.it[i] = {t.part, t.out, t.stride, (int)t.nparts, (int)t.cols};
+            b.first_block[i] = blocks;
             blocks += (int)((t.cols + 31) / 32);
         }
-        if (dtype == PTJ_F32) hipLaunchKernelGGL((partial_sums_kernel<float>), dim3(blocks), dim3(RED_THREADS), 0, st, b);
-        else hipLaunchKernelGGL((partial_sums_kernel<bf16>), dim3(blocks), dim3(RED_THREADS), 0, st, b);
+        for (int i = sums.count - first; i < N; ++i) b.first_block[i] = blocks;
+        hipLaunchKernelGGL((partial_sums_kernel<T, N>), dim3(blocks), dim3(RED_THREADS), 0, st, b);
         PTJ_CHECK_LAUNCH();
     }
     return PTJ_OK;
+}
+
+int ptj_partial_sums(const PtjPartialSums& sums, int dtype, hipStream_t st) {
+    const bool few = sums.count <= PARTIAL_SUMS_FEW;
+    if (dtype == PTJ_F32)
+        return few ? partial_sums_launch<float, PARTIAL_SUMS_FEW>(sums, st) : partial_sums_launch<float, PARTIAL_SUMS_MANY>(sums, st);
+    return few ? partial_sums_launch<bf16, PARTIAL_SUMS_FEW>(sums, st) : partial_sums_launch<bf16, PARTIAL_SUMS_MANY>(sums, st);
 }
 
 int ptj_layernorm_bwd_later(const void* dy, const void* x, const void* gamma, const void* residual, void* dx, void* dgamma,
