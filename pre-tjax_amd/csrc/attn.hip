@@ -61,19 +61,19 @@ template <typename T> struct AT {
 
 struct AttnArgs {
     const void *q, *k, *v, *o, *d_o;
-    void *out0, *out1;            // fwd: out0 = O.  bwd dkdv: out0 = dK, out1 = dV.  bwd dq: out0 = dQ
+    void *out0, *out1, *out2;     // forward: out0 = O.  Backward: dK, dV, dQ
     // nullptr = causal by index; else the mask bit-packed in both orientations (ptj_attn_pack_mask):
     //   words [0, B*T/32*T):   word (b, q/32, k) holds M[b, 32*(q/32) + r, k] in bit r   (lane = query)
     //   then the same amount:  word (b, k/32, q) holds M[b, q, 32*(k/32) + r] in bit r   (lane = key)
     //   then B*(T/32)^2 words:  class of tile (b, q/32, k/32), then the same indexed (b, k/32, q/32)
     const uint32_t* mask;
     float *ms, *ls;               // [BH, T]
-    float* delta;                 // [BH, T] rowsum(dO * O)  (backward: written by the dQ pass, read by the dK/dV pass)
+    float* delta;                 // [BH, T] rowsum(dO * O)  (backward in two launches: dQ writes it, dK/dV reads it)
     const uint32_t* keepbits;     // [BH, bitwords]  (train)
     int B, H, T, bitwords;
     // element strides: batch, head, row (the head dimension itself has unit stride)
     int64_t q_bs, q_hs, q_rs, k_bs, k_hs, k_rs, v_bs, v_hs, v_rs, o_bs, o_hs, o_rs, do_bs, do_hs, do_rs;
-    int64_t out0_bs, out0_hs, out0_rs, out1_bs, out1_hs, out1_rs;
+    int64_t out0_bs, out0_hs, out0_rs, out1_bs, out1_hs, out1_rs, out2_bs, out2_hs, out2_rs;
     int train;
     float scale;                  // 1/sqrt(dh)
 };
@@ -525,19 +525,41 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
     }
 }
 
-// ---- backward pass 1: dK, dV ------------------------------------------------------------
-// grid (B*H, ceil(T/128)); wave w owns keys key0 + 32w .. +31 (lane = key); query tiles of 64.
-template <typename T, bool HAS_MASK, bool TRAIN>
-__global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_dkdv_kernel(const AttnArgs a) {
+// ---- backward: dK, dV -------------------------------------------------------------------
+// One workgroup per (batch-head, 128 keys): wave w owns keys key0 + 32w .. +31 (lane = key); query tiles of 64.
+// OWN_DELTA: delta = rowsum(dO * O) is formed here, from the dO rows on their way into LDS and the O rows beside
+// them, instead of being read from what the dQ pass stored.
+typedef float StatTile[3][64];            // m2, 1/l, delta of a query tile
+template <typename T, int N>
+__device__ __forceinline__ void store_delta(float* __restrict__ delta, const TileLoader<T, KMAJOR, 64, ATT_THREADS> (&ld)[N],
+                                            const TileLoader<T, KMAJOR, 64, ATT_THREADS> (&lo)[N], int tid) {
+    typedef TileLoader<T, KMAJOR, 64, ATT_THREADS> L;
+    typedef typename AT<T>::F F;
+#pragma unroll
+    for (int i = 0; i < L::NV; ++i) {      // eight neighbouring lanes hold the 16-byte pieces of one row
+        float part = 0.f;
+#pragma unroll
+        for (int p = 0; p < N; ++p) {
+            const F x = __builtin_bit_cast(F, ld[p].r[i]), y = __builtin_bit_cast(F, lo[p].r[i]);
+#pragma unroll
+            for (int e = 0; e < L::VEC; ++e) part += (float)x[e] * (float)y[e];
+        }
+        part += __shfl_xor(part, 1, 64);
+        part += __shfl_xor(part, 2, 64);
+        part += __shfl_xor(part, 4, 64);
+        if ((tid & 7) == 0) delta[(tid >> 3) + L::RP * i] = part;
+    }
+}
+template <typename T> constexpr int dkdv_lds() { return 2 * 4 * AT<T>::NP * PANEL; }
+template <typename T, bool HAS_MASK, bool TRAIN, bool OWN_DELTA>
+__device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_tile, char* smem, StatTile* sstat) {
     typedef AT<T> X;
     constexpr int STAGE = 4 * X::NP * PANEL;  // Q, dO, Q^T, dO^T
-    __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
-    __shared__ __attribute__((aligned(16))) float sstat[2][3][64];  // m2, 1/l, delta per stage
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lg = lane >> 5;
     const int bh = blockIdx.x, bidx = bh / a.H, hidx = bh % a.H;
-    const int key0 = blockIdx.y * 128;                    // first key tiles see the most queries: heavy first
+    const int key0 = key_tile * 128;
     const int kw0 = key0 + wave * 32;
     const int key = kw0 + lr;
     const int krow = key < a.T ? key : a.T - 1;
@@ -546,6 +568,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_
     const T* Kb = (const T*)a.k + bidx * a.k_bs + hidx * a.k_hs;
     const T* Vb = (const T*)a.v + bidx * a.v_bs + hidx * a.v_hs;
     const T* dOb = (const T*)a.d_o + bidx * a.do_bs + hidx * a.do_hs;
+    const T* Ob = (const T*)a.o + bidx * a.o_bs + hidx * a.o_hs;
 
     typename X::F kf[X::NC], vf[X::NC];
     load_row_frags<T>(kf, Kb + (int64_t)krow * a.k_rs, lg);
@@ -553,7 +576,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_
 
     const int qt0 = key0 / 64, nqt = a.T / 64;
 
-    TileLoader<T, KMAJOR, 64, ATT_THREADS> lq[X::NP], ld[X::NP];
+    TileLoader<T, KMAJOR, 64, ATT_THREADS> lq[X::NP], ld[X::NP], lo[OWN_DELTA ? X::NP : 1];
     TileLoader<T, MNMAJOR, 64, ATT_THREADS, false, true> lqt[X::NP], ldt[X::NP];
     float st_m = 0.f, st_l = 1.f, st_d = 0.f;
     // 2-byte storage: 1/l goes into the exponent (p = 2^(s - m - log2 l)), one multiplication less
@@ -569,10 +592,11 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_
             ld[p].load_fast(dOb, a.do_rs, 1, q0__, p * X::EPP, tid);                   \
             lqt[p].load_fast(Qb, 1, a.q_rs, 0, q0__ + p * X::EPP, tid);                \
             ldt[p].load_fast(dOb, 1, a.do_rs, 0, q0__ + p * X::EPP, tid);              \
+            if constexpr (OWN_DELTA) lo[p].load_fast(Ob, a.o_rs, 1, q0__, p * X::EPP, tid); \
         }                                                                              \
         st_m = a.ms[stat0 + q0__];                                                     \
         st_l = a.ls[stat0 + q0__];                                                     \
-        st_d = a.delta[stat0 + q0__];                                                  \
+        if constexpr (!OWN_DELTA) st_d = a.delta[stat0 + q0__];                        \
     }
 #define KV_STASH(ST)                                                                   \
     {                                                                                  \
@@ -588,8 +612,9 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_
             const float m2__ = FOLD_L ? fmaf(st_m, LOG2E, __builtin_amdgcn_logf(st_l)) : st_m * LOG2E; \
             sstat[ST][0][tid] = none__ ? 0.f : m2__;                                   \
             sstat[ST][1][tid] = none__ ? 0.f : 1.0f / st_l;                            \
-            sstat[ST][2][tid] = st_d;                                                  \
+            if constexpr (!OWN_DELTA) sstat[ST][2][tid] = st_d;                        \
         }                                                                              \
+        if constexpr (OWN_DELTA) store_delta<T>(sstat[ST][2], ld, lo, tid);            \
     }
 
     f32x16 dk[2], dv[2];
@@ -699,19 +724,18 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_
     }
 }
 
-// ---- backward pass 2: dQ ----------------------------------------------------------------
+// ---- backward: dQ -----------------------------------------------------------------------
 // Same geometry as the forward (lane = query, key tiles of 64).
-template <typename T, bool HAS_MASK, bool TRAIN>
-// (2-byte storage without an explicit mask fits three wavefronts per SIMD; the bound keeps it there)
-__global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_bwd_dq_kernel(const AttnArgs a) {
+template <typename T> constexpr int dq_lds() { return 2 * 3 * AT<T>::NP * PANEL; }
+template <typename T, bool HAS_MASK, bool TRAIN, bool STORE_DELTA>
+__device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int query_tile, char* smem) {
     typedef AT<T> X;
     constexpr int STAGE = 3 * X::NP * PANEL;  // K, V, K^T
-    __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lg = lane >> 5;
     const int bh = blockIdx.x, bidx = bh / a.H, hidx = bh % a.H;
-    const int q0 = (gridDim.y - 1 - blockIdx.y) * 128;    // longest query tiles first
+    const int q0 = query_tile * 128;
     const int qw0 = q0 + wave * 32;
     const int query = qw0 + lr;
     const int qrow = query < a.T ? query : a.T - 1;
@@ -732,7 +756,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_bwd_
     const bool none = lsum == 0.f;
     const float linv = none ? 0.f : 1.0f / lsum;
     // delta = rowsum(dO * O) of the lane's query: each lane of the pair (lr, lg) holds one half
-    // of the dO row already; the dK/dV pass (launched after this one) reads the stored values.
+    // of the dO row already.
     float delta;
     {
         typename X::F of[X::NC];
@@ -744,7 +768,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_bwd_
 #pragma unroll
             for (int e = 0; e < FE; ++e) part += (float)dof[c][e] * (float)of[c][e];
         delta = part + xor32(part);
-        if (lg == 0 && query < a.T) a.delta[si] = delta;
+        if (STORE_DELTA && lg == 0 && query < a.T) a.delta[si] = delta;
     }
     const float m2 = none ? 0.f : (FOLD_L ? fmaf(a.ms[si], LOG2E, __builtin_amdgcn_logf(lsum)) : a.ms[si] * LOG2E);
 
@@ -846,7 +870,31 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_bwd_
 #undef DQ_STASH
 
     if (query < a.T)
-        store_rows<T>((T*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs, dq, a.scale, lg);
+        store_rows<T>((T*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs, dq, a.scale, lg);
+}
+
+// The backward as two launches, grid (B*H, ceil(T/128)) each: dQ, which stores delta, then dK/dV.  The tiles with the
+// longest way go first in every grid: the last query tiles, the first key tiles.
+// (2-byte storage without an explicit mask fits three wavefronts per SIMD; the bound keeps it there)
+template <typename T, bool HAS_MASK, bool TRAIN>
+__global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_bwd_dq_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) char smem[dq_lds<T>()];
+    attn_bwd_dq<T, HAS_MASK, TRAIN, true>(a, gridDim.y - 1 - blockIdx.y, smem);
+}
+template <typename T, bool HAS_MASK, bool TRAIN>
+__global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_dkdv_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<T>()];
+    __shared__ __attribute__((aligned(16))) StatTile sstat[2];
+    attn_bwd_dkdv<T, HAS_MASK, TRAIN, false>(a, blockIdx.y, smem, sstat);
+}
+// Both in one launch, grid (B*H, 2 ceil(T/128)).
+template <typename T, bool HAS_MASK, bool TRAIN>
+__global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<T>()];
+    __shared__ __attribute__((aligned(16))) StatTile sstat[2];
+    const int tile = blockIdx.y >> 1;
+    if (blockIdx.y & 1) attn_bwd_dq<T, HAS_MASK, TRAIN, false>(a, (gridDim.y >> 1) - 1 - tile, smem);
+    else attn_bwd_dkdv<T, HAS_MASK, TRAIN, true>(a, tile, smem, sstat);
 }
 
 // Launch one of the (mask, train) specialisations.
@@ -897,15 +945,24 @@ void launch_fwd(const AttnArgs& a, int dtype, hipStream_t st) {
     else ATTN_LAUNCH(attn_fwd_kernel, bf16, grid, st, a);
 }
 
-// The dQ pass also writes delta, which the dK/dV pass reads.
-void launch_bwd(const AttnArgs& dq, const AttnArgs& dkdv, int dtype, hipStream_t st) {
-    const dim3 grid((unsigned)(dq.B * dq.H), (unsigned)((dq.T + 127) / 128));
-    if (dtype == PTJ_F32) {
-        ATTN_LAUNCH(attn_bwd_dq_kernel, float, grid, st, dq);
-        ATTN_LAUNCH(attn_bwd_dkdv_kernel, float, grid, st, dkdv);
+// One launch while the two passes' workgroups make no more than four rounds of one per CU, two launches beyond.  The passes
+// then fill each other's idle CUs and a launch is saved, against an O tile read again per query tile of dK/dV (delta) and
+// the dQ tiles at the dK/dV kernel's occupancy.  GPT-2 training step, two launches / one: batch 2 x 256 (96 workgroups)
+// 3100 / 3000 us, 7 x 448 bf16 (672) 6230 / 6105, attention fp32 8 x 512 (768) 223 / 215; bf16 8 x 1024 (1536) 122 / 122,
+// step 16 x 1024 (3072) 20070 / 20330.
+void launch_bwd(const AttnArgs& a, int dtype, hipStream_t st) {
+    const int64_t nt = (a.T + 127) / 128;
+    const bool one = (int64_t)a.B * a.H * nt * 2 <= (int64_t)4 * ptj_num_cus();
+    const dim3 grid((unsigned)(a.B * a.H), (unsigned)nt), grid2((unsigned)(a.B * a.H), (unsigned)(2 * nt));
+    if (one) {
+        if (dtype == PTJ_F32) ATTN_LAUNCH(attn_bwd_kernel, float, grid2, st, a);
+        else ATTN_LAUNCH(attn_bwd_kernel, bf16, grid2, st, a);
+    } else if (dtype == PTJ_F32) {
+        ATTN_LAUNCH(attn_bwd_dq_kernel, float, grid, st, a);
+        ATTN_LAUNCH(attn_bwd_dkdv_kernel, float, grid, st, a);
     } else {
-        ATTN_LAUNCH(attn_bwd_dq_kernel, bf16, grid, st, dq);
-        ATTN_LAUNCH(attn_bwd_dkdv_kernel, bf16, grid, st, dkdv);
+        ATTN_LAUNCH(attn_bwd_dq_kernel, bf16, grid, st, a);
+        ATTN_LAUNCH(attn_bwd_dkdv_kernel, bf16, grid, st, a);
     }
 }
 
@@ -957,13 +1014,13 @@ int ptj_attn_bwd_packed(const void* d_o, const void* qkv, const void* o, const f
     a.o_hs = a.do_hs = DH;
     a.o_rs = a.do_rs = H * DH;
     const int64_t e = dtype == PTJ_BF16 ? 2 : 4;
-    AttnArgs kv = a, q = a;
-    q.out0 = dqkv;
-    q.out0_bs = a.q_bs; q.out0_hs = a.q_hs; q.out0_rs = a.q_rs;
-    kv.out0 = (char*)dqkv + DH * e;
-    kv.out1 = (char*)dqkv + 2 * DH * e;
-    kv.out0_bs = kv.out1_bs = a.q_bs; kv.out0_hs = kv.out1_hs = a.q_hs; kv.out0_rs = kv.out1_rs = a.q_rs;
-    launch_bwd(q, kv, dtype, st);
+    a.out0 = (char*)dqkv + DH * e;
+    a.out1 = (char*)dqkv + 2 * DH * e;
+    a.out2 = dqkv;
+    a.out0_bs = a.out1_bs = a.out2_bs = a.q_bs;
+    a.out0_hs = a.out1_hs = a.out2_hs = a.q_hs;
+    a.out0_rs = a.out1_rs = a.out2_rs = a.q_rs;
+    launch_bwd(a, dtype, st);
     PTJ_CHECK_LAUNCH();
     return PTJ_OK;
 }
@@ -1062,12 +1119,10 @@ int ptj_attn_bwd(const void* d_o, const void* q, const void* k, const void* v, c
         rc = launch_keepbits(bits, 1, &seed, 1, BH, a.bitwords, st);
         if (rc) return rc;
     }
-    AttnArgs a1 = a;
-    a1.out0 = dk; a1.out0_bs = dk_bs; a1.out0_hs = dk_hs; a1.out0_rs = dk_rs;
-    a1.out1 = dv; a1.out1_bs = dv_bs; a1.out1_hs = dv_hs; a1.out1_rs = dv_rs;
-    AttnArgs a2 = a;
-    a2.out0 = dq; a2.out0_bs = dq_bs; a2.out0_hs = dq_hs; a2.out0_rs = dq_rs;
-    launch_bwd(a2, a1, dtype, st);
+    a.out0 = dk; a.out0_bs = dk_bs; a.out0_hs = dk_hs; a.out0_rs = dk_rs;
+    a.out1 = dv; a.out1_bs = dv_bs; a.out1_hs = dv_hs; a.out1_rs = dv_rs;
+    a.out2 = dq; a.out2_bs = dq_bs; a.out2_hs = dq_hs; a.out2_rs = dq_rs;
+    launch_bwd(a, dtype, st);
     PTJ_CHECK_LAUNCH();
     return PTJ_OK;
 }

@@ -327,3 +327,27 @@ def test_attn_rejects_bad_shapes(mt):
     assert o2.shape == q.shape
     with pytest.raises(AssertionError):
         mt.t_scaled_dot_prod_attn_fwd3_t(torch.zeros(1, 1, 3, 64, 128, device=DEV), None, False)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T", [64, 128, 192])
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("masked", [False, True])
+def test_attn_backward_one_launch_against_two(mt, dtype, T, train, masked):
+    """A small batch takes the backward as one launch (delta formed in the dK/dV pass), a large one as two (delta stored
+    by the dQ pass).  The first row of both is the same problem; only the order of the 64 additions in delta differs:
+    a few 2^-24 of the gradients, or now and then one rounding to bf16."""
+    H, big = 12, 4 * torch.cuda.get_device_properties(0).multi_processor_count // (2 * 12 * ((T + 127) // 128)) + 1
+    qkv, dO, mask = make(big, H, T, dtype, seed=T)
+    if masked:
+        mask[:, :, : T // 3] &= torch.arange(T)[None, :, None] < T // 3
+    qkv, dO, mask = qkv.to(DEV), dO.to(DEV), mask.to(DEV)
+    got = []
+    for n in (1, big):
+        m = mask[:n].contiguous()
+        o, acts = mt.t_scaled_dot_prod_attn_fwd3_t(qkv[:n].contiguous(), m, train, 77)
+        got.append(mt.t_scaled_dot_prod_attn_bkwd3_t(dO[:n].contiguous(), acts, qkv[:n].contiguous(), m, train, 77))
+    tol = 2e-6 if dtype == torch.float32 else 2e-3
+    for a, b, what in zip(got[0], got[1], ("dq", "dk", "dv")):
+        a, b = f64(a[0]), f64(b[0])
+        assert (a - b).norm() <= tol * b.norm(), what
