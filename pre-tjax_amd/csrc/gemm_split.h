@@ -10,7 +10,11 @@
 // v_mfma_f32_32x32x2_f32 take 512.  Non-finite inputs: NaN stays NaN, an infinity gives NaN (inf - inf in the split)
 // where the fp32 instruction would give an infinity; parts of values below 2^-110 underflow.
 //
-// 4096x3072x768: 120 us, 155-163 on the fp32 instructions.
+// 4096x3072x768: 109 us, 155-163 on the fp32 instructions.  Under it the chip runs at 1.75 GHz with the matrix pipe busy 53 %
+// and LDS 35 % of the clocks: 1060 TFLOP/s of bf16 products, where the bf16 kernels of this size are too.
+// The element-wise fetch of ragged steps lies in a loop of its own: a branch in every step around two kinds of loads made
+// the register sets meet behind it, with waits and spills, and cost 119 us.  Reading the fragments of a chunk under the
+// products of the one before it (twice the fragment registers, one barrier in the middle of a step) was slower, 147-156 us.
 //
 // Panels travel HBM -> registers as fp32, two steps ahead, are split once per workgroup and stored as three bf16 planes
 // (the conversion costs 5.5 vector instructions per element, spread between the MFMAs), 32 contraction elements per
@@ -71,17 +75,23 @@ struct GsOperand {
     }
 
     // Requests the next step's values into register set SET.  kleft: contraction elements from its first one to the end.
-    template <int SET>
+    // WHOLE: no vector of the operand crosses its end.
+    template <int SET, bool WHOLE>
     __device__ __forceinline__ void load(int kleft, int tid) {
         const uint32_t records = kleft <= 0 ? 0u : (uint32_t)(left < 0xFFFFFF00ll ? left : 0xFFFFFF00ll);
         const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, records, 0x00020000);
-        if (MODE == KMAJOR ? kleft > 0 && kleft < BK : cut && kleft > 0 && kleft <= BK) {
+        if (!WHOLE && (MODE == KMAJOR ? kleft > 0 && kleft < BK : cut && kleft > 0 && kleft <= BK)) {
+            // (opaque copies: the offsets of these rare loads are formed here and hold no registers through the main loop)
+            int lane_id = tid;
+            asm volatile("" : "+v"(lane_id));
 #pragma unroll
             for (int i = 0; i < PER; ++i)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    uint32_t v = voff[i] + 4 * e;
-                    if constexpr (MODE == KMAJOR) v = ((i * NTHREADS + tid) & 7) * 4 + e < kleft ? v : 0xFFFFFFF0u;
+                    uint32_t v = voff[i];
+                    asm volatile("" : "+v"(v));
+                    v += 4 * e;
+                    if constexpr (MODE == KMAJOR) v = ((i * NTHREADS + lane_id) & 7) * 4 + e < kleft ? v : 0xFFFFFFF0u;
                     r[SET][i][e] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, v, 0, 0);
                 }
         } else {
@@ -176,13 +186,13 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
 #pragma unroll
             for (int e = 0; e < 16; ++e) { acc[i][j][e] = 0.f; low[i][j][e] = 0.f; }
 
-    auto split_piece = [&](auto set, auto i, int buf) {
+    auto split_piece = [&](auto set, auto i, int buf) __attribute__((always_inline)) {
         if constexpr (i < OA::PER) oa.template split_store<set, i>(sA + buf * C::STAGE);
         else ob.template split_store<set, i - OA::PER>(sB + buf * C::STAGE);
     };
     // One contraction chunk (16 wide) of stage `buf`: six products per MFMA tile; with `split` the vectors [v0, v1) of
     // register set `set` are converted into the other stage between them.
-    auto chunk = [&](auto c, auto buf, auto set, auto v0, auto v1) {
+    auto chunk = [&](auto c, auto buf, auto set, auto v0, auto v1) __attribute__((always_inline)) {
         bf16x8 fa[3][TMW], fb[3][TNW];
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
@@ -192,7 +202,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
             for (int t = 0; t < TNW; ++t) fb[p][t] = OB::frag(sB + buf * C::STAGE, p, wn * TNW * 32, t, c, lane);
         }
         constexpr int PA[6] = {0, 2, 0, 1, 1, 0}, PB[6] = {0, 0, 2, 1, 0, 1};
-        gt_unroll<0, 6>([&](auto term) {
+        gt_unroll<0, 6>([&](auto term) __attribute__((always_inline)) {
 #pragma unroll
             for (int tn = 0; tn < TNW; ++tn)
 #pragma unroll
@@ -214,12 +224,12 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
             constexpr int nv = v1 - v0;
             if constexpr (nv > 0)
                 gt_unroll<v0 + term * nv / 6, v0 + (term + 1) * nv / 6>(
-                    [&](auto i) { split_piece(set, i, 1 - buf); });
+                    [&](auto i) __attribute__((always_inline)) { split_piece(set, i, 1 - buf); });
         });
     };
-    auto load = [&](auto set, int kleft) {
-        oa.template load<set>(kleft, tid);
-        ob.template load<set>(kleft, tid);
+    auto load = [&](auto set, auto whole, int kleft) __attribute__((always_inline)) {
+        oa.template load<set, whole>(kleft, tid);
+        ob.template load<set, whole>(kleft, tid);
     };
     constexpr std::integral_constant<int, 0> I0{};
     constexpr std::integral_constant<int, 1> I1{};
@@ -227,24 +237,34 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
     constexpr std::integral_constant<int, NV> IN{};
     // Step kt (stage kt & 1) while the values of step kt + 1 (register set (kt + 1) & 1) are split into the other stage;
     // the set is then refilled with step kt + 3.
-    auto step = [&](auto par, int kt) {
+    auto step = [&](auto par, auto whole, int kt) __attribute__((always_inline)) {
         constexpr std::integral_constant<int, 1 - par> NEXT{};
         chunk(I0, par, NEXT, I0, IH);
         chunk(I1, par, NEXT, IH, IN);
-        load(NEXT, klen - (kt + 3) * BK);
+        load(NEXT, whole, klen - (kt + 3) * BK);
         __syncthreads();
     };
+    // no vector of either operand crosses a row's or the operand's end in any step
+    const bool whole_vectors = ((AMODE != KMAJOR && BMODE != KMAJOR) || klen % BK == 0) && (AMODE == KMAJOR || !oa.cut) &&
+                               (BMODE == KMAJOR || !ob.cut);
     if (nk > 0) {
-        load(I0, klen);
-        load(I1, klen - BK);
-        gt_unroll<0, NV>([&](auto i) { split_piece(I0, i, 0); });
-        load(I0, klen - 2 * BK);
+        constexpr std::bool_constant<true> WHOLE{};
+        constexpr std::bool_constant<false> ANY{};
+        load(I0, ANY, klen);
+        load(I1, ANY, klen - BK);
+        gt_unroll<0, NV>([&](auto i) __attribute__((always_inline)) { split_piece(I0, i, 0); });
+        load(I0, ANY, klen - 2 * BK);
         __syncthreads();
-        for (int kt = 0; kt < nk; kt += 2) {
-            step(I0, kt);
-            if (kt + 1 >= nk) break;
-            step(I1, kt + 1);
-        }
+        auto all_steps = [&](auto whole) __attribute__((always_inline)) {
+            int kt = 0;
+            for (; kt + 1 < nk; kt += 2) {
+                step(I0, whole, kt);
+                step(I1, whole, kt + 1);
+            }
+            if (kt < nk) step(I0, whole, kt);
+        };
+        if (whole_vectors) all_steps(WHOLE);
+        else all_steps(ANY);
     }
 #pragma unroll
     for (int i = 0; i < TNW; ++i)
