@@ -2,6 +2,7 @@
 // kernels are instantiated here, the fp32 ones in gemm_f32.hip (the two compile side by side).
 #include "gemm_core.h"
 #include "gemm_plan.h"
+#include "internal.h"
 
 namespace {
 
@@ -22,28 +23,10 @@ GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, 
     return e.plan;
 }
 
-}  // namespace
-
-extern "C" {
-
-size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
-    if (n <= 0 || m <= 0 || k <= 0) return 0;
-    // which kernels run depends on the operands' strides and alignment as well: enough for any
-    const int elt = dtype == PTJ_BF16 ? 2 : 4;
-    const int s = choose_splits(n, m, k, elt, (size_t)-1);
-    int first, ts, tkps;
-    size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
-    for (const int loose : {ALIGNED, LOOSE_OUTPUT, LOOSE_OPERAND}) {
-        const GemmPlan plan = cached_plan(n, m, k, elt, (size_t)-1, s, loose);
-        if (plan.cfg >= 0 && plan.splits > 1 && (size_t)plan.splits * n * m * sizeof(float) > need)
-            need = (size_t)plan.splits * n * m * sizeof(float);
-    }
-    return need;
-}
-
-int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n, int64_t m, int64_t k, int64_t a_rs,
-             int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t c_rs, int epilogue, void* c_pre, int64_t c_pre_rs,
-             void* workspace, size_t workspace_bytes, int dtype, void* stream) {
+// ptj_gemm.  `later`: a K split of the tile kernels leaves its partial sums to the caller, who finds them there.
+int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n, int64_t m, int64_t k, int64_t a_rs, int64_t a_cs,
+             int64_t b_rs, int64_t b_cs, int64_t c_rs, int epilogue, void* c_pre, int64_t c_pre_rs, void* workspace,
+             size_t workspace_bytes, int dtype, void* stream, PtjPartialProduct* later) {
     PTJ_CHECK_ARG(n >= 0 && m >= 0 && k >= 0, "gemm: negative dimension");
     PTJ_CHECK_ARG(n < (1ll << 31) && m < (1ll << 31) && k < (1ll << 31), "gemm: dimension exceeds 31 bits");
     PTJ_CHECK_ARG(epilogue >= PTJ_EPI_NONE && epilogue <= PTJ_EPI_ACCUMULATE, "gemm: unknown epilogue %d", epilogue);
@@ -69,6 +52,7 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n,
     g.c_aux_rs = c_pre_rs;
     g.epilogue = epilogue;
     g.mul = nullptr; g.mul_rs = 0; g.colpart = nullptr;
+    g.leave_partials = 0;
     if (epilogue == PTJ_EPI_ACCUMULATE) workspace = nullptr;   // no K split: the partial sums would not see the stored C
     int splits = workspace ? choose_splits(n, m, k, elt, workspace_bytes) : 1;
     int am = elt == 2 ? pick_mode<bf16>(a, a_rs, a_cs) : pick_mode<float>(a, a_rs, a_cs);
@@ -105,6 +89,11 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n,
     hipStream_t st = (hipStream_t)stream;
     if (plan.cfg >= 0) {
         g.stream = 0;
+        g.leave_partials = later != nullptr && !ragged && splits > 1 && m % 4 == 0;
+        if (g.leave_partials) {
+            later->part = g.partial;
+            later->splits = splits;
+        }
         if (ragged && dtype == PTJ_BF16)
             return ptj_gemm_detail::gemm_ragged_launch_bf16(g, plan.cfg - RAGGED_FIRST[0], am, bm, st);
         return dtype == PTJ_F32 ? ptj_gemm_detail::gemm_tile_launch_f32(g, plan.cfg, am, bm, st)
@@ -115,4 +104,38 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n,
     return dtype == PTJ_F32 ? ptj_gemm_detail::launch_plain_f32(g, splits, st) : gemm_impl<bf16>(g, splits, st);
 }
 
+}  // namespace
+
+extern "C" {
+
+size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
+    if (n <= 0 || m <= 0 || k <= 0) return 0;
+    // which kernels run depends on the operands' strides and alignment as well: enough for any
+    const int elt = dtype == PTJ_BF16 ? 2 : 4;
+    const int s = choose_splits(n, m, k, elt, (size_t)-1);
+    int first, ts, tkps;
+    size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
+    for (const int loose : {ALIGNED, LOOSE_OUTPUT, LOOSE_OPERAND}) {
+        const GemmPlan plan = cached_plan(n, m, k, elt, (size_t)-1, s, loose);
+        if (plan.cfg >= 0 && plan.splits > 1 && (size_t)plan.splits * n * m * sizeof(float) > need)
+            need = (size_t)plan.splits * n * m * sizeof(float);
+    }
+    return need;
+}
+
+int ptj_gemm(const void* a, const void* b, void* c, const void* bias, int64_t n, int64_t m, int64_t k, int64_t a_rs,
+             int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t c_rs, int epilogue, void* c_pre, int64_t c_pre_rs,
+             void* workspace, size_t workspace_bytes, int dtype, void* stream) {
+    return gemm_any(a, b, c, bias, n, m, k, a_rs, a_cs, b_rs, b_cs, c_rs, epilogue, c_pre, c_pre_rs, workspace, workspace_bytes,
+                    dtype, stream, nullptr);
+}
+
 }  // extern "C"
+
+int ptj_gemm_partial(const void* a, const void* b, void* c, const void* bias, int64_t n, int64_t m, int64_t k, int64_t a_rs,
+                     int64_t a_cs, int64_t b_rs, int64_t b_cs, void* workspace, size_t workspace_bytes, int dtype,
+                     hipStream_t st, PtjPartialProduct* out) {
+    *out = {c, nullptr, 0, bias};
+    return gemm_any(a, b, c, bias, n, m, k, a_rs, a_cs, b_rs, b_cs, m, bias ? PTJ_EPI_BIAS : PTJ_EPI_NONE, nullptr, 0, workspace,
+                    workspace_bytes, dtype, (void*)st, out);
+}

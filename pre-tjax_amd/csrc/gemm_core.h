@@ -57,6 +57,7 @@ struct GemmArgs {
     int stream;           // no K split and K is a whole even number of panels: tiles are pipelined back to back
     int vec_out;          // every output (C, pre-activation, partials) and the bias allow aligned 16-byte rows
     int epilogue;
+    int leave_partials;   // tile kernels: the caller forms the K split's sums
     // gemm_kernel<..., MUL = true> only: C = round(A.B) * mul element-wise, and the column sums of the
     // stored C over each block of 64 rows go to colpart[row / 64][m]
     const void* mul;

@@ -24,7 +24,7 @@ template <typename T, bool MUL, typename C>
 int gt_run(const GemmArgs& g, int am, int bm, int* mul_rows, hipStream_t st) {
     if (mul_rows != nullptr) *mul_rows = C::TMW * 32;
     const int rc = gt_launch<T, C, MUL>(g, am, bm, st);
-    if (rc != PTJ_OK || g.splits <= 1) return rc;
+    if (rc != PTJ_OK || g.splits <= 1 || g.leave_partials) return rc;
     return launch_splitk_reduce<T>(g, g.splits, st);
 }
 
@@ -32,7 +32,7 @@ template <bool MUL, typename C>
 int gs_run(const GemmArgs& g, int am, int bm, int* mul_rows, hipStream_t st) {
     if (mul_rows != nullptr) *mul_rows = C::TMW * 32;
     const int rc = gs_launch<C, MUL>(g, am, bm, st);
-    if (rc != PTJ_OK || g.splits <= 1) return rc;
+    if (rc != PTJ_OK || g.splits <= 1 || g.leave_partials) return rc;
     return launch_splitk_reduce<float>(g, g.splits, st);
 }
 

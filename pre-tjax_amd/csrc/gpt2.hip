@@ -27,7 +27,7 @@ struct Layout {
 };
 
 inline int elt_of(const ptj_gpt2_shape& s) { return s.dtype == PTJ_BF16 ? 2 : 4; }
-inline bool has_keep(const ptj_gpt2_shape& s) { return s.train && s.dtype == PTJ_BF16 && s.dim % 8 == 0; }
+inline bool has_keep(const ptj_gpt2_shape& s) { return s.train && s.dim % 8 == 0; }
 
 // keep: all layers' activations stay (for the backward); else one block serves every layer in turn.
 Layout make_layout(const ptj_gpt2_shape& s, bool keep) {
@@ -123,6 +123,19 @@ int check_shape(const char* what, const ptj_gpt2_shape* s) {
 enum { P_LN1G, P_LN1B, P_WQKV, P_WO, P_LN2G, P_LN2B, P_W1, P_B1, P_W2, P_B2, P_BLOCK };
 constexpr int P_FIRST = 3;   // table, its bias, positions
 
+// Dropout decisions recorded by the forward (one byte per 8 columns) for the LayerNorm backward.  The vector kernels do
+// that only: fp32 norms off the 16-byte grid recompute the decisions, bf16 ones are refused as in the single calls.
+bool keeps_bytes(const ptj_gpt2_shape& s, const void* const* params) {
+    if (!has_keep(s) || s.dtype == PTJ_BF16) return has_keep(s);
+    const void* const* fin = params + P_FIRST + s.layers * P_BLOCK;
+    bool ok = ptj_aligned16(fin[0]) && ptj_aligned16(fin[1]);
+    for (int64_t i = 0; i < s.layers; ++i) {
+        const void* const* w = params + P_FIRST + i * P_BLOCK;
+        for (const int p : {P_LN1G, P_LN1B, P_LN2G, P_LN2B}) ok = ok && ptj_aligned16(w[p]);
+    }
+    return ok;
+}
+
 #define STEP(CALL)                        \
     do {                                  \
         const int rc__ = (CALL);          \
@@ -167,6 +180,7 @@ int ptj_gpt2_fwd(const ptj_gpt2_shape* sp, const void* const* params, const int6
                        dt, stream));
     if (train) STEP(ptj_attn_keepbits_many(bits, s.layers, seeds + 1, 3, B * H, T, st));
     STEP(ptj_layernorm_fwd(base + l.x0, params[P_FIRST + P_LN1G], params[P_FIRST + P_LN1B], base + l.h0, N, D, D, D, dt, stream));
+    const bool kb = keeps_bytes(s, params);
     const char* x = base + l.x0;
     const char* hn = base + l.h0;
     for (int64_t i = 0; i < s.layers; ++i) {
@@ -174,24 +188,30 @@ int ptj_gpt2_fwd(const ptj_gpt2_shape* sp, const void* const* params, const int6
         char* const a = base + l.first_layer + i * l.layer_stride;
         const bool last = i + 1 == s.layers;
         const int64_t s1 = train ? seeds[2 + 3 * i] : 0, s2 = train ? seeds[3 + 3 * i] : 0;
-        const bool kb = has_keep(s);
         STEP(ptj_gemm(hn, w[P_WQKV], a + l.qkv, nullptr, N, 3 * D, D, D, 1, 1, D, 3 * D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt,
                       stream));
         STEP(ptj_attn_fwd_packed(a + l.qkv, mask, a + l.o, (float*)(a + l.ms), (float*)(a + l.ls), bits ? bits + i * bitlen : nullptr,
                                  B, H, T, train, dt, st));
         STEP(ptj_gemm(a + l.o, w[P_WO], ws + t.t1, nullptr, N, D, D, D, 1, 1, D, D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt, stream));
-        STEP(ptj_dropout_add_layernorm(ws + t.t1, x, w[P_LN2G], w[P_LN2B], a + l.xmid, a + l.h2, kb ? a + l.keep1 : nullptr, N, D,
-                                       train, s1, dt, stream));
+        STEP(ptj_dropout_add_layernorm_of({ws + t.t1, nullptr, 0, nullptr}, x, w[P_LN2G], w[P_LN2B], a + l.xmid, a + l.h2,
+                                          kb ? a + l.keep1 : nullptr, N, D, train, s1, dt, st));
         STEP(ptj_gemm(a + l.h2, w[P_W1], a + l.g1, w[P_B1], N, F, D, D, 1, 1, D, F,
                       keep ? PTJ_EPI_BIAS_GELU_DERIV : PTJ_EPI_BIAS_GELU, keep ? a + l.f1 : nullptr, keep ? F : 0, scratch, sb, dt,
-                      stream));
-        STEP(ptj_gemm(a + l.g1, w[P_W2], ws + t.t1, w[P_B2], N, D, F, F, 1, 1, F, D, PTJ_EPI_BIAS, nullptr, 0, scratch, sb, dt,
                       stream));
         char* const xo = last ? (char*)x_last : a + l.xout;
         char* const ho = last ? (char*)h : a + l.hnext;
         const void* const* nx = last ? fin : w + P_BLOCK;   // the norm that reads this block's output
-        STEP(ptj_dropout_add_layernorm(ws + t.t1, a + l.xmid, nx[0], nx[1], xo, ho, kb ? a + l.keep2 : nullptr, N, D, train, s2,
-                                       dt, stream));
+        // a K split's partial sums are added up by the norm, which reads them as vectors
+        PtjPartialProduct f2 = {ws + t.t1, nullptr, 0, nullptr};
+        bool vectors = true;
+        for (const void* p : {w[P_B2], nx[0], nx[1], (const void*)xo, (const void*)ho}) vectors = vectors && ptj_aligned16(p);
+        if (vectors)
+            STEP(ptj_gemm_partial(a + l.g1, w[P_W2], ws + t.t1, w[P_B2], N, D, F, F, 1, 1, F, scratch, sb, dt, st, &f2));
+        else
+            STEP(ptj_gemm(a + l.g1, w[P_W2], ws + t.t1, w[P_B2], N, D, F, F, 1, 1, F, D, PTJ_EPI_BIAS, nullptr, 0, scratch, sb, dt,
+                          stream));
+        STEP(ptj_dropout_add_layernorm_of(f2, a + l.xmid, nx[0], nx[1], xo, ho, kb ? a + l.keep2 : nullptr, N, D, train, s2, dt,
+                                          st));
         x = xo;
         hn = ho;
     }
@@ -219,7 +239,7 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* sp, const void* const* params, const uint
     const uint32_t* const bits = train ? (const uint32_t*)(base + l.keepbits) : nullptr;
     const int64_t bitlen = B * H * ptj_attn_bitwords(T);
     const int64_t L = s.layers;
-    const bool kb = has_keep(s);
+    const bool kb = keeps_bytes(s, params);
     const void* const* fin = params + P_FIRST + L * P_BLOCK;
     void* const* gfin = grads + P_FIRST + L * P_BLOCK;
     auto block = [&](int64_t i) { return base + l.first_layer + i * l.layer_stride; };

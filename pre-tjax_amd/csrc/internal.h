@@ -54,6 +54,24 @@ int ptj_gemm_mul_colsum_later(const void* a, const void* b, const void* mul, voi
                               int64_t k, int64_t a_rs, int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t mul_rs, int64_t c_rs,
                               void* workspace, size_t workspace_bytes, int dtype, PtjPartialSums* later, hipStream_t st);
 
+// A product [n, m] as stored in `c`, or, where `part` is set, as fp32 partial sums of a K split that its consumer adds up:
+// round(sum_z part[z][n][m] + bias), in the order of z.
+struct PtjPartialProduct {
+    const void* c;
+    const float* part;
+    int splits;
+    const void* bias;
+};
+// ptj_gemm(A.B (+ bias)) into contiguous rows whose K split, if it takes one, leaves the second stage to the consumer; the
+// partial sums lie in `workspace`.
+int ptj_gemm_partial(const void* a, const void* b, void* c, const void* bias, int64_t n, int64_t m, int64_t k, int64_t a_rs,
+                     int64_t a_cs, int64_t b_rs, int64_t b_cs, void* workspace, size_t workspace_bytes, int dtype,
+                     hipStream_t st, PtjPartialProduct* out);
+// ptj_dropout_add_layernorm of such a product.
+int ptj_dropout_add_layernorm_of(const PtjPartialProduct& x, const void* res, const void* gamma, const void* beta, void* y,
+                                 void* h, void* keep_bytes, int64_t rows, int64_t cols, int train, int64_t seed, int dtype,
+                                 hipStream_t st);
+
 // The two products of a linear layer's backward, which do not depend on each other: dx = d.w and dw = d^T.x with d [n, m],
 // w [m, k], x [n, k] row-major and contiguous.  In one launch where each alone would leave the chip half empty, else one
 // after the other.  With `mul` [n, k]: dx = round(d.w) * mul and its column sums to `colsum` (ptj_gemm_mul_colsum; the

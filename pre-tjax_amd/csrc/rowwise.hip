@@ -114,9 +114,40 @@ __global__ __launch_bounds__(RowGeom<TPR>::BLOCK) void layernorm_fwd_kernel(
 // A row's Philox key is uniform over its wave, so the key schedule runs on the scalar unit
 // and y is never re-read.
 // ---------------------------------------------------------------------------------
-template <typename T, int VEC, int TPR, int ITERS>
+// v += part[0][row] + part[1][row] + ... in this order, G terms requested at a time
+template <typename T, int VEC, int TPR, int ITERS, int G>
+__device__ __forceinline__ void add_partials(float (&v)[ITERS][VEC], const float* __restrict__ part, int splits, int64_t rows,
+                                             int64_t row, int cols, int nvec, int t) {
+    for (int z0 = 0; z0 < splits; z0 += G) {
+        f32x4 p[G][ITERS][VEC / 4];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int z = z0 + g < splits ? z0 + g : splits - 1;    // past the last one: read again, not added
+            const float* pz = part + ((int64_t)z * rows + row) * cols;
+#pragma unroll
+            for (int it = 0; it < ITERS; ++it) {
+                const int vi = t + it * TPR, vc = vi < nvec ? vi : nvec - 1;
+#pragma unroll
+                for (int j = 0; j < VEC / 4; ++j) p[g][it][j] = *reinterpret_cast<const f32x4*>(pz + vc * VEC + 4 * j);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            if (z0 + g >= splits) break;
+#pragma unroll
+            for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) v[it][j] += p[g][it][j / 4][j % 4];
+        }
+    }
+}
+
+// PARTIAL: x is a product that its K split left as partial sums, x = round(sum_z part[z] + bias); adding them up here saves the
+// split's second stage, a launch of 3-4 us: forward of 64 tokens 487 -> 465 us.
+template <typename T, int VEC, int TPR, int ITERS, bool PARTIAL>
 __global__ __launch_bounds__(RowGeom<TPR>::BLOCK) void dropout_add_layernorm_kernel(
-    const T* __restrict__ x, const T* __restrict__ res, const T* __restrict__ gamma, const T* __restrict__ beta,
+    const T* __restrict__ x, const float* __restrict__ part, int splits, const T* __restrict__ bias, const T* __restrict__ res, const T* __restrict__ gamma, const T* __restrict__ beta,
     T* __restrict__ y, T* __restrict__ h, uint8_t* __restrict__ keep_out, int64_t rows, int cols, int train,
     uint64_t seed) {
     __shared__ float smem[16];
@@ -132,8 +163,32 @@ __global__ __launch_bounds__(RowGeom<TPR>::BLOCK) void dropout_add_layernorm_ker
     for (int64_t row = (int64_t)blockIdx.x * RPB + sub; row < rows; row += (int64_t)gridDim.x * RPB) {
         RowRegs<T, VEC, TPR, ITERS> r;
         RawRow<T, VEC, TPR, ITERS> rr;
-        r.load(x + row * (int64_t)cols, nvec, t, 0.f);
+        if constexpr (!PARTIAL) r.load(x + row * (int64_t)cols, nvec, t, 0.f);
         rr.load(res + row * (int64_t)cols, nvec, t);
+        if constexpr (PARTIAL) {
+            static_assert(VEC % 4 == 0, "16-byte vectors of the partial sums");
+            RawRow<T, VEC, TPR, ITERS> bi;
+            if (bias != nullptr) bi.load(bias, nvec, t);
+#pragma unroll
+            for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) r.v[it][j] = 0.f;
+            // up to eight terms in flight together (as many as 96 registers hold): a round trip for each of them, one after
+            // the other, cost as much as the launch
+            constexpr int HELD = 96 / (ITERS * VEC), MOST = HELD >= 8 ? 8 : HELD >= 4 ? 4 : HELD >= 2 ? 2 : 1;
+            if (splits <= 2) add_partials<T, VEC, TPR, ITERS, (MOST < 2 ? MOST : 2)>(r.v, part, splits, rows, row, cols, nvec, t);
+            else if (splits <= 4) add_partials<T, VEC, TPR, ITERS, (MOST < 4 ? MOST : 4)>(r.v, part, splits, rows, row, cols, nvec, t);
+            else add_partials<T, VEC, TPR, ITERS, MOST>(r.v, part, splits, rows, row, cols, nvec, t);
+#pragma unroll
+            for (int it = 0; it < ITERS; ++it) {
+                const bool valid = t + it * TPR < nvec;
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) {
+                    const float v = bias != nullptr ? r.v[it][j] + bi.get(it, j) : r.v[it][j];
+                    r.v[it][j] = valid ? to_f32(from_f32<T>(v)) : 0.f;
+                }
+            }
+        }
         const uint64_t sd = seed + (uint64_t)row;
         // the row, and so the key, is the same for all lanes of the wave
         const uint32_t k0 = __builtin_amdgcn_readfirstlane((uint32_t)sd);
@@ -150,7 +205,7 @@ __global__ __launch_bounds__(RowGeom<TPR>::BLOCK) void dropout_add_layernorm_ker
                     r.v[it][j] = keep ? r.v[it][j] : 0.f;
                     bits |= keep ? (1u << j) : 0u;
                 }
-                if constexpr (sizeof(T) == 2 && (VEC == 8 || VEC == 4)) {
+                if constexpr (VEC == 8 || VEC == 4) {
                     if (keep_out != nullptr) {   // one byte per 8 columns
                         if constexpr (VEC == 8) {
                             if (valid) keep_out[row * (int64_t)(cols >> 3) + vi] = (uint8_t)bits;
@@ -1079,14 +1134,12 @@ int layernorm_fwd_impl(const void* x, const void* gamma, const void* beta, void*
 #define LAUNCH(T_, V_, TPR_, IT_)                                                                           \
     hipLaunchKernelGGL((layernorm_fwd_kernel<T_, V_, TPR_, IT_>), dim3(grid), dim3(RowGeom<TPR_>::BLOCK), 0, st, \
                        (const T_*)x, (const T_*)gamma, (const T_*)beta, (T_*)y, rows, (int)cols, xs, ys)
-    // 2-byte rows of 513..768 columns: three 8-byte vectors per lane keep all 64 lanes busy
+    // rows of 513..768 columns: three vectors of four per lane keep all 64 lanes busy
     // (the same layout, and so the same summation order, as the fused residual + norm kernel)
     bool launched = false;
-    if constexpr (sizeof(T) == 2) {
-        if (cfg.vec == 8 && cfg.tpr == 64 && cols > 512 && cols <= 768) {
-            LAUNCH(T, 4, 64, 3);
-            launched = true;
-        }
+    if (cfg.vec == VecOf<T>::N && cfg.tpr == 64 && cols > 512 && cols <= 768) {
+        LAUNCH(T, 4, 64, 3);
+        launched = true;
     }
     if (!launched) ROW_DISPATCH(T, cfg, LAUNCH);
 #undef LAUNCH
@@ -1095,30 +1148,41 @@ int layernorm_fwd_impl(const void* x, const void* gamma, const void* beta, void*
 }
 
 template <typename T>
-int dropout_add_layernorm_impl(const void* x, const void* res, const void* gamma, const void* beta, void* y, void* h,
+int dropout_add_layernorm_impl(const PtjPartialProduct& p, const void* res, const void* gamma, const void* beta, void* y, void* h,
                                void* keep, int64_t rows, int64_t cols, int train, int64_t seed, hipStream_t st) {
     RowCfg cfg;
-    const bool vok = rows_vec_ok<T>(cols, {x, res, gamma, beta, y, h}, {});
-    if (keep != nullptr && !(vok && VecOf<T>::N == 8))
-        return ptj_set_error(PTJ_ERR_INVALID, "dropout_add_layernorm: keep bytes need 2-byte elements, cols %% 8 == 0 and 16-byte aligned rows");
+    const bool partial = p.part != nullptr;
+    const bool vok = rows_vec_ok<T>(cols, {partial ? p.part : p.c, res, gamma, beta, y, h, partial ? p.bias : nullptr}, {});
+    if (partial && !vok) return ptj_set_error(PTJ_ERR_INVALID, "dropout_add_layernorm: partial sums need 16-byte vectors");
+    if (keep != nullptr && !(vok && cols % 8 == 0))
+        return ptj_set_error(PTJ_ERR_INVALID, "dropout_add_layernorm: keep bytes need cols %% 8 == 0 and 16-byte aligned rows");
     if (!pick_row_cfg(cols, VecOf<T>::N, vok, &cfg))
         return ptj_set_error(PTJ_ERR_INVALID, "dropout_add_layernorm: cols=%lld too large for the register-resident row kernel",
                              (long long)cols);
     const int grid = row_grid(rows, cfg.tpr);
-#define LAUNCH(T_, V_, TPR_, IT_)                                                                                  \
-    hipLaunchKernelGGL((dropout_add_layernorm_kernel<T_, V_, TPR_, IT_>), dim3(grid), dim3(RowGeom<TPR_>::BLOCK), 0, st, \
-                       (const T_*)x, (const T_*)res, (const T_*)gamma, (const T_*)beta, (T_*)y, (T_*)h, (uint8_t*)keep, \
+#define LAUNCH_P(T_, V_, TPR_, IT_, PART_)                                                                         \
+    hipLaunchKernelGGL((dropout_add_layernorm_kernel<T_, V_, TPR_, IT_, PART_>), dim3(grid), dim3(RowGeom<TPR_>::BLOCK), 0, st, \
+                       (const T_*)p.c, p.part, p.splits, (const T_*)p.bias, (const T_*)res, (const T_*)gamma, (const T_*)beta, (T_*)y, (T_*)h, (uint8_t*)keep, \
                        rows, (int)cols, train, (uint64_t)seed)
-    // 2-byte rows of 513..768 columns: three 8-byte vectors per lane keep all 64 lanes busy
+#define LAUNCH(T_, V_, TPR_, IT_)                                     \
+    do {                                                              \
+        if constexpr (V_ % 4 == 0) {                                  \
+            if (partial) {                                            \
+                LAUNCH_P(T_, V_, TPR_, IT_, true);                    \
+                break;                                                \
+            }                                                         \
+        }                                                             \
+        LAUNCH_P(T_, V_, TPR_, IT_, false);                           \
+    } while (0)
+    // rows of 513..768 columns: three vectors of four per lane keep all 64 lanes busy
     bool launched = false;
-    if constexpr (sizeof(T) == 2) {
-        if (cfg.vec == 8 && cfg.tpr == 64 && cols > 512 && cols <= 768) {
-            LAUNCH(T, 4, 64, 3);
-            launched = true;
-        }
+    if (cfg.vec == VecOf<T>::N && cfg.tpr == 64 && cols > 512 && cols <= 768) {
+        LAUNCH(T, 4, 64, 3);
+        launched = true;
     }
     if (!launched) ROW_DISPATCH(T, cfg, LAUNCH);
 #undef LAUNCH
+#undef LAUNCH_P
     PTJ_CHECK_LAUNCH();
     return PTJ_OK;
 }
@@ -1139,8 +1203,8 @@ int layernorm_bwd_impl(const void* dy, const void* x, const void* gamma, const v
                        PtjPartialSums* later = nullptr) {
     RowCfg cfg;
     const bool vok = rows_vec_ok<T>(cols, {dy, x, gamma, dx, res, drop}, {dys, xs, dx ? dxs : 0});
-    if (keep != nullptr && !(vok && VecOf<T>::N == 8))
-        return ptj_set_error(PTJ_ERR_INVALID, "layernorm_bwd: keep bytes need 2-byte elements and the vector path");
+    if (keep != nullptr && !(vok && cols % 8 == 0))
+        return ptj_set_error(PTJ_ERR_INVALID, "layernorm_bwd: keep bytes need cols %% 8 == 0 and the vector path");
     if (!pick_row_cfg(cols, VecOf<T>::N, vok, &cfg))
         return ptj_set_error(PTJ_ERR_INVALID, "layernorm_bwd: cols=%lld too large", (long long)cols);
     const int grid = ln_bwd_grid(rows, cfg.tpr);
@@ -1173,8 +1237,8 @@ int layernorm_bwd_impl(const void* dy, const void* x, const void* gamma, const v
             else LAUNCH_F(T_, V_, TPR_, IT_, true, false, 2);         \
         } else LAUNCH_F(T_, V_, TPR_, IT_, false, true, 0);           \
     } while (0)
-    // 2-byte rows of 513..768 columns: three 8-byte vectors per lane keep all 64 lanes busy and
-    // need a quarter fewer registers than two 16-byte vectors (one more wave per SIMD)
+    // rows of 513..768 columns: three vectors of four per lane keep all 64 lanes busy and need a quarter fewer registers
+    // than two 16-byte vectors of 2-byte elements or four of 4-byte ones (one more wave per SIMD)
     bool launched = false;
     if constexpr (sizeof(T) == 2) {
         if (cfg.vec == 8 && cfg.tpr == 64 && cols == 768 && want_dx && want_dgb && drop_mode != 2) {
@@ -1187,10 +1251,11 @@ int layernorm_bwd_impl(const void* dy, const void* x, const void* gamma, const v
             else LAUNCH_X(1);
 #undef LAUNCH_X
             launched = true;
-        } else if (cfg.vec == 8 && cfg.tpr == 64 && cols > 512 && cols <= 768) {
-            LAUNCH(T, 4, 64, 3);
-            launched = true;
         }
+    }
+    if (!launched && cfg.vec == VecOf<T>::N && cfg.tpr == 64 && cols > 512 && cols <= 768) {
+        LAUNCH(T, 4, 64, 3);
+        launched = true;
     }
     if (!launched) ROW_DISPATCH(T, cfg, LAUNCH);
 #undef LAUNCH
@@ -1356,6 +1421,13 @@ int ptj_partial_sums(const PtjPartialSums& sums, int dtype, hipStream_t st) {
     return few ? partial_sums_launch<bf16, PARTIAL_SUMS_FEW>(sums, st) : partial_sums_launch<bf16, PARTIAL_SUMS_MANY>(sums, st);
 }
 
+int ptj_dropout_add_layernorm_of(const PtjPartialProduct& x, const void* res, const void* gamma, const void* beta, void* y,
+                                 void* h, void* keep_bytes, int64_t rows, int64_t cols, int train, int64_t seed, int dtype,
+                                 hipStream_t st) {
+    DTYPE_SWITCH(dtype, (dropout_add_layernorm_impl<float>(x, res, gamma, beta, y, h, keep_bytes, rows, cols, train, seed, st)),
+                 (dropout_add_layernorm_impl<bf16>(x, res, gamma, beta, y, h, keep_bytes, rows, cols, train, seed, st)));
+}
+
 int ptj_layernorm_bwd_later(const void* dy, const void* x, const void* gamma, const void* residual, void* dx, void* dgamma,
                             void* dbeta, void* dropped, void* dropped_colsum, int drop_train, int64_t drop_seed,
                             const void* keep_bytes, void* workspace, size_t workspace_bytes, int64_t rows, int64_t cols,
@@ -1387,9 +1459,11 @@ int ptj_dropout_add_layernorm(const void* x, const void* res, const void* gamma,
     PTJ_CHECK_ARG(rows >= 0 && cols >= 2, "dropout_add_layernorm: need rows >= 0 and cols >= 2");
     if (rows == 0) return PTJ_OK;
     PTJ_CHECK_ARG(x && res && gamma && beta && y && h, "dropout_add_layernorm: null pointer");
+    PTJ_CHECK_ARG(!keep_bytes || dtype != PTJ_F32, "dropout_add_layernorm: keep bytes need 2-byte elements");
     hipStream_t st = (hipStream_t)stream;
-    DTYPE_SWITCH(dtype, (dropout_add_layernorm_impl<float>(x, res, gamma, beta, y, h, keep_bytes, rows, cols, train, seed, st)),
-                 (dropout_add_layernorm_impl<bf16>(x, res, gamma, beta, y, h, keep_bytes, rows, cols, train, seed, st)));
+    const PtjPartialProduct p = {x, nullptr, 0, nullptr};
+    DTYPE_SWITCH(dtype, (dropout_add_layernorm_impl<float>(p, res, gamma, beta, y, h, keep_bytes, rows, cols, train, seed, st)),
+                 (dropout_add_layernorm_impl<bf16>(p, res, gamma, beta, y, h, keep_bytes, rows, cols, train, seed, st)));
 }
 
 size_t ptj_layernorm_bwd_workspace_bytes(int64_t rows, int64_t cols) {
@@ -1410,6 +1484,7 @@ int ptj_layernorm_bwd_dropout(const void* dy, const void* x, const void* gamma, 
     PTJ_CHECK_ARG(!dropped_colsum || (dropped && dgamma), "layernorm_bwd: dropped_colsum needs dropped and dgamma/dbeta");
     PTJ_CHECK_ARG((dgamma == nullptr) == (dbeta == nullptr), "layernorm_bwd: dgamma and dbeta must be given together");
     PTJ_CHECK_ARG(rows >= 1 && cols >= 2, "layernorm_bwd: need rows >= 1 and cols >= 2");
+    PTJ_CHECK_ARG(!keep_bytes || dtype != PTJ_F32, "layernorm_bwd: keep bytes need 2-byte elements");
     PTJ_CHECK_ARG(dys >= cols && xs >= cols && (!dx || dxs >= cols), "layernorm_bwd: row stride smaller than cols");
     hipStream_t st = (hipStream_t)stream;
     DTYPE_SWITCH(dtype,
