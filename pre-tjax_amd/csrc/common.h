@@ -131,6 +131,11 @@ __device__ __forceinline__ float row_reduce(float v, float* smem) {
     return v;
 }
 
+// a ^ b ^ c as one v_bitop3_b32 (the compiler makes two v_xor_b32 of it)
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+}
+
 // ---- Philox4x32-10, first output word -------------------------------------------
 // Counter (offset,0,0,0), key (seed_lo, seed_hi): the generator behind the
 // reference's dropout (Triton's tl.rand).  Only word 0 is produced, so the last
@@ -142,8 +147,10 @@ __device__ __forceinline__ uint32_t philox_word0(uint32_t offset, uint32_t k0, u
     for (int r = 0; r < 10; ++r) {
         const uint64_t pa = (uint64_t)RA * c0;
         const uint64_t pb = (uint64_t)RB * c2;
-        const uint32_t n0 = (uint32_t)(pb >> 32) ^ c1 ^ k0;
-        const uint32_t n2 = (uint32_t)(pa >> 32) ^ c3 ^ k1;
+        // (the first two rounds hold zeros and wave-uniform words, which the compiler folds)
+        const uint32_t hb = (uint32_t)(pb >> 32), ha = (uint32_t)(pa >> 32);
+        const uint32_t n0 = r < 2 ? hb ^ c1 ^ k0 : xor3(hb, c1, k0);
+        const uint32_t n2 = r < 2 ? ha ^ c3 ^ k1 : xor3(ha, c3, k1);
         c1 = (uint32_t)pb;
         c3 = (uint32_t)pa;
         c0 = n0;
@@ -160,9 +167,9 @@ __device__ __forceinline__ uint32_t philox_word0(uint32_t offset, uint32_t k0, u
 // (the largest x whose product is <= 0.1f); tests check the equivalence on the host.
 #define PTJ_DROPOUT_KEEP_THRESHOLD 214748392
 __device__ __forceinline__ bool philox_keep(uint32_t offset, uint32_t k0, uint32_t k1) {
-    int32_t x = (int32_t)philox_word0(offset, k0, k1);
-    x ^= (x >> 31);  // x < 0 ? -x-1 : x
-    return x > PTJ_DROPOUT_KEEP_THRESHOLD;
+    // |x| or, for x < 0, -x - 1 above the threshold: x outside [-threshold - 1, threshold]
+    constexpr uint32_t BELOW = (uint32_t)PTJ_DROPOUT_KEEP_THRESHOLD + 1u;
+    return philox_word0(offset, k0, k1) + BELOW >= 2u * BELOW;
 }
 
 // tanh-GELU.  The reference evaluates tanh(z) as 2*sigmoid(2z) - 1, so that
