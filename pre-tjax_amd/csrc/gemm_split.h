@@ -10,10 +10,10 @@
 // v_mfma_f32_32x32x2_f32 take 512.  Non-finite inputs: NaN stays NaN, an infinity gives NaN (inf - inf in the split)
 // where the fp32 instruction would give an infinity; parts of values below 2^-110 underflow.
 //
-// 4096x3072x768: 109 us, 155-163 on the fp32 instructions.  Under it the chip runs at 1.75 GHz with the matrix pipe busy 53 %
+// 4096x3072x768: 109-118 us by box, 148-163 on the fp32 instructions.  Under it the chip runs at 1.75 GHz with the matrix pipe busy 53 %
 // and LDS 35 % of the clocks: 1060 TFLOP/s of bf16 products, where the bf16 kernels of this size are too.
 // The element-wise fetch of ragged steps lies in a loop of its own: a branch in every step around two kinds of loads made
-// the register sets meet behind it, with waits and spills, and cost 119 us.  Reading the fragments of a chunk under the
+// the register sets meet behind it, with waits and spills, and cost 119-126 us.  Reading the fragments of a chunk under the
 // products of the one before it (twice the fragment registers, one barrier in the middle of a step) was slower, 147-156 us.
 //
 // Panels travel HBM -> registers as fp32, two steps ahead, are split once per workgroup and stored as three bf16 planes
