@@ -641,6 +641,65 @@ __device__ __forceinline__ float reduce_partials(const float* __restrict__ col_b
     return r;
 }
 
+// The same sums, bit for bit, by a workgroup of 256 threads: a thread has four of the 32 slices, with the loads of all four in
+// flight together.  For launches of many sums, whose workgroups then all fit on the chip at once: the sums of a GPT-2
+// backward over 64 partial rows 32 -> 16 us, over 392 rows 36 -> 30, over 512 rows 41 -> 43.  A launch of a few sums has
+// too few workgroups for that and keeps 1024 threads for each.
+constexpr int SUM_THREADS = 256;
+__device__ __forceinline__ float reduce_partials_256(const float* __restrict__ col_base, int64_t stride, int nparts, bool active,
+                                                     float (&sm)[32][33]) {
+    const int cx = threadIdx.x & 31, py = threadIdx.x >> 5;
+    float s[4][4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s[h][u] = 0.f;
+    if (active) {
+        const int whole = nparts & ~127;      // every slice has four terms in each of these 128 rows
+#pragma unroll 2
+        for (int p = 0; p < whole; p += 128) {
+            float v[4][4];
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[h][u] = col_base[(int64_t)(p + py + 8 * h + 32 * u) * stride];
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) s[h][u] += v[h][u];
+        }
+        // up to four more terms of a slice: four go to the four chains, fewer to the first one
+        float v[4][4];
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int p = whole + py + 8 * h + 32 * u;
+                v[h][u] = p < nparts ? col_base[(int64_t)p * stride] : 0.f;
+            }
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            const int p = whole + py + 8 * h;
+            const bool four = p + 96 < nparts;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (p + 32 * u >= nparts) continue;
+                if (four) s[h][u] += v[h][u];
+                else s[h][0] += v[h][u];
+            }
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 4; ++h) sm[py + 8 * h][cx] = (s[h][0] + s[h][1]) + (s[h][2] + s[h][3]);
+    __syncthreads();
+    float r = 0.f;
+    if (py == 0) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) r += sm[i][cx];
+    }
+    return r;
+}
+
 // Second stages of column sums, up to N per launch: workgroup b belongs to the last sum whose first_block <= b and forms 32
 // of its columns.  Kernel arguments are read from host memory, two round trips here: all of first_block at once, then the
 // sum's own entry (a search that read entry after entry made one LayerNorm's second stage 1.6 us slower than a kernel of
@@ -648,8 +707,9 @@ __device__ __forceinline__ float reduce_partials(const float* __restrict__ col_b
 constexpr int PARTIAL_SUMS_FEW = 4, PARTIAL_SUMS_MANY = 64;
 struct PartialSumItem { const float* part; void* out; int64_t stride; int nparts, cols; };
 template <int N> struct PartialSumBatch { int first_block[N]; PartialSumItem it[N]; };
+template <int N> constexpr int partial_sums_threads() { return N > PARTIAL_SUMS_FEW ? SUM_THREADS : RED_THREADS; }
 template <typename T, int N>
-__global__ __launch_bounds__(RED_THREADS) void partial_sums_kernel(const PartialSumBatch<N> b) {
+__global__ __launch_bounds__(partial_sums_threads<N>()) void partial_sums_kernel(const PartialSumBatch<N> b) {
     __shared__ float sm[32][33];
     int idx = 0, first = 0;
 #pragma unroll
@@ -660,7 +720,9 @@ __global__ __launch_bounds__(RED_THREADS) void partial_sums_kernel(const Partial
     }
     const PartialSumItem& t = b.it[idx];
     const int c = ((int)blockIdx.x - first) * 32 + (threadIdx.x & 31);
-    const float r = reduce_partials(t.part + c, t.stride, t.nparts, c < t.cols, sm);
+    float r;
+    if constexpr (N > PARTIAL_SUMS_FEW) r = reduce_partials_256(t.part + c, t.stride, t.nparts, c < t.cols, sm);
+    else r = reduce_partials(t.part + c, t.stride, t.nparts, c < t.cols, sm);
     if ((threadIdx.x >> 5) == 0 && c < t.cols) ((T*)t.out)[c] = from_f32<T>(r);
 }
 
@@ -1418,7 +1480,7 @@ static int partial_sums_launch(const PtjPartialSums& sums, hipStream_t st) {
             blocks += (int)((t.cols + 31) / 32);
         }
         for (int i = sums.count - first; i < N; ++i) b.first_block[i] = blocks;
-        hipLaunchKernelGGL((partial_sums_kernel<T, N>), dim3(blocks), dim3(RED_THREADS), 0, st, b);
+        hipLaunchKernelGGL((partial_sums_kernel<T, N>), dim3(blocks), dim3(partial_sums_threads<N>()), 0, st, b);
         PTJ_CHECK_LAUNCH();
     }
     return PTJ_OK;
