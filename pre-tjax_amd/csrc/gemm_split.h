@@ -7,8 +7,8 @@
 // accumulator per rounding instead of two.  Measured against fp64 at k = 768: rms 5.7e-9 of sum |a b| for N(0,1) operands
 // and 7.2e-8 for positive ones, where the fp32 matrix instructions leave 1.4e-8 and 1.0e-7 (tests/test_gpu_gemm_split.py
 // holds the order).  Six v_mfma_f32_32x32x16_bf16 take 192 clocks where eight
-// v_mfma_f32_32x32x2_f32 take 512.  Non-finite inputs: NaN stays NaN, an infinity gives NaN (inf - inf in the split)
-// where the fp32 instruction would give an infinity; parts of values below 2^-110 underflow.
+// v_mfma_f32_32x32x2_f32 take 512.  Elements that come out NaN (an infinite operand does that) are formed again
+// by fp32 multiply-adds; parts of values below 2^-110 underflow.
 //
 // 4096x3072x768: 109-118 us by box, 148-163 on the fp32 instructions.  Under it the chip runs at 1.75 GHz with the matrix pipe busy 53 %
 // and LDS 35 % of the clocks: 1060 TFLOP/s of bf16 products, where the bf16 kernels of this size are too.
@@ -272,6 +272,34 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
         for (int j = 0; j < TMW; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] += low[i][j][e];
+    // An infinity (or a finite value that rounds to one) has no three parts and leaves NaN: such elements are formed again
+    // by multiply-adds, which give what the fp32 instructions would.
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < TNW; ++i)
+#pragma unroll
+        for (int j = 0; j < TMW; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) nan = nan || acc[i][j][e] != acc[i][j][e];
+    if (__builtin_expect(__any(nan), 0)) {
+#pragma unroll
+        for (int i = 0; i < TNW; ++i)
+#pragma unroll
+            for (int j = 0; j < TMW; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int row = row0 + (wm * TMW + j) * 32 + (lane & 31);
+                    const int col = col0 + (wn * TNW + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+                    if (acc[i][j][e] != acc[i][j][e] && row < g.n && col < g.m) {
+                        const float* pa = (const float*)g.a + (int64_t)row * g.a_row;
+                        const float* pb = (const float*)g.b + (int64_t)col * g.b_row;
+                        float s = 0.f;
+#pragma unroll 1
+                        for (int64_t k = kbeg; k < kend && s == s; ++k) s = fmaf(pa[k * g.a_k], pb[k * g.b_k], s);   // NaN stays NaN
+                        acc[i][j][e] = s;
+                    }
+                }
+    }
     __syncthreads();
     gt_write_back<float, C, MUL>(g, acc, smem, row0, col0, z, wave, lane);
 }

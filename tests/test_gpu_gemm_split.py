@@ -40,3 +40,25 @@ def test_exact_where_fp32_is_exact(mt):
     b = torch.ldexp(torch.ones(512, 256), torch.randint(0, 2, (512, 256), generator=g))
     c = mt.matmul_t(a.to(DEV), b.to(DEV))
     assert torch.equal(c.cpu().double(), a.double() @ b.double())
+
+
+@pytest.mark.parametrize("n,m,k", [(512, 768, 768), (257, 131, 77), (96, 160, 2048)])
+@pytest.mark.parametrize("b_t", [False, True])
+def test_non_finite_operands(mt, n, m, k, b_t):
+    """Infinities, NaN and values next to the largest float, which round to an infinite bf16 value, give what fp32
+    multiply-adds give: the same classes as fp64, finite elements to fp32 accuracy."""
+    g = torch.Generator().manual_seed(n)
+    a, b = torch.randn(n, k, generator=g), torch.randn(m, k, generator=g) * 1e-3
+    a[3, 5], a[7, 0], a[7, k - 1], a[n - 1, k // 2] = float("inf"), float("inf"), float("-inf"), float("nan")
+    a[11, 2], a[12, k - 1] = 3.4e38, -3.4e38
+    b[1, k - 2], b[m - 1, 9] = float("-inf"), 0.0
+    want = a.double() @ b.double().t()
+    bd = b.cuda().t() if b_t else b.t().contiguous().cuda()
+    got = mt.t_matmul_t(a.cuda(), bd).double().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    inf = torch.isinf(want)
+    assert torch.equal(got[inf], want[inf]) and torch.equal(torch.isinf(got), inf)
+    fin = torch.isfinite(want)
+    mag = torch.nan_to_num(a).double().abs() @ torch.nan_to_num(b).double().abs().t()
+    # a chain of k multiply-adds: k 2^-24 of the summed magnitudes
+    assert ((got - want).abs()[fin] <= (k * 2.0 ** -24 * mag)[fin]).all()
