@@ -274,14 +274,14 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
             for (int e = 0; e < 16; ++e) acc[i][j][e] += low[i][j][e];
     // An infinity (or a finite value that rounds to one) has no three parts and leaves NaN: such elements are formed again
     // by multiply-adds, which give what the fp32 instructions would.
-    bool nan = false;
+    float nan = 0.f;          // one multiply-add per element: 0, or NaN if one is not finite
 #pragma unroll
     for (int i = 0; i < TNW; ++i)
 #pragma unroll
         for (int j = 0; j < TMW; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) nan = nan || acc[i][j][e] != acc[i][j][e];
-    if (__builtin_expect(__any(nan), 0)) {
+            for (int e = 0; e < 16; ++e) nan = fmaf(acc[i][j][e], 0.f, nan);
+    if (__builtin_expect(__any(nan != nan), 0)) {
 #pragma unroll
         for (int i = 0; i < TNW; ++i)
 #pragma unroll
