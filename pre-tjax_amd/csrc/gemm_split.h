@@ -1,23 +1,33 @@
 // fp32 GEMM on the bf16 matrix pipe.  Included by gemm_tile_launch.h inside its unnamed namespace.
 //
-// Every fp32 value is the exact sum of three bf16 values h + m + l (each the round-to-nearest of what is left: 8 + 8 + 8
-// significant bits and two signs cover the 24), so a product of two is the sum of nine products of bf16 values, all
-// exact in the fp32 accumulator.  Six of them are formed (hh, hm, mh, hl, lh, mm); the other three together are below
-// 2^-26 |a b|, a quarter of the rounding that the fp32 multiply-add they stand in for makes.  Sixteen products enter the
-// accumulator per rounding instead of two.  Measured against fp64 at k = 768: rms 5.7e-9 of sum |a b| for N(0,1) operands
-// and 7.2e-8 for positive ones, where the fp32 matrix instructions leave 1.4e-8 and 1.0e-7 (tests/test_gpu_gemm_split.py
-// holds the order).  Six v_mfma_f32_32x32x16_bf16 take 192 clocks where eight
-// v_mfma_f32_32x32x2_f32 take 512.  Elements that come out NaN (an infinite operand does that) are formed again
-// by fp32 multiply-adds; parts of values below 2^-110 underflow.
+// The three-way split of Henry, Tang and Heinecke ("Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", 2019): every fp32 value is the exact sum of three bf16 values h + m + l (each the
+// round-to-nearest of what is left: 8 + 8 + 8 significant bits and two signs cover the 24), so a product of two is the sum of
+// nine products of bf16 values, all exact in the fp32 accumulator.  Six of them are formed (hh, hm, mh, hl, lh, mm).  Of the
+// other three, |m| <= 2^-8 and |l| <= 2^-17 of the value's power of two bound ml and lm by 2^-25 |a b| each and ll by
+// 2^-34: together at most the rounding (2^-24) that a multiply-add makes, 7e-9 rms.  Sixteen products enter the accumulator
+// per rounding where the fp32 instructions round after every one.  Measured against fp64, relative to sum |a b|: rms 5.7e-9
+// for N(0,1) operands and 7.2e-8 for positive ones at k = 768 (9.1e-9 and 4.7e-8 at k = 64, 3.0e-9 and 6.0e-8 at 4096),
+// where the fp32 instructions leave 2.8e-8 in one chain and 1.4e-8 and 1.0e-7 in four (tests/test_gpu_gemm_split.py holds
+// the order).  Six v_mfma_f32_32x32x16_bf16 take 192 clocks where eight v_mfma_f32_32x32x2_f32 take 512.
 //
-// 4096x3072x768: 109-118 us by box, 148-163 on the fp32 instructions.  Under it the chip runs at 1.75 GHz with the matrix pipe busy 53 %
-// and LDS 35 % of the clocks: 1060 TFLOP/s of bf16 products, where the bf16 kernels of this size are too.
+// Range.  Unscaled, the parts of values below 2^-110 would leave bf16's range: operands of 1e-37 would come out with 1e-4 of
+// error.  Every fp32 number is a multiple of 2^-149 and every bf16 number one of 2^-133, so 2^16 times any fp32 value has its
+// three parts exactly (the matrix instructions keep subnormal operands); both operands are split so and the 2^32 is taken
+// out of the finished sums.  What that pushes out at the other end -- operands from 2^112, sums from 2^96, also infinities
+// and NaN -- leaves an infinite or NaN sum: wavefronts that hold one form their tiles again with the fp32 instructions,
+// unscaled (4096x3072x768 wholly so: 460 us).  Contractions of up to four elements go there as well: with so few roundings
+// the products left out show (6e-8 -> 9e-8 at worst for a single product).  A scale from the largest value of a panel would
+// lose tiny values beside large ones.  The multiplication costs 3 % (108 -> 111 us).
+//
+// 4096x3072x768: 111-121 us by box, 148-163 on the fp32 instructions.  Under it the chip runs at 1.75 GHz with the matrix
+// pipe busy 53 % and LDS 35 % of the clocks: 1060 TFLOP/s of bf16 products, where the bf16 kernels of this size are too.
 // The element-wise fetch of ragged steps lies in a loop of its own: a branch in every step around two kinds of loads made
 // the register sets meet behind it, with waits and spills, and cost 119-126 us.  Reading the fragments of a chunk under the
 // products of the one before it (twice the fragment registers, one barrier in the middle of a step) was slower, 147-156 us.
 //
 // Panels travel HBM -> registers as fp32, two steps ahead, are split once per workgroup and stored as three bf16 planes
-// (the conversion costs 5.5 vector instructions per element, spread between the MFMAs), 32 contraction elements per
+// (the conversion costs 6.5 vector instructions per element, spread between the MFMAs), 32 contraction elements per
 // step, double-buffered in LDS.  KMAJOR operands: [row][64 bytes], 16-byte chunks XOR-swizzled; MNMAJOR: [k][rows], read
 // through ds_read_b64_tr_b16.  Rows may start at any element: a buffer load needs 4-byte alignment.  What
 // lies past the operand's end reads as zero (buffer descriptors), and the last step, whose vectors may hold elements of
@@ -29,8 +39,14 @@ __device__ __forceinline__ uint32_t gs_pk(float a, float b) {
     const gs_f32x2 f = {a, b};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
 }
-// two values -> their h, m and l parts, packed
+// Operands are split as 2^16 times their value, so accumulators hold 2^32 times the product.
+constexpr int GS_PLAIN_K = 4;        // contractions up to this length are left to the fp32 instructions
+constexpr float GS_SCALE = 65536.f, GS_UNSCALE = 1.f / (65536.f * 65536.f);
+
+// two values -> the h, m and l parts of GS_SCALE times them, packed
 __device__ __forceinline__ void gs_split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+    x0 *= GS_SCALE;
+    x1 *= GS_SCALE;
     h = gs_pk(x0, x1);
     const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
     m = gs_pk(r0, r1);
@@ -150,6 +166,58 @@ struct GsCfg {
     static constexpr int WAVES_EU = (BLOCKS * NW + 3) / 4;
 };
 
+// acc = the wavefront's TMW x TNW MFMA tiles (from row `row0` of A, column `col0` of B) by the fp32 matrix instructions,
+// operands straight from memory: for the rare tiles whose values the split does not take.  Every lane of the wavefront calls it.
+template <int TMW, int TNW>
+__device__ __forceinline__ void gs_plain_product(const GemmArgs& g, f32x16 (&acc)[TNW][TMW], int row0, int col0, int kbeg, int kend,
+                                                 int lane) {
+    const int lr = lane & 31, lg = lane >> 5;
+    const float *pa[TMW], *pb[TNW];
+#pragma unroll
+    for (int t = 0; t < TMW; ++t) {
+        const int row = row0 + t * 32 + lr;
+        pa[t] = (const float*)g.a + (int64_t)(row < g.n ? row : g.n - 1) * g.a_row;
+    }
+#pragma unroll
+    for (int t = 0; t < TNW; ++t) {
+        const int col = col0 + t * 32 + lr;
+        pb[t] = (const float*)g.b + (int64_t)(col < g.m ? col : g.m - 1) * g.b_row;
+    }
+#pragma unroll
+    for (int i = 0; i < TNW; ++i)
+#pragma unroll
+        for (int j = 0; j < TMW; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+#pragma unroll 1
+    for (int64_t k0 = kbeg; k0 < kend; k0 += 16) {
+        f32x4 fa[2][TMW], fb[2][TNW];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int64_t k = k0 + c * 8 + lg * 4 + e;
+#pragma unroll
+                for (int t = 0; t < TMW; ++t) fa[c][t][e] = k < kend ? pa[t][k * g.a_k] : 0.f;
+#pragma unroll
+                for (int t = 0; t < TNW; ++t) fb[c][t][e] = k < kend ? pb[t][k * g.b_k] : 0.f;
+            }
+        // these instructions round after every product: a sum per 16 of them keeps the error of a long contraction low
+#pragma unroll
+        for (int i = 0; i < TNW; ++i)
+#pragma unroll
+            for (int j = 0; j < TMW; ++j) {
+                f32x16 part;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) part[e] = 0.f;
+                mma_chunk(part, fb[0][i], fa[0][j]);
+                mma_chunk(part, fb[1][i], fa[1][j]);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] += part[e];
+            }
+    }
+}
+
 template <int AMODE, int BMODE, typename C, bool MUL>
 __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(const GemmArgs g) {
     constexpr int BK = 32, TMW = C::TMW, TNW = C::TNW;
@@ -247,7 +315,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
     // no vector of either operand crosses a row's or the operand's end in any step
     const bool whole_vectors = ((AMODE != KMAJOR && BMODE != KMAJOR) || klen % BK == 0) && (AMODE == KMAJOR || !oa.cut) &&
                                (BMODE == KMAJOR || !ob.cut);
-    if (nk > 0) {
+    if (klen > GS_PLAIN_K) {
         constexpr std::bool_constant<true> WHOLE{};
         constexpr std::bool_constant<false> ANY{};
         load(I0, ANY, klen);
@@ -272,34 +340,18 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
         for (int j = 0; j < TMW; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] += low[i][j][e];
-    // An infinity (or a finite value that rounds to one) has no three parts and leaves NaN: such elements are formed again
-    // by multiply-adds, which give what the fp32 instructions would.
     float nan = 0.f;          // one multiply-add per element: 0, or NaN if one is not finite
 #pragma unroll
     for (int i = 0; i < TNW; ++i)
 #pragma unroll
         for (int j = 0; j < TMW; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) nan = fmaf(acc[i][j][e], 0.f, nan);
-    if (__builtin_expect(__any(nan != nan), 0)) {
-#pragma unroll
-        for (int i = 0; i < TNW; ++i)
-#pragma unroll
-            for (int j = 0; j < TMW; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int row = row0 + (wm * TMW + j) * 32 + (lane & 31);
-                    const int col = col0 + (wn * TNW + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-                    if (acc[i][j][e] != acc[i][j][e] && row < g.n && col < g.m) {
-                        const float* pa = (const float*)g.a + (int64_t)row * g.a_row;
-                        const float* pb = (const float*)g.b + (int64_t)col * g.b_row;
-                        float s = 0.f;
-#pragma unroll 1
-                        for (int64_t k = kbeg; k < kend && s == s; ++k) s = fmaf(pa[k * g.a_k], pb[k * g.b_k], s);   // NaN stays NaN
-                        acc[i][j][e] = s;
-                    }
-                }
-    }
+            for (int e = 0; e < 16; ++e) {
+                nan = fmaf(acc[i][j][e], 0.f, nan);
+                acc[i][j][e] *= GS_UNSCALE;
+            }
+    if (__builtin_expect(__any(nan != nan) || klen <= GS_PLAIN_K, 0))
+        gs_plain_product<TMW, TNW>(g, acc, row0 + wm * TMW * 32, col0 + wn * TNW * 32, kbeg, kend, lane);
     __syncthreads();
     gt_write_back<float, C, MUL>(g, acc, smem, row0, col0, z, wave, lane);
 }
