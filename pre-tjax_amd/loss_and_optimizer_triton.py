@@ -215,11 +215,12 @@ def adam_w_in_place(params, grads, lr, betas, epsilon, moments, i, weight_decay=
     low-precision copies) is refreshed from them."""
     master = params
     t = i + 1
+    # every nest is read at the parameters' places: one with a group or an entry missing raises, surplus entries are ignored
+    at = lambda nest: [nest[gi][pi] for gi, grp in enumerate(master) for pi in range(len(grp))]
     ps = [p for grp in master for p in grp]
-    gs = [g if g.is_contiguous() else g.contiguous() for grp in grads for g in grp]   # copies outlive the launch
-    ms = [m for grp in moments[0] for m in grp]
-    vs = [v for grp in moments[1] for v in grp]
-    ss = [x for grp in shadow for x in grp] if shadow is not None else None
+    gs = [g if g.is_contiguous() else g.contiguous() for g in at(grads)]              # copies outlive the launch
+    ms, vs = at(moments[0]), at(moments[1])
+    ss = at(shadow) if shadow is not None else None
     cnt = len(ps)
     if cnt:
         ns = [p.numel() for p in ps]
@@ -229,7 +230,7 @@ def adam_w_in_place(params, grads, lr, betas, epsilon, moments, i, weight_decay=
         if weight_decay_mask is None:
             wds = [weight_decay] * cnt
         else:
-            wds = [weight_decay if on else 0.0 for grp in weight_decay_mask for on in grp]
+            wds = [weight_decay if on else 0.0 for on in at(weight_decay_mask)]
         arr = lambda tensors: (ctypes.c_void_p * cnt)(*[x.data_ptr() for x in tensors])
         code = {torch.float32: 0, torch.bfloat16: 1}
         check(lib().ptj_adamw_multi(cnt, arr(ps), arr(ms), arr(vs), arr(gs), arr(ss) if ss is not None else None,

@@ -115,6 +115,61 @@ def test_init_adam_w_returns_accumulators_and_two_moment_nests(lo):
     assert grads[1][0].dtype == torch.bfloat16 and moments[0][1][0].dtype == torch.float32
 
 
+class _RecordedAdamW:
+    """Stands in for the library: keeps what ptj_adamw_multi was called with."""
+    def __init__(self):
+        self.calls = []
+
+    def ptj_adamw_multi(self, cnt, p, m, v, g, shadow, n, wd, *rest):
+        self.calls.append((list(n), list(wd), list(m), list(v), list(g), None if shadow is None else list(shadow)))
+        return 0
+
+
+@pytest.fixture
+def adamw(lo, monkeypatch):
+    rec = _RecordedAdamW()
+    monkeypatch.setattr(lo, "lib", lambda: rec)
+    monkeypatch.setattr(lo, "stream", lambda: None)
+
+    def run(**changed):
+        params = [[torch.ones(3, 2), torch.zeros(3)], [torch.ones(4)], [torch.ones(5), torch.ones(2)]]
+        like = lambda dt: [[torch.zeros_like(p, dtype=dt) for p in grp] for grp in params]
+        nests = {"grads": like(torch.float32), "m": like(torch.float32), "v": like(torch.float32),
+                 "shadow": like(torch.bfloat16), "mask": [[True, False], [False], [True, True]]}
+        for name, change in changed.items():
+            change(nests[name])
+        rec.calls.clear()
+        lo.adam_w_in_place(params, nests["grads"], 0.1, (0.9, 0.95), 1e-8, [nests["m"], nests["v"]], 0, 0.25, nests["mask"],
+                           shadow=nests["shadow"])
+        return nests, rec.calls
+    return run
+
+
+def test_adam_w_in_place_pairs_nests_entry_by_entry(adamw):
+    nests, calls = adamw()
+    flat = lambda nest: [t.data_ptr() for grp in nest for t in grp]
+    assert calls == [([6, 3, 4, 5, 2], [0.25, 0.0, 0.0, 0.25, 0.25], flat(nests["m"]), flat(nests["v"]), flat(nests["grads"]),
+                      flat(nests["shadow"]))]
+
+
+@pytest.mark.parametrize("nest", ["grads", "m", "v", "shadow", "mask"])
+@pytest.mark.parametrize("change", [lambda n: n[2].pop(), lambda n: n.pop(), lambda n: n[0].pop(),
+                                    lambda n: n[1].append(n[0].pop())])
+def test_adam_w_in_place_refuses_a_nest_with_missing_entries(adamw, nest, change):
+    """An entry or a group missing, at the end or before it, or moved to another group: nothing is updated."""
+    with pytest.raises(IndexError):
+        adamw(**{nest: change})
+
+
+@pytest.mark.parametrize("nest", ["grads", "m", "v", "shadow", "mask"])
+@pytest.mark.parametrize("change", [lambda n: n[2].append(n[0][0]), lambda n: n.append([n[0][0]]), lambda n: n[0].append(n[1][0])])
+def test_adam_w_in_place_ignores_surplus_entries(adamw, nest, change):
+    nests, calls = adamw(**{nest: change})
+    assert calls[0][:2] == ([6, 3, 4, 5, 2], [0.25, 0.0, 0.0, 0.25, 0.25])
+    at = lambda n: [n[i][j].data_ptr() for i, j in ((0, 0), (0, 1), (1, 0), (2, 0), (2, 1))]
+    assert list(calls[0][2:]) == [at(nests["m"]), at(nests["v"]), at(nests["grads"]), at(nests["shadow"])]
+
+
 def test_gradient_norm_helpers_on_cpu_tensors(lo):
     g = [[torch.tensor([3.0, 4.0]), torch.tensor([[12.0]])], [torch.tensor([0.0, 5.0])]]
     assert lo.grads_grps_l2norms(g) == pytest.approx([13.0, 5.0])
