@@ -54,7 +54,7 @@ double pair_us(const PtjLinearBwd& p, int ix, int iw, int cus) {
 double single_us(int64_t n, int64_t m, int64_t k, bool may_split, int cus) {
     const int ps = may_split ? choose_splits(n, m, k, 2, (size_t)-1) : 1;
     const GemmPlan plan = gemm_plan(n, m, k, 2, may_split ? (size_t)-1 : 0, ps, cus);
-    return plan.cfg >= 0 ? gp_tile_us(GT_COST[0][plan.cfg], n, m, k, 2, plan.splits, cus) : gp_persistent_us(n, m, k, 2, ps, cus);
+    return plan.cfg >= 0 ? gp_tile_us(GT_COST[0][plan.cfg], n, m, k, 2, plan.splits, cus) : gp_persistent_us(n, m, k, ps, cus);
 }
 
 // 0: two launches; else 1 + 3 * ix + iw over {small, wide, square}

@@ -74,10 +74,8 @@ inline double gp_tile_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int
 }
 
 // The persistent bf16 kernels: 20 us per round of 256x192 tiles at k = 768; a partial panel along K goes through the
-// element-wise loader.  In fp32 they are never the fastest (158 us against 120 for 4096x3072x768) and serve only operands
-// that the tile kernels do not take.
-inline double gp_persistent_us(int64_t n, int64_t m, int64_t k, int elt, int splits, int cus) {
-    if (elt != 2) return 1e30;
+// element-wise loader.
+inline double gp_persistent_us(int64_t n, int64_t m, int64_t k, int splits, int cus) {
     const int64_t work = gp_ceil(n, 256) * gp_ceil(m, 192) * splits, steps = gp_ceil(gp_ceil(k, splits), 64);
     const int64_t full = work / cus, rem = work % cus;
     const double rounds = (double)full + (rem ? 0.35 + 0.65 * (double)rem / cus : 0.0);
@@ -95,8 +93,11 @@ inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_by
                           int loose = ALIGNED) {
     const bool ragged = loose == LOOSE_OPERAND;
     GemmPlan best = {-1, 1, (int)k};
-    // within 8 % the persistent kernels are kept: in a training step their loads run on from product to product
-    double best_us = ragged ? 1e30 : (loose ? 2.0 : 0.92) * gp_persistent_us(n, m, k, elt, persistent_splits, cus);
+    // within 8 % the persistent kernels are kept: in a training step their loads run on from product to product.  In fp32 they
+    // are never the fastest (158 us against 120 for 4096x3072x768): they serve what the tile kernels do not take (operands
+    // without a unit stride, overlapping rows, pitches from 2^21 elements, or below 8 off the vector grid), and every other
+    // fp32 product gets a configuration.
+    double best_us = ragged || elt != 2 ? 1e30 : (loose ? 2.0 : 0.92) * gp_persistent_us(n, m, k, persistent_splits, cus);
     const int type = elt == 2 ? 0 : 1;
     for (int i = ragged ? RAGGED_FIRST[type] : 0; i < (ragged ? RAGGED_END[type] : GT_CONFIGS[type]); ++i) {
         const TileCost& c = GT_COST[type][i];

@@ -225,6 +225,7 @@ __device__ __forceinline__ void gt_item(const GemmArgs& g, int pid, int num_m, i
 
 // Write-back of a finished tile: 32 rows at a time through an fp32 staging area per wavefront (the K groups'
 // accumulators are added in group order on the way), then rows of 16-byte vectors with the epilogue applied.
+// PTJ_EPI_ACCUMULATE is gemm_direct.h's alone.
 // acc[tn][tm][i] of lane (lr, lg) is C[row0 + (wm * TMW + tm) * 32 + lr][col0 + wn * CW + tn * 32 + (i/4)*8 + lg*4 + i%4].
 template <typename T, typename C, bool MUL>
 __device__ __forceinline__ void gt_write_back(const GemmArgs& g, const f32x16 (&acc)[C::TNW][C::TMW], char* __restrict__ smem,
@@ -317,7 +318,7 @@ __device__ __forceinline__ void gt_write_back(const GemmArgs& g, const f32x16 (&
                     const bool act = deriv || g.epilogue == PTJ_EPI_BIAS_GELU;
                     T* p = (T*)g.c + (int64_t)row * g.c_rs + col;
                     T* pa = g.c_aux != nullptr ? (T*)g.c_aux + (int64_t)row * g.c_aux_rs + col : nullptr;
-                    const T* add = g.epilogue == PTJ_EPI_ACCUMULATE ? p : g.epilogue != PTJ_EPI_NONE ? (const T*)g.bias + col : nullptr;
+                    const T* add = g.epilogue != PTJ_EPI_NONE ? (const T*)g.bias + col : nullptr;
                     if (whole) {
                         if (add != nullptr) {
                             const LoosePack<T, VEC> b = *reinterpret_cast<const LoosePack<T, VEC>*>(add);
