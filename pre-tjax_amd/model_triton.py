@@ -721,7 +721,9 @@ def t_gpt2_tlayer_bkwd3_t(dloss_dx, acts, layer_params, y, mask, train=True, p_g
 
 
 # ---- the whole stack in one native call (csrc/gpt2.hip) -------------------------------------------
-NATIVE_STACK = True    # False: issue the stack one wrapper call at a time (same kernels, same bits)
+# False: issue the stack one wrapper call at a time.  The same bits, except for bf16 gradients of small batches: there the
+# native call forms the two products of a linear layer's backward in one launch, whose tiles add in another order.
+NATIVE_STACK = True
 
 
 class _StackActs:

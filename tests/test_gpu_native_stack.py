@@ -1,7 +1,8 @@
 """The transformer stack issued by one native call per direction against the same launches issued one
 wrapper call at a time, with and without dropout, with and without a mask tensor, and the forward that
-keeps no activations: bit-equal forwards, bit-equal gradients in fp32, and in bf16 gradients that differ
-by the rounding of products whose contraction is added in another order."""
+keeps no activations: bit-equal forwards, bit-equal gradients in fp32, and in bf16 gradients that differ by
+the rounding of products whose contraction is added in another order (the two products of a linear layer's
+backward in one launch take other tiles and no K split) and are no further from fp64."""
 import pytest
 import torch
 
@@ -35,8 +36,20 @@ def test_native_stack_equals_single_calls(mt, lo, monkeypatch, dtype, train, L, 
         assert a.shape == b.shape
         if i < 3 or dtype == torch.float32:
             assert torch.equal(a, b), i
-        else:
-            assert (a.double() - b.double()).norm() <= 1e-2 * b.double().norm(), i
+    if dtype == torch.float32:
+        return
+    p64 = [[p.double().cpu() for p in grp] for grp in params]
+    p64[1][0] = p64[1][0][:T]
+    m64 = mask.cpu() if masked else torch.tril(torch.ones(T, T, dtype=torch.bool)).expand(B, T, T)
+    want, _ = ogpt2.grad_loss(p64, y.cpu(), m64, train, seeds)
+    for i, (a, b, w) in enumerate(zip(runs[0][3:], runs[1][3:], [w for grp in want for w in grp])):
+        a, b = a[:w.shape[0]].double().cpu(), b[:w.shape[0]].double().cpu()
+        # A sum in another order moves a few stored values by one bf16 step; once every value behind it has been rounded
+        # anew, the two differ by two independent roundings of 2^-9 / sqrt(3): 1.6e-3 per stored tensor in between, six of
+        # them between the products of one block.  Measured: 1.9e-3 at most, against 5e-3 of error in either.
+        assert (a - b).norm() <= 6 ** 0.5 * 1.6e-3 * b.norm(), i
+        # neither order is the better one: 0.99 to 1.04 measured
+        assert (a - w).norm() <= 1.1 * (b - w).norm(), i
 
 
 def test_native_stack_steps_aside(mt, lo):
