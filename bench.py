@@ -387,7 +387,10 @@ def main():
             ev.append((s, e, 2.0 * n * m * k))
             return rc
 
-    mt.NATIVE_STACK = False      # one wrapper call per launch, so that every GEMM can be bracketed
+    # One wrapper call per launch, so that every GEMM can be bracketed; the timed steps above issue the stack as one native
+    # call per direction.  At this size both launch the same GEMM kernels on the same shapes (the native call merges
+    # products only where each alone would leave the chip half empty).
+    mt.NATIVE_STACK = False
     _lib._lib.ptj_gemm = Timed(orig_gemm, 4)
     _lib._lib.ptj_gemm_mul_colsum = Timed(orig_gemm_mul, 5)   # the product whose epilogue is the GELU backward
     for i in range(args.warmup + args.steps, args.warmup + 2 * args.steps):
@@ -477,7 +480,9 @@ def main():
                                      "rocprofv3 FETCH_SIZE / WRITE_SIZE runs scaled by a 1 GiB copy, read from "
                                      "profiles/%s; algorithmic minimum %.4g" % (os.path.basename(GEMM_TRAFFIC_FILE),
                                                                                  float((traffic_src or {}).get("algorithmic_bytes_per_launch", 0))),
-                     "kernel": "gemm_kernel<bf16> (all %d launches of a step: fwd, dX, dW)" % (n_launch // args.steps),
+                     "kernel": "gemm_kernel, gemm_direct_kernel and gemm_tile_kernel, bf16 (all %d launches of a step: fwd, "
+                               "dX, dW; events around single calls, in further steps issued call by call)"
+                               % (n_launch // args.steps),
                      "avg_launch_ms": round(gemm_ms / n_launch, 4),
                      "gflop_per_launch": round(gemm_flops / n_launch / 1e9, 2),
                      "gemm_ms_per_step": round(gemm_ms / args.steps, 3)},
