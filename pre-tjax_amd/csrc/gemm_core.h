@@ -58,8 +58,8 @@ struct GemmArgs {
     int vec_out;          // every output (C, pre-activation, partials) and the bias allow aligned 16-byte rows
     int epilogue;
     int leave_partials;   // tile kernels: the caller forms the K split's sums
-    // gemm_kernel<..., MUL = true> only: C = round(A.B) * mul element-wise, and the column sums of the
-    // stored C over each block of 64 rows go to colpart[row / 64][m]
+    // kernels with MUL = true only: C = round(A.B) * mul element-wise, and the column sums of the stored C over each
+    // block of rows that one wavefront owns (64; 32 to 64 by configuration in the tile kernels) go to colpart[row / block][m]
     const void* mul;
     int64_t mul_rs;
     float* colpart;
@@ -70,7 +70,7 @@ int launch_plain_f32(const GemmArgs& g, int splits, hipStream_t st);   // gemm_f
 // column sums per *mul_rows rows of C in g.colpart.
 int gemm_tile_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
 int gemm_tile_launch_f32(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
-// gemm_ragged.hip: bf16 operands without 16-byte alignment, configuration RAGGED_BF16 + cfg of gemm_plan.h
+// gemm_ragged.hip: bf16 operands without 16-byte alignment, configuration RAGGED_FIRST[0] + cfg of gemm_plan.h
 int gemm_ragged_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
 int gemm_tile_mul_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipStream_t st);
 int gemm_tile_mul_launch_f32(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipStream_t st);

@@ -6,10 +6,11 @@
 // The choice minimises a time estimate,
 //     start + rounds * (K steps * step + finish)  [+ second stage of a K split],
 // where a round is one workgroup in every slot (256 CUs x workgroups per CU).  start, step and finish
-// (microseconds) are fitted per kernel to timings of 11 products of GPT-2's feature widths at 64 to 8192
-// tokens in all operand layouts (launches replayed from a graph, operands rotating over 200 MB): the
-// estimate is within 10 % of the measurement on average, and the kernel it picks within 1.2 % of the
-// best one.  The kernels for unaligned bf16 operands: 30 products with odd sizes up to 4001, and the LM head's.
+// (microseconds) are fitted per kernel to timings of the 11 products of a GPT-2 small block, forward, dX and dW
+// (launches replayed from a graph, operands rotating over 200 MB).  Checked on these at eight token counts from 64
+// to 8192 and both storage types, against every kernel and K split within twice the lowest estimate: the estimate
+// is off by 7 % (bf16) and 6 % (fp32) on average, and the pick is 0.4 % slower than the best one on average and
+// 8 % at worst.  The kernels for unaligned bf16 operands are fitted to products with odd sizes up to 4001.
 #pragma once
 #include "common.h"
 
