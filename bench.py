@@ -481,7 +481,7 @@ def main():
                                      "rocprofv3 FETCH_SIZE / WRITE_SIZE runs scaled by a 1 GiB copy, read from "
                                      "profiles/%s; algorithmic minimum %.4g" % (os.path.basename(GEMM_TRAFFIC_FILE),
                                                                                  float((traffic_src or {}).get("algorithmic_bytes_per_launch", 0))),
-                     "kernel": "gemm_kernel, gemm_direct_kernel and gemm_tile_kernel, bf16 (all %d launches of a step: fwd, "
+                     "kernel": "gemm_ring_kernel and gemm_tile_kernel, bf16 (all %d launches of a step: fwd, "
                                "dX, dW; events around single calls, in further steps issued call by call)"
                                % (n_launch // args.steps),
                      "avg_launch_ms": round(gemm_ms / n_launch, 4),

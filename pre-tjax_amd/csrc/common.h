@@ -195,6 +195,18 @@ __device__ __forceinline__ float gelu_f(float x) {
     const float e = __builtin_amdgcn_exp2f(x * fmaf(x * x, c3, c1));
     return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
+// Both from one exponential: e = exp(-2z), s = 1 / (1 + e), 1 - s = e s.  e may overflow to infinity, where s is 0 and the
+// product is kept from inf * 0 by the largest finite e.
+__device__ __forceinline__ void gelu_both_f(float x, float& y, float& dy) {
+    constexpr float k = 0.7978845608028654f, l2e = 1.4426950408889634f;
+    constexpr float c1 = -2.0f * l2e * k, c3 = -2.0f * l2e * k * 0.044715f;
+    const float x2 = x * x;
+    const float e = __builtin_amdgcn_exp2f(x * fmaf(x2, c3, c1));
+    const float s = __builtin_amdgcn_rcpf(1.0f + e);
+    const float om = fminf(e, 3.4028235e38f) * s;
+    y = x * s;
+    dy = s * fmaf(om, x * fmaf(x2, 6.0f * k * 0.044715f, 2.0f * k), 1.0f);
+}
 __device__ __forceinline__ float gelu_grad_f(float x) {
     constexpr float k = 0.7978845608028654f;
     const float x2 = x * x;

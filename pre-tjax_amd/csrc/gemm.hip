@@ -8,18 +8,17 @@ namespace {
 
 // gemm_plan through a small per-thread table: a training loop asks for the same few dozen products again and again,
 // and the estimate over all tile shapes and splits takes a microsecond.
-GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int persistent_splits, int loose) {
-    struct Entry { int64_t n, m, k; size_t ws; int elt, splits, cus, loose; GemmPlan plan; };
+GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int loose, int kernels = ANY_KERNEL) {
+    struct Entry { int64_t n, m, k; size_t ws; int elt, cus, loose, kernels; GemmPlan plan; };
     constexpr int ENTRIES = 128;
     static thread_local Entry table[ENTRIES] = {};
     const int cus = num_cus();
     const uint64_t h = ((uint64_t)n * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)m * 0xC2B2AE3D27D4EB4Full) ^
                        ((uint64_t)k * 0x165667B19E3779F9ull) ^ ((uint64_t)(ws_bytes + loose) * 0xD6E8FEB86659FD93ull);
     Entry& e = table[(h >> 40) % ENTRIES];
-    if (e.n != n || e.m != m || e.k != k || e.ws != ws_bytes || e.elt != elt || e.splits != persistent_splits || e.cus != cus ||
-        e.loose != loose)
-        e = {n, m, k, ws_bytes, elt, persistent_splits, cus, loose,
-             gemm_plan(n, m, k, elt, ws_bytes, persistent_splits, cus, loose)};
+    if (e.n != n || e.m != m || e.k != k || e.ws != ws_bytes || e.elt != elt || e.cus != cus || e.loose != loose ||
+        e.kernels != kernels)
+        e = {n, m, k, ws_bytes, elt, cus, loose, kernels, gemm_plan(n, m, k, elt, ws_bytes, cus, loose, kernels)};
     return e.plan;
 }
 
@@ -53,8 +52,6 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
     g.epilogue = epilogue;
     g.mul = nullptr; g.mul_rs = 0; g.colpart = nullptr;
     g.leave_partials = 0;
-    if (epilogue == PTJ_EPI_ACCUMULATE) workspace = nullptr;   // no K split: the partial sums would not see the stored C
-    int splits = workspace ? choose_splits(n, m, k, elt, workspace_bytes) : 1;
     int am = elt == 2 ? pick_mode<bf16>(a, a_rs, a_cs) : pick_mode<float>(a, a_rs, a_cs);
     int bm = elt == 2 ? pick_mode<bf16>(b, b_cs, b_rs) : pick_mode<float>(b, b_cs, b_rs);
     const bool ragged = am == GENERIC || bm == GENERIC;
@@ -66,24 +63,35 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
     bool outputs_aligned = ptj_aligned16(c) && c_rs % v == 0;
     if (c_pre) outputs_aligned = outputs_aligned && ptj_aligned16(c_pre) && c_pre_rs % v == 0;
     if (bias) outputs_aligned = outputs_aligned && (reinterpret_cast<uintptr_t>(bias) % (4 * (size_t)elt)) == 0;
-    GemmPlan plan = {-1, 1, 0};
-    if (epilogue != PTJ_EPI_ACCUMULATE && gt_eligible(g, am, bm, ragged ? 8 : 1))
-        plan = cached_plan(n, m, k, elt, workspace && ptj_aligned16(workspace) ? workspace_bytes : 0, splits,
-                           ragged ? LOOSE_OPERAND : outputs_aligned ? ALIGNED : LOOSE_OUTPUT);
-    int64_t kps = k;
-    if (plan.cfg >= 0) {
-        splits = plan.splits;
-        kps = plan.kps;
-    } else if (splits > 1) {
-        kps = ((k + splits - 1) / splits + bk - 1) / bk * bk;
-        splits = (int)((k + kps - 1) / kps);
+    const bool aligned_ws = workspace && ptj_aligned16(workspace);
+    const int loose = ragged ? LOOSE_OPERAND : outputs_aligned ? ALIGNED : LOOSE_OUTPUT;
+    GemmPlan plan = {-1, 1, 0, 0, 1, 0, 0.0};
+    if (epilogue == PTJ_EPI_ACCUMULATE) {
+        // only the ring kernels start their accumulators from the stored C
+        if (ragged || (am == KMAJOR && bm == KMAJOR) || !outputs_aligned || k == 0 || k % 64 != 0 || !ring_eligible(g, am, bm))
+            return ptj_set_error(PTJ_ERR_INVALID, "gemm: the accumulating epilogue needs a transposed 16-byte aligned "
+                                 "operand layout, k a multiple of 64 and vector-aligned C");
+        plan = cached_plan(n, m, k, elt, 0, loose, RING_ONLY);
+    } else if (gt_eligible(g, am, bm, ragged ? 8 : 1)) {
+        plan = cached_plan(n, m, k, elt, aligned_ws ? workspace_bytes : 0, loose);
+    } else if (elt == 2 && !ragged && ring_eligible(g, am, bm)) {
+        plan = cached_plan(n, m, k, elt, aligned_ws ? workspace_bytes : 0, loose, RING_ONLY);
+    }
+    int splits = plan.splits;
+    int64_t kps = plan.cfg >= 0 ? plan.kps : k;
+    g.tail_first = plan.tail_first; g.tail_splits = plan.tail_splits; g.tail_kps = plan.tail_kps;
+    if (plan.cfg < 0) {
+        splits = workspace ? choose_splits(n, m, k, elt, workspace_bytes) : 1;
+        if (splits > 1) {
+            kps = ((k + splits - 1) / splits + bk - 1) / bk * bk;
+            splits = (int)((k + kps - 1) / kps);
+        } else if (aligned_ws) {
+            choose_tail_split(n, m, k, elt, workspace_bytes, &g.tail_first, &g.tail_splits, &g.tail_kps);
+        }
     }
     if (kps < 1) kps = bk;  // k == 0: one empty pass writes bias / zeros
     g.k_per_split = (int)kps;
     g.splits = splits;
-    g.tail_first = 0; g.tail_splits = 1; g.tail_kps = 0;
-    if (plan.cfg < 0 && splits == 1 && workspace && ptj_aligned16(workspace))
-        choose_tail_split(n, m, k, elt, workspace_bytes, &g.tail_first, &g.tail_splits, &g.tail_kps);
     g.vec_out = outputs_aligned && (splits <= 1 || (ptj_aligned16(workspace) && m % 4 == 0)) ? 1 : 0;
     g.partial = (splits > 1 || g.tail_splits > 1) ? (float*)workspace : nullptr;
     hipStream_t st = (hipStream_t)stream;
@@ -94,6 +102,8 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
             later->part = g.partial;
             later->splits = splits;
         }
+        if (plan.cfg == RING_FIRST) return ptj_gemm_detail::gemm_ring_full_launch(g, am, bm, st);
+        if (plan.cfg == RING_FIRST + 1) return ptj_gemm_detail::gemm_ring_narrow_launch(g, am, bm, st);
         if (ragged && dtype == PTJ_BF16)
             return ptj_gemm_detail::gemm_ragged_launch_bf16(g, plan.cfg - RAGGED_FIRST[0], am, bm, st);
         return dtype == PTJ_F32 ? ptj_gemm_detail::gemm_tile_launch_f32(g, plan.cfg, am, bm, st)
@@ -115,11 +125,11 @@ size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
     const int s = choose_splits(n, m, k, elt, (size_t)-1);
     int first, ts, tkps;
     size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
-    for (const int loose : {ALIGNED, LOOSE_OUTPUT, LOOSE_OPERAND}) {
-        const GemmPlan plan = cached_plan(n, m, k, elt, (size_t)-1, s, loose);
-        if (plan.cfg >= 0 && plan.splits > 1 && (size_t)plan.splits * n * m * sizeof(float) > need)
-            need = (size_t)plan.splits * n * m * sizeof(float);
-    }
+    for (const int loose : {ALIGNED, LOOSE_OUTPUT, LOOSE_OPERAND})
+        for (const int kernels : {ANY_KERNEL, RING_ONLY}) {
+            const size_t bytes = gp_workspace_bytes(cached_plan(n, m, k, elt, (size_t)-1, loose, kernels), n, m);
+            if (bytes > need) need = bytes;
+        }
     return need;
 }
 

@@ -1,9 +1,12 @@
-// Tile kernels, epilogues and launch logic of the MFMA GEMM, shared by the two translation units that
-// instantiate them: gemm.hip (ptj_gemm: every operand layout, bias / GELU epilogues, K splits) and
-// gemm_mul.hip (ptj_gemm_mul_colsum: the multiplying epilogue with column sums).  Everything here lives in
-// an unnamed namespace, so each unit gets its own copy of what it uses; the two units compile side by side.
+// Tile kernels, epilogues and launch logic of the MFMA GEMM, shared by the translation units that instantiate them.
+// Everything here lives in an unnamed namespace, so each unit gets its own copy of what it uses; the units compile
+// side by side.
 //
-// MFMA GEMM for gfx950: C[n,m] = sum_k A(n,k) B(k,m) (+bias[m]) (gelu), fp32 accumulation.
+// This file holds the register-staged persistent kernel, which takes operands of any strides and alignment.  Products whose
+// operands have a unit stride go to the kernels of gemm_ring.h and gemm_tile.h instead (gemm_plan.h), so what is left here
+// are strided, unaligned or overlapping operands.
+//
+// C[n,m] = sum_k A(n,k) B(k,m) (+bias[m]) (gelu), fp32 accumulation.
 //
 // Tiling: one 512-thread workgroup (8 wavefronts, 4 along rows x 2 along columns) owns a
 // 256x192 tile of C; each wavefront owns 64x96 = 2x3 MFMA tiles of 32x32
@@ -74,6 +77,12 @@ int gemm_tile_launch_f32(const GemmArgs& g, int cfg, int am, int bm, hipStream_t
 int gemm_ragged_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
 int gemm_tile_mul_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipStream_t st);
 int gemm_tile_mul_launch_f32(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipStream_t st);
+// gemm_ring_full.hip, gemm_ring_narrow.hip: the persistent bf16 kernels with 256x256 and 256x192 tiles, and with the
+// multiplying epilogue (gemm_ring_mul_*.hip: 128 and 64 rows of C per row of column sums)
+int gemm_ring_full_launch(const GemmArgs& g, int am, int bm, hipStream_t st);
+int gemm_ring_narrow_launch(const GemmArgs& g, int am, int bm, hipStream_t st);
+int gemm_ring_mul_full_launch(const GemmArgs& g, int am, int bm, hipStream_t st);
+int gemm_ring_mul_narrow_launch(const GemmArgs& g, int am, int bm, hipStream_t st);
 }  // namespace ptj_gemm_detail
 
 namespace {
@@ -483,6 +492,7 @@ __device__ __forceinline__ void gemm_store_block(const GemmArgs& g, const f32x16
 
 // Work item -> origin of its C tile: ids are regrouped so that the items of one XCD (id mod
 // 8) cover a contiguous range of tiles, then walked in groups of 8 tile-rows.
+template <int TBN = BN>
 __device__ __forceinline__ void tile_origin(int pid, int total, int num_m, int num_n, int& row0, int& col0) {
     {
         const int chunk = total >> 3, rem = total & 7, x = pid & 7;
@@ -496,7 +506,7 @@ __device__ __forceinline__ void tile_origin(int pid, int total, int num_m, int n
     const int tile_m = first_m + (pid % width) % gsz;
     const int tile_n = (pid % width) / gsz;
     row0 = tile_m * BM;
-    col0 = tile_n * BN;
+    col0 = tile_n * TBN;
 }
 
 // Epilogue of one tile.  acc[tn][tm][i] of lane (lr, lg) is
@@ -841,24 +851,24 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce4_kernel(const float* _
 }
 
 // Second stage for the K-split tiles of the last round: tile t (work item tail_first + t) =
-// epilogue(sum_z partial[t*splits + z]) in z order; partial tiles are dense BM x BN.
-template <typename T>
+// epilogue(sum_z partial[t*splits + z]) in z order; partial tiles are dense BM x TBN.
+template <typename T, int TBN>
 __global__ __launch_bounds__(256) void gemm_tail_reduce_kernel(const GemmArgs g) {
-    const int num_m = (g.n + BM - 1) / BM, num_n = (g.m + BN - 1) / BN;
+    const int num_m = (g.n + BM - 1) / BM, num_n = (g.m + TBN - 1) / TBN;
     const int t = blockIdx.x;
     int row0, col0;
-    tile_origin(g.tail_first + t, num_m * num_n, num_m, num_n, row0, col0);
-    const float* base = g.partial + (int64_t)t * g.tail_splits * (BM * BN);
+    tile_origin<TBN>(g.tail_first + t, num_m * num_n, num_m, num_n, row0, col0);
+    const float* base = g.partial + (int64_t)t * g.tail_splits * (BM * TBN);
     // four consecutive columns per thread: 16-byte loads of the partial tiles; a quad that lies
     // wholly inside C is stored as one vector when the outputs allow it
-    for (int q = blockIdx.y * 256 + threadIdx.x; q < BM * BN / 4; q += gridDim.y * 256) {
+    for (int q = blockIdx.y * 256 + threadIdx.x; q < BM * TBN / 4; q += gridDim.y * 256) {
         const int i = q * 4;
-        const int r = i / BN, c = i - r * BN;
+        const int r = i / TBN, c = i - r * TBN;
         const int row = row0 + r, col = col0 + c;
         if (row >= g.n || col >= g.m) continue;
         f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-        for (int z = 0; z < g.tail_splits; ++z) s += *reinterpret_cast<const f32x4*>(base + (int64_t)z * (BM * BN) + i);
+        for (int z = 0; z < g.tail_splits; ++z) s += *reinterpret_cast<const f32x4*>(base + (int64_t)z * (BM * TBN) + i);
         const bool whole = col + 4 <= g.m;
         if (g.epilogue != PTJ_EPI_NONE) {
 #pragma unroll
@@ -906,8 +916,15 @@ int launch_splitk_reduce(const GemmArgs& g, int splits, hipStream_t st) {
     return PTJ_OK;
 }
 
-#include "gemm_direct.h"
+template <typename T, int TBN>
+int launch_tail_reduce(const GemmArgs& g, int tiles, hipStream_t st) {
+    hipLaunchKernelGGL((gemm_tail_reduce_kernel<T, TBN>), dim3((unsigned)(tiles - g.tail_first), 12), dim3(256), 0, st, g);
+    PTJ_CHECK_LAUNCH();
+    return PTJ_OK;
+}
+
 #include "gemm_tile.h"
+#include "gemm_ring.h"
 
 template <typename T>
 int pick_mode(const void* p, int64_t s_row, int64_t s_k) {
@@ -938,29 +955,6 @@ int gemm_impl(GemmArgs g, int splits, hipStream_t st) {
     if (g.tail_splits > 1) work = g.tail_first + ((int64_t)num_m * num_n - g.tail_first) * g.tail_splits;
     const int cus = num_cus();
     dim3 grid((unsigned)(work < cus ? work : cus)), block(GEMM_THREADS);
-    bool direct = false;
-    if constexpr (sizeof(T) == 2) {
-        // Operands that need a transpose on their way to the MFMAs (.t() views: the dX and dW products) take the
-        // loop with asynchronous copies and transposing LDS reads.  Two K-major operands stay on the register-staged
-        // loop, whose third staging set gives their loads two steps to arrive: inside a training step it is the
-        // faster of the two for them (4.67 against 4.90 ms over the step's 49 forward products), back to back
-        // in a loop it is the slower one.
-        direct = !(am == KMAJOR && bm == KMAJOR) && dg_eligible(g, am, bm);
-        // only the loop with asynchronous copies starts its accumulators from the stored C
-        if (g.epilogue == PTJ_EPI_ACCUMULATE && !(direct && g.vec_out && splits == 1 && g.tail_splits <= 1))
-            return ptj_set_error(PTJ_ERR_INVALID, "gemm: the accumulating epilogue needs a transposed 16-byte aligned "
-                                 "operand layout, k a multiple of 64 and vector-aligned C");
-        if (direct) {
-#define DG_LAUNCH(AM, BMD) hipLaunchKernelGGL((gemm_direct_kernel<AM, BMD, MUL>), grid, block, 0, st, g)
-            switch (am * 3 + bm) {
-                case 1: DG_LAUNCH(KMAJOR, MNMAJOR); break;
-                case 3: DG_LAUNCH(MNMAJOR, KMAJOR); break;
-                default: DG_LAUNCH(MNMAJOR, MNMAJOR); break;
-            }
-#undef DG_LAUNCH
-        }
-    }
-    if (!direct) {
 #define GEMM_LAUNCH(AM, BMD) hipLaunchKernelGGL((gemm_kernel<T, AM, BMD, MUL>), grid, block, 0, st, g)
     if constexpr (MUL) {
         // the multiplying epilogue exists for vector-loadable operands only (the caller checks)
@@ -985,17 +979,12 @@ int gemm_impl(GemmArgs g, int splits, hipStream_t st) {
         }
     }
 #undef GEMM_LAUNCH
-    }
     PTJ_CHECK_LAUNCH();
     if (splits > 1) {
         const int rc = launch_splitk_reduce<T>(g, splits, st);
         if (rc != PTJ_OK) return rc;
     }
-    if (g.tail_splits > 1) {
-        hipLaunchKernelGGL((gemm_tail_reduce_kernel<T>), dim3((unsigned)(num_m * num_n - g.tail_first), 12), dim3(256), 0,
-                           st, g);
-        PTJ_CHECK_LAUNCH();
-    }
+    if (g.tail_splits > 1) return launch_tail_reduce<T, BN>(g, num_m * num_n, st);
     return PTJ_OK;
 }
 

@@ -69,9 +69,17 @@ int ptj_gemm_mul_colsum_later(const void* a, const void* b, const void* mul, voi
         g.stream = (g.vec_out && k >= 2 * bk && k % bk == 0) ? 1 : 0;
         const int am = dtype == PTJ_F32 ? pick_mode<float>(a, g.a_row, g.a_k) : pick_mode<bf16>(a, g.a_row, g.a_k);
         const int bm = dtype == PTJ_F32 ? pick_mode<float>(b, g.b_row, g.b_k) : pick_mode<bf16>(b, g.b_row, g.b_k);
-        GemmPlan plan = {-1, 1, 0};
-        if (gt_eligible(g, am, bm)) plan = gemm_plan(n, m, k, elt, 0, 1, num_cus());
-        if (plan.cfg >= 0) {
+        g.leave_partials = 0;
+        GemmPlan plan = {-1, 1, 0, 0, 1, 0, 0.0};
+        const bool tiles = gt_eligible(g, am, bm);
+        if (tiles || (elt == 2 && ring_eligible(g, am, bm)))
+            plan = gemm_plan(n, m, k, elt, 0, num_cus(), ALIGNED, tiles ? ANY_KERNEL : RING_ONLY);
+        if (plan.cfg >= RING_FIRST) {
+            mul_rows = plan.cfg == RING_FIRST ? RingFull::TMW * 32 : RingNarrow::TMW * 32;
+            const int rc = plan.cfg == RING_FIRST ? ptj_gemm_detail::gemm_ring_mul_full_launch(g, am, bm, st)
+                                                  : ptj_gemm_detail::gemm_ring_mul_narrow_launch(g, am, bm, st);
+            if (rc != PTJ_OK) return rc;
+        } else if (plan.cfg >= 0) {
             const int rc = dtype == PTJ_F32 ? ptj_gemm_detail::gemm_tile_mul_launch_f32(g, plan.cfg, am, bm, &mul_rows, st)
                                             : ptj_gemm_detail::gemm_tile_mul_launch_bf16(g, plan.cfg, am, bm, &mul_rows, st);
             if (rc != PTJ_OK) return rc;

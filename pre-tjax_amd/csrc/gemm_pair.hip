@@ -44,17 +44,15 @@ double pair_us(const PtjLinearBwd& p, int ix, int iw, int cus) {
     const int per_cu = cx.per_cu < cw.per_cu ? cx.per_cu : cw.per_cu;
     const int64_t slots = (int64_t)cus * per_cu;
     const bool packed = nx + nw > cus;                     // CUs with two workgroups: their steps take longer
-    const double tx = (double)gp_ceil(p.m, cx.bkt) * cx.step * (packed ? cx.shared : 1.0) + cx.finish;
-    const double tw = (double)gp_ceil(p.n, cw.bkt) * cw.step * (packed ? cw.shared : 1.0) + cw.finish;
+    const double tx = (double)gp_ceil(p.m, cx.bkt) * gp_step_us(cx, nx + nw, cus) * (packed ? cx.shared : 1.0) + cx.finish;
+    const double tw = (double)gp_ceil(p.n, cw.bkt) * gp_step_us(cw, nx + nw, cus) * (packed ? cw.shared : 1.0) + cw.finish;
     const double start = cx.start > cw.start ? cx.start : cw.start, longest = tx > tw ? tx : tw;
     if (nx + nw <= slots) return start + longest;
     return start + ((double)nx * tx + (double)nw * tw) / (double)slots + 0.5 * longest;
 }
 
 double single_us(int64_t n, int64_t m, int64_t k, bool may_split, int cus) {
-    const int ps = may_split ? choose_splits(n, m, k, 2, (size_t)-1) : 1;
-    const GemmPlan plan = gemm_plan(n, m, k, 2, may_split ? (size_t)-1 : 0, ps, cus);
-    return plan.cfg >= 0 ? gp_tile_us(GT_COST[0][plan.cfg], n, m, k, 2, plan.splits, cus) : gp_persistent_us(n, m, k, ps, cus);
+    return gemm_plan(n, m, k, 2, may_split ? (size_t)-1 : 0, cus).us;
 }
 
 // 0: two launches; else 1 + 3 * ix + iw over {small, wide, square}

@@ -11,8 +11,9 @@
 // tiles, and a K-major operand whose length is no multiple of 16 bytes has the surplus elements of
 // its last vector cleared in LDS.
 //
-// LDS layouts are those of mma_tile.h (KMAJOR: [row][128 bytes], XOR-swizzled) and gemm_direct.h
-// (MNMAJOR, 2-byte: [k][rows] read through ds_read_b64_tr_b16; 4-byte: [k][rows] read by ds_read_b32,
+// LDS layouts: KMAJOR as in mma_tile.h ([row][128 bytes], XOR-swizzled); MNMAJOR, 2-byte:
+// [k][rows] as it lies in memory, read through ds_read_b64_tr_b16 (sixteen lanes fetch a 4 (k) x 16 (rows) block and each
+// ends up with four consecutive k of one row; 4-byte: [k][rows] read by ds_read_b32,
 // four contraction indices per fragment).
 typedef uint32_t gt_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t gt_u32x4 __attribute__((ext_vector_type(4)));
@@ -25,6 +26,10 @@ template <int ROWS> __device__ __forceinline__ int gt_mn_swz(int k) {
     else if constexpr (ROWS == 192) return 2 * (k & 3);
     else if constexpr (ROWS == 256) return 10 * (k & 3);
     else return 0;
+}
+
+__device__ __forceinline__ uint32_t gt_lds_addr(const void* p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
 }
 
 // One MFMA operand fragment (16 bytes of contraction per lane) and how it is read from a stage.
@@ -225,7 +230,7 @@ __device__ __forceinline__ void gt_item(const GemmArgs& g, int pid, int num_m, i
 
 // Write-back of a finished tile: 32 rows at a time through an fp32 staging area per wavefront (the K groups'
 // accumulators are added in group order on the way), then rows of 16-byte vectors with the epilogue applied.
-// PTJ_EPI_ACCUMULATE is gemm_direct.h's alone.
+// PTJ_EPI_ACCUMULATE is gemm_ring.h's alone.
 // acc[tn][tm][i] of lane (lr, lg) is C[row0 + (wm * TMW + tm) * 32 + lr][col0 + wn * CW + tn * 32 + (i/4)*8 + lg*4 + i%4].
 template <typename T, typename C, bool MUL>
 __device__ __forceinline__ void gt_write_back(const GemmArgs& g, const f32x16 (&acc)[C::TNW][C::TMW], char* __restrict__ smem,
@@ -396,8 +401,8 @@ __device__ __forceinline__ void gt_tile(const GemmArgs& g, int pid, char* __rest
     constexpr int PT = oa.PER + ob.PER;
     char* const sA = smem;
     char* const sB = smem + S * C::A_STAGE;
-    oa.init(g.a, g.a_row, g.a_k, row0, g.n, kbeg, g.k, dg_lds_addr(sA), wm * TMW * 32, kg, tid);
-    ob.init(g.b, g.b_row, g.b_k, col0, g.m, kbeg, g.k, dg_lds_addr(sB), wn * TNW * 32, kg, tid);
+    oa.init(g.a, g.a_row, g.a_k, row0, g.n, kbeg, g.k, gt_lds_addr(sA), wm * TMW * 32, kg, tid);
+    ob.init(g.b, g.b_row, g.b_k, col0, g.m, kbeg, g.k, gt_lds_addr(sB), wn * TNW * 32, kg, tid);
 
     constexpr int CPS = C::CPS, NSET = 4 / CPS;
     static_assert(CPS == 2 || CPS == 4, "a panel is one or two register sets");

@@ -13,7 +13,6 @@ typedef GtCfg<64, 128, 1, 4, 1, 3, 4> GtWide;
 typedef GtCfg<128, 128, 2, 4, 1, 3, 4> GtSquare;
 typedef GtCfg<128, 128, 2, 4, 1, 2, 2> GtSquare2;   // two workgroups per CU
 typedef GtCfg<128, 192, 2, 2, 1, 2, 2> GtLarge;     // two workgroups per CU
-typedef GtCfg<256, 192, 4, 2, 1, 2, 2> GtFull;
 
 #include "gemm_split.h"
 
@@ -45,8 +44,7 @@ int gt_dispatch(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipSt
             case 2: return gt_run<T, MUL, GtWide>(g, am, bm, mul_rows, st);
             case 3: return gt_run<T, MUL, GtSquare>(g, am, bm, mul_rows, st);
             case 4: return gt_run<T, MUL, GtSquare2>(g, am, bm, mul_rows, st);
-            case 5: return gt_run<T, MUL, GtLarge>(g, am, bm, mul_rows, st);
-            default: return gt_run<T, MUL, GtFull>(g, am, bm, mul_rows, st);
+            default: return gt_run<T, MUL, GtLarge>(g, am, bm, mul_rows, st);
         }
     } else {
         switch (cfg) {
