@@ -93,7 +93,8 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
     g.k_per_split = (int)kps;
     g.splits = splits;
     g.vec_out = outputs_aligned && (splits <= 1 || (ptj_aligned16(workspace) && m % 4 == 0)) ? 1 : 0;
-    g.partial = (splits > 1 || g.tail_splits > 1) ? (float*)workspace : nullptr;
+    const size_t planes = plan.cfg == PLANES_CFG ? gp_planes_bytes(n, m, k) : 0;
+    g.partial = (splits > 1 || g.tail_splits > 1) ? (float*)((char*)workspace + planes) : nullptr;
     hipStream_t st = (hipStream_t)stream;
     if (plan.cfg >= 0) {
         g.stream = 0;
@@ -102,6 +103,7 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
             later->part = g.partial;
             later->splits = splits;
         }
+        if (plan.cfg == PLANES_CFG) return ptj_gemm_detail::gemm_planes_launch(g, (char*)workspace, st);
         if (plan.cfg == RING_FIRST) return ptj_gemm_detail::gemm_ring_full_launch(g, am, bm, st);
         if (plan.cfg == RING_FIRST + 1) return ptj_gemm_detail::gemm_ring_narrow_launch(g, am, bm, st);
         if (ragged && dtype == PTJ_BF16)
@@ -127,7 +129,7 @@ size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
     size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
     for (const int loose : {ALIGNED, LOOSE_OUTPUT, LOOSE_OPERAND})
         for (const int kernels : {ANY_KERNEL, RING_ONLY}) {
-            const size_t bytes = gp_workspace_bytes(cached_plan(n, m, k, elt, (size_t)-1, loose, kernels), n, m);
+            const size_t bytes = gp_workspace_bytes(cached_plan(n, m, k, elt, (size_t)-1, loose, kernels), n, m, k);
             if (bytes > need) need = bytes;
         }
     return need;

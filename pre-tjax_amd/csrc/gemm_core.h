@@ -66,6 +66,7 @@ struct GemmArgs {
     const void* mul;
     int64_t mul_rs;
     float* colpart;
+    const char *planes_a, *planes_b;   // gemm_planes.h: the operands' three bf16 parts
 };
 int launch_plain_f32(const GemmArgs& g, int splits, hipStream_t st);   // gemm_f32.hip
 // gemm_tile_bf16.hip, gemm_tile_f32.hip: configuration `cfg` of the one-tile-per-workgroup kernels (gemm_plan.h), with
@@ -73,6 +74,9 @@ int launch_plain_f32(const GemmArgs& g, int splits, hipStream_t st);   // gemm_f
 // column sums per *mul_rows rows of C in g.colpart.
 int gemm_tile_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
 int gemm_tile_launch_f32(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
+// gemm_planes.hip: fp32 operands of any strides, split into `planes` (gs_plane_bytes of either operand) ahead of the product
+int gemm_planes_launch(const GemmArgs& g, char* planes, hipStream_t st);
+int gemm_planes_mul_launch(const GemmArgs& g, char* planes, hipStream_t st);
 // gemm_ragged.hip: bf16 operands without 16-byte alignment, configuration RAGGED_FIRST[0] + cfg of gemm_plan.h
 int gemm_ragged_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, hipStream_t st);
 int gemm_tile_mul_launch_bf16(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipStream_t st);

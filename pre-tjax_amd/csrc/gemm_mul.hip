@@ -35,7 +35,8 @@ extern "C" size_t ptj_gemm_mul_colsum_workspace_bytes(int64_t n, int64_t m) {
 
 int ptj_gemm_mul_colsum_later(const void* a, const void* b, const void* mul, void* c, void* colsum, int64_t n, int64_t m,
                               int64_t k, int64_t a_rs, int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t mul_rs, int64_t c_rs,
-                              void* workspace, size_t workspace_bytes, int dtype, PtjPartialSums* later, hipStream_t st) {
+                              void* workspace, size_t workspace_bytes, void* scratch, size_t scratch_bytes, int dtype,
+                              PtjPartialSums* later, hipStream_t st) {
     PTJ_CHECK_ARG(n >= 0 && m >= 0 && k >= 0, "gemm_mul_colsum: negative dimension");
     PTJ_CHECK_ARG(n < (1ll << 31) && m < (1ll << 31) && k < (1ll << 31), "gemm_mul_colsum: dimension exceeds 31 bits");
     PTJ_CHECK_ARG(dtype == PTJ_F32 || dtype == PTJ_BF16, "gemm_mul_colsum: unknown dtype %d", dtype);
@@ -73,8 +74,12 @@ int ptj_gemm_mul_colsum_later(const void* a, const void* b, const void* mul, voi
         GemmPlan plan = {-1, 1, 0, 0, 1, 0, 0.0};
         const bool tiles = gt_eligible(g, am, bm);
         if (tiles || (elt == 2 && ring_eligible(g, am, bm)))
-            plan = gemm_plan(n, m, k, elt, 0, num_cus(), ALIGNED, tiles ? ANY_KERNEL : RING_ONLY);
-        if (plan.cfg >= RING_FIRST) {
+            plan = gemm_plan(n, m, k, elt, 0, num_cus(), ALIGNED, tiles ? ANY_KERNEL : RING_ONLY,
+                             scratch && ptj_aligned16(scratch) ? scratch_bytes : 0);
+        if (plan.cfg == PLANES_CFG) {
+            const int rc = ptj_gemm_detail::gemm_planes_mul_launch(g, (char*)scratch, st);
+            if (rc != PTJ_OK) return rc;
+        } else if (plan.cfg >= RING_FIRST) {
             mul_rows = plan.cfg == RING_FIRST ? RingFull::TMW * 32 : RingNarrow::TMW * 32;
             const int rc = plan.cfg == RING_FIRST ? ptj_gemm_detail::gemm_ring_mul_full_launch(g, am, bm, st)
                                                   : ptj_gemm_detail::gemm_ring_mul_narrow_launch(g, am, bm, st);
@@ -112,5 +117,5 @@ extern "C" int ptj_gemm_mul_colsum(const void* a, const void* b, const void* mul
                                    int64_t k, int64_t a_rs, int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t mul_rs, int64_t c_rs,
                                    void* workspace, size_t workspace_bytes, int dtype, void* stream) {
     return ptj_gemm_mul_colsum_later(a, b, mul, c, colsum, n, m, k, a_rs, a_cs, b_rs, b_cs, mul_rs, c_rs, workspace,
-                                     workspace_bytes, dtype, nullptr, (hipStream_t)stream);
+                                     workspace_bytes, nullptr, 0, dtype, nullptr, (hipStream_t)stream);
 }

@@ -123,6 +123,6 @@ int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, i
     if (rc != PTJ_OK) return rc;
     if (p.mul)
         return ptj_gemm_mul_colsum_later(p.d, p.w, p.mul, p.dx, p.colsum, n, k, m, m, 1, k, 1, k, k, p.colpart,
-                                         ptj_gemm_mul_colsum_workspace_bytes(n, k), dtype, later, st);
+                                         ptj_gemm_mul_colsum_workspace_bytes(n, k), scratch, scratch_bytes, dtype, later, st);
     return ptj_gemm(p.d, p.w, p.dx, nullptr, n, k, m, m, 1, k, 1, k, PTJ_EPI_NONE, nullptr, 0, scratch, scratch_bytes, dtype, st);
 }

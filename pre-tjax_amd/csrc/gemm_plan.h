@@ -54,8 +54,17 @@ constexpr TileCost RING_COST[RING_CONFIGS] = {
     {256, 192, 64, 1, 4.53, 1.030, 7.65, 1.0, 0.07},
 };
 
+// gemm_planes.h (fp32): start and step of the product with the launch of the split in the start; the split itself moves 10 bytes
+// an element.  Fitted to the same products at 256 to 8192 tokens (6 % rms; with it the picks are 0.5 % slower than the best).
+// Below about 2000 tokens, and for 768-wide outputs below 8192, the split costs more than it saves.
+constexpr int PLANES_CFG = 32;
+constexpr TileCost PLANES_COST = {128, 128, 16, 2, 8.66, 0.581, 0.0, 1.90, 0.0};
+inline size_t gp_planes_bytes(int64_t n, int64_t m, int64_t k) {
+    return ((size_t)(n + 31) / 32 + (size_t)(m + 31) / 32) * ((size_t)(k + 15) / 16) * 3072;
+}
+
 struct GemmPlan {
-    int cfg;      // configuration of gemm_tile.h or gemm_ring.h, or -1: the kernels for operands of any strides
+    int cfg;      // configuration of gemm_tile.h, gemm_ring.h or gemm_planes.h, or -1: the kernels for operands of any strides
     int splits;   // K splits
     int kps;      // contraction elements per split (a multiple of bkt)
     int tail_first, tail_splits, tail_kps;   // gemm_ring.h: the tiles from tail_first on (0: none) are K-split
@@ -113,8 +122,9 @@ inline double gp_ring_tail_us(const TileCost& c, int64_t n, int64_t m, int64_t k
 // product with another epilogue add in the same order.  `loose`: operands or outputs that do not come in aligned
 // 16-byte vectors; the ring kernels take such operands not at all and write such outputs element by element (twice the
 // time at k = 768), the tile kernels write any.
+// `planes_ws`: workspace for operands split ahead of a product without a K split, where partial sums may not take any.
 inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int cus, int loose = ALIGNED,
-                          int kernels = ANY_KERNEL) {
+                          int kernels = ANY_KERNEL, size_t planes_ws = 0) {
     const bool ragged = loose == LOOSE_OPERAND;
     GemmPlan best = {-1, 1, (int)k, 0, 1, 0, 1e30};
     const int type = elt == 2 ? 0 : 1;
@@ -130,6 +140,17 @@ inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_by
                 if (us < best.us) best = {i, s, (int)(s > 1 ? kps : k), 0, 1, 0, us};
             }
         }
+    if (elt == 4 && kernels == ANY_KERNEL) {
+        const double planes = (double)gp_planes_bytes(n, m, k), split = 1e-6 * (double)(n + m) * (double)k;
+        for (int s = 1; s <= 16; ++s) {
+            if (s > 1 && (k < 1024 || k / s < 256)) break;
+            if (!fits(planes + (s > 1 ? 4.0 * s * (double)n * (double)m : 0.0)) && !(s == 1 && planes <= (double)planes_ws)) break;
+            const int64_t kps = gp_ceil(gp_ceil(k, s), 32) * 32;
+            if (s > 1 && gp_ceil(k, kps) != s) continue;
+            const double us = gp_tile_us(PLANES_COST, n, m, k, elt, s, cus) + split;
+            if (us < best.us) best = {PLANES_CFG, s, (int)(s > 1 ? kps : k), 0, 1, 0, us};
+        }
+    }
     if (elt != 2 || ragged) return best;
     for (int i = 0; i < RING_CONFIGS; ++i) {
         const TileCost& c = RING_COST[i];
@@ -153,10 +174,11 @@ inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_by
     return best;
 }
 
-// workspace that a plan's partial sums take
-inline size_t gp_workspace_bytes(const GemmPlan& p, int64_t n, int64_t m) {
-    if (p.splits > 1) return (size_t)p.splits * (size_t)n * (size_t)m * sizeof(float);
-    if (p.cfg < RING_FIRST || p.tail_splits <= 1) return 0;
+// workspace that a plan takes: split operands, then partial sums
+inline size_t gp_workspace_bytes(const GemmPlan& p, int64_t n, int64_t m, int64_t k) {
+    const size_t planes = p.cfg == PLANES_CFG ? gp_planes_bytes(n, m, k) : 0;
+    if (planes > 0 || p.splits > 1) return planes + (p.splits > 1 ? (size_t)p.splits * (size_t)n * (size_t)m * sizeof(float) : 0);
+    if (p.tail_splits <= 1) return 0;
     const TileCost& c = RING_COST[p.cfg - RING_FIRST];
     return (size_t)(gp_ceil(n, c.tbm) * gp_ceil(m, c.tbn) - p.tail_first) * p.tail_splits * c.tbm * c.tbn * sizeof(float);
 }

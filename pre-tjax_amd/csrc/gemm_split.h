@@ -218,6 +218,33 @@ __device__ __forceinline__ void gs_plain_product(const GemmArgs& g, f32x16 (&acc
     }
 }
 
+// Both accumulators -> the tile of C: unscaled, formed again by the fp32 instructions where a sum is not finite, and written.
+template <typename C, bool MUL>
+__device__ __forceinline__ void gs_finish(const GemmArgs& g, f32x16 (&acc)[C::TNW][C::TMW], const f32x16 (&low)[C::TNW][C::TMW],
+                                          char* __restrict__ smem, int row0, int col0, int z, int kbeg, int kend, int wave, int wm,
+                                          int wn, int lane) {
+#pragma unroll
+    for (int i = 0; i < C::TNW; ++i)
+#pragma unroll
+        for (int j = 0; j < C::TMW; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] += low[i][j][e];
+    float nan = 0.f;          // one multiply-add per element: 0, or NaN if one is not finite
+#pragma unroll
+    for (int i = 0; i < C::TNW; ++i)
+#pragma unroll
+        for (int j = 0; j < C::TMW; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                nan = fmaf(acc[i][j][e], 0.f, nan);
+                acc[i][j][e] *= GS_UNSCALE;
+            }
+    if (__builtin_expect(__any(nan != nan) || kend - kbeg <= GS_PLAIN_K, 0))
+        gs_plain_product<C::TMW, C::TNW>(g, acc, row0 + wm * C::TMW * 32, col0 + wn * C::TNW * 32, kbeg, kend, lane);
+    __syncthreads();
+    gt_write_back<float, C, MUL>(g, acc, smem, row0, col0, z, wave, lane);
+}
+
 template <int AMODE, int BMODE, typename C, bool MUL>
 __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(const GemmArgs g) {
     constexpr int BK = 32, TMW = C::TMW, TNW = C::TNW;
@@ -334,26 +361,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
         if (whole_vectors) all_steps(WHOLE);
         else all_steps(ANY);
     }
-#pragma unroll
-    for (int i = 0; i < TNW; ++i)
-#pragma unroll
-        for (int j = 0; j < TMW; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] += low[i][j][e];
-    float nan = 0.f;          // one multiply-add per element: 0, or NaN if one is not finite
-#pragma unroll
-    for (int i = 0; i < TNW; ++i)
-#pragma unroll
-        for (int j = 0; j < TMW; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                nan = fmaf(acc[i][j][e], 0.f, nan);
-                acc[i][j][e] *= GS_UNSCALE;
-            }
-    if (__builtin_expect(__any(nan != nan) || klen <= GS_PLAIN_K, 0))
-        gs_plain_product<TMW, TNW>(g, acc, row0 + wm * TMW * 32, col0 + wn * TNW * 32, kbeg, kend, lane);
-    __syncthreads();
-    gt_write_back<float, C, MUL>(g, acc, smem, row0, col0, z, wave, lane);
+    gs_finish<C, MUL>(g, acc, low, smem, row0, col0, z, kbeg, kend, wave, wm, wn, lane);
 }
 
 template <typename C, bool MUL>

@@ -15,6 +15,7 @@ typedef GtCfg<128, 128, 2, 4, 1, 2, 2> GtSquare2;   // two workgroups per CU
 typedef GtCfg<128, 192, 2, 2, 1, 2, 2> GtLarge;     // two workgroups per CU
 
 #include "gemm_split.h"
+#include "gemm_planes.h"
 
 typedef GsCfg<128, 128, 4, 2> GsSquare;
 typedef GsCfg<64, 64, 2, 2> GsSmall;                // two workgroups per CU

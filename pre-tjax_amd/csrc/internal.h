@@ -52,7 +52,8 @@ inline size_t ptj_layernorm_bwd_parts_bytes(int64_t rows, int64_t cols) {
 // ptj_gemm_mul_colsum whose second stage goes to `later`.
 int ptj_gemm_mul_colsum_later(const void* a, const void* b, const void* mul, void* c, void* colsum, int64_t n, int64_t m,
                               int64_t k, int64_t a_rs, int64_t a_cs, int64_t b_rs, int64_t b_cs, int64_t mul_rs, int64_t c_rs,
-                              void* workspace, size_t workspace_bytes, int dtype, PtjPartialSums* later, hipStream_t st);
+                              void* workspace, size_t workspace_bytes, void* scratch, size_t scratch_bytes, int dtype,
+                              PtjPartialSums* later, hipStream_t st);
 
 // A product [n, m] as stored in `c`, or, where `part` is set, as fp32 partial sums of a K split that its consumer adds up:
 // round(sum_z part[z][n][m] + bias), in the order of z.
