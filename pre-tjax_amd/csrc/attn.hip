@@ -10,9 +10,9 @@
 // lane's registers), so P never travels through LDS.  The dK/dV pass computes S = Q K^T
 // with the same trick mirrored: a lane owns one key, dV^T = dO^T P and dK^T = Q^T dS.
 // The operand that must be read "across" its memory layout (V^T, K^T, Q^T, dO^T: row
-// index d, contraction along keys / queries) is transposed once while it is written to
-// LDS (MNMAJOR panel loader, quads paired so that the eight positions a lane holds of an
-// accumulator tile are one 16-byte chunk) and shared by the four wavefronts.
+// index d, contraction along keys / queries): 2-byte storage reads it out of the same rows
+// with transposing LDS reads, 4-byte storage transposes it once while it is written to LDS
+// (MNMAJOR panel loader); the four wavefronts share it.
 //
 // Softmax is evaluated in base 2 (scores pre-multiplied by log2(e)/sqrt(dh)); the saved
 // statistics `ms` are converted back to natural units.  Masked scores take the
@@ -102,31 +102,98 @@ __device__ __forceinline__ void load_row_frags(typename AT<T>::F (&f)[AT<T>::NC]
         f[c] = *reinterpret_cast<const typename AT<T>::F*>(reinterpret_cast<const char*>(row) + c * 32 + lg * 16);
 }
 
+// ---- tiles of 2-byte storage: copied straight into LDS --------------------------------------
+// Tiles go from memory into LDS without registers, two tiles ahead of their use, and lie there once.  Before, they went
+// through registers one tile ahead and lay in LDS a second time, transposed by vector permutes: dK/dV and dQ read Q, dO and
+// K from memory twice, and a third of the vector instructions of a step were the loader's.  Batch 8 x 1024 x 12 heads,
+// before / after (with the order of place()): forward 26.8 / 24.6 us, dQ 38.1 / 33.3, dK/dV 51.4 / 46.5; both in one launch,
+// batch 8 x 512: 35.9 / 30.8.  What bounds them now: a step's matrix and vector instructions hardly overlap (forward: 512
+// and 1000 clocks of 1670 per SIMD and step of 64 keys, batch 16 x 1024), and the chain of a step, LDS - product - softmax
+// - product, with the two or three wavefronts per SIMD that the registers allow.  Four wavefronts per SIMD (two tiles in LDS,
+// 128 registers) changed the forward and dQ by 1 %.
+//
+// A panel is 64 rows of 128 bytes as they lie in memory, its 16-byte pieces permuted inside each row by row_swizzle: eight
+// consecutive rows read one piece each without a bank conflict (RowFrags), and so do the four rows x 64 bytes that half
+// a wavefront fetches with a transposing read (TpFrags), so ONE panel serves both directions.
+constexpr int RING = 3;                   // tiles in LDS: one in use, two on their way
+constexpr int WAVE_COPY = 64 * 16;        // bytes of one copy of a wavefront: eight rows
+__device__ __forceinline__ int row_swizzle(int row) { return ((row & 2) << 1) | ((row & 4) >> 1) | (row & 1); }
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
+}
+// lane l's 16 (4) bytes at src land at lds + 16 l (4 l).  Inline assembly: the compiler would wait for every copy under way
+// before any LDS read.  (m0 is reserved; nothing else in this file uses it.)
+__device__ __forceinline__ void copy16_to_lds(const char* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+__device__ __forceinline__ void copy4_to_lds(const void* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+// One operand's tiles of 64 rows: wavefront w copies rows 8w .. 8w+7 and 32 + 8w .. of each.
+struct PanelCopy {
+    const char* src;     // the lane's piece of tile 0
+    int64_t half;        // bytes from a row to the row 32 further on
+    __device__ __forceinline__ void init(const bf16* __restrict__ p, int64_t row_stride, int tid) {
+        const int r = tid >> 3;
+        src = reinterpret_cast<const char*>(p + r * row_stride) + (((tid & 7) ^ row_swizzle(r)) << 4);
+        half = row_stride * 64;
+    }
+    __device__ __forceinline__ void issue(int tile, uint32_t panel, int wave) const {
+        const char* s = src + (int64_t)tile * 2 * half;
+        copy16_to_lds(s, panel + wave * WAVE_COPY);
+        copy16_to_lds(s + half, panel + 32 * 128 + wave * WAVE_COPY);
+    }
+};
+// Waits for this wavefront's copies, all but the newest N of them (everything unless `more` follow).
+template <int N> __device__ __forceinline__ void copies_landed(bool more) {
+    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+// The fragments are in their registers from here on (a compiler's wait inside the loop would wait for every copy as well).
+template <typename F, int N> __device__ __forceinline__ void frags_landed(F (&f)[N]) {
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+        u32x4_t v = __builtin_bit_cast(u32x4_t, f[c]);
+        asm volatile("" : "+v"(v)::"memory");
+        f[c] = __builtin_bit_cast(F, v);
+    }
+}
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ int next_slot(int slot) { return slot == RING - 1 ? 0 : slot + 1; }
+
 // s += panel_rows(j*32 + lr) x register_rows : panel rows become MFMA rows (m), the
 // lane's register row the MFMA column (n); contraction over the 64-element axis d.
-template <typename T>
-__device__ __forceinline__ void rows_x_frags_one(f32x16& s, const char* __restrict__ panels,
-                                                 const typename AT<T>::F (&f)[AT<T>::NC], int j, int lr, int lg) {
+// (2-byte storage: NJ sub-tiles' fragments are read together ahead of the products, RowFrags::read)
+template <typename T, int NJ> struct RowFrags {
+    __device__ __forceinline__ void read(const char* __restrict__, int, int, int) {}
+    __device__ __forceinline__ void mma(f32x16 (&s)[NJ], const char* __restrict__ panels, const typename AT<T>::F (&f)[AT<T>::NC],
+                                        int j0, int lr, int lg) const {
 #pragma unroll
-    for (int c = 0; c < AT<T>::NC; ++c) {
-        typename AT<T>::F a = read_frag<T>(panels + (c / 4) * PANEL, j * 32 + lr, (c % 4) * 2 + lg);
-        mma_chunk(s, a, f[c]);
+        for (int c = 0; c < AT<T>::NC; ++c)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                typename AT<T>::F a = read_frag<T>(panels + (c / 4) * PANEL, (j0 + j) * 32 + lr, (c % 4) * 2 + lg);
+                mma_chunk(s[j], a, f[c]);
+            }
     }
-}
-template <typename T>
-__device__ __forceinline__ void rows_x_frags(f32x16 (&s)[2], const char* __restrict__ panels,
-                                             const typename AT<T>::F (&f)[AT<T>::NC], int lr, int lg) {
+};
+template <int NJ> struct RowFrags<bf16, NJ> {
+    bf16x8 a[NJ][4];
+    __device__ __forceinline__ void read(const char* __restrict__ panel, int j0, int lr, int lg) {
 #pragma unroll
-    for (int c = 0; c < AT<T>::NC; ++c) {
-        const char* pp = panels + (c / 4) * PANEL;
-        const int q = (c % 4) * 2 + lg;
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            typename AT<T>::F a = read_frag<T>(pp, j * 32 + lr, q);
-            mma_chunk(s[j], a, f[c]);
-        }
+            for (int j = 0; j < NJ; ++j)
+                a[j][c] = *reinterpret_cast<const bf16x8*>(panel + ((j0 + j) * 32 + lr) * BKB + (((c * 2 + lg) ^ row_swizzle(lr)) << 4));
     }
-}
+    __device__ __forceinline__ void mma(f32x16 (&s)[NJ], const char* __restrict__, const bf16x8 (&f)[4], int, int, int) const {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) mma_chunk(s[j], a[j][c], f[c]);
+    }
+};
 
 // Eight floats -> eight bf16, converted two at a time (one packed conversion per pair).
 __device__ __forceinline__ bf16x8 pack8_bf16(const float* __restrict__ p) {
@@ -141,25 +208,11 @@ __device__ __forceinline__ bf16x8 pack8_bf16(const float* __restrict__ p) {
     return __builtin_bit_cast(bf16x8, w);
 }
 
-// o[t] += transposed_panel_rows(t*32 + lr) x p : contraction over the 32 positions of
+// o[t] += transposed panel (row t*32 + lr of the transpose) x p : contraction over the 32 positions of
 // sub-tile j whose values p[i] the lane holds in accumulator order
 // (position = j*32 + 8*(i/4) + 4*lg + i%4).
 __device__ __forceinline__ void tp_x_regs_one(f32x16 (&o)[2], const char* __restrict__ panels, const float (&p)[16],
-                                              int j, int lr, int lg, bf16) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const bf16x8 b = pack8_bf16(&p[8 * h]);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            // the panel was stored with paired quads: chunk 4j + 2h + lg holds exactly the eight
-            // positions of b, in the same order
-            const bf16x8 a = read_frag<bf16>(panels, t * 32 + lr, 4 * j + 2 * h + lg);
-            o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, o[t], 0, 0, 0);
-        }
-    }
-}
-__device__ __forceinline__ void tp_x_regs_one(f32x16 (&o)[2], const char* __restrict__ panels, const float (&p)[16],
-                                              int j, int lr, int lg, float) {
+                                              int j, int lr, int lg) {
     const char* pp = panels + j * PANEL;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -170,13 +223,41 @@ __device__ __forceinline__ void tp_x_regs_one(f32x16 (&o)[2], const char* __rest
             for (int b = 0; b < 4; ++b) o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[b], p[4 * a + b], o[t], 0, 0, 0);
         }
 }
-template <typename T>
-__device__ __forceinline__ void tp_x_regs(f32x16 (&o)[2], const char* __restrict__ panels, const float (&p)[2][16],
-                                          int lr, int lg, T tag) {
+// The panel's fragments are read ahead of the element-wise work that forms p (TpFrags::read), so that their way out of LDS is
+// hidden behind it.
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+template <typename T> struct TpFrags {
+    __device__ __forceinline__ void read(const char* __restrict__, int, int, int) {}
+    __device__ __forceinline__ void mma(f32x16 (&o)[2], const char* __restrict__ panels, const float (&p)[16], int j, int lr, int lg) const {
+        tp_x_regs_one(o, panels, p, j, lr, lg);
+    }
+};
+template <> struct TpFrags<bf16> {
+    bf16x8 a[2][2];
+    // transposing reads: sixteen lanes fetch four positions x 16 columns, each ends up with the four positions of its column;
+    // two of them make the eight positions that a lane holds of p, in the same order
+    __device__ __forceinline__ void read(const char* __restrict__ panel, int j, int lr, int lg) {
+        const int x = 4 * lg + ((lr & 15) >> 2);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) tp_x_regs_one(o, panels, p[j], j, lr, lg, tag);
-}
-
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int piece = t * 4 + 2 * (lr >> 4) + ((lr & 3) >> 1);
+                const char* pp = panel + (j * 32 + h * 16 + x) * BKB + ((piece ^ row_swizzle(x)) << 4) + 8 * (lr & 1);
+                const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(pp));
+                const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(pp + 8 * BKB));
+                a[h][t] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+    }
+    __device__ __forceinline__ void mma(f32x16 (&o)[2], const char* __restrict__, const float (&p)[16], int, int, int) const {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bf16x8 b = pack8_bf16(&p[8 * h]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[h][t], b, o[t], 0, 0, 0);
+        }
+    }
+};
 // Keep bits of one wavefront tile as wave-uniform (scalar) words.  Element (q, k) is kept
 // iff bit q + k of the batch-head's line is set.  In the kernels whose lanes are queries
 // (keys), the element in accumulator register i of sub-tile j sits at
@@ -185,9 +266,12 @@ __device__ __forceinline__ void tp_x_regs(f32x16 (&o)[2], const char* __restrict
 // decision of ONE register across the 64 lanes is two 32-bit windows of the line at the
 // constant offsets C and C + 4: a lane mask that the scalar unit extracts with two
 // shifts and that a single v_cndmask applies -- no per-lane bit arithmetic at all.
+// Words that no kernel here writes, at wave-uniform addresses: scalar loads, also between the inline assembly's memory clobbers.
+typedef __attribute__((address_space(4))) const uint32_t* uniform_words;
+__device__ __forceinline__ uniform_words as_uniform(const uint32_t* p) { return (uniform_words)(uintptr_t)p; }
 struct KeepWords { uint32_t d0, d1, d2; };
 __device__ __forceinline__ KeepWords load_keep_words(const uint32_t* __restrict__ line, int base) {
-    const uint32_t* p = line + (base >> 5);   // wave-uniform address: scalar loads
+    const uniform_words p = as_uniform(line + (base >> 5));
     KeepWords w;
     w.d0 = p[0];
     w.d1 = p[1];
@@ -328,8 +412,9 @@ __global__ __launch_bounds__(256) void attn_mask_classes_kernel(const uint32_t* 
 struct TileClasses { uint32_t c0, c1; };
 __device__ __forceinline__ TileClasses load_classes(const uint32_t* __restrict__ row, int t) {
     TileClasses c;
-    c.c0 = row[2 * t];
-    c.c1 = row[2 * t + 1];
+    const uniform_words p = as_uniform(row + 2 * t);
+    c.c0 = p[0];
+    c.c1 = p[1];
     return c;
 }
 
@@ -357,22 +442,37 @@ __device__ __forceinline__ void apply_causal(f32x16& s, int pos0) {
 }
 
 
+// Which tile and batch-head a workgroup of a grid (B*H, tiles) takes.  In dispatch order tiles go from long to short; every
+// second layer of 256 workgroups (one per CU) runs backwards, so that the CU with the longest of one layer gets the shortest of
+// the next instead of the longest again.  Only whole layers are turned, and a workgroup keeps its number modulo 8, hence its
+// XCD and the K and V in that one's L2.  Batch 8 x 1024 x 12 heads (three layers): forward 25.9 -> 24.6 us, dQ 35.2 -> 33.3;
+// 16 x 1024 (six layers): dQ 61.0 -> 59.0, dK/dV 86.3 -> 85.1, forward within its spread (43.9, 45.2).
+struct Place { int tile, bh; };
+__device__ __forceinline__ Place place() {
+    const uint32_t total = gridDim.x * gridDim.y;
+    uint32_t id = blockIdx.y * gridDim.x + blockIdx.x;
+    if ((id & 256) && (id | 255) < total) id ^= 31 << 3;
+    return {(int)(id / gridDim.x), (int)(id % gridDim.x)};
+}
+
 // ---- forward -------------------------------------------------------------------------
-// grid (B*H, ceil(T/128)); wave w owns queries q0 + 32w .. +31; K/V tiles of 64 keys.
+// grid (B*H, ceil(T/128)), see place(); wave w owns queries q0 + 32w .. +31; K/V tiles of 64 keys.
 template <typename T, bool HAS_MASK, bool TRAIN>
 // (2-byte storage: three workgroups per CU = three wavefronts per SIMD, 168 registers each)
 __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_kernel(const AttnArgs a) {
     typedef AT<T> X;
-    constexpr int STAGE = 2 * X::NP * PANEL;  // K panels then V^T panels
-    __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+    constexpr bool ASYNC = sizeof(T) == 2;
+    constexpr int STAGE = 2 * X::NP * PANEL;  // K panels then V (4-byte storage: V^T) panels
+    __shared__ __attribute__((aligned(16))) char smem[(ASYNC ? RING : 2) * STAGE];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lg = lane >> 5;
     // grid (B*H, T/128): the batch-head index is the fast dispatch dimension and the query
     // tiles go from the longest (last) to the shortest, so the workgroups that start last
     // are the cheapest ones (causal work per tile grows with the query position).
-    const int bh = blockIdx.x, bidx = bh / a.H, hidx = bh % a.H;
-    const int q0 = (gridDim.y - 1 - blockIdx.y) * 128;
+    const Place pl = place();
+    const int bh = pl.bh, bidx = bh / a.H, hidx = bh % a.H;
+    const int q0 = (gridDim.y - 1 - pl.tile) * 128;
     const int qw0 = q0 + wave * 32;
     const int query = qw0 + lr;
     const int qrow = query < a.T ? query : a.T - 1;
@@ -390,7 +490,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
     // Flat code (no closures) keeps the prefetch registers plain SSA values; the last step
     // re-fetches its own tile instead of branching.
     TileLoader<T, KMAJOR, 64, ATT_THREADS> lk[X::NP];
-    TileLoader<T, MNMAJOR, 64, ATT_THREADS, false, true> lv[X::NP];
+    TileLoader<T, MNMAJOR, 64, ATT_THREADS> lv[X::NP];
 #define FWD_FETCH(KT)                                                                  \
     _Pragma("unroll") for (int p = 0; p < X::NP; ++p) {                                \
         lk[p].load_fast(Kb, a.k_rs, 1, (KT) * 64, p * X::EPP, tid);                    \
@@ -402,12 +502,31 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
         lv[p].store(smem + (ST) * STAGE + (X::NP + p) * PANEL, tid);                   \
     }
 
-    FWD_FETCH(0)
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const uint32_t lds0 = lds_addr(smem);
+    PanelCopy ck, cv;
+#define FWD_COPY(KT, SLOT)                                                             \
+    {                                                                                  \
+        ck.issue(KT, lds0 + (SLOT) * STAGE, wave_u);                                   \
+        cv.issue(KT, lds0 + (SLOT) * STAGE + PANEL, wave_u);                           \
+    }
+    if constexpr (ASYNC) {
+        ck.init(Kb, a.k_rs, tid);
+        cv.init(Vb, a.v_rs, tid);
+        FWD_COPY(0, 0)
+        frags_landed(qf);
+        if (nkt > 1) FWD_COPY(1, 1)
+    } else FWD_FETCH(0)
     // keep-bit line of this batch-head and the wave's first query as scalars
     const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
-    const int qw0u = q0 + __builtin_amdgcn_readfirstlane(wave) * 32;
-    FWD_STASH(0)
-    __syncthreads();
+    const int qw0u = q0 + wave_u * 32;
+    if constexpr (ASYNC) {
+        copies_landed<4>(nkt > 1);
+        lds_barrier();
+    } else {
+        FWD_STASH(0)
+        __syncthreads();
+    }
 
     const float sc = a.scale * LOG2E;
     float m_run = M_START, m_true = M_START, l_run = 0.f;
@@ -427,9 +546,11 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
         crow = a.mask + 2 * (int64_t)a.B * G * a.T + ((int64_t)bidx * G + (qw0u >> 5)) * G;
         tc_next = load_classes(crow, 0);
     }
+    int st = 0;   // this tile's place in LDS
     for (int kt = 0; kt < nkt; ++kt) {
-        const int st = kt & 1;
-        FWD_FETCH(kt + 1 < nkt ? kt + 1 : kt)
+        if constexpr (ASYNC) {
+            if (kt + 2 < nkt) FWD_COPY(kt + 2, next_slot(next_slot(st)))
+        } else FWD_FETCH(kt + 1 < nkt ? kt + 1 : kt)
         // keep bits and classes of this tile were requested one step ago; request the next tile's now
         const KeepWords kw = kw_next;
         if constexpr (TRAIN) kw_next = load_keep_words(kline, qw0u + (kt + 1) * 64);
@@ -441,12 +562,19 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
         if (key0 <= qw0 + 31 && (!HAS_MASK || (tc.c0 | tc.c1) != TILE_HIDDEN)) {
             const char* kp = smem + st * STAGE;
             const char* vp = kp + X::NP * PANEL;
+            RowFrags<T, 2> ka;
+            ka.read(kp, 0, lr, lg);
+            if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
             f32x16 s[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) s[j][e] = 0.f;
-            rows_x_frags<T>(s, kp, qf, lr, lg);
+            ka.mma(s, kp, qf, 0, lr, lg);
+            TpFrags<T> va[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) va[j].read(vp, j, lr, lg);
+            if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
 
             if (key0 + 63 > qw0) {   // tile touches the diagonal for this wave
 #pragma unroll
@@ -455,7 +583,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
             if constexpr (HAS_MASK) {
                 // one word per key: the mask bits of the wave's 32 queries (wave-uniform loads), read
                 // only for a half whose tile is not already described by the causal pattern
-                const uint32_t* mw = a.mask + ((int64_t)bidx * (a.T >> 5) + (qw0u >> 5)) * a.T + key0;
+                const uniform_words mw = as_uniform(a.mask + ((int64_t)bidx * (a.T >> 5) + (qw0u >> 5)) * a.T + key0);
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     if ((j == 0 ? tc.c0 : tc.c1) == TILE_CAUSAL) continue;
@@ -503,12 +631,21 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
                 keep_apply<0>(p[0], kw);
                 keep_apply<1>(p[1], kw);
             }
-            tp_x_regs(o, vp, p, lr, lg, T());
+#pragma unroll
+            for (int j = 0; j < 2; ++j) va[j].mma(o, vp, p[j], j, lr, lg);
         }
         __builtin_amdgcn_sched_barrier(0);
-        FWD_STASH(st ^ 1)
-        __syncthreads();
+        if constexpr (ASYNC) {
+            copies_landed<4>(kt + 2 < nkt);
+            lds_barrier();
+            st = next_slot(st);
+        } else {
+            st ^= 1;
+            FWD_STASH(st)
+            __syncthreads();
+        }
     }
+#undef FWD_COPY
 #undef FWD_FETCH
 #undef FWD_STASH
 
@@ -530,35 +667,34 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
 // OWN_DELTA: delta = rowsum(dO * O) is formed here, from the dO rows on their way into LDS and the O rows beside
 // them, instead of being read from what the dQ pass stored.
 typedef float StatTile[3][64];            // m2, 1/l, delta of a query tile
-template <typename T, int N>
-__device__ __forceinline__ void store_delta(float* __restrict__ delta, const TileLoader<T, KMAJOR, 64, ATT_THREADS> (&ld)[N],
-                                            const TileLoader<T, KMAJOR, 64, ATT_THREADS> (&lo)[N], int tid) {
-    typedef TileLoader<T, KMAJOR, 64, ATT_THREADS> L;
-    typedef typename AT<T>::F F;
+// delta of row (tid >> 3) + 32 i from the 16-byte pieces x of dO and y of O: eight neighbouring lanes hold a row
+template <typename F>
+__device__ __forceinline__ float piece_dot(const F& x, const F& y) {
+    float part = 0.f;
 #pragma unroll
-    for (int i = 0; i < L::NV; ++i) {      // eight neighbouring lanes hold the 16-byte pieces of one row
-        float part = 0.f;
-#pragma unroll
-        for (int p = 0; p < N; ++p) {
-            const F x = __builtin_bit_cast(F, ld[p].r[i]), y = __builtin_bit_cast(F, lo[p].r[i]);
-#pragma unroll
-            for (int e = 0; e < L::VEC; ++e) part += (float)x[e] * (float)y[e];
-        }
-        part += __shfl_xor(part, 1, 64);
-        part += __shfl_xor(part, 2, 64);
-        part += __shfl_xor(part, 4, 64);
-        if ((tid & 7) == 0) delta[(tid >> 3) + L::RP * i] = part;
-    }
+    for (int e = 0; e < (int)(sizeof(F) / sizeof(x[0])); ++e) part += (float)x[e] * (float)y[e];
+    return part;
 }
-template <typename T> constexpr int dkdv_lds() { return 2 * 4 * AT<T>::NP * PANEL; }
+__device__ __forceinline__ void store_delta(float* __restrict__ delta, int i, float part, int tid) {
+    part += __shfl_xor(part, 1, 64);
+    part += __shfl_xor(part, 2, 64);
+    part += __shfl_xor(part, 4, 64);
+    if ((tid & 7) == 0) delta[(tid >> 3) + 32 * i] = part;
+}
+constexpr int RAW_STATS = 3 * 64 * 4;     // bytes of a query tile's saved maxima, sums and delta
+constexpr int dkdv_stage(bool own_delta) { return (own_delta ? 3 : 2) * PANEL + RAW_STATS; }   // 2-byte storage: Q, dO (, O), statistics
+template <typename T, bool OWN_DELTA> constexpr int dkdv_lds() {
+    return sizeof(T) == 2 ? RING * dkdv_stage(OWN_DELTA) : 2 * 4 * AT<T>::NP * PANEL;
+}
 template <typename T, bool HAS_MASK, bool TRAIN, bool OWN_DELTA>
-__device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_tile, char* smem, StatTile* sstat) {
+__device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, const int key_tile, char* smem, StatTile* sstat) {
     typedef AT<T> X;
-    constexpr int STAGE = 4 * X::NP * PANEL;  // Q, dO, Q^T, dO^T
+    constexpr bool ASYNC = sizeof(T) == 2;
+    constexpr int STAGE = ASYNC ? dkdv_stage(OWN_DELTA) : 4 * X::NP * PANEL;  // 4-byte storage: Q, dO, Q^T, dO^T
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lg = lane >> 5;
-    const int bh = blockIdx.x, bidx = bh / a.H, hidx = bh % a.H;
+    const int bidx = bh / a.H, hidx = bh % a.H;
     const int key0 = key_tile * 128;
     const int kw0 = key0 + wave * 32;
     const int key = kw0 + lr;
@@ -577,7 +713,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_t
     const int qt0 = key0 / 64, nqt = a.T / 64;
 
     TileLoader<T, KMAJOR, 64, ATT_THREADS> lq[X::NP], ld[X::NP], lo[OWN_DELTA ? X::NP : 1];
-    TileLoader<T, MNMAJOR, 64, ATT_THREADS, false, true> lqt[X::NP], ldt[X::NP];
+    TileLoader<T, MNMAJOR, 64, ATT_THREADS> lqt[X::NP], ldt[X::NP];
     float st_m = 0.f, st_l = 1.f, st_d = 0.f;
     // 2-byte storage: 1/l goes into the exponent (p = 2^(s - m - log2 l)), one multiplication less
     // per element.  A row without a visible key (saved l = 0) gets m = 0 and 1/l = 0 instead: all
@@ -609,12 +745,17 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_t
         }                                                                              \
         if (tid < 64) {                                                                \
             const bool none__ = st_l == 0.f;                                           \
-            const float m2__ = FOLD_L ? fmaf(st_m, LOG2E, __builtin_amdgcn_logf(st_l)) : st_m * LOG2E; \
-            sstat[ST][0][tid] = none__ ? 0.f : m2__;                                   \
+            sstat[ST][0][tid] = none__ ? 0.f : st_m * LOG2E;                           \
             sstat[ST][1][tid] = none__ ? 0.f : 1.0f / st_l;                            \
             if constexpr (!OWN_DELTA) sstat[ST][2][tid] = st_d;                        \
         }                                                                              \
-        if constexpr (OWN_DELTA) store_delta<T>(sstat[ST][2], ld, lo, tid);            \
+        if constexpr (OWN_DELTA)                                                       \
+            _Pragma("unroll") for (int i = 0; i < 2; ++i) {                            \
+                float part__ = 0.f;                                                    \
+                _Pragma("unroll") for (int p = 0; p < X::NP; ++p)                      \
+                    part__ += piece_dot(__builtin_bit_cast(typename X::F, ld[p].r[i]), __builtin_bit_cast(typename X::F, lo[p].r[i])); \
+                store_delta(sstat[ST][2], i, part__, tid);                             \
+            }                                                                          \
     }
 
     f32x16 dk[2], dv[2];
@@ -623,16 +764,65 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_t
 #pragma unroll
         for (int e = 0; e < 16; ++e) dk[t][e] = dv[t][e] = 0.f;
 
-    if (qt0 < nqt) {
-        KV_FETCH(qt0)
-        KV_STASH(0)
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const uint32_t lds0 = lds_addr(smem);
+    PanelCopy cq, cd, co;
+    // The statistics come with the tile; the first wavefront copies them, converts them once they have landed
+    // and leaves them in sstat for the workgroup.  Each wavefront waits for its own copies only: the rows of
+    // dO and O that it multiplies for delta are those that it copied itself.
+    constexpr int RAW = (OWN_DELTA ? 3 : 2) * PANEL, COPIES = OWN_DELTA ? 6 : 4, STAT_COPIES = OWN_DELTA ? 2 : 3;
+#define KV_COPY(QT, SLOT)                                                              \
+    {                                                                                  \
+        const uint32_t to__ = lds0 + (SLOT) * STAGE;                                   \
+        cq.issue(QT, to__, wave_u);                                                    \
+        cd.issue(QT, to__ + PANEL, wave_u);                                            \
+        if constexpr (OWN_DELTA) co.issue(QT, to__ + 2 * PANEL, wave_u);               \
+        if (wave_u == 0) {                                                             \
+            copy4_to_lds(a.ms + stat0 + (QT) * 64, to__ + RAW);                        \
+            copy4_to_lds(a.ls + stat0 + (QT) * 64, to__ + RAW + 256);                  \
+            if constexpr (!OWN_DELTA) copy4_to_lds(a.delta + stat0 + (QT) * 64, to__ + RAW + 512); \
+        }                                                                              \
     }
-    __syncthreads();
+#define KV_LAND(SLOT, PAR, MORE)                                                       \
+    {                                                                                  \
+        const char* in__ = smem + (SLOT) * STAGE;                                      \
+        if (wave_u == 0) {                                                             \
+            copies_landed<COPIES + STAT_COPIES>(MORE);                                 \
+            const float* raw__ = reinterpret_cast<const float*>(in__ + RAW);           \
+            const float m__ = raw__[lane], l__ = raw__[64 + lane];                     \
+            const bool none__ = l__ == 0.f;                                            \
+            sstat[PAR][0][lane] = none__ ? 0.f : fmaf(m__, LOG2E, __builtin_amdgcn_logf(l__)); \
+            if constexpr (!OWN_DELTA) sstat[PAR][2][lane] = raw__[128 + lane];         \
+        } else copies_landed<COPIES>(MORE);                                            \
+        if constexpr (OWN_DELTA)                                                       \
+            _Pragma("unroll") for (int i = 0; i < 2; ++i) {                            \
+                const char* x__ = in__ + PANEL + i * 32 * BKB + tid * 16;              \
+                store_delta(sstat[PAR][2], i, piece_dot(*reinterpret_cast<const bf16x8*>(x__),  \
+                            *reinterpret_cast<const bf16x8*>(x__ + PANEL)), tid);      \
+            }                                                                          \
+        lds_barrier();                                                                 \
+    }
+    if constexpr (ASYNC) {
+        cq.init(Qb, a.q_rs, tid);
+        cd.init(dOb, a.do_rs, tid);
+        if constexpr (OWN_DELTA) co.init(Ob, a.o_rs, tid);
+        KV_COPY(qt0, 0)
+        frags_landed(kf);
+        frags_landed(vf);
+        if (qt0 + 1 < nqt) KV_COPY(qt0 + 1, 1)
+        KV_LAND(0, 0, qt0 + 1 < nqt)
+    } else {
+        if (qt0 < nqt) {
+            KV_FETCH(qt0)
+            KV_STASH(0)
+        }
+        __syncthreads();
+    }
 
     const float sc = a.scale * LOG2E;
     // keep-bit line of this batch-head and the wave's first key as scalars
     const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
-    const int kw0u = key0 + __builtin_amdgcn_readfirstlane(wave) * 32;
+    const int kw0u = key0 + wave_u * 32;
     KeepWords kw_next;
     if constexpr (TRAIN) kw_next = load_keep_words(kline, kw0u + qt0 * 64);
     // tile classes of the wave's 32 keys against every 32-query group (explicit mask only)
@@ -643,9 +833,12 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_t
         crow = a.mask + 2 * (int64_t)a.B * G * a.T + (int64_t)a.B * G * G + ((int64_t)bidx * G + (kw0u >> 5)) * G;
         if (qt0 < nqt) tc_next = load_classes(crow, qt0);
     }
+    int slot = 0;   // this tile's place in LDS
     for (int qt = qt0; qt < nqt; ++qt) {
         const int st = (qt - qt0) & 1;
-        KV_FETCH(qt + 1 < nqt ? qt + 1 : qt)
+        if constexpr (ASYNC) {
+            if (qt + 2 < nqt) KV_COPY(qt + 2, next_slot(next_slot(slot)))
+        } else KV_FETCH(qt + 1 < nqt ? qt + 1 : qt)
         const KeepWords kw = kw_next;   // requested one step ago
         if constexpr (TRAIN) kw_next = load_keep_words(kline, kw0u + (qt + 1) * 64);
         const TileClasses tc = tc_next;
@@ -653,7 +846,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_t
         __builtin_amdgcn_sched_barrier(0);
         const int q0 = qt * 64;
         if (q0 + 63 >= kw0) {   // some query of the tile sees some key of the wave
-            const char* base = smem + st * STAGE;
+            const char* base = smem + slot * STAGE;
             // The two 32-query halves are processed one after the other: half the live
             // accumulators, which keeps two wavefronts per SIMD resident.
 #pragma unroll
@@ -661,18 +854,28 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_t
                 if (q0 + j * 32 + 31 < kw0) continue;   // every query of this half precedes the wave's keys
                 const uint32_t cls = j == 0 ? tc.c0 : tc.c1;
                 if (HAS_MASK && cls == TILE_HIDDEN) continue;
-                f32x16 s, dp;
+                RowFrags<T, 1> qa, da;
+                qa.read(base, j, lr, lg);
+                da.read(base + X::NP * PANEL, j, lr, lg);
+                if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
+                f32x16 s1[1], dp1[1];
 #pragma unroll
-                for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
-                rows_x_frags_one<T>(s, base, kf, j, lr, lg);                      // S  [query][key]
-                rows_x_frags_one<T>(dp, base + X::NP * PANEL, vf, j, lr, lg);     // dP [query][key]
+                for (int e = 0; e < 16; ++e) s1[0][e] = dp1[0][e] = 0.f;
+                qa.mma(s1, base, kf, j, lr, lg);                                  // S  [query][key]
+                da.mma(dp1, base + X::NP * PANEL, vf, j, lr, lg);                 // dP [query][key]
+                f32x16 &s = s1[0], &dp = dp1[0];
+                const char *qt_panel = base + (ASYNC ? 0 : 2 * X::NP * PANEL), *dot_panel = base + (ASYNC ? 1 : 3 * X::NP) * PANEL;
+                TpFrags<T> dot, qtr;
+                dot.read(dot_panel, j, lr, lg);
+                qtr.read(qt_panel, j, lr, lg);
+                if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
 
                 const bool diag = q0 + j * 32 < kw0 + 31;
                 if (diag) apply_causal<false>(s, key - q0 - j * 32 - lg * 4);
                 if (HAS_MASK && cls != TILE_CAUSAL) {
                     // one word per query: the mask bits of the wave's 32 keys (wave-uniform loads)
-                    const uint32_t* mw = a.mask + (int64_t)a.B * (a.T >> 5) * a.T +
-                                         ((int64_t)bidx * (a.T >> 5) + (kw0u >> 5)) * a.T + q0 + j * 32;
+                    const uniform_words mw = as_uniform(a.mask + (int64_t)a.B * (a.T >> 5) * a.T +
+                                         ((int64_t)bidx * (a.T >> 5) + (kw0u >> 5)) * a.T + q0 + j * 32);
                     uint32_t mwords[32];
 #pragma unroll
                     for (int t = 0; t < 32; ++t) mwords[t] = mw[t];
@@ -707,14 +910,22 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_t
                 // Hidden elements (causal or masked) need no separate dS masking: their score is the
                 // fill value and the row's reference point is a real maximum (or 0 for a row without
                 // visible keys), so p, hence dS, is exactly 0 there.
-                tp_x_regs_one(dv, base + 3 * X::NP * PANEL, pd, j, lr, lg, T());  // dV^T += dO^T P
-                tp_x_regs_one(dk, base + 2 * X::NP * PANEL, ds, j, lr, lg, T());  // dK^T += Q^T dS
+                dot.mma(dv, dot_panel, pd, j, lr, lg);   // dV^T += dO^T P
+                qtr.mma(dk, qt_panel, ds, j, lr, lg);    // dK^T += Q^T dS
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        KV_STASH(st ^ 1)
-        __syncthreads();
+        if constexpr (ASYNC) {
+            slot = next_slot(slot);
+            if (qt + 1 < nqt) KV_LAND(slot, st ^ 1, qt + 2 < nqt)
+        } else {
+            slot ^= 1;
+            KV_STASH(st ^ 1)
+            __syncthreads();
+        }
     }
+#undef KV_COPY
+#undef KV_LAND
 #undef KV_FETCH
 #undef KV_STASH
 
@@ -726,15 +937,16 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int key_t
 
 // ---- backward: dQ -----------------------------------------------------------------------
 // Same geometry as the forward (lane = query, key tiles of 64).
-template <typename T> constexpr int dq_lds() { return 2 * 3 * AT<T>::NP * PANEL; }
+template <typename T> constexpr int dq_lds() { return sizeof(T) == 2 ? RING * 2 * PANEL : 2 * 3 * AT<T>::NP * PANEL; }
 template <typename T, bool HAS_MASK, bool TRAIN, bool STORE_DELTA>
-__device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int query_tile, char* smem) {
+__device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, const int query_tile, char* smem) {
     typedef AT<T> X;
-    constexpr int STAGE = 3 * X::NP * PANEL;  // K, V, K^T
+    constexpr bool ASYNC = sizeof(T) == 2;
+    constexpr int STAGE = (ASYNC ? 2 : 3 * X::NP) * PANEL;  // K, V (4-byte storage: and K^T)
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lg = lane >> 5;
-    const int bh = blockIdx.x, bidx = bh / a.H, hidx = bh % a.H;
+    const int bidx = bh / a.H, hidx = bh % a.H;
     const int q0 = query_tile * 128;
     const int qw0 = q0 + wave * 32;
     const int query = qw0 + lr;
@@ -776,7 +988,7 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int query_t
     if (nkt > a.T / 64) nkt = a.T / 64;
 
     TileLoader<T, KMAJOR, 64, ATT_THREADS> lk[X::NP], lv[X::NP];
-    TileLoader<T, MNMAJOR, 64, ATT_THREADS, false, true> lkt[X::NP];
+    TileLoader<T, MNMAJOR, 64, ATT_THREADS> lkt[X::NP];
 #define DQ_FETCH(KT)                                                                   \
     _Pragma("unroll") for (int p = 0; p < X::NP; ++p) {                                \
         lk[p].load_fast(Kb, a.k_rs, 1, (KT) * 64, p * X::EPP, tid);                    \
@@ -790,9 +1002,28 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int query_t
         lkt[p].store(smem + (ST) * STAGE + (2 * X::NP + p) * PANEL, tid);              \
     }
 
-    DQ_FETCH(0)
-    DQ_STASH(0)
-    __syncthreads();
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const uint32_t lds0 = lds_addr(smem);
+    PanelCopy ck, cv;
+#define DQ_COPY(KT, SLOT)                                                              \
+    {                                                                                  \
+        ck.issue(KT, lds0 + (SLOT) * STAGE, wave_u);                                   \
+        cv.issue(KT, lds0 + (SLOT) * STAGE + PANEL, wave_u);                           \
+    }
+    if constexpr (ASYNC) {
+        ck.init(Kb, a.k_rs, tid);
+        cv.init(Vb, a.v_rs, tid);
+        DQ_COPY(0, 0)
+        frags_landed(qf);
+        frags_landed(dof);
+        if (nkt > 1) DQ_COPY(1, 1)
+        copies_landed<4>(nkt > 1);
+        lds_barrier();
+    } else {
+        DQ_FETCH(0)
+        DQ_STASH(0)
+        __syncthreads();
+    }
 
     const float sc = a.scale * LOG2E;
     f32x16 dq[2];
@@ -802,7 +1033,7 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int query_t
         for (int e = 0; e < 16; ++e) dq[t][e] = 0.f;
 
     const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
-    const int qw0u = q0 + __builtin_amdgcn_readfirstlane(wave) * 32;
+    const int qw0u = q0 + wave_u * 32;
     KeepWords kw_next;
     if constexpr (TRAIN) kw_next = load_keep_words(kline, qw0u);
     const uint32_t* __restrict__ crow = nullptr;
@@ -812,9 +1043,11 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int query_t
         crow = a.mask + 2 * (int64_t)a.B * G * a.T + ((int64_t)bidx * G + (qw0u >> 5)) * G;
         tc_next = load_classes(crow, 0);
     }
+    int st = 0;   // this tile's place in LDS
     for (int kt = 0; kt < nkt; ++kt) {
-        const int st = kt & 1;
-        DQ_FETCH(kt + 1 < nkt ? kt + 1 : kt)
+        if constexpr (ASYNC) {
+            if (kt + 2 < nkt) DQ_COPY(kt + 2, next_slot(next_slot(st)))
+        } else DQ_FETCH(kt + 1 < nkt ? kt + 1 : kt)
         const KeepWords kw = kw_next;   // requested one step ago
         if constexpr (TRAIN) kw_next = load_keep_words(kline, qw0u + (kt + 1) * 64);
         const TileClasses tc = tc_next;
@@ -831,17 +1064,26 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int query_t
                 if (kh0 > qw0 + 31) continue;
                 const uint32_t cls = j == 0 ? tc.c0 : tc.c1;
                 if (HAS_MASK && cls == TILE_HIDDEN) continue;
-                f32x16 s, dp;
+                RowFrags<T, 1> ka, va;
+                ka.read(base, j, lr, lg);
+                va.read(base + X::NP * PANEL, j, lr, lg);
+                if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
+                f32x16 s1[1], dp1[1];
 #pragma unroll
-                for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
-                rows_x_frags_one<T>(s, base, qf, j, lr, lg);                       // S^T  [key][query]
-                rows_x_frags_one<T>(dp, base + X::NP * PANEL, dof, j, lr, lg);     // dP^T [key][query]
+                for (int e = 0; e < 16; ++e) s1[0][e] = dp1[0][e] = 0.f;
+                ka.mma(s1, base, qf, j, lr, lg);                                   // S^T  [key][query]
+                va.mma(dp1, base + X::NP * PANEL, dof, j, lr, lg);                 // dP^T [key][query]
+                f32x16 &s = s1[0], &dp = dp1[0];
+                const char* kt_panel = base + (ASYNC ? 0 : 2 * X::NP * PANEL);
+                TpFrags<T> ktr;
+                ktr.read(kt_panel, j, lr, lg);
+                if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
 
                 const bool masked = kh0 + 31 > qw0;
                 if (masked) apply_causal<true>(s, query - kh0 - lg * 4);
                 if (HAS_MASK && cls != TILE_CAUSAL) {
                     // one word per key: the mask bits of the wave's 32 queries (wave-uniform loads)
-                    const uint32_t* mw = a.mask + ((int64_t)bidx * (a.T >> 5) + (qw0u >> 5)) * a.T + kh0;
+                    const uniform_words mw = as_uniform(a.mask + ((int64_t)bidx * (a.T >> 5) + (qw0u >> 5)) * a.T + kh0);
                     uint32_t mwords[32];
 #pragma unroll
                     for (int t = 0; t < 32; ++t) mwords[t] = mw[t];
@@ -859,13 +1101,21 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int query_t
                         ds[i] = p * fmaf(dp[i], 0.9f, -delta);
                 }
                 // as in the dK/dV pass: p, hence dS, is exactly 0 on hidden elements
-                tp_x_regs_one(dq, base + 2 * X::NP * PANEL, ds, j, lr, lg, T());   // dQ^T += K^T dS^T
+                ktr.mma(dq, kt_panel, ds, j, lr, lg);   // dQ^T += K^T dS^T
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        DQ_STASH(st ^ 1)
-        __syncthreads();
+        if constexpr (ASYNC) {
+            copies_landed<4>(kt + 2 < nkt);
+            lds_barrier();
+            st = next_slot(st);
+        } else {
+            st ^= 1;
+            DQ_STASH(st)
+            __syncthreads();
+        }
     }
+#undef DQ_COPY
 #undef DQ_FETCH
 #undef DQ_STASH
 
@@ -879,22 +1129,24 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int query_t
 template <typename T, bool HAS_MASK, bool TRAIN>
 __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_bwd_dq_kernel(const AttnArgs a) {
     __shared__ __attribute__((aligned(16))) char smem[dq_lds<T>()];
-    attn_bwd_dq<T, HAS_MASK, TRAIN, true>(a, gridDim.y - 1 - blockIdx.y, smem);
+    const Place pl = place();
+    attn_bwd_dq<T, HAS_MASK, TRAIN, true>(a, pl.bh, gridDim.y - 1 - pl.tile, smem);
 }
 template <typename T, bool HAS_MASK, bool TRAIN>
 __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_dkdv_kernel(const AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<T>()];
+    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<T, false>()];
     __shared__ __attribute__((aligned(16))) StatTile sstat[2];
-    attn_bwd_dkdv<T, HAS_MASK, TRAIN, false>(a, blockIdx.y, smem, sstat);
+    const Place pl = place();
+    attn_bwd_dkdv<T, HAS_MASK, TRAIN, false>(a, pl.bh, pl.tile, smem, sstat);
 }
 // Both in one launch, grid (B*H, 2 ceil(T/128)).
 template <typename T, bool HAS_MASK, bool TRAIN>
 __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_kernel(const AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<T>()];
+    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<T, true>()];
     __shared__ __attribute__((aligned(16))) StatTile sstat[2];
     const int tile = blockIdx.y >> 1;
-    if (blockIdx.y & 1) attn_bwd_dq<T, HAS_MASK, TRAIN, false>(a, (gridDim.y >> 1) - 1 - tile, smem);
-    else attn_bwd_dkdv<T, HAS_MASK, TRAIN, true>(a, tile, smem, sstat);
+    if (blockIdx.y & 1) attn_bwd_dq<T, HAS_MASK, TRAIN, false>(a, blockIdx.x, (gridDim.y >> 1) - 1 - tile, smem);
+    else attn_bwd_dkdv<T, HAS_MASK, TRAIN, true>(a, blockIdx.x, tile, smem, sstat);
 }
 
 // Launch one of the (mask, train) specialisations.
