@@ -1199,9 +1199,9 @@ void launch_fwd(const AttnArgs& a, int dtype, hipStream_t st) {
 
 // One launch while the two passes' workgroups make no more than four rounds of one per CU, two launches beyond.  The passes
 // then fill each other's idle CUs and a launch is saved, against an O tile read again per query tile of dK/dV (delta) and
-// the dQ tiles at the dK/dV kernel's occupancy.  GPT-2 training step, two launches / one: batch 2 x 256 (96 workgroups)
-// 3100 / 3000 us, 7 x 448 bf16 (672) 6230 / 6105, attention fp32 8 x 512 (768) 223 / 215; bf16 8 x 1024 (1536) 122 / 122,
-// step 16 x 1024 (3072) 20070 / 20330.
+// the dQ tiles at the dK/dV kernel's occupancy.  From the first kernel's start to the last one's end, two launches / one, bf16
+// and 12 heads (workgroups): 2 x 256 (96) 29.6 / 14.1 us, 7 x 448 (672) 37.9 / 26.8, 8 x 512 (768) 40.5 / 31.1, 4 x 1024 (768)
+// 61.8 / 47.6, 8 x 1024 (1536) 79.1 / 77.1, 16 x 1024 (3072) 138.9 / 148.1; fp32 8 x 512 (768) 223 / 215 with the forward.
 void launch_bwd(const AttnArgs& a, int dtype, hipStream_t st) {
     const int64_t nt = (a.T + 127) / 128;
     const bool one = (int64_t)a.B * a.H * nt * 2 <= (int64_t)4 * ptj_num_cus();
