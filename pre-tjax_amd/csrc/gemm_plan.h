@@ -1,6 +1,6 @@
 // Which GEMM kernel a product takes.  Two families exist: the persistent kernels of gemm_ring.h (bf16), which stream tile after
 // tile of 256x256 or 256x192 through every CU and win when there is about a round of such tiles or more, and the
-// one-tile-per-workgroup kernels of gemm_tile.h (fp32: also gemm_split.h) below that.
+// one-tile-per-workgroup kernels of gemm_tile.h (fp32: also gemm_split.h, and gemm_planes.h for large products) below that.
 //
 // The choice minimises a time estimate,
 //     start + rounds * (K steps * step + finish)  [+ second stage of a K split],

@@ -13,6 +13,10 @@
 // fragments, each refilled for the next step right behind its last use: the step begins with the products of the middle
 // parts, whose fragments were refilled first, and the barrier comes behind those four MFMAs.
 //
+// Measured, gemm_split_kernel / this with its pass: 4096x3072x768 118.6 / 103.8 us, 4096x2304x768 106 / 94, 4096x35374x768
+// 1352 / 1074 (the pass: 11.6 us for 4096x3072x768, 4.7 TB/s); training step 8 x 512 22.65 / 22.10 ms.  Outputs 768 wide,
+// which read every operand less often, are slower so (4096x768x768 34.7 / 42.6, 4096x768x3072 123 / 128) and stay there.
+//
 // The matrix pipe rounds its accumulator more coarsely than a vector add: the leading products (hh) of two steps are formed from
 // zero and added by the vector ALU, as in gemm_split_kernel, and the five small terms have an accumulator of their own.
 constexpr int GS_FRAG = 1024;                        // bytes of 32 rows x 16 contraction elements of one part

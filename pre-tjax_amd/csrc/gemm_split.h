@@ -1,4 +1,5 @@
-// fp32 GEMM on the bf16 matrix pipe.  Included by gemm_tile_launch.h inside its unnamed namespace.
+// fp32 GEMM on the bf16 matrix pipe.  Included by gemm_tile_launch.h inside its unnamed namespace.  Products whose operands are
+// read by many tiles are split ahead of the product instead (gemm_planes.h, same arithmetic).
 //
 // The three-way split of Henry, Tang and Heinecke ("Leveraging the bfloat16 Artificial Intelligence Datatype For
 // Higher-Precision Computations", 2019): every fp32 value is the exact sum of three bf16 values h + m + l (each the
