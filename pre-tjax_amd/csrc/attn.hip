@@ -112,12 +112,13 @@ __device__ __forceinline__ void load_row_frags(typename AT<T>::F (&f)[AT<T>::NC]
 // - product, with the two or three wavefronts per SIMD that the registers allow.  Four wavefronts per SIMD (two tiles in LDS,
 // 128 registers) changed the forward and dQ by 1 %.
 //
-// A panel is 64 rows of 128 bytes as they lie in memory, its 16-byte pieces permuted inside each row by row_swizzle: eight
-// consecutive rows read one piece each without a bank conflict (RowFrags), and so do the four rows x 64 bytes that half
-// a wavefront fetches with a transposing read (TpFrags), so ONE panel serves both directions.
+// A panel is 64 rows of 128 bytes as they lie in memory, its 16-byte pieces permuted inside each row by row_swizzle: the
+// sixteen lanes that a 16-byte read serves at once (0-3, 12-15, 20-27 of the half wavefront, and the others) find their rows'
+// pieces in different banks (RowFrags), and so do the four rows x 64 bytes that half a wavefront fetches with a transposing read
+// (TpFrags), so ONE panel serves both directions.
 constexpr int RING = 3;                   // tiles in LDS: one in use, two on their way
 constexpr int WAVE_COPY = 64 * 16;        // bytes of one copy of a wavefront: eight rows
-__device__ __forceinline__ int row_swizzle(int row) { return ((row & 2) << 1) | ((row & 4) >> 1) | (row & 1); }
+__device__ __forceinline__ int row_swizzle(int row) { return ((row & 2) << 1) | ((row >> 2) & 3); }
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
 }
@@ -243,9 +244,9 @@ template <> struct TpFrags<bf16> {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const int piece = t * 4 + 2 * (lr >> 4) + ((lr & 3) >> 1);
-                const char* pp = panel + (j * 32 + h * 16 + x) * BKB + ((piece ^ row_swizzle(x)) << 4) + 8 * (lr & 1);
-                const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(pp));
-                const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(pp + 8 * BKB));
+                const char* pp = panel + (j * 32 + h * 16 + x) * BKB + 8 * (lr & 1);
+                const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(pp + ((piece ^ row_swizzle(x)) << 4)));
+                const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(pp + 8 * BKB + ((piece ^ row_swizzle(x + 8)) << 4)));
                 a[h][t] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
             }
     }
