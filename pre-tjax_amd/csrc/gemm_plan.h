@@ -9,6 +9,8 @@
 // (launches replayed from a graph, operands rotating over 200 MB).  bf16: checked on these at eight token counts from 448 to
 // 16384, against every kernel and K split within 1.6 times the lowest estimate, the estimate is off by 8 % rms and the pick is
 // 0.4 % slower than the best one on average and 11 % at worst.
+// (64x128 and two 128x128 tiles a CU were fitted again on 1280 to 2048 tokens, where the first was estimated 10 % low:
+// forward of 1536 tokens 1195 -> 1120 us, of 2048 1385 -> 1350.)
 #pragma once
 #include "common.h"
 
@@ -30,9 +32,9 @@ constexpr int RAGGED_FIRST[2] = {6, 4}, RAGGED_END[2] = {8, 6};
 constexpr TileCost GT_COST[2][8] = {
     {{32, 32, 256, 1, 2.08, 0.571, 1.33, 1.0, 0.0},
      {64, 64, 128, 1, 3.62, 0.341, 1.57, 1.0, 0.0},
-     {64, 128, 64, 2, 4.50, 0.270, 1.12, 1.73, 0.22},
+     {64, 128, 64, 2, 4.50, 0.300, 1.12, 1.87, 0.10},
      {128, 128, 64, 1, 4.59, 0.384, 1.68, 1.0, 0.34},
-     {128, 128, 64, 2, 4.25, 0.646, 2.01, 1.33, 0.23},
+     {128, 128, 64, 2, 4.25, 0.632, 2.01, 1.33, 0.23},
      {128, 192, 64, 2, 5.57, 0.587, 3.93, 1.32, 0.91},
      {128, 128, 64, 2, 4.32, 0.765, 5.66, 1.57, 0.0},
      {64, 64, 64, 2, 4.51, 0.471, 1.01, 1.08, 0.0}},
