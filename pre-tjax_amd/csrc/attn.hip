@@ -106,8 +106,8 @@ __device__ __forceinline__ void load_row_frags(typename AT<T>::F (&f)[AT<T>::NC]
 // Tiles go from memory into LDS without registers, two tiles ahead of their use, and lie there once.  Before, they went
 // through registers one tile ahead and lay in LDS a second time, transposed by vector permutes: dK/dV and dQ read Q, dO and
 // K from memory twice, and a third of the vector instructions of a step were the loader's.  Batch 8 x 1024 x 12 heads,
-// before / after (with the order of place()): forward 26.8 / 24.6 us, dQ 38.1 / 33.3, dK/dV 51.4 / 46.5; both in one launch,
-// batch 8 x 512: 35.9 / 30.8.  What bounds them now: a step's matrix and vector instructions hardly overlap (forward: 512
+// before / after (with the order of place()): forward 26.8 / 24.4 us, dQ 38.1 / 32.8, dK/dV 51.4 / 46.2; both in one launch,
+// batch 8 x 512: 35.9 / 29.6.  What bounds them now: a step's matrix and vector instructions hardly overlap (forward: 512
 // and 1000 clocks of 1670 per SIMD and step of 64 keys, batch 16 x 1024), and the chain of a step, LDS - product - softmax
 // - product, with the two or three wavefronts per SIMD that the registers allow.  Four wavefronts per SIMD (two tiles in LDS,
 // 128 registers) changed the forward and dQ by 1 %.
