@@ -176,19 +176,8 @@ __device__ __forceinline__ bool philox_keep(uint32_t offset, uint32_t k0, uint32
 //   gelu(x)  = 0.5 x (1 + tanh z)                       = x * s
 //   gelu'(x) = 0.5 (1 + tanh z) + 0.5 x (1 - tanh^2 z) z' = s + 2 x s (1 - s) z'
 // with s = sigmoid(2z), z = k (x + 0.044715 x^3), z' = k (1 + 3*0.044715 x^2).
-// s and 1-s are both formed from a = exp(-2|z|) <= 1, which avoids the cancellation
-// of (1 + tanh z) for very negative z and any overflow.
-struct SigPair { float s, om; };  // s = sigmoid(2z), om = 1 - s
-__device__ __forceinline__ SigPair sigmoid2z(float z) {
-    const float a = __expf(-2.0f * fabsf(z));
-    const float r = __builtin_amdgcn_rcpf(1.0f + a);   // denominator in [1, 2]: the 1-ulp hardware reciprocal
-    SigPair o;
-    o.s = z >= 0.f ? r : a * r;
-    o.om = z >= 0.f ? a * r : r;
-    return o;
-}
-// Forward only needs s = 1 / (1 + exp(-2z)), which is accurate for every z as it stands
-// (exp overflowing to +inf gives s = 0); -2 z log2(e) = x (c1 + c3 x^2) feeds the hardware exp2.
+// s = 1 / (1 + exp(-2z)) is accurate for every z as it stands (exp overflowing to +inf gives s = 0), by the 1-ulp hardware
+// reciprocal; -2 z log2(e) = x (c1 + c3 x^2) feeds the hardware exp2.
 __device__ __forceinline__ float gelu_f(float x) {
     constexpr float k = 0.7978845608028654f, l2e = 1.4426950408889634f;
     constexpr float c1 = -2.0f * l2e * k, c3 = -2.0f * l2e * k * 0.044715f;
@@ -196,20 +185,22 @@ __device__ __forceinline__ float gelu_f(float x) {
     return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 // Both from one exponential: e = exp(-2z), s = 1 / (1 + e), 1 - s = e s.  e may overflow to infinity, where s is 0 and the
-// product is kept from inf * 0 by the largest finite e.
+// product is kept from inf * 0 by the largest finite e.  The derivative is right for every finite x: its polynomial is that
+// of |x| <= 32, long after s has become 0 or 1, and meets x only behind the factor s (1 - s), which is 0 there.  (Infinite x
+// give NaN, as the formula does.)  Every kernel forms the derivative here, so it does not depend on which one runs.  rms error
+// for normally distributed x: 3.7e-8 (the product form s (1 + 2 x (1 - s) z'): 4.2e-8).
 __device__ __forceinline__ void gelu_both_f(float x, float& y, float& dy) {
     constexpr float k = 0.7978845608028654f, l2e = 1.4426950408889634f;
     constexpr float c1 = -2.0f * l2e * k, c3 = -2.0f * l2e * k * 0.044715f;
-    const float x2 = x * x;
+    const float x2 = fminf(x * x, 1024.0f);
     const float e = __builtin_amdgcn_exp2f(x * fmaf(x2, c3, c1));
     const float s = __builtin_amdgcn_rcpf(1.0f + e);
     const float om = fminf(e, 3.4028235e38f) * s;
     y = x * s;
-    dy = s * fmaf(om, x * fmaf(x2, 6.0f * k * 0.044715f, 2.0f * k), 1.0f);
+    dy = fmaf(y * om, fmaf(x2, 6.0f * k * 0.044715f, 2.0f * k), s);
 }
 __device__ __forceinline__ float gelu_grad_f(float x) {
-    constexpr float k = 0.7978845608028654f;
-    const float x2 = x * x;
-    const SigPair sp = sigmoid2z(k * (x + 0.044715f * x * x2));
-    return sp.s * (1.0f + 2.0f * x * sp.om * k * (1.0f + 3.0f * 0.044715f * x2));
+    float y, dy;
+    gelu_both_f(x, y, dy);
+    return dy;
 }

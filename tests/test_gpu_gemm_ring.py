@@ -54,6 +54,25 @@ def test_ring_shapes(mt, n, m, k, layout):
     assert (odd[:, 0] == 7.0).all() and (odd[:, m + 1:] == 7.0).all()
 
 
+# one shape for each kernel that forms the derivative: ring, tiles, K split, unaligned and strided operands, fp32 tiles, fp32 split
+# per tile and ahead
+@pytest.mark.parametrize("n,m,k,dtype,step", [(3001, 3080, 128, BF16, 1), (100, 776, 64, BF16, 1), (64, 768, 4096, BF16, 1),
+                                              (100, 771, 65, BF16, 1), (100, 776, 64, BF16, 2), (70, 128, 64, torch.float32, 1),
+                                              (512, 768, 256, torch.float32, 1), (4096, 3072, 128, torch.float32, 1)])
+def test_gelu_derivative_of_large_preactivations(mt, n, m, k, dtype, step):
+    """Pre-activations over the whole finite range: the GELU is x or 0 and its derivative exactly 1 or 0."""
+    g = gen(n + m + k)
+    a, b = randn(g, n, k * step, dtype=dtype, std=0.1).to(DEV)[:, ::step], randn(g, k, m, dtype=dtype, std=0.1).to(DEV)
+    big = torch.tensor([64.0, 1e3, 1.1e13, 1.3e13, 1e15, 1.7e19, 2e19, 1e30, 3.3e38])
+    bias = torch.cat([big, -big]).repeat(m // 18 + 1)[:m].to(dtype).to(DEV)
+    out, deriv = (torch.empty(n, m, dtype=dtype, device=DEV) for _ in range(2))
+    mt.matmul_t(a, b, bias, gelu=True, out=out, deriv_out=deriv)
+    pos = (bias > 0).expand(n, m)
+    assert torch.equal(deriv, pos.to(dtype))
+    x = mt.matmul_t(a, b, bias)
+    assert torch.equal(out, torch.where(pos, x, torch.zeros_like(x)))
+
+
 @pytest.mark.parametrize("n,m,k", [(3001, 3080, 770), (16400, 3076, 128)])
 @pytest.mark.parametrize("layout", ["nn", "tt"])
 def test_ring_multiply_epilogue(mt, n, m, k, layout):

@@ -70,6 +70,16 @@ def test_gelu(mt, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_gelu_of_large_inputs(mt, dtype):
+    big = torch.tensor([64.0, 1e3, 1.1e13, 1.3e13, 1e15, 1.7e19, 2e19, 1e30, 3.3e38, 0.0])
+    x = torch.cat([big, -big]).to(dtype).repeat(16).to(DEV)
+    d = torch.where(x == 0, 0.5, (x > 0).to(torch.float32)).to(dtype)
+    assert torch.equal(mt.t_gelu_fwd_t(x), torch.where(x > 0, x, torch.zeros_like(x)))
+    assert torch.equal(mt.t_gelu_bkwd2_t(torch.ones_like(x), x), d)
+    assert torch.equal(mt.t_gelu_bkwd2_colsum_t(torch.ones_like(x).view(16, 20), x.view(16, 20))[0].view(-1), d)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape", [(4096, 768), (333, 768), (64, 1024), (17, 4096), (5, 100), (3, 1001), (2, 16384)])
 def test_dropout_add_layernorm_matches_separate_calls(mt, dtype, shape):
     """Residual update + LayerNorm in one pass: bit-exact against dropout_add_t followed by
