@@ -225,7 +225,7 @@ struct RingRows {
         p1 = p0 + bytes;
     }
     // T at byte `off` of the lane's part of row 16 h
-    template <typename T> __device__ __forceinline__ __attribute__((address_space(1))) T* at(int h, int off, uint32_t voff) const {
+    template <typename T, typename OFF> __device__ __forceinline__ __attribute__((address_space(1))) T* at(int h, int off, OFF voff) const {
         return (__attribute__((address_space(1))) T*)((h ? p1 : p0) + off + voff);
     }
     __device__ __forceinline__ void next() {
@@ -234,6 +234,15 @@ struct RingRows {
         p1 = p0 + bytes;
     }
 };
+
+// Pitches from which on the offset of a lane's row, up to 15 rows, leaves 32 bits: such blocks are written like those at the
+// borders, whose offsets have 64 bits (ring_far).
+constexpr int64_t RING_WIDE = 1ll << 27;
+// bytes to the lane's part of its row, formed where they are used (opaque: only the borders hold registers for them)
+__device__ __forceinline__ int64_t ring_far(int lrow, int lcol, int64_t rs) {
+    asm volatile("" : "+v"(lrow));
+    return ((int64_t)lrow * rs + lcol) * 2;
+}
 
 // half word e of a vector (borders of C: a loop, so that the kernels stay small)
 __device__ __forceinline__ uint16_t ring_half(const gt_u32x4& v, int e) {
@@ -252,14 +261,15 @@ __device__ __forceinline__ void ring_store(__attribute__((address_space(1))) bf1
 }
 
 // The wavefront's block at (row0, col0) as ACT of the accumulators, to c (and aux).  Addresses are a wave-uniform part and one
-// 32-bit offset per lane, formed here (fresh_tid) so that they hold no registers through the main loop.
+// offset per lane, 32 bits wide in whole blocks, formed here (fresh_tid) so that they hold no registers through the main loop.
 template <typename C, int ACT>
 __device__ __forceinline__ void ring_write(const GemmArgs& g, const f32x16 (&acc)[C::TNW][C::TMW], bf16* c, int64_t rs, bf16* aux,
                                            int64_t aux_rs, int row0, int col0) {
     const int lane = fresh_tid() & 63, lrow = lane & 15, lcol = ((lane >> 4) & 1) * 16 + (lane >> 5) * 8;
     RingRows cr(c + (int64_t)row0 * rs + col0, rs, 2), ar(aux + (int64_t)row0 * aux_rs + col0, aux_rs, 2);
-    const uint32_t voff = (uint32_t)(lrow * (int)rs + lcol) * 2u, aoff = (uint32_t)(lrow * (int)aux_rs + lcol) * 2u;
-    const bool aligned = g.vec_out, whole = aligned && row0 + C::TMW * 32 <= g.n && col0 + C::TNW * 32 <= g.m;   // wave-uniform
+    const uint32_t voff = ((uint32_t)lrow * (uint32_t)rs + (uint32_t)lcol) * 2u, aoff = ((uint32_t)lrow * (uint32_t)aux_rs + (uint32_t)lcol) * 2u;
+    const bool aligned = g.vec_out, whole = aligned && rs < RING_WIDE && aux_rs < RING_WIDE && row0 + C::TMW * 32 <= g.n &&
+                                            col0 + C::TNW * 32 <= g.m;   // wave-uniform
     const int rows = g.n - row0 - lrow, cols = g.m - col0 - lcol;
 #pragma unroll
     for (int tm = 0; tm < C::TMW; ++tm) {
@@ -276,8 +286,8 @@ __device__ __forceinline__ void ring_write(const GemmArgs& g, const f32x16 (&acc
                     int ne = cols;                        // (opaque: no lane masks kept from one store to the next)
                     asm volatile("" : "+v"(ne));
                     ne = tm * 32 + h * 16 < rows ? ne - tn * 32 : 0;
-                    ring_store(cr.at<bf16>(h, tn * 64, voff), v[h], ne, aligned);
-                    if constexpr (ACT == RING_BOTH) ring_store(ar.at<bf16>(h, tn * 64, aoff), w[h], ne, aligned);
+                    ring_store(cr.at<bf16>(h, tn * 64, ring_far(lrow, lcol, rs)), v[h], ne, aligned);
+                    if constexpr (ACT == RING_BOTH) ring_store(ar.at<bf16>(h, tn * 64, ring_far(lrow, lcol, aux_rs)), w[h], ne, aligned);
                 }
             }
         }
@@ -287,13 +297,14 @@ __device__ __forceinline__ void ring_write(const GemmArgs& g, const f32x16 (&acc
 }
 
 // fp32 partial sums of the block at (row0, col0) of dst, rows of `rs` elements and 16-byte aligned where 4 divides rs; four
-// columns of row h*16 + (l & 15) per lane and store
+// columns of row h*16 + (l & 15) per lane and store.  (rs is a tile's width or that of an output of fewer than 2 num_cus
+// tiles, the only ones that are K-split: 32-bit offsets.)
 template <typename C>
 __device__ __forceinline__ void ring_write_partial(const f32x16 (&acc)[C::TNW][C::TMW], float* __restrict__ dst, int64_t rs, int row0,
                                                    int col0, int nrows, int ncols) {
     const int lane = fresh_tid() & 63, lrow = lane & 15, lcol = ((lane >> 4) & 1) * 8 + (lane >> 5) * 4;
     RingRows pr(dst + (int64_t)row0 * rs + col0, rs, 4);
-    const uint32_t voff = (uint32_t)(lrow * (int)rs + lcol) * 4u;
+    const uint32_t voff = ((uint32_t)lrow * (uint32_t)rs + (uint32_t)lcol) * 4u;
     const bool whole = rs % 4 == 0 && row0 + C::TMW * 32 <= nrows && col0 + C::TNW * 32 <= ncols;
 #pragma unroll
     for (int tm = 0; tm < C::TMW; ++tm) {
@@ -334,8 +345,9 @@ __device__ __forceinline__ void ring_write_mul(const GemmArgs& g, const f32x16 (
     const int lane = fresh_tid() & 63, lrow = lane & 15, lcol = ((lane >> 4) & 1) * 16 + (lane >> 5) * 8;
     const int64_t mul_rs = g.mul_rs, c_rs = g.c_rs;
     RingRows mr((bf16*)g.mul + (int64_t)row0 * mul_rs + col0, mul_rs, 2), cr((bf16*)g.c + (int64_t)row0 * c_rs + col0, c_rs, 2);
-    const uint32_t moff = (uint32_t)(lrow * (int)mul_rs + lcol) * 2u, coff = (uint32_t)(lrow * (int)c_rs + lcol) * 2u;
-    const bool aligned = g.vec_out, whole = aligned && row0 + TMW * 32 <= g.n && col0 + TNW * 32 <= g.m;   // wave-uniform
+    const uint32_t moff = ((uint32_t)lrow * (uint32_t)mul_rs + (uint32_t)lcol) * 2u, coff = ((uint32_t)lrow * (uint32_t)c_rs + (uint32_t)lcol) * 2u;
+    const bool aligned = g.vec_out, whole = aligned && mul_rs < RING_WIDE && c_rs < RING_WIDE && row0 + TMW * 32 <= g.n &&
+                                            col0 + TNW * 32 <= g.m;   // wave-uniform
     const int rows = g.n - row0 - lrow, cols = g.m - col0 - lcol;
     float cs[TNW][8];
 #pragma unroll
@@ -359,13 +371,13 @@ __device__ __forceinline__ void ring_write_mul(const GemmArgs& g, const f32x16 (
                     ne = tm * 32 + h * 16 < rows ? ne - tn * 32 : 0;
                     uint32_t w[4] = {0u, 0u, 0u, 0u};
                     if (aligned && ne >= 8) {
-                        const gt_u32x4 all = *mr.at<gt_u32x4>(h, tn * 64, moff);
+                        const gt_u32x4 all = *mr.at<gt_u32x4>(h, tn * 64, ring_far(lrow, lcol, mul_rs));
 #pragma unroll
                         for (int e = 0; e < 4; ++e) w[e] = all[e];
                     } else {
 #pragma unroll 1
                         for (int e = 0; e < (ne < 8 ? ne : 8); ++e) {
-                            const uint32_t x = (uint32_t)*(mr.at<uint16_t>(h, tn * 64, moff) + e) << (16 * (e & 1));
+                            const uint32_t x = (uint32_t)*(mr.at<uint16_t>(h, tn * 64, ring_far(lrow, lcol, mul_rs)) + e) << (16 * (e & 1));
 #pragma unroll
                             for (int i = 0; i < 4; ++i) w[i] |= i == e >> 1 ? x : 0u;
                         }
@@ -400,11 +412,11 @@ __device__ __forceinline__ void ring_write_mul(const GemmArgs& g, const f32x16 (
                     if (aligned && ne >= 8) {
 #pragma unroll
                         for (int e = 0; e < 8; ++e) cs[tn][e] += to_f32(s.v[e]);
-                        *cr.at<gt_u32x4>(h, tn * 64, coff) = __builtin_bit_cast(gt_u32x4, s);
+                        *cr.at<gt_u32x4>(h, tn * 64, ring_far(lrow, lcol, c_rs)) = __builtin_bit_cast(gt_u32x4, s);
                     } else {
 #pragma unroll
                         for (int e = 0; e < 8; ++e) cs[tn][e] += e < ne ? to_f32(s.v[e]) : 0.f;
-                        ring_store(cr.at<bf16>(h, tn * 64, coff), __builtin_bit_cast(gt_u32x4, s), ne, false);
+                        ring_store(cr.at<bf16>(h, tn * 64, ring_far(lrow, lcol, c_rs)), __builtin_bit_cast(gt_u32x4, s), ne, false);
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);

@@ -110,3 +110,29 @@ def test_ring_rows_that_overlap(mt, k):
     c = mt.matmul_t(a, b)
     want, scale = product(a, b)
     assert ((f64(c) - want).abs() / gemm_bound(want, scale, BF16)).max().item() <= 1.0
+
+
+def test_ring_rows_far_apart(mt):
+    """Outputs and multipliers in column slices of buffers so wide that a lane's row leaves 32-bit offsets."""
+    n, m, k, pitch, at = 24, 136, 64, 150_000_000, 1_000_000
+    g = gen(n)
+    wide = torch.zeros(n, pitch, dtype=BF16, device=DEV)
+    part = wide[:, at:at + m]
+    a, b = randn(g, k, n, dtype=BF16).to(DEV).t(), randn(g, k, m, dtype=BF16).to(DEV)
+    c0 = randn(g, n, m, dtype=BF16).to(DEV)
+    part.copy_(c0)
+    mt.matmul_t(a, b, out=part, accumulate=True)
+    want = c0.clone()
+    mt.matmul_t(a, b, out=want, accumulate=True)
+    assert torch.equal(part, want) and torch.count_nonzero(wide) == torch.count_nonzero(part)
+    # one row for all of A: operands that only these kernels take
+    row = randn(g, 1, k, dtype=BF16).to(DEV).expand(n, k)
+    bias, deriv = randn(g, m, dtype=BF16).to(DEV), torch.zeros_like(wide)
+    mt.matmul_t(row, b, bias, gelu=True, out=part, deriv_out=deriv[:, at:at + m])
+    out, d = torch.empty_like(c0), torch.empty_like(c0)
+    mt.matmul_t(row, b, bias, gelu=True, out=out, deriv_out=d)
+    assert torch.equal(part, out) and torch.equal(deriv[:, at:at + m], d)
+    assert torch.count_nonzero(wide) == torch.count_nonzero(part) and torch.count_nonzero(deriv) == torch.count_nonzero(d)
+    part.copy_(c0)
+    for x, y in zip(mt.matmul_mul_colsum_t(row, b, part), mt.matmul_mul_colsum_t(row, b, c0)):
+        assert torch.equal(x, y)
