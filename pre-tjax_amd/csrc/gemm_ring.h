@@ -735,11 +735,13 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
 }
 
 // Whether a launch can take these kernels: two vector layouts and 32-bit offsets inside a tile; where the contraction ends
-// inside a step, also rows that do not overlap (what lies past an operand's end is told by its address).
+// inside a step, also rows that do not overlap (what lies past an operand's end is told by its address).  All 64 contraction
+// indices of a step have to fit, those past the end as well: an offset that wrapped would read something else than zero there.
+// Rows past the end of an operand may read anything of it; their results are not stored.
 inline bool ring_eligible(const GemmArgs& g, int am, int bm) {
     if (am == GENERIC || bm == GENERIC || g.k < 1) return false;
     auto fits = [&](int mode, int64_t row, int64_t kst, int64_t nrows) {
-        const int64_t pitch = mode == KMAJOR ? row : kst, lines = mode == KMAJOR ? (nrows < 256 ? nrows : 256) : (g.k < 64 ? g.k : 64);
+        const int64_t pitch = mode == KMAJOR ? row : kst, lines = mode == KMAJOR ? (nrows < 256 ? nrows : 256) : 64;
         const int64_t length = mode == KMAJOR ? g.k : nrows;
         return pitch >= 0 && pitch < (1ll << 31) && (lines * pitch + 256) * 2 < 0x80000000ll + 512 && (g.k % 64 == 0 || pitch >= length);
     };

@@ -136,3 +136,14 @@ def test_ring_rows_far_apart(mt):
     part.copy_(c0)
     for x, y in zip(mt.matmul_mul_colsum_t(row, b, part), mt.matmul_mul_colsum_t(row, b, c0)):
         assert torch.equal(x, y)
+
+
+def test_ring_contraction_rows_far_apart(mt):
+    """A contraction of fewer indices than a step, its rows so far apart that those past the end leave 32-bit offsets."""
+    n, m, k, pitch = 40, 136, 16, 50_000_000
+    g = gen(k)
+    a = randn(g, n, k, dtype=BF16).to(DEV)
+    b = torch.full((k, pitch), float("nan"), dtype=BF16, device=DEV)[:, :m]
+    b.copy_(randn(g, k, m, dtype=BF16).to(DEV))
+    want, scale = product(a, b)
+    assert ((f64(mt.matmul_t(a, b)) - want).abs() / gemm_bound(want, scale, BF16)).max().item() <= 1.0
