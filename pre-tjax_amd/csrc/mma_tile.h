@@ -78,8 +78,8 @@ struct TileLoader {
 
     // Interior panels: every vector is fully inside the operand; straight-line 16-byte loads
     // (no predicates, no branches, so all of them stay in flight together).  The address is
-    // split into a wave-uniform 64-bit part (scalar registers) and one 32-bit per-lane
-    // offset that does not change along K.
+    // split into a wave-uniform 64-bit part (scalar registers) and one per-lane offset that does
+    // not change along K (64 bits as well: rows may be any distance apart).
     __device__ __forceinline__ void load_fast(const T* __restrict__ p, int64_t s_row, int64_t s_k, int row0, int k0,
                                               int tid) {
         load_fast_slice<0, 1, false>(p, s_row, s_k, row0, k0, tid, 0);
@@ -93,11 +93,11 @@ struct TileLoader {
     __device__ __forceinline__ void load_fast_slice(const T* __restrict__ p, int64_t s_row, int64_t s_k, int row0,
                                                     int k0, int tid, int nrows) {
         static_assert(MODE != GENERIC, "GENERIC panels have no vector path");
-        // Byte addressing: wave-uniform 64-bit base + one unsigned 32-bit lane offset.
+        // Byte addressing: wave-uniform base + one lane offset.
         if constexpr (MODE == KMAJOR) {
             if constexpr (!CLAMP) {
                 const char* ub = reinterpret_cast<const char*>(p + (int64_t)row0 * s_row + k0);   // uniform
-                const uint32_t loff = ((uint32_t)(tid >> 3) * (uint32_t)s_row + (tid & 7) * VEC) * (uint32_t)sizeof(T);
+                const int64_t loff = ((int64_t)(tid >> 3) * s_row + (tid & 7) * VEC) * (int64_t)sizeof(T);
 #pragma unroll
                 for (int i = 0; i < NV; ++i) {
                     if (i % N != I) continue;
@@ -106,13 +106,13 @@ struct TileLoader {
                 }
             } else {
                 // rows past the operand's last one re-read it; both addresses are a uniform
-                // base plus a 32-bit lane offset, so the clamp costs a compare and selects
+                // base plus a lane offset, so the clamp costs a compare and selects
                 const int64_t rstep = s_row * (int64_t)sizeof(T);
                 const char* ub = reinterpret_cast<const char*>(p + (int64_t)row0 * s_row + k0);   // uniform
                 const int lim = nrows - 1 - row0;
                 const char* last = ub + (int64_t)lim * rstep;                                      // uniform
                 const uint32_t col = (uint32_t)((tid & 7) * VEC * (int)sizeof(T));
-                const uint32_t loff = (uint32_t)(tid >> 3) * (uint32_t)s_row * (uint32_t)sizeof(T) + col;
+                const int64_t loff = (int64_t)(tid >> 3) * rstep + col;
 #pragma unroll
                 for (int i = 0; i < NV; ++i) {
                     if (i % N != I) continue;
@@ -135,8 +135,7 @@ struct TileLoader {
                         const int lastv = ((nrows - 1) / VEC) * VEC;        // a .t() view's pitch covers this vector
                         rowv = row0 + rowv < lastv ? row0 + rowv : lastv;
                     }
-                    const uint32_t loff =
-                        ((uint32_t)(((b / JB) * QB + kq_lo) * 4) * (uint32_t)s_k + (uint32_t)rowv) * (uint32_t)sizeof(T);
+                    const int64_t loff = ((int64_t)(((b / JB) * QB + kq_lo) * 4) * s_k + rowv) * (int64_t)sizeof(T);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         if ((qi * 4 + i) % N != I) continue;

@@ -290,6 +290,22 @@ def test_attn_strided_views_fused_qkv_layout(mt):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_attn_rows_far_apart(mt, dtype):
+    """Column slices of a buffer so wide that the offset of a row inside a tile leaves 32 bits; what lies between is NaN."""
+    g, T = gen(5), 64
+    buf = torch.full((T, 40_000_000), float("nan"), dtype=dtype, device=DEV)
+    far = [buf[:, 64 * i + 64:64 * i + 128].view(1, 1, T, 64) for i in range(5)]
+    near = [randn(g, 1, 1, T, 64, dtype=dtype).to(DEV) for _ in range(4)]
+    for f, x in zip(far, near):
+        f.copy_(x)
+    q, k, v, d_o = near
+    o, ms, ls = mt.attn_fwd_t(q, k, v, None, False, 0)
+    assert torch.equal(mt.attn_fwd_t(*far[:3], None, False, 0, out=far[4])[0], o)
+    for x, y in zip(mt.attn_bwd_t(far[3], *far[:3], far[4], ms, ls, None, False, 0), mt.attn_bwd_t(d_o, q, k, v, o, ms, ls, None, False, 0)):
+        assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("dh", [16, 32])
 @pytest.mark.parametrize("train", [False, True])
 def test_attn_smaller_head_dimensions(mt, dtype, dh, train):

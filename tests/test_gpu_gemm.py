@@ -271,3 +271,21 @@ def test_ffn_backward_through_the_fused_epilogues(mt, dtype):
     for name, got, w in zip(("dx", "dw1", "db1", "dw2", "db2"), (dx, dw1, db1, dw2, db2), want):
         rel = ((f64(got) - w).norm() / w.norm()).item()
         assert got.shape == w.shape and rel < tol, (name, rel)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("layout", ["n", "t"])
+def test_gemm_operand_rows_far_apart(mt, dtype, layout):
+    """Column slices of a buffer so wide that the offset of a row inside a tile leaves 32 bits; what lies between is NaN."""
+    g, rows, width, m = gen(9), 72, 128, 48
+    buf = torch.full((rows, 40_000_000), float("nan"), dtype=dtype, device=DEV)
+    a = randn(g, rows, width, dtype=dtype)
+    buf[:, 64:64 + width] = a.to(DEV)
+    view = buf[:, 64:64 + width]
+    if layout == "t":
+        view, a = view.t(), a.t()
+    b = randn(g, a.shape[1], m, dtype=dtype)
+    check(mt.matmul_t(view, b.to(DEV)), a, b, dtype)
+    mul = randn(g, a.shape[0], m, dtype=dtype).to(DEV)
+    for x, y in zip(mt.matmul_mul_colsum_t(view, b.to(DEV), mul), mt.matmul_mul_colsum_t(a.to(DEV).contiguous(), b.to(DEV), mul)):
+        assert (f64(x) - f64(y)).abs().max().item() <= (1e-4 if dtype == torch.float32 else 2.0 ** -7 * f64(y).abs().max().item())
