@@ -270,6 +270,9 @@ template <> struct TpFrags<bf16> {
 // Words that no kernel here writes, at wave-uniform addresses: scalar loads, also between the inline assembly's memory clobbers.
 typedef __attribute__((address_space(4))) const uint32_t* uniform_words;
 __device__ __forceinline__ uniform_words as_uniform(const uint32_t* p) { return (uniform_words)(uintptr_t)p; }
+// First row of a wavefront where it looks up such words.  With T an odd multiple of 64 the last workgroup's second pair of
+// wavefronts has no rows; theirs would be words past the end of the lines and of the mask, so they read those of the last 32 rows.
+__device__ __forceinline__ int lookup_row(int row0, int T) { return row0 < T ? row0 : T - 32; }
 struct KeepWords { uint32_t d0, d1, d2; };
 __device__ __forceinline__ KeepWords load_keep_words(const uint32_t* __restrict__ line, int base) {
     const uniform_words p = as_uniform(line + (base >> 5));
@@ -520,7 +523,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
     } else FWD_FETCH(0)
     // keep-bit line of this batch-head and the wave's first query as scalars
     const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
-    const int qw0u = q0 + wave_u * 32;
+    const int qw0u = lookup_row(q0 + wave_u * 32, a.T);
     if constexpr (ASYNC) {
         copies_landed<4>(nkt > 1);
         lds_barrier();
@@ -823,7 +826,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
     const float sc = a.scale * LOG2E;
     // keep-bit line of this batch-head and the wave's first key as scalars
     const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
-    const int kw0u = key0 + wave_u * 32;
+    const int kw0u = lookup_row(key0 + wave_u * 32, a.T);
     KeepWords kw_next;
     if constexpr (TRAIN) kw_next = load_keep_words(kline, kw0u + qt0 * 64);
     // tile classes of the wave's 32 keys against every 32-query group (explicit mask only)
@@ -1034,7 +1037,7 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
         for (int e = 0; e < 16; ++e) dq[t][e] = 0.f;
 
     const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
-    const int qw0u = q0 + wave_u * 32;
+    const int qw0u = lookup_row(q0 + wave_u * 32, a.T);
     KeepWords kw_next;
     if constexpr (TRAIN) kw_next = load_keep_words(kline, qw0u);
     const uint32_t* __restrict__ crow = nullptr;
