@@ -477,50 +477,56 @@ __device__ __forceinline__ void gt_tile(const GemmArgs& g, int pid, char* __rest
         gt_unroll<0, PT>([&](auto i) { copy_piece(i, S - 1); });
         int slot = 0;
         // The compiler takes a fragment to be there behind its read and may copy it to other registers where control flow joins
-        // or leaves the loops, so no read is under way at the end of a loop's body or around it (READ waits at the end of a
-        // phase instead of the start of the next; same time).  What the compiler does inside a phase is checked on the code
-        // that was built.
+        // or leaves a loop, so no read is under way where a loop ends: its copies there came ahead of the wait in front of the
+        // products.  (Around the loop of one register set per panel it leaves them where they are, and a wait at the turn as well
+        // would cost a launch 0.1 us.  What it does is checked on the code that was built.)
 #define GT_READ(SET)                                                                                    \
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                              \
         landed(SET);
-        // Start of a stage's last register set: the next stage has landed and this one has been read, by every
-        // wavefront after the barrier, so the next stage may be read and this one refilled.
+        // In front of a stage's last register set: the next stage has landed and this one has been read, by every wavefront
+        // after the barrier, so the next stage may be read and this one refilled.
 #define GT_TURN(SET)                                                                                    \
-        const int next = slot + 1 == S ? 0 : slot + 1;                                                  \
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * PT) : "memory");     \
-        landed(SET);                                                                                    \
-        if (ragged && kt + 2 == nk) clear_tail(next);
-        GT_READ(I0)
+        landed(SET);
         if constexpr (NSET == 2) {
+            int next = 1;
+            GT_READ(I0)
             phase(I0, I1, ILAST, I0, I0, 0u, 0u, 0);
-            GT_READ(I1)
+            GT_TURN(I1)
             for (int kt = 0; kt + 1 < nk; ++kt) {
-                GT_TURN(I1)
+                if (ragged && kt + 2 == nk) clear_tail(next);
                 phase(I1, I0, I0, I0, IPT, next * C::A_STAGE, next * C::B_STAGE, slot);
                 GT_READ(I0)
                 phase(I0, I1, ILAST, I0, I0, next * C::A_STAGE, next * C::B_STAGE, slot);
-                GT_READ(I1)
                 slot = next;
+                next = slot + 1 == S ? 0 : slot + 1;
+                asm volatile("" : "+s"(slot), "+s"(next));      // (ahead of the wait that follows)
+                GT_TURN(I1)
             }
             phase(I1, I0, NONE, I0, I0, 0u, 0u, 0);
         } else {
             int kt = 0;
             for (; kt + 2 < nk; ++kt) {
                 {
+                    const int next = slot + 1 == S ? 0 : slot + 1;
                     GT_TURN(I0)
                     phase(I0, I1, I0, I0, IPT, next * C::A_STAGE, next * C::B_STAGE, slot);
                     slot = next;
                 }
                 ++kt;
                 {
+                    const int next = slot + 1 == S ? 0 : slot + 1;
                     GT_TURN(I1)
+                    if (ragged && kt + 2 == nk) clear_tail(next);
                     phase(I1, I0, I0, I0, IPT, next * C::A_STAGE, next * C::B_STAGE, slot);
-                    GT_READ(I0)
                     slot = next;
                 }
             }
+            GT_READ(I0)
             if (kt + 1 < nk) {
+                const int next = slot + 1 == S ? 0 : slot + 1;
                 GT_TURN(I0)
+                if (ragged) clear_tail(next);
                 phase(I0, I1, I0, I0, IPT, next * C::A_STAGE, next * C::B_STAGE, slot);
                 GT_READ(I1)
                 phase(I1, I0, NONE, I0, I0, 0u, 0u, 0);

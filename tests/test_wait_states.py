@@ -6,8 +6,8 @@ before the wait that the source puts in front of their use.  And it has left out
 round a branch is shorter than the other.  Neither shows in a source file, and the results are wrong only now and then.
 
 Rules (quarter-rate issue slots, as s_nop counts them): a result of v_mfma_*_bf16 (8 passes) may be read 12 slots later, of
-v_mfma_f32_32x32x2_f32 (16 passes) 18, and written by another instruction one slot earlier; the next product is issued when
-the one before it has gone through its passes.  vmcnt and lgkmcnt count vector memory and LDS operations, which complete in order;
+v_mfma_f32_32x32x2_f32 (16 passes) 18, and overwritten by the vector ALU one slot earlier (loads take longer than that to arrive);
+the next product is issued when the one before it has gone through its passes.  vmcnt and lgkmcnt count vector memory and LDS operations, which complete in order;
 scalar loads complete in any order.  A scalar register written by the vector ALU may address memory 5 slots later."""
 import concurrent.futures
 import os
@@ -99,9 +99,12 @@ def findings(listing):
                     if r in products:
                         found[i, r] = "factor of a product too early"
             elif products and (x.counter or x.vector_alu):
-                for r in list(x.out) + list(x.into):
-                    if r in products and (r in x.into or products[r][2] - products[r][0] > 1):
-                        found[i, r] = "result of a product touched %d slots early" % (products[r][2] - products[r][0])
+                for r in x.into:
+                    if r in products:
+                        found[i, r] = "result of a product read %d slots early" % (products[r][2] - products[r][0])
+                for r in x.out if x.vector_alu else ():
+                    if r in products and products[r][2] - products[r][0] > 1:
+                        found[i, r] = "result of a product overwritten %d slots early" % (products[r][2] - products[r][0] - 1)
             if scalars and x.vector_memory:
                 for r in x.into:
                     if r in scalars:
