@@ -270,9 +270,9 @@ template <> struct TpFrags<bf16> {
 // Words that no kernel here writes, at wave-uniform addresses: scalar loads, also between the inline assembly's memory clobbers.
 typedef __attribute__((address_space(4))) const uint32_t* uniform_words;
 __device__ __forceinline__ uniform_words as_uniform(const uint32_t* p) { return (uniform_words)(uintptr_t)p; }
-// First row of a wavefront where it looks up such words.  With T an odd multiple of 64 the last workgroup's second pair of
-// wavefronts has no rows; theirs would be words past the end of the lines and of the mask, so they read those of the last 32 rows.
-__device__ __forceinline__ int lookup_row(int row0, int T) { return row0 < T ? row0 : T - 32; }
+// First row of a wavefront where it looks up such words.  With T an odd multiple of 64 the last workgroup's upper two
+// wavefronts have no rows; theirs would be words past the end of the lines and of the mask, so they read those of the lower two.
+__device__ __forceinline__ int lookup_row(int row0, int T) { return row0 - (row0 < T ? 0 : 64); }
 struct KeepWords { uint32_t d0, d1, d2; };
 __device__ __forceinline__ KeepWords load_keep_words(const uint32_t* __restrict__ line, int base) {
     const uniform_words p = as_uniform(line + (base >> 5));
