@@ -478,8 +478,10 @@ __device__ __forceinline__ void gt_tile(const GemmArgs& g, int pid, char* __rest
         int slot = 0;
         // The compiler takes a fragment to be there behind its read and may copy it to other registers where control flow joins
         // or leaves a loop, so no read is under way where a loop ends: its copies there came ahead of the wait in front of the
-        // products.  (Around the loop of one register set per panel it leaves them where they are, and a wait at the turn as well
-        // would cost a launch 0.1 us.  What it does is checked on the code that was built.)
+        // products.  Two register sets per panel: the wait is the body's last statement.  One: around its loop the compiler leaves
+        // the fragments where they are and a wait behind the loop is enough (in the body: dW on 3001 tokens 21.6 -> 22.5 us; the
+        // barrier at the end as well: 0.1 us a launch, and 3-5 % of the products of 1536 to 2560 tokens).  What the compiler
+        // does is checked on the code that was built.
 #define GT_READ(SET)                                                                                    \
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                              \
         landed(SET);
@@ -489,19 +491,18 @@ __device__ __forceinline__ void gt_tile(const GemmArgs& g, int pid, char* __rest
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * PT) : "memory");     \
         landed(SET);
         if constexpr (NSET == 2) {
-            int next = 1;
             GT_READ(I0)
             phase(I0, I1, ILAST, I0, I0, 0u, 0u, 0);
-            GT_TURN(I1)
+            GT_READ(I1)
             for (int kt = 0; kt + 1 < nk; ++kt) {
+                const int next = slot + 1 == S ? 0 : slot + 1;
+                GT_TURN(I1)
                 if (ragged && kt + 2 == nk) clear_tail(next);
                 phase(I1, I0, I0, I0, IPT, next * C::A_STAGE, next * C::B_STAGE, slot);
                 GT_READ(I0)
                 phase(I0, I1, ILAST, I0, I0, next * C::A_STAGE, next * C::B_STAGE, slot);
+                GT_READ(I1)
                 slot = next;
-                next = slot + 1 == S ? 0 : slot + 1;
-                asm volatile("" : "+s"(slot), "+s"(next));      // (ahead of the wait that follows)
-                GT_TURN(I1)
             }
             phase(I1, I0, NONE, I0, I0, 0u, 0u, 0);
         } else {
