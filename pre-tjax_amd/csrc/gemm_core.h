@@ -3,10 +3,10 @@
 // side by side.
 //
 // This file holds the register-staged persistent kernel, which takes operands of any strides and alignment.  Products whose
-// operands have a unit stride go to the kernels of gemm_ring.h and gemm_tile.h instead (gemm_plan.h), so what is left here
-// are strided, unaligned or overlapping operands.
-//
-// C[n,m] = sum_k A(n,k) B(k,m) (+bias[m]) (gelu), fp32 accumulation.
+// operands have a unit stride go to the kernels of gemm_ring.h, gemm_tile.h, gemm_ragged.h and gemm_split.h instead
+// (gemm_plan.h).  What is left here are strided operands, element by element, and for the vector loops below operands
+// whose rows overlap (bf16: with a contraction that ends inside a step) or lie 2^21 elements apart (bf16: where the
+// offsets of gemm_ring.h end) or more.
 //
 // Tiling: one 512-thread workgroup (8 wavefronts, 4 along rows x 2 along columns) owns a
 // 256x192 tile of C; each wavefront owns 64x96 = 2x3 MFMA tiles of 32x32

@@ -9,8 +9,9 @@
 // (launches replayed from a graph, operands rotating over 200 MB).  bf16: checked on these at eight token counts from 448 to
 // 16384, against every kernel and K split within 1.6 times the lowest estimate, the estimate is off by 8 % rms and the pick is
 // 0.4 % slower than the best one on average and 11 % at worst.
-// (64x128 and two 128x128 tiles a CU were fitted again on 1280 to 2048 tokens, where the first was estimated 10 % low:
-// forward of 1536 tokens 1195 -> 1120 us, of 2048 1385 -> 1350.)
+// (64x128 and two 128x128 tiles a CU were fitted again on 1280 to 2048 tokens, where the first was estimated 10 % low and the
+// picks had become up to 8 % slower than those before the ring kernels.  Forward before these / now, in turn on one box:
+// 1280 tokens 944 / 920 us, 1408 1114 / 1082, 1536 1107 / 1088, 2048 1332 / 1333.)
 #pragma once
 #include "common.h"
 

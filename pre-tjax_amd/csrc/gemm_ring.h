@@ -15,14 +15,18 @@
 // chunk per register set: 905 us for 8192^3.
 //
 // The output goes straight from the accumulators to memory: two lane swaps bring eight consecutive columns of a row
-// into a lane and 64 bytes of each of sixteen rows into a store, without LDS, which the rings fill.  At k = 768 these
-// stores are a quarter of the time (16384x3072x768: 81 us, 60 without them): the chip takes 100 MB at 4.9 TB/s
-// however they are spaced -- kept in registers and sent between the MFMAs of the next tile they evict the panels
-// from L2 and cost more (86 us), non-temporal ones help one shape (75) and hurt another (8192x50257x768: 620 -> 690).
+// into a lane and 64 bytes of each of sixteen rows into a store, without LDS, which the rings fill.  At k = 768 the
+// output is a quarter of the time (16384x3072x768: 81 us, 60 without stores; 100 MB at 4.9 TB/s are 20).
 // GELU and its derivative come from one exponential (130 -> 118 us for 16384x3072x768 with both outputs).
 //
-// The copies run ahead across the tiles of a workgroup, so only its first tile waits for them.  Rows and contraction
-// indices past the operand's end read as zero (buffer descriptors).
+// The copies run ahead across the tiles of a workgroup, but a tile's start waits for them all the same: the accumulators start
+// from bias registers that a vector path, an element path or zeros may have filled, and the compiler puts s_waitcnt vmcnt(0)
+// in front of their use, with a bias or without.  That drains the stores of the tile before as well, and in the 256x256 kernels
+// spilled registers (33-50 in all) are reloaded there.  Measured with this in place: stores kept in registers and sent between the MFMAs
+// of the next tile 86 us instead of 81; non-temporal ones 75, and 8192x50257x768 with them 620 -> 690; waits that leave
+// younger operations in flight the same.  None of it says what they would do without the drain.
+//
+// Rows and contraction indices past the operand's end read as zero (buffer descriptors).
 
 // TBM x TBN tile of C by WM x WN wavefronts
 template <int TBN_, int WM_, int WN_>
