@@ -7,8 +7,9 @@ round a branch is shorter than the other.  Neither shows in a source file, and t
 
 Rules (quarter-rate issue slots, as s_nop counts them): a result of v_mfma_*_bf16 (8 passes) may be read 12 slots later, of
 v_mfma_f32_32x32x2_f32 (16 passes) 18, and overwritten by the vector ALU one slot earlier (loads take longer than that to arrive);
-the next product is issued when the one before it has gone through its passes.  vmcnt and lgkmcnt count vector memory and LDS operations, which complete in order;
-scalar loads complete in any order.  A scalar register written by the vector ALU may address memory 5 slots later."""
+the next product is issued when the one before it has gone through its passes.  vmcnt and lgkmcnt count vector memory and LDS
+operations, which complete in order; scalar loads complete in any order.  What the vector ALU writes may be read across lanes
+(DPP, permlane) 2 slots later and, from a scalar register, by a memory address 5 slots later."""
 import concurrent.futures
 import os
 import re
@@ -39,7 +40,7 @@ class Instruction:
         self.slots, self.passes, self.factors = 1, 0, ()
         self.out = self.into = ()
         vector, lds = re.match(r"(global|buffer|flat|scratch)_", op), op.startswith("ds_")
-        self.vector_memory, self.vector_alu = bool(vector), False
+        self.vector_memory, self.vector_alu, self.lanes = bool(vector), False, False
         if op == "s_waitcnt":
             n = [re.search(r"\b%s\((\d+)\)" % c, rest) for c in ("vmcnt", "lgkmcnt")]
             self.wait = [int(m.group(1)) if m else 1 << 30 for m in n]
@@ -69,6 +70,7 @@ class Instruction:
             self.factors = registers(operands[1]) + registers(operands[2])
         self.out, self.into = out, into
         self.vector_alu = op.startswith("v_") and not self.passes
+        self.lanes = "permlane" in op or re.search(r"quad_perm|row_|wave_", rest)
 
 
 def findings(listing):
@@ -82,7 +84,7 @@ def findings(listing):
     found = {}
 
     def step(state, i):
-        x, (loads, products, scalars) = code[i], state
+        x, (loads, products, recent) = code[i], state
         if x.wait:
             vm, lgkm = x.wait
             loads = {r: (k, n) for r, (k, n) in loads.items()
@@ -105,22 +107,22 @@ def findings(listing):
                 for r in x.out if x.vector_alu else ():
                     if r in products and products[r][2] - products[r][0] > 1:
                         found[i, r] = "result of a product overwritten %d slots early" % (products[r][2] - products[r][0] - 1)
-            if scalars and x.vector_memory:
-                for r in x.into:
-                    if r in scalars:
-                        found[i, r] = "address too early"
+            for r in x.into if recent else ():
+                if r in recent and recent[r] < (5 if r[0] == "s" and x.vector_memory else 2 if r[0] == "v" and x.lanes else 0):
+                    found[i, r] = "read by %s too early" % ("an address" if r[0] == "s" else "another lane")
             if x.counter:
                 loads = {r: (k, n + (n < 64) if k == x.counter else n) for r, (k, n) in loads.items()}
             if x.load:
                 loads = {**loads, **{r: (x.load, 0) for r in x.out}}
         aged = {r: (max(e + 1, p) if x.passes else e + x.slots, p, n) for r, (e, p, n) in products.items()}
         products = {r: v for r, v in aged.items() if v[0] < v[2]}
-        scalars = {r: e + x.slots for r, e in scalars.items() if e + x.slots < 5 and not (x.op.startswith("s_") and r in x.out)}
+        recent = {r: e + x.slots for r, e in recent.items()
+                   if e + x.slots < (5 if r[0] == "s" else 2) and not (x.op.startswith("s_") and r in x.out)}
         if x.passes:
             products.update({r: (0, x.passes, 12 if x.passes == 8 else 18) for r in x.out})
         elif x.vector_alu:
-            scalars.update({r: 0 for r in x.out if r[0] == "s"})
-        return loads, products, scalars
+            recent.update({r: 0 for r in x.out})
+        return loads, products, recent
 
     def join(old, new):
         """`old` with what is nearer in `new`, or None if that adds nothing."""
@@ -220,9 +222,11 @@ def test_the_check_finds_what_is_missing():
     good = ["ds_read_b128 v[4:7], v0", "s_cbranch_scc0 L0", "s_nop 2", "L0:", "s_waitcnt lgkmcnt(0)",
             "v_mfma_f32_32x32x16_bf16 v[16:31], v[4:7], v[8:11], v[16:31]", "s_cbranch_vccz L1", "s_nop 9", "L1:", "s_nop 10",
             "v_mov_b32_e32 v2, v31", "global_load_dword v3, v[0:1], off", "global_load_dword v12, v[0:1], off", "s_waitcnt vmcnt(1)",
-            "v_add_f32_e32 v3, v3, v3", "v_readfirstlane_b32 s4, v3", "s_nop 4", "global_load_dword v13, v2, s[4:5]", "s_endpgm"]
+            "v_add_f32_e32 v3, v3, v3", "v_readfirstlane_b32 s4, v3", "s_nop 4", "global_load_dword v13, v2, s[4:5]",
+            "v_add_f32_e32 v14, v3, v3", "s_nop 1", "v_permlane32_swap_b32_e32 v14, v15", "s_nop 1",
+            "v_add_f32_dpp v15, v14, v14 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf", "s_endpgm"]
     assert findings(good) == []
-    for i, worse in ((4, None), (9, "s_nop 9"), (13, "s_waitcnt vmcnt(2)"), (13, None), (16, "s_nop 3")):
+    for i, worse in ((4, None), (9, "s_nop 9"), (13, "s_waitcnt vmcnt(2)"), (13, None), (16, "s_nop 3"), (19, "s_nop 0"), (21, "s_nop 0")):
         assert findings(good[:i] + ([worse] if worse else []) + good[i + 1:]), (good[i], worse)
     # a copy of what is still on its way, in front of the wait
     assert findings(good[:4] + ["v_mov_b64_e32 v[20:21], v[4:5]"] + good[4:])
