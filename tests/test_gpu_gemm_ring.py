@@ -1,6 +1,8 @@
 """The persistent bf16 GEMM kernels: sizes at which the size rule picks them, so that workgroups walk one, two or three tiles of
 either width, with borders in both directions, contraction lengths that end inside a step and inside a 16-byte vector, K splits,
 a last round that is split, accumulation onto C from one step per tile up, and operands whose rows overlap."""
+import importlib
+
 import pytest
 import torch
 
@@ -113,8 +115,9 @@ def test_ring_rows_that_overlap(mt, k):
 
 
 def test_ring_rows_far_apart(mt):
-    """Outputs and multipliers in column slices of buffers so wide that a lane's row leaves 32-bit offsets."""
-    n, m, k, pitch, at = 24, 136, 64, 150_000_000, 1_000_000
+    """Outputs and multipliers in column slices of buffers so wide that a lane's row leaves 32-bit offsets (the first 64 x 96 are
+    a wavefront's whole block)."""
+    n, m, k, pitch, at = 72, 136, 64, 150_000_000, 1_000_000
     g = gen(n)
     wide = torch.zeros(n, pitch, dtype=BF16, device=DEV)
     part = wide[:, at:at + m]
@@ -134,8 +137,16 @@ def test_ring_rows_far_apart(mt):
     assert torch.equal(part, out) and torch.equal(deriv[:, at:at + m], d)
     assert torch.count_nonzero(wide) == torch.count_nonzero(part) and torch.count_nonzero(deriv) == torch.count_nonzero(d)
     part.copy_(c0)
-    for x, y in zip(mt.matmul_mul_colsum_t(row, b, part), mt.matmul_mul_colsum_t(row, b, c0)):
+    c, sums = mt.matmul_mul_colsum_t(row, b, c0)
+    for x, y in zip(mt.matmul_mul_colsum_t(row, b, part), (c, sums)):
         assert torch.equal(x, y)
+    _lib = importlib.import_module("pre-tjax_amd._lib")
+    ws = torch.empty(_lib.lib().ptj_gemm_mul_colsum_workspace_bytes(n, m), dtype=torch.uint8, device=DEV)
+    sums2 = torch.empty_like(sums)
+    _lib.check(_lib.lib().ptj_gemm_mul_colsum(row.data_ptr(), b.data_ptr(), c0.data_ptr(), part.data_ptr(), sums2.data_ptr(), n, m, k,
+                                              *row.stride(), *b.stride(), m, pitch, ws.data_ptr(), ws.numel(), _lib.PTJ_BF16,
+                                              _lib.stream()), "ptj_gemm_mul_colsum")
+    assert torch.equal(part, c) and torch.equal(sums2, sums) and torch.count_nonzero(wide) == torch.count_nonzero(c)
 
 
 def test_ring_contraction_rows_far_apart(mt):
