@@ -93,16 +93,6 @@ namespace {
 using ptj_gemm_detail::GemmArgs;
 
 constexpr int BM = 256, BN = 192;   // C tile (rows from A, columns from B)
-// Register sets that stage operand panels between HBM and LDS: with 2, the loads of panel
-// kt+2 are issued during step kt and have one step to arrive; with 3, panel kt+3 is requested
-// during step kt and has two.
-constexpr int GEMM_MAX_STAGES = 3;
-// per operand layout and element size: only 2-byte operands that are copied as they are leave registers for a third
-// set (a transposing load holds its panel twice while it permutes: 104-126 spilled registers with three sets;
-// 4-byte storage: 50)
-constexpr int stages_for(int amode, int bmode, int elt) {
-    return (amode == KMAJOR && bmode == KMAJOR && elt == 2) ? GEMM_MAX_STAGES : 2;
-}
 constexpr int TM = 2, TN = 3;               // 32x32 MFMA tiles per wavefront (rows x columns)
 constexpr int WROWS = TM * 32;              // C rows per wavefront
 constexpr int WAVES_N = 2;                  // (BM/WROWS) x 2 wavefronts, each WROWS rows x 96 columns
@@ -203,7 +193,6 @@ __device__ __forceinline__ void gemm_run_fast(const GemmArgs& g, f32x16 (&acc)[T
                                               int row0, int col0, int kbeg, int nk) {
     constexpr int BK = BKB / (int)sizeof(T);
     constexpr int A_BYTES = BM * BKB, B_BYTES = BN * BKB;
-    constexpr int STAGES = stages_for(AMODE, BMODE, (int)sizeof(T));
     static_assert(TN == 3, "the pipeline below is written for three MFMA tile columns per wavefront");
     if (nk <= 0) return;
     const int tid = fresh_tid();
@@ -214,8 +203,8 @@ __device__ __forceinline__ void gemm_run_fast(const GemmArgs& g, f32x16 (&acc)[T
     const T* B = (const T*)g.b;
     char* sA = smem;
     char* sB = smem + 2 * A_BYTES;
-    TileLoader<T, AMODE, BM, GEMM_THREADS, true> la0, la1, la2;
-    TileLoader<T, BMODE, BN, GEMM_THREADS, true> lb0, lb1, lb2;
+    TileLoader<T, AMODE, BM, GEMM_THREADS, true> la0, la1;
+    TileLoader<T, BMODE, BN, GEMM_THREADS, true> lb0, lb1;
     typename Frag<T>::type fa[2][TM], fb[TN], fx[TN];
     const int last = nk - 1;
     const int arow = wm * WROWS + lr, brow = wn * 96 + lr;
@@ -272,34 +261,16 @@ __device__ __forceinline__ void gemm_run_fast(const GemmArgs& g, f32x16 (&acc)[T
     lb0.template load_fast_slice<0, 1, CLAMP>(B, g.b_row, g.b_k, col0, K0_OF(0), tid, g.m);
     la1.template load_fast_slice<0, 1, CLAMP>(A, g.a_row, g.a_k, row0, K0_OF(1), tid, g.n);
     lb1.template load_fast_slice<0, 1, CLAMP>(B, g.b_row, g.b_k, col0, K0_OF(1), tid, g.m);
-    if constexpr (STAGES == 3) {
-        la2.template load_fast_slice<0, 1, CLAMP>(A, g.a_row, g.a_k, row0, K0_OF(2), tid, g.n);
-        lb2.template load_fast_slice<0, 1, CLAMP>(B, g.b_row, g.b_k, col0, K0_OF(2), tid, g.m);
-    }
     la0.store(sA, tid);
     lb0.store(sB, tid);
     __syncthreads();
     RD_A(0, 0, 0); RD_B(fb[0], 0, 0, 0); RD_B(fb[1], 0, 0, 1); RD_B(fb[2], 0, 0, 2); SB();
     int kt = 0;
-    if constexpr (STAGES == 2) {
-        for (; kt + 1 < nk; kt += 2) {
-            RF_STEP(0, la1, lb1, la0, lb0, kt + 2);
-            RF_STEP(1, la0, lb0, la1, lb1, kt + 3);
-        }
-        if (kt < nk) RF_STEP(0, la1, lb1, la0, lb0, kt + 2);
-    } else {
-        // panel p waits in register set p mod 3; the LDS buffer alternates every step, so its
-        // index is a variable here (three steps flip it once)
-        int pb = 0;
-        for (; kt + 2 < nk; kt += 3) {
-            RF_STEP(pb, la1, lb1, la0, lb0, kt + 3);
-            RF_STEP(pb ^ 1, la2, lb2, la1, lb1, kt + 4);
-            RF_STEP(pb, la0, lb0, la2, lb2, kt + 5);
-            pb ^= 1;
-        }
-        if (kt < nk) RF_STEP(pb, la1, lb1, la0, lb0, kt + 3);
-        if (kt + 1 < nk) RF_STEP(pb ^ 1, la2, lb2, la1, lb1, kt + 4);
+    for (; kt + 1 < nk; kt += 2) {
+        RF_STEP(0, la1, lb1, la0, lb0, kt + 2);
+        RF_STEP(1, la0, lb0, la1, lb1, kt + 3);
     }
+    if (kt < nk) RF_STEP(0, la1, lb1, la0, lb0, kt + 2);
 #undef K0_OF
 #undef ROW_A
 #undef ROW_B
@@ -594,7 +565,6 @@ template <typename T, int AMODE, int BMODE, bool CLAMP, bool MUL>
 __device__ __forceinline__ void gemm_stream(const GemmArgs& g, char* __restrict__ smem) {
     constexpr int BK = BKB / (int)sizeof(T);
     constexpr int A_BYTES = BM * BKB, B_BYTES = BN * BKB;
-    constexpr int STAGES = stages_for(AMODE, BMODE, (int)sizeof(T));
     const int num_m = (g.n + BM - 1) / BM, num_n = (g.m + BN - 1) / BN;
     const int total = num_m * num_n;
     // work items: whole tiles, then (with a K-split last round) the K slices of its tiles
@@ -603,10 +573,9 @@ __device__ __forceinline__ void gemm_stream(const GemmArgs& g, char* __restrict_
     const T* B = (const T*)g.b;
     char* sA = smem;
     char* sB = smem + 2 * A_BYTES;
-    TileLoader<T, AMODE, BM, GEMM_THREADS, true> la0, la1, la2;
-    TileLoader<T, BMODE, BN, GEMM_THREADS, true> lb0, lb1, lb2;
+    TileLoader<T, AMODE, BM, GEMM_THREADS, true> la0, la1;
+    TileLoader<T, BMODE, BN, GEMM_THREADS, true> lb0, lb1;
     typename Frag<T>::type fa[2][TM], fb[TN], fx[TN];
-    int pb = 0;   // LDS buffer that holds the current tile's first panel (three staging sets only)
     // item -> tile origin, first contraction element, number of panels (even), partial tile
 #define STREAM_ITEM(ITEM, ROW0, COL0, KBEG, NK, PART)                                                    \
     do {                                                                                                 \
@@ -639,10 +608,6 @@ __device__ __forceinline__ void gemm_stream(const GemmArgs& g, char* __restrict_
         lb0.template load_fast_slice<0, 1, CLAMP>(B, g.b_row, g.b_k, col0, kbeg, tid, g.m);
         la1.template load_fast_slice<0, 1, CLAMP>(A, g.a_row, g.a_k, row0, kbeg + BK, tid, g.n);
         lb1.template load_fast_slice<0, 1, CLAMP>(B, g.b_row, g.b_k, col0, kbeg + BK, tid, g.m);
-        if constexpr (STAGES == 3) {
-            la2.template load_fast_slice<0, 1, CLAMP>(A, g.a_row, g.a_k, row0, kbeg + 2 * BK, tid, g.n);
-            lb2.template load_fast_slice<0, 1, CLAMP>(B, g.b_row, g.b_k, col0, kbeg + 2 * BK, tid, g.m);
-        }
         la0.store(sA, tid);
         lb0.store(sB, tid);
         __syncthreads();
@@ -669,20 +634,9 @@ __device__ __forceinline__ void gemm_stream(const GemmArgs& g, char* __restrict_
 #define K0_OF(KT) ((KT) < nk ? kbeg + (KT) * BK : nkbeg + ((KT) - nk) * BK)
 #define ROW_A(KT) ((KT) < nk ? row0 : nrow0)
 #define ROW_B(KT) ((KT) < nk ? col0 : ncol0)
-            if constexpr (STAGES == 2) {
-                for (int kt = 0; kt < nk; kt += 2) {
-                    RF_STEP(0, la1, lb1, la0, lb0, kt + 2);
-                    RF_STEP(1, la0, lb0, la1, lb1, kt + 3);
-                }
-            } else {
-                // nk is a multiple of 3 here: every tile starts with its panels 0, 1, 2 in LDS
-                // buffer pb, set 1 and set 2
-                for (int kt = 0; kt < nk; kt += 3) {
-                    RF_STEP(pb, la1, lb1, la0, lb0, kt + 3);
-                    RF_STEP(pb ^ 1, la2, lb2, la1, lb1, kt + 4);
-                    RF_STEP(pb, la0, lb0, la2, lb2, kt + 5);
-                    pb ^= 1;
-                }
+            for (int kt = 0; kt < nk; kt += 2) {
+                RF_STEP(0, la1, lb1, la0, lb0, kt + 2);
+                RF_STEP(1, la0, lb0, la1, lb1, kt + 3);
             }
 #undef K0_OF
 #undef ROW_A
@@ -945,15 +899,7 @@ inline int stride_mode(int64_t s_row, int64_t s_k) { return s_k == 1 ? KMAJOR : 
 template <typename T, bool MUL = false>
 int gemm_impl(GemmArgs g, int splits, hipStream_t st) {
     const int am = pick_mode<T>(g.a, g.a_row, g.a_k), bm = pick_mode<T>(g.b, g.b_row, g.b_k);
-    {
-        // the streamed loop takes K panels in groups of as many as there are staging sets
-        const int sg = stages_for(am, bm, (int)sizeof(T)), bk = BKB / (int)sizeof(T);
-        if (g.stream && !(g.k >= sg * bk && g.k % (sg * bk) == 0)) g.stream = 0;
-        if (sg != 2 && g.tail_splits > 1) {      // K slices of the last round come in pairs of panels
-            g.tail_first = 0; g.tail_splits = 1; g.tail_kps = 0;
-            if (splits == 1) g.partial = nullptr;
-        }
-    }
+    if (g.k % (2 * (BKB / (int)sizeof(T))) != 0) g.stream = 0;     // the streamed loop takes K panels in pairs
     const int num_m = (g.n + BM - 1) / BM, num_n = (g.m + BN - 1) / BN;
     int64_t work = (int64_t)num_m * num_n * splits;
     if (g.tail_splits > 1) work = g.tail_first + ((int64_t)num_m * num_n - g.tail_first) * g.tail_splits;
