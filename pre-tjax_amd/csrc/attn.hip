@@ -1,5 +1,6 @@
 // Causal flash attention for gfx950, head dimension 64: forward, and a backward that
-// recomputes P from the saved row max / row sum-exp.
+// recomputes P from the saved row max / row sum-exp.  The kernels of 2-byte storage, what masks and dropout need, and the C entry
+// points; 4-byte storage: attn_f32.hip.
 //
 // Layout trick shared by the three MFMA kernels: scores are produced TRANSPOSED.  With
 // 32x32 MFMA tiles, D[m][n] of lane l sits at n = l & 31, m = 8*(i/4) + 4*(l>>5) + i%4
@@ -10,9 +11,8 @@
 // lane's registers), so P never travels through LDS.  The dK/dV pass computes S = Q K^T
 // with the same trick mirrored: a lane owns one key, dV^T = dO^T P and dK^T = Q^T dS.
 // The operand that must be read "across" its memory layout (V^T, K^T, Q^T, dO^T: row
-// index d, contraction along keys / queries): 2-byte storage reads it out of the same rows
-// with transposing LDS reads, 4-byte storage transposes it once while it is written to LDS
-// (MNMAJOR panel loader); the four wavefronts share it.
+// index d, contraction along keys / queries) comes out of the same rows in LDS with transposing reads;
+// the four wavefronts share it.
 //
 // Softmax is evaluated in base 2 (scores pre-multiplied by log2(e)/sqrt(dh)); the saved
 // statistics `ms` are converted back to natural units.  Masked scores take the
@@ -35,74 +35,22 @@
 // The backward is two passes without atomics: dQ over query tiles (it also forms
 // delta = rowsum(dO * O) of its queries and stores it), then (dK, dV) over key tiles,
 // which reads delta; both recompute S and dP.
-#include "common.h"
-#include "internal.h"
-#include "mma_tile.h"
+#include "attn_common.h"
 
 namespace {
 
-constexpr int DH = 64;
 constexpr int ATT_THREADS = 256;
-constexpr int PANEL = 64 * BKB;  // bytes of one 64-row LDS panel
 constexpr int MAX_T = 8192;
 constexpr int MAX_BITWORDS = 2 * MAX_T / 32 + 2;
-constexpr float LOG2E = 1.4426950408889634f;
-constexpr float LN2 = 0.6931471805599453f;
-constexpr float NEG_NAT = -1e9f;
-constexpr float NEG2 = NEG_NAT * LOG2E;
 
-template <typename T> struct AT {
-    static constexpr int ROWB = DH * (int)sizeof(T);   // bytes per q/k/v row: 128 / 256
-    static constexpr int NP = ROWB / BKB;               // panels per 64-element axis: 1 / 2
-    static constexpr int NC = ROWB / 32;                // contraction chunks along d: 4 / 8
-    static constexpr int EPP = BKB / (int)sizeof(T);    // elements per panel row: 64 / 32
-    typedef typename Frag<T>::type F;
-};
+typedef bf16x8 RowPieces[4];   // the MFMA operand pieces of one 64-element row (lane half lg)
 
-struct AttnArgs {
-    const void *q, *k, *v, *o, *d_o;
-    void *out0, *out1, *out2;     // forward: out0 = O.  Backward: dK, dV, dQ
-    // nullptr = causal by index; else the mask bit-packed in both orientations (ptj_attn_pack_mask):
-    //   words [0, B*T/32*T):   word (b, q/32, k) holds M[b, 32*(q/32) + r, k] in bit r   (lane = query)
-    //   then the same amount:  word (b, k/32, q) holds M[b, q, 32*(k/32) + r] in bit r   (lane = key)
-    //   then B*(T/32)^2 words:  class of tile (b, q/32, k/32), then the same indexed (b, k/32, q/32)
-    const uint32_t* mask;
-    float *ms, *ls;               // [BH, T]
-    float* delta;                 // [BH, T] rowsum(dO * O)  (backward in two launches: dQ writes it, dK/dV reads it)
-    const uint32_t* keepbits;     // [BH, bitwords]  (train)
-    int B, H, T, bitwords;
-    // element strides: batch, head, row (the head dimension itself has unit stride)
-    int64_t q_bs, q_hs, q_rs, k_bs, k_hs, k_rs, v_bs, v_hs, v_rs, o_bs, o_hs, o_rs, do_bs, do_hs, do_rs;
-    int64_t out0_bs, out0_hs, out0_rs, out1_bs, out1_hs, out1_rs, out2_bs, out2_hs, out2_rs;
-    int train;
-    float scale;                  // 1/sqrt(dh)
-};
-
-// ---- small device helpers -----------------------------------------------------------
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-__device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32, 64); }
-// max / sum of a value with its partner in the other half of the wavefront (lane ^ 32), the same
-// in both lanes: v_permlane32_swap exchanges the upper half of one register with the lower half
-// of another inside the vector ALU (no LDS round trip); with both registers holding v the two
-// results are {lo, lo} and {hi, hi}.
-__device__ __forceinline__ float max_xor32(float v) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float sum_xor32(float v) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// The 16-byte operand pieces of one 64-element row held in registers (lane half lg).
-template <typename T>
-__device__ __forceinline__ void load_row_frags(typename AT<T>::F (&f)[AT<T>::NC], const T* __restrict__ row, int lg) {
+__device__ __forceinline__ void load_row_frags(RowPieces& f, const bf16* __restrict__ row, int lg) {
 #pragma unroll
-    for (int c = 0; c < AT<T>::NC; ++c)
-        f[c] = *reinterpret_cast<const typename AT<T>::F*>(reinterpret_cast<const char*>(row) + c * 32 + lg * 16);
+    for (int c = 0; c < 4; ++c) f[c] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(row) + c * 32 + lg * 16);
 }
 
-// ---- tiles of 2-byte storage: copied straight into LDS --------------------------------------
+// ---- tiles, copied straight into LDS ---------------------------------------------------------
 // Tiles go from memory into LDS without registers, two tiles ahead of their use, and lie there once.  Before, they went
 // through registers one tile ahead and lay in LDS a second time, transposed by vector permutes: dK/dV and dQ read Q, dO and
 // K from memory twice, and a third of the vector instructions of a step were the loader's.  Batch 8 x 1024 x 12 heads,
@@ -118,7 +66,6 @@ __device__ __forceinline__ void load_row_frags(typename AT<T>::F (&f)[AT<T>::NC]
 // (TpFrags), so ONE panel serves both directions.
 constexpr int RING = 3;                   // tiles in LDS: one in use, two on their way
 constexpr int WAVE_COPY = 64 * 16;        // bytes of one copy of a wavefront: eight rows
-__device__ __forceinline__ int row_swizzle(int row) { return ((row & 2) << 1) | ((row >> 2) & 3); }
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
 }
@@ -165,21 +112,8 @@ __device__ __forceinline__ int next_slot(int slot) { return slot == RING - 1 ? 0
 
 // s += panel_rows(j*32 + lr) x register_rows : panel rows become MFMA rows (m), the
 // lane's register row the MFMA column (n); contraction over the 64-element axis d.
-// (2-byte storage: NJ sub-tiles' fragments are read together ahead of the products, RowFrags::read)
-template <typename T, int NJ> struct RowFrags {
-    __device__ __forceinline__ void read(const char* __restrict__, int, int, int) {}
-    __device__ __forceinline__ void mma(f32x16 (&s)[NJ], const char* __restrict__ panels, const typename AT<T>::F (&f)[AT<T>::NC],
-                                        int j0, int lr, int lg) const {
-#pragma unroll
-        for (int c = 0; c < AT<T>::NC; ++c)
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                typename AT<T>::F a = read_frag<T>(panels + (c / 4) * PANEL, (j0 + j) * 32 + lr, (c % 4) * 2 + lg);
-                mma_chunk(s[j], a, f[c]);
-            }
-    }
-};
-template <int NJ> struct RowFrags<bf16, NJ> {
+// (NJ sub-tiles' fragments are read together ahead of the products)
+template <int NJ> struct RowFrags {
     bf16x8 a[NJ][4];
     __device__ __forceinline__ void read(const char* __restrict__ panel, int j0, int lr, int lg) {
 #pragma unroll
@@ -188,7 +122,7 @@ template <int NJ> struct RowFrags<bf16, NJ> {
             for (int j = 0; j < NJ; ++j)
                 a[j][c] = *reinterpret_cast<const bf16x8*>(panel + ((j0 + j) * 32 + lr) * BKB + (((c * 2 + lg) ^ row_swizzle(lr)) << 4));
     }
-    __device__ __forceinline__ void mma(f32x16 (&s)[NJ], const char* __restrict__, const bf16x8 (&f)[4], int, int, int) const {
+    __device__ __forceinline__ void mma(f32x16 (&s)[NJ], const RowPieces& f) const {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -212,28 +146,10 @@ __device__ __forceinline__ bf16x8 pack8_bf16(const float* __restrict__ p) {
 // o[t] += transposed panel (row t*32 + lr of the transpose) x p : contraction over the 32 positions of
 // sub-tile j whose values p[i] the lane holds in accumulator order
 // (position = j*32 + 8*(i/4) + 4*lg + i%4).
-__device__ __forceinline__ void tp_x_regs_one(f32x16 (&o)[2], const char* __restrict__ panels, const float (&p)[16],
-                                              int j, int lr, int lg) {
-    const char* pp = panels + j * PANEL;
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const f32x4 v = read_frag<float>(pp, t * 32 + lr, 2 * a + lg);
-#pragma unroll
-            for (int b = 0; b < 4; ++b) o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[b], p[4 * a + b], o[t], 0, 0, 0);
-        }
-}
 // The panel's fragments are read ahead of the element-wise work that forms p (TpFrags::read), so that their way out of LDS is
 // hidden behind it.
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
-template <typename T> struct TpFrags {
-    __device__ __forceinline__ void read(const char* __restrict__, int, int, int) {}
-    __device__ __forceinline__ void mma(f32x16 (&o)[2], const char* __restrict__ panels, const float (&p)[16], int j, int lr, int lg) const {
-        tp_x_regs_one(o, panels, p, j, lr, lg);
-    }
-};
-template <> struct TpFrags<bf16> {
+struct TpFrags {
     bf16x8 a[2][2];
     // transposing reads: sixteen lanes fetch four positions x 16 columns, each ends up with the four positions of its column;
     // two of them make the eight positions that a lane holds of p, in the same order
@@ -250,7 +166,7 @@ template <> struct TpFrags<bf16> {
                 a[h][t] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
             }
     }
-    __device__ __forceinline__ void mma(f32x16 (&o)[2], const char* __restrict__, const float (&p)[16], int, int, int) const {
+    __device__ __forceinline__ void mma(f32x16 (&o)[2], const float (&p)[16]) const {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const bf16x8 b = pack8_bf16(&p[8 * h]);
@@ -259,88 +175,6 @@ template <> struct TpFrags<bf16> {
         }
     }
 };
-// Keep bits of one wavefront tile as wave-uniform (scalar) words.  Element (q, k) is kept
-// iff bit q + k of the batch-head's line is set.  In the kernels whose lanes are queries
-// (keys), the element in accumulator register i of sub-tile j sits at
-//   q + k = base + C + (lane & 31) + 4 * (lane >> 5),   C = 32 j + 8 (i / 4) + i % 4,
-// with base = (wave's first query) + (tile's first key), a multiple of 32.  So the keep
-// decision of ONE register across the 64 lanes is two 32-bit windows of the line at the
-// constant offsets C and C + 4: a lane mask that the scalar unit extracts with two
-// shifts and that a single v_cndmask applies -- no per-lane bit arithmetic at all.
-// Words that no kernel here writes, at wave-uniform addresses: scalar loads, also between the inline assembly's memory clobbers.
-typedef __attribute__((address_space(4))) const uint32_t* uniform_words;
-__device__ __forceinline__ uniform_words as_uniform(const uint32_t* p) { return (uniform_words)(uintptr_t)p; }
-// First row of a wavefront where it looks up such words.  With T an odd multiple of 64 the last workgroup's upper two
-// wavefronts have no rows; theirs would be words past the end of the lines and of the mask, so they read those of the lower two.
-__device__ __forceinline__ int lookup_row(int row0, int T) { return row0 - (row0 < T ? 0 : 64); }
-struct KeepWords { uint32_t d0, d1, d2; };
-__device__ __forceinline__ KeepWords load_keep_words(const uint32_t* __restrict__ line, int base) {
-    const uniform_words p = as_uniform(line + (base >> 5));
-    KeepWords w;
-    w.d0 = p[0];
-    w.d1 = p[1];
-    w.d2 = p[2];
-    return w;
-}
-template <int C> __device__ __forceinline__ uint32_t keep_win32(const KeepWords& w) {
-    static_assert(C >= 0 && C < 64, "window offset");
-    const uint64_t v = C < 32 ? (((uint64_t)w.d1 << 32) | w.d0) : (((uint64_t)w.d2 << 32) | w.d1);
-    return (uint32_t)(v >> (C & 31));
-}
-template <int C> __device__ __forceinline__ uint64_t keep_lane_mask(const KeepWords& w) {
-    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-    const u32x2_t halves = {keep_win32<C>(w), keep_win32<C + 4>(w)};
-    return __builtin_bit_cast(uint64_t, halves);
-}
-// The same for an offset that is a constant only after loop unrolling.
-__device__ __forceinline__ uint64_t keep_lane_mask_at(const KeepWords& w, int c) {
-    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-    const uint64_t lo_pair = ((uint64_t)w.d1 << 32) | w.d0, hi_pair = ((uint64_t)w.d2 << 32) | w.d1;
-    const int c4 = c + 4;
-    const u32x2_t halves = {(uint32_t)((c < 32 ? lo_pair : hi_pair) >> (c & 31)),
-                            (uint32_t)((c4 < 32 ? lo_pair : hi_pair) >> (c4 & 31))};
-    return __builtin_bit_cast(uint64_t, halves);
-}
-// v where the lane's bit of `mask` is set, else 0.  The builtin turns a wave-uniform 64-bit
-// mask into a per-lane condition, i.e. one v_cndmask with the mask in scalar registers
-// (left to the compiler rather than inline assembly so that its hazard handling --
-// e.g. the wait state after a transcendental -- still applies).
-__device__ __forceinline__ float keep_select(float v, uint64_t mask) {
-    return __builtin_amdgcn_inverse_ballot_w64(mask) ? v : 0.f;
-}
-// Attention-mask words -> lane mask of accumulator register i of a 32x32 sub-tile: the
-// register holds column c = (i/4)*8 + i%4 for lanes 0..31 and column c + 4 for lanes 32..63,
-// and word w[c] carries the mask bits of the 32 lanes' rows for column c.
-__device__ __forceinline__ uint64_t mask_lanes(const uint32_t (&w)[32], int i) {
-    const int c = (i >> 2) * 8 + (i & 3);
-    return (uint64_t)w[c] | ((uint64_t)w[c + 4] << 32);
-}
-__device__ __forceinline__ float mask_select(float v, float other, uint64_t mask) {
-    return __builtin_amdgcn_inverse_ballot_w64(mask) ? v : other;
-}
-// p[i] = keep ? p[i] : 0 for the 16 registers of sub-tile J
-template <int J, int I = 0>
-__device__ __forceinline__ void keep_apply(float (&p)[16], const KeepWords& w) {
-    if constexpr (I < 16) {
-        p[I] = keep_select(p[I], keep_lane_mask<J * 32 + (I >> 2) * 8 + (I & 3)>(w));
-        keep_apply<J, I + 1>(p, w);
-    }
-}
-
-// Store the transposed accumulators acc[t][i] (row = the lane's position `pos`, column
-// d = t*32 + 8*(i/4) + 4*lg + i%4) scaled by `f` as rows of a [.., 64] tensor.
-template <typename T>
-__device__ __forceinline__ void store_rows(T* __restrict__ row, const f32x16 (&acc)[2], float f, int lg) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            float v[4];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) v[b] = acc[t][4 * a + b] * f;
-            store_vec<T, 4>(row + t * 32 + a * 8 + lg * 4, v);
-        }
-}
 
 // ---- keep-bit line per batch-head ---------------------------------------------------
 constexpr int KEEP_SEEDS = 64;   // attention calls per launch
@@ -389,7 +223,6 @@ __global__ __launch_bounds__(256) void attn_pack_mask_kernel(const uint8_t* __re
 //   TILE_HIDDEN  no element visible
 //   TILE_MIXED   anything else: the mask words are needed
 // written twice: cq[(b, q/32, k/32)] and ck[(b, k/32, q/32)].
-enum { TILE_HIDDEN = 0, TILE_MIXED = 1, TILE_CAUSAL = 2 };
 __global__ __launch_bounds__(256) void attn_mask_classes_kernel(const uint32_t* __restrict__ packed,
                                                                  uint32_t* __restrict__ cq, uint32_t* __restrict__ ck,
                                                                  int B, int T) {
@@ -422,30 +255,6 @@ __device__ __forceinline__ TileClasses load_classes(const uint32_t* __restrict__
     return c;
 }
 
-// ---- element-wise pieces (VALU budget: a wave64 VALU op costs 4 cycles, v_exp 16, and one
-//      K tile gives each lane 32 score elements against 16 MFMAs = 512 cycles; every
-//      instruction per element counts, so masks and dropout are compiled in only where used)
-constexpr float NEG_RAW = -8e9f;          // masked raw score: NEG_RAW * (1/sqrt(64)) = -1e9
-constexpr float RESCALE_SLACK = 8.0f;     // forward: the reference point of the exponentials may lag the row maximum by 2^8
-constexpr float M_START = -1e8f;          // log2-domain start of the running maximum: above every masked score
-                                          // (-1.44e9), below every real one, so exp2(masked - m) is exactly 0
-
-// Causal visibility of the lane's 16 elements of a sub-tile written into the raw scores
-// (invisible -> NEG_RAW).
-//   pos0 = (lane's own index) - (first index of the sub-tile along registers) - 4*lg
-//   element i = 4a+b sits at register offset 8a+b: visible iff 8a+b <= pos0 (causal part).
-template <bool LANE_IS_QUERY>
-__device__ __forceinline__ void apply_causal(f32x16& s, int pos0) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int off = (i >> 2) * 8 + (i & 3);
-        // lane = query: key offset must be <= query;  lane = key: query offset must be >= key
-        const bool ok = LANE_IS_QUERY ? (off <= pos0) : (off >= pos0);
-        s[i] = ok ? s[i] : NEG_RAW;
-    }
-}
-
-
 // Which tile and batch-head a workgroup of a grid (B*H, tiles) takes.  In dispatch order tiles go from long to short; every
 // second layer of 256 workgroups (one per CU) runs backwards, so that the CU with the longest of one layer gets the shortest of
 // the next instead of the longest again.  Only whole layers are turned, and a workgroup keeps its number modulo 8, hence its
@@ -461,13 +270,11 @@ __device__ __forceinline__ Place place() {
 
 // ---- forward -------------------------------------------------------------------------
 // grid (B*H, ceil(T/128)), see place(); wave w owns queries q0 + 32w .. +31; K/V tiles of 64 keys.
-template <typename T, bool HAS_MASK, bool TRAIN>
-// (2-byte storage: three workgroups per CU = three wavefronts per SIMD, 168 registers each)
-__global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_kernel(const AttnArgs a) {
-    typedef AT<T> X;
-    constexpr bool ASYNC = sizeof(T) == 2;
-    constexpr int STAGE = 2 * X::NP * PANEL;  // K panels then V (4-byte storage: V^T) panels
-    __shared__ __attribute__((aligned(16))) char smem[(ASYNC ? RING : 2) * STAGE];
+// (three workgroups per CU = three wavefronts per SIMD, 168 registers each)
+template <bool HAS_MASK, bool TRAIN>
+__global__ __launch_bounds__(ATT_THREADS, 3) void attn_fwd_kernel(const AttnArgs a) {
+    constexpr int STAGE = 2 * PANEL;          // K, V
+    __shared__ __attribute__((aligned(16))) char smem[RING * STAGE];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lg = lane >> 5;
@@ -481,30 +288,15 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
     const int query = qw0 + lr;
     const int qrow = query < a.T ? query : a.T - 1;
 
-    const T* Qb = (const T*)a.q + bidx * a.q_bs + hidx * a.q_hs;
-    const T* Kb = (const T*)a.k + bidx * a.k_bs + hidx * a.k_hs;
-    const T* Vb = (const T*)a.v + bidx * a.v_bs + hidx * a.v_hs;
+    const bf16* Qb = (const bf16*)a.q + bidx * a.q_bs + hidx * a.q_hs;
+    const bf16* Kb = (const bf16*)a.k + bidx * a.k_bs + hidx * a.k_hs;
+    const bf16* Vb = (const bf16*)a.v + bidx * a.v_bs + hidx * a.v_hs;
 
-    typename X::F qf[X::NC];
-    load_row_frags<T>(qf, Qb + (int64_t)qrow * a.q_rs, lg);
+    RowPieces qf;
+    load_row_frags(qf, Qb + (int64_t)qrow * a.q_rs, lg);
 
     int nkt = (q0 + 128) / 64;
     if (nkt > a.T / 64) nkt = a.T / 64;
-
-    // Flat code (no closures) keeps the prefetch registers plain SSA values; the last step
-    // re-fetches its own tile instead of branching.
-    TileLoader<T, KMAJOR, 64, ATT_THREADS> lk[X::NP];
-    TileLoader<T, MNMAJOR, 64, ATT_THREADS> lv[X::NP];
-#define FWD_FETCH(KT)                                                                  \
-    _Pragma("unroll") for (int p = 0; p < X::NP; ++p) {                                \
-        lk[p].load_fast(Kb, a.k_rs, 1, (KT) * 64, p * X::EPP, tid);                    \
-        lv[p].load_fast(Vb, 1, a.v_rs, 0, (KT) * 64 + p * X::EPP, tid);                \
-    }
-#define FWD_STASH(ST)                                                                  \
-    _Pragma("unroll") for (int p = 0; p < X::NP; ++p) {                                \
-        lk[p].store(smem + (ST) * STAGE + p * PANEL, tid);                             \
-        lv[p].store(smem + (ST) * STAGE + (X::NP + p) * PANEL, tid);                   \
-    }
 
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const uint32_t lds0 = lds_addr(smem);
@@ -514,23 +306,16 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
         ck.issue(KT, lds0 + (SLOT) * STAGE, wave_u);                                   \
         cv.issue(KT, lds0 + (SLOT) * STAGE + PANEL, wave_u);                           \
     }
-    if constexpr (ASYNC) {
-        ck.init(Kb, a.k_rs, tid);
-        cv.init(Vb, a.v_rs, tid);
-        FWD_COPY(0, 0)
-        frags_landed(qf);
-        if (nkt > 1) FWD_COPY(1, 1)
-    } else FWD_FETCH(0)
+    ck.init(Kb, a.k_rs, tid);
+    cv.init(Vb, a.v_rs, tid);
+    FWD_COPY(0, 0)
+    frags_landed(qf);
+    if (nkt > 1) FWD_COPY(1, 1)
     // keep-bit line of this batch-head and the wave's first query as scalars
     const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
     const int qw0u = lookup_row(q0 + wave_u * 32, a.T);
-    if constexpr (ASYNC) {
-        copies_landed<4>(nkt > 1);
-        lds_barrier();
-    } else {
-        FWD_STASH(0)
-        __syncthreads();
-    }
+    copies_landed<4>(nkt > 1);
+    lds_barrier();
 
     const float sc = a.scale * LOG2E;
     float m_run = M_START, m_true = M_START, l_run = 0.f;
@@ -552,9 +337,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
     }
     int st = 0;   // this tile's place in LDS
     for (int kt = 0; kt < nkt; ++kt) {
-        if constexpr (ASYNC) {
-            if (kt + 2 < nkt) FWD_COPY(kt + 2, next_slot(next_slot(st)))
-        } else FWD_FETCH(kt + 1 < nkt ? kt + 1 : kt)
+        if (kt + 2 < nkt) FWD_COPY(kt + 2, next_slot(next_slot(st)))
         // keep bits and classes of this tile were requested one step ago; request the next tile's now
         const KeepWords kw = kw_next;
         if constexpr (TRAIN) kw_next = load_keep_words(kline, qw0u + (kt + 1) * 64);
@@ -565,20 +348,20 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
         // some key of this tile is visible to some query of the wave
         if (key0 <= qw0 + 31 && (!HAS_MASK || (tc.c0 | tc.c1) != TILE_HIDDEN)) {
             const char* kp = smem + st * STAGE;
-            const char* vp = kp + X::NP * PANEL;
-            RowFrags<T, 2> ka;
+            const char* vp = kp + PANEL;
+            RowFrags<2> ka;
             ka.read(kp, 0, lr, lg);
-            if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_sched_barrier(0);
             f32x16 s[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) s[j][e] = 0.f;
-            ka.mma(s, kp, qf, 0, lr, lg);
-            TpFrags<T> va[2];
+            ka.mma(s, qf);
+            TpFrags va[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) va[j].read(vp, j, lr, lg);
-            if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_sched_barrier(0);
 
             if (key0 + 63 > qw0) {   // tile touches the diagonal for this wave
 #pragma unroll
@@ -636,28 +419,20 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_fwd_
                 keep_apply<1>(p[1], kw);
             }
 #pragma unroll
-            for (int j = 0; j < 2; ++j) va[j].mma(o, vp, p[j], j, lr, lg);
+            for (int j = 0; j < 2; ++j) va[j].mma(o, p[j]);
         }
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (ASYNC) {
-            copies_landed<4>(kt + 2 < nkt);
-            lds_barrier();
-            st = next_slot(st);
-        } else {
-            st ^= 1;
-            FWD_STASH(st)
-            __syncthreads();
-        }
+        copies_landed<4>(kt + 2 < nkt);
+        lds_barrier();
+        st = next_slot(st);
     }
 #undef FWD_COPY
-#undef FWD_FETCH
-#undef FWD_STASH
 
     if (query < a.T) {
         // l_run = 0: no key of the row is visible (a row with a visible key has l_run >= 1)
         const bool empty = l_run == 0.f;
         const float f = empty ? 0.f : (TRAIN ? 1.0f : 0.9f) / l_run;
-        store_rows<T>((T*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs, o, f, lg);
+        store_rows<bf16>((bf16*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs, o, f, lg);
         if (lg == 0) {
             // statistics relative to the true row maximum: sum exp(s - m_true) = l_run 2^(m_run - m_true)
             a.ms[(int64_t)bh * a.T + query] = empty ? NEG_NAT : m_true * LN2;
@@ -686,15 +461,11 @@ __device__ __forceinline__ void store_delta(float* __restrict__ delta, int i, fl
     if ((tid & 7) == 0) delta[(tid >> 3) + 32 * i] = part;
 }
 constexpr int RAW_STATS = 3 * 64 * 4;     // bytes of a query tile's saved maxima, sums and delta
-constexpr int dkdv_stage(bool own_delta) { return (own_delta ? 3 : 2) * PANEL + RAW_STATS; }   // 2-byte storage: Q, dO (, O), statistics
-template <typename T, bool OWN_DELTA> constexpr int dkdv_lds() {
-    return sizeof(T) == 2 ? RING * dkdv_stage(OWN_DELTA) : 2 * 4 * AT<T>::NP * PANEL;
-}
-template <typename T, bool HAS_MASK, bool TRAIN, bool OWN_DELTA>
+constexpr int dkdv_stage(bool own_delta) { return (own_delta ? 3 : 2) * PANEL + RAW_STATS; }   // Q, dO (, O), statistics
+template <bool OWN_DELTA> constexpr int dkdv_lds() { return RING * dkdv_stage(OWN_DELTA); }
+template <bool HAS_MASK, bool TRAIN, bool OWN_DELTA>
 __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, const int key_tile, char* smem, StatTile* sstat) {
-    typedef AT<T> X;
-    constexpr bool ASYNC = sizeof(T) == 2;
-    constexpr int STAGE = ASYNC ? dkdv_stage(OWN_DELTA) : 4 * X::NP * PANEL;  // 4-byte storage: Q, dO, Q^T, dO^T
+    constexpr int STAGE = dkdv_stage(OWN_DELTA);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lg = lane >> 5;
@@ -704,63 +475,22 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
     const int key = kw0 + lr;
     const int krow = key < a.T ? key : a.T - 1;
 
-    const T* Qb = (const T*)a.q + bidx * a.q_bs + hidx * a.q_hs;
-    const T* Kb = (const T*)a.k + bidx * a.k_bs + hidx * a.k_hs;
-    const T* Vb = (const T*)a.v + bidx * a.v_bs + hidx * a.v_hs;
-    const T* dOb = (const T*)a.d_o + bidx * a.do_bs + hidx * a.do_hs;
-    const T* Ob = (const T*)a.o + bidx * a.o_bs + hidx * a.o_hs;
+    const bf16* Qb = (const bf16*)a.q + bidx * a.q_bs + hidx * a.q_hs;
+    const bf16* Kb = (const bf16*)a.k + bidx * a.k_bs + hidx * a.k_hs;
+    const bf16* Vb = (const bf16*)a.v + bidx * a.v_bs + hidx * a.v_hs;
+    const bf16* dOb = (const bf16*)a.d_o + bidx * a.do_bs + hidx * a.do_hs;
+    const bf16* Ob = (const bf16*)a.o + bidx * a.o_bs + hidx * a.o_hs;
 
-    typename X::F kf[X::NC], vf[X::NC];
-    load_row_frags<T>(kf, Kb + (int64_t)krow * a.k_rs, lg);
-    load_row_frags<T>(vf, Vb + (int64_t)krow * a.v_rs, lg);
+    RowPieces kf, vf;
+    load_row_frags(kf, Kb + (int64_t)krow * a.k_rs, lg);
+    load_row_frags(vf, Vb + (int64_t)krow * a.v_rs, lg);
 
     const int qt0 = key0 / 64, nqt = a.T / 64;
 
-    TileLoader<T, KMAJOR, 64, ATT_THREADS> lq[X::NP], ld[X::NP], lo[OWN_DELTA ? X::NP : 1];
-    TileLoader<T, MNMAJOR, 64, ATT_THREADS> lqt[X::NP], ldt[X::NP];
-    float st_m = 0.f, st_l = 1.f, st_d = 0.f;
-    // 2-byte storage: 1/l goes into the exponent (p = 2^(s - m - log2 l)), one multiplication less
-    // per element.  A row without a visible key (saved l = 0) gets m = 0 and 1/l = 0 instead: all
+    // 1/l goes into the exponent (p = 2^(s - m - log2 l)), one multiplication less
+    // per element.  A row without a visible key (saved l = 0) gets m = 0 and no log2 l instead: all
     // of its scores are masked (-1.44e9 in the exponent), so its p is exactly 0.
-    constexpr bool FOLD_L = sizeof(T) == 2;
     const int64_t stat0 = (int64_t)bh * a.T + (tid & 63);
-#define KV_FETCH(QT)                                                                   \
-    {                                                                                  \
-        const int q0__ = (QT) * 64;                                                    \
-        _Pragma("unroll") for (int p = 0; p < X::NP; ++p) {                            \
-            lq[p].load_fast(Qb, a.q_rs, 1, q0__, p * X::EPP, tid);                     \
-            ld[p].load_fast(dOb, a.do_rs, 1, q0__, p * X::EPP, tid);                   \
-            lqt[p].load_fast(Qb, 1, a.q_rs, 0, q0__ + p * X::EPP, tid);                \
-            ldt[p].load_fast(dOb, 1, a.do_rs, 0, q0__ + p * X::EPP, tid);              \
-            if constexpr (OWN_DELTA) lo[p].load_fast(Ob, a.o_rs, 1, q0__, p * X::EPP, tid); \
-        }                                                                              \
-        st_m = a.ms[stat0 + q0__];                                                     \
-        st_l = a.ls[stat0 + q0__];                                                     \
-        if constexpr (!OWN_DELTA) st_d = a.delta[stat0 + q0__];                        \
-    }
-#define KV_STASH(ST)                                                                   \
-    {                                                                                  \
-        char* base__ = smem + (ST) * STAGE;                                            \
-        _Pragma("unroll") for (int p = 0; p < X::NP; ++p) {                            \
-            lq[p].store(base__ + p * PANEL, tid);                                      \
-            ld[p].store(base__ + (X::NP + p) * PANEL, tid);                            \
-            lqt[p].store(base__ + (2 * X::NP + p) * PANEL, tid);                       \
-            ldt[p].store(base__ + (3 * X::NP + p) * PANEL, tid);                       \
-        }                                                                              \
-        if (tid < 64) {                                                                \
-            const bool none__ = st_l == 0.f;                                           \
-            sstat[ST][0][tid] = none__ ? 0.f : st_m * LOG2E;                           \
-            sstat[ST][1][tid] = none__ ? 0.f : 1.0f / st_l;                            \
-            if constexpr (!OWN_DELTA) sstat[ST][2][tid] = st_d;                        \
-        }                                                                              \
-        if constexpr (OWN_DELTA)                                                       \
-            _Pragma("unroll") for (int i = 0; i < 2; ++i) {                            \
-                float part__ = 0.f;                                                    \
-                _Pragma("unroll") for (int p = 0; p < X::NP; ++p)                      \
-                    part__ += piece_dot(__builtin_bit_cast(typename X::F, ld[p].r[i]), __builtin_bit_cast(typename X::F, lo[p].r[i])); \
-                store_delta(sstat[ST][2], i, part__, tid);                             \
-            }                                                                          \
-    }
 
     f32x16 dk[2], dv[2];
 #pragma unroll
@@ -806,22 +536,14 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
             }                                                                          \
         lds_barrier();                                                                 \
     }
-    if constexpr (ASYNC) {
-        cq.init(Qb, a.q_rs, tid);
-        cd.init(dOb, a.do_rs, tid);
-        if constexpr (OWN_DELTA) co.init(Ob, a.o_rs, tid);
-        KV_COPY(qt0, 0)
-        frags_landed(kf);
-        frags_landed(vf);
-        if (qt0 + 1 < nqt) KV_COPY(qt0 + 1, 1)
-        KV_LAND(0, 0, qt0 + 1 < nqt)
-    } else {
-        if (qt0 < nqt) {
-            KV_FETCH(qt0)
-            KV_STASH(0)
-        }
-        __syncthreads();
-    }
+    cq.init(Qb, a.q_rs, tid);
+    cd.init(dOb, a.do_rs, tid);
+    if constexpr (OWN_DELTA) co.init(Ob, a.o_rs, tid);
+    KV_COPY(qt0, 0)
+    frags_landed(kf);
+    frags_landed(vf);
+    if (qt0 + 1 < nqt) KV_COPY(qt0 + 1, 1)
+    KV_LAND(0, 0, qt0 + 1 < nqt)
 
     const float sc = a.scale * LOG2E;
     // keep-bit line of this batch-head and the wave's first key as scalars
@@ -840,9 +562,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
     int slot = 0;   // this tile's place in LDS
     for (int qt = qt0; qt < nqt; ++qt) {
         const int st = (qt - qt0) & 1;
-        if constexpr (ASYNC) {
-            if (qt + 2 < nqt) KV_COPY(qt + 2, next_slot(next_slot(slot)))
-        } else KV_FETCH(qt + 1 < nqt ? qt + 1 : qt)
+        if (qt + 2 < nqt) KV_COPY(qt + 2, next_slot(next_slot(slot)))
         const KeepWords kw = kw_next;   // requested one step ago
         if constexpr (TRAIN) kw_next = load_keep_words(kline, kw0u + (qt + 1) * 64);
         const TileClasses tc = tc_next;
@@ -858,21 +578,20 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
                 if (q0 + j * 32 + 31 < kw0) continue;   // every query of this half precedes the wave's keys
                 const uint32_t cls = j == 0 ? tc.c0 : tc.c1;
                 if (HAS_MASK && cls == TILE_HIDDEN) continue;
-                RowFrags<T, 1> qa, da;
+                RowFrags<1> qa, da;
                 qa.read(base, j, lr, lg);
-                da.read(base + X::NP * PANEL, j, lr, lg);
-                if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
+                da.read(base + PANEL, j, lr, lg);
+                __builtin_amdgcn_sched_barrier(0);
                 f32x16 s1[1], dp1[1];
 #pragma unroll
                 for (int e = 0; e < 16; ++e) s1[0][e] = dp1[0][e] = 0.f;
-                qa.mma(s1, base, kf, j, lr, lg);                                  // S  [query][key]
-                da.mma(dp1, base + X::NP * PANEL, vf, j, lr, lg);                 // dP [query][key]
+                qa.mma(s1, kf);      // S  [query][key]
+                da.mma(dp1, vf);     // dP [query][key]
                 f32x16 &s = s1[0], &dp = dp1[0];
-                const char *qt_panel = base + (ASYNC ? 0 : 2 * X::NP * PANEL), *dot_panel = base + (ASYNC ? 1 : 3 * X::NP) * PANEL;
-                TpFrags<T> dot, qtr;
-                dot.read(dot_panel, j, lr, lg);
-                qtr.read(qt_panel, j, lr, lg);
-                if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
+                TpFrags dot, qtr;
+                dot.read(base + PANEL, j, lr, lg);
+                qtr.read(base, j, lr, lg);
+                __builtin_amdgcn_sched_barrier(0);
 
                 const bool diag = q0 + j * 32 < kw0 + 31;
                 if (diag) apply_causal<false>(s, key - q0 - j * 32 - lg * 4);
@@ -891,14 +610,11 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
                 for (int g4 = 0; g4 < 4; ++g4) {
                     const int qi = j * 32 + g4 * 8 + lg * 4;  // first of 4 consecutive queries (tile-relative)
                     const f32x4 m4 = *reinterpret_cast<const f32x4*>(&sstat[st][0][qi]);
-                    f32x4 l4 = {1.f, 1.f, 1.f, 1.f};
-                    if constexpr (!FOLD_L) l4 = *reinterpret_cast<const f32x4*>(&sstat[st][1][qi]);
                     const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sstat[st][2][qi]);
 #pragma unroll
                     for (int b = 0; b < 4; ++b) {
                         const int i = g4 * 4 + b;
-                        float p = fast_exp2(fmaf(s[i], sc, -m4[b]));
-                        if constexpr (!FOLD_L) p *= l4[b];
+                        const float p = fast_exp2(fmaf(s[i], sc, -m4[b]));
                         if constexpr (TRAIN) {
                             // dS = P (keep ? dP : 0) - P delta = (keep ? P : 0) dP - P delta: the dropped
                             // probability is needed anyway, so one select serves both products
@@ -914,39 +630,29 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
                 // Hidden elements (causal or masked) need no separate dS masking: their score is the
                 // fill value and the row's reference point is a real maximum (or 0 for a row without
                 // visible keys), so p, hence dS, is exactly 0 there.
-                dot.mma(dv, dot_panel, pd, j, lr, lg);   // dV^T += dO^T P
-                qtr.mma(dk, qt_panel, ds, j, lr, lg);    // dK^T += Q^T dS
+                dot.mma(dv, pd);   // dV^T += dO^T P
+                qtr.mma(dk, ds);    // dK^T += Q^T dS
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (ASYNC) {
-            slot = next_slot(slot);
-            if (qt + 1 < nqt) KV_LAND(slot, st ^ 1, qt + 2 < nqt)
-        } else {
-            slot ^= 1;
-            KV_STASH(st ^ 1)
-            __syncthreads();
-        }
+        slot = next_slot(slot);
+        if (qt + 1 < nqt) KV_LAND(slot, st ^ 1, qt + 2 < nqt)
     }
 #undef KV_COPY
 #undef KV_LAND
-#undef KV_FETCH
-#undef KV_STASH
 
     if (key < a.T) {
-        store_rows<T>((T*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)key * a.out0_rs, dk, a.scale, lg);
-        store_rows<T>((T*)a.out1 + bidx * a.out1_bs + hidx * a.out1_hs + (int64_t)key * a.out1_rs, dv, 1.0f, lg);
+        store_rows<bf16>((bf16*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)key * a.out0_rs, dk, a.scale, lg);
+        store_rows<bf16>((bf16*)a.out1 + bidx * a.out1_bs + hidx * a.out1_hs + (int64_t)key * a.out1_rs, dv, 1.0f, lg);
     }
 }
 
 // ---- backward: dQ -----------------------------------------------------------------------
 // Same geometry as the forward (lane = query, key tiles of 64).
-template <typename T> constexpr int dq_lds() { return sizeof(T) == 2 ? RING * 2 * PANEL : 2 * 3 * AT<T>::NP * PANEL; }
-template <typename T, bool HAS_MASK, bool TRAIN, bool STORE_DELTA>
+constexpr int DQ_LDS = RING * 2 * PANEL;
+template <bool HAS_MASK, bool TRAIN, bool STORE_DELTA>
 __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, const int query_tile, char* smem) {
-    typedef AT<T> X;
-    constexpr bool ASYNC = sizeof(T) == 2;
-    constexpr int STAGE = (ASYNC ? 2 : 3 * X::NP) * PANEL;  // K, V (4-byte storage: and K^T)
+    constexpr int STAGE = 2 * PANEL;          // K, V
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 31, lg = lane >> 5;
@@ -956,55 +662,36 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
     const int query = qw0 + lr;
     const int qrow = query < a.T ? query : a.T - 1;
 
-    const T* Qb = (const T*)a.q + bidx * a.q_bs + hidx * a.q_hs;
-    const T* Kb = (const T*)a.k + bidx * a.k_bs + hidx * a.k_hs;
-    const T* Vb = (const T*)a.v + bidx * a.v_bs + hidx * a.v_hs;
-    const T* dOb = (const T*)a.d_o + bidx * a.do_bs + hidx * a.do_hs;
+    const bf16* Qb = (const bf16*)a.q + bidx * a.q_bs + hidx * a.q_hs;
+    const bf16* Kb = (const bf16*)a.k + bidx * a.k_bs + hidx * a.k_hs;
+    const bf16* Vb = (const bf16*)a.v + bidx * a.v_bs + hidx * a.v_hs;
+    const bf16* dOb = (const bf16*)a.d_o + bidx * a.do_bs + hidx * a.do_hs;
 
-    typename X::F qf[X::NC], dof[X::NC];
-    load_row_frags<T>(qf, Qb + (int64_t)qrow * a.q_rs, lg);
-    load_row_frags<T>(dof, dOb + (int64_t)qrow * a.do_rs, lg);
+    RowPieces qf, dof;
+    load_row_frags(qf, Qb + (int64_t)qrow * a.q_rs, lg);
+    load_row_frags(dof, dOb + (int64_t)qrow * a.do_rs, lg);
     const int64_t si = (int64_t)bh * a.T + qrow;
-    // as in the dK/dV pass: 1/l folded into the exponent for 2-byte storage; a row without a
-    // visible key (saved l = 0) takes m = 0 and 1/l = 0, which makes its p exactly 0
-    constexpr bool FOLD_L = sizeof(T) == 2;
+    // as in the dK/dV pass: 1/l folded into the exponent, and a row without a visible key (saved l = 0) takes m = 0
     const float lsum = a.ls[si];
     const bool none = lsum == 0.f;
-    const float linv = none ? 0.f : 1.0f / lsum;
     // delta = rowsum(dO * O) of the lane's query: each lane of the pair (lr, lg) holds one half
     // of the dO row already.
     float delta;
     {
-        typename X::F of[X::NC];
-        load_row_frags<T>(of, (const T*)a.o + bidx * a.o_bs + hidx * a.o_hs + (int64_t)qrow * a.o_rs, lg);
-        constexpr int FE = (int)(sizeof(typename X::F) / sizeof(T));
+        RowPieces of;
+        load_row_frags(of, (const bf16*)a.o + bidx * a.o_bs + hidx * a.o_hs + (int64_t)qrow * a.o_rs, lg);
         float part = 0.f;
 #pragma unroll
-        for (int c = 0; c < X::NC; ++c)
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
-            for (int e = 0; e < FE; ++e) part += (float)dof[c][e] * (float)of[c][e];
+            for (int e = 0; e < 8; ++e) part += (float)dof[c][e] * (float)of[c][e];
         delta = part + xor32(part);
         if (STORE_DELTA && lg == 0 && query < a.T) a.delta[si] = delta;
     }
-    const float m2 = none ? 0.f : (FOLD_L ? fmaf(a.ms[si], LOG2E, __builtin_amdgcn_logf(lsum)) : a.ms[si] * LOG2E);
+    const float m2 = none ? 0.f : fmaf(a.ms[si], LOG2E, __builtin_amdgcn_logf(lsum));
 
     int nkt = (q0 + 128) / 64;
     if (nkt > a.T / 64) nkt = a.T / 64;
-
-    TileLoader<T, KMAJOR, 64, ATT_THREADS> lk[X::NP], lv[X::NP];
-    TileLoader<T, MNMAJOR, 64, ATT_THREADS> lkt[X::NP];
-#define DQ_FETCH(KT)                                                                   \
-    _Pragma("unroll") for (int p = 0; p < X::NP; ++p) {                                \
-        lk[p].load_fast(Kb, a.k_rs, 1, (KT) * 64, p * X::EPP, tid);                    \
-        lv[p].load_fast(Vb, a.v_rs, 1, (KT) * 64, p * X::EPP, tid);                    \
-        lkt[p].load_fast(Kb, 1, a.k_rs, 0, (KT) * 64 + p * X::EPP, tid);               \
-    }
-#define DQ_STASH(ST)                                                                   \
-    _Pragma("unroll") for (int p = 0; p < X::NP; ++p) {                                \
-        lk[p].store(smem + (ST) * STAGE + p * PANEL, tid);                             \
-        lv[p].store(smem + (ST) * STAGE + (X::NP + p) * PANEL, tid);                   \
-        lkt[p].store(smem + (ST) * STAGE + (2 * X::NP + p) * PANEL, tid);              \
-    }
 
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const uint32_t lds0 = lds_addr(smem);
@@ -1014,20 +701,14 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
         ck.issue(KT, lds0 + (SLOT) * STAGE, wave_u);                                   \
         cv.issue(KT, lds0 + (SLOT) * STAGE + PANEL, wave_u);                           \
     }
-    if constexpr (ASYNC) {
-        ck.init(Kb, a.k_rs, tid);
-        cv.init(Vb, a.v_rs, tid);
-        DQ_COPY(0, 0)
-        frags_landed(qf);
-        frags_landed(dof);
-        if (nkt > 1) DQ_COPY(1, 1)
-        copies_landed<4>(nkt > 1);
-        lds_barrier();
-    } else {
-        DQ_FETCH(0)
-        DQ_STASH(0)
-        __syncthreads();
-    }
+    ck.init(Kb, a.k_rs, tid);
+    cv.init(Vb, a.v_rs, tid);
+    DQ_COPY(0, 0)
+    frags_landed(qf);
+    frags_landed(dof);
+    if (nkt > 1) DQ_COPY(1, 1)
+    copies_landed<4>(nkt > 1);
+    lds_barrier();
 
     const float sc = a.scale * LOG2E;
     f32x16 dq[2];
@@ -1049,9 +730,7 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
     }
     int st = 0;   // this tile's place in LDS
     for (int kt = 0; kt < nkt; ++kt) {
-        if constexpr (ASYNC) {
-            if (kt + 2 < nkt) DQ_COPY(kt + 2, next_slot(next_slot(st)))
-        } else DQ_FETCH(kt + 1 < nkt ? kt + 1 : kt)
+        if (kt + 2 < nkt) DQ_COPY(kt + 2, next_slot(next_slot(st)))
         const KeepWords kw = kw_next;   // requested one step ago
         if constexpr (TRAIN) kw_next = load_keep_words(kline, qw0u + (kt + 1) * 64);
         const TileClasses tc = tc_next;
@@ -1068,20 +747,19 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
                 if (kh0 > qw0 + 31) continue;
                 const uint32_t cls = j == 0 ? tc.c0 : tc.c1;
                 if (HAS_MASK && cls == TILE_HIDDEN) continue;
-                RowFrags<T, 1> ka, va;
+                RowFrags<1> ka, va;
                 ka.read(base, j, lr, lg);
-                va.read(base + X::NP * PANEL, j, lr, lg);
-                if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
+                va.read(base + PANEL, j, lr, lg);
+                __builtin_amdgcn_sched_barrier(0);
                 f32x16 s1[1], dp1[1];
 #pragma unroll
                 for (int e = 0; e < 16; ++e) s1[0][e] = dp1[0][e] = 0.f;
-                ka.mma(s1, base, qf, j, lr, lg);                                   // S^T  [key][query]
-                va.mma(dp1, base + X::NP * PANEL, dof, j, lr, lg);                 // dP^T [key][query]
+                ka.mma(s1, qf);      // S^T  [key][query]
+                va.mma(dp1, dof);    // dP^T [key][query]
                 f32x16 &s = s1[0], &dp = dp1[0];
-                const char* kt_panel = base + (ASYNC ? 0 : 2 * X::NP * PANEL);
-                TpFrags<T> ktr;
-                ktr.read(kt_panel, j, lr, lg);
-                if constexpr (ASYNC) __builtin_amdgcn_sched_barrier(0);
+                TpFrags ktr;
+                ktr.read(base, j, lr, lg);
+                __builtin_amdgcn_sched_barrier(0);
 
                 const bool masked = kh0 + 31 > qw0;
                 if (masked) apply_causal<true>(s, query - kh0 - lg * 4);
@@ -1097,70 +775,61 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
                 float ds[16];
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    float p = fast_exp2(fmaf(s[i], sc, -m2));
-                    if constexpr (!FOLD_L) p *= linv;
+                    const float p = fast_exp2(fmaf(s[i], sc, -m2));
                     if constexpr (TRAIN)
                         ds[i] = p * (keep_select(dp[i], keep_lane_mask_at(kw, j * 32 + (i >> 2) * 8 + (i & 3))) - delta);
                     else
                         ds[i] = p * fmaf(dp[i], 0.9f, -delta);
                 }
                 // as in the dK/dV pass: p, hence dS, is exactly 0 on hidden elements
-                ktr.mma(dq, kt_panel, ds, j, lr, lg);   // dQ^T += K^T dS^T
+                ktr.mma(dq, ds);   // dQ^T += K^T dS^T
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (ASYNC) {
-            copies_landed<4>(kt + 2 < nkt);
-            lds_barrier();
-            st = next_slot(st);
-        } else {
-            st ^= 1;
-            DQ_STASH(st)
-            __syncthreads();
-        }
+        copies_landed<4>(kt + 2 < nkt);
+        lds_barrier();
+        st = next_slot(st);
     }
 #undef DQ_COPY
-#undef DQ_FETCH
-#undef DQ_STASH
 
     if (query < a.T)
-        store_rows<T>((T*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs, dq, a.scale, lg);
+        store_rows<bf16>((bf16*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs, dq, a.scale, lg);
 }
 
 // The backward as two launches, grid (B*H, ceil(T/128)) each: dQ, which stores delta, then dK/dV.  The tiles with the
 // longest way go first in every grid: the last query tiles, the first key tiles.
-// (2-byte storage without an explicit mask fits three wavefronts per SIMD; the bound keeps it there)
-template <typename T, bool HAS_MASK, bool TRAIN>
-__global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 3 : 1) void attn_bwd_dq_kernel(const AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) char smem[dq_lds<T>()];
+// (without an explicit mask it fits three wavefronts per SIMD; the bound keeps it there)
+template <bool HAS_MASK, bool TRAIN>
+__global__ __launch_bounds__(ATT_THREADS, 3) void attn_bwd_dq_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) char smem[DQ_LDS];
     const Place pl = place();
-    attn_bwd_dq<T, HAS_MASK, TRAIN, true>(a, pl.bh, gridDim.y - 1 - pl.tile, smem);
+    attn_bwd_dq<HAS_MASK, TRAIN, true>(a, pl.bh, gridDim.y - 1 - pl.tile, smem);
 }
-template <typename T, bool HAS_MASK, bool TRAIN>
-__global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_dkdv_kernel(const AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<T, false>()];
+template <bool HAS_MASK, bool TRAIN>
+__global__ __launch_bounds__(ATT_THREADS, 2) void attn_bwd_dkdv_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<false>()];
     __shared__ __attribute__((aligned(16))) StatTile sstat[2];
     const Place pl = place();
-    attn_bwd_dkdv<T, HAS_MASK, TRAIN, false>(a, pl.bh, pl.tile, smem, sstat);
+    attn_bwd_dkdv<HAS_MASK, TRAIN, false>(a, pl.bh, pl.tile, smem, sstat);
 }
 // Both in one launch, grid (B*H, 2 ceil(T/128)).
-template <typename T, bool HAS_MASK, bool TRAIN>
-__global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 2 : 1) void attn_bwd_kernel(const AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<T, true>()];
+template <bool HAS_MASK, bool TRAIN>
+__global__ __launch_bounds__(ATT_THREADS, 2) void attn_bwd_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<true>()];
     __shared__ __attribute__((aligned(16))) StatTile sstat[2];
     const int tile = blockIdx.y >> 1;
-    if (blockIdx.y & 1) attn_bwd_dq<T, HAS_MASK, TRAIN, false>(a, blockIdx.x, (gridDim.y >> 1) - 1 - tile, smem);
-    else attn_bwd_dkdv<T, HAS_MASK, TRAIN, true>(a, blockIdx.x, tile, smem, sstat);
+    if (blockIdx.y & 1) attn_bwd_dq<HAS_MASK, TRAIN, false>(a, blockIdx.x, (gridDim.y >> 1) - 1 - tile, smem);
+    else attn_bwd_dkdv<HAS_MASK, TRAIN, true>(a, blockIdx.x, tile, smem, sstat);
 }
 
 // Launch one of the (mask, train) specialisations.
-#define ATTN_LAUNCH(KERNEL, T_, grid, st, args)                                                        \
+#define ATTN_LAUNCH(KERNEL, grid, st, args)                                                        \
     do {                                                                                               \
         const bool hm__ = (args).mask != nullptr, tr__ = (args).train != 0;                            \
-        if (hm__ && tr__) hipLaunchKernelGGL((KERNEL<T_, true, true>), grid, dim3(ATT_THREADS), 0, st, args);        \
-        else if (hm__) hipLaunchKernelGGL((KERNEL<T_, true, false>), grid, dim3(ATT_THREADS), 0, st, args);          \
-        else if (tr__) hipLaunchKernelGGL((KERNEL<T_, false, true>), grid, dim3(ATT_THREADS), 0, st, args);          \
-        else hipLaunchKernelGGL((KERNEL<T_, false, false>), grid, dim3(ATT_THREADS), 0, st, args);                   \
+        if (hm__ && tr__) hipLaunchKernelGGL((KERNEL<true, true>), grid, dim3(ATT_THREADS), 0, st, args);        \
+        else if (hm__) hipLaunchKernelGGL((KERNEL<true, false>), grid, dim3(ATT_THREADS), 0, st, args);          \
+        else if (tr__) hipLaunchKernelGGL((KERNEL<false, true>), grid, dim3(ATT_THREADS), 0, st, args);          \
+        else hipLaunchKernelGGL((KERNEL<false, false>), grid, dim3(ATT_THREADS), 0, st, args);                   \
     } while (0)
 
 // ---- host side ----------------------------------------------------------------------------
@@ -1197,28 +866,25 @@ int launch_keepbits(uint32_t* bits, int64_t count, const int64_t* seeds, int64_t
 
 void launch_fwd(const AttnArgs& a, int dtype, hipStream_t st) {
     const dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.T + 127) / 128));
-    if (dtype == PTJ_F32) ATTN_LAUNCH(attn_fwd_kernel, float, grid, st, a);
-    else ATTN_LAUNCH(attn_fwd_kernel, bf16, grid, st, a);
+    if (dtype == PTJ_F32) ptj_attn_detail::launch_fwd_f32(a, st);
+    else ATTN_LAUNCH(attn_fwd_kernel, grid, st, a);
 }
 
 // One launch while the two passes' workgroups make no more than four rounds of one per CU, two launches beyond.  The passes
 // then fill each other's idle CUs and a launch is saved, against an O tile read again per query tile of dK/dV (delta) and
 // the dQ tiles at the dK/dV kernel's occupancy.  From the first kernel's start to the last one's end, two launches / one, bf16
 // and 12 heads (workgroups): 2 x 256 (96) 29.6 / 14.1 us, 7 x 448 (672) 37.9 / 26.8, 8 x 512 (768) 40.5 / 31.1, 4 x 1024 (768)
-// 61.8 / 47.6, 8 x 1024 (1536) 79.1 / 77.1, 16 x 1024 (3072) 138.9 / 148.1; fp32 8 x 512 (768) 223 / 215 with the forward.
+// 61.8 / 47.6, 8 x 1024 (1536) 79.1 / 77.1, 16 x 1024 (3072) 138.9 / 148.1.
 void launch_bwd(const AttnArgs& a, int dtype, hipStream_t st) {
+    if (dtype == PTJ_F32) return ptj_attn_detail::launch_bwd_f32(a, st);
     const int64_t nt = (a.T + 127) / 128;
     const bool one = (int64_t)a.B * a.H * nt * 2 <= (int64_t)4 * ptj_num_cus();
     const dim3 grid((unsigned)(a.B * a.H), (unsigned)nt), grid2((unsigned)(a.B * a.H), (unsigned)(2 * nt));
     if (one) {
-        if (dtype == PTJ_F32) ATTN_LAUNCH(attn_bwd_kernel, float, grid2, st, a);
-        else ATTN_LAUNCH(attn_bwd_kernel, bf16, grid2, st, a);
-    } else if (dtype == PTJ_F32) {
-        ATTN_LAUNCH(attn_bwd_dq_kernel, float, grid, st, a);
-        ATTN_LAUNCH(attn_bwd_dkdv_kernel, float, grid, st, a);
+        ATTN_LAUNCH(attn_bwd_kernel, grid2, st, a);
     } else {
-        ATTN_LAUNCH(attn_bwd_dq_kernel, bf16, grid, st, a);
-        ATTN_LAUNCH(attn_bwd_dkdv_kernel, bf16, grid, st, a);
+        ATTN_LAUNCH(attn_bwd_dq_kernel, grid, st, a);
+        ATTN_LAUNCH(attn_bwd_dkdv_kernel, grid, st, a);
     }
 }
 

@@ -1,0 +1,631 @@
+// Causal flash attention of 4-byte storage: the algorithm, layouts, masks and statistics of attn.hip, multiplied on the bf16
+// matrix pipe.
+//
+// Every factor is the exact sum of three bf16 values (Split8), and six products of the parts (those above 2^-26 of the whole)
+// stand for one: 192 clocks per 32x32x16 where the fp32 instructions take 512.  Q, K, V and dO are split once per workgroup on
+// their way into registers or LDS, P and dS where they are formed.  The parts lie in LDS as bf16 panels, which transposing reads
+// serve in both directions, so no transposed copies exist.
+// What bounds it: the matrix pipe at the clock that the part holds under such load.  Batch 8 x 1024 x 12 heads multiplies at
+// 980 (forward) and 1090 TFLOP/s (backward) of bf16 products, where this repository's fp32 GEMMs reach 1000 to 1290.
+// Eight wavefronts share a 64-row tile: four blocks of 32 rows x the two halves of the tile, so that two wavefronts per SIMD
+// overlap matrix and vector work, every conversion serves 128 rows, and the way through a row's keys is half as long; the
+// halves' results are added at the end.  The wavefronts of the second half convert the next tile before their products, those of
+// the first half behind them (8 x 1024: backward 283 -> 277 us, forward 94 -> 89).
+// fp32 instructions / this file, us, 12 heads: 8 x 512 forward 58 / 33, backward 150 / 93; 8 x 1024 140 / 89 and 477 / 277;
+// 2 x 256 24 / 15 and 46 / 26.  Error against fp64 (2-norm, 8 x 512): O 2.8e-7 / 1.6e-7, dQ 3.6e-7 / 2.8e-7, dK 5.7e-7 / 3.7e-7,
+// dV 5.6e-7 / 3.5e-7.
+#include "attn_common.h"
+
+namespace {
+
+constexpr int THREADS = 512;
+constexpr int TILE = 3 * PANEL;           // 64 x 64 elements as three panels
+
+// Eight fp32 values as three times eight bf16 values whose sum they are: exact from 2^-109 on, below that to 2^-134.
+struct Split8 { bf16x8 p[3]; };
+__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    u32x4 w[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float lo = x[2 * e], hi = x[2 * e + 1];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const f32x2_t f = {lo, hi};
+            w[i][e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+            lo -= __uint_as_float(w[i][e] << 16);
+            hi -= __uint_as_float(w[i][e] & 0xffff0000u);
+        }
+    }
+    Split8 s;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) s.p[i] = __builtin_bit_cast(bf16x8, w[i]);
+    return s;
+}
+// The same for values of the caller, which may round up to infinity or be infinite: then they are their own last part, which
+// meets nothing but the other factor's first one (a lower part may be 0 or of the other sign).
+__device__ __forceinline__ Split8 split8_any(const float (&x)[8]) {
+    float most = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(x[e]));
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(most >= 0x1p120f) == 0, 1)) return split8(x);
+    u32x4 first, last;
+    float rest[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const uint32_t top = __float_as_uint(x[e]) & 0xffff0000u;
+        const bool inf = fabsf(x[e]) == __builtin_inff();
+        rest[e] = inf ? 0.f : x[e] - __uint_as_float(top);
+        const uint32_t f = inf ? 0u : top, l = inf ? top : 0u;
+        first[e >> 1] = e & 1 ? first[e >> 1] | f : f >> 16;
+        last[e >> 1] = e & 1 ? last[e >> 1] | l : l >> 16;
+    }
+    Split8 s = split8(rest);
+    s.p[2] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, s.p[1]) | last);
+    s.p[1] = s.p[0];
+    s.p[0] = __builtin_bit_cast(bf16x8, first);
+    return s;
+}
+__device__ __forceinline__ Split8 split_row_piece(const float* __restrict__ p) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+    const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    return split8_any(x);
+}
+// The MFMA operand pieces of one 64-element row (lane half lg) in registers
+__device__ __forceinline__ void load_row_splits(Split8 (&f)[4], const float* __restrict__ row, int lg) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) f[c] = split_row_piece(row + c * 16 + lg * 8);
+}
+
+__device__ __forceinline__ void mma(f32x16& acc, const bf16x8& a, const bf16x8& b) {
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+}
+// MFMA operand pieces of rows 32 j .. of a tile, contraction chunk c
+__device__ __forceinline__ Split8 row_split(const char* __restrict__ tile, int j, int c, int lr, int lg) {
+    const char* p = tile + (j * 32 + lr) * BKB + (((c * 2 + lg) ^ row_swizzle(lr)) << 4);
+    Split8 a;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) a.p[i] = *reinterpret_cast<const bf16x8*>(p + i * PANEL);
+    return a;
+}
+// Two chains of products side by side (one after the other they wait for their own results): the lower parts first
+__device__ __forceinline__ void mma_two(f32x16& s0, const Split8& a0, const Split8& b0, f32x16& s1, const Split8& a1, const Split8& b1) {
+    constexpr int A[6] = {2, 0, 1, 1, 0, 0}, B[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+        mma(s0, a0.p[A[i]], b0.p[B[i]]);
+        mma(s1, a1.p[A[i]], b1.p[B[i]]);
+    }
+}
+
+// o[t] += (columns 32 t .. of the tile, transposed) x p: contraction over the tile's rows 32 j + 16 h .. + 15, of which the lane
+// holds p[e] for row 32 j + 16 h + 8 (e / 4) + 4 lg + e % 4
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void columns_x_regs(f32x16 (&o)[2], const char* __restrict__ tile, const Split8& p, int j, int h, int lr, int lg) {
+    const int x = 4 * lg + ((lr & 15) >> 2);
+    Split8 a[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int piece = t * 4 + 2 * (lr >> 4) + ((lr & 3) >> 1);
+        const char* pp = tile + (j * 32 + h * 16 + x) * BKB + 8 * (lr & 1);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(pp + i * PANEL + ((piece ^ row_swizzle(x)) << 4)));
+            const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(pp + i * PANEL + 8 * BKB + ((piece ^ row_swizzle(x + 8)) << 4)));
+            a[t].p[i] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    }
+    mma_two(o[0], a[0], p, o[1], a[1], p);
+}
+
+// A 64 x 64 tile on its way from memory to LDS: every thread has eight elements of a row
+struct TileCopy {
+    const float* src;        // the thread's piece of tile 0
+    int64_t step;            // elements from a tile to the next
+    f32x4 r[2];
+    __device__ __forceinline__ void init(const float* __restrict__ p, int64_t row_stride, int tid) {
+        src = p + (int64_t)(tid >> 3) * row_stride + (tid & 7) * 8;
+        step = 64 * row_stride;
+    }
+    __device__ __forceinline__ void fetch(int tile) {
+        const float* s = src + tile * step;
+        r[0] = *reinterpret_cast<const f32x4*>(s);
+        r[1] = *reinterpret_cast<const f32x4*>(s + 4);
+    }
+    __device__ __forceinline__ void store(char* __restrict__ tile, int tid) const {
+        const float x[8] = {r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1], r[1][2], r[1][3]};
+        const Split8 s = split8_any(x);
+        char* to = tile + (tid >> 3) * BKB + (((tid & 7) ^ row_swizzle(tid >> 3)) << 4);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(to + i * PANEL) = s.p[i];
+    }
+};
+
+// Keep bits of 32 x 32 elements (keep_lane_mask_at with offsets below 32 looks at two words)
+__device__ __forceinline__ KeepWords load_keep_half(const uint32_t* __restrict__ line, int base) {
+    const uniform_words p = as_uniform(line + (base >> 5));
+    return {p[0], p[1], 0u};
+}
+__device__ __forceinline__ uint64_t keep_mask(const KeepWords& w, int i) { return keep_lane_mask_at(w, (i >> 2) * 8 + (i & 3)); }
+
+// The mask words of a mixed tile: hidden elements become NEG_RAW
+__device__ __forceinline__ void apply_mask(f32x16& s, const uint32_t* __restrict__ words) {
+    const uniform_words mw = as_uniform(words);
+    uint32_t w[32];
+#pragma unroll
+    for (int t = 0; t < 32; ++t) w[t] = mw[t];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = mask_select(s[i], NEG_RAW, mask_lanes(w, i));
+}
+
+// Accumulators of this wavefront's partner (the other half of the tiles), through LDS: `give` goes, what the partner gives comes.
+// Everything in `smem` has been read.
+template <int N>
+__device__ __forceinline__ void exchange(const float (&give)[N], float (&take)[N], char* __restrict__ smem, int wave, int lane) {
+    float* const f = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int i = 0; i < N; ++i) f[(wave * N + i) * 64 + lane] = give[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) take[i] = f[((wave ^ 4) * N + i) * 64 + lane];
+}
+// 32 columns of a row: element e of lane half lg is column 8 (e / 4) + 4 lg + e % 4
+__device__ __forceinline__ void store_half_row(float* __restrict__ row, const float (&x)[16], float f, int lg) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        const float v[4] = {x[4 * a] * f, x[4 * a + 1] * f, x[4 * a + 2] * f, x[4 * a + 3] * f};
+        store_vec<float, 4>(row + a * 8 + lg * 4, v);
+    }
+}
+
+// ---- forward -------------------------------------------------------------------------
+// grid (B*H, ceil(T/128)): wavefront (half, block) owns queries q0 + 32 block .. +31 against the keys of its half of each tile
+template <bool HAS_MASK, bool TRAIN>
+__global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) char smem[2][2 * TILE];      // K, V
+
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
+    const int bh = blockIdx.x, bidx = bh / a.H, hidx = bh % a.H;
+    const int q0 = (gridDim.y - 1 - blockIdx.y) * 128;
+    const int qw0 = q0 + (wave & 3) * 32;
+    const int query = qw0 + lr;
+    const int qrow = query < a.T ? query : a.T - 1;
+
+    TileCopy ck, cv;
+    ck.init((const float*)a.k + bidx * a.k_bs + hidx * a.k_hs, a.k_rs, tid);
+    cv.init((const float*)a.v + bidx * a.v_bs + hidx * a.v_hs, a.v_rs, tid);
+    ck.fetch(0);
+    cv.fetch(0);
+    Split8 qf[4];
+    load_row_splits(qf, (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs + (int64_t)qrow * a.q_rs, lg);
+    ck.store(smem[0], tid);
+    cv.store(smem[0] + TILE, tid);
+    __syncthreads();
+
+    int nkt = (q0 + 128) / 64;
+    if (nkt > a.T / 64) nkt = a.T / 64;
+    const float sc = a.scale * LOG2E;
+    float m_run = M_START, m_true = M_START, l_run = 0.f;
+    f32x16 o[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
+
+    // keep bits and tile class of a step are requested one step ahead
+    const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
+    const int lookup = lookup_row(qw0, a.T);
+    KeepWords kw_next;
+    if constexpr (TRAIN) kw_next = load_keep_half(kline, lookup + half * 32);
+    const uint32_t* __restrict__ crow = nullptr;
+    uint32_t cls_next = TILE_CAUSAL;
+    if constexpr (HAS_MASK) {
+        const int G = a.T >> 5;
+        crow = a.mask + 2 * (int64_t)a.B * G * a.T + ((int64_t)bidx * G + (lookup >> 5)) * G + half;
+        cls_next = as_uniform(crow)[0];
+    }
+    auto fetch = [&](int tile) __attribute__((always_inline)) {
+        ck.fetch(tile);
+        cv.fetch(tile);
+    };
+    auto store = [&](int tile) __attribute__((always_inline)) {
+        ck.store(smem[tile & 1], tid);
+        cv.store(smem[tile & 1] + TILE, tid);
+    };
+    if (half && nkt > 1) fetch(1);
+    for (int kt = 0; kt < nkt; ++kt) {
+        const bool more = kt + 1 < nkt;
+        const int ahead = more ? kt + 1 : kt;
+        if (half == 0) {
+            if (more) fetch(kt + 1);
+        } else {
+            if (more) store(kt + 1);
+            if (kt + 2 < nkt) fetch(kt + 2);
+        }
+        const KeepWords kw = kw_next;
+        if constexpr (TRAIN) kw_next = load_keep_half(kline, lookup + half * 32 + ahead * 64);
+        const uint32_t cls = cls_next;
+        if constexpr (HAS_MASK) cls_next = as_uniform(crow)[2 * ahead];
+        const int key0 = kt * 64 + half * 32;
+        if (key0 <= qw0 + 31 && (!HAS_MASK || cls != TILE_HIDDEN)) {
+            const char* kp = smem[kt & 1];
+            f32x16 s, s2;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] = s2[e] = 0.f;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) mma_two(s, row_split(kp, half, c, lr, lg), qf[c], s2, row_split(kp, half, c + 2, lr, lg), qf[c + 2]);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] += s2[e];
+            if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4);
+            if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0);
+            float tmax = s[0];
+#pragma unroll
+            for (int i = 1; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
+            tmax = max_xor32(tmax) * sc;
+            m_true = fmaxf(m_true, tmax);
+            // the reference point follows the row maximum only when it has been outgrown by 2^RESCALE_SLACK, see attn.hip
+            if (__builtin_amdgcn_ballot_w64(tmax > m_run + RESCALE_SLACK) != 0) {
+                const float m_new = fmaxf(m_run, tmax), alpha = fast_exp2(m_run - m_new);
+                l_run *= alpha;
+                m_run = m_new;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
+            }
+            float lsum = 0.f;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float p[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    p[e] = fast_exp2(fmaf(s[8 * h + e], sc, -m_run));
+                    lsum += p[e];
+                    if constexpr (TRAIN) p[e] = keep_select(p[e], keep_mask(kw, 8 * h + e));
+                }
+                columns_x_regs(o, kp + TILE, split8(p), half, h, lr, lg);
+            }
+            l_run += sum_xor32(lsum);
+        }
+        if (half == 0 && more) store(kt + 1);
+        __syncthreads();
+    }
+
+    // Both halves of the keys together; each wavefront finishes the columns of its own half.
+    float give[19], take[19];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) give[e] = half ? o[0][e] : o[1][e];
+    give[16] = m_run;
+    give[17] = m_true;
+    give[18] = l_run;
+    exchange(give, take, &smem[0][0], wave, lane);
+    if (query < a.T) {
+        const float m_all = fmaxf(m_run, take[16]), mine = fast_exp2(m_run - m_all), theirs = fast_exp2(take[16] - m_all);
+        const float l = half ? fmaf(take[18], theirs, l_run * mine) : fmaf(l_run, mine, take[18] * theirs);
+        m_true = fmaxf(m_true, take[17]);
+        // l = 0: no key of the row is visible (a row with a visible key has l >= 1)
+        const bool empty = l == 0.f;
+        const float f = empty ? 0.f : (TRAIN ? 1.0f : 0.9f) / l;
+        float out[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) out[e] = (half ? o[1][e] : o[0][e]) * mine + take[e] * theirs;
+        store_half_row((float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs + half * 32, out, f, lg);
+        if (lg == 0 && half == 0) {
+            a.ms[(int64_t)bh * a.T + query] = empty ? NEG_NAT : m_true * LN2;
+            a.ls[(int64_t)bh * a.T + query] = empty ? 0.f : l * fast_exp2(m_all - m_true);
+        }
+    }
+}
+
+// ---- backward: dK, dV -------------------------------------------------------------------
+// One workgroup per (batch-head, 128 keys): wavefront (half, block) owns keys key0 + 32 block .. +31 (lane = key) against the
+// queries of its half of each tile.  delta = rowsum(dO * O) is formed on the rows' way into LDS.  The keys' rows of K wait in
+// registers, those of V in LDS: both in registers spill (8 x 512: 122 us instead of 93).
+typedef float StatTile[3][64];            // m2, 1/l, delta of a query tile
+template <bool HAS_MASK, bool TRAIN>
+__device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const int key_tile, char (*smem)[2 * TILE], char (*vrows)[TILE], StatTile* sstat) {
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
+    const int bidx = bh / a.H, hidx = bh % a.H;
+    const int kw0 = key_tile * 128 + (wave & 3) * 32;
+    const int key = kw0 + lr;
+    const int krow = key < a.T ? key : a.T - 1;
+    const int qt0 = key_tile * 2, nqt = a.T / 64;
+
+    TileCopy cq, cd, co;
+    cq.init((const float*)a.q + bidx * a.q_bs + hidx * a.q_hs, a.q_rs, tid);
+    cd.init((const float*)a.d_o + bidx * a.do_bs + hidx * a.do_hs, a.do_rs, tid);
+    co.init((const float*)a.o + bidx * a.o_bs + hidx * a.o_hs, a.o_rs, tid);
+    const int64_t stat0 = (int64_t)bh * a.T + (tid & 63);
+    float st_m = 0.f, st_l = 0.f;
+    auto fetch = [&](int qt) __attribute__((always_inline)) {
+        cq.fetch(qt);
+        cd.fetch(qt);
+        co.fetch(qt);
+        st_m = a.ms[stat0 + qt * 64];
+        st_l = a.ls[stat0 + qt * 64];
+    };
+    auto store = [&](int b) __attribute__((always_inline)) {
+        float part = 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part += cd.r[i][e] * co.r[i][e];
+        part += __shfl_xor(part, 1, 64);
+        part += __shfl_xor(part, 2, 64);
+        part += __shfl_xor(part, 4, 64);
+        if ((tid & 7) == 0) sstat[b][2][tid >> 3] = part;
+        if (tid < 64) {
+            // a row without a visible key (saved l = 0) takes m = 0 and 1/l = 0, which makes its p exactly 0
+            const bool none = st_l == 0.f;
+            sstat[b][0][tid] = none ? 0.f : st_m * LOG2E;
+            sstat[b][1][tid] = none ? 0.f : 1.0f / st_l;
+        }
+        cq.store(smem[b], tid);
+        cd.store(smem[b] + TILE, tid);
+    };
+    fetch(qt0);
+    {
+        // the workgroup's rows of V (the last tile's second half may lie past the end: repeated, not used)
+        TileCopy cv;
+        cv.init((const float*)a.v + bidx * a.v_bs + hidx * a.v_hs, a.v_rs, tid);
+        cv.fetch(key_tile * 2);
+        cv.store(vrows[0], tid);
+        cv.fetch(key_tile * 2 + 1 < nqt ? key_tile * 2 + 1 : nqt - 1);
+        cv.store(vrows[1], tid);
+    }
+    Split8 kf[4];
+    load_row_splits(kf, (const float*)a.k + bidx * a.k_bs + hidx * a.k_hs + (int64_t)krow * a.k_rs, lg);
+    store(0);
+    __syncthreads();
+
+    const float sc = a.scale * LOG2E;
+    f32x16 dk[2], dv[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dk[t][e] = dv[t][e] = 0.f;
+
+    const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
+    const int lookup = lookup_row(kw0, a.T);
+    KeepWords kw_next;
+    if constexpr (TRAIN) kw_next = load_keep_half(kline, lookup + qt0 * 64 + half * 32);
+    const uint32_t* __restrict__ crow = nullptr;
+    uint32_t cls_next = TILE_CAUSAL;
+    if constexpr (HAS_MASK) {
+        const int G = a.T >> 5;
+        crow = a.mask + 2 * (int64_t)a.B * G * a.T + (int64_t)a.B * G * G + ((int64_t)bidx * G + (lookup >> 5)) * G + half;
+        cls_next = as_uniform(crow)[2 * qt0];
+    }
+    if (half && qt0 + 1 < nqt) fetch(qt0 + 1);
+    for (int qt = qt0; qt < nqt; ++qt) {
+        const int b = (qt - qt0) & 1;
+        const bool more = qt + 1 < nqt;
+        const int ahead = more ? qt + 1 : qt;
+        const KeepWords kw = kw_next;
+        if constexpr (TRAIN) kw_next = load_keep_half(kline, lookup + half * 32 + ahead * 64);
+        const uint32_t cls = cls_next;
+        if constexpr (HAS_MASK) cls_next = as_uniform(crow)[2 * ahead];
+        const int q0 = qt * 64 + half * 32;
+        const bool live = q0 + 31 >= kw0 && (!HAS_MASK || cls != TILE_HIDDEN);
+        const char *qp = smem[b], *dp_ = smem[b] + TILE;
+        f32x16 s, dp;
+        if (half == 0) {
+            if (more) fetch(qt + 1);
+        } else {
+            if (more) store(b ^ 1);
+            if (qt + 2 < nqt) fetch(qt + 2);
+        }
+        if (live) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)       // S and dP [query][key]
+                mma_two(s, row_split(qp, half, c, lr, lg), kf[c], dp, row_split(dp_, half, c, lr, lg), row_split(vrows[(wave & 3) >> 1], wave & 1, c, lr, lg));
+        }
+        if (live) {
+            if (q0 < kw0 + 31) apply_causal<false>(s, key - q0 - lg * 4);
+            if (HAS_MASK && cls != TILE_CAUSAL)
+                apply_mask(s, a.mask + (int64_t)a.B * (a.T >> 5) * a.T + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + q0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float pd[8], ds[8];
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const int qi = half * 32 + (2 * h + g) * 8 + lg * 4;   // first of 4 consecutive queries (tile-relative)
+                    const f32x4 m4 = *reinterpret_cast<const f32x4*>(&sstat[b][0][qi]);
+                    const f32x4 l4 = *reinterpret_cast<const f32x4*>(&sstat[b][1][qi]);
+                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sstat[b][2][qi]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int i = 8 * h + 4 * g + e;
+                        const float p = fast_exp2(fmaf(s[i], sc, -m4[e])) * l4[e];
+                        if constexpr (TRAIN) {
+                            // dS = P (keep ? dP : 0) - P delta = (keep ? P : 0) dP - P delta
+                            pd[4 * g + e] = keep_select(p, keep_mask(kw, i));
+                            ds[4 * g + e] = fmaf(pd[4 * g + e], dp[i], -(p * d4[e]));
+                        } else {
+                            pd[4 * g + e] = 0.9f * p;
+                            ds[4 * g + e] = p * fmaf(dp[i], 0.9f, -d4[e]);
+                        }
+                    }
+                }
+                // p, hence dS, is exactly 0 on hidden elements, see attn.hip
+                columns_x_regs(dv, dp_, split8(pd), half, h, lr, lg);   // dV^T += dO^T P
+                columns_x_regs(dk, qp, split8(ds), half, h, lr, lg);    // dK^T += Q^T dS
+            }
+        }
+        if (half == 0 && more) store(b ^ 1);
+        __syncthreads();
+    }
+
+    // Both halves of the queries together: the wavefronts of the first half finish dK, those of the second dV.
+    float give[32], take[32];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) give[16 * t + e] = half ? dk[t][e] : dv[t][e];
+    exchange(give, take, &smem[0][0], wave, lane);
+    if (key < a.T) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) dk[t][e] = (half ? dv[t][e] : dk[t][e]) + take[16 * t + e];
+        float* const row = half ? (float*)a.out1 + bidx * a.out1_bs + hidx * a.out1_hs + (int64_t)key * a.out1_rs
+                                : (float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)key * a.out0_rs;
+        store_rows<float>(row, dk, half ? 1.0f : a.scale, lg);
+    }
+}
+
+// ---- backward: dQ -----------------------------------------------------------------------
+// Same geometry as the forward.
+template <bool HAS_MASK, bool TRAIN>
+__device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const int query_tile, char (*smem)[2 * TILE]) {
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
+    const int bidx = bh / a.H, hidx = bh % a.H;
+    const int q0 = query_tile * 128;
+    const int qw0 = q0 + (wave & 3) * 32;
+    const int query = qw0 + lr;
+    const int qrow = query < a.T ? query : a.T - 1;
+
+    TileCopy ck, cv;
+    ck.init((const float*)a.k + bidx * a.k_bs + hidx * a.k_hs, a.k_rs, tid);
+    cv.init((const float*)a.v + bidx * a.v_bs + hidx * a.v_hs, a.v_rs, tid);
+    ck.fetch(0);
+    cv.fetch(0);
+    const float* const do_row = (const float*)a.d_o + bidx * a.do_bs + hidx * a.do_hs + (int64_t)qrow * a.do_rs;
+    const float* const o_row = (const float*)a.o + bidx * a.o_bs + hidx * a.o_hs + (int64_t)qrow * a.o_rs;
+    // delta = rowsum(dO * O): each lane of the pair (lr, lg) has one half of the row
+    float delta = 0.f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const int at = (c >> 1) * 16 + lg * 8 + (c & 1) * 4;
+        const f32x4 x = *reinterpret_cast<const f32x4*>(do_row + at), y = *reinterpret_cast<const f32x4*>(o_row + at);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) delta += x[e] * y[e];
+    }
+    delta += xor32(delta);
+    const int64_t si = (int64_t)bh * a.T + qrow;
+    // as in dK/dV: a row without a visible key takes m = 0 and 1/l = 0
+    const float lsum = a.ls[si];
+    const bool none = lsum == 0.f;
+    const float linv = none ? 0.f : 1.0f / lsum, m2 = none ? 0.f : a.ms[si] * LOG2E;
+    Split8 qf[4], dof[4];
+    load_row_splits(qf, (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs + (int64_t)qrow * a.q_rs, lg);
+    load_row_splits(dof, do_row, lg);
+    ck.store(smem[0], tid);
+    cv.store(smem[0] + TILE, tid);
+    __syncthreads();
+
+    int nkt = (q0 + 128) / 64;
+    if (nkt > a.T / 64) nkt = a.T / 64;
+    const float sc = a.scale * LOG2E;
+    f32x16 dq[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dq[t][e] = 0.f;
+
+    const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
+    const int lookup = lookup_row(qw0, a.T);
+    KeepWords kw_next;
+    if constexpr (TRAIN) kw_next = load_keep_half(kline, lookup + half * 32);
+    const uint32_t* __restrict__ crow = nullptr;
+    uint32_t cls_next = TILE_CAUSAL;
+    if constexpr (HAS_MASK) {
+        const int G = a.T >> 5;
+        crow = a.mask + 2 * (int64_t)a.B * G * a.T + ((int64_t)bidx * G + (lookup >> 5)) * G + half;
+        cls_next = as_uniform(crow)[0];
+    }
+    auto fetch = [&](int tile) __attribute__((always_inline)) {
+        ck.fetch(tile);
+        cv.fetch(tile);
+    };
+    auto store = [&](int tile) __attribute__((always_inline)) {
+        ck.store(smem[tile & 1], tid);
+        cv.store(smem[tile & 1] + TILE, tid);
+    };
+    if (half && nkt > 1) fetch(1);
+    for (int kt = 0; kt < nkt; ++kt) {
+        const bool more = kt + 1 < nkt;
+        const int ahead = more ? kt + 1 : kt;
+        if (half == 0) {
+            if (more) fetch(kt + 1);
+        } else {
+            if (more) store(kt + 1);
+            if (kt + 2 < nkt) fetch(kt + 2);
+        }
+        const KeepWords kw = kw_next;
+        if constexpr (TRAIN) kw_next = load_keep_half(kline, lookup + half * 32 + ahead * 64);
+        const uint32_t cls = cls_next;
+        if constexpr (HAS_MASK) cls_next = as_uniform(crow)[2 * ahead];
+        const int key0 = kt * 64 + half * 32;
+        if (key0 <= qw0 + 31 && (!HAS_MASK || cls != TILE_HIDDEN)) {
+            const char* kp = smem[kt & 1];
+            f32x16 s, dp;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)       // S^T and dP^T [key][query]
+                mma_two(s, row_split(kp, half, c, lr, lg), qf[c], dp, row_split(kp + TILE, half, c, lr, lg), dof[c]);
+            if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4);
+            if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float ds[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int i = 8 * h + e;
+                    const float p = fast_exp2(fmaf(s[i], sc, -m2)) * linv;
+                    if constexpr (TRAIN) ds[e] = p * (keep_select(dp[i], keep_mask(kw, i)) - delta);
+                    else ds[e] = p * fmaf(dp[i], 0.9f, -delta);
+                }
+                columns_x_regs(dq, kp, split8(ds), half, h, lr, lg);   // dQ^T += K^T dS^T
+            }
+        }
+        if (half == 0 && more) store(kt + 1);
+        __syncthreads();
+    }
+
+    float give[16], take[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) give[e] = half ? dq[0][e] : dq[1][e];
+    exchange(give, take, &smem[0][0], wave, lane);
+    if (query < a.T) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) take[e] += half ? dq[1][e] : dq[0][e];
+        store_half_row((float*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs + half * 32, take, a.scale, lg);
+    }
+}
+
+// grid (B*H, 2 ceil(T/128)): both passes in one launch, the tiles with the longest way first
+template <bool HAS_MASK, bool TRAIN>
+__global__ __launch_bounds__(THREADS, 2) void attn_bwd_f32_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) char smem[2][2 * TILE];
+    __shared__ __attribute__((aligned(16))) char vrows[2][TILE];
+    __shared__ __attribute__((aligned(16))) StatTile sstat[2];
+    const int tile = blockIdx.y >> 1;
+    if (blockIdx.y & 1) bwd_dq<HAS_MASK, TRAIN>(a, blockIdx.x, (gridDim.y >> 1) - 1 - tile, smem);
+    else bwd_dkdv<HAS_MASK, TRAIN>(a, blockIdx.x, tile, smem, vrows, sstat);
+}
+
+}  // namespace
+
+#define F32_LAUNCH(KERNEL, grid)                                                                                     \
+    do {                                                                                                             \
+        if (a.mask && a.train) hipLaunchKernelGGL((KERNEL<true, true>), grid, dim3(THREADS), 0, st, a);              \
+        else if (a.mask) hipLaunchKernelGGL((KERNEL<true, false>), grid, dim3(THREADS), 0, st, a);                   \
+        else if (a.train) hipLaunchKernelGGL((KERNEL<false, true>), grid, dim3(THREADS), 0, st, a);                  \
+        else hipLaunchKernelGGL((KERNEL<false, false>), grid, dim3(THREADS), 0, st, a);                              \
+    } while (0)
+
+namespace ptj_attn_detail {
+void launch_fwd_f32(const AttnArgs& a, hipStream_t st) {
+    F32_LAUNCH(attn_fwd_f32_kernel, dim3((unsigned)(a.B * a.H), (unsigned)((a.T + 127) / 128)));
+}
+void launch_bwd_f32(const AttnArgs& a, hipStream_t st) {
+    F32_LAUNCH(attn_bwd_f32_kernel, dim3((unsigned)(a.B * a.H), (unsigned)(2 * ((a.T + 127) / 128))));
+}
+}  // namespace ptj_attn_detail

@@ -1,0 +1,70 @@
+"""fp32 attention on the bf16 matrix pipe: every factor is split into three bf16 values.  Against fp64, at the edges of the
+tiles and of what the split covers."""
+import pytest
+import torch
+
+from util import gen, randn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def case(B, H, T, seed):
+    g = gen(seed)
+    qkv, do = randn(g, B, H, 3, T, 64).to(DEV), randn(g, B, H, T, 64).to(DEV)
+    # documents that end inside a 32-row block, at its end and inside the next one, and a padded tail
+    doc = torch.bucketize(torch.arange(T), torch.tensor([24, 32, 70, T - 9]), right=True)
+    mask = torch.tril(doc[:, None] == doc[None, :]) & (doc < 4)[:, None] & (doc < 4)[None, :]
+    return qkv, do, mask.expand(B, T, T).contiguous().to(DEV)
+
+
+def both(mt, qkv, do, mask, train=False):
+    o, acts = mt.t_scaled_dot_prod_attn_fwd3_t(qkv, mask, train, 3)
+    return (o,) + tuple(mt.t_scaled_dot_prod_attn_bkwd3_t(do, acts, qkv, mask, train, 3))
+
+
+def exact(qkv, do, mask):
+    q, k, v = (qkv[:, :, i].double().cpu().requires_grad_() for i in range(3))
+    s = (q @ k.transpose(-1, -2) / 8).masked_fill(~mask.cpu()[:, None], -1e9)
+    o = 0.9 * torch.softmax(s, -1) * mask.cpu().any(-1)[:, None, :, None] @ v
+    return [x.detach() for x in (o,) + torch.autograd.grad(o, (q, k, v), do.double().cpu())]
+
+
+@pytest.mark.parametrize("B,H,T", [(1, 1, 64), (2, 1, 128), (1, 3, 192), (1, 2, 448)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_error_against_fp64(mt, B, H, T, masked):
+    """A score of 64 products is rounded 24 times, a sum over T keys 6 T / 16 times, by 2^-24 / sqrt(3) of its largest partial
+    sum each; up to T = 448 these walks stay below 2^-24 sqrt(24 + 168) / sqrt(3) = 4.8e-7, and a factor of 2 covers P and dS,
+    which carry the errors of the scores.  Two parts of a factor in place of three leave 2^-17."""
+    qkv, do, mask = case(B, H, T, T)
+    if not masked:
+        mask = torch.ones(T, T, dtype=torch.bool, device=DEV).tril().expand(B, T, T).contiguous()
+    for got, want, what in zip(both(mt, qkv, do, mask), exact(qkv, do, mask), ("o", "dq", "dk", "dv")):
+        assert (got.double().cpu() - want).norm() <= 1e-6 * want.norm(), what
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_gradients_scale_exactly(mt, train):
+    """Every gradient is linear in dO: with dO a power of two smaller all parts, products and sums are, too."""
+    qkv, do, mask = case(1, 2, 192, 5)
+    a, b = both(mt, qkv, do, mask, train), both(mt, qkv, do * 2.0 ** -60, mask, train)
+    assert all(torch.equal(x * 2.0 ** -60, y) for x, y in zip(a[1:], b[1:]))
+
+
+def test_large_and_infinite_values(mt):
+    T = 192
+    qkv, do, mask = case(1, 1, T, 6)
+    mask = torch.ones(T, T, dtype=torch.bool, device=DEV).tril()[None]
+    plain = both(mt, qkv, do, mask)[0]
+    big = qkv.clone()
+    big[:, :, 2] *= 2.0 ** 121                      # its parts are formed by truncation
+    got = both(mt, big, do, mask)[0]
+    assert (got.double() * 2.0 ** -121 - plain.double()).norm() <= 1e-6 * plain.double().norm()
+    inf = qkv.clone()
+    inf[0, 0, 2, 70, 5], inf[0, 0, 2, 130, 9] = float("inf"), float("-inf")
+    got = both(mt, inf, do, mask)[0][0, 0]
+    assert torch.isposinf(got[70:, 5]).all() and torch.isneginf(got[130:, 9]).all()
+    # (a hidden key's probability is 0 and 0 * inf is NaN where its tile is visited, as it was with fp32 products)
+    clean = torch.ones_like(got, dtype=torch.bool)
+    clean[:, 5] = clean[:, 9] = False
+    assert (got[clean] - plain[0, 0][clean]).norm() <= 1e-6 * plain.norm()
