@@ -74,3 +74,27 @@ def test_adamw_multi_equals_single_tensor_calls(lo, pkg):
     for k in range(len(sizes)):
         assert torch.equal(a_p[0][k], b_p[k]) and torch.equal(a_sh[0][k], b_sh[k])
         assert torch.equal(a_mom[0][0][k], b_m[k]) and torch.equal(a_mom[1][0][k], b_v[k])
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1025, 4 * (1 << 26) + 1029])
+def test_adamw_sizes_around_vectors_and_workgroups(pkg, n):
+    """Rests of a vector, of a workgroup, and a tensor with more vectors than a launch has threads for one tensor: equal to the
+    same update of its pieces."""
+    _lib = pkg._lib
+    g = torch.Generator(device="cuda").manual_seed(n)
+    p = torch.randn(n, generator=g, device="cuda")
+    grad = torch.randn(n, generator=g, device="cuda").to(torch.bfloat16)
+    cut = min(n, 4 * (n // 8) + 4)              # a piece boundary on the 4-element grid
+    whole, parts = ([p.clone(), torch.zeros_like(p), torch.zeros_like(p), torch.zeros_like(grad)] for _ in range(2))
+    for tensors, ranges in ((whole, [(0, n)]), (parts, [(0, cut), (cut, n)])):
+        for a, b in ranges:
+            for i in range(a, b, 1 << 26):      # pieces below the limit, but for `whole`
+                e = b if tensors is whole else min(b, i + (1 << 26))
+                t = [x[i:e] for x in tensors] + [grad[i:e]]
+                _lib.check(_lib.lib().ptj_adamw(_lib.ptr(t[0]), _lib.ptr(t[1]), _lib.ptr(t[2]), _lib.ptr(t[4]), _lib.ptr(t[3]), e - i,
+                                                1e-3, 0.9, 0.95, 1e-8, 0.1, 1, 1, 1, _lib.stream()), "ptj_adamw")
+                if tensors is whole:
+                    break
+    for x, y in zip(whole, parts):
+        assert torch.equal(x, y)
+    assert not torch.equal(whole[0], p)
