@@ -245,14 +245,15 @@ __global__ __launch_bounds__(256) void attn_mask_classes_kernel(const uint32_t* 
         ck[(b * G + kg) * (int64_t)G + qg] = cls;
     }
 }
-// classes of the two 32-wide halves of tile step `t` in the class row at `row` (wave-uniform)
+// classes of the 32-wide sub-tiles from number `g` on that a wavefront takes of a tile (wave-uniform)
 struct TileClasses { uint32_t c0, c1; };
-__device__ __forceinline__ TileClasses load_classes(const uint32_t* __restrict__ row, int t) {
-    TileClasses c;
-    const uniform_words p = as_uniform(row + 2 * t);
-    c.c0 = p[0];
-    c.c1 = p[1];
-    return c;
+template <bool HALVES> __device__ __forceinline__ TileClasses load_classes(const uint32_t* __restrict__ row, int g) {
+    const uniform_words p = as_uniform(row + g);
+    return {p[0], HALVES ? (uint32_t)TILE_HIDDEN : p[1]};
+}
+template <bool HALVES> __device__ __forceinline__ KeepWords load_keep(const uint32_t* __restrict__ line, int base) {
+    if constexpr (HALVES) return load_keep_half(line, base);
+    else return load_keep_words(line, base);
 }
 
 // Which tile and batch-head a workgroup of a grid (B*H, tiles) takes.  In dispatch order tiles go from long to short; every
@@ -333,7 +334,7 @@ __global__ __launch_bounds__(ATT_THREADS, 3) void attn_fwd_kernel(const AttnArgs
     if constexpr (HAS_MASK) {
         const int G = a.T >> 5;
         crow = a.mask + 2 * (int64_t)a.B * G * a.T + ((int64_t)bidx * G + (qw0u >> 5)) * G;
-        tc_next = load_classes(crow, 0);
+        tc_next = load_classes<false>(crow, 0);
     }
     int st = 0;   // this tile's place in LDS
     for (int kt = 0; kt < nkt; ++kt) {
@@ -342,7 +343,7 @@ __global__ __launch_bounds__(ATT_THREADS, 3) void attn_fwd_kernel(const AttnArgs
         const KeepWords kw = kw_next;
         if constexpr (TRAIN) kw_next = load_keep_words(kline, qw0u + (kt + 1) * 64);
         const TileClasses tc = tc_next;
-        if constexpr (HAS_MASK) tc_next = load_classes(crow, kt + 1 < nkt ? kt + 1 : kt);
+        if constexpr (HAS_MASK) tc_next = load_classes<false>(crow, 2 * (kt + 1 < nkt ? kt + 1 : kt));
         __builtin_amdgcn_sched_barrier(0);
         const int key0 = kt * 64;
         // some key of this tile is visible to some query of the wave
@@ -441,6 +442,15 @@ __global__ __launch_bounds__(ATT_THREADS, 3) void attn_fwd_kernel(const AttnArgs
     }
 }
 
+// How the four wavefronts of a workgroup share the backward's work on its tiles of 64 rows.  Whole: four blocks of 32 rows of their own,
+// each against every tile.  Halves: two blocks, and of every tile one half for each wavefront of a block; the two results are put
+// together at the end.
+template <bool HALVES> struct Share {
+    static constexpr int BLOCKS = HALVES ? 2 : 4, ROWS = 32 * BLOCKS, NJ = HALVES ? 1 : 2;
+    int block, half;     // the wavefront's block; first sub-tile of 32 rows that it takes of a tile
+    __device__ __forceinline__ Share(int wave) : block(wave % BLOCKS), half(wave / BLOCKS) {}
+};
+
 // ---- backward: dK, dV -------------------------------------------------------------------
 // One workgroup per (batch-head, 128 keys): wave w owns keys key0 + 32w .. +31 (lane = key); query tiles of 64.
 // OWN_DELTA: delta = rowsum(dO * O) is formed here, from the dO rows on their way into LDS and the O rows beside
@@ -463,15 +473,16 @@ __device__ __forceinline__ void store_delta(float* __restrict__ delta, int i, fl
 constexpr int RAW_STATS = 3 * 64 * 4;     // bytes of a query tile's saved maxima, sums and delta
 constexpr int dkdv_stage(bool own_delta) { return (own_delta ? 3 : 2) * PANEL + RAW_STATS; }   // Q, dO (, O), statistics
 template <bool OWN_DELTA> constexpr int dkdv_lds() { return RING * dkdv_stage(OWN_DELTA); }
-template <bool HAS_MASK, bool TRAIN, bool OWN_DELTA>
+template <bool HAS_MASK, bool TRAIN, bool OWN_DELTA, bool HALVES>
 __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, const int key_tile, char* smem, StatTile* sstat) {
     constexpr int STAGE = dkdv_stage(OWN_DELTA);
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Share<HALVES> share(wave_u);
     const int lr = lane & 31, lg = lane >> 5;
     const int bidx = bh / a.H, hidx = bh % a.H;
-    const int key0 = key_tile * 128;
-    const int kw0 = key0 + wave * 32;
+    const int key0 = key_tile * Share<HALVES>::ROWS;
+    const int kw0 = key0 + share.block * 32;
     const int key = kw0 + lr;
     const int krow = key < a.T ? key : a.T - 1;
 
@@ -498,7 +509,6 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
 #pragma unroll
         for (int e = 0; e < 16; ++e) dk[t][e] = dv[t][e] = 0.f;
 
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const uint32_t lds0 = lds_addr(smem);
     PanelCopy cq, cd, co;
     // The statistics come with the tile; the first wavefront copies them, converts them once they have landed
@@ -548,25 +558,26 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
     const float sc = a.scale * LOG2E;
     // keep-bit line of this batch-head and the wave's first key as scalars
     const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
-    const int kw0u = lookup_row(key0 + wave_u * 32, a.T);
+    const int kw0u = lookup_row(kw0, a.T);
     KeepWords kw_next;
-    if constexpr (TRAIN) kw_next = load_keep_words(kline, kw0u + qt0 * 64);
+    if constexpr (TRAIN) kw_next = load_keep<HALVES>(kline, kw0u + share.half * 32 + qt0 * 64);
     // tile classes of the wave's 32 keys against every 32-query group (explicit mask only)
     const uint32_t* __restrict__ crow = nullptr;
     TileClasses tc_next = {TILE_CAUSAL, TILE_CAUSAL};
     if constexpr (HAS_MASK) {
         const int G = a.T >> 5;
         crow = a.mask + 2 * (int64_t)a.B * G * a.T + (int64_t)a.B * G * G + ((int64_t)bidx * G + (kw0u >> 5)) * G;
-        if (qt0 < nqt) tc_next = load_classes(crow, qt0);
+        tc_next = load_classes<HALVES>(crow, 2 * qt0 + share.half);
     }
     int slot = 0;   // this tile's place in LDS
     for (int qt = qt0; qt < nqt; ++qt) {
         const int st = (qt - qt0) & 1;
         if (qt + 2 < nqt) KV_COPY(qt + 2, next_slot(next_slot(slot)))
         const KeepWords kw = kw_next;   // requested one step ago
-        if constexpr (TRAIN) kw_next = load_keep_words(kline, kw0u + (qt + 1) * 64);
+        const int ahead = qt + 1 < nqt ? qt + 1 : qt;
+        if constexpr (TRAIN) kw_next = load_keep<HALVES>(kline, kw0u + share.half * 32 + ahead * 64);
         const TileClasses tc = tc_next;
-        if constexpr (HAS_MASK) tc_next = load_classes(crow, qt + 1 < nqt ? qt + 1 : qt);
+        if constexpr (HAS_MASK) tc_next = load_classes<HALVES>(crow, 2 * ahead + share.half);
         __builtin_amdgcn_sched_barrier(0);
         const int q0 = qt * 64;
         if (q0 + 63 >= kw0) {   // some query of the tile sees some key of the wave
@@ -574,9 +585,10 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
             // The two 32-query halves are processed one after the other: half the live
             // accumulators, which keeps two wavefronts per SIMD resident.
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int jj = 0; jj < Share<HALVES>::NJ; ++jj) {
+                const int j = HALVES ? share.half : jj;
                 if (q0 + j * 32 + 31 < kw0) continue;   // every query of this half precedes the wave's keys
-                const uint32_t cls = j == 0 ? tc.c0 : tc.c1;
+                const uint32_t cls = jj == 0 ? tc.c0 : tc.c1;
                 if (HAS_MASK && cls == TILE_HIDDEN) continue;
                 RowFrags<1> qa, da;
                 qa.read(base, j, lr, lg);
@@ -618,7 +630,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
                         if constexpr (TRAIN) {
                             // dS = P (keep ? dP : 0) - P delta = (keep ? P : 0) dP - P delta: the dropped
                             // probability is needed anyway, so one select serves both products
-                            const uint64_t km = keep_lane_mask_at(kw, j * 32 + g4 * 8 + b);
+                            const uint64_t km = keep_lane_mask_at(kw, jj * 32 + g4 * 8 + b);
                             pd[i] = keep_select(p, km);
                             ds[i] = fmaf(pd[i], dp[i], -(p * d4[b]));
                         } else {
@@ -641,7 +653,23 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
 #undef KV_COPY
 #undef KV_LAND
 
-    if (key < a.T) {
+    if constexpr (HALVES) {
+        // both halves of the queries together: the wavefronts of the first half finish dK, those of the second dV
+        lds_barrier();
+        float give[32], take[32];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) give[16 * t + e] = share.half ? dk[t][e] : dv[t][e];
+        exchange(give, take, smem, wave_u, wave_u ^ 2, lane);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) dk[t][e] = (share.half ? dv[t][e] : dk[t][e]) + take[16 * t + e];
+        store_rows<bf16>(share.half ? (bf16*)a.out1 + bidx * a.out1_bs + hidx * a.out1_hs + (int64_t)key * a.out1_rs
+                                    : (bf16*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)key * a.out0_rs,
+                         dk, share.half ? 1.0f : a.scale, lg);
+    } else if (key < a.T) {
         store_rows<bf16>((bf16*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)key * a.out0_rs, dk, a.scale, lg);
         store_rows<bf16>((bf16*)a.out1 + bidx * a.out1_bs + hidx * a.out1_hs + (int64_t)key * a.out1_rs, dv, 1.0f, lg);
     }
@@ -650,15 +678,16 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnArgs& a, const int bh, c
 // ---- backward: dQ -----------------------------------------------------------------------
 // Same geometry as the forward (lane = query, key tiles of 64).
 constexpr int DQ_LDS = RING * 2 * PANEL;
-template <bool HAS_MASK, bool TRAIN, bool STORE_DELTA>
+template <bool HAS_MASK, bool TRAIN, bool STORE_DELTA, bool HALVES>
 __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, const int query_tile, char* smem) {
     constexpr int STAGE = 2 * PANEL;          // K, V
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Share<HALVES> share(wave_u);
     const int lr = lane & 31, lg = lane >> 5;
     const int bidx = bh / a.H, hidx = bh % a.H;
-    const int q0 = query_tile * 128;
-    const int qw0 = q0 + wave * 32;
+    const int q0 = query_tile * Share<HALVES>::ROWS;
+    const int qw0 = q0 + share.block * 32;
     const int query = qw0 + lr;
     const int qrow = query < a.T ? query : a.T - 1;
 
@@ -690,10 +719,9 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
     }
     const float m2 = none ? 0.f : fmaf(a.ms[si], LOG2E, __builtin_amdgcn_logf(lsum));
 
-    int nkt = (q0 + 128) / 64;
+    int nkt = (q0 + Share<HALVES>::ROWS) / 64;
     if (nkt > a.T / 64) nkt = a.T / 64;
 
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const uint32_t lds0 = lds_addr(smem);
     PanelCopy ck, cv;
 #define DQ_COPY(KT, SLOT)                                                              \
@@ -718,23 +746,24 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
         for (int e = 0; e < 16; ++e) dq[t][e] = 0.f;
 
     const uint32_t* __restrict__ kline = a.keepbits + (int64_t)bh * a.bitwords;
-    const int qw0u = lookup_row(q0 + wave_u * 32, a.T);
+    const int qw0u = lookup_row(qw0, a.T);
     KeepWords kw_next;
-    if constexpr (TRAIN) kw_next = load_keep_words(kline, qw0u);
+    if constexpr (TRAIN) kw_next = load_keep<HALVES>(kline, qw0u + share.half * 32);
     const uint32_t* __restrict__ crow = nullptr;
     TileClasses tc_next = {TILE_CAUSAL, TILE_CAUSAL};
     if constexpr (HAS_MASK) {
         const int G = a.T >> 5;
         crow = a.mask + 2 * (int64_t)a.B * G * a.T + ((int64_t)bidx * G + (qw0u >> 5)) * G;
-        tc_next = load_classes(crow, 0);
+        tc_next = load_classes<HALVES>(crow, share.half);
     }
     int st = 0;   // this tile's place in LDS
     for (int kt = 0; kt < nkt; ++kt) {
         if (kt + 2 < nkt) DQ_COPY(kt + 2, next_slot(next_slot(st)))
         const KeepWords kw = kw_next;   // requested one step ago
-        if constexpr (TRAIN) kw_next = load_keep_words(kline, qw0u + (kt + 1) * 64);
+        const int ahead = kt + 1 < nkt ? kt + 1 : kt;
+        if constexpr (TRAIN) kw_next = load_keep<HALVES>(kline, qw0u + share.half * 32 + ahead * 64);
         const TileClasses tc = tc_next;
-        if constexpr (HAS_MASK) tc_next = load_classes(crow, kt + 1 < nkt ? kt + 1 : kt);
+        if constexpr (HAS_MASK) tc_next = load_classes<HALVES>(crow, 2 * ahead + share.half);
         __builtin_amdgcn_sched_barrier(0);
         const int key0 = kt * 64;
         if (key0 <= qw0 + 31) {
@@ -742,10 +771,11 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
             // The two 32-key halves one after the other: half the live accumulators, and a half
             // whose keys all follow the wave's queries is skipped.
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int jj = 0; jj < Share<HALVES>::NJ; ++jj) {
+                const int j = HALVES ? share.half : jj;
                 const int kh0 = key0 + j * 32;
                 if (kh0 > qw0 + 31) continue;
-                const uint32_t cls = j == 0 ? tc.c0 : tc.c1;
+                const uint32_t cls = jj == 0 ? tc.c0 : tc.c1;
                 if (HAS_MASK && cls == TILE_HIDDEN) continue;
                 RowFrags<1> ka, va;
                 ka.read(base, j, lr, lg);
@@ -777,7 +807,7 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
                 for (int i = 0; i < 16; ++i) {
                     const float p = fast_exp2(fmaf(s[i], sc, -m2));
                     if constexpr (TRAIN)
-                        ds[i] = p * (keep_select(dp[i], keep_lane_mask_at(kw, j * 32 + (i >> 2) * 8 + (i & 3))) - delta);
+                        ds[i] = p * (keep_select(dp[i], keep_lane_mask_at(kw, jj * 32 + (i >> 2) * 8 + (i & 3))) - delta);
                     else
                         ds[i] = p * fmaf(dp[i], 0.9f, -delta);
                 }
@@ -792,7 +822,15 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnArgs& a, const int bh, con
     }
 #undef DQ_COPY
 
-    if (query < a.T)
+    if constexpr (HALVES) {
+        float give[16], take[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) give[e] = share.half ? dq[0][e] : dq[1][e];
+        exchange(give, take, smem, wave_u, wave_u ^ 2, lane);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) take[e] += share.half ? dq[1][e] : dq[0][e];
+        store_half_row<bf16>((bf16*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs + share.half * 32, take, a.scale, lg);
+    } else if (query < a.T)
         store_rows<bf16>((bf16*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs, dq, a.scale, lg);
 }
 
@@ -803,34 +841,35 @@ template <bool HAS_MASK, bool TRAIN>
 __global__ __launch_bounds__(ATT_THREADS, 3) void attn_bwd_dq_kernel(const AttnArgs a) {
     __shared__ __attribute__((aligned(16))) char smem[DQ_LDS];
     const Place pl = place();
-    attn_bwd_dq<HAS_MASK, TRAIN, true>(a, pl.bh, gridDim.y - 1 - pl.tile, smem);
+    attn_bwd_dq<HAS_MASK, TRAIN, true, false>(a, pl.bh, gridDim.y - 1 - pl.tile, smem);
 }
 template <bool HAS_MASK, bool TRAIN>
 __global__ __launch_bounds__(ATT_THREADS, 2) void attn_bwd_dkdv_kernel(const AttnArgs a) {
     __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<false>()];
     __shared__ __attribute__((aligned(16))) StatTile sstat[2];
     const Place pl = place();
-    attn_bwd_dkdv<HAS_MASK, TRAIN, false>(a, pl.bh, pl.tile, smem, sstat);
+    attn_bwd_dkdv<HAS_MASK, TRAIN, false, false>(a, pl.bh, pl.tile, smem, sstat);
 }
-// Both in one launch, grid (B*H, 2 ceil(T/128)).
-template <bool HAS_MASK, bool TRAIN>
+// Both in one launch, grid (B*H, 2 ceil(T/ROWS)).
+template <bool HAS_MASK, bool TRAIN, bool HALVES>
 __global__ __launch_bounds__(ATT_THREADS, 2) void attn_bwd_kernel(const AttnArgs a) {
     __shared__ __attribute__((aligned(16))) char smem[dkdv_lds<true>()];
     __shared__ __attribute__((aligned(16))) StatTile sstat[2];
     const int tile = blockIdx.y >> 1;
-    if (blockIdx.y & 1) attn_bwd_dq<HAS_MASK, TRAIN, false>(a, blockIdx.x, (gridDim.y >> 1) - 1 - tile, smem);
-    else attn_bwd_dkdv<HAS_MASK, TRAIN, true>(a, blockIdx.x, tile, smem, sstat);
+    if (blockIdx.y & 1) attn_bwd_dq<HAS_MASK, TRAIN, false, HALVES>(a, blockIdx.x, (gridDim.y >> 1) - 1 - tile, smem);
+    else attn_bwd_dkdv<HAS_MASK, TRAIN, true, HALVES>(a, blockIdx.x, tile, smem, sstat);
 }
 
-// Launch one of the (mask, train) specialisations.
-#define ATTN_LAUNCH(KERNEL, grid, st, args)                                                        \
-    do {                                                                                               \
-        const bool hm__ = (args).mask != nullptr, tr__ = (args).train != 0;                            \
-        if (hm__ && tr__) hipLaunchKernelGGL((KERNEL<true, true>), grid, dim3(ATT_THREADS), 0, st, args);        \
-        else if (hm__) hipLaunchKernelGGL((KERNEL<true, false>), grid, dim3(ATT_THREADS), 0, st, args);          \
-        else if (tr__) hipLaunchKernelGGL((KERNEL<false, true>), grid, dim3(ATT_THREADS), 0, st, args);          \
-        else hipLaunchKernelGGL((KERNEL<false, false>), grid, dim3(ATT_THREADS), 0, st, args);                   \
+// Launch one of the (mask, train) specialisations; further template arguments behind them.
+#define ATTN_LAUNCH(KERNEL, grid, st, args, ...)                                                                              \
+    do {                                                                                                                      \
+        const bool hm__ = (args).mask != nullptr, tr__ = (args).train != 0;                                                   \
+        if (hm__ && tr__) hipLaunchKernelGGL((KERNEL<true, true __VA_ARGS__>), grid, dim3(ATT_THREADS), 0, st, args);         \
+        else if (hm__) hipLaunchKernelGGL((KERNEL<true, false __VA_ARGS__>), grid, dim3(ATT_THREADS), 0, st, args);           \
+        else if (tr__) hipLaunchKernelGGL((KERNEL<false, true __VA_ARGS__>), grid, dim3(ATT_THREADS), 0, st, args);           \
+        else hipLaunchKernelGGL((KERNEL<false, false __VA_ARGS__>), grid, dim3(ATT_THREADS), 0, st, args);                    \
     } while (0)
+#define ATT_COMMA ,
 
 // ---- host side ----------------------------------------------------------------------------
 inline size_t bits_bytes(int64_t BH, int64_t T) { return (size_t)BH * ptj_attn_bitwords(T) * sizeof(uint32_t); }
@@ -867,8 +906,16 @@ int launch_keepbits(uint32_t* bits, int64_t count, const int64_t* seeds, int64_t
 void launch_fwd(const AttnArgs& a, int dtype, hipStream_t st) {
     const dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.T + 127) / 128));
     if (dtype == PTJ_F32) ptj_attn_detail::launch_fwd_f32(a, st);
-    else ATTN_LAUNCH(attn_fwd_kernel, grid, st, a);
+    else ATTN_LAUNCH(attn_fwd_kernel, grid, st, a, );
 }
+
+// Halves (Share) where the grid leaves CUs idle: twice the workgroups and half the work per wavefront and tile, against a second
+// look at every tile and the exchange at the end.  Up to three workgroups of 64 rows per CU from T = 512 on, where the short ones
+// fill in behind the long ones, and fewer below, where they are more alike.  One tile has nothing to share.  us, whole / halves, 12
+// heads with dropout: 2 x 128 11.5 / 10.7, 8 x 128 12.5 / 13.0, 2 x 192 14.1 / 12.3, 8 x 192 16.1 / 18.4, 2 x 256 16.5 / 13.9, 4 x 448
+// 24.7 / 21.5, 7 x 448 29.2 / 31.6, 2 x 1024 43.0 / 34.8, 4 x 1024 46.3 / 57.1.  (The forward would gain as well, 2 x 256 11.0 / 9.2, but its
+// bits are the same for a row in every batch.)
+bool bwd_in_halves(int64_t bh, int64_t T) { return T > 64 && bh * 2 * ((T > 512 ? T : 512) / 64) <= 3 * (int64_t)ptj_num_cus(); }
 
 // One launch while the two passes' workgroups make no more than four rounds of one per CU, two launches beyond.  The passes
 // then fill each other's idle CUs and a launch is saved, against an O tile read again per query tile of dK/dV (delta) and
@@ -878,13 +925,14 @@ void launch_fwd(const AttnArgs& a, int dtype, hipStream_t st) {
 void launch_bwd(const AttnArgs& a, int dtype, hipStream_t st) {
     if (dtype == PTJ_F32) return ptj_attn_detail::launch_bwd_f32(a, st);
     const int64_t nt = (a.T + 127) / 128;
-    const bool one = (int64_t)a.B * a.H * nt * 2 <= (int64_t)4 * ptj_num_cus();
-    const dim3 grid((unsigned)(a.B * a.H), (unsigned)nt), grid2((unsigned)(a.B * a.H), (unsigned)(2 * nt));
-    if (one) {
-        ATTN_LAUNCH(attn_bwd_kernel, grid2, st, a);
+    const unsigned bh = (unsigned)(a.B * a.H);
+    if (bwd_in_halves(bh, a.T)) {
+        ATTN_LAUNCH(attn_bwd_kernel, dim3(bh, (unsigned)(2 * (a.T / 64))), st, a, ATT_COMMA true);
+    } else if ((int64_t)bh * nt * 2 <= (int64_t)4 * ptj_num_cus()) {
+        ATTN_LAUNCH(attn_bwd_kernel, dim3(bh, (unsigned)(2 * nt)), st, a, ATT_COMMA false);
     } else {
-        ATTN_LAUNCH(attn_bwd_dq_kernel, grid, st, a);
-        ATTN_LAUNCH(attn_bwd_dkdv_kernel, grid, st, a);
+        ATTN_LAUNCH(attn_bwd_dq_kernel, dim3(bh, (unsigned)nt), st, a, );
+        ATTN_LAUNCH(attn_bwd_dkdv_kernel, dim3(bh, (unsigned)nt), st, a, );
     }
 }
 

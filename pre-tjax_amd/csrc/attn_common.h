@@ -83,6 +83,11 @@ __device__ __forceinline__ KeepWords load_keep_words(const uint32_t* __restrict_
     w.d2 = p[2];
     return w;
 }
+// The same for 32 x 32 elements (offsets below 32 look at two words)
+__device__ __forceinline__ KeepWords load_keep_half(const uint32_t* __restrict__ line, int base) {
+    const uniform_words p = as_uniform(line + (base >> 5));
+    return {p[0], p[1], 0u};
+}
 template <int C> __device__ __forceinline__ uint32_t keep_win32(const KeepWords& w) {
     static_assert(C >= 0 && C < 64, "window offset");
     const uint64_t v = C < 32 ? (((uint64_t)w.d1 << 32) | w.d0) : (((uint64_t)w.d2 << 32) | w.d1);
@@ -143,6 +148,26 @@ __device__ __forceinline__ void store_rows(T* __restrict__ row, const f32x16 (&a
         }
 }
 
+// Where two wavefronts share a block of rows, each against one half of every tile: `give` goes to the partner, what the partner
+// gives comes.  Everything in `smem` has been read.
+template <int N>
+__device__ __forceinline__ void exchange(const float (&give)[N], float (&take)[N], char* __restrict__ smem, int wave, int partner, int lane) {
+    float* const f = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int i = 0; i < N; ++i) f[(wave * N + i) * 64 + lane] = give[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) take[i] = f[(partner * N + i) * 64 + lane];
+}
+// 32 columns of a row: element e of lane half lg is column 8 (e / 4) + 4 lg + e % 4
+template <typename T>
+__device__ __forceinline__ void store_half_row(T* __restrict__ row, const float (&x)[16], float f, int lg) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        const float v[4] = {x[4 * a] * f, x[4 * a + 1] * f, x[4 * a + 2] * f, x[4 * a + 3] * f};
+        store_vec<T, 4>(row + a * 8 + lg * 4, v);
+    }
+}
 // Class of a 32x32 tile of (mask AND causal), see attn_mask_classes_kernel
 enum { TILE_HIDDEN = 0, TILE_MIXED = 1, TILE_CAUSAL = 2 };
 // ---- element-wise pieces (VALU budget: a wave64 VALU op costs 4 cycles, v_exp 16, and one

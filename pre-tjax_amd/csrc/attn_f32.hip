@@ -141,11 +141,6 @@ struct TileCopy {
     }
 };
 
-// Keep bits of 32 x 32 elements (keep_lane_mask_at with offsets below 32 looks at two words)
-__device__ __forceinline__ KeepWords load_keep_half(const uint32_t* __restrict__ line, int base) {
-    const uniform_words p = as_uniform(line + (base >> 5));
-    return {p[0], p[1], 0u};
-}
 __device__ __forceinline__ uint64_t keep_mask(const KeepWords& w, int i) { return keep_lane_mask_at(w, (i >> 2) * 8 + (i & 3)); }
 
 // The mask words of a mixed tile: hidden elements become NEG_RAW
@@ -158,24 +153,21 @@ __device__ __forceinline__ void apply_mask(f32x16& s, const uint32_t* __restrict
     for (int i = 0; i < 16; ++i) s[i] = mask_select(s[i], NEG_RAW, mask_lanes(w, i));
 }
 
-// Accumulators of this wavefront's partner (the other half of the tiles), through LDS: `give` goes, what the partner gives comes.
-// Everything in `smem` has been read.
-template <int N>
-__device__ __forceinline__ void exchange(const float (&give)[N], float (&take)[N], char* __restrict__ smem, int wave, int lane) {
-    float* const f = reinterpret_cast<float*>(smem);
+// The forward's results of both wavefronts: o[half] is finished here (f: its factor, without the row's probability sum).
+struct RowStats { float m_run, m_true, l; };
+__device__ __forceinline__ RowStats merge_halves(float (&out)[16], const f32x16 (&o)[2], RowStats mine, int half, char* __restrict__ smem, int wave,
+                                                 int partner, int lane) {
+    float give[19], take[19];
 #pragma unroll
-    for (int i = 0; i < N; ++i) f[(wave * N + i) * 64 + lane] = give[i];
-    __syncthreads();
+    for (int e = 0; e < 16; ++e) give[e] = half ? o[0][e] : o[1][e];
+    give[16] = mine.m_run;
+    give[17] = mine.m_true;
+    give[18] = mine.l;
+    exchange(give, take, smem, wave, partner, lane);
+    const float m_run = fmaxf(mine.m_run, take[16]), f0 = fast_exp2(mine.m_run - m_run), f1 = fast_exp2(take[16] - m_run);
 #pragma unroll
-    for (int i = 0; i < N; ++i) take[i] = f[((wave ^ 4) * N + i) * 64 + lane];
-}
-// 32 columns of a row: element e of lane half lg is column 8 (e / 4) + 4 lg + e % 4
-__device__ __forceinline__ void store_half_row(float* __restrict__ row, const float (&x)[16], float f, int lg) {
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const float v[4] = {x[4 * a] * f, x[4 * a + 1] * f, x[4 * a + 2] * f, x[4 * a + 3] * f};
-        store_vec<float, 4>(row + a * 8 + lg * 4, v);
-    }
+    for (int e = 0; e < 16; ++e) out[e] = (half ? o[1][e] : o[0][e]) * f0 + take[e] * f1;
+    return {m_run, fmaxf(mine.m_true, take[17]), half ? fmaf(take[18], f1, mine.l * f0) : fmaf(mine.l, f0, take[18] * f1)};
 }
 
 // ---- forward -------------------------------------------------------------------------
@@ -293,27 +285,16 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
     }
 
     // Both halves of the keys together; each wavefront finishes the columns of its own half.
-    float give[19], take[19];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) give[e] = half ? o[0][e] : o[1][e];
-    give[16] = m_run;
-    give[17] = m_true;
-    give[18] = l_run;
-    exchange(give, take, &smem[0][0], wave, lane);
+    float out[16];
+    const RowStats r = merge_halves(out, o, {m_run, m_true, l_run}, half, &smem[0][0], wave, wave ^ 4, lane);
     if (query < a.T) {
-        const float m_all = fmaxf(m_run, take[16]), mine = fast_exp2(m_run - m_all), theirs = fast_exp2(take[16] - m_all);
-        const float l = half ? fmaf(take[18], theirs, l_run * mine) : fmaf(l_run, mine, take[18] * theirs);
-        m_true = fmaxf(m_true, take[17]);
         // l = 0: no key of the row is visible (a row with a visible key has l >= 1)
-        const bool empty = l == 0.f;
-        const float f = empty ? 0.f : (TRAIN ? 1.0f : 0.9f) / l;
-        float out[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) out[e] = (half ? o[1][e] : o[0][e]) * mine + take[e] * theirs;
-        store_half_row((float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs + half * 32, out, f, lg);
+        const bool empty = r.l == 0.f;
+        const float f = empty ? 0.f : (TRAIN ? 1.0f : 0.9f) / r.l;
+        store_half_row<float>((float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs + half * 32, out, f, lg);
         if (lg == 0 && half == 0) {
-            a.ms[(int64_t)bh * a.T + query] = empty ? NEG_NAT : m_true * LN2;
-            a.ls[(int64_t)bh * a.T + query] = empty ? 0.f : l * fast_exp2(m_all - m_true);
+            a.ms[(int64_t)bh * a.T + query] = empty ? NEG_NAT : r.m_true * LN2;
+            a.ls[(int64_t)bh * a.T + query] = empty ? 0.f : r.l * fast_exp2(r.m_run - r.m_true);
         }
     }
 }
@@ -466,7 +447,7 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) give[16 * t + e] = half ? dk[t][e] : dv[t][e];
-    exchange(give, take, &smem[0][0], wave, lane);
+    exchange(give, take, &smem[0][0], wave, wave ^ 4, lane);
     if (key < a.T) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -592,11 +573,11 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const in
     float give[16], take[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) give[e] = half ? dq[0][e] : dq[1][e];
-    exchange(give, take, &smem[0][0], wave, lane);
+    exchange(give, take, &smem[0][0], wave, wave ^ 4, lane);
     if (query < a.T) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) take[e] += half ? dq[1][e] : dq[0][e];
-        store_half_row((float*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs + half * 32, take, a.scale, lg);
+        store_half_row<float>((float*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs + half * 32, take, a.scale, lg);
     }
 }
 
