@@ -1,30 +1,29 @@
 // Persistent bf16 GEMM whose operand panels travel HBM -> LDS by asynchronous buffer copies into two rings,
 // one per operand.  Included by gemm_core.h inside its unnamed namespace, after gemm_tile.h.
 //
-// What bounds it: the LDS and the matrix pipe together.  Per 64 contraction elements a 256x256 tile (eight wavefronts of
-// 128x64) costs 2048 clocks of MFMAs, 1536 of fragment reads and 512 of arriving copies; a 256x192 tile
+// What bounds it: the power budget, then the feed.  Under this load the part holds 1.5-1.9 GHz, whatever switches is paid for in
+// clock, and the 16x16x32 instructions take less for the same products than the 32x32x16 ones (their accumulators move half as
+// often): alone, with their factors in registers, 2100 against 1850 TFLOP/s.  Per 64 contraction elements a 256x256 tile (eight
+// wavefronts of 128x64) costs 2048 clocks of MFMAs, 1536 of fragment reads and 512 of arriving copies; a 256x192 tile
 // (wavefronts of 64x96) 1536, 1280 and 448, so the wider tile gets more out of the matrix pipe and the narrower one is for
-// outputs that it cuts into fuller rounds (gemm_plan.h).  The A ring has three stages and the B ring two: the chunks
-// of a step are read into registers half a step ahead, so a stage is refilled halfway through the step that
+// outputs that it cuts into fuller rounds (gemm_plan.h).  The A ring has three stages and the B ring two: the chunk
+// of half a step is read into registers half a step ahead, so a stage is refilled halfway through the step that
 // multiplies it, and the copies of A have a step more to arrive than those of B.  160 KB hold no third stage
-// of B.  Reads and copies are spread over the MFMAs (bunched behind the barrier: 5 % slower).  What a step does besides is
-// kept small and away from the barrier, where both wavefronts of a SIMD wait and the matrix pipe idles: 167
-// instructions beside 32 MFMAs.
-// 8192x8192x8192: 783 us, 1400 TFLOP/s (the loops with two stages of 56 KB before this one: 975 us); 4096^3 with both
-// operands transposed 107 (147); 16384x768x3072 68 (74), with transposed B 67 (79).  Four wavefronts of 128x128 with one
-// chunk per register set: 905 us for 8192^3.
+// of B.  Reads are spread over the first 5/8 of the MFMAs that they run beside (7/8: 8192^3 763 us instead of 755), copies over all but
+// the last ones (bunched behind the barrier: 5 % slower), and the wavefronts that are past the barrier go first (740).
+// 32x32x16 instructions before / now, us on one box: 8192^3 812 / 740 (1486 TFLOP/s), 8192x50257x768 with bias 683 / 628, its
+// two gradient products 511 / 497 and 535 / 515, 16384x3072x768 with bias 86.9 / 80.4, with GELU and its derivative 118.8 / 113.6,
+// 16384x768x3072 70.3 / 67.3, dX of it 68.9 / 66.4, dW of it 82.6 / 81.9.  (With 32x32x16 the four plain 256x256 kernels spilled 33-50
+// registers as well.)  Four wavefronts of 128x128 with one chunk per register set: 905 us for 8192^3 where eight took 783.
 //
-// The output goes straight from the accumulators to memory: two lane swaps bring eight consecutive columns of a row
-// into a lane and 64 bytes of each of sixteen rows into a store, without LDS, which the rings fill.  At k = 768 the
-// output is a quarter of the time (16384x3072x768: 81 us, 60 without stores; 100 MB at 4.9 TB/s are 20).
-// GELU and its derivative come from one exponential (130 -> 118 us for 16384x3072x768 with both outputs).
-//
-// The copies run ahead across the tiles of a workgroup, but a tile's start waits for them all the same: the accumulators start
-// from bias registers that a vector path, an element path or zeros may have filled, and the compiler puts s_waitcnt vmcnt(0)
-// in front of their use, with a bias or without.  That drains the stores of the tile before as well, and in the 256x256 kernels
-// spilled registers (33-50 in all) are reloaded there.  Measured with this in place: stores kept in registers and sent between the MFMAs
-// of the next tile 86 us instead of 81; non-temporal ones 75, and 8192x50257x768 with them 620 -> 690; waits that leave
-// younger operations in flight the same.  None of it says what they would do without the drain.
+// The output goes straight from the accumulators to memory: a lane swap brings eight consecutive columns of a row
+// into a lane and 64 bytes of each of sixteen rows into a store, without LDS, which the rings fill.  At k = 768 a workgroup
+// of 16384x3072x768 spends 4 us before its first products, 15.7-18.8 in a tile's loop, 3.7 in the write-back (9 with GELU and its
+// derivative, which are vector work; 11 with a multiplier, which is memory) and 0.6 until the next loop.  That 0.6 is a wait for
+// everything under way, the stores included: the accumulators start from bias registers that a vector path, an element path or
+// zeros may have filled, and the compiler waits in front of their use.  Measured and not kept: non-temporal stores (alone up to
+// 8 % faster, but what reads the output next takes longer: training step 16 x 1024 +0.7 %, feed-forward block of 3001 tokens +14 %),
+// workgroups that start staggered so that their stores do not coincide (no gain).
 //
 // Rows and contraction indices past the operand's end read as zero (buffer descriptors).
 
@@ -33,7 +32,8 @@ template <int TBN_, int WM_, int WN_>
 struct RingCfg {
     static constexpr int TBM = 256, TBN = TBN_, WM = WM_, WN = WN_, NA = 3, NB = 2;
     static constexpr int NW = WM * WN, THREADS = NW * 64, TMW = TBM / WM / 32, TNW = TBN / WN / 32;
-    static_assert(TMW * WM * 32 == TBM && TNW * WN * 32 == TBN && NW == 8, "whole MFMA tiles, two wavefronts per SIMD");
+    static constexpr int TM = 2 * TMW, TN = 2 * TNW;                     // MFMA tiles of 16 x 16 per wavefront
+    static_assert(TMW * WM * 32 == TBM && TNW * WN * 32 == TBN && NW == 8, "whole pairs of MFMA tiles, two wavefronts per SIMD");
     static constexpr int A_STAGE = TBM * BKB, B_STAGE = TBN * BKB, SMEM = NA * A_STAGE + NB * B_STAGE;
 };
 typedef RingCfg<256, 2, 4> RingFull;
@@ -72,17 +72,28 @@ __device__ __forceinline__ int64_t ring_uniform(int64_t v) {
                      (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
 }
 
+// Order of the 16-byte pieces in LDS (XORed into a piece's index).  A fragment is 16 rows x 32 contraction elements.  KMAJOR: half
+// a wavefront reads two pieces of each of its sixteen rows; the sixteen lanes that are served at once (0-3, 12-15, 20-27, and
+// the others) find theirs in different banks.  MNMAJOR: half a wavefront reads two pieces of the k-rows 0-3 and 8-11, which the order
+// puts into different banks (192 rows: their pitch does half of it, and the order stays inside eight pieces).
+__device__ __forceinline__ int ring_sw(int row) { return row & 6; }
+template <int ROWS> __device__ __forceinline__ int ring_mn_sw(int k) {
+    if constexpr (ROWS == 192) return ((k >> 1) & 1) * 2 + ((k >> 3) & 1) * 4;
+    else return (k & 3) * 2 + ((k >> 3) & 1) * 8;
+}
+
 // One operand: the cursor of its copies, which runs ahead of the multiplications across work items, and the LDS addresses
-// of this wavefront's fragments.  ROWS rows of the tile in a stage, NT MFMA tiles of 32 rows per wavefront.
+// of this wavefront's fragments.  ROWS rows of the tile in a stage, NT MFMA tiles of 16 rows per wavefront.
 template <int MODE, int ROWS, int NT, int STAGES>
 struct RingOperand {
     static constexpr int NW = 8, PER = ROWS * BKB / 1024 / NW;           // copies per wavefront and stage
     static constexpr int PPR = ROWS / 8, PITCH = ROWS * 2;               // MNMAJOR: 16-byte pieces and bytes per k-row
     // the copies of a stage lie a whole number of swizzle periods apart: one address register for all of them
-    static constexpr bool EVEN = MODE == KMAJOR || (NW * 64 % PPR == 0 && NW * 64 / PPR % 4 == 0);
+    static constexpr bool EVEN = MODE == KMAJOR || (NW * 64 % PPR == 0 && NW * 64 / PPR % 16 == 0);
+    static constexpr int NADDR = MODE == MNMAJOR && ROWS == 192 ? 4 : 1;   // address registers
     uint32_t voff[EVEN ? 1 : PER], istep;
     int kk;                                                              // KMAJOR: k of this lane's vector in a step
-    uint32_t raddr[MODE == KMAJOR ? 1 : NT];
+    uint32_t raddr[NADDR];
     __amdgpu_buffer_rsrc_t rsrc;
     uint32_t v0;
     const char* base;                                                    // the next stage's first element
@@ -92,26 +103,26 @@ struct RingOperand {
     __device__ __forceinline__ void init(int64_t s_row, int64_t s_k, uint32_t region, int wrow, int tid) {
         const int lane = tid & 63;
         if constexpr (MODE == KMAJOR) {
-            const int r = tid >> 3, row = wrow + (lane & 31);
-            kk = ((lane & 7) ^ sw(r)) * 8;
+            const int r = tid >> 3, row = wrow + (lane & 15);
+            kk = ((lane & 7) ^ ring_sw(r)) * 8;
             voff[0] = ((uint32_t)r * (uint32_t)s_row + (uint32_t)kk) * 2u;
             istep = NW * 8 * (uint32_t)s_row * 2u;
             step = 128;
-            raddr[0] = region + row * BKB + (((lane >> 5) ^ sw(row)) << 4);
+            raddr[0] = region + row * BKB + (((lane >> 4) ^ ring_sw(row)) << 4);
         } else {
-            const int l16 = lane & 15, mhalf = (lane >> 4) & 1, lg = lane >> 5, kq = l16 >> 2;
+            const int l16 = lane & 15, kf = 8 * (lane >> 4) + (l16 >> 2);
             kk = 0;
 #pragma unroll
             for (int i = 0; i < (EVEN ? 1 : PER); ++i) {
                 const int pc = i * NW * 64 + tid, k = pc / PPR, pos = pc - k * PPR;
-                voff[i] = ((uint32_t)k * (uint32_t)s_k + (uint32_t)(pos ^ gt_mn_swz<ROWS>(k)) * 8u) * 2u;
+                voff[i] = ((uint32_t)k * (uint32_t)s_k + (uint32_t)(pos ^ ring_mn_sw<ROWS>(k)) * 8u) * 2u;
             }
             istep = NW * 64 / PPR * (uint32_t)s_k * 2u;
             step = 128 * s_k;
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const int piece = (wrow >> 3) + t * 4 + 2 * mhalf + ((l16 & 3) >> 1);
-                raddr[t] = region + (8 * lg + kq) * PITCH + ((piece ^ gt_mn_swz<ROWS>(kq)) << 4) + 8 * (l16 & 1);
+            for (int t = 0; t < NADDR; ++t) {
+                const int piece = (wrow >> 3) + 2 * t + ((l16 & 3) >> 1);
+                raddr[t] = region + kf * PITCH + ((piece ^ ring_mn_sw<ROWS>(kf)) << 4) + 8 * (l16 & 1);
             }
         }
         slot = 0;
@@ -139,38 +150,34 @@ struct RingOperand {
         if constexpr (EVEN && I > 0) asm volatile("v_add_u32 %0, %1, %2" : "=v"(v) : "s"(I * istep), "v"(v0));   // (not kept over the loop)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(uintptr_t)(stage + I * NW * 1024), 16, v, 0, 0, 0);
     }
-    // LDS address of the fragments of chunk CH (KMAJOR: of every MFMA tile; MNMAJOR: of tile CH, every chunk) of the stage at
-    // byte offset soff
-    template <int CH>
+    // LDS address of the fragments (KMAJOR: of chunk I, every MFMA tile; MNMAJOR: of tile I, every chunk) of the stage at byte
+    // offset soff.  256 rows: the first piece of a wavefront has no bits where those of its tiles differ.
+    template <int I>
     __device__ __forceinline__ uint32_t read_addr(uint32_t soff) const {
         uint32_t a;
-        if constexpr (MODE != KMAJOR) a = raddr[CH] + soff;
-        else if constexpr (CH < 3) asm volatile("v_xad_u32 %0, %1, %2, %3" : "=v"(a) : "v"(raddr[0]), "n"(CH << 5), "s"(soff));
-        else asm volatile("v_xor_b32 %0, 0x60, %1\n\tv_add_u32 %0, %2, %0" : "=&v"(a) : "v"(raddr[0]), "s"(soff));
+        if constexpr (NADDR > 1) a = raddr[I % NADDR] + soff;
+        else if constexpr (I == 0) a = raddr[0] + soff;
+        else if constexpr ((I << (MODE == KMAJOR ? 6 : 5)) <= 64) asm volatile("v_xad_u32 %0, %1, %2, %3" : "=v"(a) : "v"(raddr[0]), "n"(I << (MODE == KMAJOR ? 6 : 5)), "s"(soff));
+        else asm volatile("v_xor_b32 %0, %1, %2\n\tv_add_u32 %0, %3, %0" : "=&v"(a) : "n"(I << 5), "v"(raddr[0]), "s"(soff));
         return a;
     }
-    // fragment of MFMA tile TI, chunk CH
+    // fragment of MFMA tile TI, chunk CH (of 32 contraction elements)
     template <int CH, int TI>
     __device__ __forceinline__ static void read_one(GtFrag<bf16, MODE>& f, uint32_t addr) {
-        if constexpr (MODE == KMAJOR) f.template read<TI * 32 * BKB>(addr);
-        else f.template read<16 * CH * PITCH, PITCH>(addr);
+        if constexpr (MODE == KMAJOR) f.template read<TI * 16 * BKB>(addr);
+        else f.template read<32 * CH * PITCH + (NADDR > 1 ? TI / NADDR * 128 : 0), PITCH>(addr);
     }
     // KMAJOR: clears the elements of every row of a stage from contraction index `tail` to the end of their vector
     __device__ __forceinline__ static void clear_tail(char* __restrict__ stage, int tail, int tid) {
         if constexpr (MODE == KMAJOR) {
             if (tail % 8 == 0 || tid >= ROWS) return;
-            bf16* p = (bf16*)(stage + tid * BKB + (((tail / 8) ^ sw(tid)) << 4));
+            bf16* p = (bf16*)(stage + tid * BKB + (((tail / 8) ^ ring_sw(tid)) << 4));
             for (int e = tail % 8; e < 8; ++e) p[e] = from_f32<bf16>(0.f);
         }
     }
 };
 
-// lanes 32-63 of a <-> lanes 0-31 of b;  in each half, lanes 16-31 of a <-> lanes 0-15 of b
-__device__ __forceinline__ void ring_swap32(uint32_t& a, uint32_t& b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    a = r[0];
-    b = r[1];
-}
+// in each half of the wavefront, lanes 16-31 of a <-> lanes 0-15 of b
 __device__ __forceinline__ void ring_swap16(uint32_t& a, uint32_t& b) {
     const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
     a = r[0];
@@ -181,38 +188,37 @@ __device__ __forceinline__ uint32_t ring_pack2(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
 }
 
-// Write-back of a 32x32 accumulator tile.  acc[i] of lane (lr, lg) is row lr, column (i/4)*8 + lg*4 + i%4; d holds those values
-// rounded, two a word.  Afterwards lane l has in out[h] the eight columns (l>>4 & 1)*16 + (l>>5)*8 ... of row h*16 + (l & 15).
-__device__ __forceinline__ void ring_rows(uint32_t (&d)[8], gt_u32x4 (&out)[2]) {
-    ring_swap32(d[0], d[2]);
-    ring_swap32(d[1], d[3]);
-    ring_swap32(d[4], d[6]);
-    ring_swap32(d[5], d[7]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ring_swap16(d[i], d[4 + i]);
-    out[0] = gt_u32x4{d[0], d[1], d[2], d[3]};
-    out[1] = gt_u32x4{d[4], d[5], d[6], d[7]};
+// Write-back of two accumulator tiles side by side.  x[i], y[i] of lane l are row l & 15, columns (l >> 4) * 4 + i and 16 more.
+// Afterwards lane l has in `out` the eight columns (l>>4 & 1)*16 + (l>>5)*8 ... of that row, rounded.
+__device__ __forceinline__ gt_u32x4 ring_rows(const f32x4& x, const f32x4& y) {
+    uint32_t x0 = ring_pack2(x[0], x[1]), x1 = ring_pack2(x[2], x[3]), y0 = ring_pack2(y[0], y[1]), y1 = ring_pack2(y[2], y[3]);
+    ring_swap16(x0, y0);
+    ring_swap16(x1, y1);
+    return gt_u32x4{x0, x1, y0, y1};
 }
 
 // What becomes of an accumulator: RAW itself, GELU its GELU, BOTH the GELU's derivative as well (second output)
 enum { RING_RAW, RING_GELU, RING_BOTH };
 template <int ACT>
-__device__ __forceinline__ void ring_pack_tile(const f32x16& acc, gt_u32x4 (&out)[2], gt_u32x4 (&aux)[2]) {
-    uint32_t d[8], a[8];
+__device__ __forceinline__ void ring_pack_tile(const f32x4& x, const f32x4& y, gt_u32x4& out, gt_u32x4& aux) {
+    if constexpr (ACT == RING_RAW) {
+        out = ring_rows(x, y);
+    } else {
+        f32x4 a[2] = {x, y}, d[2];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        float x = acc[2 * i], y = acc[2 * i + 1];
-        if constexpr (ACT == RING_GELU) { x = gelu_f(x); y = gelu_f(y); }
-        if constexpr (ACT == RING_BOTH) {
-            float dx, dy;
-            gelu_both_f(acc[2 * i], x, dx);
-            gelu_both_f(acc[2 * i + 1], y, dy);
-            a[i] = ring_pack2(dx, dy);
-        }
-        d[i] = ring_pack2(x, y);
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v = a[t][e];
+                float g, dg;
+                if constexpr (ACT == RING_GELU) g = gelu_f(v);
+                else gelu_both_f(v, g, dg);
+                a[t][e] = g;
+                if constexpr (ACT == RING_BOTH) d[t][e] = dg;
+            }
+        out = ring_rows(a[0], a[1]);
+        if constexpr (ACT == RING_BOTH) aux = ring_rows(d[0], d[1]);
     }
-    ring_rows(d, out);
-    if constexpr (ACT == RING_BOTH) ring_rows(a, aux);
 }
 
 // Memory behind a pointer that came through ring_args: the compiler cannot tell that it is global, and an access that might
@@ -267,7 +273,7 @@ __device__ __forceinline__ void ring_store(__attribute__((address_space(1))) bf1
 // The wavefront's block at (row0, col0) as ACT of the accumulators, to c (and aux).  Addresses are a wave-uniform part and one
 // offset per lane, 32 bits wide in whole blocks, formed here (fresh_tid) so that they hold no registers through the main loop.
 template <typename C, int ACT>
-__device__ __forceinline__ void ring_write(const GemmArgs& g, const f32x16 (&acc)[C::TNW][C::TMW], bf16* c, int64_t rs, bf16* aux,
+__device__ __forceinline__ void ring_write(const GemmArgs& g, const f32x4 (&acc)[C::TN][C::TM], bf16* c, int64_t rs, bf16* aux,
                                            int64_t aux_rs, int row0, int col0) {
     const int lane = fresh_tid() & 63, lrow = lane & 15, lcol = ((lane >> 4) & 1) * 16 + (lane >> 5) * 8;
     RingRows cr(c + (int64_t)row0 * rs + col0, rs, 2), ar(aux + (int64_t)row0 * aux_rs + col0, aux_rs, 2);
@@ -280,7 +286,8 @@ __device__ __forceinline__ void ring_write(const GemmArgs& g, const f32x16 (&acc
 #pragma unroll
         for (int tn = 0; tn < C::TNW; ++tn) {
             gt_u32x4 v[2], w[2];
-            ring_pack_tile<ACT>(acc[tn][tm], v, w);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) ring_pack_tile<ACT>(acc[2 * tn][2 * tm + h], acc[2 * tn + 1][2 * tm + h], v[h], w[h]);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 if (whole) {
@@ -304,47 +311,37 @@ __device__ __forceinline__ void ring_write(const GemmArgs& g, const f32x16 (&acc
 // columns of row h*16 + (l & 15) per lane and store.  (rs is a tile's width or that of an output of fewer than 2 num_cus
 // tiles, the only ones that are K-split: 32-bit offsets.)
 template <typename C>
-__device__ __forceinline__ void ring_write_partial(const f32x16 (&acc)[C::TNW][C::TMW], float* __restrict__ dst, int64_t rs, int row0,
+__device__ __forceinline__ void ring_write_partial(const f32x4 (&acc)[C::TN][C::TM], float* __restrict__ dst, int64_t rs, int row0,
                                                    int col0, int nrows, int ncols) {
-    const int lane = fresh_tid() & 63, lrow = lane & 15, lcol = ((lane >> 4) & 1) * 8 + (lane >> 5) * 4;
+    const int lane = fresh_tid() & 63, lrow = lane & 15, lcol = (lane >> 4) * 4;
     RingRows pr(dst + (int64_t)row0 * rs + col0, rs, 4);
     const uint32_t voff = ((uint32_t)lrow * (uint32_t)rs + (uint32_t)lcol) * 4u;
     const bool whole = rs % 4 == 0 && row0 + C::TMW * 32 <= nrows && col0 + C::TNW * 32 <= ncols;
 #pragma unroll
     for (int tm = 0; tm < C::TMW; ++tm) {
 #pragma unroll
-        for (int tn = 0; tn < C::TNW; ++tn)
+        for (int tn = 0; tn < C::TN; ++tn)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                uint32_t x[4], y[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    x[e] = __float_as_uint(acc[tn][tm][q * 8 + e]);
-                    y[e] = __float_as_uint(acc[tn][tm][q * 8 + 4 + e]);
-                    ring_swap16(x[e], y[e]);
-                }
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const uint32_t* s = h ? y : x;
-                    if (whole) {
-                        *pr.at<gt_u32x4>(h, (tn * 32 + q * 16) * 4, voff) = gt_u32x4{s[0], s[1], s[2], s[3]};
-                    } else {
-                        int ne = ncols - col0 - lcol;
-                        asm volatile("" : "+v"(ne));
-                        ne = row0 + tm * 32 + h * 16 + lrow < nrows ? ne - (tn * 32 + q * 16) : 0;
+            for (int h = 0; h < 2; ++h) {
+                const f32x4& x = acc[tn][2 * tm + h];
+                if (whole) {
+                    *pr.at<f32x4>(h, tn * 64, voff) = x;
+                } else {
+                    int ne = ncols - col0 - lcol;
+                    asm volatile("" : "+v"(ne));
+                    ne = row0 + tm * 32 + h * 16 + lrow < nrows ? ne - tn * 16 : 0;
 #pragma unroll 1
-                        for (int e = 0; e < (ne < 4 ? ne : 4); ++e)
-                            pr.at<float>(h, (tn * 32 + q * 16) * 4, voff)[e] = __uint_as_float(e < 2 ? (e < 1 ? s[0] : s[1]) : (e < 3 ? s[2] : s[3]));
-                    }
+                    for (int e = 0; e < (ne < 4 ? ne : 4); ++e) pr.at<float>(h, tn * 64, voff)[e] = e < 2 ? (e < 1 ? x[0] : x[1]) : (e < 3 ? x[2] : x[3]);
                 }
-            }        pr.next();
+            }
+        pr.next();
     }
 }
 
-// C = round(acc) * mul and the column sums of what is stored over the wavefront's TMW * 32 rows (g.colpart).  The
-// multipliers of a row of MFMA tiles are requested while the one before it is multiplied.
+// C = round(acc) * mul and the column sums of what is stored over the wavefront's TMW * 32 rows (g.colpart).  The multipliers of two
+// rows of MFMA tiles are under way (three: 108.2 us instead of 107.6 for 16384x3072x768; four spill).
 template <typename C>
-__device__ __forceinline__ void ring_write_mul(const GemmArgs& g, const f32x16 (&acc)[C::TNW][C::TMW], int row0, int col0) {
+__device__ __forceinline__ void ring_write_mul(const GemmArgs& g, const f32x4 (&acc)[C::TN][C::TM], int row0, int col0) {
     constexpr int TMW = C::TMW, TNW = C::TNW;
     const int lane = fresh_tid() & 63, lrow = lane & 15, lcol = ((lane >> 4) & 1) * 16 + (lane >> 5) * 8;
     const int64_t mul_rs = g.mul_rs, c_rs = g.c_rs;
@@ -358,13 +355,14 @@ __device__ __forceinline__ void ring_write_mul(const GemmArgs& g, const f32x16 (
     for (int tn = 0; tn < TNW; ++tn)
 #pragma unroll
         for (int e = 0; e < 8; ++e) cs[tn][e] = 0.f;
-    gt_u32x4 mv[2][TNW][2];
+    constexpr int AHEAD = 2;
+    gt_u32x4 mv[AHEAD][TNW][2];
     auto request = [&](auto tm) __attribute__((always_inline)) {
         if (whole) {
 #pragma unroll
             for (int tn = 0; tn < TNW; ++tn)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) mv[tm & 1][tn][h] = *mr.at<gt_u32x4>(h, tn * 64, moff);
+                for (int h = 0; h < 2; ++h) mv[tm % AHEAD][tn][h] = *mr.at<gt_u32x4>(h, tn * 64, moff);
         } else {
 #pragma unroll
             for (int tn = 0; tn < TNW; ++tn)
@@ -386,23 +384,20 @@ __device__ __forceinline__ void ring_write_mul(const GemmArgs& g, const f32x16 (
                             for (int i = 0; i < 4; ++i) w[i] |= i == e >> 1 ? x : 0u;
                         }
                     }
-                    mv[tm & 1][tn][h] = gt_u32x4{w[0], w[1], w[2], w[3]};
+                    mv[tm % AHEAD][tn][h] = gt_u32x4{w[0], w[1], w[2], w[3]};
                 }
         }
         mr.next();
     };
-    request(std::integral_constant<int, 0>{});
+    gt_unroll<0, AHEAD>([&](auto tm) __attribute__((always_inline)) { request(tm); });
+    __builtin_amdgcn_sched_barrier(0);
     gt_unroll<0, TMW>([&](auto tm) __attribute__((always_inline)) {
-        if constexpr (tm + 1 < TMW) request(std::integral_constant<int, tm + 1>{});
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int tn = 0; tn < TNW; ++tn) {
-            gt_u32x4 v[2], none[2];
-            ring_pack_tile<RING_RAW>(acc[tn][tm], v, none);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                Pack<bf16, 8> s = __builtin_bit_cast(Pack<bf16, 8>, v[h]);
-                const Pack<bf16, 8> m = __builtin_bit_cast(Pack<bf16, 8>, mv[tm & 1][tn][h]);
+                Pack<bf16, 8> s = __builtin_bit_cast(Pack<bf16, 8>, ring_rows(acc[2 * tn][2 * tm + h], acc[2 * tn + 1][2 * tm + h]));
+                const Pack<bf16, 8> m = __builtin_bit_cast(Pack<bf16, 8>, mv[tm % AHEAD][tn][h]);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) s.v[e] = from_f32<bf16>(to_f32(s.v[e]) * to_f32(m.v[e]));
                 if (whole) {
@@ -426,6 +421,7 @@ __device__ __forceinline__ void ring_write_mul(const GemmArgs& g, const f32x16 (
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if constexpr (tm + AHEAD < TMW) request(std::integral_constant<int, tm + AHEAD>{});
         cr.next();
         __builtin_amdgcn_sched_barrier(0);
     });
@@ -446,14 +442,14 @@ __device__ __forceinline__ void ring_write_mul(const GemmArgs& g, const f32x16 (
         }
 }
 
-// The bias of the lane's columns in the layout of the accumulators (ring_pack_tile)
+// The bias of the lane's columns in the layout of the accumulators (ring_rows)
 template <typename C>
-__device__ __forceinline__ void ring_load_bias(const GemmArgs& g, Pack<bf16, 4> (&b)[C::TNW * 4], int col0) {
+__device__ __forceinline__ void ring_load_bias(const GemmArgs& g, Pack<bf16, 4> (&b)[C::TN], int col0) {
     const int lane = fresh_tid() & 63;
     const __attribute__((address_space(1))) bf16* bias = (const __attribute__((address_space(1))) bf16*)g.bias;
 #pragma unroll
-    for (int q = 0; q < C::TNW * 4; ++q) {
-        const int c = col0 + q * 8 + (lane >> 5) * 4;
+    for (int q = 0; q < C::TN; ++q) {
+        const int c = col0 + q * 16 + (lane >> 4) * 4;
         if (g.vec_out && col0 + C::TNW * 32 <= g.m) {
             b[q] = __builtin_bit_cast(Pack<bf16, 4>, *(const __attribute__((address_space(1))) gt_u32x2*)(bias + c));
         } else {
@@ -464,30 +460,28 @@ __device__ __forceinline__ void ring_load_bias(const GemmArgs& g, Pack<bf16, 4> 
 }
 // PTJ_EPI_ACCUMULATE: the accumulators start from the stored C; elements outside C start from zero, their results are never stored
 template <typename C>
-__device__ __forceinline__ void ring_load_c(const GemmArgs& g, f32x16 (&acc)[C::TNW][C::TMW], int row0, int col0) {
+__device__ __forceinline__ void ring_load_c(const GemmArgs& g, f32x4 (&acc)[C::TN][C::TM], int row0, int col0) {
     const int lane = fresh_tid() & 63;
-    const int r0 = row0 + (lane & 31), c0 = col0 + (lane >> 5) * 4;
+    const int r0 = row0 + (lane & 15), c0 = col0 + (lane >> 4) * 4;
 #pragma unroll
-    for (int tn = 0; tn < C::TNW; ++tn)
+    for (int tn = 0; tn < C::TN; ++tn)
 #pragma unroll
-        for (int tm = 0; tm < C::TMW; ++tm)
+        for (int tm = 0; tm < C::TM; ++tm) {
+            const int row = r0 + tm * 16, col = c0 + tn * 16;
+            const auto* p = (const __attribute__((address_space(1))) bf16*)g.c + (int64_t)row * g.c_rs + col;
+            Pack<bf16, 4> v;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int row = r0 + tm * 32, col = c0 + tn * 32 + q * 8;
-                const auto* p = (const __attribute__((address_space(1))) bf16*)g.c + (int64_t)row * g.c_rs + col;
-                Pack<bf16, 4> v;
+            for (int e = 0; e < 4; ++e) v.v[e] = from_f32<bf16>(0.f);
+            if (row < g.n && col + 4 <= g.m) {
+                v = __builtin_bit_cast(Pack<bf16, 4>, *(const __attribute__((address_space(1))) gt_u32x2*)p);
+            } else if (row < g.n) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v.v[e] = from_f32<bf16>(0.f);
-                if (row < g.n && col + 4 <= g.m) {
-                    v = __builtin_bit_cast(Pack<bf16, 4>, *(const __attribute__((address_space(1))) gt_u32x2*)p);
-                } else if (row < g.n) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (col + e < g.m) v.v[e] = p[e];
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[tn][tm][q * 4 + e] = to_f32(v.v[e]);
+                for (int e = 0; e < 4; ++e)
+                    if (col + e < g.m) v.v[e] = p[e];
             }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[tn][tm][e] = to_f32(v.v[e]);
+        }
 }
 
 // The kernel's arguments, read again from where the launch left them: what only the start and the end of a tile need holds
@@ -503,7 +497,7 @@ constexpr int clip(int x, int most) { return x < most ? x : most; }
 
 template <int AMODE, int BMODE, typename C, bool MUL>
 __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs) {
-    constexpr int TMW = C::TMW, TNW = C::TNW, NA = C::NA, NB = C::NB;
+    constexpr int TMW = C::TMW, TNW = C::TNW, TM = C::TM, TN = C::TN, NA = C::NA, NB = C::NB;
     __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -513,8 +507,8 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
     char* const ring_a = smem;
     char* const ring_b = smem + NA * C::A_STAGE;
 
-    typedef RingOperand<AMODE, C::TBM, TMW, NA> OA;
-    typedef RingOperand<BMODE, C::TBN, TNW, NB> OB;
+    typedef RingOperand<AMODE, C::TBM, TM, NA> OA;
+    typedef RingOperand<BMODE, C::TBN, TN, NB> OB;
     constexpr int PA = OA::PER, PB = OB::PER;
     OA oa;
     OB ob;
@@ -576,49 +570,46 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
         }
     };
 
-    // two register sets of two contraction chunks each
-    GtFrag<bf16, AMODE> fa[2][2][TMW];
-    GtFrag<bf16, BMODE> fb[2][2][TNW];
-    f32x16 acc[TNW][TMW];
-    constexpr int NR = 2 * (TMW + TNW), NM = 2 * TMW * TNW, NC = PA + PB;   // reads, MFMAs of a set; copies of a step
-    // Reads end a little before the set's last MFMA, so that they have landed by then, and copies two MFMAs earlier, so that the
+    // two register sets of one contraction chunk each
+    GtFrag<bf16, AMODE> fa[2][TM];
+    GtFrag<bf16, BMODE> fb[2][TN];
+    f32x4 acc[TN][TM];
+    constexpr int NR = TM + TN, NM = TM * TN, NC = PA + PB;   // reads, MFMAs of a set; copies of a step
+    // Reads end a little before the set's last MFMA, so that they have landed by then, and copies a little earlier, so that the
     // cursors' bookkeeping runs under the last ones and not beside the barrier (8192^3: 783 us, 824 without).
-    constexpr int READ_SPAN = NM * 7 / 8, COPY_SPAN = NM - 2;
-    uint32_t addr_a[AMODE == KMAJOR ? 2 : TMW], addr_b[BMODE == KMAJOR ? 2 : TNW];
-    auto read_addresses = [&](auto first, uint32_t soff_a, uint32_t soff_b) __attribute__((always_inline)) {
-        gt_unroll<0, (AMODE == KMAJOR ? 2 : TMW)>([&](auto i) __attribute__((always_inline)) {
-            addr_a[i] = oa.template read_addr<(AMODE == KMAJOR ? first + i : i)>(soff_a);
-        });
-        gt_unroll<0, (BMODE == KMAJOR ? 2 : TNW)>([&](auto i) __attribute__((always_inline)) {
-            addr_b[i] = ob.template read_addr<(BMODE == KMAJOR ? first + i : i)>(soff_b);
-        });
+    constexpr int READ_SPAN = NM * 5 / 8, COPY_SPAN = NM - 4;
+    uint32_t addr_a, addr_b;                   // KMAJOR
+    auto read_addresses = [&](auto ch, uint32_t soff_a, uint32_t soff_b) __attribute__((always_inline)) {
+        if constexpr (AMODE == KMAJOR) addr_a = oa.template read_addr<ch>(soff_a);
+        if constexpr (BMODE == KMAJOR) addr_b = ob.template read_addr<ch>(soff_b);
     };
-    auto read_piece = [&](auto set, auto first, auto i) __attribute__((always_inline)) {
-        constexpr int c = i / (TMW + TNW), t = i % (TMW + TNW);
-        if constexpr (t < TMW) OA::template read_one<first + c, t>(fa[set][c][t], addr_a[AMODE == KMAJOR ? c : t]);
-        else OB::template read_one<first + c, t - TMW>(fb[set][c][t - TMW], addr_b[BMODE == KMAJOR ? c : t - TMW]);
+    auto read_piece = [&](auto set, auto ch, auto i, uint32_t soff_a, uint32_t soff_b) __attribute__((always_inline)) {
+        if constexpr (i < TM) {
+            if constexpr (AMODE != KMAJOR) addr_a = oa.template read_addr<i>(soff_a);
+            OA::template read_one<ch, i>(fa[set][i], addr_a);
+        } else {
+            if constexpr (BMODE != KMAJOR) addr_b = ob.template read_addr<i - TM>(soff_b);
+            OB::template read_one<ch, i - TM>(fb[set][i - TM], addr_b);
+        }
     };
     auto landed = [&](auto set) __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
+        for (int t = 0; t < TM; ++t) fa[set][t].landed();
 #pragma unroll
-            for (int t = 0; t < TMW; ++t) fa[set][c][t].landed();
-#pragma unroll
-            for (int t = 0; t < TNW; ++t) fb[set][c][t].landed();
-        }
+        for (int t = 0; t < TN; ++t) fb[set][t].landed();
     };
     uint32_t sa = 0, sb = 0;                   // offsets of the stages that hold the step being multiplied
-    // the MFMAs of register set `set`, with the reads of chunks first, first + 1 into the other one between them, and with
+    // the MFMAs of register set `set`, with the reads of chunk `ch` into the other one between them, and with
     // `copies` those of a stage of either operand
-    auto phase = [&](auto set, auto first, auto copies, uint32_t soff_a, uint32_t soff_b) __attribute__((always_inline)) {
+    auto phase = [&](auto set, auto ch, auto copies, uint32_t soff_a, uint32_t soff_b) __attribute__((always_inline)) {
         constexpr std::integral_constant<int, 1 - set> OTHER{};
-        read_addresses(first, soff_a, soff_b);
+        read_addresses(ch, soff_a, soff_b);
+        __builtin_amdgcn_s_setprio(set);
         gt_unroll<0, NM>([&](auto j) __attribute__((always_inline)) {
-            constexpr int c = j / (TMW * TNW), tn = j / TMW % TNW, tm = j % TMW;
-            mma_chunk(acc[tn][tm], fb[set][c][tn].get(), fa[set][c][tm].get());
-            __builtin_amdgcn_sched_barrier(0);
+            constexpr int tn = j / TM, tm = j % TM;
+            acc[tn][tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[set][tn].get(), fa[set][tm].get(), acc[tn][tm], 0, 0, 0);
             gt_unroll<clip(j * NR / READ_SPAN, NR), clip((j + 1) * NR / READ_SPAN, NR)>(
-                [&](auto i) __attribute__((always_inline)) { read_piece(OTHER, first, i); });
+                [&](auto i) __attribute__((always_inline)) { read_piece(OTHER, ch, i, soff_a, soff_b); });
             if constexpr (copies)
                 gt_unroll<clip(j * NC / COPY_SPAN, NC), clip((j + 1) * NC / COPY_SPAN, NC)>([&](auto i) __attribute__((always_inline)) {
                     if constexpr (i < PB) copy_b(std::integral_constant<int, i>{});
@@ -633,7 +624,6 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
     };
     constexpr std::integral_constant<int, 0> I0{};
     constexpr std::integral_constant<int, 1> I1{};
-    constexpr std::integral_constant<int, 2> I2{};
     constexpr std::bool_constant<true> YES{};
     constexpr std::bool_constant<false> NO{};
     auto clear_tails = [&](int klen) __attribute__((always_inline)) {
@@ -644,7 +634,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
     };
 
     // the accumulators of a tile start from the bias, requested before the write-back of the tile before it
-    Pack<bf16, 4> bias[TNW * 4];
+    Pack<bf16, 4> bias[TN];
     auto load_bias = [&](const RingItem& it) __attribute__((always_inline)) {
         if constexpr (!MUL) {
             const GemmArgs& g = ring_args();
@@ -654,7 +644,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
             }
         }
 #pragma unroll
-        for (int q = 0; q < TNW * 4; ++q)
+        for (int q = 0; q < TN; ++q)
 #pragma unroll
             for (int e = 0; e < 4; ++e) bias[q].v[e] = from_f32<bf16>(0.f);
     };
@@ -667,16 +657,16 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NA - 1) * PA + (NB - 1) * PB) : "memory");
     if (ragged && cur.klen <= 64) clear_tails(cur.klen);
     read_addresses(I0, 0u, 0u);
-    gt_unroll<0, NR>([&](auto i) __attribute__((always_inline)) { read_piece(I0, I0, i); });
+    gt_unroll<0, NR>([&](auto i) __attribute__((always_inline)) { read_piece(I0, I0, i, 0u, 0u); });
     for (;;) {
         const int nitem = item + (int)gridDim.x;
         const bool more = nitem < work;
 #pragma unroll
-        for (int i = 0; i < TNW; ++i)
+        for (int i = 0; i < TN; ++i)
 #pragma unroll
-            for (int j = 0; j < TMW; ++j)
+            for (int j = 0; j < TM; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[i][j][e] = to_f32(bias[i * 4 + (e >> 2)].v[e & 3]);
+                for (int e = 0; e < 4; ++e) acc[i][j][e] = to_f32(bias[i].v[e]);
         if constexpr (!MUL) {
             const GemmArgs& g = ring_args();
             if (g.epilogue == PTJ_EPI_ACCUMULATE) ring_load_c<C>(g, acc, cur.row0 + wm * TMW * 32, cur.col0 + wn * TNW * 32);
@@ -684,7 +674,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
         for (int kt = 0; kt < cur.klen; kt += 64) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             landed(I0);
-            phase(I0, I2, NO, sa, sb);
+            phase(I0, I1, NO, sa, sb);
             // This wavefront has read all of the stage and its copies of the next one have landed (younger: A's of the one
             // after it); after the barrier that holds for every wavefront, so the next stage may be read and this one refilled.
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NA - 2) * PA) : "memory");
@@ -731,7 +721,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
         // the multiplying write-back takes the registers of the next tile's first fragments, which are read again here
         if constexpr (MUL) {
             read_addresses(I0, sa, sb);
-            gt_unroll<0, NR>([&](auto i) __attribute__((always_inline)) { read_piece(I0, I0, i); });
+            gt_unroll<0, NR>([&](auto i) __attribute__((always_inline)) { read_piece(I0, I0, i, sa, sb); });
         }
     }
     // nothing of this workgroup may still be on its way into LDS when its wavefronts end
