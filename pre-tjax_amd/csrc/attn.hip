@@ -256,16 +256,18 @@ template <bool HALVES> __device__ __forceinline__ KeepWords load_keep(const uint
     else return load_keep_words(line, base);
 }
 
-// Which tile and batch-head a workgroup of a grid (B*H, tiles) takes.  In dispatch order tiles go from long to short; every
-// second layer of 256 workgroups (one per CU) runs backwards, so that the CU with the longest of one layer gets the shortest of
-// the next instead of the longest again.  Only whole layers are turned, and a workgroup keeps its number modulo 8, hence its
-// XCD and the K and V in that one's L2.  Batch 8 x 1024 x 12 heads (three layers): forward 25.9 -> 24.6 us, dQ 35.2 -> 33.3;
-// 16 x 1024 (six layers): dQ 61.0 -> 59.0, dK/dV 86.3 -> 85.1, forward within its spread (43.9, 45.2).
+// Which tile and batch-head a workgroup of a grid (B*H, tiles) takes.  In dispatch order tiles go from long to short; the
+// second layer of 256 workgroups (one per CU) runs backwards, so that the CU with the longest of the first gets the shortest of
+// the next instead of the longest again.  Only a whole layer is turned, and a workgroup keeps its number modulo 8, hence its
+// XCD and the K and V in that one's L2.  Batch 8 x 1024 x 12 heads (three layers): forward 25.9 -> 24.6 us, dQ 35.2 -> 33.3.
+// Two or three layers are there at once; later ones go to the CUs that are free first, the longest first: turned as well, the
+// last workgroups to start were not the shortest ones, and 16 x 1024 (six layers) took 43.9 us forward, now 41.9 (50.6 -> 48.0
+// with dropout).
 struct Place { int tile, bh; };
 __device__ __forceinline__ Place place() {
     const uint32_t total = gridDim.x * gridDim.y;
     uint32_t id = blockIdx.y * gridDim.x + blockIdx.x;
-    if ((id & 256) && (id | 255) < total) id ^= 31 << 3;
+    if (id >> 8 == 1 && (id | 255) < total) id ^= 31 << 3;
     return {(int)(id / gridDim.x), (int)(id % gridDim.x)};
 }
 
