@@ -465,21 +465,39 @@ __device__ __forceinline__ void gemm_store_block(const GemmArgs& g, const f32x16
     }
 }
 
-// Work item -> origin of its C tile: ids are regrouped so that the items of one XCD (id mod
-// 8) cover a contiguous range of tiles, then walked in groups of 8 tile-rows.
-template <int TBN = BN>
-__device__ __forceinline__ void tile_origin(int pid, int total, int num_m, int num_n, int& row0, int& col0) {
-    {
-        const int chunk = total >> 3, rem = total & 7, x = pid & 7;
-        pid = x * chunk + (x < rem ? x : rem) + (pid >> 3);
+// The walk over the tiles of C.  Ids are regrouped so that each XCD (id mod 8) works on a contiguous range of it, and the tiles
+// lie in groups of tile rows, column by column inside a group.  RING, the walk of gemm_ring.h's large tiles: groups of four rows
+// instead of eight, and XCD x begins x eighths into its range.  32 tiles of an XCD are under way at once; eight columns of four rows
+// make longer pieces of an output row than four columns of eight, and the XCDs, whose ranges are often whole groups, no longer write the same
+// columns at the same time.  Eight rows, all from the start / four, spread, us on one box: 16384x3072x768 with GELU and its
+// derivative 114.3 / 102.3, with bias 80.7 / 77.6, 16384x2304x768 63.5 / 62.5, 8192x2304x768 38.7 / 36.9, 8192x50257x768
+// 634 / 567 (its two gradient products 498 / 501 and 532 / 518).  Eight rows, spread: 103.0, 76.8, 62.1, 36.7, 632; five, spread: 102.4, 78.9, 62.6,
+// 37.0, 638.  Tiles of 128 x 128, which are seldom more than one round: no difference beyond 1 %, they keep eight.
+template <bool RING>
+__device__ __forceinline__ int xcd_range(int pid, int work) {
+    const int chunk = work >> 3, rem = work & 7, x = pid & 7, len = chunk + (x < rem);
+    int at = pid >> 3;
+    if constexpr (RING) {
+        at += (int)((int64_t)len * x >> 3);
+        if (at >= len) at -= len;
     }
-    constexpr int GROUP = 8;
+    return x * chunk + (x < rem ? x : rem) + at;
+}
+template <bool RING>
+__device__ __forceinline__ void tile_walk(int idx, int num_m, int num_n, int& tile_m, int& tile_n) {
+    constexpr int GROUP = RING ? 4 : 8;
     const int width = GROUP * num_n;
-    const int group_id = pid / width;
+    const int group_id = idx / width;
     const int first_m = group_id * GROUP;
     const int gsz = (num_m - first_m) < GROUP ? (num_m - first_m) : GROUP;
-    const int tile_m = first_m + (pid % width) % gsz;
-    const int tile_n = (pid % width) / gsz;
+    tile_m = first_m + (idx % width) % gsz;
+    tile_n = (idx % width) / gsz;
+}
+// Work item -> origin of its C tile (tile_walk).  RING: of gemm_ring.h's walk.
+template <int TBN = BN, bool RING = false>
+__device__ __forceinline__ void tile_origin(int pid, int total, int num_m, int num_n, int& row0, int& col0) {
+    int tile_m, tile_n;
+    tile_walk<RING>(xcd_range<RING>(pid, total), num_m, num_n, tile_m, tile_n);
     row0 = tile_m * BM;
     col0 = tile_n * TBN;
 }
@@ -810,12 +828,12 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce4_kernel(const float* _
 
 // Second stage for the K-split tiles of the last round: tile t (work item tail_first + t) =
 // epilogue(sum_z partial[t*splits + z]) in z order; partial tiles are dense BM x TBN.
-template <typename T, int TBN>
+template <typename T, int TBN, bool RING>
 __global__ __launch_bounds__(256) void gemm_tail_reduce_kernel(const GemmArgs g) {
     const int num_m = (g.n + BM - 1) / BM, num_n = (g.m + TBN - 1) / TBN;
     const int t = blockIdx.x;
     int row0, col0;
-    tile_origin<TBN>(g.tail_first + t, num_m * num_n, num_m, num_n, row0, col0);
+    tile_origin<TBN, RING>(g.tail_first + t, num_m * num_n, num_m, num_n, row0, col0);
     const float* base = g.partial + (int64_t)t * g.tail_splits * (BM * TBN);
     // four consecutive columns per thread: 16-byte loads of the partial tiles; a quad that lies
     // wholly inside C is stored as one vector when the outputs allow it
@@ -874,9 +892,9 @@ int launch_splitk_reduce(const GemmArgs& g, int splits, hipStream_t st) {
     return PTJ_OK;
 }
 
-template <typename T, int TBN>
+template <typename T, int TBN, bool RING = false>
 int launch_tail_reduce(const GemmArgs& g, int tiles, hipStream_t st) {
-    hipLaunchKernelGGL((gemm_tail_reduce_kernel<T, TBN>), dim3((unsigned)(tiles - g.tail_first), 12), dim3(256), 0, st, g);
+    hipLaunchKernelGGL((gemm_tail_reduce_kernel<T, TBN, RING>), dim3((unsigned)(tiles - g.tail_first), 12), dim3(256), 0, st, g);
     PTJ_CHECK_LAUNCH();
     return PTJ_OK;
 }

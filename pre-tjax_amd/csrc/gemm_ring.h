@@ -52,12 +52,12 @@ __device__ __forceinline__ RingItem ring_item(const GemmArgs& g, int item) {
     d.part = nullptr;
     if (g.tail_splits > 1 && item >= g.tail_first) {
         const int r = item - g.tail_first, t = r / g.tail_splits;
-        gt_item(g, g.tail_first + t, num_m, num_n, tm, tn, d.z);
+        gt_item<true>(g, g.tail_first + t, num_m, num_n, tm, tn, d.z);
         d.z = r - t * g.tail_splits;
         kps = g.tail_kps;
         d.part = g.partial + (int64_t)r * (C::TBM * C::TBN);
     } else {
-        gt_item(g, item, num_m, num_n, tm, tn, d.z);
+        gt_item<true>(g, item, num_m, num_n, tm, tn, d.z);
     }
     d.row0 = tm * C::TBM;
     d.col0 = tn * C::TBN;
@@ -759,7 +759,7 @@ int ring_launch(const GemmArgs& g, int am, int bm, hipStream_t st) {
     PTJ_CHECK_LAUNCH();
     if constexpr (!MUL) {
         if (g.splits > 1 && !g.leave_partials) return launch_splitk_reduce<bf16>(g, g.splits, st);
-        if (g.tail_splits > 1) return launch_tail_reduce<bf16, C::TBN>(g, (int)total, st);
+        if (g.tail_splits > 1) return launch_tail_reduce<bf16, C::TBN, true>(g, (int)total, st);
     }
     return PTJ_OK;
 }

@@ -197,15 +197,14 @@ struct GtCfg {
     static constexpr int WAVES_EU = (BLOCKS * NW + 3) / 4;
 };
 
-// Work item of the grid -> tile and K split.  As in gemm_core.h: ids are regrouped so that each XCD (id mod 8) works
-// on a contiguous range; without a K split tiles are walked in groups of 8 tile rows, with one the tiles along the
-// smaller C dimension vary fastest, then the other ones, then the split.
+// Work item of the grid -> tile and K split.  Without a K split as in gemm_core.h (tile_walk); with one each XCD works on a
+// contiguous range as well, and the tiles along the smaller C dimension vary fastest, then the other ones, then the split.
+template <bool RING = false>
 __device__ __forceinline__ void gt_item(const GemmArgs& g, int pid, int num_m, int num_n, int& tile_m, int& tile_n, int& z) {
-    const int total = num_m * num_n, work = total * g.splits;
-    const int chunk = work >> 3, rem = work & 7, x = pid & 7;
-    const int idx = x * chunk + (x < rem ? x : rem) + (pid >> 3);
+    const int total = num_m * num_n;
     z = 0;
     if (g.splits > 1) {
+        const int idx = xcd_range<false>(pid, total * g.splits);
         if (g.n >= g.m) {
             tile_n = idx % num_n;
             const int pair = idx / num_n;
@@ -219,13 +218,7 @@ __device__ __forceinline__ void gt_item(const GemmArgs& g, int pid, int num_m, i
         }
         return;
     }
-    constexpr int GROUP = 8;
-    const int width = GROUP * num_n;
-    const int group_id = idx / width;
-    const int first_m = group_id * GROUP;
-    const int gsz = (num_m - first_m) < GROUP ? (num_m - first_m) : GROUP;
-    tile_m = first_m + (idx % width) % gsz;
-    tile_n = (idx % width) / gsz;
+    tile_walk<RING>(xcd_range<RING>(pid, total), num_m, num_n, tile_m, tile_n);
 }
 
 // Write-back of a finished tile: 32 rows at a time through an fp32 staging area per wavefront (the K groups'

@@ -56,6 +56,18 @@ def test_ring_shapes(mt, n, m, k, layout):
     assert (odd[:, 0] == 7.0).all() and (odd[:, m + 1:] == 7.0).all()
 
 
+# The walk over the tiles: every tile once where the tile rows are fewer than a group of four or leave a smaller last group, and the
+# XCDs' ranges have different lengths (3 x 197, 9 x 49 and 5 x 33 tiles of 256 x 256, more columns at 192)
+@pytest.mark.parametrize("n,m,k", [(700, 50257, 128), (2100, 12300, 128), (1100, 8200, 256)])
+def test_ring_walk(mt, n, m, k):
+    a, b, _ = operands(n, m, k, "nt")
+    out = torch.full((n, (m + 15) // 8 * 8), 7.0, dtype=BF16, device=DEV)
+    mt.matmul_t(padded(a, BF16), padded(b, BF16), out=out[:, :m])
+    want, scale = product(a, b)
+    assert ((f64(out[:, :m]) - want).abs() / gemm_bound(want, scale, BF16)).max().item() <= 1.0
+    assert (out[:, m:] == 7.0).all()
+
+
 # one shape for each kernel that forms the derivative: ring, tiles, K split, unaligned and strided operands, fp32 tiles, fp32 split
 # per tile and ahead
 @pytest.mark.parametrize("n,m,k,dtype,step", [(3001, 3080, 128, BF16, 1), (100, 776, 64, BF16, 1), (64, 768, 4096, BF16, 1),
