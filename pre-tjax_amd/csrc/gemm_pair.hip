@@ -2,8 +2,10 @@
 //
 // At a few hundred tokens each of the two takes 7-13 us, most of it the latency of a launch, of the first panels
 // (weights that the optimizer pass has pushed out of every cache) and of the write-back, on a quarter to a half of
-// the CUs.  Side by side they cost about what the longer one costs alone: the workgroups of dx come first in the
-// grid (the next step of the backward waits for it), those of dw behind them.
+// the CUs.  Side by side they cost about what the longer one costs alone.  At some thousand tokens they make between one and
+// three rounds of tiles, and share the rounds: the product whose tiles take longer comes first in the grid and the shorter
+// tiles of the other fill the CUs as they fall free (dx: m contraction elements a tile, dw: n).  With dx first, us, before / now:
+// 3136 tokens proj 23.1 / 19.7, 6000 tokens ffn2 with its multiplier 95.6 / 84.5, qkv 61.2 / 62.0 (as two launches 75.4).
 #include "gemm_core.h"
 #include "gemm_plan.h"
 #include "internal.h"
@@ -18,59 +20,96 @@ constexpr int max_int(int a, int b) { return a > b ? a : b; }
 
 template <typename CX, typename CW, bool MUL>
 __global__ __launch_bounds__(CX::THREADS, CX::WAVES_EU < CW::WAVES_EU ? CX::WAVES_EU : CW::WAVES_EU) void gemm_pair_kernel(
-    const GemmArgs gx, const GemmArgs gw, int nx) {
+    const GemmArgs gx, const GemmArgs gw, int nx, int nw, bool dw_first) {
     static_assert(CX::THREADS == CW::THREADS, "one workgroup size");
     __shared__ __attribute__((aligned(1024))) char smem[max_int(CX::SMEM, CW::SMEM)];
-    const int b = (int)blockIdx.x;
-    if (b < nx) gt_tile<bf16, KMAJOR, MNMAJOR, CX, MUL>(gx, b, smem);
-    else gt_tile<bf16, MNMAJOR, MNMAJOR, CW, false>(gw, b - nx, smem);
+    const int x = (int)blockIdx.x - (dw_first ? nw : 0), w = (int)blockIdx.x - (dw_first ? 0 : nx);
+    if (x >= 0 && x < nx) gt_tile<bf16, KMAJOR, MNMAJOR, CX, MUL>(gx, x, smem);
+    else gt_tile<bf16, MNMAJOR, MNMAJOR, CW, false>(gw, w, smem);
 }
 
 template <typename CX, typename CW>
-int launch_pair(const GemmArgs& gx, const GemmArgs& gw, bool mul, hipStream_t st) {
+int launch_pair(const GemmArgs& gx, const GemmArgs& gw, bool mul, bool dw_first, hipStream_t st) {
     const int nx = ((gx.n + CX::TBM - 1) / CX::TBM) * ((gx.m + CX::TBN - 1) / CX::TBN);
     const int nw = ((gw.n + CW::TBM - 1) / CW::TBM) * ((gw.m + CW::TBN - 1) / CW::TBN);
-    if (mul) hipLaunchKernelGGL((gemm_pair_kernel<CX, CW, true>), dim3(nx + nw), dim3(CX::THREADS), 0, st, gx, gw, nx);
-    else hipLaunchKernelGGL((gemm_pair_kernel<CX, CW, false>), dim3(nx + nw), dim3(CX::THREADS), 0, st, gx, gw, nx);
+    const dim3 grid(nx + nw), block(CX::THREADS);
+    if (mul) hipLaunchKernelGGL((gemm_pair_kernel<CX, CW, true>), grid, block, 0, st, gx, gw, nx, nw, dw_first);
+    else hipLaunchKernelGGL((gemm_pair_kernel<CX, CW, false>), grid, block, 0, st, gx, gw, nx, nw, dw_first);
     PTJ_CHECK_LAUNCH();
     return PTJ_OK;
 }
 
-// Estimated time of a pair with configurations ix, iw of the bf16 table: both resident at once -> the longer one; more
-// workgroups than slots -> the slots shared out over the work, plus half a workgroup of imbalance.
-double pair_us(const PtjLinearBwd& p, int ix, int iw, int cus) {
+// Time of n1 tiles of t1, then n2 of t2 <= t1, on `slots` workgroups that take the next tile as they end one.
+double pair_makespan(int64_t n1, double t1, int64_t n2, double t2, int64_t slots) {
+    const int64_t full = n1 / slots, rest = n1 % slots;
+    const double first = (double)(full + (rest > 0)) * t1;
+    auto holds = [&](double t) {          // tiles of t2 that end by t
+        const double late = t - (double)(full + 1) * t1, early = t - (double)full * t1;
+        return (double)rest * floor((late > 0 ? late : 0.0) / t2 + 1e-9) + (double)(slots - rest) * floor((early > 0 ? early : 0.0) / t2 + 1e-9);
+    };
+    if (holds(first) >= (double)n2) return first;
+    double lo = first, hi = first + (double)(n2 / slots + 2) * t2;
+    for (int i = 0; i < 30; ++i) {
+        const double mid = 0.5 * (lo + hi);
+        if (holds(mid) >= (double)n2) hi = mid;
+        else lo = mid;
+    }
+    return hi;
+}
+
+// Estimated time of a pair (us) with configurations ix, iw of the bf16 table.  Fitted to the pairs themselves: the four layers of a GPT-2
+// small block, every choice here and two launches (estimated by gemm_plan; SEPARATE and, with a multiplier, SEPARATE_MUL times
+// that), alone at 25 token counts from 256 to 16384 and inside a training step at 12.  The pick is 1.6 % slower than the
+// best of them on average; the estimates of gemm_plan, and dx always first, picked 7 % above it.  Training step, before / now, us:
+// 512 tokens 2690 / 2678, 1024 3785 / 3659, 2560 5376 / 5290, 3136 5804 / 5567, 3584 6599 / 6451, 6144 9925 / 9293, 12288 the same.
+struct PairCost { double step, finish, crowd, dw; };      // us; crowd: growth of a step from half the CUs busy to all; dw: its steps
+constexpr PairCost PAIR_COST[4] = {{}, {0.21, 1.75, 0.31, 0.88}, {0.19, 1.59, 0.49, 1.07}, {0.33, 3.52, 0.15, 0.97}};
+constexpr double PAIR_START = 3.2, PAIR_MUL = 0.48, PAIR_ROUNDS = 0.55, SEPARATE = 0.95, SEPARATE_MUL = 1.22;
+constexpr double PAIR_ALONE = 0.84;                       // wide tiles, one a CU because of the small ones beside them
+constexpr double PAIR_SHARED = 2.01, PAIR_FLOWS = 0.7;    // wide tiles, two a CU: where one ends early, the other goes on faster
+
+double pair_us(const PtjLinearBwd& p, int ix, int iw, int cus, bool* dw_first) {
     const TileCost &cx = GT_COST[0][ix], &cw = GT_COST[0][iw];
-    const int64_t nx = gp_ceil(p.n, cx.tbm) * gp_ceil(p.k, cx.tbn), nw = gp_ceil(p.m, cw.tbm) * gp_ceil(p.k, cw.tbn);
-    const int per_cu = cx.per_cu < cw.per_cu ? cx.per_cu : cw.per_cu;
-    const int64_t slots = (int64_t)cus * per_cu;
-    const bool packed = nx + nw > cus;                     // CUs with two workgroups: their steps take longer
-    const double tx = (double)gp_ceil(p.m, cx.bkt) * gp_step_us(cx, nx + nw, cus) * (packed ? cx.shared : 1.0) + cx.finish;
-    const double tw = (double)gp_ceil(p.n, cw.bkt) * gp_step_us(cw, nx + nw, cus) * (packed ? cw.shared : 1.0) + cw.finish;
-    const double start = cx.start > cw.start ? cx.start : cw.start, longest = tx > tw ? tx : tw;
-    if (nx + nw <= slots) return start + longest;
-    return start + ((double)nx * tx + (double)nw * tw) / (double)slots + 0.5 * longest;
+    const int64_t nx = gp_ceil(p.n, cx.tbm) * gp_ceil(p.k, cx.tbn), nw = gp_ceil(p.m, cw.tbm) * gp_ceil(p.k, cw.tbn), all = nx + nw;
+    const int64_t slots = (int64_t)cus * (cx.per_cu < cw.per_cu ? cx.per_cu : cw.per_cu);
+    const bool two = slots > cus;
+    const double busy = all < cus ? (double)all / (double)cus : 1.0, over = all > cus ? (double)(all - cus) / (double)cus : 0.0;
+    const double shared = two ? 1.0 + (PAIR_SHARED - 1.0) * (over < 1.0 ? over : 1.0) : 1.0;
+    auto tile = [&](int i, int64_t k, bool dw) {
+        const PairCost& c = PAIR_COST[i];
+        const double step = c.step * (1.0 + (busy > 0.5 ? c.crowd * 2.0 * (busy - 0.5) : 0.0)) * (dw ? c.dw : 1.0);
+        return (double)gp_ceil(k, GT_COST[0][i].bkt) * step * (i == 2 && !two ? PAIR_ALONE : shared) + c.finish;
+    };
+    const double tx = tile(ix, p.m, false) + (p.mul ? PAIR_MUL : 0.0), tw = tile(iw, p.n, true);
+    *dw_first = tw > tx;
+    if (all <= slots) return PAIR_START + (tw > tx ? tw : tx);
+    double t = tw > tx ? pair_makespan(nw, tw, nx, tx, slots) : pair_makespan(nx, tx, nw, tw, slots);
+    if (two) t += PAIR_FLOWS * (((double)nx * tx + (double)nw * tw) / (double)slots - t);
+    return (PAIR_START + t) * (1.0 + PAIR_ROUNDS * (1.0 - (double)slots / (double)all));
 }
 
 double single_us(int64_t n, int64_t m, int64_t k, bool may_split, int cus) {
     return gemm_plan(n, m, k, 2, may_split ? (size_t)-1 : 0, cus).us;
 }
 
-// 0: two launches; else 1 + 3 * ix + iw over {small, wide, square}
-int choose_pair(const PtjLinearBwd& p) {
-    struct Entry { int64_t n, m, k; int mul, cus, choice; };
+// config 0: two launches; else 1 + 3 * ix + iw over {small, wide, square}
+struct PairChoice { int config; bool dw_first; };
+PairChoice choose_pair(const PtjLinearBwd& p) {
+    struct Entry { int64_t n, m, k; int mul, cus; PairChoice choice; };
     static thread_local Entry table[32] = {};
     const int cus = num_cus(), mul = p.mul != nullptr;
     Entry& e = table[((uint64_t)p.n * 0x9E3779B97F4A7C15ull + (uint64_t)p.m * 0xC2B2AE3D27D4EB4Full + (uint64_t)p.k * 31 + mul) >> 40 & 31];
     if (e.n == p.n && e.m == p.m && e.k == p.k && e.mul == mul && e.cus == cus) return e.choice;
-    double best = 0.95 * (single_us(p.n, p.k, p.m, !mul, cus) + single_us(p.m, p.k, p.n, true, cus));
-    int choice = 0;
+    double best = (mul ? SEPARATE_MUL : SEPARATE) * (single_us(p.n, p.k, p.m, !mul, cus) + single_us(p.m, p.k, p.n, true, cus));
+    PairChoice choice = {0, false};
     for (int ix = 1; ix <= 3; ++ix)
         for (int iw = 1; iw <= 3; ++iw) {
             if ((ix == 3) != (iw == 3)) continue;
-            const double us = pair_us(p, ix, iw, cus);
+            bool dw_first;
+            const double us = pair_us(p, ix, iw, cus, &dw_first);
             if (us < best) {
                 best = us;
-                choice = 1 + 3 * (ix - 1) + (iw - 1);
+                choice = {1 + 3 * (ix - 1) + (iw - 1), dw_first};
             }
         }
     e = {p.n, p.m, p.k, mul, cus, choice};
@@ -102,16 +141,16 @@ int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, i
         const bool ok = pick_mode<bf16>(gx.a, gx.a_row, gx.a_k) == KMAJOR && pick_mode<bf16>(gx.b, gx.b_row, gx.b_k) == MNMAJOR &&
                         pick_mode<bf16>(gw.a, gw.a_row, gw.a_k) == MNMAJOR && pick_mode<bf16>(gw.b, gw.b_row, gw.b_k) == MNMAJOR &&
                         gt_eligible(gx, KMAJOR, MNMAJOR) && gt_eligible(gw, MNMAJOR, MNMAJOR);
-        const int choice = ok ? choose_pair(p) : 0;
-        if (choice != 0) {
+        const PairChoice choice = ok ? choose_pair(p) : PairChoice{0, false};
+        if (choice.config != 0) {
             const bool mul = p.mul != nullptr;
             int rc;
-            switch (choice) {
-                case 1: rc = launch_pair<PairSmall, PairSmall>(gx, gw, mul, st); break;
-                case 2: rc = launch_pair<PairSmall, PairWide>(gx, gw, mul, st); break;
-                case 4: rc = launch_pair<PairWide, PairSmall>(gx, gw, mul, st); break;
-                case 5: rc = launch_pair<PairWide, PairWide>(gx, gw, mul, st); break;
-                default: rc = launch_pair<PairSquare, PairSquare>(gx, gw, mul, st); break;
+            switch (choice.config) {
+                case 1: rc = launch_pair<PairSmall, PairSmall>(gx, gw, mul, choice.dw_first, st); break;
+                case 2: rc = launch_pair<PairSmall, PairWide>(gx, gw, mul, choice.dw_first, st); break;
+                case 4: rc = launch_pair<PairWide, PairSmall>(gx, gw, mul, choice.dw_first, st); break;
+                case 5: rc = launch_pair<PairWide, PairWide>(gx, gw, mul, choice.dw_first, st); break;
+                default: rc = launch_pair<PairSquare, PairSquare>(gx, gw, mul, choice.dw_first, st); break;
             }
             if (rc != PTJ_OK || !mul) return rc;
             if (!later->add(p.colpart, p.colsum, (n + 63) / 64, k, k))

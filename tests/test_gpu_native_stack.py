@@ -90,3 +90,22 @@ def test_native_stack_adds_up_partial_products(mt, lo, monkeypatch, dtype, D, F,
             monkeypatch.setattr(mt, "NATIVE_STACK", native)
             runs.append(mt.t_gpt2_forward_t(p, y, None, None, train, seeds))
         assert torch.equal(runs[0], runs[1]), (train, odd)
+
+
+# rows that make between half a round and three rounds of tiles, all but one with a tile that ends inside: dX first and dW first,
+# and tiles of 64x64, 64x128 and 128x128 for either
+@pytest.mark.parametrize("B,T", [(1, 576), (5, 192), (5, 384), (7, 448), (13, 320), (6, 1024), (11, 576)])
+def test_native_stack_pairs(mt, lo, monkeypatch, B, T):
+    """The two products of a linear layer's backward in one launch, either one first, against the single calls; bound as above (one
+    block, so no more than six stored tensors between any two products)."""
+    V, D, L, H, F = 101, 768, 1, 12, 3072
+    params = [[p.to(DEV).to(torch.bfloat16) for p in grp] for grp in ogpt2.init_transformer_gpt2(V, D, L, H, F, T, seed=3)]
+    y = torch.randint(0, V, (B, T + 1), generator=torch.Generator().manual_seed(7)).to(DEV)
+    runs = []
+    for native in (True, False):
+        monkeypatch.setattr(mt, "NATIVE_STACK", native)
+        grads, _ = lo.t_loss_bkwd3_t(params, y, None, None, True, list(range(10, 14)))
+        runs.append([p for grp in grads for p in grp])
+    for i, (a, b) in enumerate(zip(*runs)):
+        a, b = a.double(), b.double()
+        assert (a - b).norm() <= 6 ** 0.5 * 1.6e-3 * b.norm(), i
