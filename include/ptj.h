@@ -163,6 +163,9 @@ int ptj_embed_fwd(const void* wemb, const void* pos, const int64_t* tokens, void
  * ids is summed in that order in fp32, so the result is deterministic. */
 int ptj_embed_bwd(const void* d, const int64_t* sorted_tokens, const int64_t* order, void* dwemb,
                   int64_t n, int64_t dim, int64_t vocab, float scale, int dtype, void* stream);
+/* The same, bit for bit, from the token ids as they are, for n up to 8192. */
+int ptj_embed_bwd_tokens(const void* d, const int64_t* tokens, void* dwemb, int64_t n, int64_t dim, int64_t vocab,
+                         float scale, int dtype, void* stream);
 
 /* ptj_dropout_add[_keep] followed by ptj_layernorm_fwd on its result, in one pass:
  * y = res + dropout(x), h = layernorm(y) with the values of y as stored -- the residual

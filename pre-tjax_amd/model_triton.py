@@ -610,6 +610,9 @@ def embed_pos_dropout_t(wemb, pos, y, train=True, p_gen_aux=None):
     return out
 
 
+EMBED_SCAN_MAX = 8192    # positions up to which the embedding's backward finds equal tokens without a sort
+
+
 def embed_bkwd_add_t(dwemb, d, y):
     """dwemb[tok] += sqrt(D) * (sum of the rows of d [N,D] whose token is tok), in place and
     deterministic (model_triton.py:2489-2521 scatter-add, accumulated onto the tied LM-head
@@ -618,7 +621,12 @@ def embed_bkwd_add_t(dwemb, d, y):
     V, D = dwemb.shape
     assert dwemb.is_contiguous() and d.dtype == dwemb.dtype
     d2 = d.reshape(-1, D).contiguous()
-    stok, order = torch.sort(y.reshape(-1).to(torch.int64), stable=True)
+    tok = y.reshape(-1).to(torch.int64).contiguous()
+    if d2.shape[0] <= EMBED_SCAN_MAX:
+        check(lib().ptj_embed_bwd_tokens(ptr(d2), ptr(tok), ptr(dwemb), d2.shape[0], D, V, math.sqrt(D), dtype_code(dwemb),
+                                         stream()), "ptj_embed_bwd_tokens")
+        return dwemb
+    stok, order = torch.sort(tok, stable=True)
     check(lib().ptj_embed_bwd(ptr(d2), ptr(stok), ptr(order), ptr(dwemb), d2.shape[0], D, V, math.sqrt(D),
                               dtype_code(dwemb), stream()), "ptj_embed_bwd")
     return dwemb

@@ -60,3 +60,17 @@ def test_embed_bwd(mt, dtype, N, V, D, hot):
     assert torch.equal(got.cpu()[absent], dw0[absent])
     again = mt.embed_bkwd_add_t(dw0.clone().to(DEV), d.to(DEV), y.to(DEV))
     assert torch.equal(got, again)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,V,D", [(1, 5, 8), (63, 3, 100), (511, 400, 768), (513, 1, 768), (2048, 50257, 768), (2049, 30, 1030),
+                                   (4096, 900, 768), (4097, 50257, 768), (8191, 50257, 768), (8192, 700, 768)])
+def test_embed_bwd_without_a_sort(mt, monkeypatch, dtype, N, V, D):
+    """Up to EMBED_SCAN_MAX positions equal tokens are found by comparison; the sums are those of the sorted path, bit for bit."""
+    g = gen(N)
+    y = torch.randint(0, V, (N,), generator=g).to(DEV)
+    d, dw0 = randn(g, N, D, dtype=dtype).to(DEV), randn(g, V, D, dtype=dtype).to(DEV)
+    got = mt.embed_bkwd_add_t(dw0.clone(), d, y)
+    monkeypatch.setattr(mt, "EMBED_SCAN_MAX", 0)
+    assert torch.equal(got, mt.embed_bkwd_add_t(dw0.clone(), d, y))
+    assert not torch.equal(got, dw0)
