@@ -202,6 +202,11 @@ int ptj_ce_fwd_bwd(const int64_t* labels, const void* logits, float* loss, int64
                    int64_t rows, int64_t cols, int64_t logits_row_stride, int64_t dlogits_row_stride,
                    int dtype, void* stream);
 
+/* Share of the labels other than 0 that pred [rows, cols] meets (loss_and_optimizer_triton.py:199-200 given the row-wise argmax);
+ * NaN where every label is 0.  Labels in rows `row_stride` elements apart; at most 2^24 of them. */
+int ptj_accuracy(const int64_t* labels, int64_t row_stride, int64_t rows, int64_t cols, const int64_t* pred, float* out,
+                 void* stream);
+
 /* ptj_ce_fwd_bwd that also returns the column sums of the stored gradient,
  * colsum[c] = sum_r dlogits[r, c] -- the `.sum(dim=0)` bias gradient of t_linear_bkwd2_p
  * (model_triton.py:426) for the layer that produced the logits (the tied LM head,

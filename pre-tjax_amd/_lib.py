@@ -43,6 +43,7 @@ SIGNATURES = {
     "ptj_log_softmax_fwd": (_int, [_p, _p, _i64, _i64, _i64, _i64, _int, _p]),
     "ptj_log_softmax_bwd": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _int, _p]),
     "ptj_ce_workspace_bytes": (_sz, [_i64]),
+    "ptj_accuracy": (_int, [_p, _i64, _i64, _i64, _p, _p, _p]),
     "ptj_ce_fwd_bwd": (_int, [_p, _p, _p, _p, _p, _p, _p, _sz, _i64, _i64, _i64, _i64, _int, _p]),
     "ptj_ce_colsum_workspace_bytes": (_sz, [_i64, _i64]),
     "ptj_ce_fwd_bwd_colsum": (_int, [_p, _p, _p, _p, _p, _p, _p, _p, _sz, _i64, _i64, _i64, _i64, _int, _p]),

@@ -583,6 +583,49 @@ int ce_impl(const int64_t* labels, const void* logits, float* loss, int64_t* cou
 inline int ce_cs_grid() { return ptj_num_cus(); }   // one workgroup per CU (its LDS landing area fills the CU)
 inline int ce_cs_pcols(int64_t cols) { return (int)((cols + 8 + 7) / 8 * 8); }
 
+// Share of the labels other than 0 that `pred` meets: hits / labels, NaN where there is none.  One workgroup, a few thousand
+// labels are a few loads per thread.  As ten tensor operations (compare, select, mean) it took 26.6 us for 512 labels, 38.0 for 3136,
+// 35.9 for 16384 and 41.7 for 32768; this takes 2.2, 2.9, 6.4 and 10.8.
+constexpr int ACC_THREADS = 1024;
+__global__ __launch_bounds__(ACC_THREADS) void accuracy_kernel(const int64_t* __restrict__ labels, int64_t row_stride, int rows,
+                                                               int cols, const int64_t* __restrict__ pred, float* __restrict__ out) {
+    __shared__ int s_hits[ACC_THREADS / 64], s_valid[ACC_THREADS / 64];
+    const int n = rows * cols;
+    int hits = 0, valid = 0;
+    constexpr int U = 4;
+    for (int i0 = threadIdx.x; i0 < n; i0 += U * ACC_THREADS) {
+        int64_t y[U], p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 + u * ACC_THREADS, r = i / cols;
+            y[u] = i < n ? labels[r * row_stride + (i - r * cols)] : 0;
+            p[u] = i < n ? pred[i] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            valid += y[u] != 0;
+            hits += y[u] != 0 && y[u] == p[u];
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        hits += __shfl_xor(hits, o, 64);
+        valid += __shfl_xor(valid, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s_hits[threadIdx.x >> 6] = hits;
+        s_valid[threadIdx.x >> 6] = valid;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < ACC_THREADS / 64; ++w) {
+            hits += s_hits[w];
+            valid += s_valid[w];
+        }
+        *out = (float)hits / (float)valid;
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -676,6 +719,17 @@ int ptj_ce_fwd_bwd(const int64_t* labels, const void* logits, float* loss, int64
         case PTJ_BF16: return ce_impl<bf16>(labels, logits, loss, count, dlogits, pred, workspace, rows, cols, xs, dxs, st);
         default: return ptj_set_error(PTJ_ERR_INVALID, "ce_fwd_bwd: unknown dtype %d", dtype);
     }
+}
+
+int ptj_accuracy(const int64_t* labels, int64_t row_stride, int64_t rows, int64_t cols, const int64_t* pred, float* out,
+                 void* stream) {
+    PTJ_CHECK_ARG(labels && pred && out, "accuracy: null pointer");
+    PTJ_CHECK_ARG(rows >= 1 && cols >= 1 && rows < (1 << 24) && cols < (1 << 24) && rows * cols <= (1 << 24) && row_stride >= cols,
+                  "accuracy: bad shape %lld x %lld", (long long)rows, (long long)cols);
+    hipLaunchKernelGGL(accuracy_kernel, dim3(1), dim3(ACC_THREADS), 0, (hipStream_t)stream, labels, row_stride, (int)rows, (int)cols,
+                       pred, out);
+    PTJ_CHECK_LAUNCH();
+    return PTJ_OK;
 }
 
 }  // extern "C"

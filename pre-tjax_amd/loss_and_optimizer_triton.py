@@ -66,8 +66,17 @@ def t_avg_cross_entropy_loss_bkwd3_t(y_labels: torch.Tensor, x_logits: torch.Ten
     return out
 
 
+ACCURACY_MAX = 1 << 15   # labels that one workgroup counts faster than the tensor operations do
+
+
 def accuracy_from_pred(y_labels, pred):
     """loss_and_optimizer_triton.py:199-200 given the row-wise argmax."""
+    if (y_labels.is_cuda and y_labels.dim() == 2 and 0 < y_labels.numel() <= ACCURACY_MAX and y_labels.stride(1) == 1
+            and y_labels.stride(0) >= y_labels.shape[1] and y_labels.dtype == pred.dtype == torch.int64
+            and pred.shape == y_labels.shape and pred.is_contiguous() and pred.device == y_labels.device):
+        acc = torch.empty((), dtype=torch.float32, device=y_labels.device)
+        check(lib().ptj_accuracy(ptr(y_labels), y_labels.stride(0), *y_labels.shape, ptr(pred), ptr(acc), stream()), "ptj_accuracy")
+        return acc
     hit = (y_labels == pred).to(torch.float32)
     return torch.nanmean(torch.where(y_labels != 0, hit, torch.full_like(hit, float("nan"))))
 

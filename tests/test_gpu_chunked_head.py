@@ -151,3 +151,19 @@ def test_chunked_head_equals_one_pass_at_b16_t1024(lo, mt):
             assert rel < 1e-2, (gi, pi, rel)
     # half of the [N, V] logits buffer (0.82 GB) is gone
     assert peak0 - peak1 > 0.7e9, (peak0, peak1)
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (3, 63), (1, 1024), (5, 1025), (16, 1024), (33, 1000)])
+@pytest.mark.parametrize("share", [0.0, 0.3, 1.0])
+def test_accuracy_of_argmax(lo, monkeypatch, B, T, share):
+    """Counted by one kernel up to ACCURACY_MAX labels, by tensor operations beyond: the same quotient of two whole numbers, and NaN
+    where every label is 0."""
+    g = torch.Generator().manual_seed(B * T)
+    y = torch.randint(1, 9, (B, T + 1), generator=g) * (torch.rand((B, T + 1), generator=g) < share)
+    pred = torch.randint(0, 9, (B, T), generator=g).cuda()
+    labels = y.cuda()[:, 1:]
+    got = lo.accuracy_from_pred(labels, pred)
+    monkeypatch.setattr(lo, "ACCURACY_MAX", 0)
+    want = lo.accuracy_from_pred(labels, pred)
+    assert got.shape == want.shape and got.dtype == want.dtype
+    assert torch.equal(got, want) or (share < 1 and got.isnan() and want.isnan())
