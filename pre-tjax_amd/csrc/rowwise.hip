@@ -830,18 +830,21 @@ __global__ __launch_bounds__(256) void gelu_bwd_kernel(const T* __restrict__ dy,
     }
 }
 
-// One thread per VEC-wide chunk; chunks never straddle rows (cols % VEC == 0).
+// A thread takes one VEC-wide chunk of columns (cols % VEC == 0) in every `apart`-th row.  Bound by Philox's multiplications, which
+// run at a quarter of the vector rate: 17 an element, one of which depends on the column alone and is formed once, and
+// the division that finds a thread's row, once as well.  bf16, us, chunk by chunk / this: 64 x 768 2.81 / 2.68, 8192 x 768 11.1 / 10.7,
+// 16384 x 768 19.4 / 18.0, 777 x 4001 11.3 / 9.1.
 template <typename T, int VEC, bool ADD>
 __global__ __launch_bounds__(256) void dropout_kernel(const T* __restrict__ x, const T* __restrict__ res,
                                                        T* __restrict__ y, int64_t rows, int cols, int64_t xs,
                                                        int64_t ys, int train, uint64_t seed,
-                                                       uint8_t* __restrict__ keep_out) {
+                                                       uint8_t* __restrict__ keep_out, int64_t apart) {
     const int vpr = cols / VEC;  // vectors per row
-    const int64_t total = rows * vpr;
-    const bool small = total <= 0x7fffffffll;  // 32-bit division is several times cheaper
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-        const int64_t row = small ? (int64_t)((uint32_t)i / (uint32_t)vpr) : i / vpr;
-        const int c0 = (int)(i - row * vpr) * VEC;
+    const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t row0 = gridDim.x <= (1u << 22) ? (int64_t)((uint32_t)first / (uint32_t)vpr) : first / vpr;   // (32-bit: several times cheaper)
+    if (row0 >= apart) return;
+    const int vec = (int)(first - row0 * vpr), c0 = vec * VEC;
+    for (int64_t row = row0; row < rows; row += apart) {
         float v[VEC];
         load_vec<T, VEC>(x + row * xs + c0, v);
         if (train) {
@@ -855,7 +858,7 @@ __global__ __launch_bounds__(256) void dropout_kernel(const T* __restrict__ x, c
                 bits |= keep ? (1u << j) : 0u;
             }
             // keep byte of this 8-column group (only requested on the 8-wide path)
-            if (VEC == 8 && keep_out != nullptr) keep_out[i] = (uint8_t)bits;
+            if (VEC == 8 && keep_out != nullptr) keep_out[row * vpr + vec] = (uint8_t)bits;
         } else {
 #pragma unroll
             for (int j = 0; j < VEC; ++j) v[j] *= 0.9f;
@@ -1419,10 +1422,13 @@ int dropout_impl(const void* x, const void* res, void* y, int64_t rows, int64_t 
                      (!res || ptj_aligned16(res));
     if (keep_out != nullptr && !(vok && FV == 8))
         return ptj_set_error(PTJ_ERR_INVALID, "dropout: keep bytes need 2-byte elements, cols %% 8 == 0 and 16-byte aligned rows");
+    // several rows per thread once eight workgroups per CU are full, evenly (four: 16384 x 768 20.0 us instead of 17.9)
+    const int64_t vpr = vok ? cols / FV : cols, full = (rows * vpr + 255) / 256 / (8 * (int64_t)ptj_num_cus());
+    const int64_t each = full > 1 ? full : 1, apart = (rows + each - 1) / each;
 #define LAUNCH(V_, ADD_)                                                                                       \
-    hipLaunchKernelGGL((dropout_kernel<T, V_, ADD_>), dim3(flat_grid(rows * (cols / V_))), dim3(256), 0, st,     \
+    hipLaunchKernelGGL((dropout_kernel<T, V_, ADD_>), dim3((unsigned)((apart * vpr + 255) / 256)), dim3(256), 0, st, \
                        (const T*)x, (const T*)res, (T*)y, rows, (int)cols, xs, ys, train, (uint64_t)seed,       \
-                       (uint8_t*)keep_out)
+                       (uint8_t*)keep_out, apart)
     if (vok) {
         if (res) LAUNCH(FV, true); else LAUNCH(FV, false);
     } else {

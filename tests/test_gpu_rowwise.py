@@ -139,6 +139,24 @@ def test_dropout_mask_bit_exact(mt, dtype, shape, seed):
     assert torch.equal(ya, (r.to(torch.float32) + y.to(torch.float32)).to(dtype))
 
 
+# a thread takes several rows from about half a million chunks on: two to eleven, the last ones not in every thread
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape", [(16411, 768), (2003, 777), (70001, 64), (3, 2000003)])
+def test_dropout_several_rows_a_thread(mt, dtype, shape):
+    seed = (1 << 32) - 7                                   # the key's upper word changes from row to row
+    x = (randn(gen(8), *shape, dtype=dtype).abs() + 1.0).to(DEV)
+    y, r = mt.t_dropout_fwd_t(x, True, seed), randn(gen(9), *shape, dtype=dtype).to(DEV)
+    rows = [0, 1, shape[0] // 2, shape[0] - 2, shape[0] - 1]
+    for i in rows:
+        keep = ops.rowwise_keep((1, shape[1]), seed + i)[0]
+        assert torch.equal((y[i] != 0).cpu(), keep), i
+    assert torch.equal(torch.where(y != 0, x, y), y)
+    assert abs((y != 0).double().mean().item() - 0.9) < 5 * 0.3 / y.numel() ** 0.5
+    for i in range(0, shape[0], 4096):                     # the same rows by calls of fewer
+        assert torch.equal(mt.t_dropout_fwd_t(x[i:i + 4096], True, seed + i), y[i:i + 4096])
+    assert torch.equal(mt.dropout_add_t(x, r, True, seed), (r.float() + y.float()).to(dtype))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape", [(8, 12, 64, 512), (4096, 1024), (3, 37), (2, 4096), (5, 1)])
 def test_log_softmax(mt, dtype, shape):
