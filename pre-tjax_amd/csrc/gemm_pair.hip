@@ -4,8 +4,8 @@
 // (weights that the optimizer pass has pushed out of every cache) and of the write-back, on a quarter to a half of
 // the CUs.  Side by side they cost about what the longer one costs alone.  At some thousand tokens they make between one and
 // three rounds of tiles, and share the rounds: the product whose tiles take longer comes first in the grid and the shorter
-// tiles of the other fill the CUs as they fall free (dx: m contraction elements a tile, dw: n).  With dx first, us, before / now:
-// 3136 tokens proj 23.1 / 19.7, 6000 tokens ffn2 with its multiplier 95.6 / 84.5, qkv 61.2 / 62.0 (as two launches 75.4).
+// tiles of the other fill the CUs as they fall free (dx: m contraction elements a tile, dw: n).  With dx first / with dw first, us:
+// 3136 tokens proj 20.4 / 19.7, 6000 tokens ffn2 with its multiplier 95.6 / 84.5, 8192 tokens qkv 79.9 / 66.2, ffn1 115.1 / 90.5.
 #include "gemm_core.h"
 #include "gemm_plan.h"
 #include "internal.h"
