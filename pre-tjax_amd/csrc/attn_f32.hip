@@ -88,13 +88,22 @@ __device__ __forceinline__ Split8 row_split(const char* __restrict__ tile, int j
     for (int i = 0; i < 3; ++i) a.p[i] = *reinterpret_cast<const bf16x8*>(p + i * PANEL);
     return a;
 }
-// Two chains of products side by side (one after the other they wait for their own results): the lower parts first
+// The parts of two factors in the order of their products: the lower ones first.  P is formed again in the backward against the
+// forward's row maximum and sum, which only cancels the errors of the scores if they are the same bits: all three kernels sum
+// the products of Q and K in one chain and in this order of (K, Q).
+constexpr int FIRST[6] = {2, 0, 1, 1, 0, 0}, SECOND[6] = {0, 2, 1, 0, 1, 0};
+__device__ __forceinline__ void mma_one(f32x16& s, const Split8& a, const Split8& b) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) mma(s, a.p[FIRST[i]], b.p[SECOND[i]]);
+}
+// Two chains side by side.  SWAPPED: the second factor's parts in the order of the first's
+template <bool SWAPPED = false>
 __device__ __forceinline__ void mma_two(f32x16& s0, const Split8& a0, const Split8& b0, f32x16& s1, const Split8& a1, const Split8& b1) {
-    constexpr int A[6] = {2, 0, 1, 1, 0, 0}, B[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
-        mma(s0, a0.p[A[i]], b0.p[B[i]]);
-        mma(s1, a1.p[A[i]], b1.p[B[i]]);
+        const int x = SWAPPED ? SECOND[i] : FIRST[i], y = SWAPPED ? FIRST[i] : SECOND[i];
+        mma(s0, a0.p[x], b0.p[y]);
+        mma(s1, a1.p[x], b1.p[y]);
     }
 }
 
@@ -242,13 +251,11 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
         const int key0 = kt * 64 + half * 32;
         if (key0 <= qw0 + 31 && (!HAS_MASK || cls != TILE_HIDDEN)) {
             const char* kp = smem[kt & 1];
-            f32x16 s, s2;
+            f32x16 s;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) s[e] = s2[e] = 0.f;
+            for (int e = 0; e < 16; ++e) s[e] = 0.f;
 #pragma unroll
-            for (int c = 0; c < 2; ++c) mma_two(s, row_split(kp, half, c, lr, lg), qf[c], s2, row_split(kp, half, c + 2, lr, lg), qf[c + 2]);
-#pragma unroll
-            for (int e = 0; e < 16; ++e) s[e] += s2[e];
+            for (int c = 0; c < 4; ++c) mma_one(s, row_split(kp, half, c, lr, lg), qf[c]);       // S^T [key][query]
             if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4);
             if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0);
             float tmax = s[0];
@@ -403,7 +410,7 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
             for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
 #pragma unroll
             for (int c = 0; c < 4; ++c)       // S and dP [query][key]
-                mma_two(s, row_split(qp, half, c, lr, lg), kf[c], dp, row_split(dp_, half, c, lr, lg), row_split(vrows[(wave & 3) >> 1], wave & 1, c, lr, lg));
+                mma_two<true>(s, row_split(qp, half, c, lr, lg), kf[c], dp, row_split(dp_, half, c, lr, lg), row_split(vrows[(wave & 3) >> 1], wave & 1, c, lr, lg));
         }
         if (live) {
             if (q0 < kw0 + 31) apply_causal<false>(s, key - q0 - lg * 4);

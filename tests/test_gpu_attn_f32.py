@@ -43,6 +43,24 @@ def test_error_against_fp64(mt, B, H, T, masked):
         assert (got.double().cpu() - want).norm() <= 1e-6 * want.norm(), what
 
 
+@pytest.mark.parametrize("T", [64, 192])
+def test_both_directions_form_the_same_scores(mt, T):
+    """Every query sees its own key alone, so P is 1 and dV = 0.9 dO, whatever the score.  The scores are sums of terms of a thousand that
+    nearly cancel: formed in another order in the backward than in the forward they would differ by 1e-4 and more, and P with them.
+    As the same bits they leave the rounding of the saved maximum (0.1), 1 / l, 0.9 P and the product: under 8 of 2^-24."""
+    g = gen(T)
+    q, v, do = (randn(g, 1, 2, T, 64) for _ in range(3))
+    k = randn(g, 1, 2, T, 64)
+    q, k = q * 30, k * 30
+    # the last column takes what is left of the score but for about 0.3
+    k[..., 63] = (0.3 - (q[..., :63].double() * k[..., :63].double()).sum(-1)).div(q[..., 63].double()).float()
+    qkv = torch.stack([q, k, v], 2).to(DEV)
+    mask = torch.eye(T, dtype=torch.bool, device=DEV)[None]
+    _, dq, dk, dv = both(mt, qkv, do.to(DEV), mask)
+    want = 0.9 * do.double()
+    assert ((dv.double().cpu() - want).abs() <= 8 * 2.0 ** -24 * want.abs()).all()
+
+
 @pytest.mark.parametrize("train", [False, True])
 def test_gradients_scale_exactly(mt, train):
     """Every gradient is linear in dO: with dO a power of two smaller all parts, products and sums are, too."""
