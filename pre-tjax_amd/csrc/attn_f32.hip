@@ -42,39 +42,32 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
     for (int i = 0; i < 3; ++i) s.p[i] = __builtin_bit_cast(bf16x8, w[i]);
     return s;
 }
-// The same for values of the caller, which may round up to infinity or be infinite: then they are their own last part, which
-// meets nothing but the other factor's first one (a lower part may be 0 or of the other sign).
-__device__ __forceinline__ Split8 split8_any(const float (&x)[8]) {
-    float most = 0.f;
+// Values of the caller, the largest of which is noted: a workgroup that meets one of SPLIT_MOST or more, and a wavefront whose results
+// are not finite, forms them again by the fp32 instructions (plain_fwd, plain_dkdv, plain_dq; 4 times the time).  The parts of an
+// infinity or of what rounds to one are not numbers.  Below SPLIT_MOST no score and no product of dO and V overflows, and what
+// overflows later is seen in the results.
+constexpr float SPLIT_MOST = 0x1p32f;
+__device__ __forceinline__ Split8 split8_noted(const float (&x)[8], float& most) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(x[e]));
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(most >= 0x1p120f) == 0, 1)) return split8(x);
-    u32x4 first, last;
-    float rest[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const uint32_t top = __float_as_uint(x[e]) & 0xffff0000u;
-        const bool inf = fabsf(x[e]) == __builtin_inff();
-        rest[e] = inf ? 0.f : x[e] - __uint_as_float(top);
-        const uint32_t f = inf ? 0u : top, l = inf ? top : 0u;
-        first[e >> 1] = e & 1 ? first[e >> 1] | f : f >> 16;
-        last[e >> 1] = e & 1 ? last[e >> 1] | l : l >> 16;
-    }
-    Split8 s = split8(rest);
-    s.p[2] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, s.p[1]) | last);
-    s.p[1] = s.p[0];
-    s.p[0] = __builtin_bit_cast(bf16x8, first);
-    return s;
+    return split8(x);
 }
-__device__ __forceinline__ Split8 split_row_piece(const float* __restrict__ p) {
+// one multiply-add per value: NaN if one of them is not finite
+template <int N> __device__ __forceinline__ bool finite(const float (&x)[N]) {
+    float nan = 0.f;
+#pragma unroll
+    for (int e = 0; e < N; ++e) nan = fmaf(x[e], 0.f, nan);
+    return nan == 0.f;
+}
+__device__ __forceinline__ Split8 split_row_piece(const float* __restrict__ p, float& most) {
     const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
     const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-    return split8_any(x);
+    return split8_noted(x, most);
 }
 // The MFMA operand pieces of one 64-element row (lane half lg) in registers
-__device__ __forceinline__ void load_row_splits(Split8 (&f)[4], const float* __restrict__ row, int lg) {
+__device__ __forceinline__ void load_row_splits(Split8 (&f)[4], const float* __restrict__ row, int lg, float& most) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) f[c] = split_row_piece(row + c * 16 + lg * 8);
+    for (int c = 0; c < 4; ++c) f[c] = split_row_piece(row + c * 16 + lg * 8, most);
 }
 
 __device__ __forceinline__ void mma(f32x16& acc, const bf16x8& a, const bf16x8& b) {
@@ -141,9 +134,9 @@ struct TileCopy {
         r[0] = *reinterpret_cast<const f32x4*>(s);
         r[1] = *reinterpret_cast<const f32x4*>(s + 4);
     }
-    __device__ __forceinline__ void store(char* __restrict__ tile, int tid) const {
+    __device__ __forceinline__ void store(char* __restrict__ tile, int tid, float& most) const {
         const float x[8] = {r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1], r[1][2], r[1][3]};
-        const Split8 s = split8_any(x);
+        const Split8 s = split8_noted(x, most);
         char* to = tile + (tid >> 3) * BKB + (((tid & 7) ^ row_swizzle(tid >> 3)) << 4);
 #pragma unroll
         for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(to + i * PANEL) = s.p[i];
@@ -162,8 +155,33 @@ __device__ __forceinline__ void apply_mask(f32x16& s, const uint32_t* __restrict
     for (int i = 0; i < 16; ++i) s[i] = mask_select(s[i], NEG_RAW, mask_lanes(w, i));
 }
 
-// The forward's results of both wavefronts: o[half] is finished here (f: its factor, without the row's probability sum).
-struct RowStats { float m_run, m_true, l; };
+struct RowStats { float m_run, m_true, l; };      // reference point of the exponentials, true maximum (both base 2), sum
+// The reference point follows the row maximum only when it has been outgrown by 2^RESCALE_SLACK, see attn.hip
+__device__ __forceinline__ void follow_maximum(const f32x16& s, float sc, RowStats& r, f32x16 (&o)[2]) {
+    float tmax = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
+    tmax = max_xor32(tmax) * sc;
+    r.m_true = fmaxf(r.m_true, tmax);
+    if (__builtin_amdgcn_ballot_w64(tmax > r.m_run + RESCALE_SLACK) != 0) {
+        const float m_new = fmaxf(r.m_run, tmax), alpha = fast_exp2(r.m_run - m_new);
+        r.l *= alpha;
+        r.m_run = m_new;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
+    }
+}
+__device__ __forceinline__ void store_stats(const AttnArgs& a, int64_t at, const RowStats& r) {
+    const bool empty = r.l == 0.f;
+    a.ms[at] = empty ? NEG_NAT : r.m_true * LN2;
+    a.ls[at] = empty ? 0.f : r.l * fast_exp2(r.m_run - r.m_true);
+}
+// l = 0: no key of the row is visible (a row with a visible key has l >= 1)
+template <bool TRAIN> __device__ __forceinline__ float row_factor(float l) { return l == 0.f ? 0.f : (TRAIN ? 1.0f : 0.9f) / l; }
+
+// The forward's results of both wavefronts: the columns of its own half are finished here.
 __device__ __forceinline__ RowStats merge_halves(float (&out)[16], const f32x16 (&o)[2], RowStats mine, int half, char* __restrict__ smem, int wave,
                                                  int partner, int lane) {
     float give[19], take[19];
@@ -179,11 +197,202 @@ __device__ __forceinline__ RowStats merge_halves(float (&out)[16], const f32x16 
     return {m_run, fmaxf(mine.m_true, take[17]), half ? fmaf(take[18], f1, mine.l * f0) : fmaf(mine.l, f0, take[18] * f1)};
 }
 
+// ---- the same by the fp32 instructions, operands straight from memory: for workgroups whose values the split does not take ----
+// Each function: one wavefront, 32 rows (all of them exist) against every tile of 32; of the results what `half` finishes.
+// s += (32 rows, the lane's at x) x (32 rows, the lane's at y), contraction over their 64 columns.  (Rolled: nothing is kept in
+// registers that the main loops need.)
+__device__ __forceinline__ void plain_rows(f32x16& s, const float* __restrict__ x, const float* __restrict__ y, int lg) {
+#pragma unroll 1
+    for (int c = 0; c < 8; ++c)
+        mma_chunk(s, *reinterpret_cast<const f32x4*>(x + c * 8 + lg * 4), *reinterpret_cast<const f32x4*>(y + c * 8 + lg * 4));
+}
+// o[t] += (columns 32 t .. of 32 rows, transposed) x p, contraction over the rows
+__device__ __forceinline__ void plain_columns(f32x16 (&o)[2], const float* __restrict__ rows, int64_t rs, const float (&p)[16], int lr, int lg) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            f32x4 x, y;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                x[e] = rows[(c * 8 + lg * 4 + e) * rs + t * 32 + lr];
+                y[e] = p[4 * c + e];
+            }
+            mma_chunk(o[t], x, y);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+__device__ __forceinline__ float plain_delta(const float* __restrict__ d_o, const float* __restrict__ o, int lg) {
+    float sum = 0.f;
+#pragma unroll 1
+    for (int c = 0; c < 8; ++c) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(d_o + c * 8 + lg * 4), y = *reinterpret_cast<const f32x4*>(o + c * 8 + lg * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum += x[e] * y[e];
+    }
+    return sum + xor32(sum);
+}
+// Mask words and tile classes of the 32 rows from row0 on (AttnArgs::mask)
+struct PlainMask { const uint32_t *words, *classes; };
+template <bool LANE_IS_QUERY> __device__ __forceinline__ PlainMask plain_mask(const AttnArgs& a, int bidx, int row0) {
+    const int64_t G = a.T >> 5, block = bidx * G + (row0 >> 5), all = (int64_t)a.B * G;
+    return {a.mask + (LANE_IS_QUERY ? 0 : all * a.T) + block * a.T, a.mask + 2 * all * a.T + (LANE_IS_QUERY ? 0 : all * G) + block * G};
+}
+
+template <bool HAS_MASK, bool TRAIN>
+__device__ __forceinline__ void plain_fwd(const AttnArgs& a, int bh, int qw0, int half) {
+    const int lane = threadIdx.x & 63, lr = lane & 31, lg = lane >> 5, bidx = bh / a.H, hidx = bh % a.H, query = qw0 + lr;
+    const float* const k = (const float*)a.k + bidx * a.k_bs + hidx * a.k_hs;
+    const float* const v = (const float*)a.v + bidx * a.v_bs + hidx * a.v_hs;
+    const float* const q_row = (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs + query * a.q_rs;
+    const float sc = a.scale * LOG2E;
+    RowStats row = {M_START, M_START, 0.f};
+    f32x16 o[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
+#pragma unroll 1
+    for (int key0 = 0; key0 <= qw0; key0 += 32) {
+        uint32_t cls = TILE_CAUSAL;
+        if constexpr (HAS_MASK) cls = as_uniform(plain_mask<true>(a, bidx, qw0).classes)[key0 >> 5];
+        if (cls == TILE_HIDDEN) continue;
+        f32x16 s;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[e] = 0.f;
+        plain_rows(s, k + (key0 + lr) * a.k_rs, q_row, lg);
+        if (key0 == qw0) apply_causal<true>(s, query - key0 - lg * 4);
+        if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, plain_mask<true>(a, bidx, qw0).words + key0);
+        follow_maximum(s, sc, row, o);
+        KeepWords kw;
+        if constexpr (TRAIN) kw = load_keep_half(a.keepbits + (int64_t)bh * a.bitwords, qw0 + key0);
+        float p[16], lsum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            p[e] = fast_exp2(fmaf(s[e], sc, -row.m_run));
+            lsum += p[e];
+            if constexpr (TRAIN) p[e] = keep_select(p[e], keep_mask(kw, e));
+        }
+        plain_columns(o, v + key0 * a.v_rs, a.v_rs, p, lr, lg);
+        row.l += sum_xor32(lsum);
+    }
+    float out[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) out[e] = half ? o[1][e] : o[0][e];
+    store_half_row<float>((float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + query * a.out0_rs + half * 32, out, row_factor<TRAIN>(row.l), lg);
+    if (lg == 0 && half == 0) store_stats(a, (int64_t)bh * a.T + query, row);
+}
+
+template <bool HAS_MASK, bool TRAIN>
+__device__ __forceinline__ void plain_dkdv(const AttnArgs& a, int bh, int kw0, int half) {
+    const int lane = threadIdx.x & 63, lr = lane & 31, lg = lane >> 5, bidx = bh / a.H, hidx = bh % a.H, key = kw0 + lr;
+    const float* const q = (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs;
+    const float* const d_o = (const float*)a.d_o + bidx * a.do_bs + hidx * a.do_hs;
+    const float* const o = (const float*)a.o + bidx * a.o_bs + hidx * a.o_hs;
+    const float* const k_row = (const float*)a.k + bidx * a.k_bs + hidx * a.k_hs + key * a.k_rs;
+    const float* const v_row = (const float*)a.v + bidx * a.v_bs + hidx * a.v_hs + key * a.v_rs;
+    const float sc = a.scale * LOG2E;
+    f32x16 dk[2], dv[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dk[t][e] = dv[t][e] = 0.f;
+#pragma unroll 1
+    for (int q0 = kw0; q0 < a.T; q0 += 32) {
+        uint32_t cls = TILE_CAUSAL;
+        if constexpr (HAS_MASK) cls = as_uniform(plain_mask<false>(a, bidx, kw0).classes)[q0 >> 5];
+        if (cls == TILE_HIDDEN) continue;
+        f32x16 s, dp;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
+        plain_rows(s, q + (q0 + lr) * a.q_rs, k_row, lg);
+        plain_rows(dp, d_o + (q0 + lr) * a.do_rs, v_row, lg);
+        if (q0 == kw0) apply_causal<false>(s, key - q0 - lg * 4);
+        if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, plain_mask<false>(a, bidx, kw0).words + q0);
+        KeepWords kw;
+        if constexpr (TRAIN) kw = load_keep_half(a.keepbits + (int64_t)bh * a.bitwords, kw0 + q0);
+        // the statistics of query q0 + lr, passed to the lanes that hold elements of its row
+        const float delta = plain_delta(d_o + (q0 + lr) * a.do_rs, o + (q0 + lr) * a.o_rs, lg);
+        const int64_t si = (int64_t)bh * a.T + q0 + lr;
+        const float l = a.ls[si];
+        const bool none = l == 0.f;
+        const float linv = none ? 0.f : 1.0f / l, m2 = none ? 0.f : a.ms[si] * LOG2E;
+        float pd[16], ds[16];
+        int first = 4 * lg;
+        asm volatile("" : "+v"(first));          // (sixteen lane numbers are not kept over the loop)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int qi = first + 8 * (i >> 2) + (i & 3);
+            const float d = __shfl(delta, qi, 64), p = fast_exp2(fmaf(s[i], sc, -__shfl(m2, qi, 64))) * __shfl(linv, qi, 64);
+            if constexpr (TRAIN) {
+                pd[i] = keep_select(p, keep_mask(kw, i));
+                ds[i] = fmaf(pd[i], dp[i], -(p * d));
+            } else {
+                pd[i] = 0.9f * p;
+                ds[i] = p * fmaf(dp[i], 0.9f, -d);
+            }
+        }
+        plain_columns(dv, d_o + q0 * a.do_rs, a.do_rs, pd, lr, lg);
+        plain_columns(dk, q + q0 * a.q_rs, a.q_rs, ds, lr, lg);
+    }
+    if (half) store_rows<float>((float*)a.out1 + bidx * a.out1_bs + hidx * a.out1_hs + key * a.out1_rs, dv, 1.0f, lg);
+    else store_rows<float>((float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + key * a.out0_rs, dk, a.scale, lg);
+}
+
+template <bool HAS_MASK, bool TRAIN>
+__device__ __forceinline__ void plain_dq(const AttnArgs& a, int bh, int qw0, int half) {
+    const int lane = threadIdx.x & 63, lr = lane & 31, lg = lane >> 5, bidx = bh / a.H, hidx = bh % a.H, query = qw0 + lr;
+    const float* const k = (const float*)a.k + bidx * a.k_bs + hidx * a.k_hs;
+    const float* const v = (const float*)a.v + bidx * a.v_bs + hidx * a.v_hs;
+    const float* const q_row = (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs + query * a.q_rs;
+    const float* const do_row = (const float*)a.d_o + bidx * a.do_bs + hidx * a.do_hs + query * a.do_rs;
+    const float delta = plain_delta(do_row, (const float*)a.o + bidx * a.o_bs + hidx * a.o_hs + query * a.o_rs, lg);
+    const int64_t si = (int64_t)bh * a.T + query;
+    const float l = a.ls[si], sc = a.scale * LOG2E;
+    const bool none = l == 0.f;
+    const float linv = none ? 0.f : 1.0f / l, m2 = none ? 0.f : a.ms[si] * LOG2E;
+    f32x16 dq[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dq[t][e] = 0.f;
+#pragma unroll 1
+    for (int key0 = 0; key0 <= qw0; key0 += 32) {
+        uint32_t cls = TILE_CAUSAL;
+        if constexpr (HAS_MASK) cls = as_uniform(plain_mask<true>(a, bidx, qw0).classes)[key0 >> 5];
+        if (cls == TILE_HIDDEN) continue;
+        f32x16 s, dp;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
+        plain_rows(s, k + (key0 + lr) * a.k_rs, q_row, lg);
+        plain_rows(dp, v + (key0 + lr) * a.v_rs, do_row, lg);
+        if (key0 == qw0) apply_causal<true>(s, query - key0 - lg * 4);
+        if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, plain_mask<true>(a, bidx, qw0).words + key0);
+        KeepWords kw;
+        if constexpr (TRAIN) kw = load_keep_half(a.keepbits + (int64_t)bh * a.bitwords, qw0 + key0);
+        float ds[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float p = fast_exp2(fmaf(s[i], sc, -m2)) * linv;
+            if constexpr (TRAIN) ds[i] = p * (keep_select(dp[i], keep_mask(kw, i)) - delta);
+            else ds[i] = p * fmaf(dp[i], 0.9f, -delta);
+        }
+        plain_columns(dq, k + key0 * a.k_rs, a.k_rs, ds, lr, lg);
+    }
+    float out[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) out[e] = half ? dq[1][e] : dq[0][e];
+    store_half_row<float>((float*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + query * a.out2_rs + half * 32, out, a.scale, lg);
+}
+
 // ---- forward -------------------------------------------------------------------------
 // grid (B*H, ceil(T/128)): wavefront (half, block) owns queries q0 + 32 block .. +31 against the keys of its half of each tile
 template <bool HAS_MASK, bool TRAIN>
 __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs a) {
     __shared__ __attribute__((aligned(16))) char smem[2][2 * TILE];      // K, V
+    __shared__ int big;
+    if (threadIdx.x == 0) big = 0;
 
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
@@ -198,16 +407,17 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
     cv.init((const float*)a.v + bidx * a.v_bs + hidx * a.v_hs, a.v_rs, tid);
     ck.fetch(0);
     cv.fetch(0);
+    float most = 0.f;
     Split8 qf[4];
-    load_row_splits(qf, (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs + (int64_t)qrow * a.q_rs, lg);
-    ck.store(smem[0], tid);
-    cv.store(smem[0] + TILE, tid);
+    load_row_splits(qf, (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs + (int64_t)qrow * a.q_rs, lg, most);
+    ck.store(smem[0], tid, most);
+    cv.store(smem[0] + TILE, tid, most);
     __syncthreads();
 
     int nkt = (q0 + 128) / 64;
     if (nkt > a.T / 64) nkt = a.T / 64;
     const float sc = a.scale * LOG2E;
-    float m_run = M_START, m_true = M_START, l_run = 0.f;
+    RowStats row = {M_START, M_START, 0.f};
     f32x16 o[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -231,8 +441,8 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
         cv.fetch(tile);
     };
     auto store = [&](int tile) __attribute__((always_inline)) {
-        ck.store(smem[tile & 1], tid);
-        cv.store(smem[tile & 1] + TILE, tid);
+        ck.store(smem[tile & 1], tid, most);
+        cv.store(smem[tile & 1] + TILE, tid, most);
     };
     if (half && nkt > 1) fetch(1);
     for (int kt = 0; kt < nkt; ++kt) {
@@ -258,34 +468,20 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
             for (int c = 0; c < 4; ++c) mma_one(s, row_split(kp, half, c, lr, lg), qf[c]);       // S^T [key][query]
             if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4);
             if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0);
-            float tmax = s[0];
-#pragma unroll
-            for (int i = 1; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
-            tmax = max_xor32(tmax) * sc;
-            m_true = fmaxf(m_true, tmax);
-            // the reference point follows the row maximum only when it has been outgrown by 2^RESCALE_SLACK, see attn.hip
-            if (__builtin_amdgcn_ballot_w64(tmax > m_run + RESCALE_SLACK) != 0) {
-                const float m_new = fmaxf(m_run, tmax), alpha = fast_exp2(m_run - m_new);
-                l_run *= alpha;
-                m_run = m_new;
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
-            }
+            follow_maximum(s, sc, row, o);
             float lsum = 0.f;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 float p[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    p[e] = fast_exp2(fmaf(s[8 * h + e], sc, -m_run));
+                    p[e] = fast_exp2(fmaf(s[8 * h + e], sc, -row.m_run));
                     lsum += p[e];
                     if constexpr (TRAIN) p[e] = keep_select(p[e], keep_mask(kw, 8 * h + e));
                 }
                 columns_x_regs(o, kp + TILE, split8(p), half, h, lr, lg);
             }
-            l_run += sum_xor32(lsum);
+            row.l += sum_xor32(lsum);
         }
         if (half == 0 && more) store(kt + 1);
         __syncthreads();
@@ -293,16 +489,14 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
 
     // Both halves of the keys together; each wavefront finishes the columns of its own half.
     float out[16];
-    const RowStats r = merge_halves(out, o, {m_run, m_true, l_run}, half, &smem[0][0], wave, wave ^ 4, lane);
-    if (query < a.T) {
-        // l = 0: no key of the row is visible (a row with a visible key has l >= 1)
-        const bool empty = r.l == 0.f;
-        const float f = empty ? 0.f : (TRAIN ? 1.0f : 0.9f) / r.l;
-        store_half_row<float>((float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs + half * 32, out, f, lg);
-        if (lg == 0 && half == 0) {
-            a.ms[(int64_t)bh * a.T + query] = empty ? NEG_NAT : r.m_true * LN2;
-            a.ls[(int64_t)bh * a.T + query] = empty ? 0.f : r.l * fast_exp2(r.m_run - r.m_true);
-        }
+    if (most >= SPLIT_MOST) big = 1;
+    const RowStats r = merge_halves(out, o, row, half, &smem[0][0], wave, wave ^ 4, lane);
+    if (qw0 >= a.T) return;
+    if (__builtin_expect(big || __any(!finite(out)), 0)) {
+        plain_fwd<HAS_MASK, TRAIN>(a, bh, qw0, half);
+    } else {
+        store_half_row<float>((float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs + half * 32, out, row_factor<TRAIN>(r.l), lg);
+        if (lg == 0 && half == 0) store_stats(a, (int64_t)bh * a.T + query, r);
     }
 }
 
@@ -312,7 +506,7 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
 // registers, those of V in LDS: both in registers spill (8 x 512: 122 us instead of 93).
 typedef float StatTile[3][64];            // m2, 1/l, delta of a query tile
 template <bool HAS_MASK, bool TRAIN>
-__device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const int key_tile, char (*smem)[2 * TILE], char (*vrows)[TILE], StatTile* sstat) {
+__device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const int key_tile, char (*smem)[2 * TILE], char (*vrows)[TILE], StatTile* sstat, int& big) {
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
     const int bidx = bh / a.H, hidx = bh % a.H;
@@ -326,7 +520,7 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
     cd.init((const float*)a.d_o + bidx * a.do_bs + hidx * a.do_hs, a.do_rs, tid);
     co.init((const float*)a.o + bidx * a.o_bs + hidx * a.o_hs, a.o_rs, tid);
     const int64_t stat0 = (int64_t)bh * a.T + (tid & 63);
-    float st_m = 0.f, st_l = 0.f;
+    float st_m = 0.f, st_l = 0.f, most = 0.f;
     auto fetch = [&](int qt) __attribute__((always_inline)) {
         cq.fetch(qt);
         cd.fetch(qt);
@@ -350,8 +544,8 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
             sstat[b][0][tid] = none ? 0.f : st_m * LOG2E;
             sstat[b][1][tid] = none ? 0.f : 1.0f / st_l;
         }
-        cq.store(smem[b], tid);
-        cd.store(smem[b] + TILE, tid);
+        cq.store(smem[b], tid, most);
+        cd.store(smem[b] + TILE, tid, most);
     };
     fetch(qt0);
     {
@@ -359,12 +553,12 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
         TileCopy cv;
         cv.init((const float*)a.v + bidx * a.v_bs + hidx * a.v_hs, a.v_rs, tid);
         cv.fetch(key_tile * 2);
-        cv.store(vrows[0], tid);
+        cv.store(vrows[0], tid, most);
         cv.fetch(key_tile * 2 + 1 < nqt ? key_tile * 2 + 1 : nqt - 1);
-        cv.store(vrows[1], tid);
+        cv.store(vrows[1], tid, most);
     }
     Split8 kf[4];
-    load_row_splits(kf, (const float*)a.k + bidx * a.k_bs + hidx * a.k_hs + (int64_t)krow * a.k_rs, lg);
+    load_row_splits(kf, (const float*)a.k + bidx * a.k_bs + hidx * a.k_hs + (int64_t)krow * a.k_rs, lg, most);
     store(0);
     __syncthreads();
 
@@ -454,14 +648,22 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) give[16 * t + e] = half ? dk[t][e] : dv[t][e];
+    if (most >= SPLIT_MOST) big = 1;
     exchange(give, take, &smem[0][0], wave, wave ^ 4, lane);
-    if (key < a.T) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) take[16 * t + e] += half ? dv[t][e] : dk[t][e];
+    if (kw0 >= a.T) return;
+    if (__builtin_expect(big || __any(!finite(take)), 0)) {
+        plain_dkdv<HAS_MASK, TRAIN>(a, bh, kw0, half);
+    } else {
+        float* const row = half ? (float*)a.out1 + bidx * a.out1_bs + hidx * a.out1_hs + (int64_t)key * a.out1_rs
+                                : (float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)key * a.out0_rs;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) dk[t][e] = (half ? dv[t][e] : dk[t][e]) + take[16 * t + e];
-        float* const row = half ? (float*)a.out1 + bidx * a.out1_bs + hidx * a.out1_hs + (int64_t)key * a.out1_rs
-                                : (float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)key * a.out0_rs;
+            for (int e = 0; e < 16; ++e) dk[t][e] = take[16 * t + e];
         store_rows<float>(row, dk, half ? 1.0f : a.scale, lg);
     }
 }
@@ -469,7 +671,7 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
 // ---- backward: dQ -----------------------------------------------------------------------
 // Same geometry as the forward.
 template <bool HAS_MASK, bool TRAIN>
-__device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const int query_tile, char (*smem)[2 * TILE]) {
+__device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const int query_tile, char (*smem)[2 * TILE], int& big) {
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
     const int bidx = bh / a.H, hidx = bh % a.H;
@@ -500,11 +702,12 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const in
     const float lsum = a.ls[si];
     const bool none = lsum == 0.f;
     const float linv = none ? 0.f : 1.0f / lsum, m2 = none ? 0.f : a.ms[si] * LOG2E;
+    float most = 0.f;
     Split8 qf[4], dof[4];
-    load_row_splits(qf, (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs + (int64_t)qrow * a.q_rs, lg);
-    load_row_splits(dof, do_row, lg);
-    ck.store(smem[0], tid);
-    cv.store(smem[0] + TILE, tid);
+    load_row_splits(qf, (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs + (int64_t)qrow * a.q_rs, lg, most);
+    load_row_splits(dof, do_row, lg, most);
+    ck.store(smem[0], tid, most);
+    cv.store(smem[0] + TILE, tid, most);
     __syncthreads();
 
     int nkt = (q0 + 128) / 64;
@@ -532,8 +735,8 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const in
         cv.fetch(tile);
     };
     auto store = [&](int tile) __attribute__((always_inline)) {
-        ck.store(smem[tile & 1], tid);
-        cv.store(smem[tile & 1] + TILE, tid);
+        ck.store(smem[tile & 1], tid, most);
+        cv.store(smem[tile & 1] + TILE, tid, most);
     };
     if (half && nkt > 1) fetch(1);
     for (int kt = 0; kt < nkt; ++kt) {
@@ -580,12 +783,14 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const in
     float give[16], take[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) give[e] = half ? dq[0][e] : dq[1][e];
+    if (most >= SPLIT_MOST) big = 1;
     exchange(give, take, &smem[0][0], wave, wave ^ 4, lane);
-    if (query < a.T) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) take[e] += half ? dq[1][e] : dq[0][e];
+    for (int e = 0; e < 16; ++e) take[e] += half ? dq[1][e] : dq[0][e];
+    if (qw0 >= a.T) return;
+    if (__builtin_expect(big || __any(!finite(take)), 0)) plain_dq<HAS_MASK, TRAIN>(a, bh, qw0, half);
+    else
         store_half_row<float>((float*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs + half * 32, take, a.scale, lg);
-    }
 }
 
 // grid (B*H, 2 ceil(T/128)): both passes in one launch, the tiles with the longest way first
@@ -594,9 +799,11 @@ __global__ __launch_bounds__(THREADS, 2) void attn_bwd_f32_kernel(const AttnArgs
     __shared__ __attribute__((aligned(16))) char smem[2][2 * TILE];
     __shared__ __attribute__((aligned(16))) char vrows[2][TILE];
     __shared__ __attribute__((aligned(16))) StatTile sstat[2];
+    __shared__ int big;
+    if (threadIdx.x == 0) big = 0;
     const int tile = blockIdx.y >> 1;
-    if (blockIdx.y & 1) bwd_dq<HAS_MASK, TRAIN>(a, blockIdx.x, (gridDim.y >> 1) - 1 - tile, smem);
-    else bwd_dkdv<HAS_MASK, TRAIN>(a, blockIdx.x, tile, smem, vrows, sstat);
+    if (blockIdx.y & 1) bwd_dq<HAS_MASK, TRAIN>(a, blockIdx.x, (gridDim.y >> 1) - 1 - tile, smem, big);
+    else bwd_dkdv<HAS_MASK, TRAIN>(a, blockIdx.x, tile, smem, vrows, sstat, big);
 }
 
 }  // namespace

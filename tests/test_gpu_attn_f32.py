@@ -69,13 +69,59 @@ def test_gradients_scale_exactly(mt, train):
     assert all(torch.equal(x * 2.0 ** -60, y) for x, y in zip(a[1:], b[1:]))
 
 
+@pytest.mark.parametrize("T", [64, 192])
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("masked", [False, True])
+def test_values_that_are_not_split(mt, T, train, masked):
+    """V from 2^32 on is multiplied by the fp32 instructions: O and the gradients of Q and K are as many times larger, that of V the
+    same, but for what either way rounds (1e-6 each as in test_error_against_fp64)."""
+    qkv, do, mask = case(2, 2, T, 7)
+    if not masked:
+        mask = torch.ones(T, T, dtype=torch.bool, device=DEV).tril().expand(2, T, T).contiguous()
+    big = qkv.clone()
+    big[:, :, 2] *= 2.0 ** 40
+    for what, x, y, e in zip(("o", "dq", "dk", "dv"), both(mt, big, do, mask, train), both(mt, qkv, do, mask, train), (40, 40, 40, 0)):
+        x, y = x.double() * 2.0 ** -e, y.double()
+        assert torch.isfinite(x).all() and (x - y).norm() <= 2e-6 * y.norm(), what
+
+
+def test_infinite_factors(mt):
+    """inf * -inf is -inf: key 10 is as good as hidden from every query, and so is every key from query 70."""
+    T = 192
+    qkv, do, _ = case(1, 1, T, 6)
+    qkv[0, 0, 0, :, 3] = qkv[0, 0, 0, :, 3].abs()
+    qkv[0, 0, 1, :, 3] = -qkv[0, 0, 1, :, 3].abs()
+    mask = torch.ones(T, T, dtype=torch.bool, device=DEV).tril()[None].contiguous()
+    mask[:, :, 10] = False
+    mask[:, 70] = False
+    want = both(mt, qkv, do, mask)[0]
+    qkv[0, 0, 0, 70, 3], qkv[0, 0, 1, 10, 3] = float("inf"), float("-inf")
+    got = both(mt, qkv, do, torch.ones_like(mask).tril())[0]
+    assert torch.equal(got[0, 0, 70], torch.zeros(64, device=DEV)) and (got - want).norm() <= 2e-6 * want.norm()
+
+
+def test_overflowing_products_of_the_backward(mt):
+    """dP of the last query and key 5 overflows, all else is finite: dQ of that query and dK of that key are infinite, with the signs
+    of K and Q."""
+    T = 64
+    qkv, do, _ = case(1, 1, T, 8)
+    qkv[0, 0, 2, :, 0], qkv[0, 0, 2, 5, 0] = 0.1, 2.0
+    do[0, 0, T - 1], do[0, 0, T - 1, 0] = 0.0, 3e38
+    _, dq, dk, dv = (x[0, 0] for x in both(mt, qkv, do, torch.ones(T, T, dtype=torch.bool, device=DEV).tril()[None]))
+    q, k = qkv[0, 0, 0], qkv[0, 0, 1]
+    assert torch.equal(dq[T - 1], float("inf") * k[5].sign()) and torch.equal(dk[5], float("inf") * q[T - 1].sign())
+    rest = torch.ones(T, dtype=torch.bool, device=DEV)
+    rest[5] = False
+    assert torch.isfinite(dv).all() and torch.isfinite(dq[:T - 1]).all() and torch.isfinite(dk[rest]).all()
+
+
 def test_large_and_infinite_values(mt):
     T = 192
     qkv, do, mask = case(1, 1, T, 6)
     mask = torch.ones(T, T, dtype=torch.bool, device=DEV).tril()[None]
     plain = both(mt, qkv, do, mask)[0]
     big = qkv.clone()
-    big[:, :, 2] *= 2.0 ** 121                      # its parts are formed by truncation
+    big[:, :, 2] *= 2.0 ** 121
     got = both(mt, big, do, mask)[0]
     assert (got.double() * 2.0 ** -121 - plain.double()).norm() <= 1e-6 * plain.double().norm()
     inf = qkv.clone()
