@@ -81,24 +81,32 @@ __device__ __forceinline__ Split8 row_split(const char* __restrict__ tile, int j
     for (int i = 0; i < 3; ++i) a.p[i] = *reinterpret_cast<const bf16x8*>(p + i * PANEL);
     return a;
 }
-// The parts of two factors in the order of their products: the lower ones first.  P is formed again in the backward against the
-// forward's row maximum and sum, which only cancels the errors of the scores if they are the same bits: all three kernels sum
-// the products of Q and K in one chain and in this order of (K, Q).
+// The leading part alone
+__device__ __forceinline__ bf16x8 row_first(const char* __restrict__ tile, int j, int c, int lr, int lg) {
+    return *reinterpret_cast<const bf16x8*>(tile + (j * 32 + lr) * BKB + (((c * 2 + lg) ^ row_swizzle(lr)) << 4));
+}
+// The parts of two factors in the order of their products: the lower ones first.  Scores are sums of one chain, with the products of
+// leading parts behind all others: the matrix pipe rounds its accumulator with every instruction, here four times at its full
+// size and twenty times at 2^-8 of it.  (All six of a chunk after one another: twice the error against fp64 in every result.)
+// P is formed again in the backward against the forward's row maximum and sum, which only cancels what error the scores have if they are
+// the same bits: all three kernels keep to this order of (K, Q).
 constexpr int FIRST[6] = {2, 0, 1, 1, 0, 0}, SECOND[6] = {0, 2, 1, 0, 1, 0};
-__device__ __forceinline__ void mma_one(f32x16& s, const Split8& a, const Split8& b) {
+__device__ __forceinline__ void mma_low(f32x16& s, const Split8& a, const Split8& b) {
 #pragma unroll
-    for (int i = 0; i < 6; ++i) mma(s, a.p[FIRST[i]], b.p[SECOND[i]]);
+    for (int i = 0; i < 5; ++i) mma(s, a.p[FIRST[i]], b.p[SECOND[i]]);
 }
 // Two chains side by side.  SWAPPED: the second factor's parts in the order of the first's
-template <bool SWAPPED = false>
+template <int N = 6, bool SWAPPED = false>
 __device__ __forceinline__ void mma_two(f32x16& s0, const Split8& a0, const Split8& b0, f32x16& s1, const Split8& a1, const Split8& b1) {
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
+    for (int i = 0; i < N; ++i) {
         const int x = SWAPPED ? SECOND[i] : FIRST[i], y = SWAPPED ? FIRST[i] : SECOND[i];
         mma(s0, a0.p[x], b0.p[y]);
         mma(s1, a1.p[x], b1.p[y]);
     }
 }
+// The leading parts are read again behind the lower products (kept in registers, the backward spills)
+__device__ __forceinline__ void forget_rows() { asm volatile("" ::: "memory"); }
 
 // o[t] += (columns 32 t .. of the tile, transposed) x p: contraction over the tile's rows 32 j + 16 h .. + 15, of which the lane
 // holds p[e] for row 32 j + 16 h + 8 (e / 4) + 4 lg + e % 4
@@ -465,7 +473,10 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
 #pragma unroll
             for (int e = 0; e < 16; ++e) s[e] = 0.f;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) mma_one(s, row_split(kp, half, c, lr, lg), qf[c]);       // S^T [key][query]
+            for (int c = 0; c < 4; ++c) mma_low(s, row_split(kp, half, c, lr, lg), qf[c]);       // S^T [key][query]
+            forget_rows();
+#pragma unroll
+            for (int c = 0; c < 4; ++c) mma(s, row_first(kp, half, c, lr, lg), qf[c].p[0]);
             if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4);
             if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0);
             follow_maximum(s, sc, row, o);
@@ -604,7 +615,13 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
             for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
 #pragma unroll
             for (int c = 0; c < 4; ++c)       // S and dP [query][key]
-                mma_two<true>(s, row_split(qp, half, c, lr, lg), kf[c], dp, row_split(dp_, half, c, lr, lg), row_split(vrows[(wave & 3) >> 1], wave & 1, c, lr, lg));
+                mma_two<5, true>(s, row_split(qp, half, c, lr, lg), kf[c], dp, row_split(dp_, half, c, lr, lg), row_split(vrows[(wave & 3) >> 1], wave & 1, c, lr, lg));
+            forget_rows();
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                mma(s, row_first(qp, half, c, lr, lg), kf[c].p[0]);
+                mma(dp, row_first(dp_, half, c, lr, lg), row_first(vrows[(wave & 3) >> 1], wave & 1, c, lr, lg));
+            }
         }
         if (live) {
             if (q0 < kw0 + 31) apply_causal<false>(s, key - q0 - lg * 4);
@@ -760,7 +777,13 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const in
             for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
 #pragma unroll
             for (int c = 0; c < 4; ++c)       // S^T and dP^T [key][query]
-                mma_two(s, row_split(kp, half, c, lr, lg), qf[c], dp, row_split(kp + TILE, half, c, lr, lg), dof[c]);
+                mma_two<5>(s, row_split(kp, half, c, lr, lg), qf[c], dp, row_split(kp + TILE, half, c, lr, lg), dof[c]);
+            forget_rows();
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                mma(s, row_first(kp, half, c, lr, lg), qf[c].p[0]);
+                mma(dp, row_first(kp + TILE, half, c, lr, lg), dof[c].p[0]);
+            }
             if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4);
             if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0);
 #pragma unroll

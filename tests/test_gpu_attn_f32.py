@@ -85,6 +85,22 @@ def test_values_that_are_not_split(mt, T, train, masked):
         assert torch.isfinite(x).all() and (x - y).norm() <= 2e-6 * y.norm(), what
 
 
+def test_sharp_scores_against_the_fp32_instructions(mt):
+    """Scores of nine times the size, whose rounding is what the results' error comes from: 32 roundings of a sum of 64 by the fp32
+    instructions (which take V from 2^32 on), four at full size here.  0.35 of the error as a random walk; 0.6 leaves room for
+    the roundings that both share, and not for six a chunk (24: 0.87)."""
+    T = 192
+    qkv, do, _ = case(4, 12, T, 12)
+    qkv[:, :, :2] *= 3
+    mask = torch.ones(T, T, dtype=torch.bool, device=DEV).tril().expand(4, T, T).contiguous()
+    want = exact(qkv, do, mask)
+    big = qkv.clone()
+    big[:, :, 2] *= 2.0 ** 40
+    for what, x, y, z, e in zip(("o", "dq", "dk", "dv"), both(mt, qkv, do, mask), both(mt, big, do, mask), want, (40, 40, 40, 0)):
+        error = [(v.double().cpu() - z).norm().item() for v in (x, y.double() * 2.0 ** -e)]
+        assert error[0] <= 0.6 * error[1], (what, error)
+
+
 def test_infinite_factors(mt):
     """inf * -inf is -inf: key 10 is as good as hidden from every query, and so is every key from query 70."""
     T = 192
