@@ -179,17 +179,17 @@ constexpr float M_START = -1e8f;          // log2-domain start of the running ma
                                           // (-1.44e9), below every real one, so exp2(masked - m) is exactly 0
 
 // Causal visibility of the lane's 16 elements of a sub-tile written into the raw scores
-// (invisible -> NEG_RAW).
+// (invisible -> `hidden`).
 //   pos0 = (lane's own index) - (first index of the sub-tile along registers) - 4*lg
 //   element i = 4a+b sits at register offset 8a+b: visible iff 8a+b <= pos0 (causal part).
 template <bool LANE_IS_QUERY>
-__device__ __forceinline__ void apply_causal(f32x16& s, int pos0) {
+__device__ __forceinline__ void apply_causal(f32x16& s, int pos0, float hidden = NEG_RAW) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int off = (i >> 2) * 8 + (i & 3);
         // lane = query: key offset must be <= query;  lane = key: query offset must be >= key
         const bool ok = LANE_IS_QUERY ? (off <= pos0) : (off >= pos0);
-        s[i] = ok ? s[i] : NEG_RAW;
+        s[i] = ok ? s[i] : hidden;
     }
 }
 

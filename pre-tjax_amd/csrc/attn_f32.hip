@@ -21,7 +21,13 @@ namespace {
 constexpr int THREADS = 512;
 constexpr int TILE = 3 * PANEL;           // 64 x 64 elements as three panels
 
-// Eight fp32 values as three times eight bf16 values whose sum they are: exact from 2^-109 on, below that to 2^-134.
+// Range, as in gemm_split.h: unscaled, the parts of factors below 2^-109 would leave bf16's range.  Q, K, V, dO and P are split as
+// 2^16 times their value, of which every fp32 number has its three parts exactly; scores, dP and the gradient of V are formed 2^32
+// times their value, dS 2^48 and the gradients of Q and K 2^64, and the powers are taken out where the sums are used.
+constexpr float UP = 0x1p16f, UP2 = 0x1p32f, DOWN = 0x1p-16f, DOWN2 = 0x1p-32f, DOWN4 = 0x1p-64f;
+constexpr float HIDDEN = NEG_RAW * UP2;
+
+// Eight fp32 values as three times eight bf16 values whose sum they are, exactly if none is below 2^-109.
 struct Split8 { bf16x8 p[3]; };
 __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
     typedef float f32x2_t __attribute__((ext_vector_type(2)));
@@ -45,12 +51,15 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
 // Values of the caller, the largest of which is noted: a workgroup that meets one of SPLIT_MOST or more, and a wavefront whose results
 // are not finite, forms them again by the fp32 instructions (plain_fwd, plain_dkdv, plain_dq; 4 times the time).  The parts of an
 // infinity or of what rounds to one are not numbers.  Below SPLIT_MOST no score and no product of dO and V overflows, and what
-// overflows later is seen in the results.
+// overflows later is seen in the results.  The parts are those of UP times the values.
 constexpr float SPLIT_MOST = 0x1p32f;
 __device__ __forceinline__ Split8 split8_noted(const float (&x)[8], float& most) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(x[e]));
-    return split8(x);
+    float up[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) up[e] = x[e] * UP;
+    return split8(up);
 }
 // one multiply-add per value: NaN if one of them is not finite
 template <int N> __device__ __forceinline__ bool finite(const float (&x)[N]) {
@@ -153,14 +162,14 @@ struct TileCopy {
 
 __device__ __forceinline__ uint64_t keep_mask(const KeepWords& w, int i) { return keep_lane_mask_at(w, (i >> 2) * 8 + (i & 3)); }
 
-// The mask words of a mixed tile: hidden elements become NEG_RAW
-__device__ __forceinline__ void apply_mask(f32x16& s, const uint32_t* __restrict__ words) {
+// The mask words of a mixed tile: hidden elements become `hidden`
+__device__ __forceinline__ void apply_mask(f32x16& s, const uint32_t* __restrict__ words, float hidden) {
     const uniform_words mw = as_uniform(words);
     uint32_t w[32];
 #pragma unroll
     for (int t = 0; t < 32; ++t) w[t] = mw[t];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = mask_select(s[i], NEG_RAW, mask_lanes(w, i));
+    for (int i = 0; i < 16; ++i) s[i] = mask_select(s[i], hidden, mask_lanes(w, i));
 }
 
 struct RowStats { float m_run, m_true, l; };      // reference point of the exponentials, true maximum (both base 2), sum
@@ -271,7 +280,7 @@ __device__ __forceinline__ void plain_fwd(const AttnArgs& a, int bh, int qw0, in
         for (int e = 0; e < 16; ++e) s[e] = 0.f;
         plain_rows(s, k + (key0 + lr) * a.k_rs, q_row, lg);
         if (key0 == qw0) apply_causal<true>(s, query - key0 - lg * 4);
-        if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, plain_mask<true>(a, bidx, qw0).words + key0);
+        if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, plain_mask<true>(a, bidx, qw0).words + key0, NEG_RAW);
         follow_maximum(s, sc, row, o);
         KeepWords kw;
         if constexpr (TRAIN) kw = load_keep_half(a.keepbits + (int64_t)bh * a.bitwords, qw0 + key0);
@@ -317,7 +326,7 @@ __device__ __forceinline__ void plain_dkdv(const AttnArgs& a, int bh, int kw0, i
         plain_rows(s, q + (q0 + lr) * a.q_rs, k_row, lg);
         plain_rows(dp, d_o + (q0 + lr) * a.do_rs, v_row, lg);
         if (q0 == kw0) apply_causal<false>(s, key - q0 - lg * 4);
-        if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, plain_mask<false>(a, bidx, kw0).words + q0);
+        if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, plain_mask<false>(a, bidx, kw0).words + q0, NEG_RAW);
         KeepWords kw;
         if constexpr (TRAIN) kw = load_keep_half(a.keepbits + (int64_t)bh * a.bitwords, kw0 + q0);
         // the statistics of query q0 + lr, passed to the lanes that hold elements of its row
@@ -376,7 +385,7 @@ __device__ __forceinline__ void plain_dq(const AttnArgs& a, int bh, int qw0, int
         plain_rows(s, k + (key0 + lr) * a.k_rs, q_row, lg);
         plain_rows(dp, v + (key0 + lr) * a.v_rs, do_row, lg);
         if (key0 == qw0) apply_causal<true>(s, query - key0 - lg * 4);
-        if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, plain_mask<true>(a, bidx, qw0).words + key0);
+        if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, plain_mask<true>(a, bidx, qw0).words + key0, NEG_RAW);
         KeepWords kw;
         if constexpr (TRAIN) kw = load_keep_half(a.keepbits + (int64_t)bh * a.bitwords, qw0 + key0);
         float ds[16];
@@ -424,7 +433,7 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
 
     int nkt = (q0 + 128) / 64;
     if (nkt > a.T / 64) nkt = a.T / 64;
-    const float sc = a.scale * LOG2E;
+    const float sc = a.scale * LOG2E * DOWN2;
     RowStats row = {M_START, M_START, 0.f};
     f32x16 o[2];
 #pragma unroll
@@ -477,8 +486,8 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
             forget_rows();
 #pragma unroll
             for (int c = 0; c < 4; ++c) mma(s, row_first(kp, half, c, lr, lg), qf[c].p[0]);
-            if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4);
-            if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0);
+            if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4, HIDDEN);
+            if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0, HIDDEN);
             follow_maximum(s, sc, row, o);
             float lsum = 0.f;
 #pragma unroll
@@ -486,13 +495,13 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
                 float p[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    p[e] = fast_exp2(fmaf(s[8 * h + e], sc, -row.m_run));
+                    p[e] = fast_exp2(fmaf(s[8 * h + e], sc, -row.m_run)) * UP;
                     lsum += p[e];
                     if constexpr (TRAIN) p[e] = keep_select(p[e], keep_mask(kw, 8 * h + e));
                 }
                 columns_x_regs(o, kp + TILE, split8(p), half, h, lr, lg);
             }
-            row.l += sum_xor32(lsum);
+            row.l += sum_xor32(lsum);         // (UP times the sum)
         }
         if (half == 0 && more) store(kt + 1);
         __syncthreads();
@@ -501,12 +510,13 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
     // Both halves of the keys together; each wavefront finishes the columns of its own half.
     float out[16];
     if (most >= SPLIT_MOST) big = 1;
-    const RowStats r = merge_halves(out, o, row, half, &smem[0][0], wave, wave ^ 4, lane);
+    RowStats r = merge_halves(out, o, row, half, &smem[0][0], wave, wave ^ 4, lane);
     if (qw0 >= a.T) return;
     if (__builtin_expect(big || __any(!finite(out)), 0)) {
         plain_fwd<HAS_MASK, TRAIN>(a, bh, qw0, half);
     } else {
-        store_half_row<float>((float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs + half * 32, out, row_factor<TRAIN>(r.l), lg);
+        r.l *= DOWN;
+        store_half_row<float>((float*)a.out0 + bidx * a.out0_bs + hidx * a.out0_hs + (int64_t)query * a.out0_rs + half * 32, out, row_factor<TRAIN>(r.l) * DOWN2, lg);
         if (lg == 0 && half == 0) store_stats(a, (int64_t)bh * a.T + query, r);
     }
 }
@@ -515,7 +525,7 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_f32_kernel(const AttnArgs
 // One workgroup per (batch-head, 128 keys): wavefront (half, block) owns keys key0 + 32 block .. +31 (lane = key) against the
 // queries of its half of each tile.  delta = rowsum(dO * O) is formed on the rows' way into LDS.  The keys' rows of K wait in
 // registers, those of V in LDS: both in registers spill (8 x 512: 122 us instead of 93).
-typedef float StatTile[3][64];            // m2, 1/l, delta of a query tile
+typedef float StatTile[3][64];            // m2, UP / l, UP2 delta of a query tile
 template <bool HAS_MASK, bool TRAIN>
 __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const int key_tile, char (*smem)[2 * TILE], char (*vrows)[TILE], StatTile* sstat, int& big) {
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
@@ -548,12 +558,12 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
         part += __shfl_xor(part, 1, 64);
         part += __shfl_xor(part, 2, 64);
         part += __shfl_xor(part, 4, 64);
-        if ((tid & 7) == 0) sstat[b][2][tid >> 3] = part;
+        if ((tid & 7) == 0) sstat[b][2][tid >> 3] = part * UP2;
         if (tid < 64) {
             // a row without a visible key (saved l = 0) takes m = 0 and 1/l = 0, which makes its p exactly 0
             const bool none = st_l == 0.f;
             sstat[b][0][tid] = none ? 0.f : st_m * LOG2E;
-            sstat[b][1][tid] = none ? 0.f : 1.0f / st_l;
+            sstat[b][1][tid] = none ? 0.f : UP / st_l;
         }
         cq.store(smem[b], tid, most);
         cd.store(smem[b] + TILE, tid, most);
@@ -573,7 +583,7 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
     store(0);
     __syncthreads();
 
-    const float sc = a.scale * LOG2E;
+    const float sc = a.scale * LOG2E * DOWN2;
     f32x16 dk[2], dv[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -624,9 +634,9 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
             }
         }
         if (live) {
-            if (q0 < kw0 + 31) apply_causal<false>(s, key - q0 - lg * 4);
+            if (q0 < kw0 + 31) apply_causal<false>(s, key - q0 - lg * 4, HIDDEN);
             if (HAS_MASK && cls != TILE_CAUSAL)
-                apply_mask(s, a.mask + (int64_t)a.B * (a.T >> 5) * a.T + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + q0);
+                apply_mask(s, a.mask + (int64_t)a.B * (a.T >> 5) * a.T + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + q0, HIDDEN);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 float pd[8], ds[8];
@@ -681,7 +691,7 @@ __device__ __forceinline__ void bwd_dkdv(const AttnArgs& a, const int bh, const 
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int e = 0; e < 16; ++e) dk[t][e] = take[16 * t + e];
-        store_rows<float>(row, dk, half ? 1.0f : a.scale, lg);
+        store_rows<float>(row, dk, half ? DOWN2 : a.scale * DOWN4, lg);
     }
 }
 
@@ -713,12 +723,12 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const in
 #pragma unroll
         for (int e = 0; e < 4; ++e) delta += x[e] * y[e];
     }
-    delta += xor32(delta);
+    delta = (delta + xor32(delta)) * UP2;
     const int64_t si = (int64_t)bh * a.T + qrow;
     // as in dK/dV: a row without a visible key takes m = 0 and 1/l = 0
     const float lsum = a.ls[si];
     const bool none = lsum == 0.f;
-    const float linv = none ? 0.f : 1.0f / lsum, m2 = none ? 0.f : a.ms[si] * LOG2E;
+    const float linv = none ? 0.f : UP / lsum, m2 = none ? 0.f : a.ms[si] * LOG2E;
     float most = 0.f;
     Split8 qf[4], dof[4];
     load_row_splits(qf, (const float*)a.q + bidx * a.q_bs + hidx * a.q_hs + (int64_t)qrow * a.q_rs, lg, most);
@@ -729,7 +739,7 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const in
 
     int nkt = (q0 + 128) / 64;
     if (nkt > a.T / 64) nkt = a.T / 64;
-    const float sc = a.scale * LOG2E;
+    const float sc = a.scale * LOG2E * DOWN2;
     f32x16 dq[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -784,8 +794,8 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const in
                 mma(s, row_first(kp, half, c, lr, lg), qf[c].p[0]);
                 mma(dp, row_first(kp + TILE, half, c, lr, lg), dof[c].p[0]);
             }
-            if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4);
-            if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0);
+            if (key0 + 31 > qw0) apply_causal<true>(s, query - key0 - lg * 4, HIDDEN);
+            if (HAS_MASK && cls != TILE_CAUSAL) apply_mask(s, a.mask + ((int64_t)bidx * (a.T >> 5) + (lookup >> 5)) * a.T + key0, HIDDEN);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 float ds[8];
@@ -813,7 +823,7 @@ __device__ __forceinline__ void bwd_dq(const AttnArgs& a, const int bh, const in
     if (qw0 >= a.T) return;
     if (__builtin_expect(big || __any(!finite(take)), 0)) plain_dq<HAS_MASK, TRAIN>(a, bh, qw0, half);
     else
-        store_half_row<float>((float*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs + half * 32, take, a.scale, lg);
+        store_half_row<float>((float*)a.out2 + bidx * a.out2_bs + hidx * a.out2_hs + (int64_t)query * a.out2_rs + half * 32, take, a.scale * DOWN4, lg);
 }
 
 // grid (B*H, 2 ceil(T/128)): both passes in one launch, the tiles with the longest way first

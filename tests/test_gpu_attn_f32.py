@@ -101,6 +101,39 @@ def test_sharp_scores_against_the_fp32_instructions(mt):
         assert error[0] <= 0.6 * error[1], (what, error)
 
 
+@pytest.mark.parametrize("train", [False, True])
+def test_tiny_factors(mt, train):
+    """Values of 2^-112, whose lowest parts are below bf16's range unless they are scaled.  Results are linear in V and dO, and with both a
+    power of two smaller they are the same but for roundings below 2^-149 (subnormal ones, of products and of results): 2^-37 of
+    the results each, a few of them a result."""
+    qkv, do, mask = case(1, 2, 192, 9)
+    small = qkv.clone()
+    small[:, :, 2] *= 2.0 ** -112
+    a, b = both(mt, qkv, do, mask, train), both(mt, small, do, mask, train)
+    c = both(mt, qkv, do * 2.0 ** -112, mask, train)
+    for what, x, y in [("o", b[0], a[0]), ("dq", b[1], a[1]), ("dk", b[2], a[2])] + [("do: " + n, x, y) for n, x, y in zip(("dq", "dk", "dv"), c[1:], a[1:])]:
+        assert (x.double() * 2.0 ** 112 - y.double()).norm() <= 2.0 ** -30 * y.double().norm(), what
+
+
+def test_tiny_probabilities(mt):
+    """Every query sees key 0, whose V is 0, and itself with a score 80 lower: O is one product of P = 2^-115, dV of the key one as well.
+    The scores have few bits, so the fp32 instructions (which take V from 2^32 on) multiply the same P where key 0 is in the same 32
+    keys (elsewhere two partial results are put together, whose reference points are rounded)."""
+    T = 128
+    g = gen(10)
+    qkv, do = torch.zeros(1, 1, 3, T, 64), randn(g, 1, 1, T, 64)
+    qkv[:, :, 2, 1:] = randn(g, T - 1, 64)
+    qkv[:, :, 0, :, 0], qkv[:, :, 1, 1:, 0] = 32.0, -20.0
+    mask = torch.eye(T, dtype=torch.bool)
+    mask[:, 0] = True
+    mask, big = mask[None].to(DEV), qkv.clone()
+    big[:, :, 2] *= 2.0 ** 40
+    x, y = both(mt, qkv.to(DEV), do.to(DEV), mask), both(mt, big.to(DEV), do.to(DEV), mask)
+    for what, got, want, n in (("o", x[0].double() * 2.0 ** 40, y[0].double(), 32), ("dv", x[3].double(), y[3].double(), T)):
+        got, want = got[:, :, 1:n], want[:, :, 1:n]
+        assert (want != 0).all() and ((got - want).abs() <= 3 * 2.0 ** -24 * want.abs() + 2.0 ** -148).all(), what
+
+
 def test_infinite_factors(mt):
     """inf * -inf is -inf: key 10 is as good as hidden from every query, and so is every key from query 70."""
     T = 192
