@@ -5,9 +5,9 @@ Reads from LDS by inline assembly are values that the compiler takes to be there
 before the wait that the source puts in front of their use.  And it has left out wait states behind a matrix product where one way
 round a branch is shorter than the other.  Neither shows in a source file, and the results are wrong only now and then.
 
-Rules (quarter-rate issue slots, as s_nop counts them): a result of v_mfma_*_bf16 (8 passes) may be read 12 slots later, of
-v_mfma_f32_32x32x2_f32 (16 passes) 18, and overwritten by the vector ALU one slot earlier (loads take longer than that to arrive);
-the next product is issued when the one before it has gone through its passes.  vmcnt and lgkmcnt count vector memory and LDS
+Rules (quarter-rate issue slots, as s_nop counts them): a result of v_mfma_f32_16x16x32_bf16 (4 passes) may be read 8 slots later, of
+v_mfma_f32_32x32x16_bf16 (8 passes) 12, of v_mfma_f32_32x32x2_f32 (16 passes) 18, and overwritten by the vector ALU one slot earlier
+(loads take longer than that to arrive); the next product is issued when the one before it has gone through its passes.  vmcnt and lgkmcnt count vector memory and LDS
 operations, which complete in order; scalar loads complete in any order.  What the vector ALU writes may be read across lanes
 (DPP, permlane) 2 slots later and, from a scalar register, by a memory address 5 slots later."""
 import concurrent.futures
@@ -66,7 +66,7 @@ class Instruction:
         if op.startswith("v_writelane"):
             into = into + out
         if op.startswith("v_mfma"):
-            self.passes = 8 if "bf16" in op else 16
+            self.passes = {"v_mfma_f32_16x16x32_bf16": 4, "v_mfma_f32_32x32x16_bf16": 8, "v_mfma_f32_32x32x2_f32": 16}[op]
             self.factors = registers(operands[1]) + registers(operands[2])
         self.out, self.into = out, into
         self.vector_alu = op.startswith("v_") and not self.passes
@@ -119,7 +119,7 @@ def findings(listing):
         recent = {r: e + x.slots for r, e in recent.items()
                    if e + x.slots < (5 if r[0] == "s" else 2) and not (x.op.startswith("s_") and r in x.out)}
         if x.passes:
-            products.update({r: (0, x.passes, 12 if x.passes == 8 else 18) for r in x.out})
+            products.update({r: (0, x.passes, {4: 8, 8: 12, 16: 18}[x.passes]) for r in x.out})
         elif x.vector_alu:
             recent.update({r: 0 for r in x.out})
         return loads, products, recent
@@ -228,5 +228,10 @@ def test_the_check_finds_what_is_missing():
     assert findings(good) == []
     for i, worse in ((4, None), (9, "s_nop 9"), (13, "s_waitcnt vmcnt(2)"), (13, None), (16, "s_nop 3"), (19, "s_nop 0"), (21, "s_nop 0")):
         assert findings(good[:i] + ([worse] if worse else []) + good[i + 1:]), (good[i], worse)
+    # the shorter product: 8 slots, and one behind another leaves after 4 passes, not after 8
+    short = "v_mfma_f32_16x16x32_bf16 v[%d:%d], v[4:7], v[8:11], 0"
+    for slots, lines in ((8, [short % (16, 19)]), (4, [short % (16, 19), short % (20, 23)]), (8, ["v_mfma_f32_32x32x16_bf16 v[32:47], v[4:7], v[8:11], 0", short % (16, 19)])):
+        for missing in (0, 1):
+            assert bool(findings(lines + ["s_nop %d" % (slots - 1 - missing), "v_mov_b32_e32 v2, v16", "s_endpgm"])) == bool(missing), (slots, lines, missing)
     # a copy of what is still on its way, in front of the wait
     assert findings(good[:4] + ["v_mov_b64_e32 v[20:21], v[4:5]"] + good[4:])
