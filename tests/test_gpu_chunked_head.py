@@ -167,3 +167,11 @@ def test_accuracy_of_argmax(lo, monkeypatch, B, T, share):
     want = lo.accuracy_from_pred(labels, pred)
     assert got.shape == want.shape and got.dtype == want.dtype
     assert torch.equal(got, want) or (share < 1 and got.isnan() and want.isnan())
+
+
+def test_accuracy_of_another_device(lo, monkeypatch):
+    """Labels that lie on another device than the current one are counted by tensor operations, which go where their operands are."""
+    labels = torch.tensor([[0, 3, 4, 5]], device="cuda")
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: labels.get_device() + 1)
+    monkeypatch.setattr(lo, "stream", lambda: pytest.fail("launched on the current device"))
+    assert lo.accuracy_from_pred(labels, torch.tensor([[0, 3, 7, 5]], device="cuda")).item() == pytest.approx(2 / 3)
