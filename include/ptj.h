@@ -403,6 +403,11 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* shape, const void* const* params, const u
                  const void* acts, size_t acts_bytes, const void* x_last, const void* dh, void* const* grads, void* demb,
                  void* workspace, size_t workspace_bytes, void* stream);
 
+/* What ptj_gpt2_bwd does in bf16 with the two products of a linear layer [n, m] = [n, k] . [m, k]^T (host only; for tests and
+ * profiles): 0 two launches, else one, 1 + 3 * i + j with tiles i for dX and j for dW out of 0: 64x64, 1: 64x128, 2: 128x128, and
+ * whether dW's come first.  `multiplied`: dX with a multiplier.  Negative: PTJ_ERR_INVALID. */
+int ptj_linear_bwd_choice(int64_t n, int64_t m, int64_t k, int multiplied, int* dw_first);
+
 #ifdef __cplusplus
 }
 #endif

@@ -66,6 +66,7 @@ SIGNATURES = {
     "ptj_gpt2_workspace_bytes": (_sz, [_p, _int]),
     "ptj_gpt2_fwd": (_int, [_p, _p, _p, _p, _p, _p, _sz, _int, _p, _p, _p, _sz, _p]),
     "ptj_gpt2_bwd": (_int, [_p, _p, _p, _p, _p, _sz, _p, _p, _p, _p, _p, _sz, _p]),
+    "ptj_linear_bwd_choice": (_int, [_i64, _i64, _i64, _int, _c.POINTER(_int)]),
     "ptj_attn_bwd": (_int, [_p] * 11 + [_p, _sz] + [_i64] * 28 + [_int, _i64, _int, _p]),
 }
 

@@ -67,6 +67,12 @@ constexpr PairCost PAIR_COST[4] = {{}, {0.21, 1.75, 0.31, 0.88}, {0.19, 1.59, 0.
 constexpr double PAIR_START = 3.2, PAIR_MUL = 0.48, PAIR_ROUNDS = 0.55, SEPARATE = 0.95, SEPARATE_MUL = 1.22;
 constexpr double PAIR_ALONE = 0.84;                       // wide tiles, one a CU because of the small ones beside them
 constexpr double PAIR_SHARED = 2.01, PAIR_FLOWS = 0.7;    // wide tiles, two a CU: where one ends early, the other goes on faster
+// Layers narrower than the fitted ones: few tiles share a panel and dW's chain of n / 64 steps is what the pair waits for, 0.20-0.25 us a step
+// where the fit has 0.18.  256 wide, two launches / the pair that the fit alone took, us: ffn2 12288 tokens 38.3 / 52.9, ffn1 8192 22.2 / 29.8,
+// qkv 6000 18.9 / 20.8; 320 wide, ffn2 6000 32.2 / 41.4, 8192 38.1 / 49.7.  Over widths of 256 to 2048 and 256 to 12288 tokens the pick is then 2.6 %
+// slower than the best choice on average (256 wide 3.0, 4.6 without it), the picks of the estimate of gemm_plan 5.9 %.
+constexpr double PAIR_NARROW = 0.3;
+constexpr int64_t PAIR_FITTED = 768;
 
 double pair_us(const PtjLinearBwd& p, int ix, int iw, int cus, bool* dw_first) {
     const TileCost &cx = GT_COST[0][ix], &cw = GT_COST[0][iw];
@@ -80,12 +86,14 @@ double pair_us(const PtjLinearBwd& p, int ix, int iw, int cus, bool* dw_first) {
         const double step = c.step * (1.0 + (busy > 0.5 ? c.crowd * 2.0 * (busy - 0.5) : 0.0)) * (dw ? c.dw : 1.0);
         return (double)gp_ceil(k, GT_COST[0][i].bkt) * step * (i == 2 && !two ? PAIR_ALONE : shared) + c.finish;
     };
+    const int64_t width = p.m < p.k ? p.m : p.k;
+    const double narrow = 1.0 + (width < PAIR_FITTED ? PAIR_NARROW * (double)(PAIR_FITTED - width) / 512.0 : 0.0);
     const double tx = tile(ix, p.m, false) + (p.mul ? PAIR_MUL : 0.0), tw = tile(iw, p.n, true);
     *dw_first = tw > tx;
-    if (all <= slots) return PAIR_START + (tw > tx ? tw : tx);
+    if (all <= slots) return (PAIR_START + (tw > tx ? tw : tx)) * narrow;
     double t = tw > tx ? pair_makespan(nw, tw, nx, tx, slots) : pair_makespan(nx, tx, nw, tw, slots);
     if (two) t += PAIR_FLOWS * (((double)nx * tx + (double)nw * tw) / (double)slots - t);
-    return (PAIR_START + t) * (1.0 + PAIR_ROUNDS * (1.0 - (double)slots / (double)all));
+    return (PAIR_START + t) * (1.0 + PAIR_ROUNDS * (1.0 - (double)slots / (double)all)) * narrow;
 }
 
 double single_us(int64_t n, int64_t m, int64_t k, bool may_split, int cus) {
@@ -164,4 +172,14 @@ int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, i
         return ptj_gemm_mul_colsum_later(p.d, p.w, p.mul, p.dx, p.colsum, n, k, m, m, 1, k, 1, k, k, p.colpart,
                                          ptj_gemm_mul_colsum_workspace_bytes(n, k), scratch, scratch_bytes, dtype, later, st);
     return ptj_gemm(p.d, p.w, p.dx, nullptr, n, k, m, m, 1, k, 1, k, PTJ_EPI_NONE, nullptr, 0, scratch, scratch_bytes, dtype, st);
+}
+
+extern "C" int ptj_linear_bwd_choice(int64_t n, int64_t m, int64_t k, int multiplied, int* dw_first) {
+    PTJ_CHECK_ARG(n >= 1 && m >= 1 && k >= 1 && n < (1 << 20) && m < (1 << 20) && k < (1 << 20) && dw_first, "linear_bwd_choice: bad shape");
+    PtjLinearBwd p{};
+    p.n = n; p.m = m; p.k = k;
+    if (multiplied) p.mul = dw_first;      // (looked at for null only)
+    const PairChoice c = choose_pair(p);
+    *dw_first = c.dw_first;
+    return c.config;
 }
