@@ -92,13 +92,17 @@ def test_native_stack_adds_up_partial_products(mt, lo, monkeypatch, dtype, D, F,
         assert torch.equal(runs[0], runs[1]), (train, odd)
 
 
-# rows that make between half a round and three rounds of tiles, all but one with a tile that ends inside: dX first and dW first,
-# and tiles of 64x64, 64x128 and 128x128 for either
-@pytest.mark.parametrize("B,T", [(1, 576), (5, 192), (5, 384), (7, 448), (13, 320), (6, 1024), (11, 576)])
-def test_native_stack_pairs(mt, lo, monkeypatch, B, T):
+# (D, B, T): rows that make between half a round and three rounds of tiles, many with a tile that ends inside.  Every pair of tiles,
+# for dX with and without a multiplier, with dX first and with dW first (test_pair_choice.py holds the list to that)
+PAIRS = [(768, 1, 576), (768, 5, 192), (768, 5, 384), (768, 7, 448), (768, 13, 320), (768, 6, 1024), (768, 11, 576),
+         (320, 1, 64), (320, 2, 128), (320, 1, 448), (320, 13, 64), (320, 3, 320)]
+
+
+@pytest.mark.parametrize("D,B,T", PAIRS)
+def test_native_stack_pairs(mt, lo, monkeypatch, D, B, T):
     """The two products of a linear layer's backward in one launch, either one first, against the single calls; bound as above (one
     block, so no more than six stored tensors between any two products)."""
-    V, D, L, H, F = 101, 768, 1, 12, 3072
+    V, L, H, F = 101, 1, D // 64, 4 * D
     params = [[p.to(DEV).to(torch.bfloat16) for p in grp] for grp in ogpt2.init_transformer_gpt2(V, D, L, H, F, T, seed=3)]
     y = torch.randint(0, V, (B, T + 1), generator=torch.Generator().manual_seed(7)).to(DEV)
     runs = []

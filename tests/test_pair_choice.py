@@ -4,11 +4,24 @@ import importlib
 
 import pytest
 
+from test_gpu_native_stack import PAIRS
+
+LAYERS = ((1, 4, True), (4, 1, False), (1, 1, False), (3, 1, False))      # outputs and inputs in widths; dX multiplied
+
 
 def choice(n, m, k, multiplied):
     first = ctypes.c_int(-1)
     config = importlib.import_module("pre-tjax_amd._lib").lib().ptj_linear_bwd_choice(n, m, k, int(multiplied), ctypes.byref(first))
     return config, bool(first.value)
+
+
+def test_the_gpu_test_sees_every_pair_of_tiles():
+    """Pairs of equal tiles of 128 x 128 (9), all four of 64 x 64 and 64 x 128 (1, 2, 4, 5), either product first."""
+    seen = {choice(B * T, a * D, b * D, mul) + (mul,) for D, B, T in PAIRS for a, b, mul in LAYERS}
+    for mul in (False, True):
+        assert {c for c, _, m in seen if m == mul} >= {1, 2, 4, 5, 9}
+    for config in (4, 5, 9):
+        assert {first for c, first, _ in seen if c == config} == {False, True}
 
 
 @pytest.mark.parametrize("n,m,k,multiplied", [(12288, 256, 1024, True), (8192, 1024, 256, False), (6000, 768, 256, False),
