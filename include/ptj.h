@@ -163,7 +163,8 @@ int ptj_embed_fwd(const void* wemb, const void* pos, const int64_t* tokens, void
  * ids is summed in that order in fp32, so the result is deterministic. */
 int ptj_embed_bwd(const void* d, const int64_t* sorted_tokens, const int64_t* order, void* dwemb,
                   int64_t n, int64_t dim, int64_t vocab, float scale, int dtype, void* stream);
-/* The same, bit for bit, from the token ids as they are, for n up to 8192. */
+/* The same, bit for bit, from the token ids as they are, for n up to PTJ_EMBED_SCAN_MAX. */
+#define PTJ_EMBED_SCAN_MAX 8192
 int ptj_embed_bwd_tokens(const void* d, const int64_t* tokens, void* dwemb, int64_t n, int64_t dim, int64_t vocab,
                          float scale, int dtype, void* stream);
 
@@ -353,10 +354,10 @@ int ptj_attn_fwd(const void* q, const void* k, const void* v, const uint32_t* ma
 
 /* Flash-attention backward with P recomputed from (ms, ls).  Outputs dq/dk/dv
  * [BH, T, dh] with explicit strides.  Deterministic: dK/dV and dQ are produced by
- * two passes, no atomics (the dQ pass runs first and leaves rowsum(dO*O) in the
- * workspace for the dK/dV pass), so no output may overlap an input.  `workspace`
- * (always required here) holds
- * ptj_attn_workspace_bytes(B, H, T) bytes.  Replaces
+ * two passes, no atomics, so no output may overlap an input.  `workspace`
+ * (always required here) holds ptj_attn_workspace_bytes(B, H, T) bytes: the keep bits, and
+ * rowsum(dO*O), which in bf16 on large grids the dQ pass leaves for the dK/dV pass (elsewhere
+ * formed where it is used, and that part is not touched).  Replaces
  * t_scaled_dot_prod_attn_bkwd3_k/_t (model_triton.py:829-1003). */
 int ptj_attn_bwd(const void* d_o, const void* q, const void* k, const void* v, const void* o,
                  const float* ms, const float* ls, const uint32_t* mask,

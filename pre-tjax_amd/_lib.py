@@ -12,6 +12,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libptj.so")
 
 PTJ_F32, PTJ_BF16 = 0, 1
+EMBED_SCAN_MAX = 8192     # PTJ_EMBED_SCAN_MAX
 EPI_NONE, EPI_BIAS, EPI_BIAS_GELU, EPI_BIAS_GELU_DERIV, EPI_ACCUMULATE = 0, 1, 2, 3, 4
 
 _c = ctypes

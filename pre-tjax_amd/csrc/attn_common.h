@@ -14,7 +14,7 @@ struct AttnArgs {
     //   then B*(T/32)^2 words:  class of tile (b, q/32, k/32), then the same indexed (b, k/32, q/32)
     const uint32_t* mask;
     float *ms, *ls;               // [BH, T]
-    float* delta;                 // [BH, T] rowsum(dO * O)  (backward in two launches: dQ writes it, dK/dV reads it)
+    float* delta;                 // [BH, T] rowsum(dO * O)  (2-byte storage in two launches: dQ writes it, dK/dV reads it)
     const uint32_t* keepbits;     // [BH, bitwords]  (train)
     int B, H, T, bitwords;
     // element strides: batch, head, row (the head dimension itself has unit stride)
@@ -37,7 +37,6 @@ constexpr int PANEL = 64 * BKB;  // bytes of one 64-row LDS panel of 2-byte elem
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LN2 = 0.6931471805599453f;
 constexpr float NEG_NAT = -1e9f;
-constexpr float NEG2 = NEG_NAT * LOG2E;
 
 // ---- small device helpers -----------------------------------------------------------
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

@@ -1,19 +1,21 @@
 // Causal flash attention of 4-byte storage: the algorithm, layouts, masks and statistics of attn.hip, multiplied on the bf16
 // matrix pipe.
 //
-// Every factor is the exact sum of three bf16 values (Split8), and six products of the parts (those above 2^-26 of the whole)
-// stand for one: 192 clocks per 32x32x16 where the fp32 instructions take 512.  Q, K, V and dO are split once per workgroup on
+// Every factor is the exact sum of three bf16 values (Split8), and six products of the parts stand for one, as in gemm_split.h, which
+// names the method and bounds the other three by 2^-25 |a b| and less: 192 clocks per 32x32x16 where the fp32 instructions take 512.  Q, K, V and dO are split once per workgroup on
 // their way into registers or LDS, P and dS where they are formed.  The parts lie in LDS as bf16 panels, which transposing reads
 // serve in both directions, so no transposed copies exist.
 // What bounds it: the matrix pipe at the clock that the part holds under such load.  Batch 8 x 1024 x 12 heads multiplies at
-// 980 (forward) and 1090 TFLOP/s (backward) of bf16 products, where this repository's fp32 GEMMs reach 1000 to 1290.
+// 940 (forward) and 1075 TFLOP/s (backward) of bf16 products, where this repository's fp32 GEMMs reach 1000 to 1290.
 // Eight wavefronts share a 64-row tile: four blocks of 32 rows x the two halves of the tile, so that two wavefronts per SIMD
 // overlap matrix and vector work, every conversion serves 128 rows, and the way through a row's keys is half as long; the
 // halves' results are added at the end.  The wavefronts of the second half convert the next tile before their products, those of
 // the first half behind them (8 x 1024: backward 283 -> 277 us, forward 94 -> 89).
-// fp32 instructions / this file, us, 12 heads: 8 x 512 forward 58 / 33, backward 150 / 93; 8 x 1024 140 / 89 and 477 / 277;
-// 2 x 256 24 / 15 and 46 / 26.  Error against fp64 (2-norm, 8 x 512): O 2.8e-7 / 1.6e-7, dQ 3.6e-7 / 2.8e-7, dK 5.7e-7 / 3.7e-7,
-// dV 5.6e-7 / 3.5e-7.
+// fp32 instructions / this file, us, 12 heads, causal mask: 8 x 512 forward 58 / 34, backward 149 / 93; 8 x 1024 136 / 93 and 481 / 281;
+// 2 x 256 24 / 16 and 46 / 25; padded documents with dropout 8 x 512 66 / 39 and 152 / 97, 8 x 1024 133 / 91 and 469 / 257.
+// Error against fp64 (2-norm, 8 x 512): O 2.8e-7 / 1.5e-7, dQ 3.6e-7 / 1.9e-7, dK 5.7e-7 / 3.1e-7, dV 5.6e-7 / 3.1e-7.  Rows by the
+// number of their terms (visible keys of a query, queries of a key; T = 64 to 448, scores of N(0, 1) and three times that), as a share of what
+// the fp32 instructions leave: one term 0.7 to 1.1 (above 1 in O alone: a product is rounded once either way), two to 64 terms 0.3 to 0.97.
 #include "attn_common.h"
 
 namespace {

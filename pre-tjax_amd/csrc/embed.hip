@@ -4,11 +4,12 @@
 // the scaling, the position add and the embedding dropout of the model's first step, with
 // the storage rounding after each of them that separate kernels would apply.
 //
-// Backward: dwemb[tok] += scale * sum_{i: token_i = tok} d[i].  The caller passes the
-// token ids sorted (stable) together with the sorting permutation; a workgroup that sits
-// on the first position of a run of equal tokens sums the run's gradient rows in fp32 in
-// sorted order (four row slots folded through LDS in slot order) and updates that table
+// Backward: dwemb[tok] += scale * sum_{i: token_i = tok} d[i].  The workgroup on the first
+// position of a token sums the gradient rows of all its positions in fp32 in order of
+// position (four row slots folded through LDS in slot order) and updates that table
 // row in place, so the result is deterministic and no [vocab, dim] scratch is touched.
+// Up to EMB_SCAN_MAX positions a workgroup finds the equal tokens by comparison; beyond, the
+// caller passes the token ids sorted (stable) together with the sorting permutation.
 #include "common.h"
 
 namespace {
@@ -16,7 +17,7 @@ namespace {
 constexpr int EMB_COLT = 128;            // column threads (one 16-byte vector each per sweep)
 constexpr int EMB_SLOTS = 4;             // row slots of the backward workgroup
 constexpr int EMB_BWD_THREADS = EMB_COLT * EMB_SLOTS;
-constexpr int EMB_SCAN_MAX = 8192;       // positions that embed_bwd_scan_kernel takes
+constexpr int EMB_SCAN_MAX = PTJ_EMBED_SCAN_MAX;       // positions that embed_bwd_scan_kernel takes
 
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void embed_fwd_kernel(const T* __restrict__ wemb, const T* __restrict__ pos,

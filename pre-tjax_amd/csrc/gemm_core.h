@@ -469,10 +469,15 @@ __device__ __forceinline__ void gemm_store_block(const GemmArgs& g, const f32x16
 // lie in groups of tile rows, column by column inside a group.  RING, the walk of gemm_ring.h's large tiles: groups of four rows
 // instead of eight, and XCD x begins x eighths into its range.  32 tiles of an XCD are under way at once; eight columns of four rows
 // make longer pieces of an output row than four columns of eight, and the XCDs, whose ranges are often whole groups, no longer write the same
-// columns at the same time.  Eight rows, all from the start / four, spread, us on one box: 16384x3072x768 with GELU and its
-// derivative 114.3 / 102.3, with bias 80.7 / 77.6, 16384x2304x768 63.5 / 62.5, 8192x2304x768 38.7 / 36.9, 8192x50257x768
-// 634 / 567 (its two gradient products 498 / 501 and 532 / 518).  Eight rows, spread: 103.0, 76.8, 62.1, 36.7, 632; five, spread: 102.4, 78.9, 62.6,
-// 37.0, 638.  Tiles of 128 x 128, which are seldom more than one round: no difference beyond 1 %, they keep eight.
+// columns at the same time.  Eight rows, all from the start / four, spread, us, one after the other on one box: 16384x3072x768 with GELU and
+// its derivative 114.3 / 102.3, with bias 80.7 / 77.6, 16384x2304x768 63.5 / 62.5, 8192x2304x768 38.7 / 36.9, 8192x50257x768
+// 634 / 567 (its two gradient products 498 / 501 and 532 / 518).  With the spread the number of rows matters to very wide outputs alone.
+// Two, three, four, five, six and eight, six of each in turn: 8192x50257x768 588 587 577 630 602 629, 4096x50257 308 302 299 313 305 312,
+// 2048x50257 161 160 159 159 159 177, 8192x35374 421 415 415 438 412 419, 4096x35374 218 214 212 211 208 210; fifteen shapes of 768 to 8192
+// columns and 2048 to 16384 rows, and dW of the head: all six within 1.5 % but one (8192x4096x1024 60.8 60.5 59.6 61.2 60.3 60.0).  Why five
+// and eight are slow there is not known; four is within 2 % of the best in every one.  These are the
+// same product many times in a row; eight calls of the head's behind the other legs of bench.py read 736.
+// Tiles of 128 x 128, which are seldom more than one round: no difference beyond 1 %, they keep eight.
 template <bool RING>
 __device__ __forceinline__ int xcd_range(int pid, int work) {
     const int chunk = work >> 3, rem = work & 7, x = pid & 7, len = chunk + (x < rem);

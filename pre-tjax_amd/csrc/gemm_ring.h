@@ -575,8 +575,8 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
     GtFrag<bf16, BMODE> fb[2][TN];
     f32x4 acc[TN][TM];
     constexpr int NR = TM + TN, NM = TM * TN, NC = PA + PB;   // reads, MFMAs of a set; copies of a step
-    // Reads end a little before the set's last MFMA, so that they have landed by then, and copies a little earlier, so that the
-    // cursors' bookkeeping runs under the last ones and not beside the barrier (8192^3: 783 us, 824 without).
+    // Reads take the first 5/8 of the set's MFMAs, so that they have landed by its end, and copies all but the last four, so that
+    // the cursors' bookkeeping runs under those and not beside the barrier (figures at the top).
     constexpr int READ_SPAN = NM * 5 / 8, COPY_SPAN = NM - 4;
     uint32_t addr_a, addr_b;                   // KMAJOR
     auto read_addresses = [&](auto ch, uint32_t soff_a, uint32_t soff_b) __attribute__((always_inline)) {

@@ -2,8 +2,11 @@
 // also refreshes the low-precision copy the kernels compute with.  HBM-bound: 14 bytes
 // read and 14 written per parameter with bf16 gradients and a bf16 shadow.
 //
-// What is read and written here is not looked at again before the next step: it passes by the caches (non-temporal), but for
-// the shadow, which the next forward reads.  One vector per thread, as many workgroups as there are vectors: nothing is gained
+// What is read and written here passes by the caches (non-temporal), but for the shadow, which the next forward reads.  Moments and
+// gradients are not looked at again before the next step.  The master weights are, where there is no shadow (fp32), and stored
+// normally there they save nothing: fp32 steps, past the caches / normally, us: 1 x 64 2774 / 2787, 2 x 256 5753 / 5777, 4 x 256 8021 / 8024,
+// 8 x 512 22998 / 22992, and with sets that the 256 MB last-level cache holds, 4.5 M parameters 4 x 128 722 / 719, 13.8 M 8 x 256 2513 / 2527
+// (all of it through the caches, with loops: 2967, 6252, 8515, 24048, 810, 2760).  One vector per thread, as many workgroups as there are vectors: nothing is gained
 // by a loop.  124 M parameters, bf16 gradients and shadow: 717 -> 645 us (4.8 -> 5.4 TB/s; a 4 GiB copy: 4.95), fp32 718 -> 625;
 // with looping workgroups and non-temporal accesses 660, without them and without a loop 699; two vectors per thread 641.
 // Inside training steps, which find more of their weights in the caches afterwards: 2 x 256 tokens 2841 -> 2697 us, 7 x 448 5767 -> 5633

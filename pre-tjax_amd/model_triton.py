@@ -12,7 +12,7 @@ import math
 import torch
 
 from . import _lib
-from ._lib import check, dtype_code, lib, ptr, require_gpu, stream
+from ._lib import EMBED_SCAN_MAX, check, dtype_code, lib, ptr, require_gpu, stream
 # plain-torch twins of the wrappers (the reference's names without `_t`); not used below
 # except `t_gelu_fwd`, which callers pass as the `activation_fn` marker
 from .spec_torch import (t_dropout_bkwd2, t_dropout_fwd, t_gelu_bkwd2, t_gelu_fwd,  # noqa: F401
@@ -608,9 +608,6 @@ def embed_pos_dropout_t(wemb, pos, y, train=True, p_gen_aux=None):
     check(lib().ptj_embed_fwd(ptr(wc), ptr(pc), ptr(tok), ptr(out), B * T, D, T, V, math.sqrt(D), int(bool(train)),
                               int(p_gen_aux if train else 0), dtype_code(wc), stream()), "ptj_embed_fwd")
     return out
-
-
-EMBED_SCAN_MAX = 8192    # positions up to which the embedding's backward finds equal tokens without a sort
 
 
 def embed_bkwd_add_t(dwemb, d, y):

@@ -26,6 +26,7 @@ def test_header_symbols_exported_and_bound():
     for n in names:
         assert hasattr(l, n), n
     assert _lib.lib().ptj_version() >= 1
+    assert "#define PTJ_EMBED_SCAN_MAX %d\n" % _lib.EMBED_SCAN_MAX in open(os.path.join(ROOT, "include", "ptj.h")).read()
 
 
 def test_argument_errors_do_not_launch():
