@@ -2,11 +2,13 @@
 // matrix pipe.
 //
 // Every factor is the exact sum of three bf16 values (Split8), and six products of the parts stand for one, as in gemm_split.h, which
-// names the method and bounds the other three by 2^-25 |a b| and less: 192 clocks per 32x32x16 where the fp32 instructions take 512.  Q, K, V and dO are split once per workgroup on
-// their way into registers or LDS, P and dS where they are formed.  The parts lie in LDS as bf16 panels, which transposing reads
-// serve in both directions, so no transposed copies exist.
-// What bounds it: the matrix pipe at the clock that the part holds under such load.  Batch 8 x 1024 x 12 heads multiplies at
-// 940 (forward) and 1075 TFLOP/s (backward) of bf16 products, where this repository's fp32 GEMMs reach 1000 to 1290.
+// names the method and bounds the other three by 2^-25 |a b| and less: 192 clocks per 32x32x16 where the fp32 instructions take
+// 512.  Q, K, V and dO are split once per workgroup on their way into registers or LDS, P and dS where they are formed.  The
+// parts lie in LDS as bf16 panels, which transposing reads serve in both directions, so no transposed copies exist.
+// What bounds it: the waits of two wavefronts per SIMD (the registers and, in the backward, 149 KB of LDS allow no third) for LDS,
+// memory and each other, 35 to 48 % of their time.  Forward / backward, matrix pipe and vector ALU busy: batch 8 x 1024 x 12 heads
+// 39 / 45 % and 47 / 39 %, 8 x 512 27 / 33 % and 38 / 35 %, 8 x 512 with padding and dropout 17 / 21 % and 32 / 30 %.  8 x 1024 multiplies at
+// 940 and 1075 TFLOP/s of bf16 products, where this repository's fp32 GEMMs reach 1000 to 1290.
 // Eight wavefronts share a 64-row tile: four blocks of 32 rows x the two halves of the tile, so that two wavefronts per SIMD
 // overlap matrix and vector work, every conversion serves 128 rows, and the way through a row's keys is half as long; the
 // halves' results are added at the end.  The wavefronts of the second half convert the next tile before their products, those of

@@ -1,9 +1,11 @@
 // Persistent bf16 GEMM whose operand panels travel HBM -> LDS by asynchronous buffer copies into two rings,
 // one per operand.  Included by gemm_core.h inside its unnamed namespace, after gemm_tile.h.
 //
-// What bounds it: the power budget, then the feed.  Under this load the part holds 1.5-1.9 GHz, whatever switches is paid for in
-// clock, and the 16x16x32 instructions take less for the same products than the 32x32x16 ones (their accumulators move half as
-// often): alone, with their factors in registers, 2100 against 1850 TFLOP/s.  Per 64 contraction elements a 256x256 tile (eight
+// What bounds it: at long contractions the clock, at K = 768 what a tile does before and behind its loop (below).  Under this load the
+// part holds 1.5-1.9 GHz, whatever switches is paid for in clock, and the 16x16x32 instructions take less for the same products than
+// the 32x32x16 ones (their accumulators move half as often).  Alone, with N(0,1) factors in registers and the matrix pipe 97-99 %
+// busy, they run at 2.03 against 1.77 GHz, 1915 against 1665 TFLOP/s (with equal factors, where little switches, both at 2.35 GHz,
+// 2440); 8192^3 reaches 78 % of that, 16384x3072x768 with bias 52 %.  Per 64 contraction elements a 256x256 tile (eight
 // wavefronts of 128x64) costs 2048 clocks of MFMAs, 1536 of fragment reads and 512 of arriving copies; a 256x192 tile
 // (wavefronts of 64x96) 1536, 1280 and 448, so the wider tile gets more out of the matrix pipe and the narrower one is for
 // outputs that it cuts into fuller rounds (gemm_plan.h).  The A ring has three stages and the B ring two: the chunk
@@ -12,8 +14,8 @@
 // of B.  Reads are spread over the first 5/8 of the MFMAs that they run beside (7/8: 8192^3 763 us instead of 755), copies over all but
 // the last ones (bunched behind the barrier: 5 % slower), and the wavefronts that are past the barrier go first (740).
 // 32x32x16 instructions before / now, us on one box: 8192^3 812 / 740 (1486 TFLOP/s), 8192x50257x768 with bias 683 / 628, its
-// two gradient products 511 / 497 and 535 / 515, 16384x3072x768 with bias 86.9 / 80.4, with GELU and its derivative 118.8 / 113.6,
-// 16384x768x3072 70.3 / 67.3, dX of it 68.9 / 66.4, dW of it 82.6 / 81.9.  (With 32x32x16 the four plain 256x256 kernels spilled 33-50
+// two gradient products 511 / 497 and 535 / 515, 16384x3072x768 with bias 86.9 / 80.4, with GELU and its derivative 118.8 / 113.6
+// (77.6 and 102.3 with the walk of gemm_core.h), 16384x768x3072 70.3 / 67.3, dX of it 68.9 / 66.4, dW of it 82.6 / 81.9.  (With 32x32x16 the four plain 256x256 kernels spilled 33-50
 // registers as well.)  Four wavefronts of 128x128 with one chunk per register set: 905 us for 8192^3 where eight took 783.
 //
 // The output goes straight from the accumulators to memory: a lane swap brings eight consecutive columns of a row
