@@ -135,7 +135,9 @@ __global__ __launch_bounds__(EMB_BWD_THREADS) void embed_bwd_kernel(const T* __r
 // and lists the equal ones, in order of position, in LDS; so the sums are the same bits.  Every token is read n times from L2
 // (8 bytes each, all of a workgroup's at once), where a sort of a few thousand keys is one workgroup's work in several launches.
 // us with the sort / without, 768 columns of bf16, ids as in text: 512 tokens 34.0 / 4.1, 2048 41.8 / 8.4,
-// 4096 58.0 / 19.9, 8192 66.8 / 56.2; it grows with n^2, and beyond that the sort is faster.
+// 4096 58.0 / 19.9, 8192 66.8 / 56.2; it grows with n^2, and beyond that the sort is faster.  With ids drawn evenly, whose workgroups
+// nearly all have a sum of their own, the line lies there: 5000 54.2 / 37.6, 8192 64.3 / 64.2 (fp32 69.6 / 73.1); with half the ids equal,
+// 8192, 228 / 145.
 template <typename T, int VEC, int PER>
 __global__ __launch_bounds__(EMB_BWD_THREADS) void embed_bwd_scan_kernel(const T* __restrict__ d, const int64_t* __restrict__ tokens,
                                                                          T* __restrict__ dwemb, int n, int dim, int64_t vocab,
