@@ -167,7 +167,7 @@ __device__ __forceinline__ void store_half_row(T* __restrict__ row, const float 
         store_vec<T, 4>(row + a * 8 + lg * 4, v);
     }
 }
-// Class of a 32x32 tile of (mask AND causal), see attn_mask_classes_kernel
+// Class of a 32x32 tile of (mask AND causal), see attn_pack_mask_kernel
 enum { TILE_HIDDEN = 0, TILE_MIXED = 1, TILE_CAUSAL = 2 };
 // ---- element-wise pieces (VALU budget: a wave64 VALU op costs 4 cycles, v_exp 16, and one
 //      K tile gives each lane 32 score elements against 16 MFMAs = 512 cycles; every
