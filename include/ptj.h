@@ -390,8 +390,9 @@ int ptj_attn_bwd(const void* d_o, const void* q, const void* k, const void* v, c
  *   x_last, h   [batch * seq, dim]: the last block's output and its LayerNorm
  * ptj_gpt2_bwd takes dh = the gradient of h and writes grads[3 ..] (entries like `params`; the first
  * three are not touched) and demb [batch * seq, dim] = the gradient of table row + position of every
- * token.  The arithmetic is that of the same sequence of single calls; two
- * products that share a launch may add their contraction in another order. */
+ * token.  The arithmetic is that of the same sequence of single calls; products that share a launch (dX and dW of a layer, or
+ * the weight gradients of several blocks, whose inputs the backward's workspace then keeps) may add their contraction in
+ * another order. */
 typedef struct ptj_gpt2_shape {
     int64_t layers, batch, seq, dim, heads, ffn, vocab, dtype, train;
 } ptj_gpt2_shape;

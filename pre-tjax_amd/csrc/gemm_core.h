@@ -34,6 +34,7 @@
 // split along K across gridDim.z into an fp32 workspace and reduced in fixed order.
 #pragma once
 #include "common.h"
+#include "internal.h"
 #include "mma_tile.h"
 #include <type_traits>
 
@@ -67,6 +68,12 @@ struct GemmArgs {
     int64_t mul_rs;
     float* colpart;
     const char *planes_a, *planes_b;   // gemm_planes.h: the operands' three bf16 parts
+};
+// Products of several blocks that share a launch (internal.h: PtjGradGroup) and, for the tile shape of the launch, the number of
+// tiles in front of each kind inside a block (first[KINDS]: all of a block).
+struct GemmGroup {
+    PtjGradGroup p;
+    int first[PtjGradGroup::KINDS + 1];
 };
 int launch_plain_f32(const GemmArgs& g, int splits, hipStream_t st);   // gemm_f32.hip
 // gemm_tile_bf16.hip, gemm_tile_f32.hip: configuration `cfg` of the one-tile-per-workgroup kernels (gemm_plan.h), with
@@ -497,6 +504,25 @@ __device__ __forceinline__ void tile_walk(int idx, int num_m, int num_n, int& ti
     const int gsz = (num_m - first_m) < GROUP ? (num_m - first_m) : GROUP;
     tile_m = first_m + (idx % width) % gsz;
     tile_n = (idx % width) / gsz;
+}
+// Tile `pid` of a group of products: block after block, so that an XCD's tiles are mostly those of one product.
+template <bool RING>
+__device__ __forceinline__ void group_tile(const ptj_gemm_detail::GemmGroup& g, int pid, int tbm, int tbn, int& kind, int& block, int& tile_m,
+                                           int& tile_n) {
+    const int per = g.first[PtjGradGroup::KINDS], idx = xcd_range<RING>(pid, per * g.p.blocks);
+    block = idx / per;
+    const int r = idx - block * per;
+    kind = 0;
+#pragma unroll
+    for (int i = 1; i < PtjGradGroup::KINDS; ++i) kind += r >= g.first[i];
+    tile_walk<RING>(r - g.first[kind], (g.p.n[kind] + tbm - 1) / tbm, (g.p.m[kind] + tbn - 1) / tbn, tile_m, tile_n);
+}
+template <typename C>
+ptj_gemm_detail::GemmGroup group_of(const PtjGradGroup& p) {
+    ptj_gemm_detail::GemmGroup g = {p, {}};
+    for (int i = 0; i < PtjGradGroup::KINDS; ++i)
+        g.first[i + 1] = g.first[i] + ((p.n[i] + C::TBM - 1) / C::TBM) * ((p.m[i] + C::TBN - 1) / C::TBN);
+    return g;
 }
 // Work item -> origin of its C tile (tile_walk).  RING: of gemm_ring.h's walk.
 template <int TBN = BN, bool RING = false>

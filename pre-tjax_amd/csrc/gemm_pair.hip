@@ -142,7 +142,7 @@ GemmArgs args_of(const void* a, const void* b, void* c, int64_t n, int64_t m, in
 
 int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, int dtype, PtjPartialSums* later, hipStream_t st) {
     const int64_t n = p.n, m = p.m, k = p.k;
-    if (dtype == PTJ_BF16 && n < (1 << 20) && m < (1 << 20) && k < (1 << 20)) {
+    if (dtype == PTJ_BF16 && p.dw && n < (1 << 20) && m < (1 << 20) && k < (1 << 20)) {
         GemmArgs gx = args_of(p.d, p.w, p.dx, n, k, m, m, 1), gw = args_of(p.d, p.x, p.dw, m, k, n, 1, m);
         gx.mul = p.mul; gx.mul_rs = k; gx.colpart = p.colpart;
         if (p.mul) gx.vec_out = gx.vec_out && ptj_aligned16(p.mul);
@@ -166,8 +166,10 @@ int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, i
             return PTJ_OK;
         }
     }
-    int rc = ptj_gemm(p.d, p.x, p.dw, nullptr, m, k, n, 1, m, k, 1, k, PTJ_EPI_NONE, nullptr, 0, scratch, scratch_bytes, dtype, st);
-    if (rc != PTJ_OK) return rc;
+    if (p.dw) {
+        const int rc = ptj_gemm(p.d, p.x, p.dw, nullptr, m, k, n, 1, m, k, 1, k, PTJ_EPI_NONE, nullptr, 0, scratch, scratch_bytes, dtype, st);
+        if (rc != PTJ_OK) return rc;
+    }
     if (p.mul)
         return ptj_gemm_mul_colsum_later(p.d, p.w, p.mul, p.dx, p.colsum, n, k, m, m, 1, k, 1, k, k, p.colpart,
                                          ptj_gemm_mul_colsum_workspace_bytes(n, k), scratch, scratch_bytes, dtype, later, st);

@@ -45,6 +45,7 @@ typedef RingCfg<192, 4, 2> RingNarrow;
 struct RingItem {
     int row0, col0, kbeg, klen, z;
     float* part;
+    int kind, block;      // GemmGroup
 };
 template <typename C>
 __device__ __forceinline__ RingItem ring_item(const GemmArgs& g, int item) {
@@ -65,6 +66,20 @@ __device__ __forceinline__ RingItem ring_item(const GemmArgs& g, int item) {
     d.col0 = tn * C::TBN;
     d.kbeg = d.z * kps;
     d.klen = (d.kbeg + kps < g.k ? d.kbeg + kps : g.k) - d.kbeg;
+    return d;
+}
+
+// The same for a tile of a group of products, whole along the contraction
+template <typename C>
+__device__ __forceinline__ RingItem ring_item(const ptj_gemm_detail::GemmGroup& g, int item) {
+    int tm, tn;
+    RingItem d;
+    group_tile<true>(g, item, C::TBM, C::TBN, d.kind, d.block, tm, tn);
+    d.row0 = tm * C::TBM;
+    d.col0 = tn * C::TBN;
+    d.kbeg = d.z = 0;
+    d.klen = g.p.k;
+    d.part = nullptr;
     return d;
 }
 
@@ -102,17 +117,16 @@ struct RingOperand {
     int64_t left, step;                                                  // bytes from there to the operand's end; per stage
     int item, kleft, slot;                                               // kleft: contraction elements of the item not yet requested
 
-    __device__ __forceinline__ void init(int64_t s_row, int64_t s_k, uint32_t region, int wrow, int tid) {
+    // where the lane's copies come from, by the operand's strides
+    __device__ __forceinline__ void source(int64_t s_row, int64_t s_k, int tid) {
         const int lane = tid & 63;
         if constexpr (MODE == KMAJOR) {
-            const int r = tid >> 3, row = wrow + (lane & 15);
+            const int r = tid >> 3;
             kk = ((lane & 7) ^ ring_sw(r)) * 8;
             voff[0] = ((uint32_t)r * (uint32_t)s_row + (uint32_t)kk) * 2u;
             istep = NW * 8 * (uint32_t)s_row * 2u;
             step = 128;
-            raddr[0] = region + row * BKB + (((lane >> 4) ^ ring_sw(row)) << 4);
         } else {
-            const int l16 = lane & 15, kf = 8 * (lane >> 4) + (l16 >> 2);
             kk = 0;
 #pragma unroll
             for (int i = 0; i < (EVEN ? 1 : PER); ++i) {
@@ -121,6 +135,16 @@ struct RingOperand {
             }
             istep = NW * 64 / PPR * (uint32_t)s_k * 2u;
             step = 128 * s_k;
+        }
+    }
+    __device__ __forceinline__ void init(int64_t s_row, int64_t s_k, uint32_t region, int wrow, int tid) {
+        source(s_row, s_k, tid);
+        const int lane = tid & 63;
+        if constexpr (MODE == KMAJOR) {
+            const int row = wrow + (lane & 15);
+            raddr[0] = region + row * BKB + (((lane >> 4) ^ ring_sw(row)) << 4);
+        } else {
+            const int l16 = lane & 15, kf = 8 * (lane >> 4) + (l16 >> 2);
 #pragma unroll
             for (int t = 0; t < NADDR; ++t) {
                 const int piece = (wrow >> 3) + 2 * t + ((l16 & 3) >> 1);
@@ -489,16 +513,20 @@ __device__ __forceinline__ void ring_load_c(const GemmArgs& g, f32x4 (&acc)[C::T
 // The kernel's arguments, read again from where the launch left them: what only the start and the end of a tile need holds
 // no scalar registers through the main loop.  (One kernel for all epilogues had 60 to 90 of them spilled otherwise and took
 // 100 us instead of 80 for 16384x3072x768.)
-__device__ __forceinline__ const GemmArgs& ring_args() {
-    auto p = (const __attribute__((address_space(4))) GemmArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+template <typename ARGS = GemmArgs>
+__device__ __forceinline__ const ARGS& ring_args() {
+    auto p = (const __attribute__((address_space(4))) ARGS*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(p));
-    return *(const GemmArgs*)p;
+    return *(const ARGS*)p;
 }
 
 constexpr int clip(int x, int most) { return x < most ? x : most; }
 
-template <int AMODE, int BMODE, typename C, bool MUL>
-__global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs) {
+// ARGS: GemmArgs, or GemmGroup (plain products of two MNMAJOR operands)
+template <int AMODE, int BMODE, typename C, bool MUL, typename ARGS = GemmArgs>
+__global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const ARGS) {
+    constexpr bool GROUP = !std::is_same<ARGS, GemmArgs>::value;
+    static_assert(!GROUP || (AMODE == MNMAJOR && BMODE == MNMAJOR && !MUL), "layouts of a group");
     constexpr int TMW = C::TMW, TNW = C::TNW, TM = C::TM, TN = C::TN, NA = C::NA, NB = C::NB;
     __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -514,23 +542,43 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
     constexpr int PA = OA::PER, PB = OB::PER;
     OA oa;
     OB ob;
-    auto start_a = [&](const GemmArgs& g, const RingItem& it) __attribute__((always_inline)) {
-        oa.start(g.a, g.a_row, g.a_k, it.row0, g.n, it.kbeg, it.klen, g.k);
+    auto start_a = [&](const ARGS& g, const RingItem& it) __attribute__((always_inline)) {
+        if constexpr (GROUP) {
+            const int n = g.p.n[it.kind];
+            oa.source(1, n, fresh_tid());
+            oa.start(g.p.d[it.kind][it.block], 1, n, it.row0, n, 0, it.klen, it.klen);
+        } else {
+            oa.start(g.a, g.a_row, g.a_k, it.row0, g.n, it.kbeg, it.klen, g.k);
+        }
     };
-    auto start_b = [&](const GemmArgs& g, const RingItem& it) __attribute__((always_inline)) {
-        ob.start(g.b, g.b_row, g.b_k, it.col0, g.m, it.kbeg, it.klen, g.k);
+    auto start_b = [&](const ARGS& g, const RingItem& it) __attribute__((always_inline)) {
+        if constexpr (GROUP) {
+            const int m = g.p.m[it.kind];
+            ob.source(1, m, fresh_tid());
+            ob.start(g.p.x[it.kind][it.block], 1, m, it.col0, m, 0, it.klen, it.klen);
+        } else {
+            ob.start(g.b, g.b_row, g.b_k, it.col0, g.m, it.kbeg, it.klen, g.k);
+        }
     };
     int item = blockIdx.x;
     RingItem cur;
     {
-        const GemmArgs& g = ring_args();
-        const int total = ((g.n + C::TBM - 1) / C::TBM) * ((g.m + C::TBN - 1) / C::TBN);
-        work = g.tail_splits > 1 ? g.tail_first + (total - g.tail_first) * g.tail_splits : total * g.splits;
-        end_k = g.k;
-        ragged = g.k % 8 != 0 && (AMODE == KMAJOR || BMODE == KMAJOR);
+        const ARGS& g = ring_args<ARGS>();
         cur = ring_item<C>(g, item);
-        oa.init(g.a_row, g.a_k, gt_lds_addr(ring_a), wm * TMW * 32, tid);
-        ob.init(g.b_row, g.b_k, gt_lds_addr(ring_b), wn * TNW * 32, tid);
+        if constexpr (GROUP) {
+            work = g.first[PtjGradGroup::KINDS] * g.p.blocks;
+            end_k = g.p.k;
+            ragged = false;
+            oa.init(1, 0, gt_lds_addr(ring_a), wm * TMW * 32, tid);
+            ob.init(1, 0, gt_lds_addr(ring_b), wn * TNW * 32, tid);
+        } else {
+            const int total = ((g.n + C::TBM - 1) / C::TBM) * ((g.m + C::TBN - 1) / C::TBN);
+            work = g.tail_splits > 1 ? g.tail_first + (total - g.tail_first) * g.tail_splits : total * g.splits;
+            end_k = g.k;
+            ragged = g.k % 8 != 0 && (AMODE == KMAJOR || BMODE == KMAJOR);
+            oa.init(g.a_row, g.a_k, gt_lds_addr(ring_a), wm * TMW * 32, tid);
+            ob.init(g.b_row, g.b_k, gt_lds_addr(ring_b), wn * TNW * 32, tid);
+        }
         oa.item = ob.item = item;
         start_a(g, cur);
         start_b(g, cur);
@@ -548,7 +596,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
             if (__builtin_expect(oa.kleft <= 0 && oa.item < work, 0)) {
                 oa.item += (int)gridDim.x;
                 if (oa.item < work) {
-                    const GemmArgs& g = ring_args();
+                    const ARGS& g = ring_args<ARGS>();
                     start_a(g, ring_item<C>(g, oa.item));
                 }
             }
@@ -565,7 +613,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
             if (__builtin_expect(ob.kleft <= 0 && ob.item < work, 0)) {
                 ob.item += (int)gridDim.x;
                 if (ob.item < work) {
-                    const GemmArgs& g = ring_args();
+                    const ARGS& g = ring_args<ARGS>();
                     start_b(g, ring_item<C>(g, ob.item));
                 }
             }
@@ -638,7 +686,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
     // the accumulators of a tile start from the bias, requested before the write-back of the tile before it
     Pack<bf16, 4> bias[TN];
     auto load_bias = [&](const RingItem& it) __attribute__((always_inline)) {
-        if constexpr (!MUL) {
+        if constexpr (!MUL && !GROUP) {
             const GemmArgs& g = ring_args();
             if (g.bias != nullptr && g.epilogue != PTJ_EPI_NONE && g.splits == 1 && it.part == nullptr) {
                 ring_load_bias<C>(g, bias, it.col0 + wn * TNW * 32);
@@ -669,7 +717,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
             for (int j = 0; j < TM; ++j)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[i][j][e] = to_f32(bias[i].v[e]);
-        if constexpr (!MUL) {
+        if constexpr (!MUL && !GROUP) {
             const GemmArgs& g = ring_args();
             if (g.epilogue == PTJ_EPI_ACCUMULATE) ring_load_c<C>(g, acc, cur.row0 + wm * TMW * 32, cur.col0 + wn * TNW * 32);
         }
@@ -685,7 +733,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
                 // the next step ends the contraction: the last one of this item, or the only one of the next
                 int end = kt + 128 >= cur.klen && kt + 64 < cur.klen && cur.kbeg + cur.klen == end_k ? cur.klen : 0;
                 if (kt + 64 >= cur.klen && more) {
-                    const RingItem n = ring_item<C>(ring_args(), nitem);
+                    const RingItem n = ring_item<C>(ring_args<ARGS>(), nitem);
                     end = n.klen <= 64 && n.kbeg + n.klen == end_k ? n.klen : 0;
                 }
                 if (end > 0) clear_tails(end);
@@ -693,13 +741,19 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_ring_kernel(const GemmArgs
             phase(I1, I0, YES, sa, sb);
         }
         const int row0 = cur.row0 + wm * TMW * 32, col0 = cur.col0 + wn * TNW * 32;
-        const GemmArgs& g = ring_args();
+        const ARGS& g = ring_args<ARGS>();
         RingItem nxt = cur;
         if (more) {
             nxt = ring_item<C>(g, nitem);
             load_bias(nxt);
         }
-        if constexpr (MUL) {
+        if constexpr (GROUP) {
+            GemmArgs out{};
+            out.n = g.p.n[cur.kind];
+            out.m = g.p.m[cur.kind];
+            out.vec_out = 1;
+            ring_write<C, RING_RAW>(out, acc, (bf16*)g.p.dw[cur.kind][cur.block], out.m, nullptr, 0, row0, col0);
+        } else if constexpr (MUL) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the reads that they are read again for)
             landed(I0);
             ring_write_mul<C>(g, acc, row0, col0);
@@ -763,5 +817,16 @@ int ring_launch(const GemmArgs& g, int am, int bm, hipStream_t st) {
         if (g.splits > 1 && !g.leave_partials) return launch_splitk_reduce<bf16>(g, g.splits, st);
         if (g.tail_splits > 1) return launch_tail_reduce<bf16, C::TBN, true>(g, (int)total, st);
     }
+    return PTJ_OK;
+}
+
+// The products of a group, whole tiles of each
+template <typename C>
+int ring_group_launch(const PtjGradGroup& p, hipStream_t st) {
+    const ptj_gemm_detail::GemmGroup g = group_of<C>(p);
+    const int work = g.first[PtjGradGroup::KINDS] * p.blocks, cus = num_cus();
+    hipLaunchKernelGGL((gemm_ring_kernel<MNMAJOR, MNMAJOR, C, false, ptj_gemm_detail::GemmGroup>), dim3((unsigned)(work < cus ? work : cus)),
+                       dim3(C::THREADS), 0, st, g);
+    PTJ_CHECK_LAUNCH();
     return PTJ_OK;
 }

@@ -247,15 +247,11 @@ __device__ __forceinline__ void gs_finish(const GemmArgs& g, f32x16 (&acc)[C::TN
 }
 
 template <int AMODE, int BMODE, typename C, bool MUL>
-__global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(const GemmArgs g) {
+__device__ __forceinline__ void gs_tile(const GemmArgs& g, int tile_m, int tile_n, int z, char* smem) {
     constexpr int BK = 32, TMW = C::TMW, TNW = C::TNW;
-    __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / C::WN, wn = wave - wm * C::WN;
-    const int num_m = (g.n + C::TBM - 1) / C::TBM, num_n = (g.m + C::TBN - 1) / C::TBN;
-    int tile_m, tile_n, z;
-    gt_item(g, blockIdx.x, num_m, num_n, tile_m, tile_n, z);
     const int row0 = tile_m * C::TBM, col0 = tile_n * C::TBN;
     const int kbeg = z * g.k_per_split;
     const int kend = g.splits > 1 && kbeg + g.k_per_split < g.k ? kbeg + g.k_per_split : g.k;
@@ -363,6 +359,41 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
         else all_steps(ANY);
     }
     gs_finish<C, MUL>(g, acc, low, smem, row0, col0, z, kbeg, kend, wave, wm, wn, lane);
+}
+
+template <int AMODE, int BMODE, typename C, bool MUL>
+__global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(const GemmArgs g) {
+    __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
+    int tile_m, tile_n, z;
+    gt_item(g, blockIdx.x, (g.n + C::TBM - 1) / C::TBM, (g.m + C::TBN - 1) / C::TBN, tile_m, tile_n, z);
+    gs_tile<AMODE, BMODE, C, MUL>(g, tile_m, tile_n, z, smem);
+}
+
+// A tile of a group of products
+template <typename C>
+__global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_group_kernel(const ptj_gemm_detail::GemmGroup group) {
+    __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
+    int kind, block, tile_m, tile_n;
+    group_tile<false>(group, blockIdx.x, C::TBM, C::TBN, kind, block, tile_m, tile_n);
+    GemmArgs g{};
+    g.a = group.p.d[kind][block];
+    g.b = group.p.x[kind][block];
+    g.c = group.p.dw[kind][block];
+    g.n = group.p.n[kind];
+    g.m = group.p.m[kind];
+    g.k = g.k_per_split = group.p.k;
+    g.a_row = g.b_row = 1;
+    g.a_k = g.n;
+    g.b_k = g.c_rs = g.m;
+    g.splits = g.tail_splits = g.vec_out = 1;
+    gs_tile<MNMAJOR, MNMAJOR, C, false>(g, tile_m, tile_n, 0, smem);
+}
+template <typename C>
+int gs_group_launch(const PtjGradGroup& p, hipStream_t st) {
+    const ptj_gemm_detail::GemmGroup g = group_of<C>(p);
+    hipLaunchKernelGGL((gemm_split_group_kernel<C>), dim3((unsigned)(g.first[PtjGradGroup::KINDS] * p.blocks)), dim3(C::THREADS), 0, st, g);
+    PTJ_CHECK_LAUNCH();
+    return PTJ_OK;
 }
 
 template <typename C, bool MUL>

@@ -74,14 +74,41 @@ size_t gemm_scratch(const ptj_gpt2_shape& s, bool backward) {
 
 // Temporaries of the two directions in front of the scratch area that the single steps share.
 struct Temps {
-    int64_t t1, df1, dqkv, dxm, dm, dx[2], dr[2], delta, ln_parts, mul_parts, scratch;   // partial rows: one slot per sum
+    int64_t t1, dxm, dx[2], delta, ln_parts, mul_parts, scratch;   // partial rows: one slot per sum
+    int64_t group;                            // blocks whose weight gradients share a launch (0: each with its dX)
+    int64_t df1, dqkv, dm, block;             // what a block's weight gradients read, and from one block's to the next
+    int64_t dr, dr_slots;                     // the gradient that enters a block, dropped
     size_t ln_slot, mul_slot, scratch_bytes, total;
 };
-Temps make_temps(const ptj_gpt2_shape& s, bool backward) {
+
+// The weight gradients of a block: d^T.x with d [tokens, outputs], x [tokens, inputs]
+enum { W_FFN2, W_FFN1, W_OUT, W_QKV };
+PtjGradGroup grad_group(const ptj_gpt2_shape& s, int64_t blocks) {
+    PtjGradGroup g = {};
+    g.k = (int)(s.batch * s.seq);
+    g.blocks = (int)blocks;
+    const int64_t D = s.dim, F = s.ffn, n[4] = {D, F, D, 3 * D}, m[4] = {F, D, D, D};
+    for (int i = 0; i < PtjGradGroup::KINDS; ++i) {
+        g.n[i] = (int)n[i];
+        g.m[i] = (int)m[i];
+    }
+    return g;
+}
+// How many blocks' weight gradients are formed in one launch: all of them, in equal parts of up to PtjGradGroup::BLOCKS, where
+// such a part has a round of tiles (gemm_group.hip), else 0.  A single block stays with the pairs: a round of its tiles takes a width of 1024.
+int64_t grad_group_blocks(const ptj_gpt2_shape& s) {
+    const int64_t N = s.batch * s.seq, D = s.dim, F = s.ffn, most = 1 << 20;
+    if (s.layers < 2 || N >= most || F >= most || 3 * D >= most || F % 8 != 0) return 0;
+    const int64_t parts = (s.layers + PtjGradGroup::BLOCKS - 1) / PtjGradGroup::BLOCKS, blocks = (s.layers + parts - 1) / parts;
+    return ptj_weight_grads_fill(grad_group(s, blocks), (int)s.dtype) ? blocks : 0;
+}
+
+// `together`: weight gradients in groups where grad_group_blocks says so
+Temps make_temps(const ptj_gpt2_shape& s, bool backward, bool together = true) {
     // the split counts behind the scratch size take some twenty estimates: kept for the shape asked for last
-    static thread_local ptj_gpt2_shape last[2] = {};
-    static thread_local Temps kept[2] = {};
-    const int dir = backward ? 1 : 0;
+    static thread_local ptj_gpt2_shape last[3] = {};
+    static thread_local Temps kept[3] = {};
+    const int dir = backward ? 1 + together : 0;
     if (memcmp(&last[dir], &s, sizeof(s)) == 0) return kept[dir];
     const int64_t N = s.batch * s.seq, e = elt_of(s), nd = up(N * s.dim * e);
     Temps t = {};
@@ -89,11 +116,17 @@ Temps make_temps(const ptj_gpt2_shape& s, bool backward) {
     auto take = [&](int64_t bytes) { const int64_t o = at; at += bytes; return o; };
     t.t1 = take(nd);
     if (backward) {
+        t.dxm = take(nd);
+        for (int i = 0; i < 2; ++i) t.dx[i] = take(nd);
+        t.group = together ? grad_group_blocks(s) : 0;
+        const int64_t first = at;
         t.df1 = take(up(N * s.ffn * e));
         t.dqkv = take(up(N * 3 * s.dim * e));
-        t.dxm = take(nd);
         t.dm = take(nd);
-        for (int i = 0; i < 2; ++i) { t.dx[i] = take(nd); t.dr[i] = take(nd); }
+        t.block = at - first;
+        if (t.group) take((t.group - 1) * t.block);
+        t.dr_slots = t.group > 2 ? t.group : 2;      // (a block's is formed while the one before it is in use)
+        t.dr = take(t.dr_slots * nd);
         t.delta = take(up(s.batch * s.heads * s.seq * 4));
         t.ln_slot = (size_t)up((int64_t)ptj_layernorm_bwd_parts_bytes(N, s.dim));
         t.mul_slot = (size_t)up((int64_t)ptj_gemm_mul_colsum_workspace_bytes(N, s.ffn));
@@ -225,7 +258,11 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* sp, const void* const* params, const uint
     const ptj_gpt2_shape& s = *sp;
     PTJ_CHECK_ARG(params && acts && x_last && dh && grads && demb && (!s.train || seeds), "gpt2_bwd: null pointer");
     const Layout l = make_layout(s, true);
-    const Temps t = make_temps(s, true);
+    Temps t = make_temps(s, true);
+    bool aligned = ptj_aligned16(acts) && ptj_aligned16(workspace);
+    for (int64_t i = 0; i < s.layers; ++i)
+        for (const int p : {P_W2, P_W1, P_WO, P_WQKV}) aligned = aligned && ptj_aligned16(grads[P_FIRST + i * P_BLOCK + p]);
+    if (t.group && !aligned) t = make_temps(s, true, false);
     if (acts_bytes < (size_t)l.total || !workspace || workspace_bytes < t.total)
         return ptj_set_error(PTJ_ERR_WORKSPACE, "gpt2_bwd: %zu / %zu bytes of activations / workspace, %zu / %zu needed",
                              acts_bytes, workspace_bytes, (size_t)l.total, t.total);
@@ -258,8 +295,10 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* sp, const void* const* params, const uint
         return ptj_layernorm_bwd_later(dy, x, gb[0], res, dx, dgb[0], dgb[1], dropped, dropped_sum, train, sd, keep,
                                        ws + t.ln_parts + slot * (int64_t)t.ln_slot, t.ln_slot, N, D, dt, &sums, st);
     };
+    auto entering = [&](int64_t i) { return ws + t.dr + i % t.dr_slots * up(N * D * elt_of(s)); };
+    PtjGradGroup group = grad_group(s, 0);
     int cur = 0;
-    STEP(ln_bwd(2 * L, dh, x_last, fin, nullptr, ws + t.dx[0], gfin, ws + t.dr[0], grads[P_FIRST + (L - 1) * P_BLOCK + P_B2],
+    STEP(ln_bwd(2 * L, dh, x_last, fin, nullptr, ws + t.dx[0], gfin, entering(L - 1), grads[P_FIRST + (L - 1) * P_BLOCK + P_B2],
                 seed(3 * L), kb ? block(L - 1) + l.keep2 : nullptr));
     for (int64_t i = L - 1; i >= 0; --i) {
         const void* const* w = params + P_FIRST + i * P_BLOCK;
@@ -268,24 +307,41 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* sp, const void* const* params, const uint
         const char* const x_in = i ? block(i - 1) + l.xout : base + l.x0;
         const char* const h1 = i ? block(i - 1) + l.hnext : base + l.h0;
         const char* const dx = ws + t.dx[cur];
-        const char* const d = ws + t.dr[cur];
+        const int64_t own = t.group ? i % t.group * t.block : 0;
+        char *const df1 = ws + t.df1 + own, *const dqkv = ws + t.dqkv + own, *const dm = ws + t.dm + own;
+        const char* const d = entering(i);
         char* const t1 = ws + t.t1;
         float* const colpart = (float*)(ws + t.mul_parts + i * (int64_t)t.mul_slot);
+        // dX, and dW with it or later with the others of its group
+        auto linear = [&](int kind, PtjLinearBwd p) {
+            if (t.group) {
+                group.d[kind][group.blocks] = p.d;
+                group.x[kind][group.blocks] = p.x;
+                group.dw[kind][group.blocks] = p.dw;
+                p.dw = nullptr;
+            }
+            return ptj_linear_bwd(p, scratch, sb, dt, &sums, st);
+        };
         // x_out = x_mid + dropout(ffn(ln2(x_mid)))
-        STEP(ptj_linear_bwd({d, w[P_W2], a + l.g1, ws + t.df1, g[P_W2], N, D, F, a + l.f1, colpart, g[P_B1]}, scratch, sb, dt, &sums, st));
-        STEP(ptj_linear_bwd({ws + t.df1, w[P_W1], a + l.h2, t1, g[P_W1], N, F, D, nullptr, nullptr, nullptr}, scratch, sb, dt, &sums,
-                            st));
-        STEP(ln_bwd(2 * i + 1, t1, a + l.xmid, w + P_LN2G, dx, ws + t.dxm, g + P_LN2G, ws + t.dm, nullptr, seed(2 + 3 * i),
+        STEP(linear(W_FFN2, {d, w[P_W2], a + l.g1, df1, g[P_W2], N, D, F, a + l.f1, colpart, g[P_B1]}));
+        STEP(linear(W_FFN1, {df1, w[P_W1], a + l.h2, t1, g[P_W1], N, F, D, nullptr, nullptr, nullptr}));
+        STEP(ln_bwd(2 * i + 1, t1, a + l.xmid, w + P_LN2G, dx, ws + t.dxm, g + P_LN2G, dm, nullptr, seed(2 + 3 * i),
                     kb ? a + l.keep1 : nullptr));
         // x_mid = x_in + dropout(attn(ln1(x_in)))
-        STEP(ptj_linear_bwd({ws + t.dm, w[P_WO], a + l.o, t1, g[P_WO], N, D, D, nullptr, nullptr, nullptr}, scratch, sb, dt, &sums, st));
-        STEP(ptj_attn_bwd_packed(t1, a + l.qkv, a + l.o, (const float*)(a + l.ms), (const float*)(a + l.ls), mask, ws + t.dqkv,
+        STEP(linear(W_OUT, {dm, w[P_WO], a + l.o, t1, g[P_WO], N, D, D, nullptr, nullptr, nullptr}));
+        STEP(ptj_attn_bwd_packed(t1, a + l.qkv, a + l.o, (const float*)(a + l.ms), (const float*)(a + l.ls), mask, dqkv,
                                  (float*)(ws + t.delta), bits ? bits + i * bitlen : nullptr, B, H, T, train, dt, st));
-        STEP(ptj_linear_bwd({ws + t.dqkv, w[P_WQKV], h1, t1, g[P_WQKV], N, 3 * D, D, nullptr, nullptr, nullptr}, scratch, sb, dt, &sums,
-                            st));
+        STEP(linear(W_QKV, {dqkv, w[P_WQKV], h1, t1, g[P_WQKV], N, 3 * D, D, nullptr, nullptr, nullptr}));
+        if (t.group) {
+            ++group.blocks;
+            if (i % t.group == 0) {      // the next block's gradients take these ones' place
+                STEP(ptj_weight_grads(group, dt, st));
+                group.blocks = 0;
+            }
+        }
         // the dropped copy feeds block i - 1 (its feed-forward dropout) or the embedding
         const bool first = i == 0;
-        STEP(ln_bwd(2 * i, t1, x_in, w + P_LN1G, ws + t.dxm, ws + t.dx[cur ^ 1], g + P_LN1G, first ? demb : ws + t.dr[cur ^ 1],
+        STEP(ln_bwd(2 * i, t1, x_in, w + P_LN1G, ws + t.dxm, ws + t.dx[cur ^ 1], g + P_LN1G, first ? demb : entering(i - 1),
                     first ? nullptr : grads[P_FIRST + (i - 1) * P_BLOCK + P_B2], seed(3 * i),
                     kb && !first ? block(i - 1) + l.keep2 : nullptr));
         cur ^= 1;

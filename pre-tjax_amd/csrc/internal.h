@@ -85,4 +85,18 @@ struct PtjLinearBwd {
     float* colpart;
     void* colsum;
 };
+// dw = nullptr: dx alone.
 int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, int dtype, PtjPartialSums* later, hipStream_t st);
+
+// The weight gradients of several blocks in one launch: dw[kind][block] = d^T.x with d [k, n[kind]], x [k, m[kind]] and dw
+// [n[kind], m[kind]] row-major and contiguous, all of one storage type and on the 16-byte grid, widths multiples of 8.
+struct PtjGradGroup {
+    static constexpr int KINDS = 4, BLOCKS = 16;
+    int k, blocks;
+    int n[KINDS], m[KINDS];
+    const void *d[KINDS][BLOCKS], *x[KINDS][BLOCKS];
+    void* dw[KINDS][BLOCKS];
+};
+int ptj_weight_grads(const PtjGradGroup& p, int dtype, hipStream_t st);
+// Whether the launch has a round of tiles or more; sizes alone count.
+bool ptj_weight_grads_fill(const PtjGradGroup& p, int dtype);

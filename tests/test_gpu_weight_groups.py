@@ -1,0 +1,44 @@
+"""The native backward with the weight gradients of several blocks in one launch against the single calls: one step of the
+contraction and many, a last one that is not whole, tiles that end inside in both directions, two groups of unequal size, and
+gradients off the 16-byte grid, which are formed block by block."""
+import pytest
+import torch
+
+from oracle import gpt2 as ogpt2
+from util import DTYPES
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def both(mt, lo, monkeypatch, dtype, D, F, L, B, T, shift=0):
+    V, H = 101, D // 64
+    params = [[p.to(DEV).to(dtype) for p in grp] for grp in ogpt2.init_transformer_gpt2(V, D, L, H, F, T, seed=3)]
+    y = torch.randint(0, V, (B, T + 1), generator=torch.Generator().manual_seed(7)).to(DEV)
+    empty_like = torch.empty_like
+    if shift:
+        def off_the_grid(p, **kw):
+            if tuple(p.shape) not in ((D, D), (F, D), (D, F), (H, 3, 64, D)):
+                return empty_like(p, **kw)
+            return torch.empty(p.numel() + shift, dtype=p.dtype, device=p.device)[shift:].view(p.shape)
+        monkeypatch.setattr(mt.torch, "empty_like", off_the_grid)
+    runs = []
+    for native in (True, False):
+        monkeypatch.setattr(mt, "NATIVE_STACK", native)
+        grads, _ = lo.t_loss_bkwd3_t(params, y, None, None, True, list(range(10, 11 + 3 * L)))
+        runs.append([p for grp in grads for p in grp])
+    return runs
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("D,F,L,B,T,shift", [(768, 3072, 2, 1, 64, 0), (768, 3072, 3, 3, 192, 0), (320, 1288, 17, 1, 320, 0),
+                                             (768, 3080, 2, 1, 448, 0), (768, 3072, 2, 1, 128, 1), (256, 1024, 12, 7, 64, 0)])
+def test_weight_gradients_together(mt, lo, monkeypatch, dtype, D, F, L, B, T, shift):
+    runs = both(mt, lo, monkeypatch, dtype, D, F, L, B, T, shift)
+    # The sums of a weight gradient are added in another order: in fp32 a few roundings of 2^-24; in bf16 a value on the edge may be
+    # stored one step of 2^-8 away, all of them two independent roundings of 2^-9 / sqrt(3) at the very most.  Everything else
+    # comes from the same products; of the pairs' (shift) in bf16 up to six stored tensors lie between two products of a block.
+    bound = 2e-6 if dtype == torch.float32 else 1.6e-3 * (L * 6 if shift else 1) ** 0.5
+    for i, (a, b) in enumerate(zip(*runs)):
+        a, b = a.double(), b.double()
+        assert (a - b).norm() <= bound * b.norm(), i
