@@ -269,6 +269,18 @@ int ptj_gemm(const void* a, const void* b, void* c, const void* bias,
              int epilogue, void* c_pre, int64_t c_pre_rs,
              void* workspace, size_t workspace_bytes, int dtype, void* stream);
 
+/* Several products c[n,m] = a.b (operands as for ptj_gemm, no epilogue) that do not depend on each other, `p` a HOST array: no c may
+ * overlap an operand or another c.  Up to four share a launch where each alone would leave the chip partly idle (the weight
+ * gradients and the input gradient of a feed-forward block, model_triton.py:1410-1428), with another order of summation;
+ * else one ptj_gemm after the other.  `workspace` as for the neediest of these. */
+typedef struct ptj_product {
+    const void *a, *b;
+    void* c;
+    int64_t n, m, k, a_rs, a_cs, b_rs, b_cs, c_rs;
+} ptj_product;
+size_t ptj_gemm_many_workspace_bytes(const ptj_product* p, int64_t count, int dtype);
+int ptj_gemm_many(const ptj_product* p, int64_t count, void* workspace, size_t workspace_bytes, int dtype, void* stream);
+
 /* C[n,m] = round(A.B) * mul[n,m] element-wise, and colsum[m] = the column sums of the stored C:
  * the product that carries a gradient back through the feed-forward block's second linear layer
  * (t_proj_bkwd2_x, model_triton.py:495-508), the GELU backward (t_gelu_bkwd2_k, :274-294; `mul` =

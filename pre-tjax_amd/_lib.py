@@ -55,6 +55,8 @@ SIGNATURES = {
                                    _p]),
     "ptj_gemm": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p, _i64, _p, _sz, _int,
                         _p]),
+    "ptj_gemm_many_workspace_bytes": (_sz, [_p, _i64, _int]),
+    "ptj_gemm_many": (_int, [_p, _i64, _p, _sz, _int, _p]),
     "ptj_adamw": (_int, [_p, _p, _p, _p, _p, _i64, _c.c_float, _c.c_float, _c.c_float, _c.c_float, _c.c_float, _i64,
                          _int, _int, _p]),
     "ptj_adamw_multi": (_int, [_i64, _p, _p, _p, _p, _p, _p, _p, _c.c_float, _c.c_float, _c.c_float, _c.c_float, _i64,
