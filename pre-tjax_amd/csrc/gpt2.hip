@@ -216,21 +216,37 @@ int ptj_gpt2_fwd(const ptj_gpt2_shape* sp, const void* const* params, const int6
     const bool kb = keeps_bytes(s, params);
     const char* x = base + l.x0;
     const char* hn = base + l.h0;
+    // few rows, and neither decisions nor activations to keep: each norm inside the product that reads it (gemm_norm.hip)
+    bool inside = !keep && !train && ptj_norm_product_fits(N, D, F, dt, false) && ptj_aligned16(acts) && ptj_aligned16(workspace);
+    for (int64_t i = P_FIRST; inside && i < P_FIRST + s.layers * P_BLOCK; ++i) inside = ptj_aligned16(params[i]);
+    PtjNormProduct entry = {};         // the norm that enters a block, with the block's input
     for (int64_t i = 0; i < s.layers; ++i) {
         const void* const* w = params + P_FIRST + i * P_BLOCK;
         char* const a = base + l.first_layer + i * l.layer_stride;
         const bool last = i + 1 == s.layers;
         const int64_t s1 = train ? seeds[2 + 3 * i] : 0, s2 = train ? seeds[3 + 3 * i] : 0;
-        STEP(ptj_gemm(hn, w[P_WQKV], a + l.qkv, nullptr, N, 3 * D, D, D, 1, 1, D, 3 * D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt,
-                      stream));
+        if (entry.res) {
+            entry.w = w[P_WQKV];
+            entry.c = a + l.qkv;
+            STEP(ptj_norm_product(entry, N, D, 3 * D, dt, st));
+            entry.res = nullptr;
+        } else {
+            STEP(ptj_gemm(hn, w[P_WQKV], a + l.qkv, nullptr, N, 3 * D, D, D, 1, 1, D, 3 * D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt,
+                          stream));
+        }
         STEP(ptj_attn_fwd_packed(a + l.qkv, mask, a + l.o, (float*)(a + l.ms), (float*)(a + l.ls), bits ? bits + i * bitlen : nullptr,
                                  B, H, T, train, dt, st));
         STEP(ptj_gemm(a + l.o, w[P_WO], ws + t.t1, nullptr, N, D, D, D, 1, 1, D, D, PTJ_EPI_NONE, nullptr, 0, scratch, sb, dt, stream));
-        STEP(ptj_dropout_add_layernorm_of({ws + t.t1, nullptr, 0, nullptr}, x, w[P_LN2G], w[P_LN2B], a + l.xmid, a + l.h2,
-                                          kb ? a + l.keep1 : nullptr, N, D, train, s1, dt, st));
-        STEP(ptj_gemm(a + l.h2, w[P_W1], a + l.g1, w[P_B1], N, F, D, D, 1, 1, D, F,
-                      keep ? PTJ_EPI_BIAS_GELU_DERIV : PTJ_EPI_BIAS_GELU, keep ? a + l.f1 : nullptr, keep ? F : 0, scratch, sb, dt,
-                      stream));
+        if (inside) {
+            STEP(ptj_norm_product({{ws + t.t1, nullptr, 0, nullptr}, x, w[P_LN2G], w[P_LN2B], w[P_W1], w[P_B1], a + l.xmid, a + l.g1, 1}, N, D, F,
+                                  dt, st));
+        } else {
+            STEP(ptj_dropout_add_layernorm_of({ws + t.t1, nullptr, 0, nullptr}, x, w[P_LN2G], w[P_LN2B], a + l.xmid, a + l.h2,
+                                              kb ? a + l.keep1 : nullptr, N, D, train, s1, dt, st));
+            STEP(ptj_gemm(a + l.h2, w[P_W1], a + l.g1, w[P_B1], N, F, D, D, 1, 1, D, F,
+                          keep ? PTJ_EPI_BIAS_GELU_DERIV : PTJ_EPI_BIAS_GELU, keep ? a + l.f1 : nullptr, keep ? F : 0, scratch, sb, dt,
+                          stream));
+        }
         char* const xo = last ? (char*)x_last : a + l.xout;
         char* const ho = last ? (char*)h : a + l.hnext;
         const void* const* nx = last ? fin : w + P_BLOCK;   // the norm that reads this block's output
@@ -243,7 +259,9 @@ int ptj_gpt2_fwd(const ptj_gpt2_shape* sp, const void* const* params, const int6
         else
             STEP(ptj_gemm(a + l.g1, w[P_W2], ws + t.t1, w[P_B2], N, D, F, F, 1, 1, F, D, PTJ_EPI_BIAS, nullptr, 0, scratch, sb, dt,
                           stream));
-        STEP(ptj_dropout_add_layernorm_of(f2, a + l.xmid, nx[0], nx[1], xo, ho, kb ? a + l.keep2 : nullptr, N, D, train, s2, dt,
+        if (inside && !last && ptj_norm_product_fits(N, D, 3 * D, dt, f2.part != nullptr)) entry = {f2, a + l.xmid, nx[0], nx[1], nullptr, nullptr, xo, nullptr, 0};
+        else
+            STEP(ptj_dropout_add_layernorm_of(f2, a + l.xmid, nx[0], nx[1], xo, ho, kb ? a + l.keep2 : nullptr, N, D, train, s2, dt,
                                           st));
         x = xo;
         hn = ho;

@@ -73,6 +73,18 @@ int ptj_dropout_add_layernorm_of(const PtjPartialProduct& x, const void* res, co
                                  void* h, void* keep_bytes, int64_t rows, int64_t cols, int train, int64_t seed, int dtype,
                                  hipStream_t st);
 
+// y = res + dropout(x) without decisions (x * 0.9) and c = layernorm(y) . w^T (+ bias) (GELU), w [m, dim], in one launch for few rows:
+// the same arithmetic as ptj_dropout_add_layernorm_of and ptj_gemm; the norm itself is not stored.  y and c may overlap no operand.
+struct PtjNormProduct {
+    PtjPartialProduct x;
+    const void *res, *gamma, *beta, *w, *bias;
+    void *y, *c;
+    int gelu;
+};
+// Whether sizes and type are taken (`partial`: x as partial sums); all pointers have to lie on the 16-byte grid.
+bool ptj_norm_product_fits(int64_t rows, int64_t dim, int64_t m, int dtype, bool partial);
+int ptj_norm_product(const PtjNormProduct& p, int64_t rows, int64_t dim, int64_t m, int dtype, hipStream_t st);
+
 // The two products of a linear layer's backward, which do not depend on each other: dx = d.w and dw = d^T.x with d [n, m],
 // w [m, k], x [n, k] row-major and contiguous.  In one launch where each alone would leave the chip half empty, else one
 // after the other.  With `mul` [n, k]: dx = round(d.w) * mul and its column sums to `colsum` (ptj_gemm_mul_colsum; the
