@@ -8,17 +8,17 @@ namespace {
 
 // gemm_plan through a small per-thread table: a training loop asks for the same few dozen products again and again,
 // and the estimate over all tile shapes and splits takes a microsecond.
-GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int loose, int kernels = ANY_KERNEL) {
-    struct Entry { int64_t n, m, k; size_t ws; int elt, cus, loose, kernels; GemmPlan plan; };
+GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int loose, int kernels = ANY_KERNEL, bool later = false) {
+    struct Entry { int64_t n, m, k; size_t ws; int elt, cus, loose, kernels, later; GemmPlan plan; };
     constexpr int ENTRIES = 128;
     static thread_local Entry table[ENTRIES] = {};
     const int cus = num_cus();
     const uint64_t h = ((uint64_t)n * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)m * 0xC2B2AE3D27D4EB4Full) ^
-                       ((uint64_t)k * 0x165667B19E3779F9ull) ^ ((uint64_t)(ws_bytes + loose) * 0xD6E8FEB86659FD93ull);
+                       ((uint64_t)k * 0x165667B19E3779F9ull) ^ ((uint64_t)(ws_bytes + loose + later) * 0xD6E8FEB86659FD93ull);
     Entry& e = table[(h >> 40) % ENTRIES];
     if (e.n != n || e.m != m || e.k != k || e.ws != ws_bytes || e.elt != elt || e.cus != cus || e.loose != loose ||
-        e.kernels != kernels)
-        e = {n, m, k, ws_bytes, elt, cus, loose, kernels, gemm_plan(n, m, k, elt, ws_bytes, cus, loose, kernels)};
+        e.kernels != kernels || e.later != later)
+        e = {n, m, k, ws_bytes, elt, cus, loose, kernels, later, gemm_plan(n, m, k, elt, ws_bytes, cus, loose, kernels, 0, later)};
     return e.plan;
 }
 
@@ -65,6 +65,9 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
     if (bias) outputs_aligned = outputs_aligned && (reinterpret_cast<uintptr_t>(bias) % (4 * (size_t)elt)) == 0;
     const bool aligned_ws = workspace && ptj_aligned16(workspace);
     const int loose = ragged ? LOOSE_OPERAND : outputs_aligned ? ALIGNED : LOOSE_OUTPUT;
+    // a bias without an activation: the end of a feed-forward block, whose partial sums the next norm adds up.  (Whether this caller
+    // is the one that leaves them does not count: the bits of a product depend on its plan.)
+    const bool left = epilogue == PTJ_EPI_BIAS && !ragged && m % 4 == 0;
     GemmPlan plan = {-1, 1, 0, 0, 1, 0, 0.0};
     if (epilogue == PTJ_EPI_ACCUMULATE) {
         // only the ring kernels start their accumulators from the stored C
@@ -73,9 +76,9 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
                                  "operand layout, k a multiple of 64 and vector-aligned C");
         plan = cached_plan(n, m, k, elt, 0, loose, RING_ONLY);
     } else if (gt_eligible(g, am, bm, ragged ? 8 : 1)) {
-        plan = cached_plan(n, m, k, elt, aligned_ws ? workspace_bytes : 0, loose);
+        plan = cached_plan(n, m, k, elt, aligned_ws ? workspace_bytes : 0, loose, ANY_KERNEL, left);
     } else if (elt == 2 && !ragged && ring_eligible(g, am, bm)) {
-        plan = cached_plan(n, m, k, elt, aligned_ws ? workspace_bytes : 0, loose, RING_ONLY);
+        plan = cached_plan(n, m, k, elt, aligned_ws ? workspace_bytes : 0, loose, RING_ONLY, left);
     }
     int splits = plan.splits;
     int64_t kps = plan.cfg >= 0 ? plan.kps : k;
@@ -128,10 +131,11 @@ size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
     int first, ts, tkps;
     size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
     for (const int loose : {ALIGNED, LOOSE_OUTPUT, LOOSE_OPERAND})
-        for (const int kernels : {ANY_KERNEL, RING_ONLY}) {
-            const size_t bytes = gp_workspace_bytes(cached_plan(n, m, k, elt, (size_t)-1, loose, kernels), n, m, k);
-            if (bytes > need) need = bytes;
-        }
+        for (const int kernels : {ANY_KERNEL, RING_ONLY})
+            for (const bool later : {false, true}) {
+                const size_t bytes = gp_workspace_bytes(cached_plan(n, m, k, elt, (size_t)-1, loose, kernels, later), n, m, k);
+                if (bytes > need) need = bytes;
+            }
     return need;
 }
 

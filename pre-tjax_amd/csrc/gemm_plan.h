@@ -26,11 +26,19 @@ struct TileCost {
     double crowd;        // growth of the step time from half the CUs busy (0) to all of them
 };
 
-// bf16 / fp32; the index is the configuration number of gemm_tile_launch
-constexpr int GT_CONFIGS[2] = {6, 6};
+// bf16 / fp32; the index is the configuration number of gemm_tile_launch (bf16: 1 is gemm_pair.hip's alone)
 // operands without 16-byte alignment: the configurations from here on (bf16: gemm_ragged.h; fp32: gemm_split.h)
 constexpr int RAGGED_FIRST[2] = {6, 4}, RAGGED_END[2] = {8, 6};
-constexpr TileCost GT_COST[2][8] = {
+// The last three of bf16 are for up to a round of tiles: a chain of K steps whose copies are on their way for 0.7-1.1 us.  Eight wavefronts
+// and four stages of 64x64 leave 0.4 us less around the loop than four and three (which they replace); 32x64 tiles put twice as many
+// CUs to work; 64x128 with two K groups has half the steps.  One product, us, the best of the others / these: 512x768x768 6.5 / 5.4,
+// 512x768x2304 10.5 / 8.7, 512x768x3072 12.6 / 10.1 (K split in two with its second stage 12.7), 256x2304x768 6.5 / 6.2, 512x2304x768 8.5 /
+// 8.0, 1536x768x768 8.5 / 8.0, 1536x768x2304 15.3 / 13.9, 1536x768x3072 19 / 17; four and five stages of 128x128, 64x64 and 32x32: no faster.
+// 32x64 and 64x128 with two K groups take no K split: their staging of partial sums costs more than the estimate knows (forward of 512
+// tokens with 64x128 in five 685 us, with 32x64 whole 645; of 1024 tokens with 64x128 in two 962, with 64x64 whole 943).
+constexpr int GT_END[2] = {11, 6};
+inline bool gt_plain(int type, int i) { return type == 1 || (i != 1 && (i < RAGGED_FIRST[0] || i >= RAGGED_END[0])); }
+constexpr TileCost GT_COST[2][11] = {
     {{32, 32, 256, 1, 2.08, 0.571, 1.33, 1.0, 0.0},
      {64, 64, 128, 1, 3.62, 0.341, 1.57, 1.0, 0.0},
      {64, 128, 64, 2, 4.50, 0.300, 1.12, 1.87, 0.10},
@@ -38,7 +46,10 @@ constexpr TileCost GT_COST[2][8] = {
      {128, 128, 64, 2, 4.25, 0.632, 2.01, 1.33, 0.23},
      {128, 192, 64, 2, 5.57, 0.587, 3.93, 1.32, 0.91},
      {128, 128, 64, 2, 4.32, 0.765, 5.66, 1.57, 0.0},
-     {64, 64, 64, 2, 4.51, 0.471, 1.01, 1.08, 0.0}},
+     {64, 64, 64, 2, 4.51, 0.471, 1.01, 1.08, 0.0},
+     {32, 64, 256, 1, 2.85, 0.530, 1.70, 1.0, 0.0},
+     {64, 64, 128, 1, 2.70, 0.364, 1.90, 1.0, 0.0},
+     {64, 128, 128, 1, 2.50, 0.487, 3.20, 1.0, 0.0}},
     // fp32: the last two multiply on the bf16 pipe (gemm_split.h)
     {{32, 32, 128, 1, 3.25, 0.663, 1.67, 1.0, 0.0},
      {64, 64, 64, 1, 3.56, 1.077, 2.37, 1.0, 0.0},
@@ -81,9 +92,12 @@ inline int64_t gp_ceil(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Second stage of a K split: its launch, and the partial sums written and read once more.  (bf16: 4.9 us and 0.23 fit best; the
 // launch is taken lower because behind a feed-forward block the next norm adds up the partial sums without one.)
-inline double gp_reduce_us(int64_t n, int64_t m, int splits, int elt) {
+// `later`, bf16: that is likely, and costs the norm 1.6 us and some more for the bytes.  Second feed-forward product in a forward: 512 tokens
+// in two parts of 64x64 685 us, with 32x64 tiles whole 645; 1536 tokens in three of 128x128 1113, with 64x128 whole 1132.
+inline double gp_reduce_us(int64_t n, int64_t m, int splits, int elt, bool later = false) {
     if (splits <= 1) return 0.0;
     const double bytes = 4.0 * (double)splits * (double)n * (double)m;
+    if (later && elt == 2) return 1.6 + 0.12e-6 * bytes;
     return 2.6 + (elt == 2 ? 0.24e-6 : 0.35e-6) * bytes;
 }
 // a K step of one workgroup when `work` of them share the chip
@@ -92,7 +106,7 @@ inline double gp_step_us(const TileCost& c, int64_t work, int cus) {
     return c.step * (1.0 + (busy > 0.5 ? c.crowd * 2.0 * (busy - 0.5) : 0.0));
 }
 
-inline double gp_tile_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int elt, int splits, int cus) {
+inline double gp_tile_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int elt, int splits, int cus, bool later) {
     const int64_t work = gp_ceil(n, c.tbm) * gp_ceil(m, c.tbn) * splits;
     const int64_t steps = gp_ceil(gp_ceil(k, splits), c.bkt);
     const double step = gp_step_us(c, work, cus);
@@ -102,17 +116,17 @@ inline double gp_tile_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int
     // bf16: a chip that stays full over several rounds shares the path from L2: measured 10 % at 1.5 rounds, 30 % at many
     const double rounds = (double)work / (double)slots;
     if (elt == 2 && rounds > 1.0) t *= 1.0 + 0.3 * (1.0 - 1.0 / rounds);
-    return t + gp_reduce_us(n, m, splits, elt);
+    return t + gp_reduce_us(n, m, splits, elt, later);
 }
 
 // The persistent kernels.  A last round that is not full costs its steps whole, but its stores only by their share; cut into
 // tail_splits K slices per tile (*tail) it costs the steps of a slice, and fp32 partial tiles written and read once.
-inline double gp_ring_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int splits, int cus) {
+inline double gp_ring_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int splits, int cus, bool later) {
     const int64_t work = gp_ceil(n, c.tbm) * gp_ceil(m, c.tbn) * splits, steps = gp_ceil(gp_ceil(k, splits), 64);
     const int64_t full = work / cus, rem = work % cus;
     const double tile = (double)steps * gp_step_us(c, work, cus);
     return c.start + (double)full * (tile + c.finish) + (rem ? tile + c.finish * (double)rem / (double)cus : 0.0) +
-           gp_reduce_us(n, m, splits, 2);
+           gp_reduce_us(n, m, splits, 2, later);
 }
 inline double gp_ring_tail_us(const TileCost& c, int64_t n, int64_t m, int64_t k, int tail_splits, int cus) {
     const int64_t work = gp_ceil(n, c.tbm) * gp_ceil(m, c.tbn), full = work / cus, items = work % cus * tail_splits;
@@ -125,21 +139,23 @@ inline double gp_ring_tail_us(const TileCost& c, int64_t n, int64_t m, int64_t k
 // product with another epilogue add in the same order.  `loose`: operands or outputs that do not come in aligned
 // 16-byte vectors; the ring kernels take such operands not at all and write such outputs element by element (twice the
 // time at k = 768), the tile kernels write any.
+// `later`: the consumer usually adds up the partial sums of a K split.
 // `planes_ws`: workspace for operands split ahead of a product without a K split, where partial sums may not take any.
 inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int cus, int loose = ALIGNED,
-                          int kernels = ANY_KERNEL, size_t planes_ws = 0) {
+                          int kernels = ANY_KERNEL, size_t planes_ws = 0, bool later = false) {
     const bool ragged = loose == LOOSE_OPERAND;
     GemmPlan best = {-1, 1, (int)k, 0, 1, 0, 1e30};
     const int type = elt == 2 ? 0 : 1;
     auto fits = [&](double bytes) { return bytes <= (double)ws_bytes; };
     if (kernels != RING_ONLY)
-        for (int i = ragged ? RAGGED_FIRST[type] : 0; i < (ragged ? RAGGED_END[type] : GT_CONFIGS[type]); ++i) {
+        for (int i = ragged ? RAGGED_FIRST[type] : 0; i < (ragged ? RAGGED_END[type] : GT_END[type]); ++i) {
+            if (!ragged && !gt_plain(type, i)) continue;
             const TileCost& c = GT_COST[type][i];
-            for (int s = 1; s <= 16; ++s) {
+            for (int s = 1; s <= (type == 0 && (i == 8 || i == 10) ? 1 : 16); ++s) {
                 if (s > 1 && (k < 1024 || k / s < 256 || !fits(4.0 * s * (double)n * (double)m))) break;
                 const int64_t kps = gp_ceil(gp_ceil(k, s), c.bkt) * c.bkt;
                 if (s > 1 && gp_ceil(k, kps) != s) continue;
-                const double us = gp_tile_us(c, n, m, k, elt, s, cus);
+                const double us = gp_tile_us(c, n, m, k, elt, s, cus, later);
                 if (us < best.us) best = {i, s, (int)(s > 1 ? kps : k), 0, 1, 0, us};
             }
         }
@@ -150,7 +166,7 @@ inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_by
             if (!fits(planes + (s > 1 ? 4.0 * s * (double)n * (double)m : 0.0)) && !(s == 1 && planes <= (double)planes_ws)) break;
             const int64_t kps = gp_ceil(gp_ceil(k, s), 32) * 32;
             if (s > 1 && gp_ceil(k, kps) != s) continue;
-            const double us = gp_tile_us(PLANES_COST, n, m, k, elt, s, cus) + split;
+            const double us = gp_tile_us(PLANES_COST, n, m, k, elt, s, cus, later) + split;
             if (us < best.us) best = {PLANES_CFG, s, (int)(s > 1 ? kps : k), 0, 1, 0, us};
         }
     }
@@ -163,7 +179,7 @@ inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_by
             if (s > 1 && (k < 1024 || k / s < 256 || tiles >= 2 * cus || !fits(4.0 * s * (double)n * (double)m))) break;
             const int64_t kps = gp_ceil(gp_ceil(k, s), 64) * 64;
             if (s > 1 && gp_ceil(k, kps) != s) continue;
-            const double us = slow * gp_ring_us(c, n, m, k, s, cus);
+            const double us = slow * gp_ring_us(c, n, m, k, s, cus, later);
             if (us < best.us) best = {RING_FIRST + i, s, (int)(s > 1 ? kps : k), 0, 1, 0, us};
         }
         for (int s = 2; s <= 32 && full > 0 && tiles > full && k >= 1024; ++s) {

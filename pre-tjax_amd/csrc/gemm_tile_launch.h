@@ -7,7 +7,10 @@ namespace {
 
 //                      tile     waves K-groups stages chunks per register set
 typedef GtCfg<32, 32, 1, 1, 4, 3, 4> GtTiny;        // few rows: four wavefronts share one 32x32 tile along K
-typedef GtCfg<64, 64, 1, 2, 2, 3, 4> GtSmall;
+typedef GtCfg<64, 64, 1, 2, 2, 3, 4> GtSmall;       // (fp32)
+typedef GtCfg<32, 64, 1, 1, 4, 3, 4> GtTinyWide;
+typedef GtCfg<64, 64, 2, 2, 2, 4, 4> GtSmall8;      // eight wavefronts
+typedef GtCfg<64, 128, 1, 4, 2, 3, 4> GtWide8;      // eight wavefronts
 typedef GtCfg<64, 64, 1, 2, 2, 2, 4> GtSmall2;      // two workgroups per CU
 typedef GtCfg<64, 128, 1, 4, 1, 3, 4> GtWide;
 typedef GtCfg<128, 128, 2, 4, 1, 3, 4> GtSquare;
@@ -41,9 +44,11 @@ int gt_dispatch(const GemmArgs& g, int cfg, int am, int bm, int* mul_rows, hipSt
     if constexpr (sizeof(T) == 2) {
         switch (cfg) {
             case 0: return gt_run<T, MUL, GtTiny>(g, am, bm, mul_rows, st);
-            case 1: return gt_run<T, MUL, GtSmall>(g, am, bm, mul_rows, st);
             case 2: return gt_run<T, MUL, GtWide>(g, am, bm, mul_rows, st);
             case 3: return gt_run<T, MUL, GtSquare>(g, am, bm, mul_rows, st);
+            case 8: return gt_run<T, MUL, GtTinyWide>(g, am, bm, mul_rows, st);
+            case 9: return gt_run<T, MUL, GtSmall8>(g, am, bm, mul_rows, st);
+            case 10: return gt_run<T, MUL, GtWide8>(g, am, bm, mul_rows, st);
             case 4: return gt_run<T, MUL, GtSquare2>(g, am, bm, mul_rows, st);
             default: return gt_run<T, MUL, GtLarge>(g, am, bm, mul_rows, st);
         }
