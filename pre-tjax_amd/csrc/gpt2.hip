@@ -280,7 +280,7 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* sp, const void* const* params, const uint
     bool aligned = ptj_aligned16(acts) && ptj_aligned16(workspace);
     for (int64_t i = 0; i < s.layers; ++i)
         for (const int p : {P_W2, P_W1, P_WO, P_WQKV}) aligned = aligned && ptj_aligned16(grads[P_FIRST + i * P_BLOCK + p]);
-    if (t.group && !aligned) t = make_temps(s, true, false);
+    if (t.group && (!aligned || workspace_bytes < t.total)) t = make_temps(s, true, false);   // (a workspace for one block's at a time will do)
     if (acts_bytes < (size_t)l.total || !workspace || workspace_bytes < t.total)
         return ptj_set_error(PTJ_ERR_WORKSPACE, "gpt2_bwd: %zu / %zu bytes of activations / workspace, %zu / %zu needed",
                              acts_bytes, workspace_bytes, (size_t)l.total, t.total);

@@ -42,3 +42,38 @@ def test_weight_gradients_together(mt, lo, monkeypatch, dtype, D, F, L, B, T, sh
     for i, (a, b) in enumerate(zip(*runs)):
         a, b = a.double(), b.double()
         assert (a - b).norm() <= bound * b.norm(), i
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_workspace_of_one_block(mt, lo, monkeypatch, dtype):
+    """A workspace without room for what several blocks' weight gradients read: the blocks one by one, in nothing but that room."""
+    L, B, T, D, F, H = 3, 1, 64, 768, 3072, 12
+    params = [[p.to(DEV).to(dtype) for p in grp] for grp in ogpt2.init_transformer_gpt2(101, D, L, H, F, T, seed=3)]
+    flat = mt._native_params(params)
+    y = torch.randint(0, 101, (B, T), generator=torch.Generator().manual_seed(7)).to(DEV)
+    h, x_last, acts = mt._native_fwd(params, flat, y, None, True, list(range(10, 11 + 3 * L)), True)
+    dh = torch.randn(h.shape, generator=torch.Generator().manual_seed(8)).to(DEV).to(dtype)
+    lib = mt.lib()
+    row = B * T * D * (2 if dtype == torch.bfloat16 else 4)
+    whole = lib.ptj_gpt2_workspace_bytes(acts.shape, 1)
+    # two blocks' d(feed-forward), d(qkv), d(residual) and one more entering gradient
+    small = whole - 2 * (F // D + 3 + 1) * row - row
+
+    def backward(ws_bytes, room):
+        grads = [torch.zeros_like(p) for p in flat]
+        demb = torch.empty_like(dh)
+        ws = torch.full((room + 4096,), 7, dtype=torch.uint8, device=DEV)
+        rc = lib.ptj_gpt2_bwd(acts.shape, mt._pointers(flat), None, acts.seeds, acts.buf.data_ptr(), acts.buf.numel(), x_last.data_ptr(),
+                              dh.data_ptr(), mt._pointers(grads), demb.data_ptr(), ws.data_ptr(), ws_bytes, mt.stream())
+        assert bool((ws[room:] == 7).all())
+        return rc, [g.double() for g in grads[3:]] + [demb.double()]
+
+    rc, want = backward(whole, whole)
+    assert rc == 0
+    rc, got = backward(small, small)
+    assert rc == 0
+    # as above; in bf16 up to six stored tensors lie between two products of a block
+    bound = 2e-6 if dtype == torch.float32 else 1.6e-3 * (L * 6) ** 0.5
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert (a - b).norm() <= bound * b.norm(), i
+    assert backward(small - 1, small)[0] != 0
