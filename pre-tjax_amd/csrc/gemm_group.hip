@@ -42,6 +42,8 @@ bool ptj_weight_grads_fill(const PtjGradGroup& p, int dtype) { return group_conf
 
 int ptj_weight_grads(const PtjGradGroup& p, int dtype, hipStream_t st) {
     if (p.blocks < 1 || p.blocks > PtjGradGroup::BLOCKS || p.k < 1) return ptj_set_error(PTJ_ERR_INVALID, "weight_grads: bad group");
+    for (int i = 0; i < PtjGradGroup::KINDS; ++i)
+        for (int j = 0; j < p.blocks; ++j) PTJ_CHECK_ARG(p.d[i][j] && p.x[i][j] && p.dw[i][j], "weight_grads: null pointer");
     if (dtype != PTJ_BF16) return gs_group_launch<GsSquare>(p, st);
     return group_config(p, dtype) == 0 ? ring_group_launch<RingFull>(p, st) : ring_group_launch<RingNarrow>(p, st);
 }

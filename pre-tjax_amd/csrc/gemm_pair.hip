@@ -142,11 +142,12 @@ GemmArgs args_of(const void* a, const void* b, void* c, int64_t n, int64_t m, in
 
 int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, int dtype, PtjPartialSums* later, hipStream_t st) {
     const int64_t n = p.n, m = p.m, k = p.k;
-    if (dtype == PTJ_BF16 && p.dw && n < (1 << 20) && m < (1 << 20) && k < (1 << 20)) {
+    if (dtype == PTJ_BF16 && !p.dx_only && n < (1 << 20) && m < (1 << 20) && k < (1 << 20)) {
         GemmArgs gx = args_of(p.d, p.w, p.dx, n, k, m, m, 1), gw = args_of(p.d, p.x, p.dw, m, k, n, 1, m);
         gx.mul = p.mul; gx.mul_rs = k; gx.colpart = p.colpart;
         if (p.mul) gx.vec_out = gx.vec_out && ptj_aligned16(p.mul);
-        const bool ok = pick_mode<bf16>(gx.a, gx.a_row, gx.a_k) == KMAJOR && pick_mode<bf16>(gx.b, gx.b_row, gx.b_k) == MNMAJOR &&
+        const bool ok = p.d && p.w && p.x && p.dx && p.dw && pick_mode<bf16>(gx.a, gx.a_row, gx.a_k) == KMAJOR &&
+                        pick_mode<bf16>(gx.b, gx.b_row, gx.b_k) == MNMAJOR &&
                         pick_mode<bf16>(gw.a, gw.a_row, gw.a_k) == MNMAJOR && pick_mode<bf16>(gw.b, gw.b_row, gw.b_k) == MNMAJOR &&
                         gt_eligible(gx, KMAJOR, MNMAJOR) && gt_eligible(gw, MNMAJOR, MNMAJOR);
         const PairChoice choice = ok ? choose_pair(p) : PairChoice{0, false};
@@ -166,7 +167,7 @@ int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, i
             return PTJ_OK;
         }
     }
-    if (p.dw) {
+    if (!p.dx_only) {
         const int rc = ptj_gemm(p.d, p.x, p.dw, nullptr, m, k, n, 1, m, k, 1, k, PTJ_EPI_NONE, nullptr, 0, scratch, scratch_bytes, dtype, st);
         if (rc != PTJ_OK) return rc;
     }

@@ -13,6 +13,7 @@
 
 #include <math.h>
 #include <string.h>
+#include <initializer_list>
 
 namespace {
 
@@ -156,6 +157,15 @@ int check_shape(const char* what, const ptj_gpt2_shape* s) {
 enum { P_LN1G, P_LN1B, P_WQKV, P_WO, P_LN2G, P_LN2B, P_W1, P_B1, P_W2, P_B2, P_BLOCK };
 constexpr int P_FIRST = 3;   // table, its bias, positions
 
+// Whether these entries of every block are there.  A missing one is refused before the first launch: the launches that several
+// products share see no single call's checks.
+bool all_given(const void* const* nest, int64_t layers, std::initializer_list<int> entries) {
+    for (int64_t i = 0; i < layers; ++i)
+        for (const int p : entries)
+            if (!nest[P_FIRST + i * P_BLOCK + p]) return false;
+    return true;
+}
+
 // Dropout decisions recorded by the forward (one byte per 8 columns) for the LayerNorm backward.  The vector kernels do
 // that only: fp32 norms off the 16-byte grid recompute the decisions, bf16 ones are refused as in the single calls.
 bool keeps_bytes(const ptj_gpt2_shape& s, const void* const* params) {
@@ -275,6 +285,9 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* sp, const void* const* params, const uint
     STEP(check_shape("gpt2_bwd", sp));
     const ptj_gpt2_shape& s = *sp;
     PTJ_CHECK_ARG(params && acts && x_last && dh && grads && demb && (!s.train || seeds), "gpt2_bwd: null pointer");
+    PTJ_CHECK_ARG(all_given(params, s.layers, {P_LN1G, P_WQKV, P_WO, P_LN2G, P_W1, P_W2}) && params[P_FIRST + s.layers * P_BLOCK],
+                  "gpt2_bwd: null parameter");
+    PTJ_CHECK_ARG(all_given(grads, s.layers, {P_WQKV, P_WO, P_W1, P_B1, P_W2}), "gpt2_bwd: null gradient of a weight or of the first bias");
     const Layout l = make_layout(s, true);
     Temps t = make_temps(s, true);
     bool aligned = ptj_aligned16(acts) && ptj_aligned16(workspace);
@@ -336,7 +349,7 @@ int ptj_gpt2_bwd(const ptj_gpt2_shape* sp, const void* const* params, const uint
                 group.d[kind][group.blocks] = p.d;
                 group.x[kind][group.blocks] = p.x;
                 group.dw[kind][group.blocks] = p.dw;
-                p.dw = nullptr;
+                p.dx_only = true;
             }
             return ptj_linear_bwd(p, scratch, sb, dt, &sums, st);
         };

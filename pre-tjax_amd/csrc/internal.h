@@ -96,8 +96,8 @@ struct PtjLinearBwd {
     const void* mul;
     float* colpart;
     void* colsum;
+    bool dx_only = false;      // dw is not formed
 };
-// dw = nullptr: dx alone.
 int ptj_linear_bwd(const PtjLinearBwd& p, void* scratch, size_t scratch_bytes, int dtype, PtjPartialSums* later, hipStream_t st);
 
 // The weight gradients of several blocks in one launch: dw[kind][block] = d^T.x with d [k, n[kind]], x [k, m[kind]] and dw
