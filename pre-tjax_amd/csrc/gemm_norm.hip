@@ -270,6 +270,7 @@ bool ptj_norm_product_fits(int64_t rows, int64_t dim, int64_t m, int dtype, bool
 
 int ptj_norm_product(const PtjNormProduct& p, int64_t rows, int64_t dim, int64_t m, int dtype, hipStream_t st) {
     const NpTile t = np_tile(rows, dim, m, dtype);
+    PTJ_CHECK_ARG((p.x.part || p.x.c) && p.res && p.gamma && p.beta && p.w && p.y && p.c && (p.bias || !p.gelu), "norm_product: null pointer");
     bool ok = t.rows > 0;
     for (const void* q : {p.x.part ? (const void*)p.x.part : p.x.c, p.x.part ? p.x.bias : nullptr, p.res, p.gamma, p.beta, p.w, p.bias, (const void*)p.y,
                           (const void*)p.c})

@@ -45,3 +45,21 @@ def test_backward_refuses_missing_weight_gradients(dtype, layers, tokens, which)
 def test_backward_refuses_missing_weights(dtype, which):
     rc, message = backward(2, 64, dtype, missing_param=FIRST + BLOCK + which)
     assert rc == -1 and b"null" in message
+
+
+def forward(layers, tokens, dtype, keep, missing):
+    l = importlib.import_module("pre-tjax_amd._lib").lib()
+    big = 1 << 50
+    rc = l.ptj_gpt2_fwd(shape(layers, tokens, dtype), nest(layers, missing), 0x600000, None, None, 0x100000, big, keep, 0x200000,
+                        0x300000, 0x500000, big, None)
+    return rc, l.ptj_last_error()
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("keep", [0, 1])
+@pytest.mark.parametrize("tokens", [64, 4096])                 # bf16: each norm inside the product that reads it, or apart
+@pytest.mark.parametrize("which", [LN1G, LN1B, WQKV, WO, LN2G, LN2B, W1, B1, W2])
+def test_forward_refuses_missing_parameters(dtype, keep, tokens, which):
+    for block in (0, 1):
+        rc, message = forward(2, tokens, dtype, keep, FIRST + BLOCK * block + which)
+        assert rc == -1 and b"null" in message
