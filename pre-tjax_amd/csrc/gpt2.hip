@@ -203,7 +203,9 @@ int ptj_gpt2_fwd(const ptj_gpt2_shape* sp, const void* const* params, const int6
     STEP(check_shape("gpt2_fwd", sp));
     const ptj_gpt2_shape& s = *sp;
     PTJ_CHECK_ARG(params && tokens && acts && x_last && h && (!s.train || seeds), "gpt2_fwd: null pointer");
-    PTJ_CHECK_ARG(all_given(params, s.layers, {P_LN1G, P_LN1B, P_WQKV, P_WO, P_LN2G, P_LN2B, P_W1, P_B1, P_W2}), "gpt2_fwd: null parameter");
+    PTJ_CHECK_ARG(all_given(params, s.layers, {P_LN1G, P_LN1B, P_WQKV, P_WO, P_LN2G, P_LN2B, P_W1, P_B1, P_W2}) &&
+                      params[P_FIRST + s.layers * P_BLOCK] && params[P_FIRST + s.layers * P_BLOCK + 1],
+                  "gpt2_fwd: null parameter");
     const Layout l = make_layout(s, keep != 0);
     const Temps t = make_temps(s, false);
     if (acts_bytes < (size_t)l.total || !workspace || workspace_bytes < t.total)

@@ -63,3 +63,9 @@ def test_forward_refuses_missing_parameters(dtype, keep, tokens, which):
     for block in (0, 1):
         rc, message = forward(2, tokens, dtype, keep, FIRST + BLOCK * block + which)
         assert rc == -1 and b"null" in message
+
+
+@pytest.mark.parametrize("entry", [0, 1])
+def test_forward_refuses_a_missing_final_norm(entry):
+    rc, message = forward(2, 64, 1, 0, FIRST + BLOCK * 2 + entry)
+    assert rc == -1 and b"null" in message
