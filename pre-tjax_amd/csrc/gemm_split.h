@@ -169,9 +169,11 @@ struct GsCfg {
 
 // acc = the wavefront's TMW x TNW MFMA tiles (from row `row0` of A, column `col0` of B) by the fp32 matrix instructions,
 // operands straight from memory: for the rare tiles whose values the split does not take.  Every lane of the wavefront calls it.
-template <int TMW, int TNW>
+// CHAIN: as for gs_tile.
+template <int TMW, int TNW, int CHAIN>
 __device__ __forceinline__ void gs_plain_product(const GemmArgs& g, f32x16 (&acc)[TNW][TMW], int row0, int col0, int kbeg, int kend,
                                                  int lane) {
+    f32x16 total[TNW][TMW];
     const int lr = lane & 31, lg = lane >> 5;
     const float *pa[TMW], *pb[TNW];
 #pragma unroll
@@ -189,7 +191,7 @@ __device__ __forceinline__ void gs_plain_product(const GemmArgs& g, f32x16 (&acc
 #pragma unroll
         for (int j = 0; j < TMW; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = total[i][j][e] = 0.f;
 #pragma unroll 1
     for (int64_t k0 = kbeg; k0 < kend; k0 += 16) {
         f32x4 fa[2][TMW], fb[2][TNW];
@@ -216,11 +218,30 @@ __device__ __forceinline__ void gs_plain_product(const GemmArgs& g, f32x16 (&acc
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[i][j][e] += part[e];
             }
+        if constexpr (CHAIN > 0) {
+            if ((k0 - kbeg) % CHAIN == CHAIN - 16)
+#pragma unroll
+                for (int i = 0; i < TNW; ++i)
+#pragma unroll
+                    for (int j = 0; j < TMW; ++j)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            total[i][j][e] += acc[i][j][e];
+                            acc[i][j][e] = 0.f;
+                        }
+        }
     }
+    if constexpr (CHAIN > 0)
+#pragma unroll
+        for (int i = 0; i < TNW; ++i)
+#pragma unroll
+            for (int j = 0; j < TMW; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] += total[i][j][e];
 }
 
 // Both accumulators -> the tile of C: unscaled, formed again by the fp32 instructions where a sum is not finite, and written.
-template <typename C, bool MUL>
+template <typename C, bool MUL, int CHAIN = 0>
 __device__ __forceinline__ void gs_finish(const GemmArgs& g, f32x16 (&acc)[C::TNW][C::TMW], const f32x16 (&low)[C::TNW][C::TMW],
                                           char* __restrict__ smem, int row0, int col0, int z, int kbeg, int kend, int wave, int wm,
                                           int wn, int lane) {
@@ -241,12 +262,25 @@ __device__ __forceinline__ void gs_finish(const GemmArgs& g, f32x16 (&acc)[C::TN
                 acc[i][j][e] *= GS_UNSCALE;
             }
     if (__builtin_expect(__any(nan != nan) || kend - kbeg <= GS_PLAIN_K, 0))
-        gs_plain_product<C::TMW, C::TNW>(g, acc, row0 + wm * C::TMW * 32, col0 + wn * C::TNW * 32, kbeg, kend, lane);
+        gs_plain_product<C::TMW, C::TNW, CHAIN>(g, acc, row0 + wm * C::TMW * 32, col0 + wn * C::TNW * 32, kbeg, kend, lane);
     __syncthreads();
     gt_write_back<float, C, MUL>(g, acc, smem, row0, col0, z, wave, lane);
 }
 
-template <int AMODE, int BMODE, typename C, bool MUL>
+// A long contraction without a K split.  One accumulator over all its steps takes a rounding of the whole sum's size in each, where a
+// K split has short chains.  So with CHAIN elements a chain the accumulators are added to totals every CHAIN elements, and the
+// rounding of that addition starts the next chain (Dekker's fast two-sum: exact where the total is the larger one, else no worse
+// than a rounding).  Weight gradients of N(0,1) operands, 2-norm of the error relative to the result, as single products / one
+// chain / this: 768x768 over 4096 elements 1.06e-7 / 2.1e-7 / 7.8e-8, 768x3072 1.33e-7 / 2.1e-7 / 7.8e-8, over 1024 8.3e-8 / 1.14e-7 /
+// 7.7e-8; positive operands 768x768 over 1024 4.6e-8 / 9.4e-8 / 4.2e-8 (tests/test_gpu_weight_groups_error.py).  Chains of 512 would leave
+// more than the single products there.  The totals lie in LDS behind the planes, which the registers have no room for (238 of 256
+// are taken): a step of 8x512 fp32 tokens takes 0.9 % longer than with one chain (19.48 / 19.66 ms); with the roundings kept apart
+// in every fold (Knuth's two-sum, chains of 256) 1.5-2 %.
+constexpr int GS_CHAIN = 384;
+template <typename C> constexpr int gs_chain_smem = C::SMEM + C::TBM * C::TBN * 4;
+
+// CHAIN = 0: one chain
+template <int AMODE, int BMODE, typename C, bool MUL, int CHAIN = 0>
 __device__ __forceinline__ void gs_tile(const GemmArgs& g, int tile_m, int tile_n, int z, char* smem) {
     constexpr int BK = 32, TMW = C::TMW, TNW = C::TNW;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -277,6 +311,32 @@ __device__ __forceinline__ void gs_tile(const GemmArgs& g, int tile_m, int tile_
         for (int j = 0; j < TMW; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) { acc[i][j][e] = 0.f; low[i][j][e] = 0.f; }
+
+    // adds the accumulators to the thread's totals and leaves the rounding of that in their place; LAST: the totals, the rounding in `low`
+    f32x4* const total = (f32x4*)(smem + C::SMEM) + wave * (TNW * TMW * 4 * 64) + lane;
+    auto fold = [&](auto last) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TNW; ++i)
+#pragma unroll
+            for (int j = 0; j < TMW; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    f32x4& t = total[((i * TMW + j) * 4 + q) * 64];
+                    const f32x4 was = t;
+                    f32x4 sum;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float a = acc[i][j][q * 4 + e], s = was[e] + a, rest = a - (s - was[e]);
+                        sum[e] = s;
+                        acc[i][j][q * 4 + e] = last ? s : rest;
+                        if constexpr (last) low[i][j][q * 4 + e] += rest;
+                    }
+                    if constexpr (!last) t = sum;
+                }
+    };
+    if constexpr (CHAIN > 0)
+#pragma unroll
+        for (int i = 0; i < TNW * TMW * 4; ++i) total[i * 64] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     auto split_piece = [&](auto set, auto i, int buf) __attribute__((always_inline)) {
         if constexpr (i < OA::PER) oa.template split_store<set, i>(sA + buf * C::STAGE);
@@ -352,13 +412,16 @@ __device__ __forceinline__ void gs_tile(const GemmArgs& g, int tile_m, int tile_
             for (; kt + 1 < nk; kt += 2) {
                 step(I0, whole, kt);
                 step(I1, whole, kt + 1);
+                if constexpr (CHAIN > 0)
+                    if ((kt + 2) % (CHAIN / BK) == 0) fold(std::bool_constant<false>{});
             }
             if (kt < nk) step(I0, whole, kt);
+            if constexpr (CHAIN > 0) fold(std::bool_constant<true>{});
         };
         if (whole_vectors) all_steps(WHOLE);
         else all_steps(ANY);
     }
-    gs_finish<C, MUL>(g, acc, low, smem, row0, col0, z, kbeg, kend, wave, wm, wn, lane);
+    gs_finish<C, MUL, CHAIN>(g, acc, low, smem, row0, col0, z, kbeg, kend, wave, wm, wn, lane);
 }
 
 template <int AMODE, int BMODE, typename C, bool MUL>
@@ -372,7 +435,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_kernel(con
 // A tile of a group of products
 template <typename C>
 __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_group_kernel(const ptj_gemm_detail::GemmGroup group) {
-    __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
+    __shared__ __attribute__((aligned(1024))) char smem[gs_chain_smem<C>];
     int kind, block, tile_m, tile_n;
     group_tile<false>(group, blockIdx.x, C::TBM, C::TBN, kind, block, tile_m, tile_n);
     GemmArgs g{};
@@ -386,7 +449,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_group_kern
     g.a_k = g.n;
     g.b_k = g.c_rs = g.m;
     g.splits = g.tail_splits = g.vec_out = 1;
-    gs_tile<MNMAJOR, MNMAJOR, C, false>(g, tile_m, tile_n, 0, smem);
+    gs_tile<MNMAJOR, MNMAJOR, C, false, GS_CHAIN>(g, tile_m, tile_n, 0, smem);
 }
 template <typename C>
 int gs_group_launch(const PtjGradGroup& p, hipStream_t st) {
