@@ -20,10 +20,15 @@ struct ManyArgs {
     int count;
 };
 
+template <typename T, typename C>
+constexpr int many_smem() {
+    if constexpr (sizeof(T) == 2) return C::SMEM;
+    else return gs_chain_smem<C>;
+}
 // One tile of one of the products; operands along the contraction and across it (dX), or both across it (dW)
 template <typename T, typename C>
 __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_many_kernel(const ManyArgs a) {
-    __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
+    __shared__ __attribute__((aligned(1024))) char smem[many_smem<T, C>()];
     int i = 0;
 #pragma unroll
     for (int j = 1; j < MANY; ++j) i += j < a.count && (int)blockIdx.x >= a.first[j];
@@ -35,7 +40,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_many_kernel(cons
         } else {
             int tile_m, tile_n, z;
             gt_item(g, pid, (g.n + C::TBM - 1) / C::TBM, (g.m + C::TBN - 1) / C::TBN, tile_m, tile_n, z);
-            gs_tile<am, bm, C, false>(g, tile_m, tile_n, z, smem);
+            gs_tile<am, bm, C, false, GS_CHAIN>(g, tile_m, tile_n, z, smem);      // (the single products are K-split)
         }
     };
     constexpr std::integral_constant<int, KMAJOR> K{};

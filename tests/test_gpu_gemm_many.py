@@ -59,3 +59,20 @@ def test_outputs_off_the_grid(dtype):
     for (a, b), c, x in zip(pairs, outs, bufs):
         check(dtype, a, b, c)
         assert (x[1:].view(a.shape[0], -1)[:, b.shape[1]:] == 7.0).all() and x[0] == 7.0
+
+
+@pytest.mark.parametrize("rows", [64, 500, 777, 1500, 3001, 6000])
+@pytest.mark.parametrize("positive", [False, True])
+def test_fp32_sums_are_no_less_exact_than_the_single_products(mt, rows, positive):
+    """A feed-forward block's three products: a single one may be K-split, whose chains of additions are short."""
+    g = gen(rows)
+    shapes = [(768, 3072, rows, "tn"), (3072, 768, rows, "tn"), (rows, 768, 3072, "nn")]
+    pairs = [operands(g, torch.float32, *s) for s in shapes]
+    if positive:
+        pairs = [(a.abs(), b.abs()) for a, b in pairs]
+    for (a, b), c in zip(pairs, mt._matmul_many_t(*pairs)):
+        want = a.double() @ b.double()
+        error = [((x.double() - want).norm() / want.norm()).item() for x in (c, mt.matmul_t(a, b))]
+        print("rows=%d %dx%d positive=%d: together %.3g, alone %.3g" % (rows, *c.shape, positive, *error))
+        # two orders of the same roundings differ by chance, under 1 % over some 10^5 elements and more
+        assert error[0] <= 1.01 * error[1]
