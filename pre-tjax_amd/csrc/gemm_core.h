@@ -74,6 +74,7 @@ struct GemmArgs {
 struct GemmGroup {
     PtjGradGroup p;
     int first[PtjGradGroup::KINDS + 1];
+    int chain[PtjGradGroup::KINDS];     // gemm_split.h
 };
 int launch_plain_f32(const GemmArgs& g, int splits, hipStream_t st);   // gemm_f32.hip
 // gemm_tile_bf16.hip, gemm_tile_f32.hip: configuration `cfg` of the one-tile-per-workgroup kernels (gemm_plan.h), with
@@ -519,7 +520,7 @@ __device__ __forceinline__ void group_tile(const ptj_gemm_detail::GemmGroup& g, 
 }
 template <typename C>
 ptj_gemm_detail::GemmGroup group_of(const PtjGradGroup& p) {
-    ptj_gemm_detail::GemmGroup g = {p, {}};
+    ptj_gemm_detail::GemmGroup g = {p, {}, {}};
     for (int i = 0; i < PtjGradGroup::KINDS; ++i)
         g.first[i + 1] = g.first[i] + ((p.n[i] + C::TBM - 1) / C::TBM) * ((p.m[i] + C::TBN - 1) / C::TBN);
     return g;

@@ -3,8 +3,8 @@
 // longest tiles go first.  One launch or one product after the other is chosen by estimate (together): the time of all tiles on CUs
 // that take the next one as they end one, against the estimates of gemm_plan.  Feed-forward block, forward and backward, 768 wide, three
 // launches / chosen, us: bf16 777 tokens 97.8 / 92.1, 1500 140.3 / 124.8, 3001 185.5 / 167.2, 4096 205.9 / 190.1, 8192 379 / 353, 11000 478 / 464,
-// 16384 (apart; together 648) 608; fp32 64 (apart; together 155) 102, 1500 411 / 376, 3001 722 / 677, 6000 1312 / 1273; bf16 3001 tokens 512 wide
-// 119 / 106, 1600 wide 504 / 491; nowhere slower by more than what two runs differ by.
+// 16384 (apart; together 648) 608; fp32 64 (apart; together 155) 102, 1500 416 / 389, 3001 720 / 689, 4096 872 / 857, 6000 1324 / 1317, 1000
+// and 8192 apart; bf16 3001 tokens 512 wide 119 / 106, 1600 wide 504 / 491; nowhere slower by more than what two runs differ by.
 #include "gemm_tile_launch.h"
 #include "gemm_plan.h"
 
@@ -17,6 +17,7 @@ struct ManyArgs {
     GemmArgs g[MANY];
     int first[MANY + 1];     // tiles in front of each product
     int modes[MANY];         // operand layouts
+    int chain[MANY];         // fp32: gemm_split.h
     int count;
 };
 
@@ -40,7 +41,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_many_kernel(cons
         } else {
             int tile_m, tile_n, z;
             gt_item(g, pid, (g.n + C::TBM - 1) / C::TBM, (g.m + C::TBN - 1) / C::TBN, tile_m, tile_n, z);
-            gs_tile<am, bm, C, false, GS_CHAIN>(g, tile_m, tile_n, z, smem);      // (the single products are K-split)
+            gs_tile<am, bm, C, false, true>(g, tile_m, tile_n, z, smem, a.chain[i]);
         }
     };
     constexpr std::integral_constant<int, KMAJOR> K{};
@@ -56,12 +57,15 @@ int launch_many(const ManyArgs& a, hipStream_t st) {
     return PTJ_OK;
 }
 
+// fp32: a step with the totals of gs_tile beside it, relative to one without (3001 to 8192 rows: 1.04 to 1.06)
+constexpr double MANY_CHAINS = 1.05;
+
 // Time of the tiles of all products, in the order of the grid, on CUs that take the next one as they end one
-double makespan(const ManyArgs& a, const TileCost& c, int cus) {
+double makespan(const ManyArgs& a, const TileCost& c, int cus, double slower) {
     struct Group { double at; int64_t count; };           // CUs that are free from then on, in order of time
     Group free[MANY + 2] = {{0.0, cus}};                  // (a product takes whole groups and part of one more)
     int groups = 1;
-    const double step = gp_step_us(c, a.first[a.count], cus);
+    const double step = gp_step_us(c, a.first[a.count], cus) * slower;
     double last = 0.0;
     for (int i = 0; i < a.count; ++i) {
         const double tile = (double)gp_ceil(a.g[i].k, c.bkt) * step + c.finish;
@@ -82,20 +86,29 @@ double makespan(const ManyArgs& a, const TileCost& c, int cus) {
     return c.start + last;
 }
 
-// Whether one launch is estimated to be faster, kept for the sizes asked for last
-bool together(const ManyArgs& a, int elt) {
+// Whether one launch is estimated to be faster, and its chains of additions; kept for the sizes asked for last
+bool together(ManyArgs& a, int elt) {
     struct Key { int n[MANY], m[MANY], k[MANY], count, elt, cus; };
     static thread_local Key last = {};
     static thread_local bool answer = false;
+    static thread_local int chain[MANY] = {};
     const int cus = num_cus();
     Key key = {};
     key.count = a.count; key.elt = elt; key.cus = cus;
     for (int i = 0; i < a.count; ++i) { key.n[i] = a.g[i].n; key.m[i] = a.g[i].m; key.k[i] = a.g[i].k; }
-    if (memcmp(&key, &last, sizeof(key)) == 0) return answer;
-    double apart = 0.0;
-    for (int i = 0; i < a.count; ++i) apart += gemm_plan(a.g[i].n, a.g[i].m, a.g[i].k, elt, (size_t)-1, cus).us;
-    answer = makespan(a, elt == 2 ? GT_COST[0][3] : GT_COST[1][4], cus) < apart;
-    last = key;
+    if (memcmp(&key, &last, sizeof(key)) != 0) {
+        double apart = 0.0;
+        for (int i = 0; i < a.count; ++i) {
+            const GemmPlan p = gemm_plan(a.g[i].n, a.g[i].m, a.g[i].k, elt, (size_t)-1, cus);
+            apart += p.us;
+            chain[i] = gs_chain(p.kps, a.g[i].k);
+        }
+        // (fp32: launches that follow each other do not wait for their start twice: 1000 rows apart 119 us, estimated 129, together 129)
+        answer = elt == 2 ? makespan(a, GT_COST[0][3], cus, 1.0) < apart
+                          : makespan(a, GT_COST[1][4], cus, MANY_CHAINS) < apart - (a.count - 1) * GT_COST[1][4].start;
+        last = key;
+    }
+    memcpy(a.chain, chain, sizeof(chain));
     return answer;
 }
 

@@ -169,10 +169,10 @@ struct GsCfg {
 
 // acc = the wavefront's TMW x TNW MFMA tiles (from row `row0` of A, column `col0` of B) by the fp32 matrix instructions,
 // operands straight from memory: for the rare tiles whose values the split does not take.  Every lane of the wavefront calls it.
-// CHAIN: as for gs_tile.
-template <int TMW, int TNW, int CHAIN>
+// LONG, chain: as for gs_tile.
+template <int TMW, int TNW, bool LONG>
 __device__ __forceinline__ void gs_plain_product(const GemmArgs& g, f32x16 (&acc)[TNW][TMW], int row0, int col0, int kbeg, int kend,
-                                                 int lane) {
+                                                 int lane, int chain) {
     f32x16 total[TNW][TMW];
     const int lr = lane & 31, lg = lane >> 5;
     const float *pa[TMW], *pb[TNW];
@@ -218,8 +218,8 @@ __device__ __forceinline__ void gs_plain_product(const GemmArgs& g, f32x16 (&acc
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[i][j][e] += part[e];
             }
-        if constexpr (CHAIN > 0) {
-            if ((k0 - kbeg) % CHAIN == CHAIN - 16)
+        if constexpr (LONG) {
+            if ((k0 - kbeg + 16) % (chain * 32) == 0)
 #pragma unroll
                 for (int i = 0; i < TNW; ++i)
 #pragma unroll
@@ -231,7 +231,7 @@ __device__ __forceinline__ void gs_plain_product(const GemmArgs& g, f32x16 (&acc
                         }
         }
     }
-    if constexpr (CHAIN > 0)
+    if constexpr (LONG)
 #pragma unroll
         for (int i = 0; i < TNW; ++i)
 #pragma unroll
@@ -241,10 +241,10 @@ __device__ __forceinline__ void gs_plain_product(const GemmArgs& g, f32x16 (&acc
 }
 
 // Both accumulators -> the tile of C: unscaled, formed again by the fp32 instructions where a sum is not finite, and written.
-template <typename C, bool MUL, int CHAIN = 0>
+template <typename C, bool MUL, bool LONG = false>
 __device__ __forceinline__ void gs_finish(const GemmArgs& g, f32x16 (&acc)[C::TNW][C::TMW], const f32x16 (&low)[C::TNW][C::TMW],
                                           char* __restrict__ smem, int row0, int col0, int z, int kbeg, int kend, int wave, int wm,
-                                          int wn, int lane) {
+                                          int wn, int lane, int chain = 0) {
 #pragma unroll
     for (int i = 0; i < C::TNW; ++i)
 #pragma unroll
@@ -262,26 +262,28 @@ __device__ __forceinline__ void gs_finish(const GemmArgs& g, f32x16 (&acc)[C::TN
                 acc[i][j][e] *= GS_UNSCALE;
             }
     if (__builtin_expect(__any(nan != nan) || kend - kbeg <= GS_PLAIN_K, 0))
-        gs_plain_product<C::TMW, C::TNW, CHAIN>(g, acc, row0 + wm * C::TMW * 32, col0 + wn * C::TNW * 32, kbeg, kend, lane);
+        gs_plain_product<C::TMW, C::TNW, LONG>(g, acc, row0 + wm * C::TMW * 32, col0 + wn * C::TNW * 32, kbeg, kend, lane, chain);
     __syncthreads();
     gt_write_back<float, C, MUL>(g, acc, smem, row0, col0, z, wave, lane);
 }
 
-// A long contraction without a K split.  One accumulator over all its steps takes a rounding of the whole sum's size in each, where a
-// K split has short chains.  So with CHAIN elements a chain the accumulators are added to totals every CHAIN elements, and the
-// rounding of that addition starts the next chain (Dekker's fast two-sum: exact where the total is the larger one, else no worse
-// than a rounding).  Weight gradients of N(0,1) operands, 2-norm of the error relative to the result, as single products / one
-// chain / this: 768x768 over 4096 elements 1.06e-7 / 2.1e-7 / 7.8e-8, 768x3072 1.33e-7 / 2.1e-7 / 7.8e-8, over 1024 8.3e-8 / 1.14e-7 /
-// 7.7e-8; positive operands 768x768 over 1024 4.6e-8 / 9.4e-8 / 4.2e-8 (tests/test_gpu_weight_groups_error.py).  Chains of 512 would leave
-// more than the single products there.  The totals lie in LDS behind the planes, which the registers have no room for (238 of 256
-// are taken): a step of 8x512 fp32 tokens takes 0.9 % longer than with one chain (19.48 / 19.66 ms); with the roundings kept apart
-// in every fold (Knuth's two-sum, chains of 256) 1.5-2 %.
-constexpr int GS_CHAIN = 384;
+// LONG: a long contraction whose K split is left out.  One accumulator over all its steps would take a rounding of the whole sum's size
+// in each, where a K split has short chains.  So the accumulators are added to totals every `chain` steps, and the rounding of that
+// addition starts the next chain (Dekker's fast two-sum: exact where the total is the larger one, else no worse than a rounding).
+// Chains are as long as the parts of the K split that the product would have by itself (gs_chain).  Weight gradients of N(0,1)
+// operands, 2-norm of the error against fp64 relative to the result, single products / one chain / this: 768x768 over 4096
+// elements 1.06e-7 / 2.1e-7 / 9.1e-8, 768x3072 1.33e-7 / 2.1e-7 / 1.28e-7, 768x768 over 1024 8.3e-8 / 1.14e-7 / 7.3e-8
+// (tests/test_gpu_weight_groups_error.py).  The totals lie in LDS behind the planes, which the registers have no room for (238 of 256
+// are taken).  Weight gradients of twelve blocks, 4096 elements: 4.03 ms in one chain, 4.22 so, 4.14 of it without a fold (the compiler
+// orders the loop in another way).  A chain of 256, 384, 512 elements whatever the product: 4.27, 4.24, 4.21; the loads of a step wait for
+// each other where the folds are a branch in the loop instead of a loop around it.
 template <typename C> constexpr int gs_chain_smem = C::SMEM + C::TBM * C::TBN * 4;
 
-// CHAIN = 0: one chain
-template <int AMODE, int BMODE, typename C, bool MUL, int CHAIN = 0>
-__device__ __forceinline__ void gs_tile(const GemmArgs& g, int tile_m, int tile_n, int z, char* smem) {
+// steps, an even number, for parts of so many elements of k (below 2^20); of one part: more than there are
+inline int gs_chain(int part, int k) { return part < 64 || part >= k ? 1 << 20 : part / 64 * 2; }
+
+template <int AMODE, int BMODE, typename C, bool MUL, bool LONG = false>
+__device__ __forceinline__ void gs_tile(const GemmArgs& g, int tile_m, int tile_n, int z, char* smem, int chain = 0) {
     constexpr int BK = 32, TMW = C::TMW, TNW = C::TNW;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -312,9 +314,11 @@ __device__ __forceinline__ void gs_tile(const GemmArgs& g, int tile_m, int tile_
 #pragma unroll
             for (int e = 0; e < 16; ++e) { acc[i][j][e] = 0.f; low[i][j][e] = 0.f; }
 
-    // adds the accumulators to the thread's totals and leaves the rounding of that in their place; LAST: the totals, the rounding in `low`
+    // FIRST: the accumulators become the thread's totals; else they are added to them and the rounding of that is left in their place;
+    // LAST: the totals there, the rounding in `low`
+    enum { FIRST, MORE, LAST };
     f32x4* const total = (f32x4*)(smem + C::SMEM) + wave * (TNW * TMW * 4 * 64) + lane;
-    auto fold = [&](auto last) __attribute__((always_inline)) {
+    auto fold = [&](auto which) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < TNW; ++i)
 #pragma unroll
@@ -322,21 +326,18 @@ __device__ __forceinline__ void gs_tile(const GemmArgs& g, int tile_m, int tile_
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     f32x4& t = total[((i * TMW + j) * 4 + q) * 64];
-                    const f32x4 was = t;
-                    f32x4 sum;
+                    f32x4 was{}, sum;
+                    if constexpr (which != FIRST) was = t;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const float a = acc[i][j][q * 4 + e], s = was[e] + a, rest = a - (s - was[e]);
-                        sum[e] = s;
-                        acc[i][j][q * 4 + e] = last ? s : rest;
-                        if constexpr (last) low[i][j][q * 4 + e] += rest;
+                        sum[e] = which == FIRST ? a : s;
+                        acc[i][j][q * 4 + e] = which == FIRST ? 0.f : which == LAST ? s : rest;
+                        if constexpr (which == LAST) low[i][j][q * 4 + e] += rest;
                     }
-                    if constexpr (!last) t = sum;
+                    if constexpr (which != LAST) t = sum;
                 }
     };
-    if constexpr (CHAIN > 0)
-#pragma unroll
-        for (int i = 0; i < TNW * TMW * 4; ++i) total[i * 64] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     auto split_piece = [&](auto set, auto i, int buf) __attribute__((always_inline)) {
         if constexpr (i < OA::PER) oa.template split_store<set, i>(sA + buf * C::STAGE);
@@ -409,19 +410,28 @@ __device__ __forceinline__ void gs_tile(const GemmArgs& g, int tile_m, int tile_
         __syncthreads();
         auto all_steps = [&](auto whole) __attribute__((always_inline)) {
             int kt = 0;
+            if constexpr (LONG) {
+                for (int end = chain; end + 1 < nk; end += chain) {
+                    for (; kt < end; kt += 2) {
+                        step(I0, whole, kt);
+                        step(I1, whole, kt + 1);
+                    }
+                    if (end == chain) fold(std::integral_constant<int, FIRST>{});
+                    else fold(std::integral_constant<int, MORE>{});
+                }
+            }
             for (; kt + 1 < nk; kt += 2) {
                 step(I0, whole, kt);
                 step(I1, whole, kt + 1);
-                if constexpr (CHAIN > 0)
-                    if ((kt + 2) % (CHAIN / BK) == 0) fold(std::bool_constant<false>{});
             }
             if (kt < nk) step(I0, whole, kt);
-            if constexpr (CHAIN > 0) fold(std::bool_constant<true>{});
+            if constexpr (LONG)
+                if (chain + 1 < nk) fold(std::integral_constant<int, LAST>{});
         };
         if (whole_vectors) all_steps(WHOLE);
         else all_steps(ANY);
     }
-    gs_finish<C, MUL, CHAIN>(g, acc, low, smem, row0, col0, z, kbeg, kend, wave, wm, wn, lane);
+    gs_finish<C, MUL, LONG>(g, acc, low, smem, row0, col0, z, kbeg, kend, wave, wm, wn, lane, chain);
 }
 
 template <int AMODE, int BMODE, typename C, bool MUL>
@@ -449,11 +459,13 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_EU) void gemm_split_group_kern
     g.a_k = g.n;
     g.b_k = g.c_rs = g.m;
     g.splits = g.tail_splits = g.vec_out = 1;
-    gs_tile<MNMAJOR, MNMAJOR, C, false, GS_CHAIN>(g, tile_m, tile_n, 0, smem);
+    gs_tile<MNMAJOR, MNMAJOR, C, false, true>(g, tile_m, tile_n, 0, smem, group.chain[kind]);
 }
+// parts[kind]: what the K split of a single product would be
 template <typename C>
-int gs_group_launch(const PtjGradGroup& p, hipStream_t st) {
-    const ptj_gemm_detail::GemmGroup g = group_of<C>(p);
+int gs_group_launch(const PtjGradGroup& p, const int (&parts)[PtjGradGroup::KINDS], hipStream_t st) {
+    ptj_gemm_detail::GemmGroup g = group_of<C>(p);
+    for (int i = 0; i < PtjGradGroup::KINDS; ++i) g.chain[i] = gs_chain(parts[i], p.k);
     hipLaunchKernelGGL((gemm_split_group_kernel<C>), dim3((unsigned)(g.first[PtjGradGroup::KINDS] * p.blocks)), dim3(C::THREADS), 0, st, g);
     PTJ_CHECK_LAUNCH();
     return PTJ_OK;
