@@ -40,6 +40,7 @@ extern "C" {
 #define PTJ_EPI_BIAS_GELU 2      /* C = gelu(A.B + bias[m])                 */
 #define PTJ_EPI_BIAS_GELU_DERIV 3 /* the same C; c_pre = gelu'(A.B + bias[m]) */
 #define PTJ_EPI_ACCUMULATE 4     /* C = C + A.B (C is read, widened, and rounded once more) */
+#define PTJ_EPI_BIAS_NORM 5      /* PTJ_EPI_BIAS in the order of summation of ptj_gpt2_fwd, below */
 
 int ptj_version(void);
 const char* ptj_last_error(void);
@@ -261,7 +262,9 @@ int ptj_ce_fwd_bwd_colsum_rows(const int64_t* labels, const void* logits, float*
  * PTJ_EPI_ACCUMULATE (no bias; 2-byte storage, 16-byte aligned operands with unit stride along one
  * axis, k a multiple of 64, no K split: anything else is refused) starts the fp32 accumulators from
  * the stored C: a weight gradient summed over row chunks of the batch (the reference forms it in one
- * product over all rows, model_triton.py:423-428). */
+ * product over all rows, model_triton.py:423-428).
+ * PTJ_EPI_BIAS_NORM chooses a K split as if the consumer added up its partial sums, as the norm behind a
+ * feed-forward block does in ptj_gpt2_fwd: the bits of that call, for the same sequence of single calls. */
 size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype);
 int ptj_gemm(const void* a, const void* b, void* c, const void* bias,
              int64_t n, int64_t m, int64_t k,

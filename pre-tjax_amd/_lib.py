@@ -13,7 +13,7 @@ LIB_PATH = os.path.join(_HERE, "libptj.so")
 
 PTJ_F32, PTJ_BF16 = 0, 1
 EMBED_SCAN_MAX = 8192     # PTJ_EMBED_SCAN_MAX
-EPI_NONE, EPI_BIAS, EPI_BIAS_GELU, EPI_BIAS_GELU_DERIV, EPI_ACCUMULATE = 0, 1, 2, 3, 4
+EPI_NONE, EPI_BIAS, EPI_BIAS_GELU, EPI_BIAS_GELU_DERIV, EPI_ACCUMULATE, EPI_BIAS_NORM = 0, 1, 2, 3, 4, 5
 
 _c = ctypes
 _p, _i64, _int, _sz = _c.c_void_p, _c.c_int64, _c.c_int, _c.c_size_t

@@ -28,7 +28,9 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
              size_t workspace_bytes, int dtype, void* stream, PtjPartialProduct* later) {
     PTJ_CHECK_ARG(n >= 0 && m >= 0 && k >= 0, "gemm: negative dimension");
     PTJ_CHECK_ARG(n < (1ll << 31) && m < (1ll << 31) && k < (1ll << 31), "gemm: dimension exceeds 31 bits");
-    PTJ_CHECK_ARG(epilogue >= PTJ_EPI_NONE && epilogue <= PTJ_EPI_ACCUMULATE, "gemm: unknown epilogue %d", epilogue);
+    PTJ_CHECK_ARG(epilogue >= PTJ_EPI_NONE && epilogue <= PTJ_EPI_BIAS_NORM, "gemm: unknown epilogue %d", epilogue);
+    const bool norm = epilogue == PTJ_EPI_BIAS_NORM;
+    if (norm) epilogue = PTJ_EPI_BIAS;
     PTJ_CHECK_ARG(epilogue != PTJ_EPI_BIAS_GELU_DERIV || c_pre, "gemm: the derivative epilogue needs its second output");
     PTJ_CHECK_ARG(epilogue == PTJ_EPI_NONE || epilogue == PTJ_EPI_ACCUMULATE || bias, "gemm: epilogue %d needs a bias", epilogue);
     PTJ_CHECK_ARG(epilogue != PTJ_EPI_ACCUMULATE || (!bias && !c_pre && dtype == PTJ_BF16),
@@ -65,9 +67,8 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
     if (bias) outputs_aligned = outputs_aligned && (reinterpret_cast<uintptr_t>(bias) % (4 * (size_t)elt)) == 0;
     const bool aligned_ws = workspace && ptj_aligned16(workspace);
     const int loose = ragged ? LOOSE_OPERAND : outputs_aligned ? ALIGNED : LOOSE_OUTPUT;
-    // a bias without an activation: the end of a feed-forward block, whose partial sums the next norm adds up.  (Whether this caller
-    // is the one that leaves them does not count: the bits of a product depend on its plan.)
-    const bool left = epilogue == PTJ_EPI_BIAS && !ragged && m % 4 == 0;
+    // (whether this caller leaves the partial sums or adds them up does not count: the bits of a product depend on its plan)
+    const bool left = norm && !ragged && m % 4 == 0;
     GemmPlan plan = {-1, 1, 0, 0, 1, 0, 0.0};
     if (epilogue == PTJ_EPI_ACCUMULATE) {
         // only the ring kernels start their accumulators from the stored C
@@ -152,6 +153,6 @@ int ptj_gemm_partial(const void* a, const void* b, void* c, const void* bias, in
                      int64_t a_cs, int64_t b_rs, int64_t b_cs, void* workspace, size_t workspace_bytes, int dtype,
                      hipStream_t st, PtjPartialProduct* out) {
     *out = {c, nullptr, 0, bias};
-    return gemm_any(a, b, c, bias, n, m, k, a_rs, a_cs, b_rs, b_cs, m, bias ? PTJ_EPI_BIAS : PTJ_EPI_NONE, nullptr, 0, workspace,
+    return gemm_any(a, b, c, bias, n, m, k, a_rs, a_cs, b_rs, b_cs, m, bias ? PTJ_EPI_BIAS_NORM : PTJ_EPI_NONE, nullptr, 0, workspace,
                     workspace_bytes, dtype, (void*)st, out);
 }

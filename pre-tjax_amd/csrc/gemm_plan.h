@@ -92,8 +92,10 @@ inline int64_t gp_ceil(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Second stage of a K split: its launch, and the partial sums written and read once more.  (bf16: 4.9 us and 0.23 fit best; the
 // launch is taken lower because behind a feed-forward block the next norm adds up the partial sums without one.)
-// `later`, bf16: that is likely, and costs the norm 1.6 us and some more for the bytes.  Second feed-forward product in a forward: 512 tokens
-// in two parts of 64x64 685 us, with 32x64 tiles whole 645; 1536 tokens in three of 128x128 1113, with 64x128 whole 1132.
+// `later`, bf16: it does, and pays 1.6 us and some more for the bytes.  Second feed-forward product in a forward: 512 tokens
+// in two parts of 64x64 685 us, with 32x64 tiles whole 645; 1536 tokens in three of 128x128 1113, with 64x128 whole 1132.  A
+// product with a bias that runs its second stage itself is planned at the full cost: 750x768x3072 15.6 us with the cost of `later`, 12.3 with
+// the full one, 1450x768x3072 20.1 / 16.9.
 inline double gp_reduce_us(int64_t n, int64_t m, int splits, int elt, bool later = false) {
     if (splits <= 1) return 0.0;
     const double bytes = 4.0 * (double)splits * (double)n * (double)m;
@@ -139,7 +141,7 @@ inline double gp_ring_tail_us(const TileCost& c, int64_t n, int64_t m, int64_t k
 // product with another epilogue add in the same order.  `loose`: operands or outputs that do not come in aligned
 // 16-byte vectors; the ring kernels take such operands not at all and write such outputs element by element (twice the
 // time at k = 768), the tile kernels write any.
-// `later`: the consumer usually adds up the partial sums of a K split.
+// `later`: the consumer adds up the partial sums of a K split (PTJ_EPI_BIAS_NORM).
 // `planes_ws`: workspace for operands split ahead of a product without a K split, where partial sums may not take any.
 inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int cus, int loose = ALIGNED,
                           int kernels = ANY_KERNEL, size_t planes_ws = 0, bool later = false) {

@@ -270,8 +270,8 @@ int ptj_gpt2_fwd(const ptj_gpt2_shape* sp, const void* const* params, const int6
         if (vectors)
             STEP(ptj_gemm_partial(a + l.g1, w[P_W2], ws + t.t1, w[P_B2], N, D, F, F, 1, 1, F, scratch, sb, dt, st, &f2));
         else
-            STEP(ptj_gemm(a + l.g1, w[P_W2], ws + t.t1, w[P_B2], N, D, F, F, 1, 1, F, D, PTJ_EPI_BIAS, nullptr, 0, scratch, sb, dt,
-                          stream));
+            STEP(ptj_gemm(a + l.g1, w[P_W2], ws + t.t1, w[P_B2], N, D, F, F, 1, 1, F, D, PTJ_EPI_BIAS_NORM, nullptr, 0, scratch, sb,
+                          dt, stream));
         if (inside && !last && ptj_norm_product_fits(N, D, 3 * D, dt, f2.part != nullptr)) entry = {f2, a + l.xmid, nx[0], nx[1], nullptr, nullptr, xo, nullptr, 0};
         else
             STEP(ptj_dropout_add_layernorm_of(f2, a + l.xmid, nx[0], nx[1], xo, ho, kb ? a + l.keep2 : nullptr, N, D, train, s2, dt,

@@ -291,7 +291,7 @@ def colsum_t(x: torch.Tensor, out=None):
 # GEMM  (reference: model_triton.py:373-398 t_matmul_t, :1258-1313 t_tlayer_ffn_fwd_t)
 # ----------------------------------------------------------------------------------
 def matmul_t(a: torch.Tensor, b: torch.Tensor, bias=None, gelu=False, out=None, pre_out=None, deriv_out=None,
-             accumulate=False):
+             accumulate=False, *, norm_follows=False):
     """``out[N,M] = a[N,K] @ b[K,M] (+ bias[M]) (tanh-GELU)`` on the MFMA GEMM kernel.
 
     `a` and `b` are 2-D tensors with arbitrary strides (``.t()`` views are consumed in
@@ -300,7 +300,8 @@ def matmul_t(a: torch.Tensor, b: torch.Tensor, bias=None, gelu=False, out=None, 
     receives ``a @ b + bias`` before the activation; `deriv_out` (instead) receives the
     GELU's derivative there, which is all the backward pass needs of it.  With
     ``accumulate=True`` the product is added onto the given `out` (the accumulators start from
-    it): a weight gradient summed over row chunks."""
+    it): a weight gradient summed over row chunks.  ``norm_follows=True`` (with a bias alone) adds in the
+    order in which the native stack leaves its sums to the next norm."""
     require_gpu(a, b, bias, out)
     assert a.dim() == 2 and b.dim() == 2 and a.shape[1] == b.shape[0], (a.shape, b.shape)
     assert a.dtype == b.dtype
@@ -321,7 +322,7 @@ def matmul_t(a: torch.Tensor, b: torch.Tensor, bias=None, gelu=False, out=None, 
     if bias is not None:
         assert bias.dtype == a.dtype and bias.numel() == M
         bias = bias.contiguous()
-        epi = _lib.EPI_BIAS_GELU if gelu else _lib.EPI_BIAS
+        epi = _lib.EPI_BIAS_GELU if gelu else _lib.EPI_BIAS_NORM if norm_follows else _lib.EPI_BIAS
     else:
         assert not gelu, "GELU epilogue is defined on top of the bias epilogue"
     code = dtype_code(a)
@@ -673,7 +674,7 @@ def t_gpt2_tlayer_fwd3_t(layer_params, y, mask, train=True, p_gen_aux=None, h1=N
     x_mid, h2, keep1 = dropout_add_layernorm_t(a_out, x_in, (ln2g, ln2b), train, p_gen_aux[1], want_keep=True)
     f1 = torch.empty((N, w1.shape[0]), dtype=y.dtype, device=y.device)  # gelu'(h2 @ W1^T + b1)
     g1 = matmul_t(h2, w1.t(), b1, gelu=True, deriv_out=f1)             # bias + GELU epilogue; its derivative kept
-    f2 = matmul_t(g1, w2.t(), b2)
+    f2 = matmul_t(g1, w2.t(), b2, norm_follows=True)
     if next_ln is not None:
         x_out, h_next, keep2 = dropout_add_layernorm_t(f2, x_mid, next_ln, train, p_gen_aux[2], want_keep=True)
     else:
