@@ -6,6 +6,10 @@
 
 namespace {
 
+uint64_t plan_hash(int64_t n, int64_t m, int64_t k) {
+    return ((uint64_t)n * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)m * 0xC2B2AE3D27D4EB4Full) ^ ((uint64_t)k * 0x165667B19E3779F9ull);
+}
+
 // gemm_plan through a small per-thread table: a training loop asks for the same few dozen products again and again,
 // and the estimate over all tile shapes and splits takes a microsecond.
 GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int loose, int kernels = ANY_KERNEL, bool later = false) {
@@ -13,8 +17,8 @@ GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, 
     constexpr int ENTRIES = 128;
     static thread_local Entry table[ENTRIES] = {};
     const int cus = num_cus();
-    const uint64_t h = ((uint64_t)n * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)m * 0xC2B2AE3D27D4EB4Full) ^
-                       ((uint64_t)k * 0x165667B19E3779F9ull) ^ ((uint64_t)(ws_bytes + loose + later) * 0xD6E8FEB86659FD93ull);
+    const uint64_t kind = (((uint64_t)loose * 2 + kernels) * 2 + later) * 2 + (elt == 2);
+    const uint64_t h = plan_hash(n, m, k) ^ (((uint64_t)ws_bytes * 32 + kind) * 0xD6E8FEB86659FD93ull);
     Entry& e = table[(h >> 40) % ENTRIES];
     if (e.n != n || e.m != m || e.k != k || e.ws != ws_bytes || e.elt != elt || e.cus != cus || e.loose != loose ||
         e.kernels != kernels || e.later != later)
@@ -124,19 +128,28 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
 
 extern "C" {
 
+// Every wrapper asks before it launches, so the answers are kept, per thread: worked out again for each product they took 5-10 us
+// (twelve plans), looked up 0.2.
 size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
     if (n <= 0 || m <= 0 || k <= 0) return 0;
+    struct Entry { int64_t n, m, k; int elt, cus; size_t need; };
+    constexpr int ENTRIES = 128;
+    static thread_local Entry table[ENTRIES] = {};
+    const int elt = dtype == PTJ_BF16 ? 2 : 4, cus = num_cus();
+    Entry& e = table[(plan_hash(n, m, k) + (uint64_t)elt * 0xD6E8FEB86659FD93ull) >> 40 & (ENTRIES - 1)];
+    if (e.n == n && e.m == m && e.k == k && e.elt == elt && e.cus == cus) return e.need;
     // which kernels run depends on the operands' strides and alignment as well: enough for any
-    const int elt = dtype == PTJ_BF16 ? 2 : 4;
     const int s = choose_splits(n, m, k, elt, (size_t)-1);
     int first, ts, tkps;
     size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
     for (const int loose : {ALIGNED, LOOSE_OUTPUT, LOOSE_OPERAND})
         for (const int kernels : {ANY_KERNEL, RING_ONLY})
             for (const bool later : {false, true}) {
-                const size_t bytes = gp_workspace_bytes(cached_plan(n, m, k, elt, (size_t)-1, loose, kernels, later), n, m, k);
+                if (elt != 2 && (later || kernels == RING_ONLY)) continue;      // bf16 alone tells these apart
+                const size_t bytes = gp_workspace_bytes(gemm_plan(n, m, k, elt, (size_t)-1, cus, loose, kernels, 0, later), n, m, k);
                 if (bytes > need) need = bytes;
             }
+    e = {n, m, k, elt, cus, need};
     return need;
 }
 
