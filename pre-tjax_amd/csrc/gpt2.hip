@@ -95,13 +95,12 @@ PtjGradGroup grad_group(const ptj_gpt2_shape& s, int64_t blocks) {
     }
     return g;
 }
-// How many blocks' weight gradients are formed in one launch: all of them, in equal parts of up to PtjGradGroup::BLOCKS, where
-// such a part has a round of tiles (gemm_group.hip), else 0.  A single block stays with the pairs: a round of its tiles takes a width of 1024.
+// How many blocks' weight gradients are formed in one launch (gemm_group.hip), 0: none.  A single block stays with the pairs: a round of
+// its tiles takes a width of 1024.
 int64_t grad_group_blocks(const ptj_gpt2_shape& s) {
     const int64_t N = s.batch * s.seq, D = s.dim, F = s.ffn, most = 1 << 20;
     if (s.layers < 2 || N >= most || F >= most || 3 * D >= most || F % 8 != 0) return 0;
-    const int64_t parts = (s.layers + PtjGradGroup::BLOCKS - 1) / PtjGradGroup::BLOCKS, blocks = (s.layers + parts - 1) / parts;
-    return ptj_weight_grads_fill(grad_group(s, blocks), (int)s.dtype) ? blocks : 0;
+    return ptj_weight_grads_blocks(grad_group(s, 1), s.layers, (int)s.dtype);
 }
 
 // `together`: weight gradients in groups where grad_group_blocks says so

@@ -110,5 +110,6 @@ struct PtjGradGroup {
     void* dw[KINDS][BLOCKS];
 };
 int ptj_weight_grads(const PtjGradGroup& p, int dtype, hipStream_t st);
-// Whether the launch has a round of tiles or more; sizes alone count.
-bool ptj_weight_grads_fill(const PtjGradGroup& p, int dtype);
+// How many blocks of `layers` to form in one launch (sizes alone count): the fewest whose launches, of so many blocks and one of the
+// rest, take no longer than larger ones; 0: no launch would have a round of tiles.
+int ptj_weight_grads_blocks(PtjGradGroup p, int64_t layers, int dtype);
