@@ -14,8 +14,8 @@
 //
 // What the products of a group read is kept for it: 9 values a token and unit of width, beside the 16 of a block's activations.  So a group
 // has the fewest blocks whose groups are estimated within GROUP_SLACK of the best: twelve blocks 768 wide in bf16 are 6.75 rounds of tiles and
-// go as five and seven (2.8 and 3.9), in fp32
-// 20.25 and three times four (6.75).  Peak memory and time of a training step, all twelve in one launch / so: 16x1024 bf16 10.25 / 9.12 GB, 17.24 / 17.18 ms, 8x512 fp32 6.75 / 5.85 GB, 19.8 / 19.6 ms.
+// go as five and seven (2.8 and 3.9), in fp32 20.25 and three times four (6.75).  Peak memory and time of a training step, all twelve in
+// one launch / so: 16x1024 bf16 10.25 / 9.12 GB, 17.24 / 17.18 ms, 8x512 fp32 6.75 / 5.85 GB, 19.8 / 19.6 ms.
 #include "gemm_tile_launch.h"
 #include "gemm_plan.h"
 

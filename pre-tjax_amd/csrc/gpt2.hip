@@ -193,7 +193,7 @@ size_t ptj_gpt2_acts_bytes(const ptj_gpt2_shape* s, int keep) {
 }
 
 size_t ptj_gpt2_workspace_bytes(const ptj_gpt2_shape* s, int backward) {
-    return check_shape("gpt2_workspace_bytes", s) == PTJ_OK ? make_temps(*s, backward != 0).total : 0;
+    return check_shape("gpt2_workspace_bytes", s) == PTJ_OK ? make_temps(*s, backward != 0, backward != 2).total : 0;
 }
 
 int ptj_gpt2_fwd(const ptj_gpt2_shape* sp, const void* const* params, const int64_t* tokens, const uint32_t* mask,

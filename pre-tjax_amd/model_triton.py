@@ -807,7 +807,11 @@ def _native_bwd(acts, params, x_last, dh):
     dh = dh.contiguous()
     demb = torch.empty_like(dh)
     ws_bytes = lib().ptj_gpt2_workspace_bytes(acts.shape, 1)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dh.device)
+    try:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dh.device)
+    except torch.OutOfMemoryError:             # the weight gradients block by block, slower and in less room
+        ws_bytes = lib().ptj_gpt2_workspace_bytes(acts.shape, 2)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dh.device)
     weights = [p.contiguous() for grp in params for p in grp]
     check(lib().ptj_gpt2_bwd(acts.shape, _pointers(weights), ptr(acts.mask), acts.seeds,
                              acts.buf.data_ptr(), acts.buf.numel(), x_last.data_ptr(), dh.data_ptr(), _pointers(flat),

@@ -31,3 +31,11 @@ def test_never_more_than_sixteen_blocks(dtype, layers, tokens):
     a_block = tokens * (F + 5 * D) * (4 if dtype == 0 else 2)
     sums = 4 * ((tokens + 31) // 32 * F + 2 * 512 * 3 * D) + 4096
     assert workspace(layers, tokens, dtype) - workspace(1, tokens, dtype) <= min(layers, 16) * a_block + layers * sums
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_the_least_that_is_taken(dtype):
+    a_block = 4096 * (F + 5 * D) * (4 if dtype == 0 else 2)
+    least, whole = workspace(12, 4096, dtype, 2), workspace(12, 4096, dtype)
+    assert least <= whole - 2 * a_block
+    assert workspace(1, 4096, dtype, 2) == workspace(1, 4096, dtype)

@@ -1,6 +1,8 @@
 """The native backward with the weight gradients of several blocks in one launch against the single calls: one step of the
 contraction and many, a last one that is not whole, tiles that end inside in both directions, two groups of unequal size, and
 gradients off the 16-byte grid, which are formed block by block."""
+import ctypes
+
 import pytest
 import torch
 
@@ -77,3 +79,35 @@ def test_workspace_of_one_block(mt, lo, monkeypatch, dtype):
     for i, (a, b) in enumerate(zip(got, want)):
         assert (a - b).norm() <= bound * b.norm(), i
     assert backward(small - 1, small)[0] != 0
+
+
+def test_out_of_memory_takes_the_small_workspace(mt, lo, monkeypatch):
+    """Where the room for several blocks' weight gradients is not to be had, a step runs in that for one block; where that is not to be had
+    either, the error is torch's."""
+    L, T, D, F, H = 3, 64, 768, 3072, 12
+    params = [[p.to(DEV) for p in grp] for grp in ogpt2.init_transformer_gpt2(101, D, L, H, F, T, seed=3)]
+    y = torch.randint(0, 101, (1, T + 1), generator=torch.Generator().manual_seed(7)).to(DEV)
+    seeds = list(range(10, 11 + 3 * L))
+    want, _ = lo.t_loss_bkwd3_t(params, y, None, None, True, seeds)
+    shape = (ctypes.c_int64 * 9)(L, 1, T, D, H, F, 101, 0, 1)
+    whole, least = (mt.lib().ptj_gpt2_workspace_bytes(shape, b) for b in (1, 2))
+    assert least < whole
+    empty, asked = torch.empty, []
+
+    def limited(limit):
+        def f(*args, **kw):
+            if args and args[0] in (whole, least):
+                asked.append(args[0])
+                if args[0] > limit:
+                    raise torch.OutOfMemoryError("no room")
+            return empty(*args, **kw)
+        return f
+
+    monkeypatch.setattr(mt.torch, "empty", limited(least))
+    got, _ = lo.t_loss_bkwd3_t(params, y, None, None, True, seeds)
+    assert asked == [whole, least]
+    for a, b in zip([p for g in got for p in g], [p for g in want for p in g]):
+        assert (a.double() - b.double()).norm() <= 2e-6 * b.double().norm()
+    monkeypatch.setattr(mt.torch, "empty", limited(least - 1))
+    with pytest.raises(torch.OutOfMemoryError):
+        lo.t_loss_bkwd3_t(params, y, None, None, True, seeds)
