@@ -1,5 +1,5 @@
 """The native backward with the weight gradients of several blocks in one launch against the single calls: one step of the
-contraction and many, a last one that is not whole, tiles that end inside in both directions, two groups of unequal size, and
+contraction and many (whole ones: token counts are multiples of 64), tiles that end inside in both directions, two groups of unequal size, and
 gradients off the 16-byte grid, which are formed block by block."""
 import ctypes
 
