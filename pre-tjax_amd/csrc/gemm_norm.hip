@@ -251,8 +251,12 @@ NpTile np_tile(int64_t rows, int64_t dim, int64_t m, int dtype) {
 template <int ITERS, int TBM, int TBN>
 void np_launch(const NormProductArgs& g, hipStream_t st) {
     const dim3 grid((unsigned)(((g.rows + TBM - 1) / TBM) * ((g.m + TBN - 1) / TBN)));
-    if (g.part != nullptr) hipLaunchKernelGGL((norm_product_kernel<ITERS, TBM, TBN, true>), grid, dim3(NP_THREADS), 0, st, g);
-    else hipLaunchKernelGGL((norm_product_kernel<ITERS, TBM, TBN, false>), grid, dim3(NP_THREADS), 0, st, g);
+    if constexpr (TBM == 16)
+        if (g.part != nullptr) {
+            hipLaunchKernelGGL((norm_product_kernel<ITERS, TBM, TBN, true>), grid, dim3(NP_THREADS), 0, st, g);
+            return;
+        }
+    hipLaunchKernelGGL((norm_product_kernel<ITERS, TBM, TBN, false>), grid, dim3(NP_THREADS), 0, st, g);
 }
 template <int ITERS>
 void np_launch(const NormProductArgs& g, const NpTile& t, hipStream_t st) {
@@ -271,11 +275,11 @@ bool ptj_norm_product_fits(int64_t rows, int64_t dim, int64_t m, int dtype, bool
 int ptj_norm_product(const PtjNormProduct& p, int64_t rows, int64_t dim, int64_t m, int dtype, hipStream_t st) {
     const NpTile t = np_tile(rows, dim, m, dtype);
     PTJ_CHECK_ARG((p.x.part || p.x.c) && p.res && p.gamma && p.beta && p.w && p.y && p.c && (p.bias || !p.gelu), "norm_product: null pointer");
-    bool ok = t.rows > 0;
+    bool ok = t.rows > 0 && (!p.x.part || t.rows == 16);
     for (const void* q : {p.x.part ? (const void*)p.x.part : p.x.c, p.x.part ? p.x.bias : nullptr, p.res, p.gamma, p.beta, p.w, p.bias, (const void*)p.y,
                           (const void*)p.c})
         ok = ok && ptj_aligned16(q);
-    if (!ok) return ptj_set_error(PTJ_ERR_INVALID, "norm_product: %lld rows of %lld, %lld outputs or unaligned operands", (long long)rows,
+    if (!ok) return ptj_set_error(PTJ_ERR_INVALID, "norm_product: %lld rows of %lld, %lld outputs, partial sums or unaligned operands", (long long)rows,
                                   (long long)dim, (long long)m);
     const NormProductArgs g = {(const bf16*)p.x.c, p.x.part, (const bf16*)p.x.bias, (const bf16*)p.res, (const bf16*)p.gamma, (const bf16*)p.beta,
                                (const bf16*)p.w, (const bf16*)p.bias, (bf16*)p.y, (bf16*)p.c, p.x.splits, (int)rows, (int)m, p.gelu};
