@@ -389,8 +389,9 @@ def main():
             return rc
 
     # One wrapper call per launch, so that every GEMM can be bracketed; the timed steps above issue the stack as one native
-    # call per direction.  At this size both launch the same GEMM kernels on the same shapes (the native call merges
-    # products only where each alone would leave the chip half empty).
+    # call per direction.  The forward and dX products are the same launches either way at this size; the blocks' weight
+    # gradients are single products with K splits here, while the native call forms those of several blocks in one launch,
+    # which this figure does not time.
     mt.NATIVE_STACK = False
     _lib._lib.ptj_gemm = Timed(orig_gemm, 4)
     _lib._lib.ptj_gemm_mul_colsum = Timed(orig_gemm_mul, 5)   # the product whose epilogue is the GELU backward
@@ -477,12 +478,13 @@ def main():
                                            "note": "the same step with mask=None (kernels mask by index, nothing packed)"}},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 1), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_BF16_TFLOPS, 4), "traffic": traffic,
-                     "traffic_note": "bytes per GEMM launch at the L2 boundary (average over the launches of a step) from "
+                     "traffic_note": "bytes per GEMM launch at the L2 boundary (average over the launches of a step, call by call) from "
                                      "rocprofv3 FETCH_SIZE / WRITE_SIZE runs scaled by a 1 GiB copy, read from "
                                      "profiles/%s; algorithmic minimum %.4g" % (os.path.basename(GEMM_TRAFFIC_FILE),
                                                                                  float((traffic_src or {}).get("algorithmic_bytes_per_launch", 0))),
                      "kernel": "gemm_ring_kernel and gemm_tile_kernel, bf16 (all %d launches of a step: fwd, "
-                               "dX, dW; events around single calls, in further steps issued call by call)"
+                               "dX, dW; events around single calls, in further steps issued call by call: the timed steps form "
+                               "the blocks' dW in shared launches instead)"
                                % (n_launch // args.steps),
                      "avg_launch_ms": round(gemm_ms / n_launch, 4),
                      "gflop_per_launch": round(gemm_flops / n_launch / 1e9, 2),

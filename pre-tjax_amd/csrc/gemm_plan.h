@@ -8,7 +8,8 @@
 // (microseconds) are fitted per kernel to timings of the 12 products of a GPT-2 small block, forward, dX and dW
 // (launches replayed from a graph, operands rotating over 200 MB).  bf16: checked on these at eight token counts from 448 to
 // 16384, against every kernel and K split within 1.6 times the lowest estimate, the estimate is off by 8 % rms and the pick is
-// 0.4 % slower than the best one on average and 11 % at worst.
+// 0.4 % slower than the best one on average and 11 % at worst.  (Before the configurations for up to a round of tiles, 8 to 10, which are
+// fitted to their own sizes below.)
 // (64x128 and two 128x128 tiles a CU were fitted again on 1280 to 2048 tokens, where the first was estimated 10 % low and the
 // picks had become up to 8 % slower than those before the ring kernels.  Forward before these / now, in turn on one box:
 // 1280 tokens 944 / 920 us, 1408 1114 / 1082, 1536 1107 / 1088, 2048 1332 / 1333.)

@@ -495,7 +495,7 @@ __global__ __launch_bounds__(LnBwdGeom<TPR>::BLOCK, (TPR == 64 && ITERS <= 3 && 
 // the current one is requested -- all of its vectors at once, in storage form -- before the current
 // row's arithmetic starts (the general kernel's loads end up interleaved with the conversions that
 // consume them, a row at a time).  Same operations in the same order as the general kernel: the
-// results are bit-equal to it.
+// results are bit-equal to it, in both types (tests/test_gpu_row_widths.py).  768 columns, the only such width that the models here have.
 template <typename T, int VEC, int ITERS, int DROP>
 __global__ __launch_bounds__(512, DROP == 1 ? 2 : 4) void layernorm_bwd_exact_kernel(
     const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ gamma, const T* __restrict__ res,

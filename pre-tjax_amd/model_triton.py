@@ -743,8 +743,9 @@ def t_gpt2_tlayer_bkwd3_t(dloss_dx, acts, layer_params, y, mask, train=True, p_g
 
 
 # ---- the whole stack in one native call (csrc/gpt2.hip) -------------------------------------------
-# False: issue the stack one wrapper call at a time.  The same bits, except for bf16 gradients of small batches: there the
-# native call forms the two products of a linear layer's backward in one launch, whose tiles add in another order.
+# False: issue the stack one wrapper call at a time.  The same bits, except where the native call puts several products in one
+# launch, whose tiles add in another order: the weight gradients of several blocks (both types, from a round of tiles on), the two
+# products of a linear layer's backward (bf16), and the norms inside products of the bf16 forward of few tokens without dropout.
 NATIVE_STACK = True
 
 
