@@ -5,7 +5,7 @@
 // on each other, and nothing in the backward waits for them: what they read is kept and all of them go at once, whole tiles along
 // the contraction, in rounds that are full but for the last.  The kernels are those of gemm_ring.h and gemm_split.h with another way
 // from a work item to its operands.  Twelve blocks 768 wide, all weight gradients: 16384 tokens bf16 3.30 ms in 48 launches with
-// 36 second stages, 2.22 ms (1250 TFLOP/s) in one; 4096 tokens fp32 4.6 -> 4.2 ms.
+// 36 second stages, 2.22 ms (1250 TFLOP/s) in one and 2.03 in two; 4096 tokens fp32 4.6 -> 4.2 ms.
 //
 // Taken from a round of tiles on (ptj_weight_grads_blocks).  Training steps, each with its dX / together, us: 12 blocks of 768, bf16, 64 tokens
 // 1914 / 1686, 512 2469 / 2455, 1536 3663 / 3598, 4096 6437 / 5772, 16384 18165 / 17059, fp32 64 2634 / 2322, 1024 7757 / 7057, 3072 17255 /
@@ -13,9 +13,10 @@
 // 6305 / 6141; no size was slower.
 //
 // What the products of a group read is kept for it: 9 values a token and unit of width, beside the 16 of a block's activations.  So a group
-// has the fewest blocks whose groups are estimated within GROUP_SLACK of the best: twelve blocks 768 wide in bf16 are 6.75 rounds of tiles and
-// go as five and seven (2.8 and 3.9), in fp32 20.25 and three times four (6.75).  Peak memory and time of a training step, all twelve in
-// one launch / so: 16x1024 bf16 10.25 / 9.12 GB, 17.24 / 17.18 ms, 8x512 fp32 6.75 / 5.85 GB, 19.8 / 19.6 ms.
+// has the fewest blocks whose groups are estimated within GROUP_SLACK of the best: twelve blocks 768 wide in bf16 go as
+// five in 2.8 rounds of 256x192 tiles and seven in 2.95 of 256x256, in fp32 as three times four (6.75 rounds, all at once 20.25).  Peak memory
+// and time of a training step, all twelve in one launch / so: 16x1024 bf16 10.25 / 9.12 GB, 17.24 / 17.18 ms, 8x512 fp32 6.75 / 5.85 GB,
+// 19.8 / 19.6 ms.
 #include "gemm_tile_launch.h"
 #include "gemm_plan.h"
 

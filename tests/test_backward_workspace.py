@@ -15,8 +15,8 @@ def workspace(layers, tokens, dtype, backward=1):
 
 @pytest.mark.parametrize("dtype,tokens,blocks", [(1, 16384, 7), (1, 65536, 7), (0, 4096, 4), (0, 32768, 4)])
 def test_a_part_of_the_blocks_is_kept(dtype, tokens, blocks):
-    """Of 256x192 tiles (bf16) twelve blocks are 6.75 rounds and seven and five 3.9 and 2.8: seven rounds either way; of 128x128 (fp32)
-    20.25, and 6.75 for four."""
+    """bf16: seven blocks are 2.95 rounds of 256x256 tiles and five 2.8 of 256x192, all twelve 5.1 and 6.75; fp32: twelve 20.25 of 128x128,
+    four 6.75."""
     a_block = tokens * (F + 5 * D) * (4 if dtype == 0 else 2)          # d(feed-forward), d(qkv), d(residual), the gradient that enters
     sums = 4 * ((tokens + 31) // 32 * F + 2 * 512 * 3 * D)             # and the partial rows of its column sums, which stay for all
     # a block that is not kept adds its partial rows (and its share of alignment) alone
