@@ -12,17 +12,18 @@ uint64_t plan_hash(int64_t n, int64_t m, int64_t k) {
 
 // gemm_plan through a small per-thread table: a training loop asks for the same few dozen products again and again,
 // and the estimate over all tile shapes and splits takes a microsecond.
-GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int loose, int kernels = ANY_KERNEL, bool later = false) {
-    struct Entry { int64_t n, m, k; size_t ws; int elt, cus, loose, kernels, later; GemmPlan plan; };
+GemmPlan cached_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int loose, int kernels = ANY_KERNEL, bool later = false,
+                     bool along = false) {
+    struct Entry { int64_t n, m, k; size_t ws; int elt, cus, loose, kernels, later, along; GemmPlan plan; };
     constexpr int ENTRIES = 128;
     static thread_local Entry table[ENTRIES] = {};
     const int cus = num_cus();
-    const uint64_t kind = (((uint64_t)loose * 2 + kernels) * 2 + later) * 2 + (elt == 2);
-    const uint64_t h = plan_hash(n, m, k) ^ (((uint64_t)ws_bytes * 32 + kind) * 0xD6E8FEB86659FD93ull);
+    const uint64_t kind = ((((uint64_t)loose * 2 + kernels) * 2 + later) * 2 + along) * 2 + (elt == 2);
+    const uint64_t h = plan_hash(n, m, k) ^ (((uint64_t)ws_bytes * 64 + kind) * 0xD6E8FEB86659FD93ull);
     Entry& e = table[(h >> 40) % ENTRIES];
     if (e.n != n || e.m != m || e.k != k || e.ws != ws_bytes || e.elt != elt || e.cus != cus || e.loose != loose ||
-        e.kernels != kernels || e.later != later)
-        e = {n, m, k, ws_bytes, elt, cus, loose, kernels, later, gemm_plan(n, m, k, elt, ws_bytes, cus, loose, kernels, 0, later)};
+        e.kernels != kernels || e.later != later || e.along != along)
+        e = {n, m, k, ws_bytes, elt, cus, loose, kernels, later, along, gemm_plan(n, m, k, elt, ws_bytes, cus, loose, kernels, 0, later, along)};
     return e.plan;
 }
 
@@ -81,7 +82,7 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
                                  "operand layout, k a multiple of 64 and vector-aligned C");
         plan = cached_plan(n, m, k, elt, 0, loose, RING_ONLY);
     } else if (gt_eligible(g, am, bm, ragged ? 8 : 1)) {
-        plan = cached_plan(n, m, k, elt, aligned_ws ? workspace_bytes : 0, loose, ANY_KERNEL, left);
+        plan = cached_plan(n, m, k, elt, aligned_ws ? workspace_bytes : 0, loose, ANY_KERNEL, left, am == KMAJOR && bm == KMAJOR);
     } else if (elt == 2 && !ragged && ring_eligible(g, am, bm)) {
         plan = cached_plan(n, m, k, elt, aligned_ws ? workspace_bytes : 0, loose, RING_ONLY, left);
     }
@@ -129,7 +130,7 @@ int gemm_any(const void* a, const void* b, void* c, const void* bias, int64_t n,
 extern "C" {
 
 // Every wrapper asks before it launches, so the answers are kept, per thread: worked out again for each product they took 5-10 us
-// (twelve plans), looked up 0.2.
+// (some dozen plans), looked up 0.2.
 size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
     if (n <= 0 || m <= 0 || k <= 0) return 0;
     struct Entry { int64_t n, m, k; int elt, cus; size_t need; };
@@ -144,9 +145,9 @@ size_t ptj_gemm_workspace_bytes(int64_t n, int64_t m, int64_t k, int dtype) {
     size_t need = s > 1 ? (size_t)s * n * m * sizeof(float) : choose_tail_split(n, m, k, elt, (size_t)-1, &first, &ts, &tkps);
     for (const int loose : {ALIGNED, LOOSE_OUTPUT, LOOSE_OPERAND})
         for (const int kernels : {ANY_KERNEL, RING_ONLY})
-            for (const bool later : {false, true}) {
-                if (elt != 2 && (later || kernels == RING_ONLY)) continue;      // bf16 alone tells these apart
-                const size_t bytes = gp_workspace_bytes(gemm_plan(n, m, k, elt, (size_t)-1, cus, loose, kernels, 0, later), n, m, k);
+            for (const int sums : {0, 1, 2}) {                                  // neither, left to the next norm, operands along
+                if (elt != 2 && (sums || kernels == RING_ONLY)) continue;       // bf16 alone tells these apart
+                const size_t bytes = gp_workspace_bytes(gemm_plan(n, m, k, elt, (size_t)-1, cus, loose, kernels, 0, sums == 1, sums == 2), n, m, k);
                 if (bytes > need) need = bytes;
             }
     e = {n, m, k, elt, cus, need};

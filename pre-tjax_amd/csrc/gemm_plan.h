@@ -37,6 +37,12 @@ constexpr int RAGGED_FIRST[2] = {6, 4}, RAGGED_END[2] = {8, 6};
 // 8.0, 1536x768x768 8.5 / 8.0, 1536x768x2304 15.3 / 13.9, 1536x768x3072 19 / 17; four and five stages of 128x128, 64x64 and 32x32: no faster.
 // 32x64 and 64x128 with two K groups take no K split: their staging of partial sums costs more than the estimate knows (forward of 512
 // tokens with 64x128 in five 685 us, with 32x64 whole 645; of 1024 tokens with 64x128 in two 962, with 64x64 whole 943).
+// `along` below: 32x32 tiles of operands that both run along the contraction take whole lines of either, and go faster than estimated, where
+// the panels of an operand across it come in half lines.  So there a K split of 64x64 tiles has to start as late as that of the four
+// wavefronts before.  us, operands from memory, 32x32 / 64x64 in parts: along 2183x64x2624 9.9 / 11.9, 700x192x2624 9.1 / 11.2, 312x64x1280 5.3 /
+// 6.6, 814x320x1920 9.7 / 11.6, 526x640x3584 14.0 / 15.6; across 192x768x3072 13.0 / 11.6, 256x768x3072 13.0 / 11.8, 982x256x3456 13.8 / 12.4.
+// (Partial sums that the next norm adds up have a cost of their own, fitted with these tiles.)
+constexpr double SMALL8_SPLIT = 0.92;
 constexpr int GT_END[2] = {11, 6};
 inline bool gt_plain(int type, int i) { return type == 1 || (i != 1 && (i < RAGGED_FIRST[0] || i >= RAGGED_END[0])); }
 constexpr TileCost GT_COST[2][11] = {
@@ -142,10 +148,10 @@ inline double gp_ring_tail_us(const TileCost& c, int64_t n, int64_t m, int64_t k
 // product with another epilogue add in the same order.  `loose`: operands or outputs that do not come in aligned
 // 16-byte vectors; the ring kernels take such operands not at all and write such outputs element by element (twice the
 // time at k = 768), the tile kernels write any.
-// `later`: the consumer adds up the partial sums of a K split (PTJ_EPI_BIAS_NORM).
+// `later`: the consumer adds up the partial sums of a K split (PTJ_EPI_BIAS_NORM).  `along`: both operands run along the contraction.
 // `planes_ws`: workspace for operands split ahead of a product without a K split, where partial sums may not take any.
 inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_bytes, int cus, int loose = ALIGNED,
-                          int kernels = ANY_KERNEL, size_t planes_ws = 0, bool later = false) {
+                          int kernels = ANY_KERNEL, size_t planes_ws = 0, bool later = false, bool along = false) {
     const bool ragged = loose == LOOSE_OPERAND;
     GemmPlan best = {-1, 1, (int)k, 0, 1, 0, 1e30};
     const int type = elt == 2 ? 0 : 1;
@@ -158,7 +164,7 @@ inline GemmPlan gemm_plan(int64_t n, int64_t m, int64_t k, int elt, size_t ws_by
                 if (s > 1 && (k < 1024 || k / s < 256 || !fits(4.0 * s * (double)n * (double)m))) break;
                 const int64_t kps = gp_ceil(gp_ceil(k, s), c.bkt) * c.bkt;
                 if (s > 1 && gp_ceil(k, kps) != s) continue;
-                const double us = gp_tile_us(c, n, m, k, elt, s, cus, later);
+                const double us = gp_tile_us(c, n, m, k, elt, s, cus, later) + (type == 0 && i == 9 && s > 1 && along && !later ? SMALL8_SPLIT : 0.0);
                 if (us < best.us) best = {i, s, (int)(s > 1 ? kps : k), 0, 1, 0, us};
             }
         }
