@@ -407,8 +407,8 @@ int ptj_attn_bwd(const void* d_o, const void* q, const void* k, const void* v, c
  * three are not touched) and demb [batch * seq, dim] = the gradient of table row + position of every
  * token.  The arithmetic is that of the same sequence of single calls; products that share a launch (dX and dW of a layer, or
  * the weight gradients of several blocks, whose inputs the backward's workspace then keeps) may add their contraction in
- * another order.  What is kept is bounded: of 16 blocks at most, and of the fewest whose launches fill the chip as well as
- * larger ones.  A workspace that holds these inputs for one block alone (backward = 2 in ptj_gpt2_workspace_bytes; 1: as many as are
+ * another order.  What is kept is bounded: of 16 blocks at most, and from 2048 tokens on of the fewest whose launches
+ * fill the chip as well as larger ones.  A workspace that holds these inputs for one block alone (backward = 2 in ptj_gpt2_workspace_bytes; 1: as many as are
  * fastest; 0: the forward's) is taken too, and the blocks go one by one.
  * A null gradient of a weight or of b1 is refused, as is a null entry of `params` that is read. */
 typedef struct ptj_gpt2_shape {

@@ -16,13 +16,16 @@
 // has the fewest blocks whose groups are estimated within GROUP_SLACK of the best: twelve blocks 768 wide in bf16 go as
 // five in 2.8 rounds of 256x192 tiles and seven in 2.95 of 256x256, in fp32 as three times four (6.75 rounds, all at once 20.25).  Peak memory
 // and time of a training step, all twelve in one launch / so: 16x1024 bf16 10.25 / 9.12 GB, 17.24 / 17.18 ms, 8x512 fp32 6.75 / 5.85 GB,
-// 19.8 / 19.6 ms.
+// 19.8 / 19.6 ms.  Up to GROUP_SPLIT_FROM tokens (28 MB a block in bf16) the further launches cost more than the memory is worth: all / so, us: bf16
+// 128 tokens 49 / 60, 512 110 / 112, 1024 176 / 180, 2048 324 / 322, 4096 620 / 608, fp32 128 229 / 245, 512 591 / 623, 1024 1101 / 1100,
+// 2048 2139 / 2126, 4096 4256 / 4176.
 #include "gemm_tile_launch.h"
 #include "gemm_plan.h"
 
 namespace {
 
 constexpr double GROUP_SLACK = 1.02;
+constexpr int GROUP_SPLIT_FROM = 2048;
 
 struct GroupPlan { int cfg; double us; };
 // Tile shape with the lowest estimate (bf16: of gemm_ring.h); `round`: of those with a round of tiles or more, cfg = -1: none
@@ -53,7 +56,9 @@ int ptj_weight_grads_blocks(PtjGradGroup p, int64_t layers, int dtype) {
     auto all = [&](int blocks) { return (double)(layers / blocks) * us[blocks] + us[layers % blocks]; };
     auto fills = [&](int blocks) { p.blocks = blocks; return group_plan(p, dtype, true).cfg >= 0; };
     const int64_t parts = (layers + PtjGradGroup::BLOCKS - 1) / PtjGradGroup::BLOCKS;
-    if (!fills((int)((layers + parts - 1) / parts))) return 0;       // (equal parts, so that no launch is left with a few tiles alone)
+    const int equal = (int)((layers + parts - 1) / parts);
+    if (!fills(equal)) return 0;                      // (equal parts, so that no launch is left with a few tiles alone)
+    if (p.k < GROUP_SPLIT_FROM) return equal;
     for (int i = 1; i <= most; ++i)
         if (fills(i) && all(i) < best) best = all(i);
     for (int i = 1; i <= most; ++i)

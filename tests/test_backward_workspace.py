@@ -25,6 +25,14 @@ def test_a_part_of_the_blocks_is_kept(dtype, tokens, blocks):
 
 
 @pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("tokens", [64, 512, 1984])
+def test_all_blocks_of_few_tokens(dtype, tokens):
+    """Further launches cost 2 to 20 % of them (us in csrc/gemm_group.hip), what is kept is at most 28 MB a block in bf16."""
+    a_block = tokens * (F + 5 * D) * (4 if dtype == 0 else 2)
+    assert workspace(12, tokens, dtype) - workspace(7, tokens, dtype) >= 5 * a_block
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
 @pytest.mark.parametrize("layers", [1, 2, 3, 12, 17, 48])
 @pytest.mark.parametrize("tokens", [64, 512, 4096, 16384])
 def test_never_more_than_sixteen_blocks(dtype, layers, tokens):
